@@ -85,6 +85,16 @@ int metis_rmsnorm_colmean(const void* x, const void* gamma, float eps, int64_t r
                            workspace_bytes, (hipStream_t)stream);
 }
 
+size_t metis_rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols) { return rmsnorm_backward_workspace_bytes(rows, cols); }
+
+int metis_rmsnorm_backward(const void* x, const void* grad, const void* gamma, float eps, int64_t rows, int64_t cols, void* grad_x,
+                           void* grad_gamma, int grad_gamma_dtype, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (grad_gamma_dtype != METIS_DTYPE_BF16 && grad_gamma_dtype != METIS_DTYPE_F32) return METIS_E_ARG;
+    return rmsnorm_backward(x, grad, gamma, eps, rows, cols, grad_x, grad_gamma, grad_gamma_dtype == METIS_DTYPE_BF16, workspace,
+                            workspace_bytes, (hipStream_t)stream);
+}
+
 int metis_nvfp4_quant_dequant_row(const void* x, int64_t rows, int64_t cols, int mode, void* codes, void* scales, float* unit,
                                   void* out, void* workspace, size_t workspace_bytes, void* stream)
 {

@@ -322,23 +322,137 @@ __global__ __launch_bounds__(256) void rmsnorm_colsum_rows_kernel(const uint4* _
     for (uint32_t q = threadIdx.x; q < cpr * 2u; q += 256u) out[q] = sums[q >> 1][q & 1u];
 }
 
+// ---------------------------------------------------------------------------------------------
+// Backward of the norm: one pass over x and the output gradient g instead of a chain of fifteen elementwise and reduction
+// kernels over binary32 copies.  In binary32, with xh = x * rstd:
+//   gx = bf16(rstd * (g gamma - xh * mean(g gamma xh))),   ggamma[c] = sum over rows of g * bf16(xh)
+// (the product of a row's output with gamma is taken from the bf16-rounded xh, so its gradient is too).
+// One wave owns a row (cols <= 4096) and holds it in registers, the two row sums are folded across the wave with DPP
+// moves, and the column sums stay in registers: rows in order within a wave, then the workgroup's waves in order, then
+// (rmsnorm_colmean_finish_kernel) the workgroups in order -- a fixed order from call to call.
+// Bound by memory: 6 B per element.  The sums cost registers (NL = 8: two waves per SIMD), so the loads of a row are not
+// issued ahead of the previous one.  An MLP's training step (bf16 arithmetic) with it: 4096 tokens, 1536 -> 8960:
+// 1906 -> 1762 us; 2103 tokens, 3584 -> 18944: 4502 -> 4338 us.
+// ---------------------------------------------------------------------------------------------
+template <int NL, bool SUMS>
+__global__ __launch_bounds__(256, 2) void rmsnorm_backward_rows_kernel(const uint4* __restrict__ x, const uint4* __restrict__ g,
+                                                                       const uint4* __restrict__ gamma, float eps, uint32_t rows, uint32_t cols,
+                                                                       uint4* __restrict__ gx, float* __restrict__ partial)
+{
+    __shared__ float4 sums[SUMS ? NL * 64 : 1][2];             // column sums of the workgroup, chunk by chunk
+    const uint32_t cpr = cols / 8u;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const float fcols = (float)cols;
+    float acc[SUMS ? NL : 1][8];
+#pragma unroll
+    for (int i = 0; i < (SUMS ? NL : 1); ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = 0.0f;
+    __shared__ uint4 gm[NL * 64];
+    for (uint32_t c = threadIdx.x; c < (uint32_t)NL * 64u; c += 256u) gm[c] = c < cpr ? gamma[c] : make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    for (uint32_t row = blockIdx.x * 4u + wave; row < rows; row += gridDim.x * 4u) {
+        uint4 xr[NL], gr[NL];
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint32_t c = i * 64u + lane;
+            xr[i] = gr[i] = make_uint4(0u, 0u, 0u, 0u);
+            if (c < cpr) {
+                xr[i] = x[(size_t)row * cpr + c];
+                gr[i] = g[(size_t)row * cpr + c];
+            }
+        }
+        float ss = 0.0f, dot = 0.0f;                           // sum x^2, sum (g gamma) x
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint32_t xw[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w}, gw[4] = {gr[i].x, gr[i].y, gr[i].z, gr[i].w};
+            const uint4 m = gm[i * 64 + lane];
+            const uint32_t mw[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float x0 = bf16_lo(xw[j]), x1 = bf16_hi(xw[j]);
+                ss = fmaf(x0, x0, ss);
+                ss = fmaf(x1, x1, ss);
+                dot = fmaf(bf16_lo(gw[j]) * bf16_lo(mw[j]), x0, dot);
+                dot = fmaf(bf16_hi(gw[j]) * bf16_hi(mw[j]), x1, dot);
+            }
+        }
+        // the row stays packed: without this the compiler keeps every unpacked value alive to the second loop (256 registers, spills)
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            asm volatile("" : "+v"(xr[i].x), "+v"(xr[i].y), "+v"(xr[i].z), "+v"(xr[i].w), "+v"(gr[i].x), "+v"(gr[i].y), "+v"(gr[i].z), "+v"(gr[i].w));
+        ss = wave_sum_dpp(ss);
+        dot = wave_sum_dpp(dot);
+        const float rstd = 1.0f / sqrtf(ss / fcols + eps);
+        const float mean = dot * rstd / fcols;                 // mean over the row of g gamma xh
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint32_t c = i * 64u + lane;
+            if (i * 64u >= cpr) break;                         // wave-uniform: chunks beyond the row
+            const uint32_t xw[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w}, gw[4] = {gr[i].x, gr[i].y, gr[i].z, gr[i].w};
+            const uint4 m = gm[c];
+            const uint32_t mw[4] = {m.x, m.y, m.z, m.w};
+            uint32_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float h0 = bf16_lo(xw[j]) * rstd, h1 = bf16_hi(xw[j]) * rstd;
+                const float g0 = bf16_lo(gw[j]), g1 = bf16_hi(gw[j]);
+                if constexpr (SUMS) {
+                    const uint32_t hb = rb_pair(h0, h1);
+                    acc[i][2 * j] = fmaf(g0, bf16_lo(hb), acc[i][2 * j]);
+                    acc[i][2 * j + 1] = fmaf(g1, bf16_hi(hb), acc[i][2 * j + 1]);
+                }
+                w[j] = rb_pair(rstd * (g0 * bf16_lo(mw[j]) - h0 * mean), rstd * (g1 * bf16_hi(mw[j]) - h1 * mean));
+            }
+            if (c < cpr) gx[(size_t)row * cpr + c] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+    if constexpr (SUMS) {
+#pragma unroll 1
+        for (uint32_t v = 0; v < 4u; ++v) {                    // the four waves' sums, added in wave order
+            if (wave == v) {
+#pragma unroll
+                for (int i = 0; i < NL; ++i) {
+                    const uint32_t c = i * 64u + lane;
+                    if (c < cpr) {
+                        float4 lo = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]), hi = make_float4(acc[i][4], acc[i][5], acc[i][6], acc[i][7]);
+                        if (v) {
+                            const float4 pl = sums[c][0], ph = sums[c][1];
+                            lo = make_float4(pl.x + lo.x, pl.y + lo.y, pl.z + lo.z, pl.w + lo.w);
+                            hi = make_float4(ph.x + hi.x, ph.y + hi.y, ph.z + hi.z, ph.w + hi.w);
+                        }
+                        sums[c][0] = lo;
+                        sums[c][1] = hi;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        float4* out = reinterpret_cast<float4*>(partial + (size_t)blockIdx.x * cols);
+        for (uint32_t q = threadIdx.x; q < cpr * 2u; q += 256u) out[q] = sums[q >> 1][q & 1u];
+    }
+}
+
 constexpr int kColmeanBatch = 8;
-template <bool OUT_BF16>
-__global__ __launch_bounds__(256) void rmsnorm_colmean_finish_kernel(const float* __restrict__ partial, uint32_t slabs, uint32_t cols,
+// W waves share a column group's partial rows.  Sixteen where there are enough of them: 512 rows of 3584 columns are 56
+// workgroups, and four waves each walk 128 rows eight loads at a time (10.3 us for the launch; with
+// sixteen waves the 4 rounds of loads of a wave are one).
+template <bool OUT_BF16, int W>
+__global__ __launch_bounds__(64 * W) void rmsnorm_colmean_finish_kernel(const float* __restrict__ partial, uint32_t slabs, uint32_t cols,
                                                                      float count, void* __restrict__ out, const void* __restrict__ cached,
                                                                      float cached_count, float rows_f, float* __restrict__ out32)
 {
-    __shared__ float part[4][64];
+    __shared__ float part[W][64];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t c = blockIdx.x * 64u + lane;
     float s = 0.0f;
     if (c < cols) {
-        // wave w adds the partial rows w, w + 4, ... in order, kColmeanBatch loads in flight at a time
-        for (uint32_t k0 = wave; k0 < slabs; k0 += 4u * kColmeanBatch) {
+        // wave w adds the partial rows w, w + W, ... in order, kColmeanBatch loads in flight at a time
+        for (uint32_t k0 = wave; k0 < slabs; k0 += (uint32_t)W * kColmeanBatch) {
             float v[kColmeanBatch];
 #pragma unroll
             for (int b = 0; b < kColmeanBatch; ++b) {
-                const uint32_t k = k0 + 4u * b;
+                const uint32_t k = k0 + (uint32_t)W * b;
                 v[b] = k < slabs ? partial[(size_t)k * cols + c] : 0.0f;
             }
 #pragma unroll
@@ -348,7 +462,9 @@ __global__ __launch_bounds__(256) void rmsnorm_colmean_finish_kernel(const float
     part[wave][lane] = s;
     __syncthreads();
     if (wave != 0 || c >= cols) return;
-    s = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    s = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; w += 4) s += (part[w][lane] + part[w + 1][lane]) + (part[w + 2][lane] + part[w + 3][lane]);
     auto rnd = [](float x) { return OUT_BF16 ? __uint_as_float(bf16_bits(x) << 16) : x; };
     float m = rnd(s / count);
     if (cached) {                                              // weighted running mean of decode calls, bitlinear.py:316-323
@@ -360,6 +476,18 @@ __global__ __launch_bounds__(256) void rmsnorm_colmean_finish_kernel(const float
     if (OUT_BF16) static_cast<uint16_t*>(out)[c] = (uint16_t)bf16_bits(m);
     else static_cast<float*>(out)[c] = m;
     if (out32) out32[c] = m;
+}
+
+static int finish_column_sums(const float* partial, int slabs, int64_t cols, float count, void* out, int out_bf16, const void* cached,
+                              float cached_count, float rows_f, float* out32, hipStream_t st)
+{
+    const dim3 g((unsigned)((cols + 63) / 64));
+#define METIS_CF(B, W) hipLaunchKernelGGL((rmsnorm_colmean_finish_kernel<B, W>), g, dim3(64 * W), 0, st, partial, (uint32_t)slabs, (uint32_t)cols, \
+        count, out, cached, cached_count, rows_f, out32)
+    if (slabs >= 64) { if (out_bf16) METIS_CF(true, 16); else METIS_CF(false, 16); }
+    else { if (out_bf16) METIS_CF(true, 4); else METIS_CF(false, 4); }
+#undef METIS_CF
+    return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 
 static int colmean_grid(int64_t rows)
@@ -394,14 +522,48 @@ int rmsnorm_colmean(const void* x, const void* gamma, float eps, int64_t rows, i
     if (nl <= 2) METIS_RC(2); else if (nl <= 4) METIS_RC(4); else METIS_RC(8);
 #undef METIS_RC
     if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
-    const dim3 g2((unsigned)((cols + 63) / 64));
-    if (mean_bf16)
-        hipLaunchKernelGGL(rmsnorm_colmean_finish_kernel<true>, g2, dim3(256), 0, st, partial, (uint32_t)g, (uint32_t)cols, (float)rows, mean, cached,
-                           (float)cached_count, (float)rows, mean32);
-    else
-        hipLaunchKernelGGL(rmsnorm_colmean_finish_kernel<false>, g2, dim3(256), 0, st, partial, (uint32_t)g, (uint32_t)cols, (float)rows, mean, cached,
-                           (float)cached_count, (float)rows, mean32);
-    return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
+    return finish_column_sums(partial, g, cols, (float)rows, mean, mean_bf16, cached, (float)cached_count, (float)rows, mean32, st);
+}
+
+// One workgroup per compute unit with the column sums (each leaves a partial row for the finishing launch), enough of
+// them to fill the device without.
+static int backward_grid(int64_t rows, bool sums)
+{
+    int64_t g = (rows + 3) / 4;
+    const int64_t cap = (int64_t)device_cus() * (sums ? 2 : 4);
+    if (g > cap) g = cap;
+    return g < 1 ? 1 : (int)g;
+}
+
+size_t rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols)
+{
+    if (rows <= 0 || cols <= 0) return 0;
+    return (size_t)backward_grid(rows, true) * (size_t)cols * sizeof(float);
+}
+
+int rmsnorm_backward(const void* x, const void* g, const void* gamma, float eps, int64_t rows, int64_t cols, void* gx, void* ggamma,
+                     int ggamma_bf16, void* workspace, size_t workspace_bytes, hipStream_t st)
+{
+    if (rows <= 0 || cols <= 0 || rows > INT32_MAX) return METIS_E_ARG;
+    if (cols % kBlock) return METIS_E_SHAPE;
+    if (cols > 4096) return METIS_E_ARG;                      // one wave per row
+    if (!x || !g || !gamma || !gx) return METIS_E_ARG;
+    if (((uintptr_t)x % 16) || ((uintptr_t)g % 16) || ((uintptr_t)gamma % 16) || ((uintptr_t)gx % 16) || ((uintptr_t)ggamma % (ggamma_bf16 ? 2 : 4)))
+        return METIS_E_ARG;
+    const bool sums = ggamma != nullptr;
+    if (sums && (!workspace || ((uintptr_t)workspace % 16) || workspace_bytes < rmsnorm_backward_workspace_bytes(rows, cols))) return METIS_E_WORKSPACE;
+    const int grid = backward_grid(rows, sums);
+    const int nl = (int)((cols / 8 + 63) / 64);
+    float* partial = static_cast<float*>(workspace);
+#define METIS_RB(NL, S) hipLaunchKernelGGL((rmsnorm_backward_rows_kernel<NL, S>), dim3(grid), dim3(256), 0, st, (const uint4*)x, (const uint4*)g, \
+        (const uint4*)gamma, eps, (uint32_t)rows, (uint32_t)cols, (uint4*)gx, partial)
+#define METIS_RBN(S) do { if (nl <= 2) METIS_RB(2, S); else if (nl <= 4) METIS_RB(4, S); else METIS_RB(8, S); } while (0)
+    if (sums) METIS_RBN(true); else METIS_RBN(false);
+#undef METIS_RBN
+#undef METIS_RB
+    if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
+    if (!sums) return METIS_OK;
+    return finish_column_sums(partial, grid, cols, 1.0f, ggamma, ggamma_bf16, nullptr, 0.0f, 0.0f, nullptr, st);   // (a division by one)
 }
 
 // deferred: stop after the main kernel; `workspace` is then the caller-owned parked data of the deferred form

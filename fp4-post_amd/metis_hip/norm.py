@@ -35,6 +35,9 @@ class _NormedWithGrad(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         x, weight = ctx.saved_tensors
+        if not torch.is_grad_enabled() and ops.rmsnorm_backward_applies(x, g, weight):
+            # one pass on the device; with create_graph the formula below is recorded instead
+            return (*ops.rmsnorm_backward(x, g, weight, ctx.eps, ctx.needs_input_grad[1]), None, None)
         xf, gf = x.float(), g.float()
         rstd = torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + ctx.eps)
         xhat = xf * rstd

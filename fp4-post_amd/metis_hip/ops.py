@@ -887,6 +887,39 @@ def rmsnorm_colmean(x: torch.Tensor, gamma: torch.Tensor, eps: float, mean_dtype
     return normed, me, me32
 
 
+def rmsnorm_backward_applies(x: torch.Tensor, g: torch.Tensor, gamma: torch.Tensor) -> bool:
+    """rmsnorm_backward takes these: bf16 device tensors of the same non-empty shape, a wave per row."""
+    cols = x.shape[-1]
+    return bool(x.is_cuda and x.dtype == torch.bfloat16 and g.dtype == torch.bfloat16 and gamma.dtype == torch.bfloat16
+                and g.device == x.device and gamma.device == x.device and g.shape == x.shape and cols % BLOCK == 0
+                and 0 < cols <= 4096 and x.numel() > 0)
+
+
+def rmsnorm_backward(x: torch.Tensor, g: torch.Tensor, gamma: torch.Tensor, eps: float, want_gamma: bool = True):
+    """(gradient of x, gradient of gamma or None) of y = bf16(bf16(x rstd) gamma) for the gradient g of y, all bf16: one
+    pass over x and g, binary32 arithmetic, column sums in a fixed order rounded once."""
+    def dense(t, cols):
+        t = t.reshape(-1, cols)
+        t = t if t.is_contiguous() else t.contiguous()
+        return t if t.data_ptr() % 16 == 0 else t.clone()
+    cols = x.shape[-1]
+    x2, g2 = dense(x, cols), dense(g, cols)
+    gm = dense(gamma, cols)
+    rows = x2.shape[0]
+    gx = torch.empty(rows, cols, dtype=torch.bfloat16, device=x.device)
+    L = load()
+    gg = ws = None
+    need = 0
+    if want_gamma:
+        gg = torch.empty(cols, dtype=torch.bfloat16, device=x.device)
+        need = L.metis_rmsnorm_backward_workspace_bytes(rows, cols)
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    rc = L.metis_rmsnorm_backward(x2.data_ptr(), g2.data_ptr(), gm.data_ptr(), float(eps), rows, cols, gx.data_ptr(),
+                                  None if gg is None else gg.data_ptr(), DTYPE_BF16, None if ws is None else ws.data_ptr(), need, _stream())
+    check(rc, "metis_rmsnorm_backward", x.shape)
+    return gx.reshape(x.shape), gg
+
+
 @functools.lru_cache(maxsize=16)
 def _device_cus(device_index: int) -> int:
     return int(torch.cuda.get_device_properties(device_index).multi_processor_count)

@@ -249,6 +249,20 @@ int metis_rmsnorm_colmean(const void *x, const void *gamma, float eps, int64_t r
                           void *stream);
 
 /*
+ * Gradients of that RMSNorm (y = bf16(bf16(x rstd) gamma), src/Metis/models/llama.py:23-31) from one pass over x and the
+ * gradient of y, in binary32 with xh = x * rstd:
+ *   grad_x = bf16(rstd * (grad gamma - xh * mean(grad gamma xh)))
+ *   grad_gamma[c] = sum over rows of grad * bf16(xh), binary32 sums in a fixed order, rounded once to grad_gamma_dtype
+ *   x, grad, grad_x  bf16 [rows, cols], cols <= 4096 and a multiple of 16; gamma bf16 [cols]; all 16-byte aligned
+ *   grad_gamma       [cols], or NULL when it is not wanted (no workspace needed then)
+ *   workspace        metis_rmsnorm_backward_workspace_bytes(rows, cols) bytes, 16-byte aligned, no initialisation needed
+ */
+size_t metis_rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols);
+int metis_rmsnorm_backward(const void *x, const void *grad, const void *gamma, float eps, int64_t rows,
+                           int64_t cols, void *grad_x, void *grad_gamma, int grad_gamma_dtype,
+                           void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Block-scaled NVFP4 GEMM with an optional bf16 low-rank extension and bias:
  *   out[M,N] = ua*ub * sum_k deq(A)[m,k] * deq(B)[n,k]  +  sum_j T[m,j] * U[n,j]  +  bias[n]
  * A (M x K) and B (N x K) are packed NVFP4 with blocks of 16 along K; *ua, *ub are their units.

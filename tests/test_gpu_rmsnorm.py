@@ -81,3 +81,37 @@ def test_value_error_and_limits():
     with pytest.raises(ValueError):
         ops.rmsnorm_quantize(torch.zeros(4, 40, dtype=torch.bfloat16, device="cuda"),
                              torch.ones(40, dtype=torch.bfloat16, device="cuda"), 1e-6)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 16), (5, 48), (7, 512), (33, 528), (300, 1040), (2049, 1536), (513, 3584), (9, 4096)])
+def test_rmsnorm_backward(rows, cols):
+    """Both gradients against the same formula in double precision.  gx carries one rounding to bf16 (eight significant bits: 2^-8 of the value)
+    of a difference formed in binary32 (its two terms rounded a few times: 2^-20 of their sizes); ggamma one rounding of a
+    binary32 sum whose terms hold bf16(x rstd): a term may round to the neighbouring bf16 value (2^-8 of the term) where
+    rstd differs in its last bit, which is rare."""
+    from metis_hip import ops
+    eps = 1e-6
+    x = synthetic_activation(40 + rows, rows, cols).cuda()
+    gamma = _gamma(9, cols).cuda()
+    g = (torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows)) * 1e-3).bfloat16().cuda()
+    xd, gd, md = x.double(), g.double(), gamma.double()
+    rstd = (xd.pow(2).mean(-1, keepdim=True) + eps).rsqrt()
+    xh = xd * rstd
+    gh = gd * md
+    mean = (gh * xh).mean(-1, keepdim=True)
+    want = rstd * (gh - xh * mean)
+    terms = gd * xh.float().bfloat16().double()
+    gx, gg = ops.rmsnorm_backward(x, g, gamma, eps)
+    assert bool(((gx.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * rstd * (gh.abs() + (xh * mean).abs()) + 1e-30).all())
+    want_g = terms.sum(0)
+    slack = 2.0 ** -8 * terms.abs().amax(0) * (1 + rows / 2000) + 2.0 ** -20 * terms.abs().sum(0)
+    assert bool(((gg.double() - want_g).abs() <= 2.0 ** -8 * want_g.abs() + slack).all())
+    # without gamma's gradient, from a gradient that is a strided view, and from one that is not 16-byte aligned: the same bits
+    wide = torch.zeros(rows, cols + 8, dtype=torch.bfloat16, device="cuda")
+    wide[:, 1:cols + 1] = g
+    odd = torch.zeros(rows * cols + 1, dtype=torch.bfloat16, device="cuda")[1:].view(rows, cols).copy_(g)
+    assert torch.equal(ops.rmsnorm_backward(x, wide[:, 1:cols + 1], gamma, eps)[0], gx)
+    again = ops.rmsnorm_backward(x, odd, gamma, eps)
+    assert torch.equal(again[0], gx) and torch.equal(again[1], gg)
+    only, none = ops.rmsnorm_backward(x, g, gamma, eps, want_gamma=False)
+    assert none is None and torch.equal(only, gx)
