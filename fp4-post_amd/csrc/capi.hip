@@ -211,6 +211,25 @@ int metis_nvfp4_quant_sr_both(const void* x, int64_t rows, int64_t cols, int64_t
                             unit_col, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+int metis_nvfp4_quant_col_padded(const void* x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld, int mode, const void* center,
+                                 int sr, uint64_t seed, uint64_t offset, void* codes, void* scales, float* unit, void* workspace,
+                                 size_t workspace_bytes, void* stream)
+{
+    if (rows < 0 || rows > padded_rows) return METIS_E_ARG;
+    return quantize(x, padded_rows, cols, ld, mode, sr != 0, true, nullptr, seed, offset, codes, scales, unit, workspace, workspace_bytes,
+                    (hipStream_t)stream, center, false, 0, nullptr, rows);
+}
+
+int metis_nvfp4_quant_sr_both_padded(const void* x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld, int mode, uint64_t seed,
+                                     uint64_t offset_row, uint64_t offset_col, void* codes_row, void* scales_row, float* unit_row,
+                                     void* codes_col, void* scales_col, float* unit_col, void* workspace, size_t workspace_bytes,
+                                     void* stream)
+{
+    if (rows < 0 || rows > padded_rows) return METIS_E_ARG;
+    return quantize_both_sr(x, padded_rows, cols, ld, mode, seed, offset_row, offset_col, codes_row, scales_row, unit_row, codes_col,
+                            scales_col, unit_col, workspace, workspace_bytes, (hipStream_t)stream, rows);
+}
+
 size_t metis_nvfp4_deferred_bytes(int64_t rows, int64_t cols) { return deferred_bytes(rows, cols); }
 
 int metis_nvfp4_quant_row_deferred(const void* x, int64_t rows, int64_t cols, int mode, const void* center, void* codes, void* deferred,

@@ -63,11 +63,11 @@ int launch_scales(int mode, const Workspace& ws, uint32_t ngroups, void* scales,
 int quantize(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, bool sr, bool col, const void* noise,
              uint64_t seed, uint64_t offset, void* codes, void* scales, float* unit, void* workspace,
              size_t workspace_bytes, hipStream_t st, const void* center = nullptr, bool resident = false,
-             uint32_t spin_limit = 0, void* decode = nullptr);
+             uint32_t spin_limit = 0, void* decode = nullptr, int64_t valid = -1);   // valid >= 0 (col): rows that x has, the rest is padding
 // both packings (blocks along rows, blocks down columns) of one tensor with stochastic rounding in one pass; nvfp4_quant.hip
 int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, uint64_t seed, uint64_t offset_row,
                      uint64_t offset_col, void* codes_row, void* scales_row, float* unit_row, void* codes_col, void* scales_col,
-                     float* unit_col, void* workspace, size_t bytes, hipStream_t st);
+                     float* unit_col, void* workspace, size_t bytes, hipStream_t st, int64_t valid = -1);
 // deferred scale bytes (nvfp4_quant.hip): phase 1 alone into caller-owned parked data, phase 2 on it later or never
 size_t deferred_bytes(int64_t rows, int64_t cols);
 int carve_deferred(void* p, size_t bytes, int64_t rows, int64_t cols, Workspace* ws);

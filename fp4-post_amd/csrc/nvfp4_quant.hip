@@ -259,6 +259,9 @@ __global__ __launch_bounds__(256) void quant_codes_kernel(
 // instruction reading 64 consecutive columns of one row.  Codes and block maxima are transposed
 // through LDS so that they leave as 32-byte (8-byte) pieces of the 128 (32) contiguous bytes each
 // column owns in the tile, instead of one scattered 8-byte and 2-byte store per lane.
+// Rows from `valid` on (valid < rows: a ragged token count padded to the contraction step) are not read: their residual is
+// zero, as if the tensor had been copied and filled up with rows equal to the centre.  Without those copies of x and dY a
+// training step of an MLP on 2103 tokens (3584 -> 18944, mean mode) takes 4061 instead of 4338 us.
 // ---------------------------------------------------------------------------------------------
 constexpr int kColTileBlocks = 16, kColTileCols = 64;
 // F32IN (WIDE only): the input tensor itself is binary32; a compile-time choice, so that the sixteen loads of a block are
@@ -267,7 +270,7 @@ template <int MODE, bool SR, bool WIDE = false, bool F32IN = false>
 __global__ __launch_bounds__(256) void quant_codes_col_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, const void* __restrict__ noise,
     uint64_t seed, uint64_t offset, uint2* __restrict__ codes, void* __restrict__ ws_amax_v,
-    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, const void* __restrict__ center)
+    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, const void* __restrict__ center, uint32_t valid)
 {
     static_assert(!F32IN || WIDE, "binary32 input implies binary32 values");
     static_assert(!WIDE || MODE == 0, "binary32 values imply binary32 arithmetic");
@@ -289,10 +292,22 @@ __global__ __launch_bounds__(256) void quant_codes_col_kernel(
             float am = 0.0f;
             if (c < cols && b < nbc) {
                 float v[kBlock], u[kBlock] = {};
+                const uint32_t have = valid > b * kBlock ? valid - b * kBlock : 0u;   // rows of this block that x has (the same for the wave)
+                if (have >= (uint32_t)kBlock) {
 #pragma unroll
-                for (int j = 0; j < kBlock; ++j) {
-                    if constexpr (F32IN) v[j] = static_cast<const float*>(xv)[(int64_t)(b * kBlock + j) * ld + c];
-                    else v[j] = bf16_lo(x[(int64_t)(b * kBlock + j) * ld + c]);
+                    for (int j = 0; j < kBlock; ++j) {
+                        if constexpr (F32IN) v[j] = static_cast<const float*>(xv)[(int64_t)(b * kBlock + j) * ld + c];
+                        else v[j] = bf16_lo(x[(int64_t)(b * kBlock + j) * ld + c]);
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < kBlock; ++j) {
+                        v[j] = 0.0f;
+                        if ((uint32_t)j < have) {
+                            if constexpr (F32IN) v[j] = static_cast<const float*>(xv)[(int64_t)(b * kBlock + j) * ld + c];
+                            else v[j] = bf16_lo(x[(int64_t)(b * kBlock + j) * ld + c]);
+                        }
+                    }
                 }
                 if (center) {                                  // one centre per column: the same for the whole block
                     if constexpr (MODE == 0) {
@@ -303,6 +318,10 @@ __global__ __launch_bounds__(256) void quant_codes_col_kernel(
                         const float cen = bf16_lo(static_cast<const uint16_t*>(center)[c]);
 #pragma unroll
                         for (int j = 0; j < kBlock; ++j) v[j] = rb(v[j] - cen);
+                    }
+                    if (have < (uint32_t)kBlock) {
+#pragma unroll
+                        for (int j = 0; j < kBlock; ++j) v[j] = (uint32_t)j < have ? v[j] : 0.0f;
                     }
                 }
                 if (SR && noise) {
@@ -363,7 +382,7 @@ template <int MODE, bool WIDE = false>
 __global__ __launch_bounds__(256) void quant_codes_both_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, uint64_t seed, uint64_t offset_row, uint64_t offset_col,
     uint2* __restrict__ codes_row, void* __restrict__ amax_row_v, uint2* __restrict__ codes_col, void* __restrict__ amax_col_v,
-    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total)
+    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, uint32_t valid)
 {
     static_assert(!WIDE || MODE == 0, "binary32 values imply binary32 arithmetic");
     using amax_t = typename std::conditional<WIDE, float, uint16_t>::type;
@@ -406,6 +425,7 @@ __global__ __launch_bounds__(256) void quant_codes_both_kernel(
 #pragma unroll
             for (int i = 0; i < NQ; ++i) {
                 const int64_t at = (int64_t)(b * kBlock + i * RPI + lrow) * ld + col;
+                if (b * kBlock + i * RPI + lrow >= valid) continue;        // padding rows (zero), as quant_codes_col_kernel
                 q[i] = WIDE ? *reinterpret_cast<const uint4*>(static_cast<const float*>(xv) + at)
                             : *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(xv) + at);
             }
@@ -1052,7 +1072,7 @@ static void launch_contig(const void* x, void* codes, const Workspace& ws, uint3
 template <int MODE, bool SR, bool COL, bool WIDE = false, bool HAD = false>
 static int launch_quant(const void* x, int64_t rows, int64_t cols, int64_t ld, const void* noise, uint64_t seed,
                         uint64_t offset, void* codes, void* scales, float* unit, const Workspace& ws, hipStream_t st,
-                        int in_f32 = 0, const void* center = nullptr, uint32_t sign_mask = 0, void* decode = nullptr)
+                        int in_f32 = 0, const void* center = nullptr, uint32_t sign_mask = 0, void* decode = nullptr, int64_t valid = -1)
 {
     static_assert(!HAD || !COL, "the rotation runs along the last dimension, as the row blocks do");
     const uint32_t nblocks = (uint32_t)(rows * cols / kBlock);
@@ -1067,11 +1087,11 @@ static int launch_quant(const void* x, int64_t rows, int64_t cols, int64_t ld, c
         if (WIDE && in_f32)
             hipLaunchKernelGGL((quant_codes_col_kernel<MODE, SR, WIDE, WIDE>), dim3((unsigned)g), dim3(256), 0, st, x,
                                (uint32_t)rows, (uint32_t)cols, ld, noise, seed, offset, (uint2*)codes, (void*)ws.amax, ws.gmax, tiles_c,
-                               (uint32_t)tiles, center);
+                               (uint32_t)tiles, center, (uint32_t)(valid < 0 ? rows : valid));
         else
             hipLaunchKernelGGL((quant_codes_col_kernel<MODE, SR, WIDE, false>), dim3((unsigned)g), dim3(256), 0, st, x,
                                (uint32_t)rows, (uint32_t)cols, ld, noise, seed, offset, (uint2*)codes, (void*)ws.amax, ws.gmax, tiles_c,
-                               (uint32_t)tiles, center);
+                               (uint32_t)tiles, center, (uint32_t)(valid < 0 ? rows : valid));
         return launch_scales(WIDE ? METIS_MODE_P32_F32 : MODE, ws, (uint32_t)g, scales, unit, nblocks, st);
     } else {
         if constexpr (!SR && !HAD && (WIDE ? MODE == 0 : MODE == 1)) {
@@ -1102,9 +1122,10 @@ static int launch_quant(const void* x, int64_t rows, int64_t cols, int64_t ld, c
 
 int quantize(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, bool sr, bool col, const void* noise,
              uint64_t seed, uint64_t offset, void* codes, void* scales, float* unit, void* workspace,
-             size_t workspace_bytes, hipStream_t st, const void* center, bool resident, uint32_t spin_limit, void* decode)
+             size_t workspace_bytes, hipStream_t st, const void* center, bool resident, uint32_t spin_limit, void* decode, int64_t valid)
 {
     if (rows < 0 || cols < 0 || ld < cols) return METIS_E_ARG;
+    if (valid >= 0 && (!col || valid > rows || noise)) return METIS_E_ARG;
     if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16 && mode != METIS_MODE_P32_F32) return METIS_E_ARG;
     const bool f32in = mode == METIS_MODE_P32_F32;
     if ((col ? rows : cols) % kBlock) return METIS_E_SHAPE;
@@ -1127,8 +1148,8 @@ int quantize(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, bo
                        : launch_fused<1>(x, codes, scales, unit, ws, nblocks, st, spin_limit);
         if (rc != 1) return rc;
     }
-#define METIS_Q(M, S, C) return launch_quant<M, S, C>(x, rows, cols, ld, noise, seed, offset, codes, scales, unit, ws, st, 0, center, 0u, decode)
-#define METIS_QF(S, C) return launch_quant<0, S, C, true>(x, rows, cols, ld, noise, seed, offset, codes, scales, unit, ws, st, f32in, center)
+#define METIS_Q(M, S, C) return launch_quant<M, S, C>(x, rows, cols, ld, noise, seed, offset, codes, scales, unit, ws, st, 0, center, 0u, decode, valid)
+#define METIS_QF(S, C) return launch_quant<0, S, C, true>(x, rows, cols, ld, noise, seed, offset, codes, scales, unit, ws, st, f32in, center, 0u, nullptr, valid)
     if (wide) {
         if (!sr) { if (!col) METIS_QF(false, false); else METIS_QF(false, true); }
         else { if (!col) METIS_QF(true, false); else METIS_QF(true, true); }
@@ -1197,9 +1218,9 @@ static int both_capacity()
 // ---------------------------------------------------------------------------------------------
 int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, uint64_t seed, uint64_t offset_row,
                      uint64_t offset_col, void* codes_row, void* scales_row, float* unit_row, void* codes_col, void* scales_col,
-                     float* unit_col, void* workspace, size_t bytes, hipStream_t st)
+                     float* unit_col, void* workspace, size_t bytes, hipStream_t st, int64_t valid)
 {
-    if (rows < 0 || cols < 0 || ld < cols) return METIS_E_ARG;
+    if (rows < 0 || cols < 0 || ld < cols || valid > rows) return METIS_E_ARG;
     if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16 && mode != METIS_MODE_P32_F32) return METIS_E_ARG;
     const bool f32in = mode == METIS_MODE_P32_F32;
     if (rows % kBlock || cols % kBlock) return METIS_E_SHAPE;
@@ -1224,7 +1245,7 @@ int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int 
     if (g > kMaxGroups) g = kMaxGroups;
 #define METIS_QB(M, W) hipLaunchKernelGGL((quant_codes_both_kernel<M, W>), dim3((unsigned)g), dim3(256), 0, st, x, (uint32_t)rows, \
                                           (uint32_t)cols, ld, seed, offset_row, offset_col, (uint2*)codes_row, (void*)wr.amax, (uint2*)codes_col, \
-                                          (void*)wc.amax, wr.gmax, tiles_c, (uint32_t)tiles)
+                                          (void*)wc.amax, wr.gmax, tiles_c, (uint32_t)tiles, (uint32_t)(valid < 0 ? rows : valid))
     if (f32in) METIS_QB(0, true);
     else if (mode == 0) METIS_QB(0, false);
     else METIS_QB(1, false);

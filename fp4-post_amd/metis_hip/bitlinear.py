@@ -407,36 +407,29 @@ class LinearLowbitFunction(torch.autograd.Function):
         cd = F.compute_dtype
         qg, qi = F.q_backward_outputgrad, F.q_backward_input
         me_dy = F._token_mean(dy2) if F.enable_backward_svd else None
-        # The weight gradient contracts over tokens in steps of 32.  A ragged token count is padded, not sent down
-        # another code path: rows equal to the centre (zero rows in direct mode) have a zero residual, so they change
-        # no block maximum, no tensor unit and no sum; the padded rows of grad_input are dropped at the end.
+        # The weight gradient contracts over tokens in steps of 32.  A ragged token count is padded, not sent down another
+        # code path: the column quantizers take rows beyond the tensor's own as equal to the centre (zero in direct mode),
+        # whose residual is zero, so they change no block maximum, no tensor unit and no sum.  The input gradient
+        # contracts over features and sees the tensor's own rows.
         L = dy2.shape[0]
-        pad = (-L) % 32
-        if pad:
-            def padded(v, centre):
-                if centre is None:
-                    return torch.cat((v, v.new_zeros(pad, v.shape[1])), dim=0)
-                if v.dtype != centre.dtype:
-                    v = v.to(centre.dtype)                     # the padding rows must equal the centre exactly
-                return torch.cat((v, centre.reshape(1, -1).expand(pad, -1)), dim=0)
-            dy2, x2 = padded(dy2, me_dy), padded(x2, center_x)
-            if gx_lowrank is not None:
-                gx_lowrank = (padded(gx_lowrank[0], None), gx_lowrank[1])
+        more = {}
+        if L % 32:
+            more["pad_rows"] = L + (-L) % 32
+            # the row quantizer's 16-byte loads: a gradient that starts elsewhere is copied
+            dy2 = dy2 if dy2.data_ptr() % 16 == 0 else dy2.clone()
         if me_dy is None and hasattr(qg, "pack_both"):
-            p_dy, p_dyt = qg.pack_both(dy2, arith=cd)          # one pass over dY for both products
+            p_dy, p_dyt = qg.pack_both(dy2, arith=cd, **more)  # one pass over dY for both products
         else:
-            p_dy, p_dyt = qg.pack(dy2, arith=cd, center=me_dy), None
+            p_dy, p_dyt = qg.pack(dy2, arith=cd, center=me_dy, **more), None
         if me_dy is None and gx_lowrank is None:
             gx = ops.linear_dgrad(p_dy, pw_col, out_dtype=gx_dtype)
         else:
             lt, lu = gx_lowrank if gx_lowrank is not None else (None, None)
             gx = ops.linear_fwd(p_dy, pw_col, t=lt, u=lu, bias=None if me_dy is None else ops.matvec(pw_col, me_dy),
                                 out_dtype=gx_dtype)
-        if pad:
-            gx = gx[:L]
         if p_dyt is None:
-            p_dyt = qg.pack(dy2, col=True, arith=cd, center=me_dy)
-        p_xt = qi.pack(x2, col=True, arith=cd, center=center_x)
+            p_dyt = qg.pack(dy2, col=True, arith=cd, center=me_dy, **more)
+        p_xt = qi.pack(x2, col=True, arith=cd, center=center_x, **more)
         if me_dy is None and center_x is None:
             # autograd rounds the gradient to the parameter's dtype anyway: let the GEMM epilogue do that rounding
             return gx, ops.linear_wgrad(p_dyt, p_xt, out_dtype=gw_dtype)

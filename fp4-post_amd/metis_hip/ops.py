@@ -196,7 +196,7 @@ def _as_2d_for_quant(x: torch.Tensor, mode: int) -> tuple[torch.Tensor, int]:
 def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bool = False,
              noise: torch.Tensor | None = None, seed: int = 0, offset: int = 0,
              center: torch.Tensor | None = None, resident: bool = False, spin_limit: int = 0,
-             deferred: bool = False) -> PackedNVFP4:
+             deferred: bool = False, pad_rows: int | None = None) -> PackedNVFP4:
     """NVFP4-quantize x (flattened to [R, C]).
 
     col=False: blocks of 16 along C -> PackedNVFP4 of shape (R, C).
@@ -211,9 +211,13 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
     deferred : round-to-nearest rows of a bf16 tensor: only the first of the two launches now (codes, parked block
                maxima); `scales` and `unit` of the result appear on first access, or never if the only consumer is
                expand_tiled, which forms the bytes itself.  Same bits either way.
+    pad_rows : col=True: pack as if x had pad_rows rows, those beyond its own with a zero residual (equal to the centre,
+               zero without one); no copy of x is made.  Only without caller noise.
     """
     x2, kmode = _as_2d_for_quant(x, mode)
     rows, cols = x2.shape
+    if pad_rows is not None and pad_rows != rows:
+        return _quantize_col_padded(x2, kmode, mode, pad_rows, col, sr, noise, seed, offset, center)
     blocked = rows if col else cols
     if blocked % BLOCK:
         raise ValueError(f"NVFP4 block shape (1, 16) does not divide tensor shape {tuple(x.shape)}")
@@ -276,6 +280,29 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
     return PackedNVFP4(codes, scales, unit, prow, pcol, mode)
 
 
+def _quantize_col_padded(x2, kmode, mode, pad_rows, col, sr, noise, seed, offset, center) -> PackedNVFP4:
+    rows, cols = x2.shape
+    if not col or noise is not None or pad_rows < rows:
+        raise ValueError("pad_rows: column blocks of at least as many rows as the tensor has, without caller noise")
+    if pad_rows % BLOCK:
+        raise ValueError(f"NVFP4 block shape (1, 16) does not divide tensor shape {(cols, pad_rows)}")
+    dev = x2.device
+    cen = None
+    if center is not None:
+        cen = center.reshape(-1).to(device=dev, dtype=torch.bfloat16 if mode == MODE_PB16 else torch.float32).contiguous()
+        if cen.numel() != cols:
+            raise ValueError(f"center must have one value per column ({cols}), got {cen.numel()}")
+    codes = torch.empty(cols, pad_rows // 2, dtype=torch.uint8, device=dev)
+    scales = torch.empty(cols, pad_rows // BLOCK, dtype=torch.uint8, device=dev)
+    unit = torch.empty(1, dtype=torch.float32, device=dev)
+    ws = _workspace(pad_rows, cols, dev)
+    rc = load().metis_nvfp4_quant_col_padded(x2.data_ptr(), rows, pad_rows, cols, x2.stride(0), kmode, None if cen is None else cen.data_ptr(),
+                                             int(sr), seed & (2 ** 64 - 1), offset, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(),
+                                             ws.data_ptr(), ws.numel(), _stream())
+    check(rc, "metis_nvfp4_quant_col_padded", (rows, cols))
+    return PackedNVFP4(codes, scales, unit, cols, pad_rows, mode)
+
+
 def quantize_dequantize(x: torch.Tensor, mode: int = MODE_P32) -> tuple[PackedNVFP4, torch.Tensor]:
     """(quantize(x, mode), its dequantized bf16 tensor) of a bf16 tensor with round to nearest, from one call of two
     launches: the second forms scale bytes and dequantized values in one pass over the codes.  Same bytes as
@@ -335,12 +362,16 @@ def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tenso
 
 
 def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, offset_row: int = 0,
-                     offset_col: int = 0) -> tuple[PackedNVFP4, PackedNVFP4]:
+                     offset_col: int = 0, pad_rows: int | None = None) -> tuple[PackedNVFP4, PackedNVFP4]:
     """(quantize(x, sr=True, offset=offset_row), quantize(x, col=True, sr=True, offset=offset_col)) from ONE pass over x:
     the two packings of an output gradient that the input-gradient and weight-gradient products contract.  Same
-    bytes as the two calls.  Both dimensions of x flattened to [R, C] have to be multiples of 16."""
+    bytes as the two calls.  Both dimensions of x flattened to [R, C] have to be multiples of 16; with pad_rows, that
+    and C: the column packing is that of x filled up with zero rows to pad_rows, the row packing that of x."""
     x2, kmode = _as_2d_for_quant(x, mode)
-    rows, cols = x2.shape
+    have, cols = x2.shape
+    rows = have if pad_rows is None else pad_rows
+    if rows < have:
+        raise ValueError("pad_rows: at least as many rows as the tensor has")
     if rows % BLOCK or cols % BLOCK:
         raise ValueError(f"NVFP4 block shape (1, 16) does not divide tensor shape {tuple(x.shape)} both ways")
     dev = x2.device
@@ -358,11 +389,11 @@ def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, of
         _workspaces[key] = ws
     (cr, sr_, ur), (cc, sc, uc) = packs
     if rows * cols:
-        rc = L.metis_nvfp4_quant_sr_both(x2.data_ptr(), rows, cols, x2.stride(0), kmode, seed & (2 ** 64 - 1), offset_row, offset_col,
-                                         cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(), uc.data_ptr(),
-                                         ws.data_ptr(), ws.numel(), _stream())
-        check(rc, "metis_nvfp4_quant_sr_both", x.shape)
-    return PackedNVFP4(cr, sr_, ur, rows, cols, mode), PackedNVFP4(cc, sc, uc, cols, rows, mode)
+        rc = L.metis_nvfp4_quant_sr_both_padded(x2.data_ptr(), have, rows, cols, x2.stride(0), kmode, seed & (2 ** 64 - 1), offset_row,
+                                                offset_col, cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(),
+                                                uc.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
+        check(rc, "metis_nvfp4_quant_sr_both_padded", x.shape)
+    return PackedNVFP4(cr[:have], sr_[:have], ur, have, cols, mode), PackedNVFP4(cc, sc, uc, cols, rows, mode)
 
 
 def dequantize(p: PackedNVFP4, dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:

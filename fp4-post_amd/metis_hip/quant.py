@@ -89,13 +89,17 @@ class _NVFP4Base(BlockQuantFunc):
     @torch.no_grad()
     def pack(cls, x: torch.Tensor, col: bool = False, noise: torch.Tensor | None = None,
              arith: torch.dtype | None = None, center: torch.Tensor | None = None, rht: int | None = None,
-             deferred: bool = False) -> ops.PackedNVFP4:
+             deferred: bool = False, pad_rows: int | None = None) -> ops.PackedNVFP4:
         """Packed NVFP4 (codes, E4M3 scale bytes, unit) of x in the arithmetic of x's dtype, or of `arith`
         when given: a bf16 tensor packed with arith=float32 gives what x.float() would, without the copy.
         center: per-column vector subtracted first (mean mode): the packed tensor is that of x - center.
         rht: sign mask of the NV recipe's rotation: the packed tensor is that of the rotated x (see ops.quantize_rht).
-        deferred: round-to-nearest rows only: one launch now, the scale bytes when (and if) somebody reads them (ops.quantize)."""
+        deferred: round-to-nearest rows only: one launch now, the scale bytes when (and if) somebody reads them (ops.quantize).
+        pad_rows: x stands for a tensor of pad_rows rows whose rows beyond x's own have a zero residual: col=True packs that
+        tensor, row blocks are those of x; either way the random stream advances as for the larger tensor."""
         _need_gpu(x)
+        drawn = x.numel() if pad_rows is None else pad_rows * x.shape[-1]
+        more = {"pad_rows": pad_rows} if (col and pad_rows is not None) else {}
         if not col:
             cls._check(x)
         mode = _mode_of(x) if arith is None else (MODE_P32 if arith == torch.float32 else MODE_PB16)
@@ -108,23 +112,27 @@ class _NVFP4Base(BlockQuantFunc):
             return ops.quantize_rht(x, mode, rht)
         if cls.stochastic:
             return ops.quantize(x, mode, col=col, sr=True, noise=noise, seed=_NVFP4Base.sr_seed,
-                                offset=cls._next_offset(x.numel()) if noise is None else 0, center=center)
-        return ops.quantize(x, mode, col=col, center=center, deferred=deferred)
+                                offset=cls._next_offset(drawn) if noise is None else 0, center=center, **more)
+        return ops.quantize(x, mode, col=col, center=center, deferred=deferred, **more)
 
     @classmethod
     @torch.no_grad()
-    def pack_both(cls, x: torch.Tensor, arith: torch.dtype | None = None) -> tuple[ops.PackedNVFP4, ops.PackedNVFP4]:
+    def pack_both(cls, x: torch.Tensor, arith: torch.dtype | None = None,
+                  pad_rows: int | None = None) -> tuple[ops.PackedNVFP4, ops.PackedNVFP4]:
         """(pack(x), pack(x, col=True)): the same two tensors, and under stochastic rounding the same draws in the same
-        order, from one pass over x where the kernels have one (stochastic rounding, both dimensions multiples of 16)."""
+        order, from one pass over x where the kernels have one (stochastic rounding, both dimensions multiples of 16).
+        pad_rows: as in pack."""
         _need_gpu(x)
         cls._check(x)
         rows = x.numel() // x.shape[-1] if x.numel() else 0
-        if cls.stochastic and rows and rows % 16 == 0 and x.dtype in (torch.bfloat16, torch.float32):
+        more = {} if pad_rows is None else {"pad_rows": pad_rows}
+        drawn = x.numel() if pad_rows is None else pad_rows * x.shape[-1]
+        if cls.stochastic and rows and (pad_rows or rows) % 16 == 0 and x.dtype in (torch.bfloat16, torch.float32):
             mode = _mode_of(x) if arith is None else (MODE_P32 if arith == torch.float32 else MODE_PB16)
-            first = cls._next_offset(x.numel())
-            second = cls._next_offset(x.numel())
-            return ops.quantize_both_sr(x, mode, seed=_NVFP4Base.sr_seed, offset_row=first, offset_col=second)
-        return cls.pack(x, arith=arith), cls.pack(x, col=True, arith=arith)
+            first = cls._next_offset(drawn)
+            second = cls._next_offset(drawn)
+            return ops.quantize_both_sr(x, mode, seed=_NVFP4Base.sr_seed, offset_row=first, offset_col=second, **more)
+        return cls.pack(x, arith=arith, **more), cls.pack(x, col=True, arith=arith, **more)
 
     @classmethod
     @torch.no_grad()

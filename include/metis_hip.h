@@ -189,6 +189,25 @@ int metis_nvfp4_quant_sr_both(const void *x, int64_t rows, int64_t cols, int64_t
                               size_t workspace_bytes, void *stream);
 
 /*
+ * A ragged token count: the weight gradient contracts over tokens in steps of 32, so its operands are packed as if x had
+ * padded_rows rows, those from `rows` on equal to the centre (zero without one), i.e. with a zero residual.  x itself has
+ * `rows` rows; nothing beyond them is read.  The results are those of the calls on a tensor copied and filled up that way.
+ *   metis_nvfp4_quant_col_padded      metis_nvfp4_quant_col / _sr_col / _centered(col = 1), the library's own random stream;
+ *                                     center may be NULL; padded_rows % 16 == 0
+ *   metis_nvfp4_quant_sr_both_padded  metis_nvfp4_quant_sr_both; the row packing is written for padded_rows rows, too
+ *   rows <= padded_rows, else METIS_E_ARG; workspace as for padded_rows rows
+ */
+int metis_nvfp4_quant_col_padded(const void *x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld,
+                                 int mode, const void *center, int sr, uint64_t seed, uint64_t offset,
+                                 void *codes, void *scales, float *unit, void *workspace,
+                                 size_t workspace_bytes, void *stream);
+int metis_nvfp4_quant_sr_both_padded(const void *x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld,
+                                     int mode, uint64_t seed, uint64_t offset_row, uint64_t offset_col,
+                                     void *codes_row, void *scales_row, float *unit_row, void *codes_col,
+                                     void *scales_col, float *unit_col, void *workspace,
+                                     size_t workspace_bytes, void *stream);
+
+/*
  * The reference's three-call form on dequantized tensors of dtype D (float32 in METIS_MODE_P32, bf16 in
  * METIS_MODE_PB16), for callers that use the quantizer classes directly.  All tensors contiguous [rows, cols].
  *   metis_nvfp4_get_scalar : Cast2NVFp4e2m1Block[NOSR].get_scalar (src/Metis/Metis/quant.py:435-455)

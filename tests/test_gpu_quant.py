@@ -656,3 +656,35 @@ def test_both_packings_argument_checks(ops):
     assert call(64, 64, 64, mode=7) == _lib.E_ARG
     assert call(64, 64, 64, wsn=ws.numel() // 2) == _lib.E_WORKSPACE  # one workspace is not enough for two sets of maxima
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows,pad,cols", [(1, 32, 16), (15, 32, 80), (16, 32, 64), (17, 32, 48), (33, 64, 144), (250, 256, 64), (257, 288, 208), (701, 704, 1536)])
+def test_column_packing_of_a_ragged_row_count_equals_packing_a_filled_up_copy(rows, pad, cols):
+    """pad_rows: the rows beyond the tensor's own count as equal to the centre (zero without one) and are never read -- the
+    same bytes as packing a copy with such rows appended, for every arithmetic, both roundings, bf16 and binary32 tensors,
+    with and without a centre; and both packings of an output gradient likewise."""
+    from metis_hip import ops
+    g = torch.Generator().manual_seed(rows)
+    for dtype, mode in ((torch.bfloat16, 0), (torch.bfloat16, 1), (torch.float32, 0)):
+        x = torch.randn(rows, cols, generator=g).to(dtype).cuda()
+        for center in (None, torch.randn(cols, generator=g).cuda().to(torch.bfloat16 if mode else torch.float32)):
+            fill = x.new_zeros(pad - rows, cols) if center is None else center.reshape(1, -1).expand(pad - rows, -1)
+            if center is not None and mode == 0:
+                full = torch.cat((x.float(), fill), 0)
+            else:
+                full = torch.cat((x, fill.to(x.dtype)), 0)
+            for sr in (False, True):
+                kw = dict(col=True, sr=sr, seed=11, offset=5, center=center)
+                want, got = ops.quantize(full, mode, **kw), ops.quantize(x, mode, pad_rows=pad, **kw)
+                assert (got.rows, got.cols) == (cols, pad)
+                assert torch.equal(got.codes, want.codes) and torch.equal(got.scales, want.scales) and torch.equal(got.unit, want.unit)
+        full = torch.cat((x, x.new_zeros(pad - rows, cols)), 0)
+        wr, wc = ops.quantize_both_sr(full, mode, seed=3, offset_row=7, offset_col=9)
+        gr, gc = ops.quantize_both_sr(x, mode, seed=3, offset_row=7, offset_col=9, pad_rows=pad)
+        assert (gr.rows, gr.cols) == (rows, cols)
+        assert torch.equal(gr.codes, wr.codes[:rows]) and torch.equal(gr.scales, wr.scales[:rows]) and torch.equal(gr.unit, wr.unit)
+        assert torch.equal(gc.codes, wc.codes) and torch.equal(gc.scales, wc.scales) and torch.equal(gc.unit, wc.unit)
+    with pytest.raises(ValueError):
+        ops.quantize(x, 0, pad_rows=pad)                          # row blocks take the tensor as it is
+    with pytest.raises(ValueError):
+        ops.quantize(x, 0, col=True, pad_rows=rows + 16 - rows % 16 + 3)
