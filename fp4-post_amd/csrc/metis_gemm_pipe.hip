@@ -30,7 +30,10 @@ __host__ __device__ __forceinline__ int xt_swz(int q) { return ((q >> 2) & 1) | 
 // ---------------------------------------------------------------------------------------------
 // packed NVFP4 -> tiled 16-bit operands.  One wave per tile: lane l writes slot l (row l / 4).  A wave walks
 // eight consecutive k tiles of one tile row, so the 128-byte lines of codes it touches are used whole.
-// HBM-bound: 0.5625 B read, 2 B written per element.
+// HBM-bound: 0.5625 B read, 2 B written per element.  The unit's eight words of codes and eight scales are requested
+// together: one at a time, between the stores, the lines of codes (16 bytes of each of 16 rows per load) were pushed out of L2
+// by the output before the next visit.  16384 x 18944 from a deferred activation 249 -> 209 us, 16384 x 3584 36.9 -> 32.6,
+// the 18944 x 3584 weight 48.0 -> 41.3, 8192 x 4096 17.0 -> 16.3.  Streaming stores on top change nothing (214, 31.7).
 //   PB16 = 0: binary16, e2m1(code) * e4m3(scale) * 2^-8, exact (the tensor unit is applied by the GEMM)
 //   PB16 = 1: bf16, the reference's dequantized value with every op rounded to bf16
 //             (src/Metis/Metis/quant.py:23-24, 32-35: bf16(bf16(e4m3 * unit) * v / 2)), unit included
@@ -74,15 +77,29 @@ __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restri
         const int rb_ = (int)(un / kgroups), kg = (int)(un - (int64_t)rb_ * kgroups);
         const int row = rb_ * 16 + q;
         const bool live = row < rows;
-        const int kend = min(kt, kg * 8 + 8);
-        for (int kb = kg * 8; kb < kend; ++kb) {
+        const int kb0 = kg * 8, kend = min(kt, kb0 + 8);
+        uint32_t cw[8] = {}, sw[8] = {};                         // every tile's codes and scales are requested before the first is expanded
+        if (live) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (kb0 + i < kend) {
+                    const int k8 = (kb0 + i) * 4 + chunk;        // index of the 8-element chunk inside the row
+                    cw[i] = codes[(int64_t)row * (K / 8) + k8];
+                    if constexpr (DEF != 0) sw[i] = maxima[(int64_t)row * (K / 16) + (k8 >> 1)];
+                    else sw[i] = scales[(int64_t)row * (K / 16) + (k8 >> 1)];
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int kb = kb0 + i;
+            if (kb >= kend) break;                               // the same for the whole wave
             uint4 v = make_uint4(0u, 0u, 0u, 0u);
             if (live) {                                          // lane pairs (l, l ^ 1) share their row: both live or neither
-                const int k8 = kb * 4 + chunk;                   // index of the 8-element chunk inside the row
-                const uint32_t c = codes[(int64_t)row * (K / 8) + k8];
+                const uint32_t c = cw[i];
                 uint32_t sb;
-                if constexpr (DEF != 0) sb = scale_byte_of<QMODE>(maxima[(int64_t)row * (K / 16) + (k8 >> 1)], unit);
-                else sb = scales[(int64_t)row * (K / 16) + (k8 >> 1)];
+                if constexpr (DEF != 0) sb = scale_byte_of<QMODE>((uint16_t)sw[i], unit);
+                else sb = sw[i];
                 if constexpr (RHT != 0) {
                     const float dq = PB16 ? rb(e4m3_value(sb) * unit) : e4m3_value(sb) * 0.00390625f;
                     const float2_t p[4] = {__builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 1),
@@ -132,7 +149,7 @@ __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restri
                     v.z = rb_pair(p2[0] * dq, p2[1] * dq);
                     v.w = rb_pair(p3[0] * dq, p3[1] * dq);
                     if (center) {
-                        const uint4 cw = *reinterpret_cast<const uint4*>(center + k8 * 8);
+                        const uint4 cw = *reinterpret_cast<const uint4*>(center + (kb * 4 + chunk) * 8);
                         v.x = rb_pair(bf16_lo(cw.x) + bf16_lo(v.x), bf16_hi(cw.x) + bf16_hi(v.x));
                         v.y = rb_pair(bf16_lo(cw.y) + bf16_lo(v.y), bf16_hi(cw.y) + bf16_hi(v.y));
                         v.z = rb_pair(bf16_lo(cw.z) + bf16_lo(v.z), bf16_hi(cw.z) + bf16_hi(v.z));
