@@ -7,10 +7,14 @@
 //   lowrank_tn:  out[C, R] = sum_l a[l, C] . b[l, R]                     the two products of the backward pass that
 //                contract over tokens: dY^T . (xv * s) -> grad of U, x^T . g_xv -> grad of V (written transposed)
 //
-// lowrank_nt: a workgroup owns 32 rows of x and walks K in steps of 256.  The x rows (32 x 512 B) and the R rows of v
-// (R x 512 B, from L2 after the first workgroup touched them) are fetched two steps ahead into registers, 16 bytes
-// per thread and load, and staged in LDS with 528-byte rows; wave w multiplies the w-th quarter (64 k) of the step
-// for all R columns, and the four partial sums meet in LDS at the end.
+// lowrank_nt: a workgroup owns 32 or 64 rows of x and walks K in stages of 64 or 128.  The x rows and the R rows of v of a
+// stage (v from L2 after the first workgroup touched it) go straight from memory to LDS, into a ring of two to four stages,
+// so that no wave waits for the loads it issued last; the waves share a stage's k, 32 each, and their partial sums meet in
+// LDS at the end.  (Staged through registers two steps ahead, with two barriers per step and the encoder between them, the
+// loads in flight per compute unit were what its registers held: 16384 x 3584, R = 64 34.8 -> 27.7 us; with the quantizer
+// 61.7 -> 47.5, 16384 x 18944 309 -> 230; 2103 x 18944 27 -> 24.  The read of x alone at 5 TB/s: 23.5; with codes and
+// maxima written 30.8 and 163.  Bound by HBM, with the quantizer by the encoder's vector work at two waves per SIMD; deeper
+// rings change nothing.)
 //
 // lowrank_tn: the contraction runs down the rows of both operands, so each has to be turned: a workgroup owns 64
 // columns of a and one slice of the tokens; a step of 64 tokens is loaded row by row (coalesced) and staged in LDS as it
@@ -20,232 +24,209 @@
 #include "metis_device.h"
 #include "metis_host.h"
 #include "nvfp4_encode.h"
+#include "gemm_common.h"
 
 namespace metis {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
+// A form of the kernel: ROWS rows of x per workgroup, KS k per stage, NS stages in the ring; one thread per block of 16 of x.
+template <int RT, int ROWS, int KS, int NS> struct NtForm {
+    static constexpr int kThreads = ROWS * KS / 16, kWaves = kThreads / 64;
+    static constexpr int kRowBytes = KS * 2, kRowsPerPiece = 1024 / kRowBytes, kChunks = kRowBytes / 16;
+    static constexpr int kStage = (ROWS + RT * 32) * kRowBytes;               // bytes of a stage: x rows, then v rows
+    static constexpr int kLoads = kStage / 1024 / kWaves, kXLoads = ROWS / kRowsPerPiece / kWaves;   // 1 KiB loads per wave and stage; those of x
+    static constexpr int kRowTiles = ROWS / 32, kParts = kWaves / kRowTiles;  // the waves of a row tile share the stage's k, 32 each
+    static constexpr int kLds = NS * kStage;
+    static_assert((KS == 64 || KS == 128) && kParts * 32 == KS && kStage % (1024 * kWaves) == 0 && kXLoads >= 1, "every wave loads whole pieces and multiplies two steps of 16");
+    static_assert(((kParts - 1) * kRowTiles * RT * 4096 + 64) <= kLds, "the partial sums fit the ring");
+};
+// Leaves at most VM of the wave's vector memory operations in flight.  Assembly with a memory clobber: no load or store of
+// the loop may move across it, the counts at its uses rely on that.
+template <int VM> __device__ __forceinline__ void nt_wait()
+{
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(VM) : "memory");
+}
 
-constexpr int NT_STEP = 256;                     // k per step of lowrank_nt
-constexpr int NT_STRIDE = NT_STEP + 8;           // halves per staged row: 528 bytes, conflict-free 16-byte reads
-
-// K slices: with 32 rows per workgroup a tensor of a few thousand rows gives one workgroup per compute unit, too few
-// bytes in flight to cover the memory latency.  gridDim.y workgroups then share a row tile, each walking its own range
-// of steps; their binary32 partial sums go to a caller workspace ([slice][row][R]) and lowrank_nt_finish_kernel adds
-// them in slice order.  One slice: the result is written directly.
+// K slices: a tensor of a few thousand rows has too few row tiles to keep every compute unit's loads in flight.  gridDim.y
+// workgroups then share a row tile, each walking its own range of stages; their binary32 partial sums go to a caller
+// workspace ([slice][row][R]) and lowrank_nt_finish_kernel adds them in slice order.  One slice: written directly.
 //
-// QMODE >= 0: the same pass also quantizes x (round to nearest, rows; METIS_MODE_P32 or _PB16 arithmetic).  The workgroup
-// then has four more waves that take no part in the product: after the barrier that publishes a staged step they read
-// the x rows back from LDS, two blocks of 16 per thread, and encode them while the first four waves wait for the next
-// loads -- E2M1 codes, the block maximum parked as bf16, one partial tensor maximum per workgroup: what
-// quant_codes_contig_kernel leaves for a consumer that forms the scale bytes itself.  (Encoding in the loading waves
-// themselves put the encoder's ~250 vector instructions per step between their wait and their barrier.)
-// EW = false: the loading waves encode the block they fetched themselves, one step later (kept in px), after the next
-// loads are issued: 256 threads and fewer registers per workgroup, so two workgroups fit a compute unit -- the better
-// form when there are more row tiles than compute units (16384 rows: 41 against 46 us; 8192 rows: 38 against 30 us).
-template <int RT, int QMODE = -1, bool EW = false>  // R / 32 column tiles: 1, 2 or 4
-__global__ __launch_bounds__((QMODE >= 0 && EW) ? 512 : 256) void lowrank_nt_kernel(
+// QMODE >= 0: the same pass also quantizes x (round to nearest, rows; METIS_MODE_P32 or _PB16 arithmetic): a stage holds one
+// block of 16 per thread, read back from LDS -- E2M1 codes, the block maximum parked as bf16, one partial tensor maximum per
+// workgroup: what quant_codes_contig_kernel leaves for a consumer that forms the scale bytes itself.
+// CUT: K % KS == 64.
+template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
+__global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v, const uint16_t* __restrict__ s,
     uint16_t* __restrict__ xv, uint16_t* __restrict__ t, int M, int K, float* __restrict__ part, uint2* __restrict__ codes,
     uint16_t* __restrict__ q_amax, uint32_t* __restrict__ q_gmax, uint32_t fill_to, int rotate)
 {
-    constexpr int R = RT * 32;
-    constexpr int TILE_BYTES = (32 + R) * NT_STRIDE * 2;        // one staged step: x rows, then v rows
-    constexpr int RED_BYTES = 4 * RT * 16 * 64 * 4;
-    constexpr int LDS_BYTES = TILE_BYTES > RED_BYTES ? TILE_BYTES : RED_BYTES;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];     // the staged step, then the four partial sums
-    uint16_t* tile = reinterpret_cast<uint16_t*>(lds);
-    float* red = reinterpret_cast<float*>(lds);                 // [wave][j][e][lane]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.x * 32;
-    const int steps_all = (K + NT_STEP - 1) / NT_STEP;          // K % 64 == 0; a short last step is padded with zeros
+    using F = NtForm<RT, ROWS, KS, NS>;
+    constexpr int R = RT * 32, STAGE = F::kStage, LPW = F::kLoads, XL = F::kXLoads, RPP = F::kRowsPerPiece, RB = F::kRowBytes;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];     // the ring, then the waves' partial sums
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m0 = blockIdx.x * ROWS;
+    // CUT (K % 64 == 0, KS = 128): the last stage has only its first half.  The lanes of the other half then fetch the
+    // first again, its waves do not multiply, its threads encode the first half's blocks once more (the same bytes).
+    // A template parameter: the branch would keep product and encoder from being interleaved (8192 x 4096: 27.4 -> 35.6 us).
+    const int steps_all = (K + KS - 1) / KS;
     const int per = (steps_all + (int)gridDim.y - 1) / (int)gridDim.y;
     const int first = (int)blockIdx.y * per, steps = max(0, min(steps_all, first + per) - first);
-    __shared__ float smax[4];
-    // Every row tile starts at a different step of its K range and wraps around: at any moment the workgroups then read
-    // different column stripes of x instead of the same one.  With rows a multiple of 4 KiB long, 512-byte pieces at the
-    // same offset of every row can fall on the same few memory channels (flushed caches, 8192 x 14336: 146 -> 104 us on one
-    // machine, 126 -> 107 us on another; 8192 x 4096: 39 -> 31 us on the first, no change on the second; row lengths like
-    // 7168 or 17920 bytes are indifferent).  The binary32 sums of a tile are therefore added in an order that depends on
-    // the tile, the same for every call and for both forms of the kernel.
+    // Every row tile starts at a different stage of its K range and wraps around: at any moment the workgroups then read
+    // different column stripes of x instead of the same one.  With rows a multiple of 4 KiB long, pieces at the same offset
+    // of every row can fall on the same few memory channels.  The binary32 sums of a tile are therefore added in an order
+    // that depends on the tile, the same for every call and with or without the quantizer.  (An offset of 13 stages per tile:
+    // 8192 x 4096 from flushed caches 40 us, 45 with 5, 41-46 without; other row lengths within 2 %.)
     const int rot = (rotate && steps > 0) ? (int)((blockIdx.x * (unsigned)rotate) % (unsigned)steps) : 0;
-    auto kof = [&](int st) { int q = st + rot; if (q >= steps) q -= steps; return (first + q) * NT_STEP; };
-    if constexpr (QMODE >= 0 && EW) {
-        if (tid >= 256) {                                       // the encoding waves: same barriers as the others, nothing else shared
-            const int et = tid - 256;
-            float gmax = 0.0f;
-            for (int st = 0; st < steps; ++st) {
-                __syncthreads();                                // the step is staged
-                uint4 b[2][2];
+    auto kof = [&](int st) { int q = st + rot; if (q >= steps) q -= steps; return (first + q) * KS; };
+
+    // ---- loads go straight to LDS: piece p = j * waves + wave of a stage is 1 KiB, whole rows of x | v.  The 16-byte chunk c
+    // of row q lies at position c ^ swz(q) of the row, so that the fragment reads (32 rows at the same chunk) spread over all
+    // banks; the lanes of a piece fetch their chunks in that order.
+    // Written as assembly with waits placed by hand: the compiler would order every LDS read behind all loads in flight.
+    auto swz = [](int row) { return KS == 64 ? (row >> 1) & 7 : row & 15; };
+    const uint16_t* src[LPW];                                   // (64-bit: a stage spans up to 256 rows of any length)
+    uint32_t upper = 0u;                                        // bit j: the lane's chunk of load j lies in the second 64 k
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int id = i * 256 + et, row = id >> 4, blk = id & 15;
-                    b[i][0] = *reinterpret_cast<const uint4*>(tile + row * NT_STRIDE + blk * 16);
-                    b[i][1] = *reinterpret_cast<const uint4*>(tile + row * NT_STRIDE + blk * 16 + 8);
-                }
-                __syncthreads();                                // the tile may be overwritten: the blocks are in registers
-                const int k0 = kof(st);
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int id = i * 256 + et, row = id >> 4, k = k0 + (id & 15) * 16;
-                    if (m0 + row < M && k < K) {
-                        float val[kBlock];
-                        const float none[kBlock] = {};
-                        unpack16(b[i][0], b[i][1], val);
-                        const float am = block_amax(val);
-                        gmax = fmaxf(gmax, am);
-                        const int64_t ib = (int64_t)(m0 + row) * (K / kBlock) + k / kBlock;
-                        q_amax[ib] = (uint16_t)(__float_as_uint(am) >> 16);
-                        codes[ib] = encode_block<QMODE < 0 ? 0 : QMODE, false>(val, block_scalar<QMODE < 0 ? 0 : QMODE>(am), none);
-                    }
-                }
-            }
-            // one partial maximum per workgroup, indexed over the whole grid; unused entries cleared for the folding reader
-            const float wm = wave_max(gmax);
-            if (lane == 0) smax[wave - 4] = wm;
-            __syncthreads();                                    // the barrier the other waves pass after parking their sums
-            const uint32_t gid = blockIdx.y * gridDim.x + blockIdx.x, gsize = gridDim.x * gridDim.y;
-            if (et == 0) q_gmax[gid] = __float_as_uint(fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])));
-            for (uint32_t j = gsize + gid * 256u + et; j < fill_to; j += gsize * 256u) q_gmax[j] = 0u;
-            return;
-        }
+    for (int j = 0; j < LPW; ++j) {
+        const int row = ((j < XL ? j : j - XL) * F::kWaves + wave) * RPP + lane / F::kChunks;
+        const int chunk = (lane % F::kChunks) ^ swz(row);
+        src[j] = (j < XL ? x + (int64_t)min(m0 + row, M - 1) * ldx : v + (int64_t)row * K) + chunk * 8;
+        upper |= (uint32_t)(chunk >> 3) << j;
     }
-    // staging: a thread fetches two blocks of 16 of x per step (32 contiguous bytes each; 16 threads cover the 512
-    // bytes of a row) and 4 RT 16-byte chunks of v (a wave covers two rows x 512 contiguous bytes per load).
-    // It keeps two whole steps in registers while the one before them is multiplied: that is what keeps bytes in flight.
-    uint4 rx[2][4], rv[2][RT * 4];
-    auto fetch = [&](uint4 (&qx)[4], uint4 (&qv)[RT * 4], int k0) {
+    auto issue = [&](int slot, int st) {
+        const int k0 = kof(st);
+        const bool cut = CUT && k0 + KS > K;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int id = i * 256 + tid, row = id >> 4, k = k0 + (id & 15) * 16;
-            const uint4* src = reinterpret_cast<const uint4*>(x + (int64_t)min(m0 + row, M - 1) * ldx + k);
-            qx[2 * i] = k < K ? src[0] : make_uint4(0u, 0u, 0u, 0u);
-            qx[2 * i + 1] = k < K ? src[1] : make_uint4(0u, 0u, 0u, 0u);
-        }
-#pragma unroll
-        for (int i = 0; i < RT * 4; ++i) {
-            const int id = i * 256 + tid, row = id >> 5, k = k0 + (id & 31) * 8;
-            qv[i] = k < K ? *reinterpret_cast<const uint4*>(v + (int64_t)row * K + k) : make_uint4(0u, 0u, 0u, 0u);
+        for (int j = 0; j < LPW; ++j) {
+            const uint32_t dst = (uint32_t)(slot * STAGE + (j * F::kWaves + wave) * 1024);
+            const uint16_t* g = src[j] + k0;
+            if (cut) g -= ((upper >> j) & 1u) * 64u;
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(dst) : "memory");
         }
     };
-    float gmax = 0.0f;
-    uint4 px[(QMODE >= 0 && !EW) ? 4 : 1];
-    auto stage = [&](const uint4 (&qx)[4], const uint4 (&qv)[RT * 4]) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int id = i * 256 + tid, row = id >> 4, blk = id & 15;
-            *reinterpret_cast<uint4*>(tile + row * NT_STRIDE + blk * 16) = qx[2 * i];
-            *reinterpret_cast<uint4*>(tile + row * NT_STRIDE + blk * 16 + 8) = qx[2 * i + 1];
-        }
-        if constexpr (QMODE >= 0 && !EW) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) px[i] = qx[i];
-        }
-#pragma unroll
-        for (int i = 0; i < RT * 4; ++i) {
-            const int id = i * 256 + tid;
-            *reinterpret_cast<uint4*>(tile + (32 + (id >> 5)) * NT_STRIDE + (id & 31) * 8) = qv[i];
-        }
-    };
-    auto encode = [&](int k0) {
-        if constexpr (QMODE >= 0 && !EW) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int id = i * 256 + tid, row = id >> 4, k = k0 + (id & 15) * 16;
-                if (m0 + row < M && k < K) {
-                    float val[kBlock];
-                    const float none[kBlock] = {};
-                    unpack16(px[2 * i], px[2 * i + 1], val);
-                    const float am = block_amax(val);
-                    gmax = fmaxf(gmax, am);
-                    const int64_t ib = (int64_t)(m0 + row) * (K / kBlock) + k / kBlock;
-                    q_amax[ib] = (uint16_t)(__float_as_uint(am) >> 16);
-                    codes[ib] = encode_block<QMODE < 0 ? 0 : QMODE, false>(val, block_scalar<QMODE < 0 ? 0 : QMODE>(am), none);
-                }
-            }
-        }
-    };
+
     float16_t acc[RT];
 #pragma unroll
     for (int j = 0; j < RT; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
-
-    // wave w multiplies the quarter [64 w, 64 w + 64) of every step
-    const int foff = (lane & 31) * NT_STRIDE + wave * 64 + (lane >> 5) * 8;
-    auto multiply = [&]() {
+    // wave w: 32-row tile w % row tiles, k part w / row tiles of the stage; lane l of an operand: row l % 32, chunk 2 ks + l / 32
+    const int wr = wave % F::kRowTiles, kp = wave / F::kRowTiles;
+    const int lr = lane & 31;
+    int foff[2];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const bf16x8_t fa = *reinterpret_cast<const bf16x8_t*>(tile + foff + ks * 16);
+    for (int ks = 0; ks < 2; ++ks) foff[ks] = lr * RB + (((kp * 4 + ks * 2 + (lane >> 5)) ^ swz(lr)) * 16);
+    auto multiply = [&](int slot, int k0) {
+        const bool out = CUT && k0 + kp * 32 >= K;              // a select, not a branch: product and encoder stay interleaved
+        const unsigned char* b = lds + slot * STAGE;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            bf16x8_t fa = *reinterpret_cast<const bf16x8_t*>(b + wr * 32 * RB + foff[ks]);
+            if (out) fa = bf16x8_t{};
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
-                const bf16x8_t fb = *reinterpret_cast<const bf16x8_t*>(tile + (32 + j * 32) * NT_STRIDE + foff + ks * 16);
+                bf16x8_t fb = *reinterpret_cast<const bf16x8_t*>(b + (ROWS + j * 32) * RB + foff[ks]);
+                if (out) fb = bf16x8_t{};
                 acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb, fa, acc[j], 0, 0, 0);
             }
         }
     };
-    // two steps are in flight while a third is multiplied: the time of one step is then half the memory latency
-    if (steps > 0) fetch(rx[0], rv[0], kof(0));
-    if (steps > 1) fetch(rx[1], rv[1], kof(1));
-    for (int st = 0; st < steps; st += 2) {
-        stage(rx[0], rv[0]);
-        __syncthreads();
-        if (st + 2 < steps) fetch(rx[0], rv[0], kof(st + 2));
-        multiply();
-        encode(kof(st));
-        __syncthreads();
-        if (st + 1 < steps) {
-            stage(rx[1], rv[1]);
-            __syncthreads();
-            if (st + 3 < steps) fetch(rx[1], rv[1], kof(st + 3));
-            multiply();
-            encode(kof(st + 1));
-            __syncthreads();
+    // a thread encodes one block of the stage, consecutive threads consecutive blocks of a row.  Rows past the tensor repeat its last row: the stores below are
+    // never skipped, which the counted waits rely on (the same bytes to the same place).
+    float gmax = 0.0f;
+    const int erow = tid / (KS / 16), eblk = tid % (KS / 16), eswz = swz(erow);
+    const int64_t eib = (int64_t)min(m0 + erow, M - 1) * (K / kBlock);
+    auto encode = [&](int slot, int k0) {
+        if constexpr (QMODE >= 0) {
+            const unsigned char* b = lds + slot * STAGE + erow * RB;
+            const int blk = (CUT && k0 + eblk * kBlock >= K) ? eblk - 4 : eblk;
+            const uint4 c0 = *reinterpret_cast<const uint4*>(b + ((2 * blk) ^ eswz) * 16);
+            const uint4 c1 = *reinterpret_cast<const uint4*>(b + ((2 * blk + 1) ^ eswz) * 16);
+            float val[kBlock];
+            const float none[kBlock] = {};
+            unpack16(c0, c1, val);
+            const float am = block_amax(val);
+            gmax = fmaxf(gmax, am);
+            const int64_t ib = eib + k0 / kBlock + blk;
+            q_amax[ib] = (uint16_t)(__float_as_uint(am) >> 16);
+            codes[ib] = encode_block<QMODE < 0 ? 0 : QMODE, false>(val, block_scalar<QMODE < 0 ? 0 : QMODE>(am), none);
         }
+    };
+
+    // ---- stage st lies in slot st % NS.  Per stage: wait for its own loads (a stage is requested NS - 1 iterations ahead),
+    // barrier, request stage st + NS - 1 into the slot that everybody left before the barrier, multiply, encode.
+    // The counter also counts the two stores of an encoded stage: (NS - 1) iterations of them follow a stage's loads.
+    constexpr int STORES = QMODE >= 0 ? 2 : 0;
+#pragma unroll
+    for (int p = 0; p < NS - 1; ++p)
+        if (p < steps) issue(p, p);
+    int slot = 0;
+    for (int st = 0; st < steps; ++st) {
+        if (st + NS - 1 > steps) nt_wait<0>();                 // fewer stages behind it than counted below
+        else if (st < NS - 1) nt_wait<(NS - 2) * LPW>();
+        else nt_wait<(NS - 2) * LPW + (NS - 1) * STORES>();
+        __syncthreads();
+        if (st + NS - 1 < steps) issue(slot == 0 ? NS - 1 : slot - 1, st + NS - 1);
+        const int k0 = kof(st);
+        multiply(slot, k0);
+        encode(slot, k0);
+        slot = slot + 1 == NS ? 0 : slot + 1;
     }
-    if constexpr (QMODE >= 0 && !EW) {
+    __syncthreads();                                            // the ring is free
+    float* red = reinterpret_cast<float*>(lds);                 // [part - 1][row tile][j][e][lane], then the waves' maxima
+    if constexpr (QMODE >= 0) {
+        float* smax = red + (F::kParts - 1) * F::kRowTiles * RT * 1024;
         const float wm = wave_max(gmax);
         if (lane == 0) smax[wave] = wm;
-        __syncthreads();
-        const uint32_t gid = blockIdx.y * gridDim.x + blockIdx.x, gsize = gridDim.x * gridDim.y;
-        if (tid == 0) q_gmax[gid] = __float_as_uint(fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])));
-        for (uint32_t j = gsize + gid * 256u + tid; j < fill_to; j += gsize * 256u) q_gmax[j] = 0u;
     }
-    // acc[j][e] of lane l: row m0 + l % 32, column 32 j + 8 (e / 4) + 4 (l / 32) + e % 4.  The four waves hold the four
-    // quarters of every step of K: their sums meet in LDS (the staged tile is dead after the last barrier), and
-    // wave w finishes the quarter e / 4 == w of the columns, adding the waves' shares in the order 0, 1, 2, 3.
+    // acc[j][e] of lane l: row m0 + 32 wr + l % 32, column 32 j + 8 (e / 4) + 4 (l / 32) + e % 4.  The other parts of
+    // every stage's k join the first in LDS, in ascending order.
+    if (kp > 0) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) red[((((kp - 1) * F::kRowTiles + wr) * RT + j) * 16 + e) * 64 + lane] = acc[j][e];
+    }
+    __syncthreads();
+    if constexpr (QMODE >= 0) {
+        const float* smax = red + (F::kParts - 1) * F::kRowTiles * RT * 1024;
+        const uint32_t gid = blockIdx.y * gridDim.x + blockIdx.x, gsize = gridDim.x * gridDim.y;
+        if (tid == 0) {
+            float wm = smax[0];
+#pragma unroll
+            for (int w = 1; w < F::kWaves; ++w) wm = fmaxf(wm, smax[w]);
+            q_gmax[gid] = __float_as_uint(wm);
+        }
+        for (uint32_t j = gsize + gid * F::kThreads + tid; j < fill_to; j += gsize * F::kThreads) q_gmax[j] = 0u;
+    }
+    const int m = m0 + wr * 32 + lr;
+    if (kp > 0 || m >= M) return;
 #pragma unroll
     for (int j = 0; j < RT; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) red[((wave * RT + j) * 16 + e) * 64 + lane] = acc[j][e];
-    __syncthreads();
-    const int m = m0 + (lane & 31);
-    if (m >= M) return;
+        for (int g = 0; g < 4; ++g) {
+            const int col = j * 32 + 8 * g + 4 * (lane >> 5);
+            float sum[4];
+            uint32_t h[4], ts[4];
 #pragma unroll
-    for (int j = 0; j < RT; ++j) {
-        const int col = j * 32 + 8 * wave + 4 * (lane >> 5);
-        float sum4[4];
-        uint32_t h[4], ts[4];
+            for (int e = 0; e < 4; ++e) {
+                sum[e] = acc[j][4 * g + e];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int ee = 4 * wave + e;
-            float sum = red[((0 * RT + j) * 16 + ee) * 64 + lane];
+                for (int p = 0; p + 1 < F::kParts; ++p) sum[e] += red[(((p * F::kRowTiles + wr) * RT + j) * 16 + 4 * g + e) * 64 + lane];
+            }
+            if (part) {                                         // one of several slices: the finishing kernel rounds
+                *reinterpret_cast<float4*>(part + ((int64_t)blockIdx.y * M + m) * R + col) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+                continue;
+            }
 #pragma unroll
-            for (int w = 1; w < 4; ++w) sum += red[((w * RT + j) * 16 + ee) * 64 + lane];
-            sum4[e] = sum;
+            for (int e = 0; e < 4; ++e) {
+                h[e] = bf16_bits(sum[e]);
+                if (t) ts[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(s[col + e]));
+            }
+            *reinterpret_cast<uint2*>(xv + (int64_t)m * R + col) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+            if (t) *reinterpret_cast<uint2*>(t + (int64_t)m * R + col) = make_uint2(ts[0] | (ts[1] << 16), ts[2] | (ts[3] << 16));
         }
-        if (part) {                                             // one of several slices: the finishing kernel rounds
-            *reinterpret_cast<float4*>(part + ((int64_t)blockIdx.y * M + m) * R + col) = make_float4(sum4[0], sum4[1], sum4[2], sum4[3]);
-            continue;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            h[e] = bf16_bits(sum4[e]);
-            if (t) ts[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(s[col + e]));
-        }
-        *reinterpret_cast<uint2*>(xv + (int64_t)m * R + col) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-        if (t) *reinterpret_cast<uint2*>(t + (int64_t)m * R + col) = make_uint2(ts[0] | (ts[1] << 16), ts[2] | (ts[3] << 16));
-    }
 }
 
 // xv = bf16(sum over slices, ascending), t = bf16(xv * s): four columns per thread
@@ -271,14 +252,13 @@ __global__ __launch_bounds__(256) void lowrank_nt_finish_kernel(const float* __r
     }
 }
 
-// K slices for M rows: none when the row tiles alone give every compute unit a workgroup (measured: slices then cost
-// what the second launch costs); otherwise about two workgroups per compute unit, at least four steps per slice, and
-// never more workgroups than the quantizer's partial maxima have room for.
+// K slices for M rows: none when 32-row tiles give every compute unit a workgroup; otherwise about two such tiles per compute
+// unit, at least 1024 k per slice, and never more workgroups than the quantizer's partial maxima have room for.
 static int nt_slices(int64_t M, int64_t K, size_t workspace_bytes, int64_t R)
 {
-    const int64_t tiles = (M + 31) / 32, steps = (K + NT_STEP - 1) / NT_STEP, cus = device_cus();
+    const int64_t tiles = (M + 31) / 32, steps = (K + 255) / 256, cus = device_cus();
     if (tiles >= cus) return 1;
-    int64_t sl = (2 * cus + tiles - 1) / tiles;
+    int64_t sl = 2 * cus / tiles;                               // (one more round of workgroups for a few of them costs a third: 2103 x 18944 28 -> 26 us)
     if (sl > steps / 4) sl = steps / 4;
     if (sl * tiles > (int64_t)kDeferredPartials) sl = (int64_t)kDeferredPartials / tiles;
     if (sl > 16) sl = 16;
@@ -293,22 +273,35 @@ size_t lowrank_nt_workspace_bytes(int64_t M, int64_t R, int64_t K)
     return sl > 1 ? (size_t)sl * M * R * 4 : 0;
 }
 
+template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
+static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, const void* v, const void* s, void* xv, void* t, int64_t M, int64_t K,
+                     float* part, void* codes, uint16_t* amax, uint32_t* gmax)
+{
+    using F = NtForm<RT, ROWS, KS, NS>;
+    static bool attr_set[64] = {};
+    if (const int rc = allow_dynamic_lds((const void*)lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>, F::kLds, attr_set)) return rc;
+    hipLaunchKernelGGL((lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>), dim3((unsigned)((M + ROWS - 1) / ROWS), (unsigned)slices), dim3(F::kThreads), F::kLds, st,
+                       (const uint16_t*)x, ldx, (const uint16_t*)v, (const uint16_t*)s, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part,
+                       (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 13));
+    return METIS_OK;
+}
+
 // qmode < 0: the product alone.  qmode = METIS_MODE_P32 / _PB16: x (contiguous rows, ldx == K) is quantized on the way,
 // codes and the deferred data (partial maxima, parked block maxima) as quantize_row_deferred leaves them.
 int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
                hipStream_t st, void* workspace, size_t workspace_bytes, int qmode, void* codes, void* deferred, size_t deferred_size)
 {
     if (M < 0 || R <= 0 || K <= 0 || ldx < K) return METIS_E_ARG;
-    if ((R != 32 && R != 64 && R != 128) || K % 64 || ldx % 8) return METIS_E_SHAPE;
+    if ((R != 32 && R != 64 && R != 96 && R != 128 && R != 192 && R != 256) || K % 64 || ldx % 8) return METIS_E_SHAPE;
     if (M == 0) return METIS_OK;
-    if (M > INT32_MAX - 32 || K > INT32_MAX) return METIS_E_ARG;
+    if (M > INT32_MAX - 64 || K > INT32_MAX) return METIS_E_ARG;
     if (!x || !v || !xv || (t && !s)) return METIS_E_ARG;
     if (((uintptr_t)x % 16) || ((uintptr_t)v % 16) || ((uintptr_t)xv % 8) || ((uintptr_t)t % 8) || ((uintptr_t)s % 2)) return METIS_E_ARG;
     if (workspace && ((uintptr_t)workspace % 16)) return METIS_E_WORKSPACE;
     Workspace q = {nullptr, nullptr, nullptr};
     if (qmode >= 0) {
         if (qmode != METIS_MODE_P32 && qmode != METIS_MODE_PB16) return METIS_E_ARG;
-        if (R == 128) return METIS_E_SHAPE;
+        if (R > 64) return METIS_E_SHAPE;
         if (ldx != K || !codes || ((uintptr_t)codes % 8)) return METIS_E_ARG;
         if ((M + 31) / 32 > (int64_t)kDeferredPartials) return METIS_E_TOO_LARGE;
         if (M * K / kBlock >= (int64_t)1 << 31) return METIS_E_ARG;
@@ -316,21 +309,37 @@ int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, 
     }
     const int slices = workspace ? nt_slices(M, K, workspace_bytes, R) : 1;
     float* part = slices > 1 ? static_cast<float*>(workspace) : nullptr;
-    const dim3 grid((unsigned)((M + 31) / 32), (unsigned)slices);
-    // encoding waves of their own when a compute unit gets one workgroup anyway
-    const bool ew = (int64_t)grid.x * grid.y <= (int64_t)device_cus();
-#define METIS_NT(RT, Q) METIS_NT2(RT, Q, false)
-#define METIS_NT2(RT, Q, E) hipLaunchKernelGGL((lowrank_nt_kernel<RT, Q, E>), grid, dim3((Q >= 0 && E) ? 512 : 256), 0, st, (const uint16_t*)x, ldx, (const uint16_t*)v, \
-                                           (const uint16_t*)s, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part, (uint2*)codes, q.amax, \
-                                           q.gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 5))
-#define METIS_NTQ(RT) do { if (qmode < 0) METIS_NT(RT, -1); else if (qmode == 0) { if (ew) METIS_NT2(RT, 0, true); else METIS_NT(RT, 0); } \
-                           else { if (ew) METIS_NT2(RT, 1, true); else METIS_NT(RT, 1); } } while (0)
-    if (R == 32) METIS_NTQ(1);
-    else if (R == 64) METIS_NTQ(2);
-    else METIS_NT(4, -1);                                      // R = 128 fills the register file with the product alone
-#undef METIS_NTQ
-#undef METIS_NT2
+    int rc = METIS_OK;
+    // 64-row tiles read v half as often, but only where they still give every compute unit a workgroup; stages of 128 k
+    // leave whole 64-byte pieces of codes (with 64 k the quantizing form takes 338 us in place of 229 below).  Microseconds,
+    // 64 rows | 32 rows:
+    //   16384 x 3584, R = 64    28 | 33                 8192 x 4096, R = 64    18.5 | 15.7
+    //   16384 x 18944, R = 64, quantized  229 | 270     8192 x 14336, R = 64   76 | 60
+    //   16384 x 3584, R = 192 (64 k | 128 k)  50 | 81   1024 x 3584, R = 192   17.1 | 16.2
+    const bool tall = ((M + 63) / 64) * slices >= device_cus(), cut = K % 128 != 0;
+#define METIS_NT(RT, Q, ROWS, KS, NS, CUT) rc = launch_nt<RT, Q, ROWS, KS, NS, CUT>(slices, st, x, ldx, v, s, xv, t, M, K, part, codes, q.amax, q.gmax)
+#define METIS_NT128(RT, Q, ROWS, NS) do { if (cut) METIS_NT(RT, Q, ROWS, 128, NS, true); else METIS_NT(RT, Q, ROWS, 128, NS, false); } while (0)
+#define METIS_NTF(RT, Q) do { if (tall) METIS_NT128(RT, Q, 64, 3); else METIS_NT128(RT, Q, 32, 3); } while (0)
+#define METIS_NTG(RT, NT, NW) do { if (tall) METIS_NT(RT, -1, 64, 64, NT, false); else METIS_NT128(RT, -1, 32, NW); } while (0)
+    if (qmode < 0) {
+        if (R == 32) METIS_NTF(1, -1);
+        else if (R == 64) METIS_NTF(2, -1);
+        else if (R == 96) METIS_NTG(3, 4, 3);
+        else if (R == 128) METIS_NTG(4, 4, 3);
+        else if (R == 192) METIS_NTG(6, 4, 2);
+        else METIS_NTG(8, 3, 2);
+    } else if (qmode == METIS_MODE_P32) {
+        if (R == 32) METIS_NTF(1, 0);
+        else METIS_NTF(2, 0);
+    } else {
+        if (R == 32) METIS_NTF(1, 1);
+        else METIS_NTF(2, 1);
+    }
+#undef METIS_NTG
+#undef METIS_NTF
+#undef METIS_NT128
 #undef METIS_NT
+    if (rc) return rc;
     if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     if (slices > 1) {
         const int64_t MR = M * R;

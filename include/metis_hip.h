@@ -533,7 +533,7 @@ int metis_lowrank_project(const void *x, int64_t ldx, const void *v, int64_t M, 
  * The same projection for training and prefill batches (any M; meant for M >= 256), one pass over x:
  *     xv[M, R] = x[M, K] . v[R, K]^T,  t = bf16(xv * s) when t != NULL     (src/Metis/Metis/bitlinear.py:752-756)
  * and, with v = U^T [r, N] and x = dY [L, N], the product dY . U of the backward pass.
- *   R in {32, 64, 128}, K % 64 == 0, ldx % 8 == 0 (METIS_E_SHAPE otherwise); x, v 16-byte aligned; no workspace
+ *   R in {32, 64, 96, 128, 192, 256}, K % 64 == 0, ldx % 8 == 0 (METIS_E_SHAPE otherwise); x, v 16-byte aligned; no workspace
  */
 int metis_lowrank_project_rows(const void *x, int64_t ldx, const void *v, int64_t M, int64_t R, int64_t K,
                                const void *s, void *xv, void *t, void *stream);

@@ -633,6 +633,30 @@ def test_rank_r_projection_at_training_sizes(M, R, K):
     assert torch.equal(ops.lowrank_project(wide[:, :K], v), xv)
 
 
+@pytest.mark.parametrize("M,R,K", [(256, 96, 64), (257, 192, 192), (411, 256, 1536), (16385, 192, 128), (16384, 64, 192), (20000, 32, 320),
+                                   (2103, 64, 18944), (300, 128, 4160), (16400, 96, 256)])
+def test_rank_r_projection_tiles_of_32_and_64_rows(M, R, K):
+    """Both tile heights, K that ends in half a stage, one stage or fewer than the ring holds, the ranks of stacked factors: bf16
+    of a binary32 sum (K products of bf16 values, relative error at most K 2^-24 of the sum of magnitudes) against double."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(6100 + M + R)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    v = (torch.randn(R, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    s = (torch.rand(R, generator=g, device="cuda") * 4 + 0.1).bfloat16()
+    xv, t = ops.lowrank_project(x, v, s)
+    want = x.double() @ v.double().T
+    bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ v.double().abs().T) * (K * 2.0 ** -24)
+    torch.cuda.synchronize()
+    assert bool(((xv.double() - want).abs() <= bound).all())
+    assert torch.equal(t, (xv.float() * s.float()).bfloat16())
+    if R <= 64:
+        for mode in (0, 1):
+            p, qxv, qt = ops.quantize_project(x, v, s, mode)
+            ref = ops.quantize(x, mode)
+            assert torch.equal(p.codes, ref.codes) and torch.equal(p.scales, ref.scales) and torch.equal(p.unit, ref.unit)
+            assert torch.equal(qxv, xv) and torch.equal(qt, t)
+
+
 @pytest.mark.parametrize("L,C,R", [(1000, 520, 32), (4096, 1536, 64), (4096, 8960, 32), (2048, 14336, 64), (777, 256, 128)])
 def test_rank_r_products_that_contract_over_tokens(L, C, R):
     """out[C, R] = sum_l a[l, C] b[l, R] (gradients of U and, transposed, of V): token slices added in a fixed order,
