@@ -293,6 +293,18 @@ int metis_linear_fwd_tiled(const void* a_xt, const float* a_unit, const void* b_
                    workspace_bytes, (hipStream_t)stream);
 }
 
+size_t metis_linear_tiled_grouped_workspace_bytes(int64_t M, int64_t K, const metis_linear_member* members, int count)
+{
+    return gemm_xt_grouped_workspace_bytes(M, K, reinterpret_cast<const GemmMember*>(members), count);
+}
+
+int metis_linear_fwd_tiled_grouped(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const metis_linear_member* members, int count,
+                                   int out_dtype, int mode, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return gemm_xt_grouped(a_xt, a_unit, M, K, reinterpret_cast<const GemmMember*>(members), count, out_dtype, mode, workspace, workspace_bytes,
+                           (hipStream_t)stream);
+}
+
 int metis_linear_dgrad(const void* dy_codes, const void* dy_scales, const float* dy_unit, const void* wt_codes,
                        const void* wt_scales, const float* wt_unit, int64_t L, int64_t N, int64_t K, void* grad_input,
                        int out_dtype, void* stream)

@@ -164,6 +164,39 @@ __device__ __forceinline__ void tile_origin(int logical, int tiles_m, int tiles_
     n0 = tn * L_BN;
 }
 
+// The weight side of a tiled GEMM: up to four matrices that share the activation, their tile columns end to end.
+constexpr int kTiledMembers = 4;
+struct TiledMember {
+    const uint8_t* b;            // tiled operand (the packed kernel has its own)
+    const float* b_unit;
+    const uint16_t *t, *u, *bias;
+    void* out;
+    int N, r, ldt, bias_f32;     // ldt: row stride of t (members may take columns of a stacked projection)
+    int tile0;                   // first tile column
+};
+struct TiledGroup {
+    TiledMember m[kTiledMembers];
+    int count, tiles_n;
+};
+__device__ __forceinline__ int tiled_member_of(const TiledGroup& g, int tn)
+{
+    int i = 0;
+#pragma unroll
+    for (int q = 1; q < kTiledMembers; ++q)
+        if (q < g.count && tn >= g.m[q].tile0) i = q;
+    return __builtin_amdgcn_readfirstlane(i);
+}
+// one matrix
+inline TiledGroup tiled_group_of(const void* b, const float* b_unit, int64_t N, const void* t, const void* u, int64_t r, const void* bias,
+                                 int bias_f32, void* out)
+{
+    TiledGroup g = {};
+    g.m[0] = {(const uint8_t*)b, b_unit, (const uint16_t*)t, (const uint16_t*)u, (const uint16_t*)bias, out, (int)N, (int)r, (int)r, bias_f32, 0};
+    g.count = 1;
+    g.tiles_n = (int)((N + L_BN - 1) / L_BN);
+    return g;
+}
+
 // Dynamic LDS above 64 KiB has to be allowed per kernel function and per device: done once for each pair.
 inline int allow_dynamic_lds(const void* fn, size_t bytes, bool (&done)[64])
 {
@@ -184,12 +217,10 @@ inline int allow_dynamic_lds(const void* fn, size_t bytes, bool (&done)[64])
 // PB16 (every op of the reference rounded to bf16): the sum of the partial tiles is rounded to bf16 as the reference's
 // bf16 matmul rounds it, the bias is added in bf16, then the low-rank term and the final rounding.
 template <int OUT_F32, int PB16 = 0>
-__global__ __launch_bounds__(64) void gemm_splitk_reduce_kernel(const float* __restrict__ ws, int nsplit, int M, int N,
-                                                                int tiles_m, int tiles_n, void* __restrict__ out, int nfull,
-                                                                const uint16_t* __restrict__ bias, int bias_f32,
-                                                                const uint16_t* __restrict__ t = nullptr,
-                                                                const uint16_t* __restrict__ u = nullptr, int r = 0)
+__global__ __launch_bounds__(64) void gemm_splitk_reduce_kernel(const float* __restrict__ ws, int nsplit, int M, int tiles_m, int nfull,
+                                                                const TiledGroup grp)
 {
+    const int tiles_n = grp.tiles_n;
     constexpr int TN = 2, WTN = 64, NTHREADS = 512, TILE = L_BM * L_BN;
     __shared__ __attribute__((aligned(16))) uint16_t cw[32 * 72];
     const int total = tiles_m * tiles_n - nfull;                 // split tiles
@@ -198,6 +229,11 @@ __global__ __launch_bounds__(64) void gemm_splitk_reduce_kernel(const float* __r
     const int wm = wave / 4, wn = wave % 4;
     int m0, n0;
     tile_origin(nfull + tile, tiles_m, tiles_n, m0, n0);
+    const int mi = tiled_member_of(grp, n0 / L_BN);
+    n0 -= grp.m[mi].tile0 * L_BN;
+    const int N = grp.m[mi].N, r = grp.m[mi].r, ldt = grp.m[mi].ldt, bias_f32 = grp.m[mi].bias_f32;
+    const uint16_t *bias = grp.m[mi].bias, *t = grp.m[mi].t, *u = grp.m[mi].u;
+    void* out = grp.m[mi].out;
     const int mbase = m0 + wm * 128 + i * 32, nbase = n0 + wn * WTN;
     if (mbase >= M || nbase >= N) return;
 
@@ -224,7 +260,7 @@ __global__ __launch_bounds__(64) void gemm_splitk_reduce_kernel(const float* __r
         for (int e = 0; e < 16; ++e) low[j][e] = 0.0f;
     {
         if (r > 0) {                                             // lane l: row l % 32 of its operand, columns 8 (l / 32) .. of the step
-            const uint16_t* tp = t + (int64_t)min(mbase + (lane & 31), M - 1) * r + 8 * (lane >> 5);
+            const uint16_t* tp = t + (int64_t)min(mbase + (lane & 31), M - 1) * ldt + 8 * (lane >> 5);
             const uint16_t* up[TN];
 #pragma unroll
             for (int j = 0; j < TN; ++j) up[j] = u + (int64_t)min(nbase + j * 32 + (lane & 31), N - 1) * r + 8 * (lane >> 5);
@@ -317,11 +353,10 @@ struct SplitPlan {
     int nsplit;
     int nfull;                   // leading tiles that run unsplit (a multiple of the compute units)
 };
-inline SplitPlan split_plan(int64_t M, int64_t N, int64_t K)
+inline SplitPlan split_plan_tiles(int64_t tiles, int64_t K)
 {
     const SplitPlan none = {1, 0};
-    if (M < L_BM || N < L_BN || K % BK) return none;
-    const int64_t tiles = ((M + L_BM - 1) / L_BM) * ((N + L_BN - 1) / L_BN);
+    if (K % BK) return none;
     const int cus = device_cus();
     if (cus <= 0 || cus % 8 || tiles > INT32_MAX) return none;
     int64_t part = tiles, nfull = 0;                            // tiles to split
@@ -335,6 +370,11 @@ inline SplitPlan split_plan(int64_t M, int64_t N, int64_t K)
     if (s > 16) s = 16;
     if (s < 2) return none;
     return SplitPlan{(int)s, (int)nfull};
+}
+inline SplitPlan split_plan(int64_t M, int64_t N, int64_t K)
+{
+    if (M < L_BM || N < L_BN) return SplitPlan{1, 0};
+    return split_plan_tiles(((M + L_BM - 1) / L_BM) * ((N + L_BN - 1) / L_BN), K);
 }
 
 }  // namespace metis

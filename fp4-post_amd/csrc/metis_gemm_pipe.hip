@@ -412,10 +412,8 @@ __host__ __device__ constexpr int waitcnt_imm(int vm, int lgkm)
 
 template <int OUT_F32, int PB16, int SPLIT>
 __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
-    const uint8_t* __restrict__ a_xt, const float* __restrict__ a_unit, const uint8_t* __restrict__ b_xt,
-    const float* __restrict__ b_unit, int M, int N, int K, const uint16_t* __restrict__ t, const uint16_t* __restrict__ u,
-    int r, const uint16_t* __restrict__ bias, void* __restrict__ out, int tiles_m, int tiles_n, int bias_f32,
-    float* __restrict__ ws, int nsplit, int nfull)
+    const uint8_t* __restrict__ a_xt, const float* __restrict__ a_unit, int M, int K, int tiles_m, float* __restrict__ ws, int nsplit,
+    int nfull, const TiledGroup grp)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t xlds[];
     constexpr int TM = 4, TN = 2, WTN = 64, NWAVES = 8, NTHREADS = 512, NS = XT_NS;
@@ -426,7 +424,7 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
 
     // ---- tile assignment: contiguous range per XCD, groups of four tile rows (see tile_origin).  SPLIT: the first
     //      nfull tiles (a multiple of 8) run unsplit, every XCD its share of them first; the rest have nsplit workgroups each.
-    const int total = tiles_m * tiles_n;
+    const int tiles_n = grp.tiles_n, total = tiles_m * tiles_n;
     int logical, split = 0;
     bool partial = false;
     if constexpr (SPLIT != 0) {
@@ -448,6 +446,14 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
     }
     int m0, n0;
     tile_origin(logical, tiles_m, tiles_n, m0, n0);
+    // the matrix that this tile column belongs to, columns counted from its first
+    const int mi = tiled_member_of(grp, n0 / L_BN);
+    n0 -= grp.m[mi].tile0 * L_BN;
+    const int N = grp.m[mi].N, r = grp.m[mi].r, ldt = grp.m[mi].ldt, bias_f32 = grp.m[mi].bias_f32;
+    const uint8_t* __restrict__ b_xt = grp.m[mi].b;
+    const float* __restrict__ b_unit = grp.m[mi].b_unit;
+    const uint16_t *__restrict__ t = grp.m[mi].t, *__restrict__ u = grp.m[mi].u, *__restrict__ bias = grp.m[mi].bias;
+    void* __restrict__ out = grp.m[mi].out;
     const int kt = K / 32;
     const int step_begin = partial ? (int)((int64_t)split * kt / nsplit) : 0;
     const int steps = (partial ? (int)((int64_t)(split + 1) * kt / nsplit) : kt) - step_begin;   // >= 1: the host never asks for more splits than stages
@@ -493,7 +499,7 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
                 const int ot = j * NWAVES + wave;
                 const bool is_a = ot < 16;
                 const int64_t row = is_a ? min(m0 + ot * 16 + q, M - 1) : min(n0 + (ot - 16) * 16 + q, N - 1);
-                const uint16_t* g = (is_a ? t : u) + row * r + p * 32 + chunk * 8;
+                const uint16_t* g = (is_a ? t + row * ldt : u + row * r) + p * 32 + chunk * 8;
                 const uint32_t dst = (uint32_t)((NS + p) * XT_STAGE + ot * 1024);
                 asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(dst) : "memory");
             }
@@ -654,7 +660,7 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
             const int trow = tid;                               // 512 threads, 512 rows of the T|U tile
             const bool is_a = trow < L_BM;
             const int64_t grow = is_a ? min(m0 + trow, M - 1) : min(n0 + trow - L_BM, N - 1);
-            const uint4* sp = reinterpret_cast<const uint4*>((is_a ? t : u) + grow * r + j0);
+            const uint4* sp = reinterpret_cast<const uint4*>((is_a ? t + grow * ldt : u + grow * r) + j0);
             uint4* dp = reinterpret_cast<uint4*>(plds + trow * L_STRIDE);
 #pragma unroll
             for (int c = 0; c < 4; ++c) dp[c] = sp[c];
@@ -757,9 +763,9 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
 }
 
 // K splits of the pipelined kernel: the plan of the packed kernel (same tiles), with a stage of 32 k as the unit.
-static SplitPlan xt_split_plan(int64_t M, int64_t N, int64_t K)
+static SplitPlan xt_split_plan(int64_t M, int64_t N, int64_t K, int64_t group_tiles = 0)
 {
-    SplitPlan p = split_plan(M, N, K);                          // needs K % 64 == 0, M and N >= 256
+    SplitPlan p = group_tiles && M >= L_BM ? split_plan_tiles(group_tiles, K) : split_plan(M, N, K);   // needs K % 64 == 0, M and N >= 256
     if (p.nsplit > K / 32) p.nsplit = (int)(K / 32);
     return p.nsplit < 2 ? SplitPlan{1, 0} : p;
 }
@@ -775,32 +781,48 @@ size_t gemm_xt_workspace_bytes(int64_t M, int64_t N, int64_t K, int mode)
 }
 
 template <int OUT_F32, int PB16, int SPLIT>
-static int launch_xt(const void* a_xt, const float* a_unit, const void* b_xt, const float* b_unit, int64_t M, int64_t N, int64_t K,
-                     const void* t, const void* u, int64_t r, const void* bias, int bias_f32, void* out, hipStream_t st, float* ws,
-                     int nsplit, int nfull)
+static int launch_xt(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const TiledGroup& grp, hipStream_t st, float* ws, int nsplit,
+                     int nfull)
 {
     static bool attr_set[64] = {};
     const void* fn = (const void*)gemm_xt_kernel<OUT_F32, PB16, SPLIT>;
     const size_t lds_bytes = (size_t)XT_LDS;
     if (const int rc = allow_dynamic_lds(fn, lds_bytes, attr_set)) return rc;
-    const int tiles_m = (int)((M + L_BM - 1) / L_BM), tiles_n = (int)((N + L_BN - 1) / L_BN);
-    const int total = tiles_m * tiles_n;
+    int tiles_m = (int)((M + L_BM - 1) / L_BM);
+    const int total = tiles_m * grp.tiles_n;
     const unsigned grid_x = SPLIT ? 8u * (unsigned)(nfull / 8 + ((total - nfull) * nsplit + 7) / 8) : (unsigned)(((total + 7) / 8) * 8);
-    const uint8_t *ae = (const uint8_t*)a_xt, *be = (const uint8_t*)b_xt;
-    const uint16_t *tp = (const uint16_t*)t, *up = (const uint16_t*)u, *bp = (const uint16_t*)bias;
-    int Mi = (int)M, Ni = (int)N, Ki = (int)K, ri = (int)r, tmi = tiles_m, tni = tiles_n;
-    void* args[] = {&ae, &a_unit, &be, &b_unit, &Mi, &Ni, &Ki, &tp, &up, &ri, &bp, &out, &tmi, &tni, &bias_f32, &ws, &nsplit, &nfull};
+    const uint8_t* ae = (const uint8_t*)a_xt;
+    int Mi = (int)M, Ki = (int)K;
+    TiledGroup g = grp;
+    void* args[] = {&ae, &a_unit, &Mi, &Ki, &tiles_m, &ws, &nsplit, &nfull, &g};
     if (hipLaunchKernel(fn, dim3(grid_x), dim3(512), args, lds_bytes, st) != hipSuccess) {
         (void)hipGetLastError();
         return METIS_E_LAUNCH;
     }
     if (SPLIT) {
         const dim3 rgrid((unsigned)(total - nfull) * 32u);
-        hipLaunchKernelGGL((gemm_splitk_reduce_kernel<OUT_F32, PB16>), rgrid, dim3(64), 0, st, (const float*)ws, nsplit, Mi, Ni, tmi, tni, out,
-                           nfull, bp, bias_f32, tp, up, ri);
+        hipLaunchKernelGGL((gemm_splitk_reduce_kernel<OUT_F32, PB16>), rgrid, dim3(64), 0, st, (const float*)ws, nsplit, Mi, tiles_m, nfull, g);
         if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     }
     return METIS_OK;
+}
+
+static int dispatch_xt(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const TiledGroup& grp, int out_dtype, int mode,
+                       SplitPlan plan, void* workspace, hipStream_t st)
+{
+    const int f32 = out_dtype == METIS_DTYPE_F32, pb = mode == METIS_MODE_PB16, sp = plan.nsplit > 1;
+#define METIS_XT(F, P, S) launch_xt<F, P, S>(a_xt, a_unit, M, K, grp, st, (float*)workspace, plan.nsplit, plan.nfull)
+    switch (f32 * 4 + pb * 2 + sp) {
+        case 0: return METIS_XT(0, 0, 0);
+        case 1: return METIS_XT(0, 0, 1);
+        case 2: return METIS_XT(0, 1, 0);
+        case 3: return METIS_XT(0, 1, 1);
+        case 4: return METIS_XT(1, 0, 0);
+        case 5: return METIS_XT(1, 0, 1);
+        case 6: return METIS_XT(1, 1, 0);
+        default: return METIS_XT(1, 1, 1);
+    }
+#undef METIS_XT
 }
 
 int gemm_xt(const void* a_xt, const float* a_unit, const void* b_xt, const float* b_unit, int64_t M, int64_t N, int64_t K,
@@ -824,20 +846,65 @@ int gemm_xt(const void* a_xt, const float* a_unit, const void* b_xt, const float
         plan = xt_split_plan(M, N, K);
         if (plan.nsplit > 1 && (((uintptr_t)workspace % 16) || workspace_bytes < gemm_xt_workspace_bytes(M, N, K, mode))) return METIS_E_WORKSPACE;
     }
-    const int f32 = out_dtype == METIS_DTYPE_F32, pb = mode == METIS_MODE_PB16, sp = plan.nsplit > 1;
-#define METIS_XT(F, P, S) launch_xt<F, P, S>(a_xt, a_unit, b_xt, b_unit, M, N, K, t, u, r, bias, bias_f32, out, st, (float*)workspace, \
-                                            plan.nsplit, plan.nfull)
-    switch (f32 * 4 + pb * 2 + sp) {
-        case 0: return METIS_XT(0, 0, 0);
-        case 1: return METIS_XT(0, 0, 1);
-        case 2: return METIS_XT(0, 1, 0);
-        case 3: return METIS_XT(0, 1, 1);
-        case 4: return METIS_XT(1, 0, 0);
-        case 5: return METIS_XT(1, 0, 1);
-        case 6: return METIS_XT(1, 1, 0);
-        default: return METIS_XT(1, 1, 1);
+    return dispatch_xt(a_xt, a_unit, M, K, tiled_group_of(b_xt, b_unit, N, t, u, r, bias, bias_f32, out), out_dtype, mode, plan, workspace, st);
+}
+
+// Several weight matrices against one activation in one launch, their tile columns end to end: the last, partly filled round of
+// 256 tiles is paid once instead of once per matrix, narrow matrices (k, v) ride along, and one launch adds the split tiles.
+// 16384 tokens, 3584 -> 18944 twice: 37 rounds in place of 2 x 18.5 (19); -> 3584 + 512 + 512: 4.5 in place of 3.5 + 0.5 + 0.5
+// with three reductions.
+static int64_t group_tile_columns(const GemmMember* members, int count)
+{
+    int64_t n = 0;
+    for (int i = 0; i < count; ++i) n += (members[i].N + L_BN - 1) / L_BN;
+    return n;
+}
+
+static bool group_shapes_ok(int64_t M, int64_t K, const GemmMember* members, int count)
+{
+    if (M <= 0 || K <= 0 || K % 32 || !members || count < 1 || count > kTiledMembers || M > INT32_MAX - 256 || K > INT32_MAX) return false;
+    for (int i = 0; i < count; ++i)
+        if (members[i].N <= 0 || members[i].N > INT32_MAX / 8) return false;
+    return ((M + L_BM - 1) / L_BM) * group_tile_columns(members, count) <= INT32_MAX / 16;
+}
+
+size_t gemm_xt_grouped_workspace_bytes(int64_t M, int64_t K, const GemmMember* members, int count)
+{
+    if (!group_shapes_ok(M, K, members, count)) return 0;
+    const int64_t tiles = ((M + L_BM - 1) / L_BM) * group_tile_columns(members, count);
+    const SplitPlan p = xt_split_plan(M, 0, K, tiles);
+    return p.nsplit <= 1 ? 0 : (size_t)p.nsplit * (size_t)(tiles - p.nfull) * L_BM * L_BN * sizeof(float);
+}
+
+int gemm_xt_grouped(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const GemmMember* members, int count, int out_dtype, int mode,
+                    void* workspace, size_t workspace_bytes, hipStream_t st)
+{
+    if (out_dtype != METIS_DTYPE_BF16 && out_dtype != METIS_DTYPE_F32) return METIS_E_ARG;
+    if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16) return METIS_E_ARG;
+    if (M < 0 || count < 1 || count > kTiledMembers || !members) return METIS_E_ARG;
+    if (K <= 0 || K % kBlock) return METIS_E_SHAPE;
+    if (M == 0) return METIS_OK;
+    if (!group_shapes_ok(M, K, members, count) || !a_xt || ((uintptr_t)a_xt % 16) || (mode == METIS_MODE_P32 && !a_unit)) return METIS_E_ARG;
+    TiledGroup g = {};
+    for (int i = 0; i < count; ++i) {
+        const GemmMember& m = members[i];
+        const int64_t ldt = m.ldt ? m.ldt : m.r;
+        if (m.N % 4 || m.r < 0 || m.r % 32 || m.r > INT32_MAX || (m.r > 0 && (!m.t || !m.u || ldt < m.r || ldt % 8 || ldt > INT32_MAX))) return METIS_E_ARG;
+        if (!m.b_codes || !m.out || (mode == METIS_MODE_P32 && !m.b_unit)) return METIS_E_ARG;
+        if (((uintptr_t)m.b_codes % 16) || ((uintptr_t)m.out % 16) || ((uintptr_t)m.t % 16) || ((uintptr_t)m.u % 16) ||
+            ((uintptr_t)m.bias % (m.bias_is_f32 ? 4 : 2)))
+            return METIS_E_ARG;
+        g.m[i] = {(const uint8_t*)m.b_codes, m.b_unit, (const uint16_t*)m.t, (const uint16_t*)m.u, (const uint16_t*)m.bias, m.out, (int)m.N, (int)m.r,
+                  (int)ldt, m.bias_is_f32 != 0, g.tiles_n};
+        g.tiles_n += (int)((m.N + L_BN - 1) / L_BN);
     }
-#undef METIS_XT
+    g.count = count;
+    SplitPlan plan = {1, 0};
+    if (workspace) {
+        plan = xt_split_plan(M, 0, K, ((M + L_BM - 1) / L_BM) * g.tiles_n);
+        if (plan.nsplit > 1 && (((uintptr_t)workspace % 16) || workspace_bytes < gemm_xt_grouped_workspace_bytes(M, K, members, count))) return METIS_E_WORKSPACE;
+    }
+    return dispatch_xt(a_xt, a_unit, M, K, g, out_dtype, mode, plan, workspace, st);
 }
 
 }  // namespace metis

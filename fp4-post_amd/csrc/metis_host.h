@@ -215,5 +215,9 @@ size_t gemm_xt_workspace_bytes(int64_t M, int64_t N, int64_t K, int mode);
 int gemm_xt(const void* a_xt, const float* a_unit, const void* b_xt, const float* b_unit, int64_t M, int64_t N, int64_t K,
             const void* t, const void* u, int64_t r, const void* bias, int bias_f32, void* out, int out_dtype, int mode,
             void* workspace, size_t workspace_bytes, hipStream_t st);
+// several weights (b_codes: the tiled operand) against one activation in one launch
+size_t gemm_xt_grouped_workspace_bytes(int64_t M, int64_t K, const GemmMember* members, int count);
+int gemm_xt_grouped(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const GemmMember* members, int count, int out_dtype, int mode,
+                    void* workspace, size_t workspace_bytes, hipStream_t st);
 
 }  // namespace metis

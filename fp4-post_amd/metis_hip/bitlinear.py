@@ -1018,7 +1018,7 @@ class BitLinear(nn.Module):
         return super()._apply(fn, recurse=recurse)
 
     # ------------------------------------------------------------------ projection group in one launch (inference)
-    grouped_inference = True      # q/k/v and gate/up of a decode-sized batch as one GEMM launch when autograd is off
+    grouped_inference = True      # q/k/v and gate/up as one GEMM launch when autograd is off
 
     def _packed_residual(self):
         """Packed residual weight for the fused launch, or None when the kernel path does not apply."""
@@ -1073,21 +1073,17 @@ class BitLinear(nn.Module):
         group = self.activation_group
         members = group["members"]
         rows = x.numel() // max(x.shape[-1], 1)
-        if rows >= 256 or not all(m._fusable() and m.compute_dtype == self.compute_dtype for m in members):
+        if not all(m._fusable() and m.compute_dtype == self.compute_dtype for m in members):
             return None
         packed = [m._packed_residual() for m in members]
         if any(p is None for p in packed):
             return None
+        if rows >= 256:
+            return self._forward_group_tiled(x, shared_input, members, packed)
         rotated = any(p.rht is not None for p in packed)          # NV recipe: the activation's operand carries the rotation
         cd = torch.bfloat16
         x2 = _flat2d(x).to(cd)
-        # one product for every member's rank-r projection: V of all members stacked, cached on their versions
-        key = tuple((_pkey(m.vlinear.weight), _pkey(m.s)) for m in members) + (x2.device,)
-        cached = group.get("stacked_v")
-        if cached is None or cached[0] != key:
-            cached = (key, torch.cat([m.vlinear.weight.to(cd) for m in members], dim=0),
-                      torch.cat([m.s.to(cd) for m in members], dim=0))
-            group["stacked_v"] = cached
+        cached = self._stacked_factors(x2.device)
         centre = shared_input.center32 if isinstance(shared_input, CenteredNVFP4) else None
         px = shared_input.residual if centre is not None else shared_input
         if centre is not None and all(F._mean_in_operand(shared_input, p) for p in packed):
@@ -1117,6 +1113,52 @@ class BitLinear(nn.Module):
         # mean mode: every member also receives W^ me, inside the same launch (binary32)
         outs = ops.linear_fwd_grouped(px, calls, out_dtype=out_dtype, center=centre, reference_rounding=F.reference_rounding,
                                       a_operand=aop)
+        lead = x.shape[:-1]
+        return {id(m): y.reshape(*lead, y.shape[-1]).to(F.compute_dtype) for m, y in zip(members, outs)}
+
+    def _stacked_factors(self, device):
+        """(key, V, s) of all members of the group stacked: one product gives every member's rank-r projection.  Kept on the
+        group until a member's parameter changes."""
+        cd = torch.bfloat16
+        group = self.activation_group
+        members = group["members"]
+        key = tuple((_pkey(m.vlinear.weight), _pkey(m.s)) for m in members) + (device,)
+        cached = group.get("stacked_v")
+        if cached is None or cached[0] != key:
+            cached = (key, torch.cat([m.vlinear.weight.to(cd) for m in members], dim=0),
+                      torch.cat([m.s.to(cd) for m in members], dim=0))
+            group["stacked_v"] = cached
+        return cached
+
+    def _forward_group_tiled(self, x: torch.Tensor, shared_input, members, packed):
+        """_forward_group at prefill size (256 rows or more): one pass over x for all projections, one launch of the tiled GEMM
+        for all products, the same arithmetic as member by member (_MetisFusedFunction.forward)."""
+        F = LinearLowbitFunction
+        cd = torch.bfloat16
+        centered = isinstance(shared_input, CenteredNVFP4)
+        px = shared_input.residual if centered else shared_input
+        in_operand = centered and all(F._mean_in_operand(shared_input, p) for p in packed)
+        rounding = F.reference_rounding and (in_operand or not centered)
+        if (not ops.tiled_group_applies(px, packed, rounding)
+                or (centered and not in_operand and any(F._mean_in_operand(shared_input, p) or p.rht is not None for p in packed))):
+            return None
+        x2 = _flat2d(x).to(cd)
+        _, v, s = self._stacked_factors(x2.device)
+        _, t_all = ops.lowrank_project(x2, v, s)
+        f32 = F.compute_dtype == torch.float32
+        calls, c0 = [], 0
+        for m, p_res in zip(members, packed):
+            r = m.args.forward_svd_rank
+            bias = m.warmup_linear.bias
+            if centered and not in_operand:
+                w_mean = ops.matvec(p_res, shared_input.center32)          # the mean's share rides in a binary32 bias
+                bias = w_mean if bias is None else w_mean + m._bias_as(torch.float32)
+            elif bias is not None:
+                bias = m._bias_as(torch.float32 if f32 else cd)
+            calls.append((p_res, t_all[:, c0:c0 + r], m.ulinear.weight.to(cd), bias))
+            c0 += r
+        outs = ops.linear_fwd_tiled_grouped(px, calls, out_dtype=torch.float32 if f32 else torch.bfloat16,
+                                            center=shared_input.mean if in_operand else None, reference_rounding=rounding)
         lead = x.shape[:-1]
         return {id(m): y.reshape(*lead, y.shape[-1]).to(F.compute_dtype) for m, y in zip(members, outs)}
 

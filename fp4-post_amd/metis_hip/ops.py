@@ -5,6 +5,7 @@ PyTorch is used only to own device memory and streams.
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 from dataclasses import dataclass
 
@@ -822,8 +823,9 @@ def gemm_tiled(ax: torch.Tensor, a_unit: torch.Tensor, bx: torch.Tensor, b_unit:
 def linear_fwd_tiled(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None = None, u: torch.Tensor | None = None,
                      bias: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16,
                      a_tiled: torch.Tensor | None = None, reference_rounding: bool = False,
-                     split_k: bool = True, center: torch.Tensor | None = None) -> torch.Tensor:
+                     split_k: bool = True, center: torch.Tensor | None = None, batch: "_TiledBatch | None" = None) -> torch.Tensor:
     """linear_fwd on tiled 16-bit expansions: b's is cached on b when b is persistent, a's is made here unless given.
+    batch: the product is queued there and its output, returned, is filled when the batch runs (linear_fwd_tiled_grouped).
 
     reference_rounding (both operands packed in bf16 arithmetic): operands are the reference's bf16 dequantized
     values and the epilogue rounds where the reference's all-bf16 forward rounds; otherwise exact products.
@@ -840,8 +842,86 @@ def linear_fwd_tiled(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None =
         raise ValueError("a centre inside the operand belongs to reference_rounding")
     bx = expand_tiled(b, cache=b.persistent, mode=mode)
     ax = a_tiled if a_tiled is not None else expand_tiled(a, cache=a.shared, mode=mode, center=center)
+    if batch is not None:
+        return batch.add(bx, b, t, u, bias)
     return gemm_tiled(ax, a.unit, bx, b.unit, a.rows, b.rows, a.cols, mode=mode, t=t, u=u, bias=bias, out_dtype=out_dtype,
                       split_k=split_k)
+
+
+def tiled_group_applies(a: PackedNVFP4, weights, reference_rounding: bool) -> bool:
+    """Whether linear_fwd would run every product of this activation with `weights` on the tiled kernel in one format, so
+    that linear_fwd_tiled_grouped can run them in one launch: 256 rows or more, all of them in the reference's bf16
+    roundings, or all of them exact (cached weights with a kept expansion, or weights in the rotated domain)."""
+    if not (a.rows >= 256 and a.cols % 32 == 0 and a.rht is None and 0 < len(weights) <= 4 and all(b.cols == a.cols for b in weights)):
+        return False
+    rounded = [reference_rounding and a.mode == MODE_PB16 and b.mode == MODE_PB16 for b in weights]
+    return all(rounded) or (not any(rounded) and all(b.rht is not None or _tiled_applies(a, b) for b in weights))
+
+
+def linear_fwd_tiled_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.bfloat16, center: torch.Tensor | None = None,
+                             reference_rounding: bool = False) -> list[torch.Tensor]:
+    """[linear_fwd_tiled(a, b, t=t, u=u, bias=bias, ...) for (b, t, u, bias) in members] in one launch: a projection group at
+    prefill size (tiled_group_applies).  t may be a column slice of a stacked projection.  center: as linear_fwd_tiled."""
+    if not tiled_group_applies(a, [m[0] for m in members], reference_rounding):
+        raise ValueError("linear_fwd_tiled_grouped: outside the call's domain (see tiled_group_applies)")
+    mode = MODE_PB16 if (reference_rounding and a.mode == MODE_PB16 and members[0][0].mode == MODE_PB16) else MODE_P32
+    if center is not None and mode != MODE_PB16:
+        raise ValueError("a centre inside the operand belongs to reference_rounding")
+    ax = expand_tiled(a, cache=False, mode=mode, center=center)
+    batch = _TiledBatch(a, ax, len(members), out_dtype, mode)
+    outs = [linear_fwd_tiled(a, b, t=t, u=u, bias=bias, out_dtype=out_dtype, a_tiled=ax, reference_rounding=mode == MODE_PB16, center=center,
+                             batch=batch) for b, t, u, bias in members]
+    batch.run()
+    return outs
+
+
+class _TiledBatch:
+    """Products of one tiled activation that run as one launch."""
+
+    def __init__(self, a: PackedNVFP4, ax: torch.Tensor, count: int, out_dtype: torch.dtype, mode: int):
+        self.a, self.ax, self.out_dtype, self.mode = a, ax, out_dtype, mode
+        self.members = (_lib.LinearMember * count)()
+        self.rows: list[int] = []
+        self.keep: list = []                                       # until the launch is enqueued
+
+    def add(self, bx, b, t, u, bias) -> torch.Tensor:
+        M = self.a.rows
+        r = ldt = 0
+        if t is not None:
+            t, u = t.to(torch.bfloat16), u.to(torch.bfloat16).contiguous()
+            r = t.shape[1]
+            if t.shape != (M, r) or u.shape != (b.rows, r):
+                raise ValueError("low-rank operands must be t[M, r], u[N, r]")
+            if t.stride(1) != 1 or t.stride(0) % 8 or t.data_ptr() % 16:
+                t = t.contiguous()
+            ldt = t.stride(0)
+        bias_f32 = bias is not None and bias.dtype == torch.float32
+        if bias is not None:
+            bias = bias.contiguous() if bias_f32 else bias.to(torch.bfloat16).contiguous()
+        out = torch.empty(M, b.rows, dtype=self.out_dtype, device=self.ax.device)
+        self.members[len(self.rows)] = _lib.LinearMember(
+            bx.data_ptr(), None, b.unit.data_ptr(), None if t is None else t.data_ptr(), None if u is None else u.data_ptr(), r,
+            None if bias is None else bias.data_ptr(), out.data_ptr(), b.rows, int(bias_f32), ldt, None)
+        self.rows.append(b.rows)
+        self.keep += [bx, t, u, bias]
+        return out
+
+    def run(self) -> None:
+        a, dev = self.a, self.ax.device
+        need = _tiled_group_workspace_bytes(a.rows, a.cols, tuple(self.rows), dev.index or 0)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+        rc = load().metis_linear_fwd_tiled_grouped(self.ax.data_ptr(), a.unit.data_ptr(), a.rows, a.cols, ctypes.cast(self.members, ctypes.c_void_p),
+                                                   len(self.rows), DTYPE_F32 if self.out_dtype == torch.float32 else DTYPE_BF16, self.mode,
+                                                   None if ws is None else ws.data_ptr(), need, _stream())
+        check(rc, "metis_linear_fwd_tiled_grouped", (a.rows, a.cols, self.rows))
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiled_group_workspace_bytes(M: int, K: int, ns: tuple, device_index: int) -> int:
+    arr = (_lib.LinearMember * len(ns))()
+    for i, n in enumerate(ns):
+        arr[i].N = n
+    return int(load().metis_linear_tiled_grouped_workspace_bytes(M, K, ctypes.cast(arr, ctypes.c_void_p), len(ns)))
 
 
 def rmsnorm_quantize(x: torch.Tensor, gamma: torch.Tensor, eps: float, mode: int = MODE_P32,
@@ -979,7 +1059,6 @@ def _lowrank_workspace_bytes(M: int, R: int, K: int) -> int:
 @functools.lru_cache(maxsize=4096)
 def _grouped_plan(M: int, K: int, ns: tuple, device_index: int) -> tuple[int, bool]:
     """(split-K scratch bytes, whether a centre can ride inside the launch) of a grouped call; shape-only queries."""
-    import ctypes
     arr = (_lib.LinearMember * len(ns))()
     for i, n in enumerate(ns):
         arr[i].N = n
@@ -1271,7 +1350,6 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
 
     a_operand: decode_operand(a, MODE_PB16, center) when the caller has it already (project_and_operand); read only
     where grouped_operand_applies says the call reads ready operands."""
-    import ctypes
     M, K = a.rows, a.cols
     dev = a.codes.device
     rounded = (reference_rounding and (center is None or center.dtype == torch.bfloat16) and a.mode == MODE_PB16

@@ -620,6 +620,19 @@ typedef struct metis_linear_member {
 /* sizeof(metis_linear_member) as the library was built: a caller compiled against another revision of this header
  * compares it with its own before passing member arrays (a mismatch would make the library read past the caller's array). */
 size_t metis_linear_member_size(void);
+/*
+ * metis_linear_fwd_tiled for a projection group at prefill size: one tiled activation [M, K] against up to four tiled weights in
+ * one launch (their 256-wide tile columns end to end, one partly filled last round instead of one per weight).  members[i]:
+ * b_codes = the tiled operand of metis_nvfp4_expand_tiled, b_unit, t / u / r / ldt (any ldt % 8 == 0 >= r here), bias, out, N;
+ * b_scales and b_decode are not read.  Result i is that of metis_linear_fwd_tiled with the same operands; K is split as for one
+ * product with the sum of the tile columns, so a split sum may be grouped differently.
+ *   limits     as metis_linear_fwd_tiled; count 1 .. 4; N > 0
+ *   workspace  metis_linear_tiled_grouped_workspace_bytes (0: not split), 16-byte aligned, no initialisation; NULL = never split
+ */
+size_t metis_linear_tiled_grouped_workspace_bytes(int64_t M, int64_t K, const metis_linear_member *members, int count);
+int metis_linear_fwd_tiled_grouped(const void *a_xt, const float *a_unit, int64_t M, int64_t K,
+                                   const metis_linear_member *members, int count, int out_dtype, int mode,
+                                   void *workspace, size_t workspace_bytes, void *stream);
 /* A packed weight [N, K] in the decode layout, derived data to be cached beside the packed form (the reference caches
  * its dequantized weight the same way, src/Metis/Metis/bitlinear.py:563-589): 0.5625 B per element as packed, rows
  * grouped in tiles of 32 and K in steps of 256 so that every load instruction of a wave of the decode-sized kernel

@@ -633,6 +633,43 @@ def test_rank_r_projection_at_training_sizes(M, R, K):
     assert torch.equal(ops.lowrank_project(wide[:, :K], v), xv)
 
 
+@pytest.mark.parametrize("M,K,ns,mode", [(256, 128, (256,), 0), (257, 1536, (1536, 256, 260), 0), (411, 1536, (1536, 256, 256), 1), (300, 2048, (100, 4), 1),
+                                         (1000, 512, (8960, 8960), 0), (1000, 512, (8960, 8960), 1), (4100, 192, (3584, 512, 516, 256), 0)])
+def test_projection_group_at_prefill_size_in_one_launch(M, K, ns, mode):
+    """metis_linear_fwd_tiled_grouped against the products one by one: narrow and ragged members, four of them, split and
+    unsplit tiles, low-rank terms in columns of a stacked projection, bias in either type.  Exact mode: the same exact products
+    summed in another order (K 2^-23 of the sum of magnitudes); bf16 mode: one bf16 rounding apart at most where that moves one."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(6300 + M)
+    r = 32
+    px = ops.quantize(torch.randn(M, K, generator=g, device="cuda").bfloat16(), mode)
+    stacked = torch.randn(M, r * len(ns), generator=g, device="cuda").bfloat16()
+    members = []
+    for i, n in enumerate(ns):
+        pw = ops.quantize((torch.randn(n, K, generator=g, device="cuda") / K ** 0.5).bfloat16(), mode)
+        pw.persistent = True
+        u = (torch.randn(n, r, generator=g, device="cuda") / r).bfloat16() if i != 1 else None
+        bias = None if i == 2 else torch.randn(n, generator=g, device="cuda").to(torch.bfloat16 if (mode or i) else torch.float32)
+        members.append((pw, stacked[:, i * r:(i + 1) * r] if u is not None else None, u, bias))
+    assert ops.tiled_group_applies(px, [m[0] for m in members], mode == 1)
+    got = ops.linear_fwd_tiled_grouped(px, members, out_dtype=torch.float32, reference_rounding=mode == 1)
+    xd = px.dequantize(torch.float32).double()
+    for (pw, t, u, bias), y in zip(members, got):
+        one = ops.linear_fwd_tiled(px, pw, t=None if t is None else t.contiguous(), u=u, bias=bias, out_dtype=torch.float32, reference_rounding=mode == 1)
+        assert y.shape == one.shape == (M, pw.rows)
+        mag = xd.abs() @ pw.dequantize(torch.float32).double().abs().T
+        if u is not None:
+            mag = mag + t.double().abs() @ u.double().abs().T
+        if bias is not None:
+            mag = mag + bias.double().abs()
+        bound = mag * ((K + r) * 2.0 ** -23) + (mag * 2.0 ** -7 if mode else 0.0)
+        assert bool(((y.double() - one.double()).abs() <= bound).all())
+        assert mode == 0 or float((y != one).float().mean()) <= 0.02
+    for bad in (px, ops.quantize(torch.zeros(255, K, dtype=torch.bfloat16, device="cuda"), mode)):
+        with pytest.raises(ValueError):
+            ops.linear_fwd_tiled_grouped(bad, members * 5 if bad is px else members, reference_rounding=mode == 1)
+
+
 @pytest.mark.parametrize("M,R,K", [(256, 96, 64), (257, 192, 192), (411, 256, 1536), (16385, 192, 128), (16384, 64, 192), (20000, 32, 320),
                                    (2103, 64, 18944), (300, 128, 4160), (16400, 96, 256)])
 def test_rank_r_projection_tiles_of_32_and_64_rows(M, R, K):
