@@ -198,9 +198,16 @@ __device__ __forceinline__ uint2 encode_rne_wide(const float (&v)[kBlock], float
 // compress/round/expand sequence is a function of the bf16 value q alone, and over all bf16 q in
 // [0, 13] it equals the round-to-nearest-even conversion onto the E2M1 grid except at q = 5+1ulp,
 // 7-1ulp and 10+1ulp (bf16 ulps), where its intermediate roundings land on the tie 5, 7, 10.
-// div3() followed by the bf16 rounding gives exactly bf16(RN(x / h)) for bf16 x and h: a binary32
-// quotient that is not exactly representable stays at least 2^-17 (relative) away from every bf16
-// midpoint, far more than div3's error.  Checked on the host for every (h, x) pair of bf16 values.
+// bf16(RN(x / h)) for bf16 x and h is had from any quotient that is exact when x / h is a binary32 number and within
+// 2^-17 of it otherwise: a quotient that is no binary32 number stays at least 2^-17 (relative) away from every bf16
+// midpoint.  div3() is one (checked on the host for every (h, x) pair of bf16 values); quot2() is another, in two
+// operations: hi + lo = 1/h to 2^-46 and one rounding at the end, for every h whose reciprocal and its remainder are
+// normal numbers (2^-31 <= h < 2^60 here: the scalar is at least 1e-9).
+// The three exceptions are moved onto their ties two at a time in packed 16-bit integer arithmetic: one ulp down for q in
+// [4, 6) and [8, 12), one up in [6, 8).  The other values there move too, but only within their code: 4 -> 4 - 1ulp and
+// 5 -> 5 - 1ulp stay above 3.5 and below 5, 7 -> 7 + 1ulp above 7, 8 -> 8 - 1ulp above 7.  The converter takes the signed
+// bf16 pair.  (Both elements apart -- unpacked, compared with the three values, the sign masked in -- this was 27 vector
+// instructions a pair in place of 14: 18944 x 3584 with its scale bytes 45.3 -> 38.2 us, the 8192 x 4096 round trip 37.9 -> 35.7.)
 __device__ __forceinline__ float nudge_pb16(float q)          // q >= 0
 {
     q = (q == 5.03125f) ? 5.0f : q;
@@ -208,39 +215,45 @@ __device__ __forceinline__ float nudge_pb16(float q)          // q >= 0
     q = (q == 10.0625f) ? 10.0f : q;
     return q;
 }
-__device__ __forceinline__ uint2 encode_rne_pb16(const float (&v)[kBlock], float s)
+typedef unsigned short ushort2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t nudge_pair_pb16(uint32_t qq)       // two signed bf16 quotients
 {
-    const float h = 0.5f * s;                                 // bf16(s / 2), exact
-    const float rh = __builtin_amdgcn_rcpf(h);                // 1 ulp
-    uint32_t w[2] = {0u, 0u}, sg[2] = {0u, 0u};
-#pragma unroll
-    for (int j = 0; j < kBlock; j += 2) {
-        // signed quotients: div3 turns a -0.0 input into +0.0, which is the reference's sign(x) = 0
-        const uint32_t qq = rb_pair(div3(v[j], h, rh), div3(v[j + 1], h, rh));
-        const float q0 = nudge_pb16(fabsf(bf16_lo(qq))), q1 = nudge_pb16(fabsf(bf16_hi(qq)));
-        sg[j >> 3] |= (((qq >> 12) & 0x8u) | ((qq >> 24) & 0x80u)) << (4 * (j & 7));
-        // magnitude code = E2M1(q / 2): the converter divides by the power of two given as its scale
-        switch ((j >> 1) & 3) {
-        case 0: w[j >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[j >> 3], q0, q1, 2.0f, 0); break;
-        case 1: w[j >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[j >> 3], q0, q1, 2.0f, 1); break;
-        case 2: w[j >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[j >> 3], q0, q1, 2.0f, 2); break;
-        default: w[j >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[j >> 3], q0, q1, 2.0f, 3); break;
-        }
-    }
-    return make_uint2(w[0] | sg[0], w[1] | sg[1]);
+    const ushort2_t p = __builtin_bit_cast(ushort2_t, qq & 0x7fff7fffu);
+    const uint32_t above = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(p, (ushort2_t)(unsigned short)0x407f));
+    uint32_t t, r;                                                       // t: 1 where q >= 4
+    // (assembly: the compiler turns the packed minimum into compares and selects, half by half)
+    asm("v_pk_min_u16 %0, %1, %2" : "=v"(t) : "v"(above), "s"(0x00010001u));
+    const uint32_t up = t & __builtin_bit_cast(uint32_t, (ushort2_t)(p >> (ushort2_t)(unsigned short)6));   // 1 where q in [6, 8)
+    asm("v_pk_mad_i16 %0, %1, %2, %3 clamp" : "=v"(r) : "v"(up), "s"(0x00020002u), "v"(__builtin_bit_cast(uint32_t, p)));   // (saturates: a NaN stays one)
+    r = __builtin_bit_cast(uint32_t, (ushort2_t)(__builtin_bit_cast(ushort2_t, r) - __builtin_bit_cast(ushort2_t, t)));
+    return r | (qq & 0x80008000u);
 }
-
-// the same for N elements (8: half a block, one packed word)
+// N elements of a block with scalar s (8: half a block, one packed word)
 template <int N>
 __device__ __forceinline__ void encode_rne_pb16_n(const float (&v)[N], float s, uint32_t (&out)[N / 8])
 {
-    const float h = 0.5f * s;
-    const float rh = __builtin_amdgcn_rcpf(h);
+    typedef __bf16 bf16_pair_t __attribute__((ext_vector_type(2)));
+    const float h = 0.5f * s;                                 // bf16(s / 2), exact
+    if (s < 0x1p60f) {
+        const SplitReciprocal r = split_reciprocal(h);
+#pragma unroll
+        for (int k = 0; k < N / 8; ++k) {
+            uint32_t w = 0u;
+#define METIS_PAIR(P) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(w, __builtin_bit_cast(bf16_pair_t, \
+            nudge_pair_pb16(rb_pair(quot2(v[8 * k + 2 * P], r), quot2(v[8 * k + 2 * P + 1], r)))), 2.0f, P)   /* divides by its scale */
+            METIS_PAIR(0); METIS_PAIR(1); METIS_PAIR(2); METIS_PAIR(3);
+#undef METIS_PAIR
+            out[k] = w;
+        }
+        return;
+    }
+    const float rh = __builtin_amdgcn_rcpf(h);                // scalars of 2^60 and more, infinite or NaN: element by element
 #pragma unroll
     for (int k = 0; k < N / 8; ++k) {
         uint32_t w = 0u, sg = 0u;
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
+            // signed quotients: div3 turns a -0.0 input into +0.0, which is the reference's sign(x) = 0
             const uint32_t qq = rb_pair(div3(v[8 * k + j], h, rh), div3(v[8 * k + j + 1], h, rh));
             const float q0 = nudge_pb16(fabsf(bf16_lo(qq))), q1 = nudge_pb16(fabsf(bf16_hi(qq)));
             sg |= (((qq >> 12) & 0x8u) | ((qq >> 24) & 0x80u)) << (4 * j);
@@ -253,6 +266,12 @@ __device__ __forceinline__ void encode_rne_pb16_n(const float (&v)[N], float s, 
         }
         out[k] = w | sg;
     }
+}
+__device__ __forceinline__ uint2 encode_rne_pb16(const float (&v)[kBlock], float s)
+{
+    uint32_t w[2];
+    encode_rne_pb16_n<kBlock>(v, s, w);
+    return make_uint2(w[0], w[1]);
 }
 
 // One v_cvt_scalef32_sr_pk_fp4_f32: converts (q0, q1) / 2^MODE with stochastic rounding into byte `byte` of w
@@ -335,7 +354,6 @@ __device__ __forceinline__ float block_amax(const float (&v)[kBlock])
 }
 
 // maximum magnitude of the 16 packed bf16 values, computed on the bit patterns (two per dword)
-typedef unsigned short ushort2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float block_amax_packed(const uint4 a, const uint4 b)
 {
     const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};

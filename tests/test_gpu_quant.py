@@ -688,3 +688,19 @@ def test_column_packing_of_a_ragged_row_count_equals_packing_a_filled_up_copy(ro
         ops.quantize(x, 0, pad_rows=pad)                          # row blocks take the tensor as it is
     with pytest.raises(ValueError):
         ops.quantize(x, 0, col=True, pad_rows=rows + 16 - rows % 16 + 3)
+
+
+@pytest.mark.parametrize("top", [0x0001, 0x0c80, 0x3000, 0x4040, 0x5d7f, 0x5e80, 0x7e00])
+def test_bf16_arithmetic_encoder_on_every_quotient_of_a_binade(ops, top):
+    """Every bf16 element of the twelve binades below each of 128 block maxima, both signs, in bf16 arithmetic: the codes of the C
+    oracle, for maxima of every size (subnormal ones, and the scalars of 2^60 and more that take the other quotient)."""
+    from oracle import c_oracle as C
+    am = torch.arange(top, top + 128, dtype=torch.int32).clamp(max=0x7f7f)
+    off = torch.arange(1530, dtype=torch.int32)
+    e = (am[:, None] - off[None, :]).clamp_min(0) | ((off[None, :] & 1) << 15)
+    e = e.reshape(128, 102, 15)
+    x = torch.cat([am[:, None, None].expand(-1, 102, 1), e], 2).reshape(128, 1632).to(torch.int16).view(torch.bfloat16)
+    for y in (x, x.flip(1).contiguous()):
+        codes, scales, unit, _ = C.nvfp4_pack(y, 1)
+        _check_packed(ops.quantize(y.cuda(), 1), codes, scales, unit, hex(top))
+        _check_packed(ops.quantize(y.T.contiguous().cuda(), 1, col=True), codes, scales, unit, hex(top))
