@@ -106,6 +106,8 @@ __device__ __forceinline__ float code_literal(float ax, float h, float u)
 
 // Philox4x32-10 (Salmon et al., SC'11): counter-based generator for stochastic rounding.
 struct Philox {
+    // one three-input operation (truth table 0x96 = parity)
+    static __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { return (uint32_t)__builtin_amdgcn_bitop3_b32(a, b, c, 0x96); }
     static __device__ __forceinline__ uint4 draw(uint64_t ctr, uint64_t seed)
     {
         uint32_t c0 = (uint32_t)ctr, c1 = (uint32_t)(ctr >> 32), c2 = 0u, c3 = 0u;
@@ -115,7 +117,7 @@ struct Philox {
             // both halves of each product from one 32 x 32 -> 64 bit multiply-add (integer multiplies run at quarter rate)
             const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
             const uint32_t h0 = (uint32_t)(p0 >> 32), l0 = (uint32_t)p0, h1 = (uint32_t)(p1 >> 32), l1 = (uint32_t)p1;
-            c0 = h1 ^ c1 ^ k0; c1 = l1; c2 = h0 ^ c3 ^ k1; c3 = l0;
+            c0 = xor3(h1, c1, k0); c1 = l1; c2 = xor3(h0, c3, k1); c3 = l0;
             k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
         }
         return make_uint4(c0, c1, c2, c3);

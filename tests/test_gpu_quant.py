@@ -704,3 +704,21 @@ def test_bf16_arithmetic_encoder_on_every_quotient_of_a_binade(ops, top):
         codes, scales, unit, _ = C.nvfp4_pack(y, 1)
         _check_packed(ops.quantize(y.cuda(), 1), codes, scales, unit, hex(top))
         _check_packed(ops.quantize(y.T.contiguous().cuda(), 1, col=True), codes, scales, unit, hex(top))
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 8), (32, 64), (272, 72), (528, 200), (256, 100), (288, 68), (2112, 1536)])
+@pytest.mark.parametrize("center", [False, True])
+def test_column_blocks_in_whole_slabs_and_element_by_element(ops, rows, cols, center):
+    """The column quantizers with 16-byte loads and without (columns that are no multiple of 8): the packing of the transposed
+    tensor's rows, round to nearest, and the stochastic packing of the transposed copy's blocks, drawn alike."""
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x = torch.randn(rows, cols, generator=g, device="cuda").bfloat16()
+    for mode in (0, 1):
+        cen = torch.randn(cols, generator=g, device="cuda").to(torch.float32 if mode == 0 else torch.bfloat16) if center else None
+        p = ops.quantize(x, mode, col=True, center=cen)
+        dense = x if cen is None else (x.float() - cen.float()).to(torch.float32 if mode == 0 else torch.bfloat16)
+        want = ops.quantize(dense.T.contiguous(), mode)
+        assert torch.equal(p.codes, want.codes) and torch.equal(p.scales, want.scales) and torch.equal(p.unit, want.unit)
+        sr = ops.quantize(x, mode, col=True, sr=True, seed=7, offset=3, center=cen)
+        want = ops.quantize(dense.T.contiguous(), mode, sr=True, seed=7, offset=3)
+        assert torch.equal(sr.codes, want.codes) and torch.equal(sr.scales, want.scales)
