@@ -392,7 +392,7 @@ class LinearLowbitFunction(torch.autograd.Function):
         return F.quantize_input(input_, mean_cache=mean_cache, cache_key=cache_key)
 
     @staticmethod
-    def _packed_grads(dy2, x2, pw_col, center_x, gx_dtype, gw_dtype, gx_lowrank=None):
+    def _packed_grads(dy2, x2, pw_col, center_x, gx_dtype, gw_dtype, gx_lowrank=None, center_x32=None):
         """(grad_input [L, K], grad_weight [N, K]) on packed operands.  dgrad contracts over N, wgrad over tokens.
 
         Direct mode: dY^ = SR-Q(dY).  Mean mode (enable_backward_svd): dY^ = 1 me_dy^T + SR-Q(dY - me_dy)
@@ -402,11 +402,17 @@ class LinearLowbitFunction(torch.autograd.Function):
             gX = R_dy W^ + 1 (W^^T me_dy)^T
             gW = R_dy^T R_x + (sum_l R_dy) center_x^T + me_dy (sum_l R_x + L center_x)^T
         gx_lowrank = (t [L, r], u [K, r]) adds t u^T to grad_input inside the same launch (the rank-r branch's share).
+        center_x32: center_x as float32 when the caller has it (the matrix-vector products read binary32: each use of the
+        bf16 one is a conversion launch).
         """
         F = LinearLowbitFunction
         cd = F.compute_dtype
         qg, qi = F.q_backward_outputgrad, F.q_backward_input
-        me_dy = F._token_mean(dy2) if F.enable_backward_svd else None
+        me_dy, me_dy32 = F._token_mean2(dy2) if F.enable_backward_svd else (None, None)
+        if me_dy32 is None:
+            me_dy32 = me_dy
+        if center_x32 is None:
+            center_x32 = center_x
         # The weight gradient contracts over tokens in steps of 32.  A ragged token count is padded, not sent down another
         # code path: the column quantizers take rows beyond the tensor's own as equal to the centre (zero in direct mode),
         # whose residual is zero, so they change no block maximum, no tensor unit and no sum.  The input gradient
@@ -425,7 +431,7 @@ class LinearLowbitFunction(torch.autograd.Function):
             gx = ops.linear_dgrad(p_dy, pw_col, out_dtype=gx_dtype)
         else:
             lt, lu = gx_lowrank if gx_lowrank is not None else (None, None)
-            gx = ops.linear_fwd(p_dy, pw_col, t=lt, u=lu, bias=None if me_dy is None else ops.matvec(pw_col, me_dy),
+            gx = ops.linear_fwd(p_dy, pw_col, t=lt, u=lu, bias=None if me_dy is None else ops.matvec(pw_col, me_dy32),
                                 out_dtype=gx_dtype)
         if p_dyt is None:
             p_dyt = qg.pack(dy2, col=True, arith=cd, center=me_dy, **more)
@@ -436,10 +442,10 @@ class LinearLowbitFunction(torch.autograd.Function):
         # the rank-one terms ride in the GEMM's low-rank operands (three bf16 terms per factor: binary32 precision)
         first = second = None
         if center_x is not None:
-            first = (ops.matvec(p_dyt), center_x)
+            first = (ops.matvec(p_dyt), center_x32)
         if me_dy is not None:
-            tail = ops.matvec(p_xt) if center_x is None else ops.matvec(p_xt, z=center_x, beta=float(L))
-            second = (me_dy, tail)
+            tail = ops.matvec(p_xt) if center_x is None else ops.matvec(p_xt, z=center_x32, beta=float(L))
+            second = (me_dy32, tail)
         t, u = ops.rank_one_operands(p_dyt.rows, p_xt.rows, first or second, second if first else None)
         return gx, ops.linear_fwd(p_dyt, p_xt, t=t, u=u, out_dtype=gw_dtype)
 
@@ -556,7 +562,7 @@ class LinearLowbitFunction(torch.autograd.Function):
             # activation (its factors are randomized and cannot be derived again), kept only when autograd will ask.
             ctx.pw = quantized_weight
             ctx.weight_ref = weight
-            ctx.center = None
+            ctx.center = ctx.center32 = None
             ctx.lowrank = True
             saved = quantized_input.dense if quantized_input.dense is not None else input_.new_empty(0)
             ctx.save_for_backward(saved, bias if bias is not None else input_.new_empty(0))
@@ -568,16 +574,16 @@ class LinearLowbitFunction(torch.autograd.Function):
             ctx.pw = quantized_weight
             ctx.weight_ref = weight
             ctx.save_for_backward(input_, bias if bias is not None else input_.new_empty(0))
-            ctx.center = None
+            ctx.center = ctx.center32 = None
             out_dtype = torch.float32 if F.compute_dtype == torch.float32 else torch.bfloat16
             if isinstance(quantized_input, CenteredNVFP4) and F._mean_in_operand(quantized_input, quantized_weight):
-                ctx.center = quantized_input.mean
+                ctx.center, ctx.center32 = quantized_input.mean, quantized_input.center32
                 out = ops.linear_fwd_grouped(quantized_input.residual, [(quantized_weight, None, None, bias)], out_dtype=out_dtype,
                                              center=quantized_input.mean, reference_rounding=True)[0]
                 return out.reshape(*lead, quantized_weight.rows).to(F.compute_dtype)
             if isinstance(quantized_input, CenteredNVFP4):
                 # (1 me^T + R) W^^T = R W^^T + 1 (W^ me)^T: the mean's term rides in a binary32 bias
-                ctx.center = quantized_input.mean
+                ctx.center, ctx.center32 = quantized_input.mean, quantized_input.center32
                 w_mean = ops.matvec(quantized_weight, quantized_input.mean)
                 bias = w_mean if bias is None else w_mean + bias.float()
                 quantized_input = quantized_input.residual
@@ -622,7 +628,7 @@ class LinearLowbitFunction(torch.autograd.Function):
                 pw_col = ctx.pw.transposed                    # lives as long as the (possibly cached) packed weight
                 if pw_col is None:
                     pw_col = ctx.pw.transposed = F.q_forward_weight.pack(ctx.weight_ref, col=True, arith=cd)
-                gx, gw = F._packed_grads(dy2, x2, pw_col, ctx.center, gx_dtype, gw_dtype)
+                gx, gw = F._packed_grads(dy2, x2, pw_col, ctx.center, gx_dtype, gw_dtype, center_x32=ctx.center32)
                 return gx.reshape(*ctx.lead, gx.shape[-1]), gw, grad_bias, None, None
             grad_output = grad_output.to(F.compute_dtype)
             dy2 = _flat2d(grad_output)
@@ -718,7 +724,10 @@ class LinearLowbit(nn.Module):
             q = F._apply_hadamard_blocks(weight_compute, inverse=False)
             q = F._apply_hadamard_blocks(F.q_forward_weight.quantize_dequantize(q), inverse=True)
         elif _packable(weight_compute, F.q_forward_weight) and weight_compute.shape[0] % 4 == 0:
-            q = F.q_forward_weight.pack(weight_compute, arith=arith)
+            # packed for this one forward in the reference's bf16 roundings: its operand is expanded by a launch that forms the
+            # scale bytes anyway (any other reader has them made on first access)
+            more = {"deferred": True} if (not self.cache_quantized_weight and arith == torch.bfloat16 and F._bf16_rounding()) else {}
+            q = F.q_forward_weight.pack(weight_compute, arith=arith, **more)
         else:
             q = F.q_forward_weight.quantize_dequantize(weight_compute)
         if self.cache_quantized_weight:
@@ -766,12 +775,12 @@ class _MetisFusedFunction(torch.autograd.Function):
             else:
                 xv, t = ops.lowrank_project(x2, vb, sb)
         out_dtype = torch.float32 if F.compute_dtype == torch.float32 else torch.bfloat16
-        ctx.center = None
+        ctx.center = ctx.center32 = None
         # binary32 arithmetic keeps a binary32 bias (as LinearLowbit and the centred path do); bf16 arithmetic adds it in bf16
         gemm_bias = None if bias is None else (bias.float() if F.compute_dtype == torch.float32 else bias.to(cd))
         if isinstance(px, CenteredNVFP4):
             # mean mode: the residual branch sees 1 me^T + R
-            ctx.center = px.mean
+            ctx.center, ctx.center32 = px.mean, px.center32
             if F._mean_in_operand(px, p_res):
                 # bf16 arithmetic: the activation operand is the reference's bf16 tensor me + QDQ(x - me)
                 y = ops.linear_fwd_grouped(px.residual, [(p_res, t, u.to(cd), gemm_bias)], out_dtype=out_dtype, center=px.mean,
@@ -842,7 +851,7 @@ class _MetisFusedFunction(torch.autograd.Function):
             # the rank-r branch's share of grad_input, g_xv V, rides in the dgrad launch as its low-rank extension
             gx, g_res = F._packed_grads(dyq, xq_src, p_res_col, ctx.center, cd,
                                         torch.bfloat16 if res.dtype == torch.bfloat16 else torch.float32,
-                                        gx_lowrank=(g_xv, _MetisFusedFunction._transposed_bf16(v)))
+                                        gx_lowrank=(g_xv, _MetisFusedFunction._transposed_bf16(v)), center_x32=ctx.center32)
         else:
             gx = torch.matmul(g_xv, v.to(cd))                  # [L, K]
             cdt = F.compute_dtype
