@@ -98,7 +98,14 @@ int metis_rmsnorm_backward(const void* x, const void* grad, const void* gamma, f
 int metis_nvfp4_quant_dequant_row(const void* x, int64_t rows, int64_t cols, int mode, void* codes, void* scales, float* unit,
                                   void* out, void* workspace, size_t workspace_bytes, void* stream)
 {
+    if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16) return METIS_E_ARG;
     return quantize_dequantize_row(x, rows, cols, mode, codes, scales, unit, out, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int metis_nvfp4_quant_dequant_row_f32(const void* x, int64_t rows, int64_t cols, void* codes, void* scales, float* unit, void* out, void* workspace,
+                                      size_t workspace_bytes, void* stream)
+{
+    return quantize_dequantize_row(x, rows, cols, METIS_MODE_P32_F32, codes, scales, unit, out, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int metis_nvfp4_quant_row_static(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, void* codes, void* scales,

@@ -1013,32 +1013,51 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
 // of a wave covers consecutive bytes; the hardware converter turns two codes into their binary32 values (E2M1 = v / 2
 // with its sign).  The scale bytes of a wave's 32 blocks leave as eight dwords.
 // ---------------------------------------------------------------------------------------------
+// WIDE: a binary32 tensor (maxima parked as binary32, IEEE divisions), dequantized to binary32.
 typedef float metis_f32x2_t __attribute__((ext_vector_type(2)));
-template <int MODE>
-__global__ __launch_bounds__(256) void quant_scales_dequant_kernel(const uint32_t* __restrict__ codes, const uint16_t* __restrict__ ws_amax,
+typedef float metis_f32x4_t __attribute__((ext_vector_type(4)));
+template <int MODE, bool WIDE = false>
+__global__ __launch_bounds__(256) void quant_scales_dequant_kernel(const uint32_t* __restrict__ codes,
+                                                                   const typename std::conditional<WIDE, float, uint16_t>::type* __restrict__ ws_amax,
                                                                    const uint32_t* __restrict__ ws_gmax, uint32_t ngroups,
                                                                    uint8_t* __restrict__ scales, float* __restrict__ unit_out,
                                                                    metis_u32x4_t* __restrict__ out, uint32_t nhalves)
 {
+    static_assert(!WIDE || MODE == 0, "binary32 values imply binary32 arithmetic");
+    using amax_t = typename std::conditional<WIDE, float, uint32_t>::type;
     __shared__ float smax[4];
     const uint32_t step = gridDim.x * 256u;
     uint32_t i = blockIdx.x * 256u + threadIdx.x;               // half-block index
-    uint32_t cw = 0u, aw = 0u;
+    uint32_t cw = 0u;
+    amax_t aw = 0;
     if (i < nhalves) { cw = codes[i]; aw = ws_amax[i >> 1]; }
     float m = 0.0f;
     for (uint32_t g = threadIdx.x; g < ngroups; g += 256u) m = fmaxf(m, __uint_as_float(ws_gmax[g]));
     m = wave_max(m);
     if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = m;
     __syncthreads();
-    const float unit = tensor_unit_of<MODE>(fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])));
+    const float amax = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
+    float unit;
+    if constexpr (WIDE) unit = block_scalar_ieee(amax) / 448.0f;
+    else unit = tensor_unit_of<MODE>(amax);
     if (blockIdx.x == 0 && threadIdx.x == 0) *unit_out = unit;
     const uint32_t lane = threadIdx.x & 63u;
     while (i < nhalves) {
         const uint32_t nxt = i + step;
-        uint32_t ncw = 0u, naw = 0u;
+        uint32_t ncw = 0u;
+        amax_t naw = 0;
         if (nxt < nhalves) { ncw = codes[nxt]; naw = ws_amax[nxt >> 1]; }
-        const uint32_t byte = scale_byte_of<MODE>(aw, unit);
+        uint32_t byte;
+        if constexpr (WIDE) byte = e4m3_byte(block_scalar_ieee(aw) / unit);
+        else byte = scale_byte_of<MODE>(aw, unit);
         const float dq = rd<MODE>(e4m3_value(byte) * unit);
+        if constexpr (WIDE) {
+            metis_f32x4_t* o = reinterpret_cast<metis_f32x4_t*>(out) + 2 * (size_t)i;
+            const metis_f32x2_t v0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw, 1.0f, 0), v1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw, 1.0f, 1),
+                                v2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw, 1.0f, 2), v3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw, 1.0f, 3);
+            o[0] = (metis_f32x4_t){v0.x * dq, v0.y * dq, v1.x * dq, v1.y * dq};
+            o[1] = (metis_f32x4_t){v2.x * dq, v2.y * dq, v3.x * dq, v3.y * dq};
+        } else {
         uint32_t w[4];
 #define METIS_DQ_PAIR(J)                                                                                  \
         {                                                                                                 \
@@ -1048,6 +1067,7 @@ __global__ __launch_bounds__(256) void quant_scales_dequant_kernel(const uint32_
         METIS_DQ_PAIR(0) METIS_DQ_PAIR(1) METIS_DQ_PAIR(2) METIS_DQ_PAIR(3)
 #undef METIS_DQ_PAIR
         __builtin_nontemporal_store((metis_u32x4_t){w[0], w[1], w[2], w[3]}, out + i);
+        }
         // scale bytes: the wave's 32 blocks; lane 8 j + {0, 2, 4, 6} hold the bytes of dword j
         const uint32_t b1 = __shfl(byte, (lane & ~7u) + 2u, 64), b2 = __shfl(byte, (lane & ~7u) + 4u, 64), b3 = __shfl(byte, (lane & ~7u) + 6u, 64);
         if ((lane & 7u) == 0u) {
@@ -1275,7 +1295,7 @@ int quantize_dequantize_row(const void* x, int64_t rows, int64_t cols, int mode,
                             void* workspace, size_t workspace_bytes, hipStream_t st)
 {
     if (rows < 0 || cols < 0) return METIS_E_ARG;
-    if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16) return METIS_E_ARG;
+    if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16 && mode != METIS_MODE_P32_F32) return METIS_E_ARG;
     if (cols % kBlock) return METIS_E_SHAPE;
     if (rows == 0 || cols == 0) return METIS_OK;
     if (!x || !codes || !scales || !unit || !out) return METIS_E_ARG;
@@ -1284,14 +1304,21 @@ int quantize_dequantize_row(const void* x, int64_t rows, int64_t cols, int mode,
     Workspace ws;
     if (const int rc = carve_workspace(workspace, workspace_bytes, rows, cols, &ws)) return rc;
     const uint32_t nblocks = (uint32_t)(rows * cols / kBlock);
-    const int g1 = grid_for(nblocks, kContigPerCu);
-    if (mode == 0) launch_contig<0>(x, codes, ws, nblocks, 0u, g1, st);
+    const bool f32in = mode == METIS_MODE_P32_F32;
+    const int g1 = f32in ? grid_for(nblocks) : grid_for(nblocks, kContigPerCu);
+    if (f32in)
+        hipLaunchKernelGGL((quant_codes_kernel<0, false, true>), dim3(g1), dim3(256), 0, st, x, (uint32_t)rows, (uint32_t)cols, cols, (const void*)nullptr,
+                           (uint64_t)0, (uint64_t)0, (uint2*)codes, (void*)ws.amax, ws.gmax, nblocks, 1, (const void*)nullptr, 0u, 0u);
+    else if (mode == 0) launch_contig<0>(x, codes, ws, nblocks, 0u, g1, st);
     else launch_contig<1>(x, codes, ws, nblocks, 0u, g1, st);
     if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     const uint32_t nhalves = nblocks * 2u;
     // whole waves of 32 blocks per iteration: the stride is a multiple of 64 halves by construction (256 threads)
     const int g2 = grid_for((nhalves + 3) / 4);                 // four halves per thread
-    if (mode == 0)
+    if (f32in)
+        hipLaunchKernelGGL((quant_scales_dequant_kernel<0, true>), dim3(g2), dim3(256), 0, st, (const uint32_t*)codes, (const float*)ws.amax, ws.gmax,
+                           (uint32_t)g1, (uint8_t*)scales, unit, (metis_u32x4_t*)out, nhalves);
+    else if (mode == 0)
         hipLaunchKernelGGL((quant_scales_dequant_kernel<0>), dim3(g2), dim3(256), 0, st, (const uint32_t*)codes, ws.amax, ws.gmax, (uint32_t)g1,
                            (uint8_t*)scales, unit, (metis_u32x4_t*)out, nhalves);
     else

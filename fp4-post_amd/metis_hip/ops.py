@@ -327,6 +327,27 @@ def quantize_dequantize(x: torch.Tensor, mode: int = MODE_P32) -> tuple[PackedNV
     return PackedNVFP4(codes, scales, unit, rows, cols, mode), out
 
 
+def quantize_dequantize_f32(x: torch.Tensor) -> tuple[PackedNVFP4, torch.Tensor]:
+    """quantize_dequantize of a binary32 tensor in binary32 arithmetic: (quantize(x), its dequantized binary32 tensor)."""
+    if x.dtype != torch.float32 or not x.is_cuda:
+        raise ValueError("quantize_dequantize_f32: a float32 device tensor")
+    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x2 if x2.is_contiguous() else x2.contiguous()
+    rows, cols = x2.shape
+    if cols % BLOCK:
+        raise ValueError(f"NVFP4 block shape (1, 16) does not divide tensor shape {tuple(x.shape)}")
+    dev = x2.device
+    codes = torch.empty(rows, cols // 2, dtype=torch.uint8, device=dev)
+    scales = torch.empty(rows, cols // BLOCK, dtype=torch.uint8, device=dev)
+    unit = torch.empty(1, dtype=torch.float32, device=dev)
+    out = torch.empty(rows, cols, dtype=torch.float32, device=dev)
+    ws = _workspace(rows, cols, dev)
+    rc = load().metis_nvfp4_quant_dequant_row_f32(x2.data_ptr(), rows, cols, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(), out.data_ptr(),
+                                                  ws.data_ptr(), ws.numel(), _stream())
+    check(rc, "metis_nvfp4_quant_dequant_row_f32", x.shape)
+    return PackedNVFP4(codes, scales, unit, rows, cols, MODE_P32), out
+
+
 def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tensor, mode: int = MODE_P32,
                               dense: bool = False) -> tuple[PackedNVFP4, torch.Tensor | None]:
     """The packed residual QDQ(x - ker) with ker = us @ vt formed in registers (the "svd" mode of the activation

@@ -95,6 +95,9 @@ int metis_nvfp4_quant_row(const void *x, int64_t rows, int64_t cols, int64_t ld,
 int metis_nvfp4_quant_dequant_row(const void *x, int64_t rows, int64_t cols, int mode, void *codes,
                                   void *scales, float *unit, void *out, void *workspace,
                                   size_t workspace_bytes, void *stream);
+/* The same for a binary32 tensor: x and out float [rows, cols], contiguous, binary32 arithmetic (METIS_MODE_P32_F32). */
+int metis_nvfp4_quant_dequant_row_f32(const void *x, int64_t rows, int64_t cols, void *codes, void *scales,
+                                      float *unit, void *out, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * metis_nvfp4_quant_row without a workspace argument and without any allocation: the scratch (per-workgroup

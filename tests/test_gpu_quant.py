@@ -722,3 +722,18 @@ def test_column_blocks_in_whole_slabs_and_element_by_element(ops, rows, cols, ce
         sr = ops.quantize(x, mode, col=True, sr=True, seed=7, offset=3, center=cen)
         want = ops.quantize(dense.T.contiguous(), mode, sr=True, seed=7, offset=3)
         assert torch.equal(sr.codes, want.codes) and torch.equal(sr.scales, want.scales)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 16), (3, 48), (77, 1536), (1000, 4096), (4099, 272)])
+def test_binary32_round_trip_from_one_call(ops, rows, cols):
+    """metis_nvfp4_quant_dequant_row_f32: the bytes of the quantizer and the values of its dequantization, ragged tails included."""
+    from metis_hip import quant_func
+    x = _f32_valued(rows + cols, rows, cols).cuda()
+    x.view(-1)[::97] = -0.0
+    want = ops.quantize(x, 0)
+    p, out = ops.quantize_dequantize_f32(x)
+    torch.cuda.synchronize()
+    assert torch.equal(p.codes, want.codes) and torch.equal(p.scales, want.scales) and torch.equal(p.unit, want.unit)
+    assert same_bits(out.cpu(), ops.dequantize(want, torch.float32).cpu())
+    q = quant_func["nvfp4e2m1bnosr"]
+    assert same_bits(q.quantize_dequantize(x).cpu(), out.cpu())
