@@ -36,6 +36,13 @@ from .quant import (Cast2Fp32, Cast2NVFp4e2m1Block, Cast2NVFp4e2m1BlockNOSR, Qua
 __all__ = ["LinearLowbitFunction", "LinearLowbit", "BitLinear"]
 
 
+def _param(module: nn.Module, name: str) -> torch.Tensor:
+    """module.name for a parameter, without nn.Module's attribute lookup (a third of a microsecond; a decode step makes 160);
+    a parametrized module, whose parameter is a property, has it from there."""
+    p = module._parameters.get(name)
+    return p if p is not None else getattr(module, name)
+
+
 def _pkey(p: torch.Tensor) -> tuple:
     """Cache key of a parameter: its identity and storage as well as its version counter, so that a Parameter that is
     REPLACED (load_state_dict(assign=True), `m.s = nn.Parameter(...)`) is seen although a fresh one starts at the same
@@ -706,16 +713,30 @@ class LinearLowbit(nn.Module):
         quantized_weight = self._get_quantized_weight(weight_compute)
         return F.apply(input, weight_compute, bias_compute, quantized_weight, quantized_input)
 
-    @torch.no_grad()
+    def _weight_key(self, device, arith) -> tuple:
+        F = LinearLowbitFunction
+        return (_pkey(_param(self, "weight")), device, arith, F.q_forward_weight, F.enable_nv_recipe)
+
+    def _cached_quantized_weight(self, arith):
+        """The kept quantized weight of this arithmetic if there is a current one, else None."""
+        cached = self._quantized_weight_cache
+        if cached is None or not self.cache_quantized_weight:
+            return None
+        return cached[1] if cached[0] == self._weight_key(_param(self, "weight").device, arith) else None
+
     def _get_quantized_weight(self, weight_compute, arith=None):
         """Quantized weight, cached on Parameter._version when enabled (reference 563-589).  Returns a
         PackedNVFP4 when the kernel path applies, otherwise the dequantized tensor."""
-        F = LinearLowbitFunction
-        key = (_pkey(self.weight), weight_compute.device, arith or weight_compute.dtype, F.q_forward_weight, F.enable_nv_recipe)
+        key = self._weight_key(weight_compute.device, arith or weight_compute.dtype)
         if self.cache_quantized_weight and self._quantized_weight_cache is not None:
             cached_key, cached = self._quantized_weight_cache
             if cached_key == key:
                 return cached
+        return self._quantize_weight(weight_compute, arith, key)
+
+    @torch.no_grad()
+    def _quantize_weight(self, weight_compute, arith, key):
+        F = LinearLowbitFunction
         if F._nv_on_kernels() and arith is not None and _packable(weight_compute, F.q_forward_weight) and weight_compute.shape[0] % 4 == 0:
             # reference 577-585 on the kernels: the packed tensor holds the ROTATED weight's codes, rotated in the
             # quantizer's registers; whoever reads it (tiled GEMM operand, dequantize) rotates back
@@ -1032,7 +1053,10 @@ class BitLinear(nn.Module):
     def _packed_residual(self):
         """Packed residual weight for the fused launch, or None when the kernel path does not apply."""
         F = LinearLowbitFunction
-        wl = self.warmup_linear
+        wl = self._modules["warmup_linear"]                     # (nn.Module's attribute lookup costs a third of a microsecond each)
+        cached = wl._cached_quantized_weight(self.compute_dtype)
+        if cached is not None:
+            return cached if isinstance(cached, PackedNVFP4) else None
         if (not F.enable_nv_recipe or F._nv_on_kernels()) and _packable(wl.weight, F.q_forward_weight) and wl.weight.shape[0] % 4 == 0:
             p_res = wl._get_quantized_weight(wl.weight, arith=self.compute_dtype)       # cache hit: no pass over W
         else:
@@ -1041,8 +1065,9 @@ class BitLinear(nn.Module):
 
     def _fusable(self) -> bool:
         r = self.args.forward_svd_rank
-        return (self.is_svd_quant and isinstance(self.vlinear, LinearLowbit) and isinstance(self.warmup_linear, LinearLowbit)
-                and r > 0 and r % 32 == 0 and self.ulinear.bias is None and not BitLinear.quantized_lowrank_branch)
+        mods = self._modules
+        return (self.is_svd_quant and isinstance(mods.get("vlinear"), LinearLowbit) and isinstance(mods.get("warmup_linear"), LinearLowbit)
+                and r > 0 and r % 32 == 0 and mods["ulinear"].bias is None and not BitLinear.quantized_lowrank_branch)
 
     def _quantize_and_project(self, x: torch.Tensor):
         """(packed activation, x V^T, bf16((x V^T) s)) from one pass over an activation that no sibling shares (direct
@@ -1054,17 +1079,19 @@ class BitLinear(nn.Module):
                 or not x.is_cuda or x.dtype != torch.bfloat16 or F.compute_dtype not in (torch.float32, torch.bfloat16)):
             return None
         x2 = _flat2d(x)
-        v = self.vlinear.weight
-        if v.dtype != torch.bfloat16 or self._packed_residual() is None:
+        v, s = _param(self._modules["vlinear"], "weight"), _param(self, "s")
+        if v.dtype != torch.bfloat16:
+            return None
+        p_res = self._packed_residual()
+        if p_res is None:
             return None
         mode = ops.MODE_P32 if F.compute_dtype == torch.float32 else ops.MODE_PB16
         if not F.enable_nv_recipe and ops.quantize_project_applies(x2, v, mode):
-            return ops.quantize_project(x2, v.detach(), self.s.detach(), mode)
+            return ops.quantize_project(x2, v.detach(), s.detach(), mode)
         # decode-sized call: the quantizer's launch carries the projection's first step, and the launch that builds the
         # GEMM's activation operands its finishing step (bf16 arithmetic; under the NV recipe either arithmetic, the
         # operand rotated for the weight's domain)
-        p_res = self._packed_residual()
-        if (self.s.dtype == torch.bfloat16 and ops.quantize_project_decode_applies(x2, v, mode) and x2.shape[0] * x2.shape[1] > 0
+        if (s.dtype == torch.bfloat16 and ops.quantize_project_decode_applies(x2, v, mode) and x2.shape[0] * x2.shape[1] > 0
                 and (p_res.rht is not None or (mode == ops.MODE_PB16 and F.reference_rounding))):
             probe = SimpleNamespace(rows=x2.shape[0], cols=x2.shape[1], mode=mode, rht=None)   # what the packed activation will be
             takes = (ops.nv_decode_applies(probe, [p_res], [v.shape[0]]) if p_res.rht is not None
@@ -1113,10 +1140,10 @@ class BitLinear(nn.Module):
         calls, c0 = [], 0
         for m, p_res in zip(members, packed):
             r = m.args.forward_svd_rank
-            bias = m.warmup_linear.bias
+            bias = m._modules["warmup_linear"].bias
             if bias is not None:
                 bias = m._bias_as(torch.float32 if (centre is not None and centre.dtype == torch.float32) else cd)
-            calls.append((p_res, t_all[:, c0:c0 + r], m.ulinear.weight.to(cd), bias))      # a column slice: no copy
+            calls.append((p_res, t_all[:, c0:c0 + r], _param(m._modules["ulinear"], "weight").to(cd), bias))      # a column slice: no copy
             c0 += r
         out_dtype = torch.float32 if F.compute_dtype == torch.float32 else torch.bfloat16
         # mean mode: every member also receives W^ me, inside the same launch (binary32)
@@ -1131,7 +1158,7 @@ class BitLinear(nn.Module):
         cd = torch.bfloat16
         group = self.activation_group
         members = group["members"]
-        key = tuple((_pkey(m.vlinear.weight), _pkey(m.s)) for m in members) + (device,)
+        key = [(_pkey(_param(m._modules["vlinear"], "weight")), _pkey(_param(m, "s"))) for m in members] + [device]
         cached = group.get("stacked_v")
         if cached is None or cached[0] != key:
             cached = (key, torch.cat([m.vlinear.weight.to(cd) for m in members], dim=0),
@@ -1158,13 +1185,13 @@ class BitLinear(nn.Module):
         calls, c0 = [], 0
         for m, p_res in zip(members, packed):
             r = m.args.forward_svd_rank
-            bias = m.warmup_linear.bias
+            bias = m._modules["warmup_linear"].bias
             if centered and not in_operand:
                 w_mean = ops.matvec(p_res, shared_input.center32)          # the mean's share rides in a binary32 bias
                 bias = w_mean if bias is None else w_mean + m._bias_as(torch.float32)
             elif bias is not None:
                 bias = m._bias_as(torch.float32 if f32 else cd)
-            calls.append((p_res, t_all[:, c0:c0 + r], m.ulinear.weight.to(cd), bias))
+            calls.append((p_res, t_all[:, c0:c0 + r], _param(m._modules["ulinear"], "weight").to(cd), bias))
             c0 += r
         outs = ops.linear_fwd_tiled_grouped(px, calls, out_dtype=torch.float32 if f32 else torch.bfloat16,
                                             center=shared_input.mean if in_operand else None, reference_rounding=rounding)
@@ -1173,7 +1200,7 @@ class BitLinear(nn.Module):
 
     def _bias_as(self, dtype: torch.dtype) -> torch.Tensor:
         """The residual branch's bias in `dtype`, converted once per parameter version (decode calls are launch-bound)."""
-        b = self.warmup_linear.bias
+        b = self._modules["warmup_linear"].bias
         if b.dtype == dtype:
             return b
         key = (_pkey(b), b.device, dtype)
@@ -1191,10 +1218,12 @@ class BitLinear(nn.Module):
             return self.warmup_linear(x)
         group = self.activation_group
         if (BitLinear.grouped_inference and group is not None and not torch.is_grad_enabled() and len(group.get("members", ())) > 1
-                and x.is_cuda and self._fusable()):
+                and x.is_cuda):
             ready = group.get("grouped_outputs")
             if ready is not None and ready[0]() is x and id(self) in ready[1]:
-                return ready[1].pop(id(self))
+                return ready[1].pop(id(self))                   # evaluated with the first member of the group
+        if (BitLinear.grouped_inference and group is not None and not torch.is_grad_enabled() and len(group.get("members", ())) > 1
+                and x.is_cuda and self._fusable()):
             shared_input = self._get_shared_quantized_input(x)
             if isinstance(shared_input, (PackedNVFP4, CenteredNVFP4)):
                 outs = self._forward_group(x, shared_input)
@@ -1206,21 +1235,23 @@ class BitLinear(nn.Module):
                             group["grouped_outputs"] = None
                     group["grouped_outputs"] = (weakref.ref(x, drop), outs)
                     return mine
-        share_activation = (isinstance(self.vlinear, LinearLowbit) and isinstance(self.warmup_linear, LinearLowbit)
+        mods = self._modules
+        share_activation = (isinstance(mods.get("vlinear"), LinearLowbit) and isinstance(mods.get("warmup_linear"), LinearLowbit)
                             and self.args.forward_svd_rank > 0)
         if share_activation:
             r = self.args.forward_svd_rank
             fused = self._quantize_and_project(x) if (group is None and self._fusable()) else None
             shared_input = fused[0] if fused is not None else self._get_shared_quantized_input(x)
-            if (isinstance(shared_input, (PackedNVFP4, CenteredNVFP4)) and r % 32 == 0 and self.ulinear.bias is None
+            if (isinstance(shared_input, (PackedNVFP4, CenteredNVFP4)) and r % 32 == 0 and mods["ulinear"].bias is None
                     and not BitLinear.quantized_lowrank_branch):
                 # one fused launch for both branches; it already is the "merged" evaluation, so the
                 # rollout switch changes nothing on this path
                 p_res = self._packed_residual()
                 if p_res is not None:
                     more = () if fused is None else fused[1:]
-                    return _MetisFusedFunction.apply(x, self.vlinear.weight, self.s, self.ulinear.weight,
-                                                     self.warmup_linear.weight, self.warmup_linear.bias, shared_input, p_res, *more)
+                    wl = mods["warmup_linear"]
+                    return _MetisFusedFunction.apply(x, _param(mods["vlinear"], "weight"), _param(self, "s"), _param(mods["ulinear"], "weight"),
+                                                     _param(wl, "weight"), wl.bias, shared_input, p_res, *more)
             if BitLinear.rollout_merge_active and not torch.is_grad_enabled():
                 return self._rollout_forward(shared_input, x.shape)
             y = self.vlinear(x, quantized_input=shared_input)

@@ -78,15 +78,18 @@ class PackedNVFP4:
         scales = torch.empty(self.rows, self.cols // BLOCK, dtype=torch.uint8, device=self.codes.device)
         rc = load().metis_nvfp4_deferred_scales(d["deferred"].data_ptr(), self.rows, self.cols, self.mode, scales.data_ptr(),
                                                 d["_unit"].data_ptr(), _stream())
-        check(rc, "metis_nvfp4_deferred_scales", (self.rows, self.cols))
+        if rc:
+            check(rc, "metis_nvfp4_deferred_scales", (self.rows, self.cols))
         d["_scales"], d["_unit_ready"] = scales, True
 
 
 def _packed_scales(self):
     d = self.__dict__
-    if d.get("_scales") is None and d.get("deferred") is not None:
+    s = d.get("_scales")
+    if s is None and d.get("deferred") is not None:
         self._materialize()
-    return d.get("_scales")
+        s = d["_scales"]
+    return s
 
 
 def _packed_unit(self):
@@ -152,18 +155,50 @@ class LowRankNVFP4:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream() -> int:
-    """Handle of torch's current stream on the current device (the raw getter skips the Stream object: this is
-    called several times per layer)."""
-    if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+    """Handle of torch's current stream on the current device (the raw getters skip the Stream object and the check for an
+    initialised runtime, which a device tensor implies: this is called several times per layer)."""
+    if _raw_stream is not None and _raw_device is not None:
+        return _raw_stream(_raw_device())
     return torch.cuda.current_stream().cuda_stream
 
 
+# Sizes that depend on the shape alone; a library call costs as much host time as an allocation.
+@functools.lru_cache(maxsize=4096)
+def _deferred_bytes(rows: int, cols: int) -> int:
+    return int(load().metis_nvfp4_deferred_bytes(rows, cols))
+
+
+@functools.lru_cache(maxsize=4096)
+def _decode_operand_bytes(rows: int, cols: int) -> int:
+    return int(load().metis_nvfp4_decode_operand_bytes(rows, cols))
+
+
+@functools.lru_cache(maxsize=4096)
+def _expand_tiled_bytes(rows: int, cols: int) -> int:
+    return int(load().metis_nvfp4_expand_tiled_bytes(rows, cols))
+
+
+@functools.lru_cache(maxsize=4096)
+def _column_mean_bytes(cols: int) -> int:
+    return int(load().metis_column_mean_workspace_bytes(cols))
+
+
+@functools.lru_cache(maxsize=4096)
+def _quant_workspace_bytes(rows: int, cols: int) -> int:
+    return int(load().metis_nvfp4_workspace_bytes(rows, cols))
+
+
+@functools.lru_cache(maxsize=4096)
+def _lowrank_rows_workspace_bytes(M: int, R: int, K: int, device_index: int) -> int:
+    return int(load().metis_lowrank_project_rows_workspace_bytes(M, R, K))       # depends on the device's CU count only
+
+
 def _workspace(rows: int, cols: int, device: torch.device) -> torch.Tensor:
-    need = load().metis_nvfp4_workspace_bytes(rows, cols)
+    need = _quant_workspace_bytes(rows, cols)
     key = (device.index, _stream())
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < need:
@@ -234,10 +269,11 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
             cen = center.reshape(-1).to(device=dev, dtype=torch.bfloat16).contiguous()
             if cen.numel() != cols:
                 raise ValueError(f"center must have one value per column ({cols}), got {cen.numel()}")
-        parked = torch.empty(L.metis_nvfp4_deferred_bytes(rows, cols), dtype=torch.uint8, device=dev)
+        parked = torch.empty(_deferred_bytes(rows, cols), dtype=torch.uint8, device=dev)
         rc = L.metis_nvfp4_quant_row_deferred(x2.data_ptr(), rows, cols, kmode, None if cen is None else cen.data_ptr(),
                                               codes.data_ptr(), parked.data_ptr(), parked.numel(), _stream())
-        check(rc, "metis_nvfp4_quant_row_deferred", x.shape)
+        if rc:
+            check(rc, "metis_nvfp4_quant_row_deferred", x.shape)
         return PackedNVFP4(codes, None, unit, prow, pcol, mode, deferred=parked)
     scales = torch.empty(prow, pcol // BLOCK, dtype=torch.uint8, device=dev)
     ws = _workspace(rows, cols, dev)
@@ -252,7 +288,8 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
                                           None if nz is None else nz.data_ptr(), seed & (2 ** 64 - 1), offset,
                                           codes.data_ptr(), scales.data_ptr(), unit.data_ptr(), ws.data_ptr(), ws.numel(),
                                           _stream())
-        check(rc, "metis_nvfp4_quant_centered", x.shape)
+        if rc:
+            check(rc, "metis_nvfp4_quant_centered", x.shape)
         return PackedNVFP4(codes, scales, unit, prow, pcol, mode)
     if sr:
         nz = None
@@ -271,13 +308,15 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
         dec = torch.empty(L.metis_nvfp4_decode_weight_bytes(rows, cols), dtype=torch.uint8, device=dev)
         rc = L.metis_nvfp4_quant_row_decode(x2.data_ptr(), rows, cols, kmode, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(),
                                             dec.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-        check(rc, "metis_nvfp4_quant_row_decode", x.shape)
+        if rc:
+            check(rc, "metis_nvfp4_quant_row_decode", x.shape)
         return PackedNVFP4(codes, scales, unit, prow, pcol, mode, decode_layout=dec)
     else:
         fn = L.metis_nvfp4_quant_col if col else L.metis_nvfp4_quant_row
         rc = fn(x2.data_ptr(), rows, cols, x2.stride(0), kmode, codes.data_ptr(), scales.data_ptr(),
                 unit.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_nvfp4_quant", x.shape)
+    if rc:
+        check(rc, "metis_nvfp4_quant", x.shape)
     return PackedNVFP4(codes, scales, unit, prow, pcol, mode)
 
 
@@ -300,7 +339,8 @@ def _quantize_col_padded(x2, kmode, mode, pad_rows, col, sr, noise, seed, offset
     rc = load().metis_nvfp4_quant_col_padded(x2.data_ptr(), rows, pad_rows, cols, x2.stride(0), kmode, None if cen is None else cen.data_ptr(),
                                              int(sr), seed & (2 ** 64 - 1), offset, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(),
                                              ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_nvfp4_quant_col_padded", (rows, cols))
+    if rc:
+        check(rc, "metis_nvfp4_quant_col_padded", (rows, cols))
     return PackedNVFP4(codes, scales, unit, cols, pad_rows, mode)
 
 
@@ -323,7 +363,8 @@ def quantize_dequantize(x: torch.Tensor, mode: int = MODE_P32) -> tuple[PackedNV
     ws = _workspace(rows, cols, dev)
     rc = load().metis_nvfp4_quant_dequant_row(x2.data_ptr(), rows, cols, mode, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(),
                                               out.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_nvfp4_quant_dequant_row", x.shape)
+    if rc:
+        check(rc, "metis_nvfp4_quant_dequant_row", x.shape)
     return PackedNVFP4(codes, scales, unit, rows, cols, mode), out
 
 
@@ -344,7 +385,8 @@ def quantize_dequantize_f32(x: torch.Tensor) -> tuple[PackedNVFP4, torch.Tensor]
     ws = _workspace(rows, cols, dev)
     rc = load().metis_nvfp4_quant_dequant_row_f32(x2.data_ptr(), rows, cols, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(), out.data_ptr(),
                                                   ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_nvfp4_quant_dequant_row_f32", x.shape)
+    if rc:
+        check(rc, "metis_nvfp4_quant_dequant_row_f32", x.shape)
     return PackedNVFP4(codes, scales, unit, rows, cols, MODE_P32), out
 
 
@@ -379,7 +421,8 @@ def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tenso
                                                    vt.data_ptr(), rows, cols, r, mode, codes.data_ptr(), scales.data_ptr(),
                                                    unit.data_ptr(), None if out is None else out.data_ptr(), ws.data_ptr(),
                                                    ws.numel(), _stream())
-    check(rc, "metis_nvfp4_quant_lowrank_residual", (rows, cols, r))
+    if rc:
+        check(rc, "metis_nvfp4_quant_lowrank_residual", (rows, cols, r))
     return PackedNVFP4(codes, scales, unit, rows, cols, mode), out
 
 
@@ -414,7 +457,8 @@ def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, of
         rc = L.metis_nvfp4_quant_sr_both_padded(x2.data_ptr(), have, rows, cols, x2.stride(0), kmode, seed & (2 ** 64 - 1), offset_row,
                                                 offset_col, cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(),
                                                 uc.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-        check(rc, "metis_nvfp4_quant_sr_both_padded", x.shape)
+        if rc:
+            check(rc, "metis_nvfp4_quant_sr_both_padded", x.shape)
     return PackedNVFP4(cr[:have], sr_[:have], ur, have, cols, mode), PackedNVFP4(cc, sc, uc, cols, rows, mode)
 
 
@@ -425,7 +469,8 @@ def dequantize(p: PackedNVFP4, dtype: torch.dtype = torch.bfloat16) -> torch.Ten
     rc = load().metis_nvfp4_dequant(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols,
                                     p.mode, out.data_ptr(), DTYPE_F32 if dtype == torch.float32 else DTYPE_BF16,
                                     _stream())
-    check(rc, "metis_nvfp4_dequant", (p.rows, p.cols))
+    if rc:
+        check(rc, "metis_nvfp4_dequant", (p.rows, p.cols))
     if p.rht is not None:                     # packed in the rotated domain: back to the tensor's own
         out = hadamard16(out, p.rht, inverse=True)
     return out
@@ -443,7 +488,8 @@ def hadamard16(x: torch.Tensor, sign_mask: int, inverse: bool = False) -> torch.
     out = torch.empty_like(x2)
     rc = load().metis_hadamard16(x2.data_ptr(), x2.shape[0], cols, cols, DTYPE_F32 if x.dtype == torch.float32 else DTYPE_BF16,
                                  int(inverse), int(sign_mask), out.data_ptr(), cols, _stream())
-    check(rc, "metis_hadamard16", tuple(x.shape))
+    if rc:
+        check(rc, "metis_hadamard16", tuple(x.shape))
     return out.reshape(x.shape)
 
 
@@ -461,7 +507,8 @@ def quantize_rht(x: torch.Tensor, mode: int, sign_mask: int, *, sr: bool = False
     ws = _workspace(rows, cols, dev)
     rc = load().metis_nvfp4_quant_row_rht(x2.data_ptr(), rows, cols, x2.stride(0), kmode, int(sign_mask), int(sr), int(seed), int(offset),
                                           codes.data_ptr(), scales.data_ptr(), unit.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_nvfp4_quant_row_rht", (rows, cols))
+    if rc:
+        check(rc, "metis_nvfp4_quant_row_rht", (rows, cols))
     return PackedNVFP4(codes, scales, unit, rows, cols, MODE_PB16 if mode == MODE_PB16 else MODE_P32, rht=int(sign_mask))
 
 
@@ -482,7 +529,7 @@ def column_mean(x: torch.Tensor, out_dtype: torch.dtype = torch.float32, _sum_on
     rows, cols = x2.shape
     out = torch.empty(cols, dtype=out_dtype, device=x2.device)
     L = load()
-    ws = torch.empty(L.metis_column_mean_workspace_bytes(cols), dtype=torch.uint8, device=x2.device)
+    ws = torch.empty(_column_mean_bytes(cols), dtype=torch.uint8, device=x2.device)
     fn = L.metis_column_sum if _sum_only else L.metis_column_mean
     rc = fn(x2.data_ptr(), rows, cols, x2.stride(0), DTYPE_F32 if x2.dtype == torch.float32 else DTYPE_BF16,
             out.data_ptr(), DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, ws.data_ptr(), ws.numel(), _stream())
@@ -510,12 +557,13 @@ def column_mean_running(x: torch.Tensor, cached: torch.Tensor | None, cached_cou
     out = torch.empty(cols, dtype=out_dtype, device=x2.device)
     out32 = out if out_dtype == torch.float32 else torch.empty(cols, dtype=torch.float32, device=x2.device)
     L = load()
-    ws = torch.empty(L.metis_column_mean_workspace_bytes(cols), dtype=torch.uint8, device=x2.device)
+    ws = torch.empty(_column_mean_bytes(cols), dtype=torch.uint8, device=x2.device)
     rc = L.metis_column_mean_running(x2.data_ptr(), rows, cols, x2.stride(0), DTYPE_F32 if x2.dtype == torch.float32 else DTYPE_BF16,
                                      None if cached is None else cached.data_ptr(), int(cached_count), out.data_ptr(),
                                      None if out32 is out else out32.data_ptr(),
                                      DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_column_mean_running", x.shape)
+    if rc:
+        check(rc, "metis_column_mean_running", x.shape)
     return out, out32
 
 
@@ -544,7 +592,8 @@ def matvec(p: PackedNVFP4, v: torch.Tensor | None = None, alpha: float = 1.0, *,
             raise ValueError(f"z must have one value per packed row ({p.rows}), got {z.numel()}")
         rc = load().metis_nvfp4_matvec_affine(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, vp,
                                               float(alpha), z.data_ptr(), float(beta), out.data_ptr(), _stream())
-        check(rc, "metis_nvfp4_matvec_affine", (p.rows, p.cols))
+        if rc:
+            check(rc, "metis_nvfp4_matvec_affine", (p.rows, p.cols))
         return out
     sp, sld = None, 0
     if split is not None:
@@ -553,7 +602,8 @@ def matvec(p: PackedNVFP4, v: torch.Tensor | None = None, alpha: float = 1.0, *,
         sp, sld = split.data_ptr(), split.stride(0)
     rc = load().metis_nvfp4_matvec(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, vp,
                                    float(alpha), None if out is None else out.data_ptr(), sp, sld, int(split_col), _stream())
-    check(rc, "metis_nvfp4_matvec", (p.rows, p.cols))
+    if rc:
+        check(rc, "metis_nvfp4_matvec", (p.rows, p.cols))
     return out
 
 
@@ -577,7 +627,8 @@ def rank_one_operands(n: int, k: int, first: tuple | None, second: tuple | None 
     t = torch.empty(n, 32, dtype=torch.bfloat16, device=dev)
     u = torch.empty(k, 32, dtype=torch.bfloat16, device=dev)
     rc = load().metis_rank_one_operands(ptrs[0], ptrs[1], ptrs[2], ptrs[3], n, k, t.data_ptr(), u.data_ptr(), _stream())
-    check(rc, "metis_rank_one_operands", (n, k))
+    if rc:
+        check(rc, "metis_rank_one_operands", (n, k))
     return t, u
 
 
@@ -589,7 +640,8 @@ def expand(p: PackedNVFP4) -> torch.Tensor:
     if p.expanded is None:
         out = torch.empty(p.rows, p.cols, dtype=torch.float16, device=p.codes.device)
         rc = load().metis_nvfp4_expand_f16(p.codes.data_ptr(), p.scales.data_ptr(), p.rows, p.cols, out.data_ptr(), _stream())
-        check(rc, "metis_nvfp4_expand_f16", (p.rows, p.cols))
+        if rc:
+            check(rc, "metis_nvfp4_expand_f16", (p.rows, p.cols))
         p.expanded = out
     return p.expanded
 
@@ -613,7 +665,7 @@ def expand_tiled(p: PackedNVFP4, cache: bool = True, mode: int = MODE_P32, cente
         kept = d.get("_tiled_centered")
         if cache and kept is not None and kept[0] == key:
             return kept[1]
-        out = torch.empty(L.metis_nvfp4_expand_tiled_bytes(p.rows, p.cols), dtype=torch.uint8, device=p.codes.device)
+        out = torch.empty(_expand_tiled_bytes(p.rows, p.cols), dtype=torch.uint8, device=p.codes.device)
         if cache:
             d["_tiled_centered"] = (key, out, center)                 # (the centre is kept alive with its address)
         if lazy:
@@ -623,17 +675,19 @@ def expand_tiled(p: PackedNVFP4, cache: bool = True, mode: int = MODE_P32, cente
         else:
             rc = L.metis_nvfp4_expand_tiled_centered(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols,
                                                      center.data_ptr(), out.data_ptr(), _stream())
-        check(rc, "metis_nvfp4_expand_tiled_centered", (p.rows, p.cols))
+        if rc:
+            check(rc, "metis_nvfp4_expand_tiled_centered", (p.rows, p.cols))
         return out
     have = p.tiled_pb16 if mode == MODE_PB16 else p.tiled
     if have is not None:
         return have
-    out = torch.empty(L.metis_nvfp4_expand_tiled_bytes(p.rows, p.cols), dtype=torch.uint8, device=p.codes.device)
+    out = torch.empty(_expand_tiled_bytes(p.rows, p.cols), dtype=torch.uint8, device=p.codes.device)
     if lazy:
         # the scale bytes were never written: this kernel forms them from the parked block maxima, and writes the unit
         rc = L.metis_nvfp4_expand_tiled_deferred(p.codes.data_ptr(), d["deferred"].data_ptr(), p.rows, p.cols, p.mode, mode,
                                                  None, d["_unit"].data_ptr(), out.data_ptr(), _stream())
-        check(rc, "metis_nvfp4_expand_tiled_deferred", (p.rows, p.cols))
+        if rc:
+            check(rc, "metis_nvfp4_expand_tiled_deferred", (p.rows, p.cols))
         d["_unit_ready"] = True
     elif p.rht is not None:                   # NV recipe: the operand holds the values rotated back
         rc = L.metis_nvfp4_expand_tiled_rht(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, mode,
@@ -641,7 +695,8 @@ def expand_tiled(p: PackedNVFP4, cache: bool = True, mode: int = MODE_P32, cente
     else:
         rc = L.metis_nvfp4_expand_tiled(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, mode,
                                         out.data_ptr(), _stream())
-    check(rc, "metis_nvfp4_expand_tiled", (p.rows, p.cols))
+    if rc:
+        check(rc, "metis_nvfp4_expand_tiled", (p.rows, p.cols))
     if cache and (tiled_weight_copies or not p.persistent):
         if mode == MODE_PB16:
             p.tiled_pb16 = out
@@ -660,7 +715,8 @@ def expand_tiled_transposed(p: PackedNVFP4, cache: bool = False, mode: int = MOD
     out = torch.empty(L.metis_nvfp4_expand_tiled_bytes(p.cols, p.rows), dtype=torch.uint8, device=p.codes.device)
     rc = L.metis_nvfp4_expand_tiled_rht(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, mode,
                                         p.rht or 0, int(p.rht is not None), 1, out.data_ptr(), _stream())
-    check(rc, "metis_nvfp4_expand_tiled_rht", (p.rows, p.cols))
+    if rc:
+        check(rc, "metis_nvfp4_expand_tiled_rht", (p.rows, p.cols))
     if cache and (tiled_weight_copies or not p.persistent):
         if mode == MODE_PB16:
             p.tiled_t_pb16 = out
@@ -687,7 +743,8 @@ def decode_operand(p: PackedNVFP4, mode: int = MODE_P32, center: torch.Tensor | 
                                               d["_unit"].data_ptr() if lazy else p.unit.data_ptr(),
                                               d["deferred"].data_ptr() if lazy else None, p.rows, p.cols, p.mode, mode, int(rotate),
                                               out.data_ptr(), _stream())
-        check(rc, "metis_nvfp4_decode_operand_rht", (p.rows, p.cols))
+        if rc:
+            check(rc, "metis_nvfp4_decode_operand_rht", (p.rows, p.cols))
         if lazy:
             d["_unit_ready"] = True
         return out
@@ -701,12 +758,14 @@ def decode_operand(p: PackedNVFP4, mode: int = MODE_P32, center: torch.Tensor | 
         rc = L.metis_nvfp4_decode_operand_deferred(p.codes.data_ptr(), d["deferred"].data_ptr(), p.rows, p.cols, p.mode, mode,
                                                    None if center is None else center.data_ptr(), d["_unit"].data_ptr(),
                                                    out.data_ptr(), _stream())
-        check(rc, "metis_nvfp4_decode_operand_deferred", (p.rows, p.cols))
+        if rc:
+            check(rc, "metis_nvfp4_decode_operand_deferred", (p.rows, p.cols))
         d["_unit_ready"] = True
         return out
     rc = L.metis_nvfp4_decode_operand(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, mode,
                                       None if center is None else center.data_ptr(), out.data_ptr(), _stream())
-    check(rc, "metis_nvfp4_decode_operand", (p.rows, p.cols))
+    if rc:
+        check(rc, "metis_nvfp4_decode_operand", (p.rows, p.cols))
     return out
 
 
@@ -715,10 +774,13 @@ def grouped_operand_applies(a: PackedNVFP4, weights, ranks, center: torch.Tensor
     operands (decode_operand): bf16 arithmetic on every tensor, decode-sized shapes in wide runs.  weights: the
     members' packed weights, ranks: the widths of their low-rank terms (0 without)."""
     M, K = a.rows, a.cols
-    return bool(reference_rounding and (center is None or center.dtype == torch.bfloat16) and a.mode == MODE_PB16
-                and all(b.mode == MODE_PB16 and b.rht is None for b in weights) and len(weights) <= 4 and K % 256 == 0
-                and all(_decode_kernel_takes(M, b.rows, K, r) for b, r in zip(weights, ranks))
-                and all(b.scales.data_ptr() % 8 == 0 for b in weights))
+    if not (reference_rounding and 0 < M < 256 and a.mode == MODE_PB16 and K % 256 == 0 and len(weights) <= 4
+            and (center is None or center.dtype == torch.bfloat16)):
+        return False
+    for b, r in zip(weights, ranks):
+        if b.mode != MODE_PB16 or b.rht is not None or not _decode_kernel_takes(M, b.rows, K, r) or b.scales.data_ptr() % 8:
+            return False
+    return True
 
 
 def project_and_operand_applies(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: PackedNVFP4) -> bool:
@@ -756,8 +818,8 @@ def project_and_operand(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: P
             raise ValueError(f"center must have {K} values, got {center.numel()}")
     xv = torch.empty(M, R, dtype=torch.bfloat16, device=dev)
     t = torch.empty_like(xv)
-    out = torch.empty(L.metis_nvfp4_decode_operand_bytes(M, K), dtype=torch.uint8, device=dev)
-    need = L.metis_lowrank_project_workspace_bytes(M, R, K)
+    out = torch.empty(_decode_operand_bytes(M, K), dtype=torch.uint8, device=dev)
+    need = _lowrank_workspace_bytes(M, R, K)
     if pending is not None and (pending.numel() < need or pending.device != dev or R > 128):
         raise ValueError("project_and_operand: `pending` is not what quantize_project_decode returns for these shapes")
     ws = pending if pending is not None else torch.empty(need, dtype=torch.uint8, device=dev)
@@ -767,7 +829,8 @@ def project_and_operand(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: P
                                          ws.data_ptr(), need, p.codes.data_ptr(), d["deferred"].data_ptr(), M, K, p.mode, mode,
                                          None if center is None else center.data_ptr(), d["_unit"].data_ptr(), out.data_ptr(),
                                          int(rotate is not None), int(rotate or 0), _stream())
-    check(rc, "metis_decode_prepare_deferred", (M, K, R))
+    if rc:
+        check(rc, "metis_decode_prepare_deferred", (M, K, R))
     d["_unit_ready"] = True
     return xv, t, out
 
@@ -783,7 +846,8 @@ def decode_weight(p: PackedNVFP4, cache: bool = True) -> torch.Tensor | None:
     L = load()
     out = torch.empty(L.metis_nvfp4_decode_weight_bytes(p.rows, p.cols), dtype=torch.uint8, device=p.codes.device)
     rc = L.metis_nvfp4_decode_weight(p.codes.data_ptr(), p.scales.data_ptr(), p.rows, p.cols, out.data_ptr(), _stream())
-    check(rc, "metis_nvfp4_decode_weight", (p.rows, p.cols))
+    if rc:
+        check(rc, "metis_nvfp4_decode_weight", (p.rows, p.cols))
     if cache:
         p.decode_layout = out
     return out
@@ -803,7 +867,8 @@ def dense_expand_tiled(x: torch.Tensor, mode: int = MODE_P32, col_scale: torch.T
     cs = None if col_scale is None else col_scale.to(torch.bfloat16).contiguous()
     rc = L.metis_dense_expand_tiled(x.data_ptr(), rows, cols, x.stride(0), DTYPE_F32 if x.dtype == torch.float32 else DTYPE_BF16,
                                     None if cs is None else cs.data_ptr(), mode, out.data_ptr(), _stream())
-    check(rc, "metis_dense_expand_tiled", (rows, cols))
+    if rc:
+        check(rc, "metis_dense_expand_tiled", (rows, cols))
     return out
 
 
@@ -837,7 +902,8 @@ def gemm_tiled(ax: torch.Tensor, a_unit: torch.Tensor, bx: torch.Tensor, b_unit:
                                        None if bias is None else bias.data_ptr(), int(bias_f32), out.data_ptr(),
                                        DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, mode,
                                        None if ws is None else ws.data_ptr(), need, _stream())
-    check(rc, "metis_linear_fwd_tiled", (M, N, K))
+    if rc:
+        check(rc, "metis_linear_fwd_tiled", (M, N, K))
     return out
 
 
@@ -934,7 +1000,8 @@ class _TiledBatch:
         rc = load().metis_linear_fwd_tiled_grouped(self.ax.data_ptr(), a.unit.data_ptr(), a.rows, a.cols, ctypes.cast(self.members, ctypes.c_void_p),
                                                    len(self.rows), DTYPE_F32 if self.out_dtype == torch.float32 else DTYPE_BF16, self.mode,
                                                    None if ws is None else ws.data_ptr(), need, _stream())
-        check(rc, "metis_linear_fwd_tiled_grouped", (a.rows, a.cols, self.rows))
+        if rc:
+            check(rc, "metis_linear_fwd_tiled_grouped", (a.rows, a.cols, self.rows))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -960,11 +1027,12 @@ def rmsnorm_quantize(x: torch.Tensor, gamma: torch.Tensor, eps: float, mode: int
     unit = torch.empty(1, dtype=torch.float32, device=dev)
     if deferred and rows * cols > 0:
         L = load()
-        parked = torch.empty(L.metis_nvfp4_deferred_bytes(rows, cols), dtype=torch.uint8, device=dev)
+        parked = torch.empty(_deferred_bytes(rows, cols), dtype=torch.uint8, device=dev)
         rc = L.metis_rmsnorm_nvfp4_quant_deferred(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, mode,
                                                   None if normed is None else normed.data_ptr(), codes.data_ptr(),
                                                   parked.data_ptr(), parked.numel(), _stream())
-        check(rc, "metis_rmsnorm_nvfp4_quant_deferred", x.shape)
+        if rc:
+            check(rc, "metis_rmsnorm_nvfp4_quant_deferred", x.shape)
         if normed is not None:
             normed = normed.reshape(x.shape)
         return normed, PackedNVFP4(codes, None, unit, rows, cols, mode, deferred=parked)
@@ -982,7 +1050,8 @@ def rmsnorm_quantize(x: torch.Tensor, gamma: torch.Tensor, eps: float, mode: int
         rc = load().metis_rmsnorm_nvfp4_quant(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, mode,
                                               None if normed is None else normed.data_ptr(), codes.data_ptr(),
                                               scales.data_ptr(), unit.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_rmsnorm_nvfp4_quant", x.shape)
+    if rc:
+        check(rc, "metis_rmsnorm_nvfp4_quant", x.shape)
     if normed is not None:
         normed = normed.reshape(x.shape)
     return normed, PackedNVFP4(codes, scales, unit, rows, cols, mode, decode_layout=dec)
@@ -1015,7 +1084,8 @@ def rmsnorm_colmean(x: torch.Tensor, gamma: torch.Tensor, eps: float, mean_dtype
     rc = L.metis_rmsnorm_colmean(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, normed.data_ptr(), me.data_ptr(),
                                  DTYPE_F32 if mean_dtype == torch.float32 else DTYPE_BF16, cp, int(cached_count),
                                  None if me32 is me else me32.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_rmsnorm_colmean", x.shape)
+    if rc:
+        check(rc, "metis_rmsnorm_colmean", x.shape)
     return normed, me, me32
 
 
@@ -1048,7 +1118,8 @@ def rmsnorm_backward(x: torch.Tensor, g: torch.Tensor, gamma: torch.Tensor, eps:
         ws = torch.empty(need, dtype=torch.uint8, device=x.device)
     rc = L.metis_rmsnorm_backward(x2.data_ptr(), g2.data_ptr(), gm.data_ptr(), float(eps), rows, cols, gx.data_ptr(),
                                   None if gg is None else gg.data_ptr(), DTYPE_BF16, None if ws is None else ws.data_ptr(), need, _stream())
-    check(rc, "metis_rmsnorm_backward", x.shape)
+    if rc:
+        check(rc, "metis_rmsnorm_backward", x.shape)
     return gx.reshape(x.shape), gg
 
 
@@ -1188,24 +1259,28 @@ def linear_fwd(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None = None,
         ae, be = expand(a), expand(b)
         rc = load().metis_linear_fwd_expanded(ae.data_ptr(), a.unit.data_ptr(), be.data_ptr(), b.unit.data_ptr(), M, N, K,
                                               tp, up, r, bp, out.data_ptr(), dt, _stream())
-        check(rc, "metis_linear_fwd_expanded", (M, N, K))
+        if rc:
+            check(rc, "metis_linear_fwd_expanded", (M, N, K))
         return out
     ws = _gemm_workspace(M, N, K, dev) if split_k else None
     if bias_f32:
         rc = load().metis_linear_fwd_f32bias(a.codes.data_ptr(), a.scales.data_ptr(), a.unit.data_ptr(), b.codes.data_ptr(),
                                              b.scales.data_ptr(), b.unit.data_ptr(), M, N, K, tp, up, r, bp, out.data_ptr(), dt,
                                              None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream())
-        check(rc, "metis_linear_fwd_f32bias", (M, N, K))
+        if rc:
+            check(rc, "metis_linear_fwd_f32bias", (M, N, K))
         return out
     if ws is not None:
         rc = load().metis_linear_fwd_ws(a.codes.data_ptr(), a.scales.data_ptr(), a.unit.data_ptr(), b.codes.data_ptr(),
                                         b.scales.data_ptr(), b.unit.data_ptr(), M, N, K, tp, up, r, bp, out.data_ptr(), dt,
                                         ws.data_ptr(), ws.numel(), _stream())
-        check(rc, "metis_linear_fwd_ws", (M, N, K))
+        if rc:
+            check(rc, "metis_linear_fwd_ws", (M, N, K))
         return out
     rc = load().metis_linear_fwd(a.codes.data_ptr(), a.scales.data_ptr(), a.unit.data_ptr(), b.codes.data_ptr(),
                                  b.scales.data_ptr(), b.unit.data_ptr(), M, N, K, tp, up, r, bp, out.data_ptr(), dt, _stream())
-    check(rc, "metis_linear_fwd", (M, N, K))
+    if rc:
+        check(rc, "metis_linear_fwd", (M, N, K))
     return out
 
 
@@ -1229,16 +1304,18 @@ def lowrank_project(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None = 
     t = None if s is None else torch.empty_like(xv)
     sp = None if s is None else s.contiguous().data_ptr()
     if large:
-        need = L.metis_lowrank_project_rows_workspace_bytes(M, R, K)
+        need = _lowrank_rows_workspace_bytes(M, R, K, x2.device.index or 0)
         ws = torch.empty(need, dtype=torch.uint8, device=x2.device) if need else None
         rc = L.metis_lowrank_project_rows_ws(x2.data_ptr(), x2.stride(0), v.data_ptr(), M, R, K, sp, xv.data_ptr(),
                                              None if t is None else t.data_ptr(), None if ws is None else ws.data_ptr(), need, _stream())
-        check(rc, "metis_lowrank_project_rows_ws", (M, R, K))
+        if rc:
+            check(rc, "metis_lowrank_project_rows_ws", (M, R, K))
         return xv if s is None else (xv, t)
     ws = torch.empty(_lowrank_workspace_bytes(M, R, K), dtype=torch.uint8, device=x2.device)
     rc = L.metis_lowrank_project(x2.data_ptr(), x2.stride(0), v.data_ptr(), M, R, K, sp,
                                  xv.data_ptr(), None if t is None else t.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    check(rc, "metis_lowrank_project", (M, R, K))
+    if rc:
+        check(rc, "metis_lowrank_project", (M, R, K))
     return xv if s is None else (xv, t)
 
 
@@ -1267,13 +1344,14 @@ def quantize_project(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, mode: i
     t = torch.empty_like(xv)
     codes = torch.empty(M, K // 2, dtype=torch.uint8, device=dev)
     unit = torch.empty(1, dtype=torch.float32, device=dev)
-    parked = torch.empty(L.metis_nvfp4_deferred_bytes(M, K), dtype=torch.uint8, device=dev)
-    need = L.metis_lowrank_project_rows_workspace_bytes(M, R, K)
+    parked = torch.empty(_deferred_bytes(M, K), dtype=torch.uint8, device=dev)
+    need = _lowrank_rows_workspace_bytes(M, R, K, dev.index or 0)
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
     rc = L.metis_nvfp4_quant_project_deferred(x2.data_ptr(), M, K, mode, v.data_ptr(), R, s.data_ptr(), xv.data_ptr(), t.data_ptr(),
                                               codes.data_ptr(), parked.data_ptr(), parked.numel(),
                                               None if ws is None else ws.data_ptr(), need, _stream())
-    check(rc, "metis_nvfp4_quant_project_deferred", (M, K, R))
+    if rc:
+        check(rc, "metis_nvfp4_quant_project_deferred", (M, K, R))
     return PackedNVFP4(codes, None, unit, M, K, mode, deferred=parked), xv, t
 
 
@@ -1299,12 +1377,13 @@ def quantize_project_decode(x2: torch.Tensor, v: torch.Tensor, mode: int = MODE_
     v = v.contiguous()
     codes = torch.empty(M, K // 2, dtype=torch.uint8, device=dev)
     unit = torch.empty(1, dtype=torch.float32, device=dev)
-    parked = torch.empty(L.metis_nvfp4_deferred_bytes(M, K), dtype=torch.uint8, device=dev)
-    need = L.metis_lowrank_project_workspace_bytes(M, R, K)
+    parked = torch.empty(_deferred_bytes(M, K), dtype=torch.uint8, device=dev)
+    need = _lowrank_workspace_bytes(M, R, K)
     pending = torch.empty(need, dtype=torch.uint8, device=dev)
     rc = L.metis_decode_quant_project_deferred(x2.data_ptr(), M, K, mode, codes.data_ptr(), parked.data_ptr(), parked.numel(),
                                                v.data_ptr(), R, pending.data_ptr(), need, _stream())
-    check(rc, "metis_decode_quant_project_deferred", (M, K, R))
+    if rc:
+        check(rc, "metis_decode_quant_project_deferred", (M, K, R))
     return PackedNVFP4(codes, None, unit, M, K, mode, deferred=parked), pending
 
 
@@ -1329,7 +1408,8 @@ def lowrank_contract_tokens(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.d
     rc = L.metis_lowrank_contract_tokens(a.data_ptr(), a.stride(0), b.data_ptr(), Lt, C, R, out.data_ptr(),
                                          DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, int(transpose),
                                          ws.data_ptr(), need, _stream())
-    check(rc, "metis_lowrank_contract_tokens", (Lt, C, R))
+    if rc:
+        check(rc, "metis_lowrank_contract_tokens", (Lt, C, R))
     return out
 
 
@@ -1345,7 +1425,8 @@ def lowrank_scale_grad(g: torch.Tensor, xv: torch.Tensor, out_dtype: torch.dtype
     out = torch.empty(R, dtype=out_dtype, device=g.device)
     rc = load().metis_lowrank_scale_grad(g.data_ptr(), xv.data_ptr(), g.shape[0], R, out.data_ptr(),
                                          DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, _stream())
-    check(rc, "metis_lowrank_scale_grad", tuple(g.shape))
+    if rc:
+        check(rc, "metis_lowrank_scale_grad", tuple(g.shape))
     return out
 
 
@@ -1353,6 +1434,43 @@ def linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.b
                        center: torch.Tensor | None = None, split_k: bool = True,
                        reference_rounding: bool = False, a_operand: torch.Tensor | None = None) -> list[torch.Tensor]:
     return _linear_fwd_grouped(a, members, out_dtype, center, split_k, reference_rounding, a_operand)
+
+
+def _grouped_members(members, M: int, K: int, out_dtype: torch.dtype, dev, decode_layout: bool):
+    """(member array, outputs, tensors to keep until the launch is enqueued) of a grouped call.  decode_layout: cached weights
+    are streamed in that layout (whole lines per load instruction) by the decode-sized kernel."""
+    arr = (_lib.LinearMember * len(members))()
+    outs, keep = [], []
+    for i, (b, t, u, bias) in enumerate(members):
+        if b.cols != K:
+            raise ValueError(f"contraction mismatch: {K} vs {b.cols}")
+        r = ldt = 0
+        if t is not None:
+            if t.dtype != torch.bfloat16:
+                t = t.to(torch.bfloat16)
+            if u.dtype != torch.bfloat16 or not u.is_contiguous():
+                u = u.to(torch.bfloat16).contiguous()
+            r = t.shape[1]
+            if t.shape != (M, r) or u.shape != (b.rows, r):
+                raise ValueError("low-rank operands must be t[M, r], u[N, r]")
+            # a column slice of a stacked projection is taken as it is by the single-launch path
+            if not t.is_contiguous():
+                if M < 256 and K % 64 == 0 and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0:
+                    ldt = t.stride(0)
+                else:
+                    t = t.contiguous()
+        bias_f32 = bias is not None and bias.dtype == torch.float32
+        if bias is not None:
+            bias = bias.contiguous() if bias_f32 else bias.to(torch.bfloat16).contiguous()
+        out = torch.empty(M, b.rows, dtype=out_dtype, device=dev)
+        keep += [t, u, bias]
+        outs.append(out)
+        dec = decode_weight(b) if (decode_layout and b.persistent) else None
+        arr[i] = _lib.LinearMember(b.codes.data_ptr(), b.scales.data_ptr(), b.unit.data_ptr(),
+                                   None if t is None else t.data_ptr(), None if u is None else u.data_ptr(), r,
+                                   None if bias is None else bias.data_ptr(), out.data_ptr(), b.rows, int(bias_f32), ldt,
+                                   None if dec is None else dec.data_ptr())
+    return arr, outs, keep
 
 
 def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.bfloat16,
@@ -1373,6 +1491,18 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
     where grouped_operand_applies says the call reads ready operands."""
     M, K = a.rows, a.cols
     dev = a.codes.device
+    if a_operand is not None and split_k and grouped_operand_applies(a, [m[0] for m in members], [0 if m[1] is None else m[1].shape[1] for m in members],
+                                                                     center, reference_rounding):
+        # the usual decode step: every question below has its answer
+        arr, outs, keep = _grouped_members(members, M, K, out_dtype, dev, decode_layout_weights)
+        need, _ = _grouped_plan(M, K, tuple([m[0].rows for m in members]), dev.index or 0)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+        rc = load().metis_linear_fwd_grouped_operand(a_operand.data_ptr(), a.unit.data_ptr(), M, K, ctypes.addressof(arr), len(members),
+                                                     DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, MODE_PB16,
+                                                     None if ws is None else ws.data_ptr(), need, _stream())
+        if rc:
+            check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
+        return outs
     rounded = (reference_rounding and (center is None or center.dtype == torch.bfloat16) and a.mode == MODE_PB16
                and all(m[0].mode == MODE_PB16 for m in members))
     takes = len(members) <= 4 and all(_decode_kernel_takes(M, m[0].rows, K, 0 if m[1] is None else m[1].shape[1]) for m in members)
@@ -1398,35 +1528,7 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
     if rounded and not takes:
         return [linear_fwd(a, b, t=t, u=u, bias=bias, out_dtype=out_dtype, split_k=split_k, reference_rounding=True)
                 for b, t, u, bias in members]
-    arr = (_lib.LinearMember * len(members))()
-    outs, keep = [], []
-    for i, (b, t, u, bias) in enumerate(members):
-        if b.cols != K:
-            raise ValueError(f"contraction mismatch: {K} vs {b.cols}")
-        r = ldt = 0
-        if t is not None:
-            t, u = t.to(torch.bfloat16), u.to(torch.bfloat16).contiguous()
-            r = t.shape[1]
-            if t.shape != (M, r) or u.shape != (b.rows, r):
-                raise ValueError("low-rank operands must be t[M, r], u[N, r]")
-            # a column slice of a stacked projection is taken as it is by the single-launch path
-            strided_ok = M < 256 and K % 64 == 0 and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
-            if t.is_contiguous() or not strided_ok:
-                t = t.contiguous()
-            else:
-                ldt = t.stride(0)
-        bias_f32 = bias is not None and bias.dtype == torch.float32
-        if bias is not None:
-            bias = bias.contiguous() if bias_f32 else bias.to(torch.bfloat16).contiguous()
-        out = torch.empty(M, b.rows, dtype=out_dtype, device=dev)
-        keep += [t, u, bias]
-        outs.append(out)
-        # a cached weight is streamed in its decode layout (whole lines per load instruction) by the decode-sized kernel
-        dec = decode_weight(b) if (b.persistent and takes and M < 256 and decode_layout_weights) else None
-        arr[i] = _lib.LinearMember(b.codes.data_ptr(), b.scales.data_ptr(), b.unit.data_ptr(),
-                                   None if t is None else t.data_ptr(), None if u is None else u.data_ptr(), r,
-                                   None if bias is None else bias.data_ptr(), out.data_ptr(), b.rows, int(bias_f32), ldt,
-                                   None if dec is None else dec.data_ptr())
+    arr, outs, keep = _grouped_members(members, M, K, out_dtype, dev, takes and M < 256 and decode_layout_weights)
     L = load()
     ap = ctypes.cast(arr, ctypes.c_void_p)
     # split-K scratch (long K, few columns) and whether a centre fits the launch: functions of the shape alone
@@ -1441,14 +1543,16 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
         aop = a_operand if a_operand is not None else decode_operand(a, op_mode, None, rotate=rotate)
         rc = L.metis_linear_fwd_grouped_operand(aop.data_ptr(), a.unit.data_ptr(), M, K, ap, len(members), dt, op_mode,
                                                 None if ws is None else ws.data_ptr(), need, _stream())
-        check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
+        if rc:
+            check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
         return outs
     if operand:
         # (a quantizer call that deferred its scale bytes never gets them: the operand kernel forms them on the way)
         aop = a_operand if a_operand is not None else decode_operand(a, MODE_PB16, center)
         rc = L.metis_linear_fwd_grouped_operand(aop.data_ptr(), a.unit.data_ptr(), M, K, ap, len(members), dt, MODE_PB16,
                                                 None if ws is None else ws.data_ptr(), need, _stream())
-        check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
+        if rc:
+            check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
         return outs
     # the activation's decode layout (written by its quantizer) in place of the row-major packing: wide runs only
     a_dec = a.decode_layout if (takes and K % 256 == 0 and all(m[0].scales.data_ptr() % 8 == 0 for m in members)) else None
@@ -1462,7 +1566,8 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
             rc = L.metis_linear_fwd_grouped_centered(a_codes, a_scales, a.unit.data_ptr(), M, K, ap,
                                                      len(members), dt, center.data_ptr(),
                                                      None if ws is None else ws.data_ptr(), need, _stream())
-            check(rc, "metis_linear_fwd_grouped_centered", (M, K, [m[0].rows for m in members]))
+            if rc:
+                check(rc, "metis_linear_fwd_grouped_centered", (M, K, [m[0].rows for m in members]))
             return outs
         # two passes: W^ center as a binary32 bias per member
         shifted = []
@@ -1473,7 +1578,8 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
     fn = L.metis_linear_fwd_grouped_bf16 if rounded else L.metis_linear_fwd_grouped
     rc = fn(a_codes, a_scales, a.unit.data_ptr(), M, K, ap, len(members),
             dt, None if ws is None else ws.data_ptr(), need, _stream())
-    check(rc, "metis_linear_fwd_grouped_bf16" if rounded else "metis_linear_fwd_grouped", (M, K, [m[0].rows for m in members]))
+    if rc:
+        check(rc, "metis_linear_fwd_grouped_bf16" if rounded else "metis_linear_fwd_grouped", (M, K, [m[0].rows for m in members]))
     return outs
 
 
@@ -1502,11 +1608,13 @@ def linear_dgrad(dy: PackedNVFP4, wt: PackedNVFP4, out_dtype: torch.dtype = torc
         rc = load().metis_linear_dgrad_ws(dy.codes.data_ptr(), dy.scales.data_ptr(), dy.unit.data_ptr(), wt.codes.data_ptr(),
                                           wt.scales.data_ptr(), wt.unit.data_ptr(), L, N, K, out.data_ptr(), dt,
                                           ws.data_ptr(), ws.numel(), _stream())
-        check(rc, "metis_linear_dgrad_ws", (L, N, K))
+        if rc:
+            check(rc, "metis_linear_dgrad_ws", (L, N, K))
         return out
     rc = load().metis_linear_dgrad(dy.codes.data_ptr(), dy.scales.data_ptr(), dy.unit.data_ptr(), wt.codes.data_ptr(),
                                    wt.scales.data_ptr(), wt.unit.data_ptr(), L, N, K, out.data_ptr(), dt, _stream())
-    check(rc, "metis_linear_dgrad", (L, N, K))
+    if rc:
+        check(rc, "metis_linear_dgrad", (L, N, K))
     return out
 
 
@@ -1524,10 +1632,12 @@ def linear_wgrad(dyt: PackedNVFP4, xt: PackedNVFP4, out_dtype: torch.dtype = tor
         rc = load().metis_linear_wgrad_ws(dyt.codes.data_ptr(), dyt.scales.data_ptr(), dyt.unit.data_ptr(),
                                           xt.codes.data_ptr(), xt.scales.data_ptr(), xt.unit.data_ptr(), L, N, K,
                                           out.data_ptr(), dt, ws.data_ptr(), ws.numel(), _stream())
-        check(rc, "metis_linear_wgrad_ws", (L, N, K))
+        if rc:
+            check(rc, "metis_linear_wgrad_ws", (L, N, K))
         return out
     rc = load().metis_linear_wgrad(dyt.codes.data_ptr(), dyt.scales.data_ptr(), dyt.unit.data_ptr(),
                                    xt.codes.data_ptr(), xt.scales.data_ptr(), xt.unit.data_ptr(), L, N, K,
                                    out.data_ptr(), dt, _stream())
-    check(rc, "metis_linear_wgrad", (L, N, K))
+    if rc:
+        check(rc, "metis_linear_wgrad", (L, N, K))
     return out

@@ -86,7 +86,6 @@ class _NVFP4Base(BlockQuantFunc):
         return off
 
     @classmethod
-    @torch.no_grad()
     def pack(cls, x: torch.Tensor, col: bool = False, noise: torch.Tensor | None = None,
              arith: torch.dtype | None = None, center: torch.Tensor | None = None, rht: int | None = None,
              deferred: bool = False, pad_rows: int | None = None) -> ops.PackedNVFP4:
@@ -97,6 +96,13 @@ class _NVFP4Base(BlockQuantFunc):
         deferred: round-to-nearest rows only: one launch now, the scale bytes when (and if) somebody reads them (ops.quantize).
         pad_rows: x stands for a tensor of pad_rows rows whose rows beyond x's own have a zero residual: col=True packs that
         tensor, row blocks are those of x; either way the random stream advances as for the larger tensor."""
+        if torch.is_grad_enabled():
+            with torch.no_grad():
+                return cls._pack(x, col, noise, arith, center, rht, deferred, pad_rows)
+        return cls._pack(x, col, noise, arith, center, rht, deferred, pad_rows)
+
+    @classmethod
+    def _pack(cls, x, col, noise, arith, center, rht, deferred, pad_rows) -> ops.PackedNVFP4:
         _need_gpu(x)
         drawn = x.numel() if pad_rows is None else pad_rows * x.shape[-1]
         more = {"pad_rows": pad_rows} if (col and pad_rows is not None) else {}
