@@ -1179,20 +1179,23 @@ class BitLinear(nn.Module):
                 or (centered and not in_operand and any(F._mean_in_operand(shared_input, p) or p.rht is not None for p in packed))):
             return None
         x2 = _flat2d(x).to(cd)
-        _, v, s = self._stacked_factors(x2.device)
-        _, t_all = ops.lowrank_project(x2, v, s)
+        ranks = [m.args.forward_svd_rank for m in members]
+        if sum(ranks) in ops.ONE_PASS_RANKS:
+            _, v, s = self._stacked_factors(x2.device)
+            projected = ops.lowrank_project(x2, v, s)[1].split(ranks, dim=1)
+        else:
+            # wider than one pass of the kernel (q/k/v of rank 128): a pass per member, each of a rank that it takes
+            projected = [ops.lowrank_project(x2, m.vlinear.weight.to(cd), m.s.to(cd))[1] for m in members]
         f32 = F.compute_dtype == torch.float32
-        calls, c0 = [], 0
-        for m, p_res in zip(members, packed):
-            r = m.args.forward_svd_rank
+        calls = []
+        for m, p_res, t in zip(members, packed, projected):
             bias = m._modules["warmup_linear"].bias
             if centered and not in_operand:
                 w_mean = ops.matvec(p_res, shared_input.center32)          # the mean's share rides in a binary32 bias
                 bias = w_mean if bias is None else w_mean + m._bias_as(torch.float32)
             elif bias is not None:
                 bias = m._bias_as(torch.float32 if f32 else cd)
-            calls.append((p_res, t_all[:, c0:c0 + r], _param(m._modules["ulinear"], "weight").to(cd), bias))
-            c0 += r
+            calls.append((p_res, t, _param(m._modules["ulinear"], "weight").to(cd), bias))
         outs = ops.linear_fwd_tiled_grouped(px, calls, out_dtype=torch.float32 if f32 else torch.bfloat16,
                                             center=shared_input.mean if in_operand else None, reference_rounding=rounding)
         lead = x.shape[:-1]

@@ -1284,6 +1284,9 @@ def linear_fwd(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None = None,
     return out
 
 
+ONE_PASS_RANKS = (32, 64, 96, 128, 192, 256)      # of lowrank_project from 256 rows on: the kernel holds a row's R sums in registers
+
+
 def lowrank_project(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None = None):
     """Rank-r projection of the low-rank branch: xv = x2[M, K] . v[R, K]^T in bf16 (binary32 accumulation) and, with
     `s` [R], t = bf16(xv * s): returns xv or (xv, t).  Decode-sized batches (M < 256, R <= 256) run on the library's
@@ -1294,7 +1297,7 @@ def lowrank_project(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None = 
     common = (x2.is_cuda and x2.dtype == torch.bfloat16 and v.dtype == torch.bfloat16 and M > 0 and K % 64 == 0 and v.shape[1] == K
               and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 and (s is None or s.dtype == torch.bfloat16))
     small = common and M < 256 and R % 32 == 0 and 0 < R <= 256
-    large = common and M >= 256 and R in (32, 64, 96, 128, 192, 256)
+    large = common and M >= 256 and R in ONE_PASS_RANKS
     if not (small or large):
         xv = torch.matmul(x2, v.T)
         return xv if s is None else (xv, xv * s.to(xv.dtype))

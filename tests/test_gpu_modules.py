@@ -877,3 +877,37 @@ def test_merged_decode_launches_leave_the_layer_output_unchanged(mean_mode, fuse
     separate = run()
     assert seen == {"prepare": 0, "quant_project": 0}
     assert torch.equal(merged, separate)
+
+
+@pytest.mark.parametrize("ranks", [(32, 32, 32), (128, 128, 128), (32, 128), (64, 64, 64, 64)])
+def test_projection_group_at_prefill_size_keeps_every_rank_on_the_kernel(ranks, monkeypatch):
+    """Stacked factors wider than one pass of the rank-r kernel are projected member by member: no product of the group falls to
+    torch, and each member has the output that it has on its own."""
+    from metis_hip import BitLinear, LinearLowbit, MetisArgs, ops
+    K, N, M = 256, 384, 300
+    g = torch.Generator(device="cuda").manual_seed(5)
+    group = {"name": "g", "mean_cache": {}, "input_ref": None, "quantized_input": None, "members": []}
+    for r in ranks:
+        args = MetisArgs.direct_fp4(forward_svd_rank=r)
+        m = BitLinear(K, N, args=args, bias=False, dtype=torch.bfloat16, compute_dtype=torch.float32)
+        make = dict(args=args, device="cuda", storage_dtype=torch.bfloat16, compute_dtype=torch.float32)
+        m.warmup_linear, m.vlinear = LinearLowbit(K, N, bias=False, **make), LinearLowbit(K, r, bias=False, **make)
+        m.ulinear = torch.nn.Linear(r, N, bias=False, device="cuda", dtype=torch.bfloat16)
+        m.s = torch.nn.Parameter(torch.rand(r, generator=g, device="cuda").bfloat16() + 0.5)
+        with torch.no_grad():
+            for p in (m.warmup_linear.weight, m.vlinear.weight, m.ulinear.weight):
+                p.copy_(torch.randn(p.shape, generator=g, device="cuda") * 0.1)
+        m.is_svd_quant, m.activation_group = True, group
+        group["members"].append(m)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    seen, real = [], ops.lowrank_project
+    monkeypatch.setattr(ops, "lowrank_project", lambda x2, v, s=None: (seen.append(v.shape[0]), real(x2, v, s))[1])
+    with torch.no_grad():
+        got = [m(x) for m in group["members"]]
+        assert seen == ([sum(ranks)] if sum(ranks) in ops.ONE_PASS_RANKS else list(ranks)) and all(r in ops.ONE_PASS_RANKS for r in seen)
+        monkeypatch.setattr(BitLinear, "grouped_inference", False)
+        want = [m(x) for m in group["members"]]
+    for y, w in zip(got, want):
+        # the same products in binary32 sums of another order; where that moves bf16(x V^T s) across a midpoint, the rank-r term
+        # moves by one bf16 rounding (2^-8) of that factor
+        assert rel_fro(y.float().cpu(), w.float().cpu()) <= 2.0 ** -8
