@@ -58,10 +58,11 @@ template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
 __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v, const uint16_t* __restrict__ s,
     uint16_t* __restrict__ xv, uint16_t* __restrict__ t, int M, int K, float* __restrict__ part, uint2* __restrict__ codes,
-    uint16_t* __restrict__ q_amax, uint32_t* __restrict__ q_gmax, uint32_t fill_to, int rotate)
+    uint16_t* __restrict__ q_amax, uint32_t* __restrict__ q_gmax, uint32_t fill_to, int rotate, int R)
 {
     using F = NtForm<RT, ROWS, KS, NS>;
-    constexpr int R = RT * 32, STAGE = F::kStage, LPW = F::kLoads, XL = F::kXLoads, RPP = F::kRowsPerPiece, RB = F::kRowBytes;
+    const int col0 = QMODE < 0 ? (int)blockIdx.z * RT * 32 : 0; // R: all columns; the workgroup's are RT * 32 of them from here on
+    constexpr int STAGE = F::kStage, LPW = F::kLoads, XL = F::kXLoads, RPP = F::kRowsPerPiece, RB = F::kRowBytes;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];     // the ring, then the waves' partial sums
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     for (int j = 0; j < LPW; ++j) {
         const int row = ((j < XL ? j : j - XL) * F::kWaves + wave) * RPP + lane / F::kChunks;
         const int chunk = (lane % F::kChunks) ^ swz(row);
-        src[j] = (j < XL ? x + (int64_t)min(m0 + row, M - 1) * ldx : v + (int64_t)row * K) + chunk * 8;
+        src[j] = (j < XL ? x + (int64_t)min(m0 + row, M - 1) * ldx : v + (int64_t)(col0 + row) * K) + chunk * 8;
         upper |= (uint32_t)(chunk >> 3) << j;
     }
     auto issue = [&](int slot, int st) {
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     for (int j = 0; j < RT; ++j)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int col = j * 32 + 8 * g + 4 * (lane >> 5);
+            const int col = col0 + j * 32 + 8 * g + 4 * (lane >> 5);
             float sum[4];
             uint32_t h[4], ts[4];
 #pragma unroll
@@ -273,16 +274,34 @@ size_t lowrank_nt_workspace_bytes(int64_t M, int64_t R, int64_t K)
     return sl > 1 ? (size_t)sl * M * R * 4 : 0;
 }
 
+// Columns per workgroup of the 32-row form without the quantizer, for `groups` workgroups per column range.  Where these leave
+// compute units idle, the time is that of one workgroup's stages, and a stage of R columns takes the longer the more of v it
+// fetches and multiplies (and the wide forms' rings hold only two of them): workgroups of 32 or 64 columns side by side (gridDim.z)
+// read x again from L2 and finish sooner, with the same bits.  Microseconds at 32 | 64 | all R columns:
+//   411 x 1536, R = 192 (13 groups)    6.2 | 9.1 | 20.3         2103 x 1536, R = 128 (66)    7.8 | 9.4 | 15.1
+//   800 x 3584, R = 128 (75)           8.8 | 8.9 | 11.3         1500 x 3584, R = 192 (141)  17.0 | 12.8 | 15.7
+//   1500 x 3584, R = 64 (141)          8.2 |  -  | 8.8          4096 x 3584, R = 192 (384)  24.8 | 23.7 | 29.0
+//   2103 x 3584, R = 64 (198)          9.4 |  -  | 9.1          800 x 18944, R = 256 (400)  51.5 | 41.5 | 51.4
+//   4096 x 1536, R = 96 (128)          7.8 |  -  | 12.2         1500 x 18944, R = 128 (470) 45.8 | 32.0 | 29.7
+//   2103 x 3584, R = 96 (198)         13.6 |  -  | 10.9         8000 x 18944, R = 128 (500)  213 | 144  | 112
+// 32 columns up to about a workgroup per compute unit (a rank that has no half of 64 columns: up to 7/4), 64 up to 8/5 row groups.
+static int nt_column_group(int64_t groups, int64_t R)
+{
+    const int64_t cus = device_cus();
+    if (groups * (R / 32) * 8 <= cus * (R % 64 ? 14 : 9)) return 32;
+    return R % 64 == 0 && groups * 5 <= cus * 8 ? 64 : (int)R;
+}
+
 template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
-static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, const void* v, const void* s, void* xv, void* t, int64_t M, int64_t K,
+static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, const void* v, const void* s, void* xv, void* t, int64_t M, int64_t R, int64_t K,
                      float* part, void* codes, uint16_t* amax, uint32_t* gmax)
 {
     using F = NtForm<RT, ROWS, KS, NS>;
     static bool attr_set[64] = {};
     if (const int rc = allow_dynamic_lds((const void*)lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>, F::kLds, attr_set)) return rc;
-    hipLaunchKernelGGL((lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>), dim3((unsigned)((M + ROWS - 1) / ROWS), (unsigned)slices), dim3(F::kThreads), F::kLds, st,
+    hipLaunchKernelGGL((lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>), dim3((unsigned)((M + ROWS - 1) / ROWS), (unsigned)slices, (unsigned)(R / (RT * 32))), dim3(F::kThreads), F::kLds, st,
                        (const uint16_t*)x, ldx, (const uint16_t*)v, (const uint16_t*)s, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part,
-                       (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 13));
+                       (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 13), (int)R);
     return METIS_OK;
 }
 
@@ -317,11 +336,14 @@ int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, 
     //   16384 x 18944, R = 64, quantized  229 | 270     8192 x 14336, R = 64   76 | 60
     //   16384 x 3584, R = 192 (64 k | 128 k)  50 | 81   1024 x 3584, R = 192   17.1 | 16.2
     const bool tall = ((M + 63) / 64) * slices >= device_cus(), cut = K % 128 != 0;
-#define METIS_NT(RT, Q, ROWS, KS, NS, CUT) rc = launch_nt<RT, Q, ROWS, KS, NS, CUT>(slices, st, x, ldx, v, s, xv, t, M, K, part, codes, q.amax, q.gmax)
+#define METIS_NT(RT, Q, ROWS, KS, NS, CUT) rc = launch_nt<RT, Q, ROWS, KS, NS, CUT>(slices, st, x, ldx, v, s, xv, t, M, R, K, part, codes, q.amax, q.gmax)
 #define METIS_NT128(RT, Q, ROWS, NS) do { if (cut) METIS_NT(RT, Q, ROWS, 128, NS, true); else METIS_NT(RT, Q, ROWS, 128, NS, false); } while (0)
 #define METIS_NTF(RT, Q) do { if (tall) METIS_NT128(RT, Q, 64, 3); else METIS_NT128(RT, Q, 32, 3); } while (0)
 #define METIS_NTG(RT, NT, NW) do { if (tall) METIS_NT(RT, -1, 64, 64, NT, false); else METIS_NT128(RT, -1, 32, NW); } while (0)
-    if (qmode < 0) {
+    const int width = (qmode < 0 && !tall) ? nt_column_group(((M + 31) / 32) * slices, R) : (int)R;
+    if (width == 32 && R > 32) METIS_NT128(1, -1, 32, 3);
+    else if (width == 64 && R > 64) METIS_NT128(2, -1, 32, 3);
+    else if (qmode < 0) {
         if (R == 32) METIS_NTF(1, -1);
         else if (R == 64) METIS_NTF(2, -1);
         else if (R == 96) METIS_NTG(3, 4, 3);

@@ -694,6 +694,22 @@ def test_rank_r_projection_tiles_of_32_and_64_rows(M, R, K):
             assert torch.equal(qxv, xv) and torch.equal(qt, t)
 
 
+@pytest.mark.parametrize("M,R,K", [(256, 64, 64), (257, 256, 192), (411, 192, 1536), (1500, 256, 320), (2200, 128, 1088), (4768, 96, 192),
+                                   (4800, 96, 128), (800, 192, 4160), (8000, 128, 192), (260, 128, 18944)])
+def test_rank_r_projection_in_column_groups(M, R, K):
+    """Workgroups of 32, 64 or all R columns, with and without K slices, K that ends in half a stage, both sides of the rule's
+    lines: each 32 columns have the bits of the projection onto these 32 alone (the same stages, added in the same order)."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(6200 + M + R)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
+    v = (torch.randn(R, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    s = (torch.rand(R, generator=g, device="cuda") * 4 + 0.1).bfloat16()
+    xv, t = ops.lowrank_project(x, v, s)
+    for c in range(0, R, 32):
+        one, ts = ops.lowrank_project(x, v[c:c + 32], s[c:c + 32])
+        assert torch.equal(xv[:, c:c + 32], one) and torch.equal(t[:, c:c + 32], ts)
+
+
 @pytest.mark.parametrize("L,C,R", [(1000, 520, 32), (4096, 1536, 64), (4096, 8960, 32), (2048, 14336, 64), (777, 256, 128)])
 def test_rank_r_products_that_contract_over_tokens(L, C, R):
     """out[C, R] = sum_l a[l, C] b[l, R] (gradients of U and, transposed, of V): token slices added in a fixed order,
