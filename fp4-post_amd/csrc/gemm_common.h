@@ -164,7 +164,8 @@ __device__ __forceinline__ void tile_origin(int logical, int tiles_m, int tiles_
     n0 = tn * L_BN;
 }
 
-// The weight side of a tiled GEMM: up to four matrices that share the activation, their tile columns end to end.
+// The weight side of a tiled GEMM: up to four matrices that share the activation.  Each keeps the tile order and the split of K
+// that it has alone, so its result has the bits of its own call.
 constexpr int kTiledMembers = 4;
 struct TiledMember {
     const uint8_t* b;            // tiled operand (the packed kernel has its own)
@@ -172,30 +173,55 @@ struct TiledMember {
     const uint16_t *t, *u, *bias;
     void* out;
     int N, r, ldt, bias_f32;     // ldt: row stride of t (members may take columns of a stacked projection)
-    int tile0;                   // first tile column
+    int tiles_n;                 // tile columns
+    int nfull, part, nsplit;     // tiles that run unsplit, tiles after them that are split, splits of K of those
+    int full_x, part_x;          // workgroups per XCD for either kind,
+    int full_at, part_at;        // and where they begin among those of the group
+    int part0, slot0;            // split tiles of the members before, and their partial tiles in the workspace
 };
 struct TiledGroup {
     TiledMember m[kTiledMembers];
-    int count, tiles_n;
+    int count, full_x;           // full_x: workgroups per XCD for the unsplit tiles of all members; the split tiles come after them
 };
-__device__ __forceinline__ int tiled_member_of(const TiledGroup& g, int tn)
+// the matrix of workgroup li of its XCD
+__device__ __forceinline__ int tiled_member_at(const TiledGroup& g, int li, bool part)
 {
     int i = 0;
 #pragma unroll
-    for (int q = 1; q < kTiledMembers; ++q)
-        if (q < g.count && tn >= g.m[q].tile0) i = q;
+    for (int q = 0; q < kTiledMembers; ++q)
+        if (q < g.count && (part ? g.m[q].part_x : g.m[q].full_x) > 0 && li >= (part ? g.m[q].part_at : g.m[q].full_at)) i = q;
     return __builtin_amdgcn_readfirstlane(i);
 }
-// one matrix
-inline TiledGroup tiled_group_of(const void* b, const float* b_unit, int64_t N, const void* t, const void* u, int64_t r, const void* bias,
-                                 int bias_f32, void* out)
+// the member at the end of the group: plan_full tiles unsplit, the others in nsplit ranges of K (1: all unsplit)
+inline void tiled_group_add(TiledGroup& g, int64_t M, const void* b, const float* b_unit, int64_t N, const void* t, const void* u, int64_t r, int64_t ldt,
+                            const void* bias, int bias_f32, void* out, int nsplit, int plan_full)
 {
-    TiledGroup g = {};
-    g.m[0] = {(const uint8_t*)b, b_unit, (const uint16_t*)t, (const uint16_t*)u, (const uint16_t*)bias, out, (int)N, (int)r, (int)r, bias_f32, 0};
-    g.count = 1;
-    g.tiles_n = (int)((N + L_BN - 1) / L_BN);
-    return g;
+    TiledMember& m = g.m[g.count];
+    m = TiledMember{(const uint8_t*)b, b_unit, (const uint16_t*)t, (const uint16_t*)u, (const uint16_t*)bias, out, (int)N, (int)r, (int)ldt, bias_f32};
+    m.tiles_n = (int)((N + L_BN - 1) / L_BN);
+    const int total = (int)((M + L_BM - 1) / L_BM) * m.tiles_n;
+    m.nsplit = nsplit;
+    m.nfull = nsplit > 1 ? plan_full : total;
+    m.part = total - m.nfull;
+    m.full_x = (m.nfull + 7) / 8;
+    m.part_x = (m.part * nsplit + 7) / 8;
+    if (g.count) {
+        const TiledMember& p = g.m[g.count - 1];
+        m.part0 = p.part0 + p.part;
+        m.slot0 = p.slot0 + p.part * p.nsplit;
+    }
+    ++g.count;
+    g.full_x = 0;
+    for (int i = 0; i < g.count; ++i) {
+        g.m[i].full_at = g.full_x;
+        g.full_x += g.m[i].full_x;
+    }
+    for (int i = 0; i < g.count; ++i) g.m[i].part_at = i ? g.m[i - 1].part_at + g.m[i - 1].part_x : g.full_x;
 }
+// workgroups per XCD, split tiles and partial tiles of the whole group
+inline int tiled_group_blocks(const TiledGroup& g) { return g.m[g.count - 1].part_at + g.m[g.count - 1].part_x; }
+inline int tiled_group_parts(const TiledGroup& g) { return g.m[g.count - 1].part0 + g.m[g.count - 1].part; }
+inline int64_t tiled_group_slots(const TiledGroup& g) { return (int64_t)g.m[g.count - 1].slot0 + (int64_t)g.m[g.count - 1].part * g.m[g.count - 1].nsplit; }
 
 // Dynamic LDS above 64 KiB has to be allowed per kernel function and per device: done once for each pair.
 inline int allow_dynamic_lds(const void* fn, size_t bytes, bool (&done)[64])
@@ -217,20 +243,21 @@ inline int allow_dynamic_lds(const void* fn, size_t bytes, bool (&done)[64])
 // PB16 (every op of the reference rounded to bf16): the sum of the partial tiles is rounded to bf16 as the reference's
 // bf16 matmul rounds it, the bias is added in bf16, then the low-rank term and the final rounding.
 template <int OUT_F32, int PB16 = 0>
-__global__ __launch_bounds__(64) void gemm_splitk_reduce_kernel(const float* __restrict__ ws, int nsplit, int M, int tiles_m, int nfull,
-                                                                const TiledGroup grp)
+__global__ __launch_bounds__(64) void gemm_splitk_reduce_kernel(const float* __restrict__ ws, int M, int tiles_m, const TiledGroup grp)
 {
-    const int tiles_n = grp.tiles_n;
     constexpr int TN = 2, WTN = 64, NTHREADS = 512, TILE = L_BM * L_BN;
     __shared__ __attribute__((aligned(16))) uint16_t cw[32 * 72];
-    const int total = tiles_m * tiles_n - nfull;                 // split tiles
-    const int tile = blockIdx.x >> 5, wave = (blockIdx.x >> 2) & 7, i = blockIdx.x & 3;
+    int mi = 0;                                                  // the matrix of this split tile
+#pragma unroll
+    for (int q = 1; q < kTiledMembers; ++q)
+        if (q < grp.count && grp.m[q].part > 0 && (int)(blockIdx.x >> 5) >= grp.m[q].part0) mi = q;
+    mi = __builtin_amdgcn_readfirstlane(mi);
+    const int nsplit = grp.m[mi].nsplit, total = grp.m[mi].part;  // total: its split tiles
+    const int tile = (int)(blockIdx.x >> 5) - grp.m[mi].part0, wave = (blockIdx.x >> 2) & 7, i = blockIdx.x & 3;
     const int lane = threadIdx.x, tid = wave * 64 + lane;
     const int wm = wave / 4, wn = wave % 4;
     int m0, n0;
-    tile_origin(nfull + tile, tiles_m, tiles_n, m0, n0);
-    const int mi = tiled_member_of(grp, n0 / L_BN);
-    n0 -= grp.m[mi].tile0 * L_BN;
+    tile_origin(grp.m[mi].nfull + tile, tiles_m, grp.m[mi].tiles_n, m0, n0);
     const int N = grp.m[mi].N, r = grp.m[mi].r, ldt = grp.m[mi].ldt, bias_f32 = grp.m[mi].bias_f32;
     const uint16_t *bias = grp.m[mi].bias, *t = grp.m[mi].t, *u = grp.m[mi].u;
     void* out = grp.m[mi].out;
@@ -238,7 +265,7 @@ __global__ __launch_bounds__(64) void gemm_splitk_reduce_kernel(const float* __r
     if (mbase >= M || nbase >= N) return;
 
     float4 v[TN][4];
-    const float* src = ws + (size_t)tile * TILE + (size_t)(i * TN * 4) * (NTHREADS * 4) + tid * 4;
+    const float* src = ws + (size_t)(grp.m[mi].slot0 + tile) * TILE + (size_t)(i * TN * 4) * (NTHREADS * 4) + tid * 4;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -353,28 +380,24 @@ struct SplitPlan {
     int nsplit;
     int nfull;                   // leading tiles that run unsplit (a multiple of the compute units)
 };
-inline SplitPlan split_plan_tiles(int64_t tiles, int64_t K)
+inline SplitPlan split_plan(int64_t M, int64_t N, int64_t K)
 {
     const SplitPlan none = {1, 0};
-    if (K % BK) return none;
+    if (M < L_BM || N < L_BN || K % BK) return none;
+    const int64_t tiles = ((M + L_BM - 1) / L_BM) * ((N + L_BN - 1) / L_BN);
     const int cus = device_cus();
     if (cus <= 0 || cus % 8 || tiles > INT32_MAX) return none;
     int64_t part = tiles, nfull = 0;                            // tiles to split
     if (tiles * 2 > cus) {
         part = tiles % cus;
         nfull = tiles - part;
-        if (tiles < cus || part == 0 || part * 2 > cus || nfull > 4 * (int64_t)cus || false) return none;
+        if (tiles < cus || part == 0 || part * 2 > cus || nfull > 4 * (int64_t)cus) return none;
     }
     int64_t s = cus / part;
     if (s > K / BK / 8) s = K / BK / 8;
     if (s > 16) s = 16;
     if (s < 2) return none;
     return SplitPlan{(int)s, (int)nfull};
-}
-inline SplitPlan split_plan(int64_t M, int64_t N, int64_t K)
-{
-    if (M < L_BM || N < L_BN) return SplitPlan{1, 0};
-    return split_plan_tiles(((M + L_BM - 1) / L_BM) * ((N + L_BN - 1) / L_BN), K);
 }
 
 }  // namespace metis

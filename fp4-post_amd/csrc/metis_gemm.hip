@@ -554,11 +554,12 @@ static int launch_large(const void* a_codes, const void* a_scales, const float* 
     }
     if (split) {
         const dim3 rgrid((unsigned)(total - nfull) * 32u);
-        const TiledGroup grp = tiled_group_of(nullptr, nullptr, N, nullptr, nullptr, 0, nullptr, 0, out);   // (low-rank term and bias are in split 0)
+        TiledGroup grp = {};
+        tiled_group_add(grp, M, nullptr, nullptr, N, nullptr, nullptr, 0, 0, nullptr, 0, out, nsplit, nfull);   // (low-rank term and bias are in split 0)
         if (f32)
-            hipLaunchKernelGGL((gemm_splitk_reduce_kernel<1, 0>), rgrid, dim3(64), 0, st, ws, nsplit, Mi, tmi, nfull, grp);
+            hipLaunchKernelGGL((gemm_splitk_reduce_kernel<1, 0>), rgrid, dim3(64), 0, st, ws, Mi, tmi, grp);
         else
-            hipLaunchKernelGGL((gemm_splitk_reduce_kernel<0, 0>), rgrid, dim3(64), 0, st, ws, nsplit, Mi, tmi, nfull, grp);
+            hipLaunchKernelGGL((gemm_splitk_reduce_kernel<0, 0>), rgrid, dim3(64), 0, st, ws, Mi, tmi, grp);
         if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     }
     return METIS_OK;

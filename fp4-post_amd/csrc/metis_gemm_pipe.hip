@@ -412,8 +412,7 @@ __host__ __device__ constexpr int waitcnt_imm(int vm, int lgkm)
 
 template <int OUT_F32, int PB16, int SPLIT>
 __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
-    const uint8_t* __restrict__ a_xt, const float* __restrict__ a_unit, int M, int K, int tiles_m, float* __restrict__ ws, int nsplit,
-    int nfull, const TiledGroup grp)
+    const uint8_t* __restrict__ a_xt, const float* __restrict__ a_unit, int M, int K, int tiles_m, float* __restrict__ ws, const TiledGroup grp)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t xlds[];
     constexpr int TM = 4, TN = 2, WTN = 64, NWAVES = 8, NTHREADS = 512, NS = XT_NS;
@@ -422,33 +421,25 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / 4, wn = wave % 4;
 
-    // ---- tile assignment: contiguous range per XCD, groups of four tile rows (see tile_origin).  SPLIT: the first
-    //      nfull tiles (a multiple of 8) run unsplit, every XCD its share of them first; the rest have nsplit workgroups each.
-    const int tiles_n = grp.tiles_n, total = tiles_m * tiles_n;
+    // ---- tile assignment: the unsplit tiles of every matrix first, each matrix a contiguous range per XCD in groups of four
+    //      tile rows (see tile_origin).  SPLIT: then the tiles that nsplit workgroups share, likewise.
+    const int xcd = blockIdx.x & 7, li = blockIdx.x >> 3;
+    const int mi = tiled_member_at(grp, li, SPLIT != 0 && li >= grp.full_x);
+    const int nfull = grp.m[mi].nfull, tail = grp.m[mi].part, nsplit = grp.m[mi].nsplit;
     int logical, split = 0;
     bool partial = false;
-    if constexpr (SPLIT != 0) {
-        const int xcd = blockIdx.x & 7, li = blockIdx.x >> 3, full_x = nfull >> 3;
-        if (li < full_x) {
-            logical = xcd * full_x + li;
-        } else {
-            const int tail = total - nfull, tail_all = tail * nsplit, per_xcd = (tail_all + 7) / 8;
-            const int j = xcd * per_xcd + (li - full_x);
-            if (li - full_x >= per_xcd || j >= tail_all) return;
-            split = j / tail;                                    // consecutive workgroups of an XCD share a K range
-            logical = nfull + j % tail;
-            partial = true;
-        }
+    if (SPLIT == 0 || li < grp.full_x) {
+        logical = xcd * grp.m[mi].full_x + (li - grp.m[mi].full_at);
+        if (logical >= nfull) return;
     } else {
-        const int per_xcd = (total + 7) / 8;
-        logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-        if (logical >= total) return;
+        const int j = xcd * grp.m[mi].part_x + (li - grp.m[mi].part_at);
+        if (j >= tail * nsplit) return;
+        split = j / tail;                                        // consecutive workgroups of an XCD share a K range
+        logical = nfull + j % tail;
+        partial = true;
     }
     int m0, n0;
-    tile_origin(logical, tiles_m, tiles_n, m0, n0);
-    // the matrix that this tile column belongs to, columns counted from its first
-    const int mi = tiled_member_of(grp, n0 / L_BN);
-    n0 -= grp.m[mi].tile0 * L_BN;
+    tile_origin(logical, tiles_m, grp.m[mi].tiles_n, m0, n0);
     const int N = grp.m[mi].N, r = grp.m[mi].r, ldt = grp.m[mi].ldt, bias_f32 = grp.m[mi].bias_f32;
     const uint8_t* __restrict__ b_xt = grp.m[mi].b;
     const float* __restrict__ b_unit = grp.m[mi].b_unit;
@@ -582,7 +573,7 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
     __syncthreads();                                            // the ring is free for the epilogue
 
     float* wt = nullptr;
-    if (SPLIT != 0 && partial) wt = ws + (size_t)(split * (total - nfull) + (logical - nfull)) * (L_BM * L_BN) + tid * 4;
+    if (SPLIT != 0 && partial) wt = ws + (size_t)(grp.m[mi].slot0 + split * tail + (logical - nfull)) * (L_BM * L_BN) + tid * 4;
     auto store_partial = [&](float* dst, bool with_bias) {      // accumulator-register order, 1 KiB per store instruction
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -763,9 +754,9 @@ __global__ __launch_bounds__(512, 1) void gemm_xt_kernel(
 }
 
 // K splits of the pipelined kernel: the plan of the packed kernel (same tiles), with a stage of 32 k as the unit.
-static SplitPlan xt_split_plan(int64_t M, int64_t N, int64_t K, int64_t group_tiles = 0)
+static SplitPlan xt_split_plan(int64_t M, int64_t N, int64_t K)
 {
-    SplitPlan p = group_tiles && M >= L_BM ? split_plan_tiles(group_tiles, K) : split_plan(M, N, K);   // needs K % 64 == 0, M and N >= 256
+    SplitPlan p = split_plan(M, N, K);                          // needs K % 64 == 0, M and N >= 256
     if (p.nsplit > K / 32) p.nsplit = (int)(K / 32);
     return p.nsplit < 2 ? SplitPlan{1, 0} : p;
 }
@@ -781,37 +772,34 @@ size_t gemm_xt_workspace_bytes(int64_t M, int64_t N, int64_t K, int mode)
 }
 
 template <int OUT_F32, int PB16, int SPLIT>
-static int launch_xt(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const TiledGroup& grp, hipStream_t st, float* ws, int nsplit,
-                     int nfull)
+static int launch_xt(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const TiledGroup& grp, hipStream_t st, float* ws)
 {
     static bool attr_set[64] = {};
     const void* fn = (const void*)gemm_xt_kernel<OUT_F32, PB16, SPLIT>;
     const size_t lds_bytes = (size_t)XT_LDS;
     if (const int rc = allow_dynamic_lds(fn, lds_bytes, attr_set)) return rc;
     int tiles_m = (int)((M + L_BM - 1) / L_BM);
-    const int total = tiles_m * grp.tiles_n;
-    const unsigned grid_x = SPLIT ? 8u * (unsigned)(nfull / 8 + ((total - nfull) * nsplit + 7) / 8) : (unsigned)(((total + 7) / 8) * 8);
     const uint8_t* ae = (const uint8_t*)a_xt;
     int Mi = (int)M, Ki = (int)K;
     TiledGroup g = grp;
-    void* args[] = {&ae, &a_unit, &Mi, &Ki, &tiles_m, &ws, &nsplit, &nfull, &g};
-    if (hipLaunchKernel(fn, dim3(grid_x), dim3(512), args, lds_bytes, st) != hipSuccess) {
+    void* args[] = {&ae, &a_unit, &Mi, &Ki, &tiles_m, &ws, &g};
+    if (hipLaunchKernel(fn, dim3(8u * (unsigned)tiled_group_blocks(g)), dim3(512), args, lds_bytes, st) != hipSuccess) {
         (void)hipGetLastError();
         return METIS_E_LAUNCH;
     }
     if (SPLIT) {
-        const dim3 rgrid((unsigned)(total - nfull) * 32u);
-        hipLaunchKernelGGL((gemm_splitk_reduce_kernel<OUT_F32, PB16>), rgrid, dim3(64), 0, st, (const float*)ws, nsplit, Mi, tiles_m, nfull, g);
+        const dim3 rgrid((unsigned)tiled_group_parts(g) * 32u);
+        hipLaunchKernelGGL((gemm_splitk_reduce_kernel<OUT_F32, PB16>), rgrid, dim3(64), 0, st, (const float*)ws, Mi, tiles_m, g);
         if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     }
     return METIS_OK;
 }
 
-static int dispatch_xt(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const TiledGroup& grp, int out_dtype, int mode,
-                       SplitPlan plan, void* workspace, hipStream_t st)
+static int dispatch_xt(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const TiledGroup& grp, int out_dtype, int mode, void* workspace,
+                       hipStream_t st)
 {
-    const int f32 = out_dtype == METIS_DTYPE_F32, pb = mode == METIS_MODE_PB16, sp = plan.nsplit > 1;
-#define METIS_XT(F, P, S) launch_xt<F, P, S>(a_xt, a_unit, M, K, grp, st, (float*)workspace, plan.nsplit, plan.nfull)
+    const int f32 = out_dtype == METIS_DTYPE_F32, pb = mode == METIS_MODE_PB16, sp = tiled_group_parts(grp) > 0;
+#define METIS_XT(F, P, S) launch_xt<F, P, S>(a_xt, a_unit, M, K, grp, st, (float*)workspace)
     switch (f32 * 4 + pb * 2 + sp) {
         case 0: return METIS_XT(0, 0, 0);
         case 1: return METIS_XT(0, 0, 1);
@@ -846,34 +834,34 @@ int gemm_xt(const void* a_xt, const float* a_unit, const void* b_xt, const float
         plan = xt_split_plan(M, N, K);
         if (plan.nsplit > 1 && (((uintptr_t)workspace % 16) || workspace_bytes < gemm_xt_workspace_bytes(M, N, K, mode))) return METIS_E_WORKSPACE;
     }
-    return dispatch_xt(a_xt, a_unit, M, K, tiled_group_of(b_xt, b_unit, N, t, u, r, bias, bias_f32, out), out_dtype, mode, plan, workspace, st);
+    TiledGroup g = {};
+    tiled_group_add(g, M, b_xt, b_unit, N, t, u, r, r, bias, bias_f32, out, plan.nsplit, plan.nfull);
+    return dispatch_xt(a_xt, a_unit, M, K, g, out_dtype, mode, workspace, st);
 }
 
-// Several weight matrices against one activation in one launch, their tile columns end to end: the last, partly filled round of
-// 256 tiles is paid once instead of once per matrix, narrow matrices (k, v) ride along, and one launch adds the split tiles.
-// 16384 tokens, 3584 -> 18944 twice: 37 rounds in place of 2 x 18.5 (19); -> 3584 + 512 + 512: 4.5 in place of 3.5 + 0.5 + 0.5
-// with three reductions.
-static int64_t group_tile_columns(const GemmMember* members, int count)
-{
-    int64_t n = 0;
-    for (int i = 0; i < count; ++i) n += (members[i].N + L_BN - 1) / L_BN;
-    return n;
-}
-
+// Several weight matrices against one activation in one launch: the unsplit tiles of all of them, then the split ones, so that
+// the partly filled rounds of 256 workgroups meet, narrow matrices (k, v) ride along, and one launch adds the split tiles.  Every
+// matrix is split as it is alone: a prompt has the same bits in a group and member by member (with autograd).
 static bool group_shapes_ok(int64_t M, int64_t K, const GemmMember* members, int count)
 {
     if (M <= 0 || K <= 0 || K % 32 || !members || count < 1 || count > kTiledMembers || M > INT32_MAX - 256 || K > INT32_MAX) return false;
-    for (int i = 0; i < count; ++i)
+    int64_t tiles = 0;
+    for (int i = 0; i < count; ++i) {
         if (members[i].N <= 0 || members[i].N > INT32_MAX / 8) return false;
-    return ((M + L_BM - 1) / L_BM) * group_tile_columns(members, count) <= INT32_MAX / 16;
+        tiles += ((M + L_BM - 1) / L_BM) * ((members[i].N + L_BN - 1) / L_BN);
+    }
+    return tiles <= INT32_MAX / 16;
 }
 
 size_t gemm_xt_grouped_workspace_bytes(int64_t M, int64_t K, const GemmMember* members, int count)
 {
     if (!group_shapes_ok(M, K, members, count)) return 0;
-    const int64_t tiles = ((M + L_BM - 1) / L_BM) * group_tile_columns(members, count);
-    const SplitPlan p = xt_split_plan(M, 0, K, tiles);
-    return p.nsplit <= 1 ? 0 : (size_t)p.nsplit * (size_t)(tiles - p.nfull) * L_BM * L_BN * sizeof(float);
+    int64_t slots = 0;
+    for (int i = 0; i < count; ++i) {
+        const SplitPlan p = xt_split_plan(M, members[i].N, K);
+        if (p.nsplit > 1) slots += p.nsplit * (((M + L_BM - 1) / L_BM) * ((members[i].N + L_BN - 1) / L_BN) - p.nfull);
+    }
+    return (size_t)slots * L_BM * L_BN * sizeof(float);
 }
 
 int gemm_xt_grouped(const void* a_xt, const float* a_unit, int64_t M, int64_t K, const GemmMember* members, int count, int out_dtype, int mode,
@@ -894,17 +882,11 @@ int gemm_xt_grouped(const void* a_xt, const float* a_unit, int64_t M, int64_t K,
         if (((uintptr_t)m.b_codes % 16) || ((uintptr_t)m.out % 16) || ((uintptr_t)m.t % 16) || ((uintptr_t)m.u % 16) ||
             ((uintptr_t)m.bias % (m.bias_is_f32 ? 4 : 2)))
             return METIS_E_ARG;
-        g.m[i] = {(const uint8_t*)m.b_codes, m.b_unit, (const uint16_t*)m.t, (const uint16_t*)m.u, (const uint16_t*)m.bias, m.out, (int)m.N, (int)m.r,
-                  (int)ldt, m.bias_is_f32 != 0, g.tiles_n};
-        g.tiles_n += (int)((m.N + L_BN - 1) / L_BN);
+        const SplitPlan p = workspace ? xt_split_plan(M, m.N, K) : SplitPlan{1, 0};
+        tiled_group_add(g, M, m.b_codes, m.b_unit, m.N, m.t, m.u, m.r, ldt, m.bias, m.bias_is_f32 != 0, m.out, p.nsplit, p.nfull);
     }
-    g.count = count;
-    SplitPlan plan = {1, 0};
-    if (workspace) {
-        plan = xt_split_plan(M, 0, K, ((M + L_BM - 1) / L_BM) * g.tiles_n);
-        if (plan.nsplit > 1 && (((uintptr_t)workspace % 16) || workspace_bytes < gemm_xt_grouped_workspace_bytes(M, K, members, count))) return METIS_E_WORKSPACE;
-    }
-    return dispatch_xt(a_xt, a_unit, M, K, g, out_dtype, mode, plan, workspace, st);
+    if (workspace && (((uintptr_t)workspace % 16) || workspace_bytes < (size_t)tiled_group_slots(g) * L_BM * L_BN * sizeof(float))) return METIS_E_WORKSPACE;
+    return dispatch_xt(a_xt, a_unit, M, K, g, out_dtype, mode, workspace, st);
 }
 
 }  // namespace metis

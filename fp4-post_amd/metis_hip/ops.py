@@ -947,8 +947,9 @@ def tiled_group_applies(a: PackedNVFP4, weights, reference_rounding: bool) -> bo
 
 def linear_fwd_tiled_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.bfloat16, center: torch.Tensor | None = None,
                              reference_rounding: bool = False) -> list[torch.Tensor]:
-    """[linear_fwd_tiled(a, b, t=t, u=u, bias=bias, ...) for (b, t, u, bias) in members] in one launch: a projection group at
-    prefill size (tiled_group_applies).  t may be a column slice of a stacked projection.  center: as linear_fwd_tiled."""
+    """[linear_fwd_tiled(a, b, t=t, u=u, bias=bias, ...) for (b, t, u, bias) in members] in one launch, with the same bits: a
+    projection group at prefill size (tiled_group_applies).  t may be a column slice of a stacked projection.  center: as
+    linear_fwd_tiled."""
     if not tiled_group_applies(a, [m[0] for m in members], reference_rounding):
         raise ValueError("linear_fwd_tiled_grouped: outside the call's domain (see tiled_group_applies)")
     mode = MODE_PB16 if (reference_rounding and a.mode == MODE_PB16 and members[0][0].mode == MODE_PB16) else MODE_P32

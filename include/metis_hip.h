@@ -625,10 +625,10 @@ typedef struct metis_linear_member {
 size_t metis_linear_member_size(void);
 /*
  * metis_linear_fwd_tiled for a projection group at prefill size: one tiled activation [M, K] against up to four tiled weights in
- * one launch (their 256-wide tile columns end to end, one partly filled last round instead of one per weight).  members[i]:
+ * one launch (their partly filled rounds of workgroups meet, instead of one such round per weight).  members[i]:
  * b_codes = the tiled operand of metis_nvfp4_expand_tiled, b_unit, t / u / r / ldt (any ldt % 8 == 0 >= r here), bias, out, N;
- * b_scales and b_decode are not read.  Result i is that of metis_linear_fwd_tiled with the same operands; K is split as for one
- * product with the sum of the tile columns, so a split sum may be grouped differently.
+ * b_scales and b_decode are not read.  Result i is that of metis_linear_fwd_tiled with the same operands, bit for bit: K is
+ * split for every weight as it is for that weight alone.
  *   limits     as metis_linear_fwd_tiled; count 1 .. 4; N > 0
  *   workspace  metis_linear_tiled_grouped_workspace_bytes (0: not split), 16-byte aligned, no initialisation; NULL = never split
  */

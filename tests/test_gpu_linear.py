@@ -670,6 +670,34 @@ def test_projection_group_at_prefill_size_in_one_launch(M, K, ns, mode):
             ops.linear_fwd_tiled_grouped(bad, members * 5 if bad is px else members, reference_rounding=mode == 1)
 
 
+@pytest.mark.parametrize("M,K,ns,mode", [(411, 1536, (1536, 256, 256), 1), (411, 1536, (8960, 8960), 1), (300, 2048, (2048, 100, 512, 4), 0), (1000, 1024, (8960, 8960), 0),
+                                         (1000, 1024, (8960, 2304), 1), (4100, 192, (3584, 512, 516, 256), 0), (256, 4096, (768, 256), 1)])
+def test_projection_group_has_the_bits_of_its_products(M, K, ns, mode):
+    """Every member keeps its own split of K: whole, in the last tiles only, or not at all (narrow members, short K, many tiles);
+    with and without low-rank term and bias, each output equals its own call bit for bit, in both output types."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(6400 + M + len(ns))
+    r = 64
+    px = ops.quantize(torch.randn(M, K, generator=g, device="cuda").bfloat16(), mode)
+    stacked = torch.randn(M, r * len(ns), generator=g, device="cuda").bfloat16()
+    members = []
+    for i, n in enumerate(ns):
+        pw = ops.quantize((torch.randn(n, K, generator=g, device="cuda") / K ** 0.5).bfloat16(), mode)
+        pw.persistent = True
+        u = (torch.randn(n, r, generator=g, device="cuda") / r).bfloat16() if i != 1 else None
+        bias = None if i == 2 else torch.randn(n, generator=g, device="cuda").to(torch.float32 if (mode == 0 and i) else torch.bfloat16)
+        # (a narrow weight is not tiled on its own in exact mode, see tiled_group_applies: its operand is made here)
+        ops.expand_tiled(pw, mode=mode)
+        members.append((pw, stacked[:, i * r:(i + 1) * r] if u is not None else None, u, bias))
+    if not ops.tiled_group_applies(px, [m[0] for m in members], mode == 1):
+        members = [m for m in members if m[0].rows >= 256]
+    for dt in (torch.float32, torch.bfloat16):
+        got = ops.linear_fwd_tiled_grouped(px, members, out_dtype=dt, reference_rounding=mode == 1)
+        for (pw, t, u, bias), y in zip(members, got):
+            one = ops.linear_fwd_tiled(px, pw, t=None if t is None else t.contiguous(), u=u, bias=bias, out_dtype=dt, reference_rounding=mode == 1)
+            assert torch.equal(y, one), (pw.rows, float((y.double() - one.double()).abs().max()))
+
+
 @pytest.mark.parametrize("M,R,K", [(256, 96, 64), (257, 192, 192), (411, 256, 1536), (16385, 192, 128), (16384, 64, 192), (20000, 32, 320),
                                    (2103, 64, 18944), (300, 128, 4160), (16400, 96, 256)])
 def test_rank_r_projection_tiles_of_32_and_64_rows(M, R, K):
