@@ -35,9 +35,10 @@ template <int RT, int ROWS, int KS, int NS> struct NtForm {
     static constexpr int kStage = (ROWS + RT * 32) * kRowBytes;               // bytes of a stage: x rows, then v rows
     static constexpr int kLoads = kStage / 1024 / kWaves, kXLoads = ROWS / kRowsPerPiece / kWaves;   // 1 KiB loads per wave and stage; those of x
     static constexpr int kRowTiles = ROWS / 32, kParts = kWaves / kRowTiles;  // the waves of a row tile share the stage's k, 32 each
-    static constexpr int kLds = NS * kStage;
+    static constexpr int kHalves = 128 / KS;                                  // stages of a step of 128 k, each with sums of its own
+    static constexpr int kRed = kHalves * (kParts - 1) * kRowTiles * RT * 4096 + 64;   // partial sums of the waves, then their maxima
+    static constexpr int kLds = NS * kStage > kRed ? NS * kStage : kRed;
     static_assert((KS == 64 || KS == 128) && kParts * 32 == KS && kStage % (1024 * kWaves) == 0 && kXLoads >= 1, "every wave loads whole pieces and multiplies two steps of 16");
-    static_assert(((kParts - 1) * kRowTiles * RT * 4096 + 64) <= kLds, "the partial sums fit the ring");
 };
 // Leaves at most VM of the wave's vector memory operations in flight.  Assembly with a memory clobber: no load or store of
 // the loop may move across it, the counts at its uses rely on that.
@@ -53,7 +54,10 @@ template <int VM> __device__ __forceinline__ void nt_wait()
 // QMODE >= 0: the same pass also quantizes x (round to nearest, rows; METIS_MODE_P32 or _PB16 arithmetic): a stage holds one
 // block of 16 per thread, read back from LDS -- E2M1 codes, the block maximum parked as bf16, one partial tensor maximum per
 // workgroup: what quant_codes_contig_kernel leaves for a consumer that forms the scale bytes itself.
-// CUT: K % KS == 64.
+// CUT: K % 128 == 64.
+// Every form adds an element's products in the same order -- the four quarters of each step of 128 k in sums of their own, the
+// steps of a row tile from the same one on, the quarters' sums at the end -- so that a column of v gives the same bits alone
+// and beside any others.  Stages of 64 k therefore keep two sums per wave and element, one for each half of a step.
 template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
 __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v, const uint16_t* __restrict__ s,
@@ -67,19 +71,22 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m0 = blockIdx.x * ROWS;
-    // CUT (K % 64 == 0, KS = 128): the last stage has only its first half.  The lanes of the other half then fetch the
-    // first again, its waves do not multiply, its threads encode the first half's blocks once more (the same bytes).
+    // CUT (K % 64 == 0): the last step of 128 has only its first half.  The lanes of the other half (the second stage of that
+    // step, where a stage is 64) then fetch the first again, multiply zeros, and their threads encode the first half's blocks once
+    // more (the same bytes).
     // A template parameter: the branch would keep product and encoder from being interleaved (8192 x 4096: 27.4 -> 35.6 us).
-    const int steps_all = (K + KS - 1) / KS;
+    constexpr int NH = F::kHalves;
+    const int steps_all = (K + 127) / 128;
     const int per = (steps_all + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int first = (int)blockIdx.y * per, steps = max(0, min(steps_all, first + per) - first);
+    const int first = (int)blockIdx.y * per, wide_steps = max(0, min(steps_all, first + per) - first);
+    const int steps = wide_steps * NH;                          // stages
     // Every row tile starts at a different stage of its K range and wraps around: at any moment the workgroups then read
     // different column stripes of x instead of the same one.  With rows a multiple of 4 KiB long, pieces at the same offset
     // of every row can fall on the same few memory channels.  The binary32 sums of a tile are therefore added in an order
-    // that depends on the tile, the same for every call and with or without the quantizer.  (An offset of 13 stages per tile:
+    // that depends on the tile, the same for every call and with or without the quantizer.  (An offset of 13 steps per tile:
     // 8192 x 4096 from flushed caches 40 us, 45 with 5, 41-46 without; other row lengths within 2 %.)
-    const int rot = (rotate && steps > 0) ? (int)((blockIdx.x * (unsigned)rotate) % (unsigned)steps) : 0;
-    auto kof = [&](int st) { int q = st + rot; if (q >= steps) q -= steps; return (first + q) * KS; };
+    const int rot = (rotate && steps > 0) ? (int)((blockIdx.x * (unsigned)rotate) % (unsigned)wide_steps) : 0;
+    auto kof = [&](int st) { int q = st / NH + rot; if (q >= wide_steps) q -= wide_steps; return (first + q) * 128 + st % NH * KS; };
 
     // ---- loads go straight to LDS: piece p = j * waves + wave of a stage is 1 KiB, whole rows of x | v.  The 16-byte chunk c
     // of row q lies at position c ^ swz(q) of the row, so that the fragment reads (32 rows at the same chunk) spread over all
@@ -102,23 +109,25 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
         for (int j = 0; j < LPW; ++j) {
             const uint32_t dst = (uint32_t)(slot * STAGE + (j * F::kWaves + wave) * 1024);
             const uint16_t* g = src[j] + k0;
-            if (cut) g -= ((upper >> j) & 1u) * 64u;
+            if (cut) g -= KS == 64 ? 64u : ((upper >> j) & 1u) * 64u;
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(dst) : "memory");
         }
     };
 
-    float16_t acc[RT];
+    float16_t acc[NH][RT];
 #pragma unroll
-    for (int j = 0; j < RT; ++j)
+    for (int h = 0; h < NH; ++h)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[h][j][e] = 0.0f;
     // wave w: 32-row tile w % row tiles, k part w / row tiles of the stage; lane l of an operand: row l % 32, chunk 2 ks + l / 32
     const int wr = wave % F::kRowTiles, kp = wave / F::kRowTiles;
     const int lr = lane & 31;
     int foff[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) foff[ks] = lr * RB + (((kp * 4 + ks * 2 + (lane >> 5)) ^ swz(lr)) * 16);
-    auto multiply = [&](int slot, int k0) {
+    auto multiply = [&](int slot, int k0, float16_t (&sums)[RT]) {
         const bool out = CUT && k0 + kp * 32 >= K;              // a select, not a branch: product and encoder stay interleaved
         const unsigned char* b = lds + slot * STAGE;
 #pragma unroll
@@ -129,7 +138,7 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
             for (int j = 0; j < RT; ++j) {
                 bf16x8_t fb = *reinterpret_cast<const bf16x8_t*>(b + (ROWS + j * 32) * RB + foff[ks]);
                 if (out) fb = bf16x8_t{};
-                acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb, fa, acc[j], 0, 0, 0);
+                sums[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb, fa, sums[j], 0, 0, 0);
             }
         }
     };
@@ -163,21 +172,32 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     for (int p = 0; p < NS - 1; ++p)
         if (p < steps) issue(p, p);
     int slot = 0;
-    for (int st = 0; st < steps; ++st) {
-        if (st + NS - 1 > steps) nt_wait<0>();                 // fewer stages behind it than counted below
-        else if (st < NS - 1) nt_wait<(NS - 2) * LPW>();
-        else nt_wait<(NS - 2) * LPW + (NS - 1) * STORES>();
-        __syncthreads();
-        if (st + NS - 1 < steps) issue(slot == 0 ? NS - 1 : slot - 1, st + NS - 1);
-        const int k0 = kof(st);
-        multiply(slot, k0);
-        encode(slot, k0);
-        slot = slot + 1 == NS ? 0 : slot + 1;
+    for (int step = 0; step < steps; step += NH) {
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const int st = step + h;
+            if (st + NS - 1 > steps) nt_wait<0>();             // fewer stages behind it than counted below
+            else if (st < NS - 1) nt_wait<(NS - 2) * LPW>();
+            else nt_wait<(NS - 2) * LPW + (NS - 1) * STORES>();
+            __syncthreads();
+            if (st + NS - 1 < steps) issue(slot == 0 ? NS - 1 : slot - 1, st + NS - 1);
+            const int k0 = kof(st);
+            multiply(slot, k0, acc[h]);
+            encode(slot, k0);
+            slot = slot + 1 == NS ? 0 : slot + 1;
+        }
+    }
+    if constexpr (NH * RT > 12) {                               // R = 256: 256 sums per lane, left in the accumulation registers until they are read
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int j = 0; j < RT; ++j) asm volatile("" : "+a"(acc[h][j]));
     }
     __syncthreads();                                            // the ring is free
-    float* red = reinterpret_cast<float*>(lds);                 // [part - 1][row tile][j][e][lane], then the waves' maxima
+    float* red = reinterpret_cast<float*>(lds);                 // [half][part - 1][row tile][j][e][lane], then the waves' maxima
+    auto red_at = [&](int h, int p, int j, int e) -> float& { return red[((((h * (F::kParts - 1) + p) * F::kRowTiles + wr) * RT + j) * 16 + e) * 64 + lane]; };
     if constexpr (QMODE >= 0) {
-        float* smax = red + (F::kParts - 1) * F::kRowTiles * RT * 1024;
+        float* smax = red + F::kHalves * (F::kParts - 1) * F::kRowTiles * RT * 1024;
         const float wm = wave_max(gmax);
         if (lane == 0) smax[wave] = wm;
     }
@@ -185,13 +205,15 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     // every stage's k join the first in LDS, in ascending order.
     if (kp > 0) {
 #pragma unroll
-        for (int j = 0; j < RT; ++j)
+        for (int h = 0; h < NH; ++h)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) red[((((kp - 1) * F::kRowTiles + wr) * RT + j) * 16 + e) * 64 + lane] = acc[j][e];
+            for (int j = 0; j < RT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) red_at(h, kp - 1, j, e) = acc[h][j][e];
     }
     __syncthreads();
     if constexpr (QMODE >= 0) {
-        const float* smax = red + (F::kParts - 1) * F::kRowTiles * RT * 1024;
+        const float* smax = red + F::kHalves * (F::kParts - 1) * F::kRowTiles * RT * 1024;
         const uint32_t gid = blockIdx.y * gridDim.x + blockIdx.x, gsize = gridDim.x * gridDim.y;
         if (tid == 0) {
             float wm = smax[0];
@@ -212,9 +234,13 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
             uint32_t h[4], ts[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                sum[e] = acc[j][4 * g + e];
+                sum[e] = acc[0][j][4 * g + e];
 #pragma unroll
-                for (int p = 0; p + 1 < F::kParts; ++p) sum[e] += red[(((p * F::kRowTiles + wr) * RT + j) * 16 + 4 * g + e) * 64 + lane];
+                for (int h = 0; h < NH; ++h) {
+                    if (h) sum[e] += acc[h][j][4 * g + e];
+#pragma unroll
+                    for (int p = 0; p + 1 < F::kParts; ++p) sum[e] += red_at(h, p, j, 4 * g + e);
+                }
             }
             if (part) {                                         // one of several slices: the finishing kernel rounds
                 *reinterpret_cast<float4*>(part + ((int64_t)blockIdx.y * M + m) * R + col) = make_float4(sum[0], sum[1], sum[2], sum[3]);
@@ -339,7 +365,7 @@ int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, 
 #define METIS_NT(RT, Q, ROWS, KS, NS, CUT) rc = launch_nt<RT, Q, ROWS, KS, NS, CUT>(slices, st, x, ldx, v, s, xv, t, M, R, K, part, codes, q.amax, q.gmax)
 #define METIS_NT128(RT, Q, ROWS, NS) do { if (cut) METIS_NT(RT, Q, ROWS, 128, NS, true); else METIS_NT(RT, Q, ROWS, 128, NS, false); } while (0)
 #define METIS_NTF(RT, Q) do { if (tall) METIS_NT128(RT, Q, 64, 3); else METIS_NT128(RT, Q, 32, 3); } while (0)
-#define METIS_NTG(RT, NT, NW) do { if (tall) METIS_NT(RT, -1, 64, 64, NT, false); else METIS_NT128(RT, -1, 32, NW); } while (0)
+#define METIS_NTG(RT, NT, NW) do { if (!tall) METIS_NT128(RT, -1, 32, NW); else if (cut) METIS_NT(RT, -1, 64, 64, NT, true); else METIS_NT(RT, -1, 64, 64, NT, false); } while (0)
     const int width = (qmode < 0 && !tall) ? nt_column_group(((M + 31) / 32) * slices, R) : (int)R;
     if (width == 32 && R > 32) METIS_NT128(1, -1, 32, 3);
     else if (width == 64 && R > 64) METIS_NT128(2, -1, 32, 3);

@@ -738,6 +738,21 @@ def test_rank_r_projection_in_column_groups(M, R, K):
         assert torch.equal(xv[:, c:c + 32], one) and torch.equal(t[:, c:c + 32], ts)
 
 
+@pytest.mark.parametrize("M,R,K", [(16385, 96, 320), (16384, 128, 64), (16400, 192, 1088), (16321, 256, 192), (4096, 192, 4160), (4090, 96, 4096), (4100, 128, 8960)])
+def test_rank_r_columns_have_the_same_bits_at_every_width(M, R, K):
+    """The forms with 64 rows per workgroup, stages of 64 k and of 128, with and without K slices: 32 columns have the bits of the
+    projection onto these 32 alone, so that a group's common projection equals its members' own."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(6500 + M + R)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    v = (torch.randn(R, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    s = (torch.rand(R, generator=g, device="cuda") * 4 + 0.1).bfloat16()
+    xv, t = ops.lowrank_project(x, v, s)
+    for c in range(0, R, 32):
+        one, ts = ops.lowrank_project(x, v[c:c + 32], s[c:c + 32])
+        assert torch.equal(xv[:, c:c + 32], one) and torch.equal(t[:, c:c + 32], ts)
+
+
 @pytest.mark.parametrize("L,C,R", [(1000, 520, 32), (4096, 1536, 64), (4096, 8960, 32), (2048, 14336, 64), (777, 256, 128)])
 def test_rank_r_products_that_contract_over_tokens(L, C, R):
     """out[C, R] = sum_l a[l, C] b[l, R] (gradients of U and, transposed, of V): token slices added in a fixed order,
