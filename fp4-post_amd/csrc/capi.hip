@@ -515,6 +515,12 @@ int metis_lowrank_project_rows_ws(const void* x, int64_t ldx, const void* v, int
     return lowrank_nt(x, ldx, v, M, R, K, s, xv, t, (hipStream_t)stream, workspace, workspace_bytes);
 }
 
+int metis_lowrank_project_rows_grouped(const void* x, int64_t ldx, int64_t M, int64_t K, const metis_lowrank_factor* factors, int count, void* xv,
+                                       void* t, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return lowrank_nt_grouped(x, ldx, M, K, reinterpret_cast<const LowrankFactor*>(factors), count, xv, t, (hipStream_t)stream, workspace, workspace_bytes);
+}
+
 int metis_nvfp4_quant_project_deferred(const void* x, int64_t rows, int64_t cols, int mode, const void* v, int64_t R, const void* s,
                                        void* xv, void* t, void* codes, void* deferred, size_t deferred_bytes, void* workspace,
                                        size_t workspace_bytes, void* stream)

@@ -40,6 +40,35 @@ template <int RT, int ROWS, int KS, int NS> struct NtForm {
     static constexpr int kLds = NS * kStage > kRed ? NS * kStage : kRed;
     static_assert((KS == 64 || KS == 128) && kParts * 32 == KS && kStage % (1024 * kWaves) == 0 && kXLoads >= 1, "every wave loads whole pieces and multiplies two steps of 16");
 };
+// The factors of up to four projections of the same x, their columns side by side in xv and t: a group's members hand in
+// their own V and s (stacked copies would have to be made anew whenever one of them changes).
+struct NtFactors {
+    const uint16_t* v[kTiledMembers];
+    const uint16_t* s[kTiledMembers];
+    int end[kTiledMembers];                                    // columns up to and with this member; a multiple of 32
+};
+__device__ __forceinline__ int nt_member(const NtFactors& f, int col)
+{
+    int i = 0;
+#pragma unroll
+    for (int q = 0; q + 1 < kTiledMembers; ++q) i += col >= f.end[q];
+    return i;
+}
+__device__ __forceinline__ const uint16_t* nt_pick(const uint16_t* const (&p)[kTiledMembers], int i)
+{
+    return i == 0 ? p[0] : i == 1 ? p[1] : i == 2 ? p[2] : p[3];
+}
+// s of column col
+__device__ __forceinline__ const uint16_t* nt_s(const NtFactors& f, int col)
+{
+    const int i = nt_member(f, col);
+    return nt_pick(f.s, i) + (col - (i == 0 ? 0 : i == 1 ? f.end[0] : i == 2 ? f.end[1] : f.end[2]));
+}
+__device__ __forceinline__ const uint16_t* nt_v(const NtFactors& f, int col, int64_t K)
+{
+    const int i = nt_member(f, col);
+    return nt_pick(f.v, i) + (col - (i == 0 ? 0 : i == 1 ? f.end[0] : i == 2 ? f.end[1] : f.end[2])) * K;
+}
 // Leaves at most VM of the wave's vector memory operations in flight.  Assembly with a memory clobber: no load or store of
 // the loop may move across it, the counts at its uses rely on that.
 template <int VM> __device__ __forceinline__ void nt_wait()
@@ -60,8 +89,7 @@ template <int VM> __device__ __forceinline__ void nt_wait()
 // and beside any others.  Stages of 64 k therefore keep two sums per wave and element, one for each half of a step.
 template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
 __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
-    const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v, const uint16_t* __restrict__ s,
-    uint16_t* __restrict__ xv, uint16_t* __restrict__ t, int M, int K, float* __restrict__ part, uint2* __restrict__ codes,
+    const uint16_t* __restrict__ x, int64_t ldx, const NtFactors fac, uint16_t* __restrict__ xv, uint16_t* __restrict__ t, int M, int K, float* __restrict__ part, uint2* __restrict__ codes,
     uint16_t* __restrict__ q_amax, uint32_t* __restrict__ q_gmax, uint32_t fill_to, int rotate, int R)
 {
     using F = NtForm<RT, ROWS, KS, NS>;
@@ -99,7 +127,7 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     for (int j = 0; j < LPW; ++j) {
         const int row = ((j < XL ? j : j - XL) * F::kWaves + wave) * RPP + lane / F::kChunks;
         const int chunk = (lane % F::kChunks) ^ swz(row);
-        src[j] = (j < XL ? x + (int64_t)min(m0 + row, M - 1) * ldx : v + (int64_t)(col0 + row) * K) + chunk * 8;
+        src[j] = (j < XL ? x + (int64_t)min(m0 + row, M - 1) * ldx : nt_v(fac, col0 + row, K)) + chunk * 8;
         upper |= (uint32_t)(chunk >> 3) << j;
     }
     auto issue = [&](int slot, int st) {
@@ -226,7 +254,8 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     const int m = m0 + wr * 32 + lr;
     if (kp > 0 || m >= M) return;
 #pragma unroll
-    for (int j = 0; j < RT; ++j)
+    for (int j = 0; j < RT; ++j) {
+        const uint16_t* sj = t && !part ? nt_s(fac, col0 + j * 32) : nullptr;      // the 32 columns belong to one member
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const int col = col0 + j * 32 + 8 * g + 4 * (lane >> 5);
@@ -249,17 +278,17 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 h[e] = bf16_bits(sum[e]);
-                if (t) ts[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(s[col + e]));
+                if (t) ts[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(sj[8 * g + 4 * (lane >> 5) + e]));
             }
             *reinterpret_cast<uint2*>(xv + (int64_t)m * R + col) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
             if (t) *reinterpret_cast<uint2*>(t + (int64_t)m * R + col) = make_uint2(ts[0] | (ts[1] << 16), ts[2] | (ts[3] << 16));
         }
+    }
 }
 
 // xv = bf16(sum over slices, ascending), t = bf16(xv * s): four columns per thread
 __global__ __launch_bounds__(256) void lowrank_nt_finish_kernel(const float* __restrict__ part, int slices, int64_t MR, int R,
-                                                                const uint16_t* __restrict__ s, uint16_t* __restrict__ xv,
-                                                                uint16_t* __restrict__ t)
+                                                                const NtFactors fac, uint16_t* __restrict__ xv, uint16_t* __restrict__ t)
 {
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= MR) return;
@@ -271,10 +300,10 @@ __global__ __launch_bounds__(256) void lowrank_nt_finish_kernel(const float* __r
     const uint32_t h[4] = {bf16_bits(a.x), bf16_bits(a.y), bf16_bits(a.z), bf16_bits(a.w)};
     *reinterpret_cast<uint2*>(xv + i) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
     if (t) {
-        const int col = (int)(i % R);
+        const uint16_t* s = nt_s(fac, (int)(i % R));
         uint32_t ts[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ts[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(s[col + e]));
+        for (int e = 0; e < 4; ++e) ts[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(s[e]));
         *reinterpret_cast<uint2*>(t + i) = make_uint2(ts[0] | (ts[1] << 16), ts[2] | (ts[3] << 16));
     }
 }
@@ -319,15 +348,14 @@ static int nt_column_group(int64_t groups, int64_t R)
 }
 
 template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
-static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, const void* v, const void* s, void* xv, void* t, int64_t M, int64_t R, int64_t K,
+static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, const NtFactors& fac, void* xv, void* t, int64_t M, int64_t R, int64_t K,
                      float* part, void* codes, uint16_t* amax, uint32_t* gmax)
 {
     using F = NtForm<RT, ROWS, KS, NS>;
     static bool attr_set[64] = {};
     if (const int rc = allow_dynamic_lds((const void*)lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>, F::kLds, attr_set)) return rc;
     hipLaunchKernelGGL((lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>), dim3((unsigned)((M + ROWS - 1) / ROWS), (unsigned)slices, (unsigned)(R / (RT * 32))), dim3(F::kThreads), F::kLds, st,
-                       (const uint16_t*)x, ldx, (const uint16_t*)v, (const uint16_t*)s, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part,
-                       (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 13), (int)R);
+                       (const uint16_t*)x, ldx, fac, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part, (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 13), (int)R);
     return METIS_OK;
 }
 
@@ -336,12 +364,36 @@ static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, con
 int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
                hipStream_t st, void* workspace, size_t workspace_bytes, int qmode, void* codes, void* deferred, size_t deferred_size)
 {
-    if (M < 0 || R <= 0 || K <= 0 || ldx < K) return METIS_E_ARG;
+    if (R <= 0) return METIS_E_ARG;
+    const LowrankFactor one = {v, s, R};
+    return lowrank_nt_grouped(x, ldx, M, K, &one, 1, xv, t, st, workspace, workspace_bytes, qmode, codes, deferred, deferred_size);
+}
+
+int lowrank_nt_grouped(const void* x, int64_t ldx, int64_t M, int64_t K, const LowrankFactor* factors, int count, void* xv, void* t, hipStream_t st,
+                       void* workspace, size_t workspace_bytes, int qmode, void* codes, void* deferred, size_t deferred_size)
+{
+    if (M < 0 || K <= 0 || ldx < K || !factors || count < 1 || count > kTiledMembers) return METIS_E_ARG;
+    int64_t R = 0;
+    for (int i = 0; i < count; ++i) {
+        if (factors[i].r <= 0 || factors[i].r % 32 || factors[i].r > 256) return METIS_E_SHAPE;
+        R += factors[i].r;
+    }
     if ((R != 32 && R != 64 && R != 96 && R != 128 && R != 192 && R != 256) || K % 64 || ldx % 8) return METIS_E_SHAPE;
     if (M == 0) return METIS_OK;
     if (M > INT32_MAX - 64 || K > INT32_MAX) return METIS_E_ARG;
-    if (!x || !v || !xv || (t && !s)) return METIS_E_ARG;
-    if (((uintptr_t)x % 16) || ((uintptr_t)v % 16) || ((uintptr_t)xv % 8) || ((uintptr_t)t % 8) || ((uintptr_t)s % 2)) return METIS_E_ARG;
+    if (!x || !xv || ((uintptr_t)x % 16) || ((uintptr_t)xv % 8) || ((uintptr_t)t % 8)) return METIS_E_ARG;
+    NtFactors fac = {};
+    int col = 0;
+    for (int i = 0; i < kTiledMembers; ++i) {
+        if (i < count) {
+            const LowrankFactor& f = factors[i];
+            if (!f.v || (t && !f.s) || ((uintptr_t)f.v % 16) || ((uintptr_t)f.s % 2)) return METIS_E_ARG;
+            fac.v[i] = (const uint16_t*)f.v;
+            fac.s[i] = (const uint16_t*)f.s;
+            col += (int)f.r;
+        }
+        fac.end[i] = col;
+    }
     if (workspace && ((uintptr_t)workspace % 16)) return METIS_E_WORKSPACE;
     Workspace q = {nullptr, nullptr, nullptr};
     if (qmode >= 0) {
@@ -362,7 +414,7 @@ int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, 
     //   16384 x 18944, R = 64, quantized  229 | 270     8192 x 14336, R = 64   76 | 60
     //   16384 x 3584, R = 192 (64 k | 128 k)  50 | 81   1024 x 3584, R = 192   17.1 | 16.2
     const bool tall = ((M + 63) / 64) * slices >= device_cus(), cut = K % 128 != 0;
-#define METIS_NT(RT, Q, ROWS, KS, NS, CUT) rc = launch_nt<RT, Q, ROWS, KS, NS, CUT>(slices, st, x, ldx, v, s, xv, t, M, R, K, part, codes, q.amax, q.gmax)
+#define METIS_NT(RT, Q, ROWS, KS, NS, CUT) rc = launch_nt<RT, Q, ROWS, KS, NS, CUT>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax)
 #define METIS_NT128(RT, Q, ROWS, NS) do { if (cut) METIS_NT(RT, Q, ROWS, 128, NS, true); else METIS_NT(RT, Q, ROWS, 128, NS, false); } while (0)
 #define METIS_NTF(RT, Q) do { if (tall) METIS_NT128(RT, Q, 64, 3); else METIS_NT128(RT, Q, 32, 3); } while (0)
 #define METIS_NTG(RT, NT, NW) do { if (!tall) METIS_NT128(RT, -1, 32, NW); else if (cut) METIS_NT(RT, -1, 64, 64, NT, true); else METIS_NT(RT, -1, 64, 64, NT, false); } while (0)
@@ -391,8 +443,8 @@ int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, 
     if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     if (slices > 1) {
         const int64_t MR = M * R;
-        hipLaunchKernelGGL(lowrank_nt_finish_kernel, dim3((unsigned)((MR / 4 + 255) / 256)), dim3(256), 0, st, part, slices, MR, (int)R,
-                           (const uint16_t*)s, (uint16_t*)xv, (uint16_t*)t);
+        hipLaunchKernelGGL(lowrank_nt_finish_kernel, dim3((unsigned)((MR / 4 + 255) / 256)), dim3(256), 0, st, part, slices, MR, (int)R, fac,
+                           (uint16_t*)xv, (uint16_t*)t);
         if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     }
     return METIS_OK;

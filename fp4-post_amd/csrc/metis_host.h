@@ -189,6 +189,14 @@ int scale_grad(const void* g, const void* xv, int64_t L, int64_t R, void* out, i
 int lowrank_nt(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
                hipStream_t st, void* workspace = nullptr, size_t workspace_bytes = 0, int qmode = -1, void* codes = nullptr,
                void* deferred = nullptr, size_t deferred_size = 0);
+// the projections of up to four (V, s) pairs side by side in xv and t; the same layout as metis_lowrank_factor
+struct LowrankFactor {
+    const void *v, *s;
+    int64_t r;
+};
+int lowrank_nt_grouped(const void* x, int64_t ldx, int64_t M, int64_t K, const LowrankFactor* factors, int count, void* xv, void* t, hipStream_t st,
+                       void* workspace, size_t workspace_bytes, int qmode = -1, void* codes = nullptr, void* deferred = nullptr,
+                       size_t deferred_size = 0);
 size_t lowrank_nt_workspace_bytes(int64_t M, int64_t R, int64_t K);
 size_t lowrank_tn_workspace_bytes(int64_t L, int64_t C, int64_t R);
 int lowrank_tn(const void* a, int64_t lda, const void* b, int64_t L, int64_t C, int64_t R, void* out, int out_dtype, int transpose,

@@ -43,6 +43,11 @@ def _param(module: nn.Module, name: str) -> torch.Tensor:
     return p if p is not None else getattr(module, name)
 
 
+def _as_dtype(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """x.to(dtype) without the call where x has it already (half a microsecond; a prompt's groups make thirty)."""
+    return x if x.dtype == dtype else x.to(dtype)
+
+
 def _pkey(p: torch.Tensor) -> tuple:
     """Cache key of a parameter: its identity and storage as well as its version counter, so that a Parameter that is
     REPLACED (load_state_dict(assign=True), `m.s = nn.Parameter(...)`) is seen although a fresh one starts at the same
@@ -780,7 +785,7 @@ class _MetisFusedFunction(torch.autograd.Function):
         elif xv is None:
             # [L, r] rank-r projection and its product with s (bf16) on the library's kernels (split-K below 256 rows,
             # one pass over x from there on); the caller has it already when the quantizer's pass produced it
-            x2, vb, sb = _flat2d(x).to(cd), v.to(cd), s.to(cd)
+            x2, vb, sb = _as_dtype(_flat2d(x), cd), _as_dtype(v, cd), _as_dtype(s, cd)
             in_operand = isinstance(px, CenteredNVFP4) and F._mean_in_operand(px, p_res)
             target = px.residual if in_operand else px
             if (isinstance(px, PackedNVFP4) and p_res.rht is not None and ops.nv_decode_applies(px, [p_res], [vb.shape[0]])
@@ -1150,7 +1155,7 @@ class BitLinear(nn.Module):
         outs = ops.linear_fwd_grouped(px, calls, out_dtype=out_dtype, center=centre, reference_rounding=F.reference_rounding,
                                       a_operand=aop)
         lead = x.shape[:-1]
-        return {id(m): y.reshape(*lead, y.shape[-1]).to(F.compute_dtype) for m, y in zip(members, outs)}
+        return {id(m): _as_dtype(y.reshape(*lead, y.shape[-1]), F.compute_dtype) for m, y in zip(members, outs)}
 
     def _stacked_factors(self, device):
         """(key, V, s) of all members of the group stacked: one product gives every member's rank-r projection.  Kept on the
@@ -1168,7 +1173,7 @@ class BitLinear(nn.Module):
 
     def _forward_group_tiled(self, x: torch.Tensor, shared_input, members, packed):
         """_forward_group at prefill size (256 rows or more): one pass over x for all projections, one launch of the tiled GEMM
-        for all products, the same arithmetic as member by member (_MetisFusedFunction.forward)."""
+        for all products; every member has the bits that it has alone and with autograd (_MetisFusedFunction.forward)."""
         F = LinearLowbitFunction
         cd = torch.bfloat16
         centered = isinstance(shared_input, CenteredNVFP4)
@@ -1178,14 +1183,14 @@ class BitLinear(nn.Module):
         if (not ops.tiled_group_applies(px, packed, rounding)
                 or (centered and not in_operand and any(F._mean_in_operand(shared_input, p) or p.rht is not None for p in packed))):
             return None
-        x2 = _flat2d(x).to(cd)
-        ranks = [m.args.forward_svd_rank for m in members]
-        if sum(ranks) in ops.ONE_PASS_RANKS:
-            _, v, s = self._stacked_factors(x2.device)
-            projected = ops.lowrank_project(x2, v, s)[1].split(ranks, dim=1)
+        x2 = _as_dtype(_flat2d(x), cd)
+        factors = [(_as_dtype(_param(m._modules["vlinear"], "weight"), cd), _as_dtype(_param(m, "s"), cd)) for m in members]
+        if ops.lowrank_stack_applies(x2, factors):
+            v, s = zip(*factors)
+            projected = ops.lowrank_project(x2, ops.FactorStack(v), ops.FactorStack(s))[1].split([f.shape[0] for f in v], dim=1)
         else:
             # wider than one pass of the kernel (q/k/v of rank 128): a pass per member, each of a rank that it takes
-            projected = [ops.lowrank_project(x2, m.vlinear.weight.to(cd), m.s.to(cd))[1] for m in members]
+            projected = [ops.lowrank_project(x2, v, s)[1] for v, s in factors]
         f32 = F.compute_dtype == torch.float32
         calls = []
         for m, p_res, t in zip(members, packed, projected):
@@ -1195,11 +1200,10 @@ class BitLinear(nn.Module):
                 bias = w_mean if bias is None else w_mean + m._bias_as(torch.float32)
             elif bias is not None:
                 bias = m._bias_as(torch.float32 if f32 else cd)
-            calls.append((p_res, t, _param(m._modules["ulinear"], "weight").to(cd), bias))
-        outs = ops.linear_fwd_tiled_grouped(px, calls, out_dtype=torch.float32 if f32 else torch.bfloat16,
-                                            center=shared_input.mean if in_operand else None, reference_rounding=rounding)
+            calls.append((p_res, t, _as_dtype(_param(m._modules["ulinear"], "weight"), cd), bias))
+        outs = ops._linear_fwd_tiled_grouped(px, calls, torch.float32 if f32 else torch.bfloat16, shared_input.mean if in_operand else None, rounding)
         lead = x.shape[:-1]
-        return {id(m): y.reshape(*lead, y.shape[-1]).to(F.compute_dtype) for m, y in zip(members, outs)}
+        return {id(m): _as_dtype(y.reshape(*lead, y.shape[-1]), F.compute_dtype) for m, y in zip(members, outs)}
 
     def _bias_as(self, dtype: torch.dtype) -> torch.Tensor:
         """The residual branch's bias in `dtype`, converted once per parameter version (decode calls are launch-bound)."""

@@ -952,6 +952,10 @@ def linear_fwd_tiled_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = t
     linear_fwd_tiled."""
     if not tiled_group_applies(a, [m[0] for m in members], reference_rounding):
         raise ValueError("linear_fwd_tiled_grouped: outside the call's domain (see tiled_group_applies)")
+    return _linear_fwd_tiled_grouped(a, members, out_dtype, center, reference_rounding)
+
+
+def _linear_fwd_tiled_grouped(a: PackedNVFP4, members, out_dtype, center, reference_rounding) -> list[torch.Tensor]:
     mode = MODE_PB16 if (reference_rounding and a.mode == MODE_PB16 and members[0][0].mode == MODE_PB16) else MODE_P32
     if center is not None and mode != MODE_PB16:
         raise ValueError("a centre inside the operand belongs to reference_rounding")
@@ -976,7 +980,10 @@ class _TiledBatch:
         M = self.a.rows
         r = ldt = 0
         if t is not None:
-            t, u = t.to(torch.bfloat16), u.to(torch.bfloat16).contiguous()
+            if t.dtype != torch.bfloat16:
+                t = t.to(torch.bfloat16)
+            if u.dtype != torch.bfloat16 or not u.is_contiguous():
+                u = u.to(torch.bfloat16).contiguous()
             r = t.shape[1]
             if t.shape != (M, r) or u.shape != (b.rows, r):
                 raise ValueError("low-rank operands must be t[M, r], u[N, r]")
@@ -998,7 +1005,7 @@ class _TiledBatch:
         a, dev = self.a, self.ax.device
         need = _tiled_group_workspace_bytes(a.rows, a.cols, tuple(self.rows), dev.index or 0)
         ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-        rc = load().metis_linear_fwd_tiled_grouped(self.ax.data_ptr(), a.unit.data_ptr(), a.rows, a.cols, ctypes.cast(self.members, ctypes.c_void_p),
+        rc = load().metis_linear_fwd_tiled_grouped(self.ax.data_ptr(), a.unit.data_ptr(), a.rows, a.cols, ctypes.addressof(self.members),
                                                    len(self.rows), DTYPE_F32 if self.out_dtype == torch.float32 else DTYPE_BF16, self.mode,
                                                    None if ws is None else ws.data_ptr(), need, _stream())
         if rc:
@@ -1288,15 +1295,72 @@ def linear_fwd(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None = None,
 ONE_PASS_RANKS = (32, 64, 96, 128, 192, 256)      # of lowrank_project from 256 rows on: the kernel holds a row's R sums in registers
 
 
-def lowrank_project(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None = None):
+class FactorStack:
+    """V (or s) of up to four members of a projection group on top of each other, each where it is: what lowrank_project takes
+    for one pass over their common x (lowrank_stack_applies).  Nothing is copied, so nothing is outdated by a write to a member."""
+
+    def __init__(self, parts):
+        self.parts = parts
+        self.shape = (sum([p.shape[0] for p in parts]), *parts[0].shape[1:])
+
+
+def _lowrank_operands(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None) -> bool:
+    """The operands have a form that the library's projection kernels read (shapes aside)."""
+    M, K = x2.shape
+    return (x2.is_cuda and x2.dtype == torch.bfloat16 and v.dtype == torch.bfloat16 and M > 0 and K % 64 == 0 and v.shape[1] == K
+            and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 and (s is None or s.dtype == torch.bfloat16))
+
+
+def lowrank_stack_applies(x2: torch.Tensor, factors) -> bool:
+    """lowrank_project takes the (v, s) pairs of a projection group as FactorStacks: 256 rows or more, every rank and their sum
+    ranks of the one-pass kernel.  Column for column the bits of the members' own projections."""
+    M, K = x2.shape
+    if M < 256 or len(factors) > 4:
+        return False
+    total = 0
+    for v, s in factors:
+        r = v.shape[0]
+        if r not in ONE_PASS_RANKS or v.shape[1] != K or v.dtype != torch.bfloat16 or s.dtype != torch.bfloat16:
+            return False
+        total += r
+    return total in ONE_PASS_RANKS and _lowrank_operands(x2, *factors[0])
+
+
+_FactorArrays = [None] + [ctypes.c_int64 * (3 * n) for n in range(1, 5)]     # metis_lowrank_factor is three 64-bit words
+
+
+def _lowrank_project_stack(x2: torch.Tensor, v: FactorStack, s: FactorStack):
+    (M, K), R = x2.shape, v.shape[0]
+    keep, words = [], []
+    for a, b in zip(v.parts, s.parts):
+        if not a.is_contiguous():
+            a = a.contiguous()
+        if not b.is_contiguous():
+            b = b.contiguous()
+        keep.append((a, b))
+        words += (a.data_ptr(), b.data_ptr(), a.shape[0])
+    arr = _FactorArrays[len(keep)](*words)
+    xv = torch.empty(M, R, dtype=torch.bfloat16, device=x2.device)
+    t = torch.empty_like(xv)
+    need = _lowrank_rows_workspace_bytes(M, R, K, x2.device.index or 0)
+    ws = torch.empty(need, dtype=torch.uint8, device=x2.device) if need else None
+    rc = load().metis_lowrank_project_rows_grouped(x2.data_ptr(), x2.stride(0), M, K, ctypes.addressof(arr), len(keep), xv.data_ptr(), t.data_ptr(),
+                                                   None if ws is None else ws.data_ptr(), need, _stream())
+    if rc:
+        check(rc, "metis_lowrank_project_rows_grouped", (M, [a.shape[0] for a, _ in keep], K))
+    return xv, t
+
+
+def lowrank_project(x2: torch.Tensor, v: "torch.Tensor | FactorStack", s: "torch.Tensor | FactorStack | None" = None):
     """Rank-r projection of the low-rank branch: xv = x2[M, K] . v[R, K]^T in bf16 (binary32 accumulation) and, with
     `s` [R], t = bf16(xv * s): returns xv or (xv, t).  Decode-sized batches (M < 256, R <= 256) run on the library's
     split-K kernel, larger ones (R in 32 / 64 / 96 / 128 / 192 / 256) on its one-pass kernel; other shapes are a torch
-    matmul."""
+    matmul.  FactorStacks (lowrank_stack_applies): the members' columns side by side."""
+    if isinstance(v, FactorStack):
+        return _lowrank_project_stack(x2, v, s)
     M, K = x2.shape
     R = v.shape[0]
-    common = (x2.is_cuda and x2.dtype == torch.bfloat16 and v.dtype == torch.bfloat16 and M > 0 and K % 64 == 0 and v.shape[1] == K
-              and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 and (s is None or s.dtype == torch.bfloat16))
+    common = _lowrank_operands(x2, v, s)
     small = common and M < 256 and R % 32 == 0 and 0 < R <= 256
     large = common and M >= 256 and R in ONE_PASS_RANKS
     if not (small or large):

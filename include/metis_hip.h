@@ -555,6 +555,21 @@ int metis_lowrank_project_rows_ws(const void *x, int64_t ldx, const void *v, int
                                   void *stream);
 
 /*
+ * The projections of a projection group (q/k/v, gate/up) in one pass over their common x: member i has its own V [r, K] and
+ * s [r] (host array of `count` pairs of device pointers), its columns of xv and t follow those of the members before it.
+ * Column for column the bits of metis_lowrank_project_rows_ws of that member alone with a workspace of its size.
+ *   count 1 .. 4; every r a multiple of 32, their sum R as above; s of all members, or t == NULL
+ *   workspace  metis_lowrank_project_rows_workspace_bytes(M, R, K), as above
+ */
+typedef struct metis_lowrank_factor {
+    const void *v, *s;
+    int64_t r;
+} metis_lowrank_factor;
+int metis_lowrank_project_rows_grouped(const void *x, int64_t ldx, int64_t M, int64_t K, const metis_lowrank_factor *factors,
+                                       int count, void *xv, void *t, void *workspace, size_t workspace_bytes,
+                                       void *stream);
+
+/*
  * Both things BitLinear.forward does with its activation, in one pass over it: the NVFP4 quantization that feeds the
  * residual branch (src/Metis/Metis/bitlinear.py:566-576 via quant.py:6-36) and the rank-r projection of the low-rank
  * branch (bitlinear.py:752-756).  Results: xv / t as metis_lowrank_project_rows_ws, codes / deferred as

@@ -911,3 +911,61 @@ def test_projection_group_at_prefill_size_keeps_every_rank_on_the_kernel(ranks, 
         # the same products in binary32 sums of another order; where that moves bf16(x V^T s) across a midpoint, the rank-r term
         # moves by one bf16 rounding (2^-8) of that factor
         assert rel_fro(y.float().cpu(), w.float().cpu()) <= 2.0 ** -8
+
+
+def _prefill_group(K, ns, r, mean, compute, bias, seed=7, cached=True):
+    """A projection group of layers of unequal width, factors in bf16, as replace_linear_with_metis wires it."""
+    from metis_hip import BitLinear, LinearLowbit, MetisArgs
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    group = {"name": "g", "mean_cache": {}, "input_ref": None, "quantized_input": None, "members": []}
+    for n in ns:
+        args = MetisArgs(forward_svd_rank=r, cache_quantized_weight=cached) if mean else MetisArgs.direct_fp4(forward_svd_rank=r)
+        args.cache_quantized_weight = cached
+        m = BitLinear(K, n, args=args, bias=bias, dtype=torch.bfloat16, compute_dtype=compute)
+        make = dict(args=args, device="cuda", storage_dtype=torch.bfloat16, compute_dtype=compute)
+        m.warmup_linear, m.vlinear = LinearLowbit(K, n, bias=bias, **make), LinearLowbit(K, r, bias=False, **make)
+        m.ulinear = torch.nn.Linear(r, n, bias=False, device="cuda", dtype=torch.bfloat16)
+        m.s = torch.nn.Parameter(torch.rand(r, generator=g, device="cuda").bfloat16() + 0.5)
+        with torch.no_grad():
+            for p in (m.warmup_linear.weight, m.vlinear.weight, m.ulinear.weight) + ((m.warmup_linear.bias,) if bias else ()):
+                p.copy_(torch.randn(p.shape, generator=g, device="cuda") * 0.1)
+        m.is_svd_quant, m.activation_group = True, group
+        group["members"].append(m)
+    return group["members"], g
+
+
+@pytest.mark.parametrize("rows", [300, 411])
+@pytest.mark.parametrize("mean", [False, True])
+@pytest.mark.parametrize("compute", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_prompt_of_a_group_has_the_same_bits_with_and_without_autograd(rows, mean, compute, bias, monkeypatch):
+    """Without autograd the group runs as one pass of the rank-r kernel and one GEMM launch, with it member by member: equal
+    outputs (and so equal to grouped_inference = False), in direct and mean mode, both arithmetics, with and without bias."""
+    from metis_hip import BitLinear, ops
+    members, g = _prefill_group(1024, (2304, 512, 260), 64, mean, compute, bias)
+    x = synthetic_activation(3, rows, 1024).cuda()
+    calls, real = [], ops._linear_fwd_tiled_grouped
+    monkeypatch.setattr(ops, "_linear_fwd_tiled_grouped", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    with torch.no_grad():
+        got = [m(x) for m in members]
+    assert len(calls) == 1                                       # (compute in binary32: all weights are 256 wide or more)
+    with_grad = [m(x.clone()) for m in members]
+    monkeypatch.setattr(BitLinear, "grouped_inference", False)
+    with torch.no_grad():
+        alone = [m(x.clone()) for m in members]
+    for y, w, a in zip(got, with_grad, alone):
+        assert y.dtype == w.dtype and torch.equal(y, w) and torch.equal(y, a)
+
+
+@pytest.mark.parametrize("which", ["vlinear", "s"])
+def test_a_prompt_of_a_group_sees_writes_through_data(which):
+    """V and s of a member are read where they are: a write through .data, which moves no version counter, counts at once."""
+    members, _ = _prefill_group(256, (384, 384), 64, False, torch.bfloat16, False)
+    x = synthetic_activation(3, 300, 256).cuda()
+    with torch.no_grad():
+        before = [m(x) for m in members]
+        p = members[1].s if which == "s" else members[1].vlinear.weight
+        p.data.mul_(2)
+        after = [m(x.clone()) for m in members]
+    want = members[1](x.clone())                                 # member by member, with autograd
+    assert torch.equal(before[0], after[0]) and not torch.equal(before[1], after[1]) and torch.equal(after[1], want)
