@@ -433,38 +433,50 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_backward_rows_kernel(const uin
     }
 }
 
-constexpr int kColmeanBatch = 8;
-// W waves share a column group's partial rows.  Sixteen where there are enough of them: 512 rows of 3584 columns are 56
-// workgroups, and four waves each walk 128 rows eight loads at a time (10.3 us for the launch; with
-// sixteen waves the 4 rounds of loads of a wave are one).
-template <bool OUT_BF16, int W>
-__global__ __launch_bounds__(64 * W) void rmsnorm_colmean_finish_kernel(const float* __restrict__ partial, uint32_t slabs, uint32_t cols,
+// Four sums per column, each of every fourth partial row in order, added in pairs at the end.  Q waves fetch the rows of a sum:
+// one, which adds them as they come, where there are few; four, which hand theirs to the adding one through LDS, eight
+// loads in flight in each, where there are enough (512 partial rows of 3584 columns are 56 workgroups: with one wave per sum
+// the call at 2103 x 3584 takes 22.8 us, 19.3 with 32 loads in flight in it, 17.8 with four).  The order is the same for both.
+template <bool OUT_BF16, int Q>
+__global__ __launch_bounds__(256 * Q) void rmsnorm_colmean_finish_kernel(const float* __restrict__ partial, uint32_t slabs, uint32_t cols,
                                                                      float count, void* __restrict__ out, const void* __restrict__ cached,
                                                                      float cached_count, float rows_f, float* __restrict__ out32)
 {
-    __shared__ float part[W][64];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    constexpr uint32_t BATCH = 8;
+    __shared__ float part[4][64];
+    __shared__ float rows[Q > 1 ? 4 : 1][Q * BATCH][64];
+    const uint32_t lane = threadIdx.x & 63u, chain = (threadIdx.x >> 6) & 3u, q = threadIdx.x >> 8;
     const uint32_t c = blockIdx.x * 64u + lane;
-    float s = 0.0f;
-    if (c < cols) {
-        // wave w adds the partial rows w, w + W, ... in order, kColmeanBatch loads in flight at a time
-        for (uint32_t k0 = wave; k0 < slabs; k0 += (uint32_t)W * kColmeanBatch) {
-            float v[kColmeanBatch];
+    float s = 0.0f, v[BATCH];
+    auto fetch = [&](uint32_t i0) {                            // partial rows i0 .. of the wave's share, 4 apart
 #pragma unroll
-            for (int b = 0; b < kColmeanBatch; ++b) {
-                const uint32_t k = k0 + (uint32_t)W * b;
-                v[b] = k < slabs ? partial[(size_t)k * cols + c] : 0.0f;
+        for (uint32_t b = 0; b < BATCH; ++b) {
+            const uint32_t k = chain + 4u * (i0 + q * BATCH + b);
+            v[b] = (k < slabs && c < cols) ? partial[(size_t)k * cols + c] : 0.0f;
+        }
+    };
+    fetch(0u);
+    for (uint32_t i0 = 0u; 4u * i0 < slabs; i0 += Q * BATCH) {
+        if constexpr (Q > 1) {
+#pragma unroll
+            for (uint32_t b = 0; b < BATCH; ++b) rows[chain][q * BATCH + b][lane] = v[b];
+            fetch(i0 + Q * BATCH);
+            __syncthreads();
+            if (q == 0u) {
+#pragma unroll
+                for (uint32_t i = 0; i < Q * BATCH; ++i) s += rows[chain][i][lane];
             }
+            __syncthreads();
+        } else {
 #pragma unroll
-            for (int b = 0; b < kColmeanBatch; ++b) s += v[b];
+            for (uint32_t b = 0; b < BATCH; ++b) s += v[b];
+            fetch(i0 + BATCH);
         }
     }
-    part[wave][lane] = s;
+    if (q == 0u) part[chain][lane] = s;
     __syncthreads();
-    if (wave != 0 || c >= cols) return;
-    s = 0.0f;
-#pragma unroll
-    for (int w = 0; w < W; w += 4) s += (part[w][lane] + part[w + 1][lane]) + (part[w + 2][lane] + part[w + 3][lane]);
+    if (threadIdx.x >= 64u || c >= cols) return;
+    s = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
     auto rnd = [](float x) { return OUT_BF16 ? __uint_as_float(bf16_bits(x) << 16) : x; };
     float m = rnd(s / count);
     if (cached) {                                              // weighted running mean of decode calls, bitlinear.py:316-323
@@ -482,10 +494,10 @@ static int finish_column_sums(const float* partial, int slabs, int64_t cols, flo
                               float cached_count, float rows_f, float* out32, hipStream_t st)
 {
     const dim3 g((unsigned)((cols + 63) / 64));
-#define METIS_CF(B, W) hipLaunchKernelGGL((rmsnorm_colmean_finish_kernel<B, W>), g, dim3(64 * W), 0, st, partial, (uint32_t)slabs, (uint32_t)cols, \
+#define METIS_CF(B, Q) hipLaunchKernelGGL((rmsnorm_colmean_finish_kernel<B, Q>), g, dim3(256 * Q), 0, st, partial, (uint32_t)slabs, (uint32_t)cols, \
         count, out, cached, cached_count, rows_f, out32)
-    if (slabs >= 64) { if (out_bf16) METIS_CF(true, 16); else METIS_CF(false, 16); }
-    else { if (out_bf16) METIS_CF(true, 4); else METIS_CF(false, 4); }
+    if (slabs >= 64) { if (out_bf16) METIS_CF(true, 4); else METIS_CF(false, 4); }
+    else { if (out_bf16) METIS_CF(true, 1); else METIS_CF(false, 1); }
 #undef METIS_CF
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }

@@ -653,3 +653,32 @@ def test_mean_mode_linear_against_reference_vectors(monkeypatch):
     assert rel_fro(xr.grad.cpu(), t(g["mean_lin_gx"])) <= 1e-5
     assert rel_fro(lin.weight.grad.cpu(), t(g["mean_lin_gw"])) <= 1e-5
     assert rel_fro(lin.bias.grad.cpu(), t(g["mean_lin_gb"])) <= 1e-5
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 64), (250, 128), (256, 64), (2103, 192), (4099, 64)])
+def test_column_mean_of_the_normed_tensor_is_added_in_its_documented_order(rows, cols):
+    """Rows in order within a wave, a workgroup's four waves in order, the workgroups' partial rows 4 apart in four sums that are
+    added in pairs: binary32 on the CPU in that order gives the same bits, for few partial rows and for many."""
+    from metis_hip import ops
+    x = synthetic_activation(31, rows, cols).cuda()
+    gamma = (1 + 0.1 * torch.randn(cols, generator=torch.Generator().manual_seed(2))).bfloat16().cuda()
+    normed, me, _ = ops.rmsnorm_colmean(x, gamma, 1e-6, torch.float32)
+    nf = normed.float().cpu()
+    groups = max(1, min((rows + 3) // 4, 2 * torch.cuda.get_device_properties(0).multi_processor_count))
+    partial = torch.zeros(groups, cols)
+    for b in range(groups):
+        waves = []
+        for w in range(4):
+            acc = torch.zeros(cols)
+            for r in range(4 * b + w, rows, 4 * groups):
+                acc = acc + nf[r]
+            waves.append(acc)
+        partial[b] = ((waves[0] + waves[1]) + waves[2]) + waves[3]
+    sums = []
+    for w in range(4):
+        s = torch.zeros(cols)
+        for k in range(w, groups, 4):
+            s = s + partial[k]
+        sums.append(s)
+    total = (sums[0] + sums[1]) + (sums[2] + sums[3])
+    assert torch.equal(me.cpu(), total / rows)
