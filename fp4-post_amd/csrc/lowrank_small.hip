@@ -72,39 +72,44 @@ int lowrank_small(const void* x, int64_t ldx, const void* v, int64_t M, int64_t 
 // forms it for torch.mul on bf16 tensors (src/Metis/Metis/bitlinear.py:755), the sum in binary32.  Two [L, R] bf16
 // tensors, a few hundred KB: one workgroup per 8 columns walks all rows (a thread takes every 256th row, 16 bytes of
 // each tensor per row), and the 256 per-thread sums of a column are added in thread order -- a fixed order, one launch.
+// Bound by latency: eight rows of a thread are requested together (one at a time, each waited for, 6.7 us at 4096 x 32; this
+// 6.3), and the adder has sixteen of the sums in flight.
 // ---------------------------------------------------------------------------------------------
-// 16 waves per 8 columns (a token and 16 bytes of g and xv per thread and step), the threads' sums folded within a wave by
-// exchanges and the waves' in order.  256 threads with one of them adding up all sums took 12 us at 4096 x 32, this 5.
-__global__ __launch_bounds__(1024) void scale_grad_kernel(const uint16_t* __restrict__ g, const uint16_t* __restrict__ xv, int L, int R,
+__global__ __launch_bounds__(256) void scale_grad_kernel(const uint16_t* __restrict__ g, const uint16_t* __restrict__ xv, int L, int R,
                                                          void* __restrict__ out, int out_f32)
 {
-    __shared__ float part[16][8];
+    constexpr int BATCH = 8;
+    __shared__ float part[256][9];
     const int c0 = blockIdx.x * 8, tid = threadIdx.x;
     float acc[8] = {};
-#pragma unroll 4
-    for (int l = tid; l < L; l += 1024) {
-        const uint4 a = *reinterpret_cast<const uint4*>(g + (int64_t)l * R + c0);
-        const uint4 b = *reinterpret_cast<const uint4*>(xv + (int64_t)l * R + c0);
-        const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+    for (int l0 = tid; l0 < L; l0 += 256 * BATCH) {
+        uint4 a[BATCH], b[BATCH];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            acc[2 * j] += rb(bf16_lo(aw[j]) * bf16_lo(bw[j]));
-            acc[2 * j + 1] += rb(bf16_hi(aw[j]) * bf16_hi(bw[j]));
+        for (int i = 0; i < BATCH; ++i) {
+            const int64_t l = (int64_t)l0 + 256 * i;
+            a[i] = b[i] = make_uint4(0u, 0u, 0u, 0u);             // (rows past the end add zeros)
+            if (l < L) {
+                a[i] = *reinterpret_cast<const uint4*>(g + l * R + c0);
+                b[i] = *reinterpret_cast<const uint4*>(xv + l * R + c0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const uint32_t aw[4] = {a[i].x, a[i].y, a[i].z, a[i].w}, bw[4] = {b[i].x, b[i].y, b[i].z, b[i].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                acc[2 * j] += rb(bf16_lo(aw[j]) * bf16_lo(bw[j]));
+                acc[2 * j + 1] += rb(bf16_hi(aw[j]) * bf16_hi(bw[j]));
+            }
         }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] += __shfl_xor(acc[j], o, 64);
-    if ((tid & 63) == 0) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) part[tid >> 6][j] = acc[j];
-    }
+    for (int j = 0; j < 8; ++j) part[tid][j] = acc[j];
     __syncthreads();
     if (tid < 8) {
         float sum = 0.0f;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) sum += part[t][tid];
+#pragma unroll 16
+        for (int t = 0; t < 256; ++t) sum += part[t][tid];
         if (out_f32) static_cast<float*>(out)[c0 + tid] = sum;
         else static_cast<uint16_t*>(out)[c0 + tid] = (uint16_t)bf16_bits(sum);
     }
@@ -117,7 +122,7 @@ int scale_grad(const void* g, const void* xv, int64_t L, int64_t R, void* out, i
     if (L > INT32_MAX || R > INT32_MAX) return METIS_E_ARG;
     if (!out || ((uintptr_t)out % 4)) return METIS_E_ARG;
     if (L > 0 && (!g || !xv || ((uintptr_t)g % 16) || ((uintptr_t)xv % 16))) return METIS_E_ARG;
-    hipLaunchKernelGGL(scale_grad_kernel, dim3((unsigned)(R / 8)), dim3(1024), 0, st, (const uint16_t*)g, (const uint16_t*)xv, (int)L, (int)R,
+    hipLaunchKernelGGL(scale_grad_kernel, dim3((unsigned)(R / 8)), dim3(256), 0, st, (const uint16_t*)g, (const uint16_t*)xv, (int)L, (int)R,
                        out, (int)(out_dtype == METIS_DTYPE_F32));
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }

@@ -850,6 +850,24 @@ def test_gradient_of_the_rank_r_scale_vector(L, R):
     assert torch.equal(ops.lowrank_scale_grad(g[:0], xv[:0]), torch.zeros(R, device="cuda"))
     assert torch.equal(ops.lowrank_scale_grad(g, xv, out_dtype=torch.bfloat16), got.bfloat16())
 
+
+@pytest.mark.parametrize("L,R", [(1, 8), (255, 40), (257, 32), (2047, 32), (2049, 8), (4096, 32), (5000, 64)])
+def test_gradient_of_the_rank_r_scale_vector_is_added_in_its_documented_order(L, R):
+    """256 sums of every 256th row, in row order, then these in order: binary32 on the CPU in that order gives the same bits."""
+    from metis_hip import ops
+    g_ = torch.Generator().manual_seed(8100 + L)
+    g, xv = torch.randn(L, R, generator=g_).bfloat16(), (torch.randn(L, R, generator=g_) * 3).bfloat16()
+    prod = torch.zeros((L + 255) // 256 * 256, R)
+    prod[:L] = (g * xv).float()
+    chains = torch.zeros(256, R)
+    for rows in prod.view(-1, 256, R):
+        chains = chains + rows
+    total = torch.zeros(R)
+    for c in chains:
+        total = total + c
+    assert torch.equal(ops.lowrank_scale_grad(g.cuda(), xv.cuda()).cpu(), total)
+
+
 def test_memory_bound_deployments_can_drop_the_derived_weight_copies(monkeypatch):
     """A cached weight holds 0.5625 B per parameter packed; the tiled binary16 expansion (2 B, one per arithmetic) and
     the decode layout (0.5625 B) are built on first use.  With both switches off nothing but the packed form stays,
