@@ -1116,6 +1116,11 @@ class BitLinear(nn.Module):
         rows = x.numel() // max(x.shape[-1], 1)
         if not all(m._fusable() and m.compute_dtype == self.compute_dtype for m in members):
             return None
+        if rows >= 256 and not all([m._modules["warmup_linear"].cache_quantized_weight for m in members]):
+            # weights packed for this one call: only if the group will use them (each member packs its own otherwise)
+            probes = [m._residual_probe() for m in members]
+            if None in probes or not self._tiles_as_group(shared_input, probes):
+                return None
         packed = [m._packed_residual() for m in members]
         if any(p is None for p in packed):
             return None
@@ -1171,6 +1176,27 @@ class BitLinear(nn.Module):
             group["stacked_v"] = cached
         return cached
 
+    def _residual_probe(self):
+        """What _packed_residual would return, as far as _tiles_as_group asks, without packing anything."""
+        F = LinearLowbitFunction
+        w = _param(self._modules["warmup_linear"], "weight")
+        if not ((not F.enable_nv_recipe or F._nv_on_kernels()) and _packable(w, F.q_forward_weight) and w.shape[0] % 4 == 0):
+            return None
+        return SimpleNamespace(rows=w.shape[0], cols=w.shape[1], mode=ops.MODE_P32 if self.compute_dtype == torch.float32 else ops.MODE_PB16,
+                               rht=F._hadamard_mask() if F.enable_nv_recipe else None, tiled=None,
+                               persistent=self._modules["warmup_linear"].cache_quantized_weight)
+
+    @staticmethod
+    def _tiles_as_group(shared_input, weights) -> bool:
+        """Whether the members' own calls at prefill size would all run on the tiled GEMM in one format, so that one launch can
+        take their place."""
+        F = LinearLowbitFunction
+        if not isinstance(shared_input, CenteredNVFP4):
+            return ops.tiled_group_applies(shared_input, weights, F.reference_rounding)
+        inside = [F._mean_in_operand(shared_input, p) for p in weights]
+        return (all(inside) or not (any(inside) or any(p.rht is not None for p in weights))) and \
+            ops.tiled_group_applies(shared_input.residual, weights, F.reference_rounding and all(inside))
+
     def _forward_group_tiled(self, x: torch.Tensor, shared_input, members, packed):
         """_forward_group at prefill size (256 rows or more): one pass over x for all projections, one launch of the tiled GEMM
         for all products; every member has the bits that it has alone and with autograd (_MetisFusedFunction.forward)."""
@@ -1180,8 +1206,7 @@ class BitLinear(nn.Module):
         px = shared_input.residual if centered else shared_input
         in_operand = centered and all(F._mean_in_operand(shared_input, p) for p in packed)
         rounding = F.reference_rounding and (in_operand or not centered)
-        if (not ops.tiled_group_applies(px, packed, rounding)
-                or (centered and not in_operand and any(F._mean_in_operand(shared_input, p) or p.rht is not None for p in packed))):
+        if not self._tiles_as_group(shared_input, packed):
             return None
         x2 = _as_dtype(_flat2d(x), cd)
         factors = [(_as_dtype(_param(m._modules["vlinear"], "weight"), cd), _as_dtype(_param(m, "s"), cd)) for m in members]

@@ -969,3 +969,21 @@ def test_a_prompt_of_a_group_sees_writes_through_data(which):
         after = [m(x.clone()) for m in members]
     want = members[1](x.clone())                                 # member by member, with autograd
     assert torch.equal(before[0], after[0]) and not torch.equal(before[1], after[1]) and torch.equal(after[1], want)
+
+
+@pytest.mark.parametrize("mean", [False, True])
+@pytest.mark.parametrize("compute", [torch.float32, torch.bfloat16])
+def test_a_prompt_of_a_group_packs_every_uncached_weight_once(mean, compute, monkeypatch):
+    """cache_quantized_weight=False: the group runs as one only where it uses the packed weights that it makes (bf16 arithmetic);
+    otherwise (binary32) every member packs its own, once."""
+    from metis_hip.quant import Cast2NVFp4e2m1BlockNOSR
+    members, _ = _prefill_group(256, (384, 256, 512), 64, mean, compute, False, cached=False)
+    x = synthetic_activation(3, 300, 256).cuda()
+    weights = {m.warmup_linear.weight.data_ptr() for m in members}
+    seen, real = [], Cast2NVFp4e2m1BlockNOSR._pack.__func__
+    monkeypatch.setattr(Cast2NVFp4e2m1BlockNOSR, "_pack", classmethod(lambda cls, t_, *a: (seen.append(t_.data_ptr()), real(cls, t_, *a))[1]))
+    with torch.no_grad():
+        got = [m(x) for m in members]
+    assert sum(p in weights for p in seen) == len(members)
+    want = [m(x.clone()) for m in members]
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
