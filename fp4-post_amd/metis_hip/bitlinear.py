@@ -55,6 +55,11 @@ def _pkey(p: torch.Tensor) -> tuple:
     return (id(p), p.data_ptr(), p._version)
 
 
+def _version_of(x: torch.Tensor):
+    """x's version counter, which every in-place write moves; None for an inference tensor, which has none."""
+    return None if x.is_inference() else x._version
+
+
 def _flat2d(x: torch.Tensor) -> torch.Tensor:
     return x.reshape(-1, x.shape[-1])
 
@@ -969,7 +974,7 @@ class BitLinear(nn.Module):
             return F._prepare_input(x, mean_cache=self.mean_cache, cache_key=f"{self.layer_name}.shared",
                                     weights_cached=self._weights_cached())
         input_ref = group.get("input_ref")
-        if input_ref is not None and input_ref() is x:
+        if input_ref is not None and input_ref() is x and group.get("input_version") == _version_of(x):
             return group["quantized_input"]
         quantized_input = F._prepare_input(x, mean_cache=group["mean_cache"], cache_key=f"{group['name']}.shared",
                                            weights_cached=all(m._weights_cached() for m in group.get("members", ())))
@@ -980,6 +985,7 @@ class BitLinear(nn.Module):
                 group["quantized_input"] = None
 
         group["input_ref"] = weakref.ref(x, clear_cached_input)
+        group["input_version"] = _version_of(x)                  # a tensor that was written to since is another input
         group["quantized_input"] = quantized_input
         # every member's GEMM reads this activation: its tiled expansion is made once and kept while it lives
         packed = quantized_input.residual if isinstance(quantized_input, CenteredNVFP4) else quantized_input
@@ -1252,7 +1258,7 @@ class BitLinear(nn.Module):
         if (BitLinear.grouped_inference and group is not None and not torch.is_grad_enabled() and len(group.get("members", ())) > 1
                 and x.is_cuda):
             ready = group.get("grouped_outputs")
-            if ready is not None and ready[0]() is x and id(self) in ready[1]:
+            if ready is not None and ready[0]() is x and id(self) in ready[1] and ready[2] == _version_of(x):
                 return ready[1].pop(id(self))                   # evaluated with the first member of the group
         if (BitLinear.grouped_inference and group is not None and not torch.is_grad_enabled() and len(group.get("members", ())) > 1
                 and x.is_cuda and self._fusable()):
@@ -1265,7 +1271,7 @@ class BitLinear(nn.Module):
                     def drop(ref, group=group):
                         if group.get("grouped_outputs") is not None and group["grouped_outputs"][0] is ref:
                             group["grouped_outputs"] = None
-                    group["grouped_outputs"] = (weakref.ref(x, drop), outs)
+                    group["grouped_outputs"] = (weakref.ref(x, drop), outs, _version_of(x))
                     return mine
         mods = self._modules
         share_activation = (isinstance(mods.get("vlinear"), LinearLowbit) and isinstance(mods.get("warmup_linear"), LinearLowbit)

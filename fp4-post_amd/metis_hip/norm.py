@@ -18,7 +18,7 @@ from torch import nn
 from . import ops
 from ._lib import MODE_P32, MODE_PB16
 from .ops import CenteredNVFP4
-from .bitlinear import BitLinear, LinearLowbitFunction
+from .bitlinear import BitLinear, LinearLowbitFunction, _version_of
 from .quant import is_hip_nvfp4
 
 
@@ -136,6 +136,7 @@ class FusedRMSNormQuant(nn.Module):
         if not mean_mode:
             packed.shared = True                 # read by every member of the group: its tiled expansion is kept while it lives
         group["input_ref"] = weakref.ref(out, clear)
+        group["input_version"] = _version_of(out)
         group["quantized_input"] = packed
         return out
 

@@ -987,3 +987,43 @@ def test_a_prompt_of_a_group_packs_every_uncached_weight_once(mean, compute, mon
     assert sum(p in weights for p in seen) == len(members)
     want = [m(x.clone()) for m in members]
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("rows", [5, 64, 300])
+@pytest.mark.parametrize("mean", [False, True])
+@pytest.mark.parametrize("grad", [False, True])
+def test_an_input_written_to_between_the_members_of_a_group_is_another_input(rows, mean, grad, monkeypatch):
+    """q(x), then new contents in the same buffer, then k(x): the packed activation (and, without autograd, k's output) made with q
+    belong to the old contents."""
+    from metis_hip import BitLinear
+    members, _ = _prefill_group(256, (384, 256), 64, mean, torch.bfloat16, True)
+    x, other = synthetic_activation(3, rows, 256).cuda(), synthetic_activation(4, rows, 256).cuda()
+
+    def alone(m, t_):
+        m.activation_group["mean_cache"].clear()
+        with torch.no_grad():
+            return m(t_.clone())
+    with torch.set_grad_enabled(grad):
+        first = members[0](x)
+        x.copy_(other)
+        members[0].activation_group["mean_cache"].clear()
+        second, again = members[1](x), members[0](x)
+    monkeypatch.setattr(BitLinear, "grouped_inference", False)
+    tol = 0.0 if rows >= 256 else 2e-3                           # (decode sizes: a group's sums may be split differently)
+    assert rel_fro(second.detach().float().cpu(), alone(members[1], other).float().cpu()) <= tol
+    assert rel_fro(again.detach().float().cpu(), alone(members[0], other).float().cpu()) <= tol
+    assert not torch.equal(first, again)
+
+
+def test_a_normed_tensor_written_to_is_packed_anew():
+    """The norm leaves its packed output in the group for the tensor that it returned, as it returned it."""
+    from metis_hip import FusedRMSNormQuant
+    members, g = _prefill_group(256, (384, 256), 64, False, torch.bfloat16, False)
+    norm = FusedRMSNormQuant(torch.nn.Parameter(torch.ones(256, device="cuda").bfloat16()), 1e-6, members[0].activation_group)
+    x = synthetic_activation(3, 300, 256).cuda()
+    with torch.no_grad():
+        n = norm(x)
+        n.mul_(2).add_(1)
+        got = [m(n) for m in members]
+        want = [m(n.clone()) for m in members]
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
