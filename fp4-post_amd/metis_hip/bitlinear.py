@@ -1168,6 +1168,29 @@ class BitLinear(nn.Module):
         lead = x.shape[:-1]
         return {id(m): _as_dtype(y.reshape(*lead, y.shape[-1]), F.compute_dtype) for m, y in zip(members, outs)}
 
+    def _output_key(self) -> tuple:
+        """What this member's output depends on beside its input, as far as identities and version counters tell."""
+        F = LinearLowbitFunction
+        mods = self._modules
+        wl = mods["warmup_linear"]
+        v, s, u, w, b = _param(mods["vlinear"], "weight"), _param(self, "s"), _param(mods["ulinear"], "weight"), _param(wl, "weight"), wl.bias
+        # (_pkey of each, written out: a prompt's groups ask six times)
+        return (id(v), v.data_ptr(), v._version, id(s), s.data_ptr(), s._version, id(u), u.data_ptr(), u._version, id(w), w.data_ptr(), w._version,
+                None if b is None else _pkey(b), F.compute_dtype, F.reference_rounding, F.q_forward_weight, F.enable_nv_recipe)
+
+    def _ready_output(self, group, x: torch.Tensor):
+        """This member's output if it was evaluated with the first member of its group on this very input: the same tensor, not
+        written to since, on the stream that asks now, and (from 256 rows on; a decode step is launch-bound and asks for less)
+        with the parameters and switches of now.  Each is handed out once."""
+        ready = group.get("grouped_outputs")
+        if ready is None or ready[0]() is not x or id(self) not in ready[1]:
+            return None
+        _, outs, version, stream, keys = ready
+        if version != _version_of(x) or stream != ops._stream() or (keys is not None and keys[id(self)] != self._output_key()):
+            group["grouped_outputs"] = None
+            return None
+        return outs.pop(id(self))
+
     def _stacked_factors(self, device):
         """(key, V, s) of all members of the group stacked: one product gives every member's rank-r projection.  Kept on the
         group until a member's parameter changes."""
@@ -1256,12 +1279,10 @@ class BitLinear(nn.Module):
             return self.warmup_linear(x)
         group = self.activation_group
         if (BitLinear.grouped_inference and group is not None and not torch.is_grad_enabled() and len(group.get("members", ())) > 1
-                and x.is_cuda):
-            ready = group.get("grouped_outputs")
-            if ready is not None and ready[0]() is x and id(self) in ready[1] and ready[2] == _version_of(x):
-                return ready[1].pop(id(self))                   # evaluated with the first member of the group
-        if (BitLinear.grouped_inference and group is not None and not torch.is_grad_enabled() and len(group.get("members", ())) > 1
                 and x.is_cuda and self._fusable()):
+            mine = self._ready_output(group, x)
+            if mine is not None:
+                return mine
             shared_input = self._get_shared_quantized_input(x)
             if isinstance(shared_input, (PackedNVFP4, CenteredNVFP4)):
                 outs = self._forward_group(x, shared_input)
@@ -1271,7 +1292,8 @@ class BitLinear(nn.Module):
                     def drop(ref, group=group):
                         if group.get("grouped_outputs") is not None and group["grouped_outputs"][0] is ref:
                             group["grouped_outputs"] = None
-                    group["grouped_outputs"] = (weakref.ref(x, drop), outs, _version_of(x))
+                    keys = {id(m): m._output_key() for m in group["members"] if m is not self} if x.numel() >= 256 * x.shape[-1] else None
+                    group["grouped_outputs"] = (weakref.ref(x, drop), outs, _version_of(x), ops._stream(), keys)
                     return mine
         mods = self._modules
         share_activation = (isinstance(mods.get("vlinear"), LinearLowbit) and isinstance(mods.get("warmup_linear"), LinearLowbit)

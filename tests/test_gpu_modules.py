@@ -1027,3 +1027,43 @@ def test_a_normed_tensor_written_to_is_packed_anew():
         got = [m(n) for m in members]
         want = [m(n.clone()) for m in members]
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("what", ["s", "vlinear", "ulinear", "residual", "bias", "replaced", "switch"])
+def test_a_member_changed_between_the_calls_of_its_group_is_seen(what, monkeypatch):
+    """At prefill size a member's own call has always read its parameters and switches when it is made: a change after the first
+    member of the group was called counts for the second."""
+    from metis_hip import BitLinear
+    members, _ = _prefill_group(256, (384, 256), 64, False, torch.bfloat16, True)
+    x = synthetic_activation(3, 300, 256).cuda()
+    k = members[1]
+    with torch.no_grad():
+        members[0](x)
+        if what == "replaced":
+            k.s = torch.nn.Parameter(k.s.detach() * 2)
+        elif what == "switch":
+            monkeypatch.setattr(BitLinear, "quantized_lowrank_branch", True)
+        else:
+            {"s": k.s, "vlinear": k.vlinear.weight, "ulinear": k.ulinear.weight, "residual": k.warmup_linear.weight, "bias": k.warmup_linear.bias}[what].mul_(2)
+        got = k(x)
+        monkeypatch.setattr(BitLinear, "grouped_inference", False)
+        want = k(x.clone())
+    assert torch.equal(got, want)
+
+
+def test_a_member_called_on_another_stream_is_evaluated_there():
+    """The siblings' outputs are queued on the first member's stream: a member called on another one does not take its own from them
+    (that stream has not waited for it, and its memory belongs to the first)."""
+    members, _ = _prefill_group(256, (384, 256), 64, False, torch.bfloat16, False)
+    group = members[0].activation_group
+    x = synthetic_activation(3, 300, 256).cuda()
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        members[0](x)
+        waiting = group["grouped_outputs"][1][id(members[1])]
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            got = members[1](x)
+        torch.cuda.current_stream().wait_stream(side)
+    assert got.data_ptr() != waiting.data_ptr() and torch.equal(got, waiting)
+    torch.cuda.synchronize()
