@@ -1191,6 +1191,30 @@ class BitLinear(nn.Module):
             return None
         return outs.pop(id(self))
 
+    def _called_alone(self, group, x: torch.Tensor) -> bool:
+        """Whether this member is evaluated by itself although it belongs to a group (prompts; same bits either way): its siblings'
+        outputs of the last evaluation were never asked for (one layer probed on its own, a calibration pass), so theirs are
+        not computed and held again, until a sibling is called with the same input as this member."""
+        version = _version_of(x)
+        last = group.get("alone_input")
+        if last is not None and last[0]() is x and last[1] == version:
+            if id(self) not in last[2]:
+                last[2].add(id(self))
+                group["called_alone"] = False                    # a sibling on the same input: as a group from the next input on
+                return True
+            group["alone_input"] = None                          # another pass over it
+        ready = group.get("grouped_outputs")
+        if ready is not None and ready[4] is not None and ready[1]:
+            group["called_alone"], group["grouped_outputs"] = True, None
+        if not group.get("called_alone"):
+            return False
+
+        def drop(ref, group=group):
+            if group.get("alone_input") is not None and group["alone_input"][0] is ref:
+                group["alone_input"] = None
+        group["alone_input"] = (weakref.ref(x, drop), version, {id(self)})
+        return True
+
     def _stacked_factors(self, device):
         """(key, V, s) of all members of the group stacked: one product gives every member's rank-r projection.  Kept on the
         group until a member's parameter changes."""
@@ -1283,16 +1307,19 @@ class BitLinear(nn.Module):
             mine = self._ready_output(group, x)
             if mine is not None:
                 return mine
+            prompt = x.numel() >= 256 * x.shape[-1]
             shared_input = self._get_shared_quantized_input(x)
-            if isinstance(shared_input, (PackedNVFP4, CenteredNVFP4)):
+            if isinstance(shared_input, (PackedNVFP4, CenteredNVFP4)) and not (prompt and self._called_alone(group, x)):
                 outs = self._forward_group(x, shared_input)
                 if outs is not None:
                     mine = outs.pop(id(self))
 
-                    def drop(ref, group=group):
+                    def drop(ref, group=group, prompt=prompt):
                         if group.get("grouped_outputs") is not None and group["grouped_outputs"][0] is ref:
+                            if prompt and group["grouped_outputs"][1]:
+                                group["called_alone"] = True
                             group["grouped_outputs"] = None
-                    keys = {id(m): m._output_key() for m in group["members"] if m is not self} if x.numel() >= 256 * x.shape[-1] else None
+                    keys = {id(m): m._output_key() for m in group["members"] if m is not self} if prompt else None
                     group["grouped_outputs"] = (weakref.ref(x, drop), outs, _version_of(x), ops._stream(), keys)
                     return mine
         mods = self._modules

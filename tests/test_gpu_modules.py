@@ -1067,3 +1067,31 @@ def test_a_member_called_on_another_stream_is_evaluated_there():
         torch.cuda.current_stream().wait_stream(side)
     assert got.data_ptr() != waiting.data_ptr() and torch.equal(got, waiting)
     torch.cuda.synchronize()
+
+
+def test_a_member_probed_on_its_own_does_not_compute_its_siblings_over_and_over(monkeypatch):
+    """One member of a group called with prompts of its own: the siblings' outputs are computed once, found unused, and from then on
+    neither computed nor held; when the whole group is called again it runs as one from the second input on.  Same bits throughout."""
+    from metis_hip import BitLinear, ops
+    members, _ = _prefill_group(256, (384, 256, 260), 64, False, torch.bfloat16, False)
+    group = members[0].activation_group
+    calls, real = [], ops._linear_fwd_tiled_grouped
+    monkeypatch.setattr(ops, "_linear_fwd_tiled_grouped", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    inputs = [synthetic_activation(10 + i, 300, 256).cuda() for i in range(4)]
+    with torch.no_grad():
+        lone = [members[1](x) for x in inputs]                   # inputs stay alive
+        assert len(calls) == 1 and group.get("grouped_outputs") is None
+        lone += [members[1](synthetic_activation(20, 300, 256).cuda()) for _ in range(3)]
+        assert len(calls) == 1
+        whole = [[m(x) for m in members] for x in inputs]
+        assert len(calls) == 1 + len(inputs) - 1 and not group["grouped_outputs"][1]
+        again = [[m(x) for m in members] for x in inputs]
+        assert len(calls) == 1 + 2 * len(inputs) - 1
+        monkeypatch.setattr(BitLinear, "grouped_inference", False)
+        want = [[m(x.clone()) for m in members] for x in inputs]
+    for i in range(len(inputs)):
+        assert torch.equal(lone[i], want[i][1])
+        for y, z, w in zip(whole[i], again[i], want[i]):
+            assert torch.equal(y, w) and torch.equal(z, w)
+    del inputs
+    assert group["alone_input"] is None and group["grouped_outputs"] is None
