@@ -1310,18 +1310,35 @@ def _lowrank_operands(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None)
             and x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 and (s is None or s.dtype == torch.bfloat16))
 
 
+def _one_pass_takes(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None) -> bool:
+    """A projection of 256 rows or more runs on the one-pass kernel: ranks 32, 64 and 128 always; 96, 192 and 256, which have few
+    stages of the wide tile in flight and fetch all of V again for every row tile, up to a bound on the work.  Microseconds,
+    kernel | library product and its multiplication by s:
+        R = 96   8000 x 8960 40.8 | 43.1, 16384 x 8960 67.8 | 66.3, 16384 x 18944 167 | 139
+        R = 192  800 x 18944 35 | 72, 4096 x 3584 23.9 | 27.3, 8000 x 1536 22.2 | 24.3, 2103 x 8960 33.5 | 29.5, 16384 x 18944 328 | 215
+        R = 256  800 x 18944 42 | 87, 2103 x 3584 20.6 | 24.7, 4096 x 3584 28.2 | 24.3, 8000 x 3584 44.6 | 36.8, 16384 x 18944 428 | 252
+    The library product also takes what the kernel does not read there (rows that overlap, an unaligned V) and what autograd records."""
+    R = v.shape[0]
+    if R in (32, 64, 128):
+        return True
+    if R not in ONE_PASS_RANKS:
+        return False
+    M, K = x2.shape
+    return ((M <= 1024 or M * K * R <= (10 ** 10 if R == 96 else 3 * 10 ** 9)) and x2.stride(0) >= K and (v.data_ptr() % 16 == 0 or not v.is_contiguous())
+            and not (torch.is_grad_enabled() and (x2.requires_grad or v.requires_grad or (s is not None and s.requires_grad))))
+
+
 def lowrank_stack_applies(x2: torch.Tensor, factors) -> bool:
-    """lowrank_project takes the (v, s) pairs of a projection group as FactorStacks: 256 rows or more, every rank and their sum
-    ranks of the one-pass kernel.  Column for column the bits of the members' own projections."""
+    """lowrank_project takes the (v, s) pairs of a projection group as FactorStacks: 256 rows or more, every member's own projection
+    and the sum of the ranks on the one-pass kernel.  Column for column the bits of the members' own projections."""
     M, K = x2.shape
     if M < 256 or len(factors) > 4:
         return False
     total = 0
     for v, s in factors:
-        r = v.shape[0]
-        if r not in ONE_PASS_RANKS or v.shape[1] != K or v.dtype != torch.bfloat16 or s.dtype != torch.bfloat16:
+        if v.shape[1] != K or v.dtype != torch.bfloat16 or s.dtype != torch.bfloat16 or not _one_pass_takes(x2, v, s):
             return False
-        total += r
+        total += v.shape[0]
     return total in ONE_PASS_RANKS and _lowrank_operands(x2, *factors[0])
 
 
@@ -1353,15 +1370,14 @@ def _lowrank_project_stack(x2: torch.Tensor, v: FactorStack, s: FactorStack):
 def lowrank_project(x2: torch.Tensor, v: "torch.Tensor | FactorStack", s: "torch.Tensor | FactorStack | None" = None):
     """Rank-r projection of the low-rank branch: xv = x2[M, K] . v[R, K]^T in bf16 (binary32 accumulation) and, with
     `s` [R], t = bf16(xv * s): returns xv or (xv, t).  Decode-sized batches (M < 256, R <= 256) run on the library's
-    split-K kernel, larger ones (R in 32 / 64 / 96 / 128 / 192 / 256) on its one-pass kernel; other shapes are a torch
-    matmul.  FactorStacks (lowrank_stack_applies): the members' columns side by side."""
+    split-K kernel, larger ones on its one-pass kernel (_one_pass_takes); other shapes are a torch matmul.  FactorStacks (lowrank_stack_applies): the members' columns side by side."""
     if isinstance(v, FactorStack):
         return _lowrank_project_stack(x2, v, s)
     M, K = x2.shape
     R = v.shape[0]
     common = _lowrank_operands(x2, v, s)
     small = common and M < 256 and R % 32 == 0 and 0 < R <= 256
-    large = common and M >= 256 and R in ONE_PASS_RANKS
+    large = common and M >= 256 and _one_pass_takes(x2, v, s)
     if not (small or large):
         xv = torch.matmul(x2, v.T)
         return xv if s is None else (xv, xv * s.to(xv.dtype))

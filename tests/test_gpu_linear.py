@@ -740,17 +740,43 @@ def test_rank_r_projection_in_column_groups(M, R, K):
 
 @pytest.mark.parametrize("M,R,K", [(16385, 96, 320), (16384, 128, 64), (16400, 192, 1088), (16321, 256, 192), (4096, 192, 4160), (4090, 96, 4096), (4100, 128, 8960)])
 def test_rank_r_columns_have_the_same_bits_at_every_width(M, R, K):
-    """The forms with 64 rows per workgroup, stages of 64 k and of 128, with and without K slices: 32 columns have the bits of the
-    projection onto these 32 alone, so that a group's common projection equals its members' own."""
+    """The forms with 64 rows per workgroup, stages of 64 k and of 128, with and without K slices: the members of a group have the
+    bits of their own projections."""
     from metis_hip import ops
     g = torch.Generator(device="cuda").manual_seed(6500 + M + R)
     x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
     v = (torch.randn(R, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
     s = (torch.rand(R, generator=g, device="cuda") * 4 + 0.1).bfloat16()
+    ranks = {96: (32, 64), 128: (64, 32, 32), 192: (64, 64, 64), 256: (32, 64, 32, 128)}[R]
+    vs, ss = v.split(ranks), s.split(ranks)
+    assert ops.lowrank_stack_applies(x, list(zip(vs, ss)))
+    xv, t = ops.lowrank_project(x, ops.FactorStack(vs), ops.FactorStack(ss))
+    for a, b, va, sa in zip(xv.split(ranks, dim=1), t.split(ranks, dim=1), vs, ss):
+        one, ts = ops.lowrank_project(x, va, sa)
+        assert torch.equal(a, one) and torch.equal(b, ts)
+
+
+@pytest.mark.parametrize("R", [96, 192, 256])
+def test_wide_ranks_take_what_the_library_product_took(R):
+    """Ranks 96, 192 and 256 from 256 rows on: an unaligned V, rows that overlap, operands that autograd records and large products
+    are the library's, as they were before the kernel knew these ranks (torch's own product: equal bits)."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(6600 + R)
+    K = 256
+    x = torch.randn(300, K, generator=g, device="cuda").bfloat16()
+    flat = torch.randn(R * K + 1, generator=g, device="cuda").bfloat16()
+    s = torch.rand(R, generator=g, device="cuda").bfloat16()
+    v = flat[1:].view(R, K)
     xv, t = ops.lowrank_project(x, v, s)
-    for c in range(0, R, 32):
-        one, ts = ops.lowrank_project(x, v[c:c + 32], s[c:c + 32])
-        assert torch.equal(xv[:, c:c + 32], one) and torch.equal(t[:, c:c + 32], ts)
+    assert torch.equal(xv, torch.matmul(x, v.T)) and torch.equal(t, xv * s)
+    assert torch.equal(ops.lowrank_project(x[:1].expand(300, K), v.clone()), torch.matmul(x[:1].expand(300, K), v.T))
+    w = v.clone().requires_grad_(True)
+    y = ops.lowrank_project(x, w, s)[1]
+    grad, = torch.autograd.grad(y.sum(), w)
+    assert torch.allclose(grad.float(), (s.float()[:, None] * x.float().sum(0)), rtol=2e-2, atol=2e-1)
+    big = torch.randn(12000, 8960, generator=g, device="cuda").bfloat16()
+    vb = torch.randn(R, 8960, generator=g, device="cuda").bfloat16()
+    assert torch.equal(ops.lowrank_project(big, vb), torch.matmul(big, vb.T))
 
 
 @pytest.mark.parametrize("L,C,R", [(1000, 520, 32), (4096, 1536, 64), (4096, 8960, 32), (2048, 14336, 64), (777, 256, 128)])
