@@ -30,7 +30,7 @@ __host__ __device__ __forceinline__ int xt_swz(int q) { return ((q >> 2) & 1) | 
 // ---------------------------------------------------------------------------------------------
 // packed NVFP4 -> tiled 16-bit operands.  One wave per tile: lane l writes slot l (row l / 4).  A wave walks
 // eight consecutive k tiles of one tile row, so the 128-byte lines of codes it touches are used whole.
-// HBM-bound: 0.5625 B read, 2 B written per element.  The unit's eight words of codes and eight scales are requested
+// HBM-bound: 0.5625 B read, 2 B written per element.  The unit's eight words of codes and eight scales (AHEAD) are requested
 // together: one at a time, between the stores, the lines of codes (16 bytes of each of 16 rows per load) were pushed out of L2
 // by the output before the next visit.  16384 x 18944 from a deferred activation 249 -> 209 us, 16384 x 3584 36.9 -> 32.6,
 // the 18944 x 3584 weight 48.0 -> 41.3, 8192 x 4096 17.0 -> 16.3.  Streaming stores on top change nothing (214, 31.7).
@@ -51,7 +51,7 @@ __host__ __device__ __forceinline__ int xt_swz(int q) { return ((q >> 2) & 1) | 
 //        block maximum per block instead of E4M3 bytes, `partials` the partial tensor maxima.  The kernel forms the
 //        tensor unit (written to unit_out by the first workgroup) and every scale byte itself, in the arithmetic the
 //        tensor was quantized in (QMODE) -- the expressions of quant_scales_kernel, so the bytes it would have written.
-template <int PB16, int RHT = 0, int DEF = 0, int QMODE = 0>
+template <int PB16, int RHT = 0, int DEF = 0, int QMODE = 0, int AHEAD = 8>
 __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restrict__ codes, const uint8_t* __restrict__ scales,
                                                         const float* __restrict__ unit_p, uint4* __restrict__ out, int rows,
                                                         int K, int row_tiles, uint32_t sign_mask,
@@ -77,29 +77,30 @@ __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restri
         const int rb_ = (int)(un / kgroups), kg = (int)(un - (int64_t)rb_ * kgroups);
         const int row = rb_ * 16 + q;
         const bool live = row < rows;
-        const int kb0 = kg * 8, kend = min(kt, kb0 + 8);
-        uint32_t cw[8] = {}, sw[8] = {};                         // every tile's codes and scales are requested before the first is expanded
-        if (live) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                if (kb0 + i < kend) {
-                    const int k8 = (kb0 + i) * 4 + chunk;        // index of the 8-element chunk inside the row
-                    cw[i] = codes[(int64_t)row * (K / 8) + k8];
-                    if constexpr (DEF != 0) sw[i] = maxima[(int64_t)row * (K / 16) + (k8 >> 1)];
-                    else sw[i] = scales[(int64_t)row * (K / 16) + (k8 >> 1)];
-                }
-            }
-        }
+        const int kend = min(kt, kg * 8 + 8);
+        uint32_t cw[AHEAD], sw[AHEAD];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int kb = kb0 + i;
+            const int kb = kg * 8 + i;
             if (kb >= kend) break;                               // the same for the whole wave
+            if (i % AHEAD == 0) {                                // AHEAD tiles' codes and scales are requested before the first is expanded
+#pragma unroll
+                for (int n = 0; n < AHEAD; ++n) {
+                    cw[n] = sw[n] = 0u;
+                    if (live && kb + n < kend) {
+                        const int k8 = (kb + n) * 4 + chunk;     // index of the 8-element chunk inside the row
+                        cw[n] = codes[(int64_t)row * (K / 8) + k8];
+                        if constexpr (DEF != 0) sw[n] = maxima[(int64_t)row * (K / 16) + (k8 >> 1)];
+                        else sw[n] = scales[(int64_t)row * (K / 16) + (k8 >> 1)];
+                    }
+                }
+            }
             uint4 v = make_uint4(0u, 0u, 0u, 0u);
             if (live) {                                          // lane pairs (l, l ^ 1) share their row: both live or neither
-                const uint32_t c = cw[i];
+                const uint32_t c = cw[i % AHEAD];
                 uint32_t sb;
-                if constexpr (DEF != 0) sb = scale_byte_of<QMODE>((uint16_t)sw[i], unit);
-                else sb = sw[i];
+                if constexpr (DEF != 0) sb = scale_byte_of<QMODE>((uint16_t)sw[i % AHEAD], unit);
+                else sb = sw[i % AHEAD];
                 if constexpr (RHT != 0) {
                     const float dq = PB16 ? rb(e4m3_value(sb) * unit) : e4m3_value(sb) * 0.00390625f;
                     const float2_t p[4] = {__builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 1),
@@ -162,6 +163,16 @@ __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restri
             out[((int64_t)rb_ * kt + kb) * 64 + lane] = v;
         }
     }
+}
+
+// Ten to twenty units per compute unit are all resident at once and start together: with eight tiles requested ahead each of them
+// first reads, then writes, and HBM does one at a time; two tiles ahead keep both going.  Microseconds, eight | two ahead (bf16
+// operands of a deferred activation): 800 x 18944 10.9 | 9.9, 2103 x 8960 12.4 | 11.2, 4096 x 3584 10.9 | 9.8; fewer units (800 x 3584
+// 5.0 | 5.6) have no reads to overlap, more of them (16384 x 3584 26.7 | 33.3) drift apart and want whole lines of codes.
+static bool expand_two_ahead(int64_t units)
+{
+    const int64_t cus = device_cus();
+    return units >= 10 * cus && units <= 20 * cus;
 }
 
 // Transposing variant: the packed [R, C] tensor (blocks along C) becomes the tiled operand [C, R], the layout a GEMM
@@ -313,15 +324,11 @@ int expand_xt(const void* codes, const void* scales, const float* unit, int64_t 
     int64_t g = (units + 3) / 4;
     const int64_t cap = (int64_t)device_cus() * 16;
     if (g > cap) g = cap;
-#define METIS_EX(P, R) hipLaunchKernelGGL((expand_xt_kernel<P, R>), dim3((unsigned)g), dim3(256), 0, st, (const uint32_t*)codes, \
-                                          (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols, row_tiles, sign_mask)
-    if (center) {
-        hipLaunchKernelGGL((expand_xt_kernel<1, 0>), dim3((unsigned)g), dim3(256), 0, st, (const uint32_t*)codes, (const uint8_t*)scales,
-                           unit, (uint4*)out, (int)rows, (int)cols, row_tiles, sign_mask, (const uint16_t*)center);
-        return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
-    }
-    if (mode == METIS_MODE_PB16) { if (rht) METIS_EX(1, 1); else METIS_EX(1, 0); }
-    else { if (rht) METIS_EX(0, 1); else METIS_EX(0, 0); }
+    const bool two = !rht && expand_two_ahead(units);
+#define METIS_EX(P, R, A) hipLaunchKernelGGL((expand_xt_kernel<P, R, 0, 0, A>), dim3((unsigned)g), dim3(256), 0, st, (const uint32_t*)codes, \
+                                          (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols, row_tiles, sign_mask, (const uint16_t*)center)
+    if (mode == METIS_MODE_PB16) { if (rht) METIS_EX(1, 1, 8); else if (two) METIS_EX(1, 0, 2); else METIS_EX(1, 0, 8); }
+    else { if (rht) METIS_EX(0, 1, 8); else if (two) METIS_EX(0, 0, 2); else METIS_EX(0, 0, 8); }
 #undef METIS_EX
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
@@ -344,12 +351,15 @@ int expand_xt_deferred(const void* codes, const void* deferred, int64_t rows, in
     int64_t g = (units + 3) / 4;
     const int64_t cap = (int64_t)device_cus() * 16;
     if (g > cap) g = cap;
-#define METIS_EXD(P, Q) hipLaunchKernelGGL((expand_xt_kernel<P, 0, 1, Q>), dim3((unsigned)g), dim3(256), 0, st, (const uint32_t*)codes, \
+#define METIS_EXDA(P, Q, A) hipLaunchKernelGGL((expand_xt_kernel<P, 0, 1, Q, A>), dim3((unsigned)g), dim3(256), 0, st, (const uint32_t*)codes, \
                                            (const uint8_t*)ws.amax, nullptr, (uint4*)out, (int)rows, (int)cols, row_tiles, 0u, \
                                            (const uint16_t*)center, (const uint32_t*)ws.gmax, unit_out)
+#define METIS_EXD(P, Q) do { if (two) METIS_EXDA(P, Q, 2); else METIS_EXDA(P, Q, 8); } while (0)
+    const bool two = expand_two_ahead(units);
     if (mode == METIS_MODE_PB16) { if (qmode) METIS_EXD(1, 1); else METIS_EXD(1, 0); }
     else { if (qmode) METIS_EXD(0, 1); else METIS_EXD(0, 0); }
 #undef METIS_EXD
+#undef METIS_EXDA
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 

@@ -894,6 +894,29 @@ def test_gradient_of_the_rank_r_scale_vector_is_added_in_its_documented_order(L,
     assert torch.equal(ops.lowrank_scale_grad(g.cuda(), xv.cuda()).cpu(), total)
 
 
+
+@pytest.mark.parametrize("rows,cols", [(2925, 3584), (2560, 4096), (5112, 4096), (800, 18848), (40900, 288)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_tiled_expansion_of_middling_tensors(rows, cols, mode):
+    """The sizes whose tiles are requested two at a time (both ends of the range, rows and tiles that do not fill the last unit): the
+    operand's rows equal those of expansions of 512-row parts, which request eight; deferred scale bytes and a centre likewise."""
+    from metis_hip import ops
+    x = torch.randn(rows, cols, generator=torch.Generator(device="cuda").manual_seed(rows), device="cuda").bfloat16()
+    p, d = ops.quantize(x, mode), ops.quantize(x, mode, deferred=True)
+    center = torch.randn(cols, device="cuda").bfloat16() if mode else None
+    for cen in ([None, center] if mode else [None]):
+        kw = dict(cache=False, mode=mode, center=cen)
+        got = ops.expand_tiled(p, **kw)
+        assert torch.equal(got, ops.expand_tiled(d, **kw))
+        at = 0
+        for r0 in range(0, rows, 512):
+            n = min(512, rows - r0)
+            part = ops.expand_tiled(ops.PackedNVFP4(p.codes[r0:r0 + n], p.scales[r0:r0 + n], p.unit, n, cols, mode), **kw)
+            assert torch.equal(got[at:at + part.numel()], part)
+            at += part.numel()
+        assert at == got.numel()
+
+
 def test_memory_bound_deployments_can_drop_the_derived_weight_copies(monkeypatch):
     """A cached weight holds 0.5625 B per parameter packed; the tiled binary16 expansion (2 B, one per arithmetic) and
     the decode layout (0.5625 B) are built on first use.  With both switches off nothing but the packed form stays,
