@@ -459,7 +459,9 @@ def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, of
                                                 uc.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
         if rc:
             check(rc, "metis_nvfp4_quant_sr_both_padded", x.shape)
-    return PackedNVFP4(cr[:have], sr_[:have], ur, have, cols, mode), PackedNVFP4(cc, sc, uc, cols, rows, mode)
+    if have != rows:
+        cr, sr_ = cr[:have], sr_[:have]
+    return PackedNVFP4(cr, sr_, ur, have, cols, mode), PackedNVFP4(cc, sc, uc, cols, rows, mode)
 
 
 def dequantize(p: PackedNVFP4, dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:

@@ -913,14 +913,14 @@ def test_projection_group_at_prefill_size_keeps_every_rank_on_the_kernel(ranks, 
         assert rel_fro(y.float().cpu(), w.float().cpu()) <= 2.0 ** -8
 
 
-def _prefill_group(K, ns, r, mean, compute, bias, seed=7, cached=True):
+def _prefill_group(K, ns, r, mean, compute, bias, seed=7, cached=True, nv=False):
     """A projection group of layers of unequal width, factors in bf16, as replace_linear_with_metis wires it."""
     from metis_hip import BitLinear, LinearLowbit, MetisArgs
     g = torch.Generator(device="cuda").manual_seed(seed)
     group = {"name": "g", "mean_cache": {}, "input_ref": None, "quantized_input": None, "members": []}
     for n in ns:
         args = MetisArgs(forward_svd_rank=r, cache_quantized_weight=cached) if mean else MetisArgs.direct_fp4(forward_svd_rank=r)
-        args.cache_quantized_weight = cached
+        args.cache_quantized_weight, args.enable_nv_recipe = cached, nv
         m = BitLinear(K, n, args=args, bias=bias, dtype=torch.bfloat16, compute_dtype=compute)
         make = dict(args=args, device="cuda", storage_dtype=torch.bfloat16, compute_dtype=compute)
         m.warmup_linear, m.vlinear = LinearLowbit(K, n, bias=bias, **make), LinearLowbit(K, r, bias=False, **make)
@@ -1095,3 +1095,19 @@ def test_a_member_probed_on_its_own_does_not_compute_its_siblings_over_and_over(
             assert torch.equal(y, w) and torch.equal(z, w)
     del inputs
     assert group["alone_input"] is None and group["grouped_outputs"] is None
+
+
+@pytest.mark.parametrize("compute", [torch.bfloat16, torch.float32])
+def test_a_prompt_of_a_group_under_the_nv_recipe_has_the_same_bits_with_and_without_autograd(compute, monkeypatch):
+    """Weights packed in the rotated domain: the group's launch on their rotated-back operands, and the members' own calls."""
+    from metis_hip import LinearLowbitFunction as F, ops
+    monkeypatch.setattr(F, "enable_nv_recipe", F.enable_nv_recipe)          # (each layer sets it: back to what it was)
+    members, _ = _prefill_group(1024, (2304, 512, 260), 64, False, compute, True, nv=True)
+    x = synthetic_activation(3, 411, 1024).cuda()
+    calls, real = [], ops._linear_fwd_tiled_grouped
+    monkeypatch.setattr(ops, "_linear_fwd_tiled_grouped", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    with torch.no_grad():
+        got = [m(x) for m in members]
+    assert len(calls) == 1
+    for y, w in zip(got, [m(x.clone()) for m in members]):
+        assert torch.equal(y, w)

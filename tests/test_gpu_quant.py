@@ -737,3 +737,12 @@ def test_binary32_round_trip_from_one_call(ops, rows, cols):
     assert same_bits(out.cpu(), ops.dequantize(want, torch.float32).cpu())
     q = quant_func["nvfp4e2m1bnosr"]
     assert same_bits(q.quantize_dequantize(x).cpu(), out.cpu())
+
+
+def test_both_packings_of_a_whole_row_count_are_tensors_of_their_own(ops):
+    """Only a padded call hands out views (the row packing of the tensor's own rows)."""
+    x = torch.randn(64, 128, device="cuda").bfloat16()
+    row, col = ops.quantize_both_sr(x, 0, seed=1)
+    assert all(t_._base is None for t_ in (row.codes, row.scales, col.codes, col.scales))
+    padded, _ = ops.quantize_both_sr(x[:50], 0, seed=1, pad_rows=64)
+    assert (padded.rows, padded.codes.shape[0], padded.scales.shape[0]) == (50, 50, 50)
