@@ -912,8 +912,9 @@ def gemm_tiled(ax: torch.Tensor, a_unit: torch.Tensor, bx: torch.Tensor, b_unit:
 def linear_fwd_tiled(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None = None, u: torch.Tensor | None = None,
                      bias: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16,
                      a_tiled: torch.Tensor | None = None, reference_rounding: bool = False,
-                     split_k: bool = True, center: torch.Tensor | None = None) -> torch.Tensor:
+                     split_k: bool = True, center: torch.Tensor | None = None, batch: "_TiledBatch | None" = None) -> torch.Tensor:
     """linear_fwd on tiled 16-bit expansions: b's is cached on b when b is persistent, a's is made here unless given.
+    batch: the product is queued there and its output, returned, is filled when the batch runs (linear_fwd_tiled_grouped).
 
     reference_rounding (both operands packed in bf16 arithmetic): operands are the reference's bf16 dequantized
     values and the epilogue rounds where the reference's all-bf16 forward rounds; otherwise exact products.
@@ -930,6 +931,8 @@ def linear_fwd_tiled(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None =
         raise ValueError("a centre inside the operand belongs to reference_rounding")
     bx = expand_tiled(b, cache=b.persistent, mode=mode)
     ax = a_tiled if a_tiled is not None else expand_tiled(a, cache=a.shared, mode=mode, center=center)
+    if batch is not None:
+        return batch.add(bx, b, t, u, bias)
     return gemm_tiled(ax, a.unit, bx, b.unit, a.rows, b.rows, a.cols, mode=mode, t=t, u=u, bias=bias, out_dtype=out_dtype,
                       split_k=split_k)
 
@@ -960,10 +963,8 @@ def _linear_fwd_tiled_grouped(a: PackedNVFP4, members, out_dtype, center, refere
         raise ValueError("a centre inside the operand belongs to reference_rounding")
     ax = expand_tiled(a, cache=False, mode=mode, center=center)
     batch = _TiledBatch(a, ax, len(members), out_dtype, mode)
-    outs = []
-    for b, t, u, bias in members:
-        kept = b.tiled_pb16 if mode == MODE_PB16 else b.tiled
-        outs.append(batch.add(kept if kept is not None else expand_tiled(b, cache=b.persistent, mode=mode), b, t, u, bias))
+    outs = [linear_fwd_tiled(a, b, t=t, u=u, bias=bias, out_dtype=out_dtype, a_tiled=ax, reference_rounding=mode == MODE_PB16, center=center,
+                             batch=batch) for b, t, u, bias in members]
     batch.run()
     return outs
 
