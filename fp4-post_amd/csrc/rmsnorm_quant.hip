@@ -537,8 +537,8 @@ int rmsnorm_colmean(const void* x, const void* gamma, float eps, int64_t rows, i
     return finish_column_sums(partial, g, cols, (float)rows, mean, mean_bf16, cached, (float)cached_count, (float)rows, mean32, st);
 }
 
-// One workgroup per compute unit with the column sums (each leaves a partial row for the finishing launch), enough of
-// them to fill the device without.
+// Two workgroups per compute unit with the column sums (their registers leave room for no more, and each leaves a partial row for
+// the finishing launch), four without.
 static int backward_grid(int64_t rows, bool sums)
 {
     int64_t g = (rows + 3) / 4;

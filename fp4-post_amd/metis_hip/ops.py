@@ -1671,11 +1671,12 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
 
 def _tiled_backward_pays(M: int, N: int, K: int, device_index: int) -> bool:
     """Whether a backward product out[M, N] over a contraction of K goes to the pipelined kernel on tiled expansions made
-    for this one call: from about 2e11 flop on, with at least one 256 x 256 tile per compute unit, the faster GEMM more
-    than pays for writing the expansions (8192 x 4096 x 14336: input gradient 858 -> 749 us with the weight's
-    expansion cached, weight gradient 915 -> 835 us with both operands expanded; 4096 x 1536 x 8960: 134 -> 149 and
-    117 -> 141 us, so small products stay on the packed kernel).  Plain products keep their bits; with a low-rank term
-    the binary32 sums are taken in another order."""
+    for this one call: from about 2e11 flop on, with at least one 256 x 256 tile per compute unit, the faster GEMM pays
+    for writing the expansions.  Microseconds, packed | tiled with both operands expanded | with the weight's
+    expansion kept: 8192 x 4096 over 14336 826 | 791 | 754, 14336 x 4096 over 8192 851 | 797, 18944 x 3584 over 2112 301 | 277; below
+    either bound the two are close and the order varies: 4096 x 1536 over 8960 152 | 144 | 136, 8960 x 1536 over 4096
+    115 | 119, 2103 x 3584 over 18944 307 | 315 | 273, 4096 x 3584 over 18944 496 | 494 | 451.  Plain products keep their
+    bits; with a low-rank term the binary32 sums are taken in another order."""
     return (tiled_weight_copies and M >= 256 and N >= 256 and K % 32 == 0 and 2.0 * M * N * K >= 2e11
             and (M // 256) * (N // 256) >= _device_cus(device_index))
 
