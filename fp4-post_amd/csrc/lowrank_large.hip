@@ -2,19 +2,20 @@
 // accumulation on MFMA.  Both are bound by one pass over the tall operand in HBM.
 //
 //   lowrank_nt:  xv[M, R] = x[M, K] . v[R, K]^T,  t = bf16(xv * s)      `vlinear(x)` and `torch.mul(self.s, y)` of
-//                BitLinear.forward with the bf16 V of the north-star formula (src/Metis/Metis/bitlinear.py:752-756);
+//                BitLinear.forward with V in bf16 (src/Metis/Metis/bitlinear.py:752-756);
 //                with v = U^T also dY . U of the backward pass
 //   lowrank_tn:  out[C, R] = sum_l a[l, C] . b[l, R]                     the two products of the backward pass that
 //                contract over tokens: dY^T . (xv * s) -> grad of U, x^T . g_xv -> grad of V (written transposed)
 //
-// lowrank_nt: a workgroup owns 32 or 64 rows of x and walks K in stages of 64 or 128.  The x rows and the R rows of v of a
-// stage (v from L2 after the first workgroup touched it) go straight from memory to LDS, into a ring of two to four stages,
-// so that no wave waits for the loads it issued last; the waves share a stage's k, 32 each, and their partial sums meet in
-// LDS at the end.  (Staged through registers two steps ahead, with two barriers per step and the encoder between them, the
-// loads in flight per compute unit were what its registers held: 16384 x 3584, R = 64 34.8 -> 27.7 us; with the quantizer
-// 61.7 -> 47.5, 16384 x 18944 309 -> 230; 2103 x 18944 27 -> 24.  The read of x alone at 5 TB/s: 23.5; with codes and
-// maxima written 30.8 and 163.  Bound by HBM, with the quantizer by the encoder's vector work at two waves per SIMD; deeper
-// rings change nothing.)
+// lowrank_nt: a workgroup owns 32 rows of x and walks K in stages of 64 or 128.  The x rows and the R rows of v of a stage (v
+// from L2 after the first workgroup touched it) go straight from memory to LDS, into a ring of two to four stages, so that no
+// wave waits for the loads it issued last; the waves share a stage's quarters of 64 k and the column tiles.  (Staged through
+// registers two steps ahead, with two barriers per step and the encoder between them, the loads in flight per compute unit were
+// what its registers held: 16384 x 3584, R = 64 25.7 -> 23.4 us, 8192 x 4096 22.2 -> 15.9; with the quantizer 40.9 -> 32.4 and
+// 27.9 -> 26.4, 4096 x 8960 31.2 -> 26.6.  The read of x alone at 5 TB/s: 23.5 and 13.4 from HBM; with codes and maxima written 30.8
+// and 17.6.  Bound by memory, with the quantizer by the encoder's vector work.  64 rows per workgroup read v half as often --
+// 16384 x 3584, R = 192 41 us in place of 48, the quantizing pass of 16384 x 18944 203 in place of 245 -- but their two row tiles
+// have to start at the same step of K: another order of the sums.)
 //
 // lowrank_tn: the contraction runs down the rows of both operands, so each has to be turned: a workgroup owns 64
 // columns of a and one slice of the tokens; a step of 64 tokens is loaded row by row (coalesced) and staged in LDS as it
@@ -28,17 +29,21 @@
 
 namespace metis {
 
-// A form of the kernel: ROWS rows of x per workgroup, KS k per stage, NS stages in the ring; one thread per block of 16 of x.
-template <int RT, int ROWS, int KS, int NS> struct NtForm {
-    static constexpr int kThreads = ROWS * KS / 16, kWaves = kThreads / 64;
+constexpr int NT_ROWS = 32;                      // rows of x per workgroup
+// A form of the kernel: KS k per stage, NS stages in the ring; one thread per block of 16 of x.
+template <int RT, int KS, int NS> struct NtForm {
+    static constexpr int kThreads = NT_ROWS * KS / 16, kWaves = kThreads / 64;
     static constexpr int kRowBytes = KS * 2, kRowsPerPiece = 1024 / kRowBytes, kChunks = kRowBytes / 16;
-    static constexpr int kStage = (ROWS + RT * 32) * kRowBytes;               // bytes of a stage: x rows, then v rows
-    static constexpr int kLoads = kStage / 1024 / kWaves, kXLoads = ROWS / kRowsPerPiece / kWaves;   // 1 KiB loads per wave and stage; those of x
-    static constexpr int kRowTiles = ROWS / 32, kParts = kWaves / kRowTiles;  // the waves of a row tile share the stage's k, 32 each
-    static constexpr int kHalves = 128 / KS;                                  // stages of a step of 128 k, each with sums of its own
-    static constexpr int kRed = kHalves * (kParts - 1) * kRowTiles * RT * 4096 + 64;   // partial sums of the waves, then their maxima
+    static constexpr int kStage = (NT_ROWS + RT * 32) * kRowBytes;            // bytes of a stage: x rows, then v rows
+    static constexpr int kLoads = kStage / 1024 / kWaves, kXLoads = NT_ROWS / kRowsPerPiece / kWaves;   // 1 KiB loads per wave and stage; those of x
+    // K is walked in steps of 256, whose quarters of 64 have sums of their own: the waves share the quarters of a stage and the
+    // column tiles; a step is kStages stages, with a set of sums for each.
+    static constexpr int kQuarters = KS / 64, kStages = 4 / kQuarters;
+    static constexpr int kColGroups = kWaves / kQuarters, kColTiles = (RT + kColGroups - 1) / kColGroups;
+    static constexpr int kRed = kStages * (kQuarters - 1) * RT * 4096 + 64;   // partial sums of the waves, then their maxima
     static constexpr int kLds = NS * kStage > kRed ? NS * kStage : kRed;
-    static_assert((KS == 64 || KS == 128) && kParts * 32 == KS && kStage % (1024 * kWaves) == 0 && kXLoads >= 1, "every wave loads whole pieces and multiplies two steps of 16");
+    static_assert((KS == 64 || KS == 128) && kColGroups * kQuarters == kWaves && kStage % (1024 * kWaves) == 0 && kXLoads >= 1,
+                  "every wave loads whole pieces and multiplies a quarter");
 };
 // The factors of up to four projections of the same x, their columns side by side in xv and t: a group's members hand in
 // their own V and s (stacked copies would have to be made anew whenever one of them changes).
@@ -83,38 +88,39 @@ template <int VM> __device__ __forceinline__ void nt_wait()
 // QMODE >= 0: the same pass also quantizes x (round to nearest, rows; METIS_MODE_P32 or _PB16 arithmetic): a stage holds one
 // block of 16 per thread, read back from LDS -- E2M1 codes, the block maximum parked as bf16, one partial tensor maximum per
 // workgroup: what quant_codes_contig_kernel leaves for a consumer that forms the scale bytes itself.
-// CUT: K % 128 == 64.
-// Every form adds an element's products in the same order -- the four quarters of each step of 128 k in sums of their own, the
-// steps of a row tile from the same one on, the quarters' sums at the end -- so that a column of v gives the same bits alone
-// and beside any others.  Stages of 64 k therefore keep two sums per wave and element, one for each half of a step.
-template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
-__global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
+// Every form adds an element's products in the same order -- the four quarters of each step of 256 k in sums of their own, the
+// steps from the row tile's own first one on, the quarters' sums at the end, in order -- so that a column of v gives the same
+// bits alone and beside any others, with and without the quantizer.
+// TAIL: K % 256 != 0.
+template <int RT, int QMODE, int KS, int NS, bool TAIL>
+__global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const NtFactors fac, uint16_t* __restrict__ xv, uint16_t* __restrict__ t, int M, int K, float* __restrict__ part, uint2* __restrict__ codes,
     uint16_t* __restrict__ q_amax, uint32_t* __restrict__ q_gmax, uint32_t fill_to, int rotate, int R)
 {
-    using F = NtForm<RT, ROWS, KS, NS>;
+    using F = NtForm<RT, KS, NS>;
     const int col0 = QMODE < 0 ? (int)blockIdx.z * RT * 32 : 0; // R: all columns; the workgroup's are RT * 32 of them from here on
     constexpr int STAGE = F::kStage, LPW = F::kLoads, XL = F::kXLoads, RPP = F::kRowsPerPiece, RB = F::kRowBytes;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];     // the ring, then the waves' partial sums
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int m0 = blockIdx.x * ROWS;
-    // CUT (K % 64 == 0): the last step of 128 has only its first half.  The lanes of the other half (the second stage of that
-    // step, where a stage is 64) then fetch the first again, multiply zeros, and their threads encode the first half's blocks once
-    // more (the same bytes).
+    const int m0 = blockIdx.x * NT_ROWS;
+    // TAIL (K % 64 == 0): the last step is cut.  A stage that begins past the end fetches the step's first again, the lanes of a
+    // half that does its other half; the quarters past the end multiply zeros, and the threads of such blocks encode the ones that
+    // were fetched once more (the same bytes).
     // A template parameter: the branch would keep product and encoder from being interleaved (8192 x 4096: 27.4 -> 35.6 us).
-    constexpr int NH = F::kHalves;
-    const int steps_all = (K + 127) / 128;
+    constexpr int NH = F::kStages;
+    const int steps_all = (K + 255) / 256;
     const int per = (steps_all + (int)gridDim.y - 1) / (int)gridDim.y;
     const int first = (int)blockIdx.y * per, wide_steps = max(0, min(steps_all, first + per) - first);
     const int steps = wide_steps * NH;                          // stages
-    // Every row tile starts at a different stage of its K range and wraps around: at any moment the workgroups then read
+    // Every row tile starts at a different step of its K range and wraps around: at any moment the workgroups then read
     // different column stripes of x instead of the same one.  With rows a multiple of 4 KiB long, pieces at the same offset
     // of every row can fall on the same few memory channels.  The binary32 sums of a tile are therefore added in an order
-    // that depends on the tile, the same for every call and with or without the quantizer.  (An offset of 13 steps per tile:
-    // 8192 x 4096 from flushed caches 40 us, 45 with 5, 41-46 without; other row lengths within 2 %.)
+    // that depends on the tile, the same for every call.  (An offset of 5 steps per tile: 8192 x 4096 from flushed caches 31 us,
+    // 39 without; other row lengths within 2 %.)
     const int rot = (rotate && steps > 0) ? (int)((blockIdx.x * (unsigned)rotate) % (unsigned)wide_steps) : 0;
-    auto kof = [&](int st) { int q = st / NH + rot; if (q >= wide_steps) q -= wide_steps; return (first + q) * 128 + st % NH * KS; };
+    auto kof = [&](int st) { int q = st / NH + rot; if (q >= wide_steps) q -= wide_steps; return (first + q) * 256 + st % NH * KS; };
+    auto fetched = [&](int k0) { return TAIL && k0 >= K ? k0 & ~255 : k0; };   // where the stage at k0 is fetched from
 
     // ---- loads go straight to LDS: piece p = j * waves + wave of a stage is 1 KiB, whole rows of x | v.  The 16-byte chunk c
     // of row q lies at position c ^ swz(q) of the row, so that the fragment reads (32 rows at the same chunk) spread over all
@@ -131,40 +137,44 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
         upper |= (uint32_t)(chunk >> 3) << j;
     }
     auto issue = [&](int slot, int st) {
-        const int k0 = kof(st);
-        const bool cut = CUT && k0 + KS > K;
+        const int k0 = fetched(kof(st));
+        const bool cut = TAIL && KS == 128 && k0 + KS > K;
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
             const uint32_t dst = (uint32_t)(slot * STAGE + (j * F::kWaves + wave) * 1024);
             const uint16_t* g = src[j] + k0;
-            if (cut) g -= KS == 64 ? 64u : ((upper >> j) & 1u) * 64u;
+            if (cut) g -= ((upper >> j) & 1u) * 64u;
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(dst) : "memory");
         }
     };
 
-    float16_t acc[NH][RT];
+    constexpr int CT = F::kColTiles;
+    float16_t acc[NH][CT];
 #pragma unroll
     for (int h = 0; h < NH; ++h)
 #pragma unroll
-        for (int j = 0; j < RT; ++j)
+        for (int j = 0; j < CT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[h][j][e] = 0.0f;
-    // wave w: 32-row tile w % row tiles, k part w / row tiles of the stage; lane l of an operand: row l % 32, chunk 2 ks + l / 32
-    const int wr = wave % F::kRowTiles, kp = wave / F::kRowTiles;
+    // wave: quarter of the stage, column group; lane l of an operand: row l % 32, chunk 2 ks + l / 32 of the quarter.
+    // (An odd number of column tiles: the second group's last is its neighbour's again, and not written.)
+    const int qi = wave % F::kQuarters, cg = wave / F::kQuarters;
     const int lr = lane & 31;
-    int foff[2];
+    int foff[4], coff[CT];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) foff[ks] = lr * RB + (((kp * 4 + ks * 2 + (lane >> 5)) ^ swz(lr)) * 16);
-    auto multiply = [&](int slot, int k0, float16_t (&sums)[RT]) {
-        const bool out = CUT && k0 + kp * 32 >= K;              // a select, not a branch: product and encoder stay interleaved
+    for (int ks = 0; ks < 4; ++ks) foff[ks] = lr * RB + (((qi * 8 + ks * 2 + (lane >> 5)) ^ swz(lr)) * 16);
+#pragma unroll
+    for (int j = 0; j < CT; ++j) coff[j] = (NT_ROWS + min(cg * CT + j, RT - 1) * 32) * RB;
+    auto multiply = [&](int slot, int k0, float16_t (&sums)[CT]) {
+        const bool out = TAIL && k0 + qi * 64 >= K;             // a select, not a branch: product and encoder stay interleaved
         const unsigned char* b = lds + slot * STAGE;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            bf16x8_t fa = *reinterpret_cast<const bf16x8_t*>(b + wr * 32 * RB + foff[ks]);
+        for (int ks = 0; ks < 4; ++ks) {
+            bf16x8_t fa = *reinterpret_cast<const bf16x8_t*>(b + foff[ks]);
             if (out) fa = bf16x8_t{};
 #pragma unroll
-            for (int j = 0; j < RT; ++j) {
-                bf16x8_t fb = *reinterpret_cast<const bf16x8_t*>(b + (ROWS + j * 32) * RB + foff[ks]);
+            for (int j = 0; j < CT; ++j) {
+                bf16x8_t fb = *reinterpret_cast<const bf16x8_t*>(b + coff[j] + foff[ks]);
                 if (out) fb = bf16x8_t{};
                 sums[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb, fa, sums[j], 0, 0, 0);
             }
@@ -178,7 +188,7 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
     auto encode = [&](int slot, int k0) {
         if constexpr (QMODE >= 0) {
             const unsigned char* b = lds + slot * STAGE + erow * RB;
-            const int blk = (CUT && k0 + eblk * kBlock >= K) ? eblk - 4 : eblk;
+            const int blk = (TAIL && k0 + eblk * kBlock >= K) ? eblk - 4 : eblk;
             const uint4 c0 = *reinterpret_cast<const uint4*>(b + ((2 * blk) ^ eswz) * 16);
             const uint4 c1 = *reinterpret_cast<const uint4*>(b + ((2 * blk + 1) ^ eswz) * 16);
             float val[kBlock];
@@ -211,37 +221,40 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
             if (st + NS - 1 < steps) issue(slot == 0 ? NS - 1 : slot - 1, st + NS - 1);
             const int k0 = kof(st);
             multiply(slot, k0, acc[h]);
-            encode(slot, k0);
+            encode(slot, fetched(k0));
             slot = slot + 1 == NS ? 0 : slot + 1;
         }
     }
-    if constexpr (NH * RT > 12) {                               // R = 256: 256 sums per lane, left in the accumulation registers until they are read
+    if constexpr (NH * CT > 12) {                               // R = 256: 256 sums per lane, left in the accumulation registers until they are read
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
-            for (int j = 0; j < RT; ++j) asm volatile("" : "+a"(acc[h][j]));
+            for (int j = 0; j < CT; ++j) asm volatile("" : "+a"(acc[h][j]));
     }
     __syncthreads();                                            // the ring is free
-    float* red = reinterpret_cast<float*>(lds);                 // [half][part - 1][row tile][j][e][lane], then the waves' maxima
-    auto red_at = [&](int h, int p, int j, int e) -> float& { return red[((((h * (F::kParts - 1) + p) * F::kRowTiles + wr) * RT + j) * 16 + e) * 64 + lane]; };
+    float* red = reinterpret_cast<float*>(lds);                 // [stage of the step][column tile][e][lane], then the waves' maxima
+    auto red_at = [&](int h, int jt, int e) -> float& { return red[((h * RT + jt) * 16 + e) * 64 + lane]; };
+    constexpr int MAXIMA = F::kStages * (F::kQuarters - 1) * RT * 1024;
     if constexpr (QMODE >= 0) {
-        float* smax = red + F::kHalves * (F::kParts - 1) * F::kRowTiles * RT * 1024;
+        float* smax = red + MAXIMA;
         const float wm = wave_max(gmax);
         if (lane == 0) smax[wave] = wm;
     }
-    // acc[j][e] of lane l: row m0 + 32 wr + l % 32, column 32 j + 8 (e / 4) + 4 (l / 32) + e % 4.  The other parts of
-    // every stage's k join the first in LDS, in ascending order.
-    if (kp > 0) {
+    // acc[h][j][e] of lane l: row m0 + l % 32, column 32 (cg CT + j) + 8 (e / 4) + 4 (l / 32) + e % 4.  The odd quarters
+    // join the even ones in LDS.
+    if (qi > 0) {
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
-            for (int j = 0; j < RT; ++j)
+            for (int j = 0; j < CT; ++j)
+                if (cg * CT + j < RT) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) red_at(h, kp - 1, j, e) = acc[h][j][e];
+                    for (int e = 0; e < 16; ++e) red_at(h, cg * CT + j, e) = acc[h][j][e];
+                }
     }
     __syncthreads();
     if constexpr (QMODE >= 0) {
-        const float* smax = red + F::kHalves * (F::kParts - 1) * F::kRowTiles * RT * 1024;
+        const float* smax = red + MAXIMA;
         const uint32_t gid = blockIdx.y * gridDim.x + blockIdx.x, gsize = gridDim.x * gridDim.y;
         if (tid == 0) {
             float wm = smax[0];
@@ -251,14 +264,16 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
         }
         for (uint32_t j = gsize + gid * F::kThreads + tid; j < fill_to; j += gsize * F::kThreads) q_gmax[j] = 0u;
     }
-    const int m = m0 + wr * 32 + lr;
-    if (kp > 0 || m >= M) return;
+    const int m = m0 + lr;
+    if (qi > 0 || m >= M) return;
 #pragma unroll
-    for (int j = 0; j < RT; ++j) {
-        const uint16_t* sj = t && !part ? nt_s(fac, col0 + j * 32) : nullptr;      // the 32 columns belong to one member
+    for (int j = 0; j < CT; ++j) {
+        const int jt = cg * CT + j;
+        if (jt >= RT) break;
+        const uint16_t* sj = t && !part ? nt_s(fac, col0 + jt * 32) : nullptr;     // the 32 columns belong to one member
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int col = col0 + j * 32 + 8 * g + 4 * (lane >> 5);
+            const int col = col0 + jt * 32 + 8 * g + 4 * (lane >> 5);
             float sum[4];
             uint32_t h[4], ts[4];
 #pragma unroll
@@ -267,8 +282,7 @@ __global__ __launch_bounds__(ROWS * KS / 16) void lowrank_nt_kernel(
 #pragma unroll
                 for (int h = 0; h < NH; ++h) {
                     if (h) sum[e] += acc[h][j][4 * g + e];
-#pragma unroll
-                    for (int p = 0; p + 1 < F::kParts; ++p) sum[e] += red_at(h, p, j, 4 * g + e);
+                    if constexpr (F::kQuarters > 1) sum[e] += red_at(h, jt, 4 * g + e);
                 }
             }
             if (part) {                                         // one of several slices: the finishing kernel rounds
@@ -308,13 +322,13 @@ __global__ __launch_bounds__(256) void lowrank_nt_finish_kernel(const float* __r
     }
 }
 
-// K slices for M rows: none when 32-row tiles give every compute unit a workgroup; otherwise about two such tiles per compute
-// unit, at least 1024 k per slice, and never more workgroups than the quantizer's partial maxima have room for.
+// K slices for M rows: none when 32-row tiles give every compute unit a workgroup; otherwise two such tiles per compute unit or a few
+// more, at least 1024 k per slice, and never more workgroups than the quantizer's partial maxima have room for.
 static int nt_slices(int64_t M, int64_t K, size_t workspace_bytes, int64_t R)
 {
     const int64_t tiles = (M + 31) / 32, steps = (K + 255) / 256, cus = device_cus();
     if (tiles >= cus) return 1;
-    int64_t sl = 2 * cus / tiles;                               // (one more round of workgroups for a few of them costs a third: 2103 x 18944 28 -> 26 us)
+    int64_t sl = (2 * cus + tiles - 1) / tiles;
     if (sl > steps / 4) sl = steps / 4;
     if (sl * tiles > (int64_t)kDeferredPartials) sl = (int64_t)kDeferredPartials / tiles;
     if (sl > 16) sl = 16;
@@ -329,33 +343,33 @@ size_t lowrank_nt_workspace_bytes(int64_t M, int64_t R, int64_t K)
     return sl > 1 ? (size_t)sl * M * R * 4 : 0;
 }
 
-// Columns per workgroup of the 32-row form without the quantizer, for `groups` workgroups per column range.  Where these leave
-// compute units idle, the time is that of one workgroup's stages, and a stage of R columns takes the longer the more of v it
-// fetches and multiplies (and the wide forms' rings hold only two of them): workgroups of 32 or 64 columns side by side (gridDim.z)
-// read x again from L2 and finish sooner, with the same bits.  Microseconds at 32 | 64 | all R columns:
-//   411 x 1536, R = 192 (13 groups)    6.2 | 9.1 | 20.3         2103 x 1536, R = 128 (66)    7.8 | 9.4 | 15.1
-//   800 x 3584, R = 128 (75)           8.8 | 8.9 | 11.3         1500 x 3584, R = 192 (141)  17.0 | 12.8 | 15.7
-//   1500 x 3584, R = 64 (141)          8.2 |  -  | 8.8          4096 x 3584, R = 192 (384)  24.8 | 23.7 | 29.0
-//   2103 x 3584, R = 64 (198)          9.4 |  -  | 9.1          800 x 18944, R = 256 (400)  51.5 | 41.5 | 51.4
-//   4096 x 1536, R = 96 (128)          7.8 |  -  | 12.2         1500 x 18944, R = 128 (470) 45.8 | 32.0 | 29.7
-//   2103 x 3584, R = 96 (198)         13.6 |  -  | 10.9         8000 x 18944, R = 128 (500)  213 | 144  | 112
-// 32 columns up to about a workgroup per compute unit (a rank that has no half of 64 columns: up to 7/4), 64 up to 8/5 row groups.
+// Columns per workgroup without the quantizer, for `groups` workgroups per column range.  Where these leave compute units
+// idle, the time is that of one workgroup's stages, and a stage of R columns takes the longer the more of v it fetches and
+// multiplies (and the wide forms' rings hold only two of them): workgroups of 32 or 64 columns side by side (gridDim.z) read x
+// again from L2 and finish sooner, with the same bits.  Microseconds at 32 | 64 | all R columns:
+//   411 x 1536, R = 192 (13 groups)    7.2 | 8.5 | 17.7         1024 x 3584, R = 192 (96)   11.4 | 10.4 | 14.8
+//   2103 x 1536, R = 128 (66)          9.2 | 8.7 | 13.6         1500 x 3584, R = 192 (141)  18.5 | 14.4 | 15.8
+//   800 x 3584, R = 128 (75)          10.0 | 9.3 | 12.1         8192 x 4096, R = 192 (256)  53.3 | 37.5 | 40.1
+//   4096 x 1536, R = 96 (128)          8.8 |  -  | 11.9         1500 x 8960, R = 128 (376)  22.6 | 20.8 | 18.3
+//   2103 x 3584, R = 96 (198)         15.0 |  -  | 11.9         800 x 18944, R = 256 (400)  47.0 | 38.2 | 31.1
+//   2103 x 3584, R = 64 (198)         10.5 |  -  | 9.6          4096 x 8960, R = 128 (512)  48.9 | 32.6 | 25.6
+// 32 columns up to about a workgroup per compute unit (a rank that has no half of 64 columns: up to 7/4), 64 up to one row group each.
 static int nt_column_group(int64_t groups, int64_t R)
 {
     const int64_t cus = device_cus();
     if (groups * (R / 32) * 8 <= cus * (R % 64 ? 14 : 9)) return 32;
-    return R % 64 == 0 && groups * 5 <= cus * 8 ? 64 : (int)R;
+    return R % 64 == 0 && groups <= cus ? 64 : (int)R;
 }
 
-template <int RT, int QMODE, int ROWS, int KS, int NS, bool CUT>
+template <int RT, int QMODE, int KS, int NS, bool TAIL>
 static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, const NtFactors& fac, void* xv, void* t, int64_t M, int64_t R, int64_t K,
                      float* part, void* codes, uint16_t* amax, uint32_t* gmax)
 {
-    using F = NtForm<RT, ROWS, KS, NS>;
+    using F = NtForm<RT, KS, NS>;
     static bool attr_set[64] = {};
-    if (const int rc = allow_dynamic_lds((const void*)lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>, F::kLds, attr_set)) return rc;
-    hipLaunchKernelGGL((lowrank_nt_kernel<RT, QMODE, ROWS, KS, NS, CUT>), dim3((unsigned)((M + ROWS - 1) / ROWS), (unsigned)slices, (unsigned)(R / (RT * 32))), dim3(F::kThreads), F::kLds, st,
-                       (const uint16_t*)x, ldx, fac, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part, (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 13), (int)R);
+    if (const int rc = allow_dynamic_lds((const void*)lowrank_nt_kernel<RT, QMODE, KS, NS, TAIL>, F::kLds, attr_set)) return rc;
+    hipLaunchKernelGGL((lowrank_nt_kernel<RT, QMODE, KS, NS, TAIL>), dim3((unsigned)((M + NT_ROWS - 1) / NT_ROWS), (unsigned)slices, (unsigned)(R / (RT * 32))), dim3(F::kThreads), F::kLds, st,
+                       (const uint16_t*)x, ldx, fac, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part, (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 5), (int)R);
     return METIS_OK;
 }
 
@@ -407,37 +421,34 @@ int lowrank_nt_grouped(const void* x, int64_t ldx, int64_t M, int64_t K, const L
     const int slices = workspace ? nt_slices(M, K, workspace_bytes, R) : 1;
     float* part = slices > 1 ? static_cast<float*>(workspace) : nullptr;
     int rc = METIS_OK;
-    // 64-row tiles read v half as often, but only where they still give every compute unit a workgroup; stages of 128 k
-    // leave whole 64-byte pieces of codes (with 64 k the quantizing form takes 338 us in place of 229 below).  Microseconds,
-    // 64 rows | 32 rows:
-    //   16384 x 3584, R = 64    28 | 33                 8192 x 4096, R = 64    18.5 | 15.7
-    //   16384 x 18944, R = 64, quantized  229 | 270     8192 x 14336, R = 64   76 | 60
-    //   16384 x 3584, R = 192 (64 k | 128 k)  50 | 81   1024 x 3584, R = 192   17.1 | 16.2
-    const bool tall = ((M + 63) / 64) * slices >= device_cus(), cut = K % 128 != 0;
-#define METIS_NT(RT, Q, ROWS, KS, NS, CUT) rc = launch_nt<RT, Q, ROWS, KS, NS, CUT>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax)
-#define METIS_NT128(RT, Q, ROWS, NS) do { if (cut) METIS_NT(RT, Q, ROWS, 128, NS, true); else METIS_NT(RT, Q, ROWS, 128, NS, false); } while (0)
-#define METIS_NTF(RT, Q) do { if (tall) METIS_NT128(RT, Q, 64, 3); else METIS_NT128(RT, Q, 32, 3); } while (0)
-#define METIS_NTG(RT, NT, NW) do { if (!tall) METIS_NT128(RT, -1, 32, NW); else if (cut) METIS_NT(RT, -1, 64, 64, NT, true); else METIS_NT(RT, -1, 64, 64, NT, false); } while (0)
-    const int width = (qmode < 0 && !tall) ? nt_column_group(((M + 31) / 32) * slices, R) : (int)R;
-    if (width == 32 && R > 32) METIS_NT128(1, -1, 32, 3);
-    else if (width == 64 && R > 64) METIS_NT128(2, -1, 32, 3);
-    else if (qmode < 0) {
-        if (R == 32) METIS_NTF(1, -1);
-        else if (R == 64) METIS_NTF(2, -1);
-        else if (R == 96) METIS_NTG(3, 4, 3);
-        else if (R == 128) METIS_NTG(4, 4, 3);
-        else if (R == 192) METIS_NTG(6, 4, 2);
-        else METIS_NTG(8, 3, 2);
-    } else if (qmode == METIS_MODE_P32) {
-        if (R == 32) METIS_NTF(1, 0);
-        else METIS_NTF(2, 0);
-    } else {
-        if (R == 32) METIS_NTF(1, 1);
-        else METIS_NTF(2, 1);
-    }
-#undef METIS_NTG
-#undef METIS_NTF
-#undef METIS_NT128
+    // Stages of 128 k, three in the ring (two with the quantizer, whose vector work wants more workgroups per compute unit, and where
+    // V is wide).  From 96 columns on and with more than one workgroup for a compute unit, stages of 64 k, so that two fit beside
+    // each other.  Microseconds, 128 k | 64 k:
+    //   R = 96   4096 x 8960 28 | 22, 16384 x 3584 37 | 30, 8192 x 4096 (one workgroup each) 21.7 | 27
+    //   R = 128  4096 x 8960 33 | 25, 16384 x 3584 44 | 34, 8192 x 4096 25 | 28
+    //   R = 192  4096 x 8960 44 | 36, 16384 x 3584 62 | 48, 8192 x 4096 40 | 47;   R = 256  54 | 48, 75 | 59, 47 | 54
+    // An x of more than the memory-side cache wants its rows in longer pieces: 8000 x 18944, R = 128 114 | 138, R = 96 99 | 107; from
+    // 192 columns on V's share outweighs that (16384 x 18944 433 | 361).
+    //   with the quantizer, R = 64, three | two stages of 128 k: 411 x 1536 12.8 | 11.7, 16384 x 3584 33.4 | 31.7; three where a compute
+    //   unit has one workgroup and x comes from HBM: 8192 x 14336 91 | 105
+    const int64_t groups = ((M + NT_ROWS - 1) / NT_ROWS) * slices;
+    const bool tail = K % 256 != 0, shared = groups > device_cus() && (R > 128 || M * K <= (int64_t)1 << 27);
+#define METIS_NT(RT, Q, KS, NS) do { if (tail) rc = launch_nt<RT, Q, KS, NS, true>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); \
+                                     else rc = launch_nt<RT, Q, KS, NS, false>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); } while (0)
+#define METIS_NTS(RT, NS, NS64) do { if (shared) METIS_NT(RT, -1, 64, NS64); else METIS_NT(RT, -1, 128, NS); } while (0)
+    const int width = qmode < 0 ? nt_column_group(groups, R) : (int)R;
+    const bool deep = groups <= device_cus() && M * K >= 100000000;
+#define METIS_NTQ(RT, Q) do { if (deep) METIS_NT(RT, Q, 128, 3); else METIS_NT(RT, Q, 128, 2); } while (0)
+    if (qmode == METIS_MODE_P32) { if (R == 32) METIS_NTQ(1, 0); else METIS_NTQ(2, 0); }
+    else if (qmode >= 0) { if (R == 32) METIS_NTQ(1, 1); else METIS_NTQ(2, 1); }
+    else if (width == 32) METIS_NT(1, -1, 128, 3);
+    else if (width == 64) METIS_NT(2, -1, 128, 3);
+    else if (width == 96) METIS_NTS(3, 3, 4);
+    else if (width == 128) METIS_NTS(4, 3, 4);
+    else if (width == 192) METIS_NTS(6, 2, 2);
+    else METIS_NTS(8, 2, 2);
+#undef METIS_NTS
+#undef METIS_NTQ
 #undef METIS_NT
     if (rc) return rc;
     if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;

@@ -1317,9 +1317,9 @@ def _one_pass_takes(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None) -
     """A projection of 256 rows or more runs on the one-pass kernel: ranks 32, 64 and 128 always; 96, 192 and 256, which have few
     stages of the wide tile in flight and fetch all of V again for every row tile, up to a bound on the work.  Microseconds,
     kernel | library product and its multiplication by s:
-        R = 96   8000 x 8960 40.8 | 43.1, 16384 x 8960 67.8 | 66.3, 16384 x 18944 167 | 139
-        R = 192  800 x 18944 35 | 72, 4096 x 3584 23.9 | 27.3, 8000 x 1536 22.2 | 24.3, 2103 x 8960 33.5 | 29.5, 16384 x 18944 328 | 215
-        R = 256  800 x 18944 42 | 87, 2103 x 3584 20.6 | 24.7, 4096 x 3584 28.2 | 24.3, 8000 x 3584 44.6 | 36.8, 16384 x 18944 428 | 252
+        R = 96   4096 x 8960 22 | 35, 8000 x 3584 24 | 21, 16384 x 3584 30 | 28, 16384 x 8960 96 | 67, 16384 x 18944 200 | 144
+        R = 192  800 x 18944 35 | 72, 4096 x 3584 23 | 27, 8000 x 1536 22 | 24, 8000 x 3584 39 | 31, 16384 x 18944 359 | 215
+        R = 256  800 x 18944 38 | 87, 2103 x 3584 21 | 25, 4096 x 3584 28 | 24, 8000 x 3584 47 | 37, 16384 x 18944 469 | 252
     The library product also takes what the kernel does not read there (rows that overlap, an unaligned V) and what autograd records."""
     R = v.shape[0]
     if R in (32, 64, 128):
@@ -1327,7 +1327,7 @@ def _one_pass_takes(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor | None) -
     if R not in ONE_PASS_RANKS:
         return False
     M, K = x2.shape
-    return ((M <= 1024 or M * K * R <= (10 ** 10 if R == 96 else 3 * 10 ** 9)) and x2.stride(0) >= K and (v.data_ptr() % 16 == 0 or not v.is_contiguous())
+    return ((M <= 1024 or M * K * R <= (5 * 10 ** 9 if R == 96 else 3 * 10 ** 9)) and x2.stride(0) >= K and (v.data_ptr() % 16 == 0 or not v.is_contiguous())
             and not (torch.is_grad_enabled() and (x2.requires_grad or v.requires_grad or (s is not None and s.requires_grad))))
 
 

@@ -756,6 +756,42 @@ def test_rank_r_columns_have_the_same_bits_at_every_width(M, R, K):
         assert torch.equal(a, one) and torch.equal(b, ts)
 
 
+@pytest.mark.parametrize("M,K", [(300, 1792), (257, 1856), (411, 1984), (1030, 1536), (300, 4096), (2103, 8960), (4096, 4160)])
+def test_rank_r_projection_adds_in_its_documented_order(M, K):
+    """One product per quarter of 64 in every step of 256, of 1, 2^24 and -2^24, so that the order of the binary32 sums decides the
+    result: the quarters in sums of their own, the steps from (5 x row tile) mod steps on, the quarters added in order, then the
+    slices of K in order -- for every rank and with the quantizer."""
+    from metis_hip import ops
+    g = torch.Generator().manual_seed(M + K)
+    steps = (K + 255) // 256
+    pick = torch.tensor([0.0, 1.0, 1.0, 2.0 ** 24, -2.0 ** 24])[torch.randint(5, (M, steps * 4), generator=g)]
+    pick[:, K // 64:] = 0.0
+    x = torch.zeros(M, K)
+    at = torch.arange(K // 64) * 64 + torch.randint(64, (K // 64,), generator=g)
+    x[:, at] = pick[:, :K // 64]
+    cus, tiles = torch.cuda.get_device_properties(0).multi_processor_count, (M + 31) // 32
+    slices = 1 if tiles >= cus else max(1, min((2 * cus + tiles - 1) // tiles, steps // 4, 16))
+    per = (steps + slices - 1) // slices
+    q = pick.view(M, steps, 4)
+    total = torch.zeros(M)
+    for y in range(slices):
+        s0, n = y * per, max(0, min(steps, y * per + per) - y * per)
+        sums = torch.zeros(M, 4)
+        for i in range(n):
+            step = s0 + (torch.arange(M) // 32 * 5 + i) % n
+            sums = sums + q[torch.arange(M), step]
+        part = ((sums[:, 0] + sums[:, 1]) + sums[:, 2]) + sums[:, 3]
+        total = part if y == 0 else total + part
+    want = total.bfloat16().cuda()[:, None]
+    xd = x.bfloat16().cuda()
+    for R in (32, 64, 96, 128):
+        v, s = torch.ones(R, K, device="cuda").bfloat16(), torch.ones(R, device="cuda").bfloat16()
+        xv, t = ops.lowrank_project(xd, v, s)
+        assert torch.equal(xv, want.expand(M, R)) and torch.equal(t, xv)
+        if R <= 64:
+            assert torch.equal(ops.quantize_project(xd, v, s, 0)[1], xv)
+
+
 @pytest.mark.parametrize("R", [96, 192, 256])
 def test_wide_ranks_take_what_the_library_product_took(R):
     """Ranks 96, 192 and 256 from 256 rows on: an unaligned V, rows that overlap, operands that autograd records and large products
