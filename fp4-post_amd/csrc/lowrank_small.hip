@@ -1,6 +1,6 @@
 // Rank-r projection for decode-sized batches:  xv[M, R] = x[M, K] . v[R, K]^T  (bf16 operands and result, binary32
-// accumulation), t = bf16(xv * s) -- `vlinear(x)` and `torch.mul(self.s, y)` of BitLinear.forward with the bf16 V of
-// the north-star formula (src/Metis/Metis/bitlinear.py:752-756), for M < 256.
+// accumulation), t = bf16(xv * s) -- `vlinear(x)` and `torch.mul(self.s, y)` of BitLinear.forward with V in
+// bf16 (src/Metis/Metis/bitlinear.py:752-756), for M < 256.
 //
 // The output is tiny (M x R) and the contraction long (K up to 18944): the vendor library runs such a product as one
 // or a few workgroups walking all of K (35 us at 64 x 64 x 18944).  Here K is cut into up to 128 chunks of one to three

@@ -519,7 +519,7 @@ int metis_linear_wgrad_ws(const void *dyt_codes, const void *dyt_scales, const f
  * Rank-r projection of the low-rank branch for decode-sized batches (M < 256):
  *     xv[M, R] = x[M, K] . v[R, K]^T   bf16 operands and result, binary32 accumulation
  *     t [M, R] = bf16(xv * s[R])       when t != NULL
- * `vlinear(x)` and `torch.mul(self.s, y)` of BitLinear.forward with the bf16 V of the north-star formula
+ * `vlinear(x)` and `torch.mul(self.s, y)` of BitLinear.forward with V in bf16
  * (src/Metis/Metis/bitlinear.py:752-756).  The contraction is cut into up to 32 chunks that run as separate
  * workgroups (the vendor library walks all of K in one or a few workgroups: 35 us at 64 x 64 x 18944) and a second
  * kernel adds the chunks in order.  Larger batches are served well by the vendor library.

@@ -236,7 +236,7 @@ def metis_forward(x: torch.Tensor, v: torch.Tensor, s: torch.Tensor, u: torch.Te
     y = ulinear(s * vlinear(x)) + warmup_linear(x)
       = ((x . v^T) * s) . u^T  +  QDQ(x) . QDQ(w_res)^T + bias
     x [M,K] bf16, v [r,K], s [r], u [N,r], w_res [N,K] (all bf16).
-    Default (north-star) variant: the low-rank operands are bf16 -- t = bf16(bf16(x . v^T) * s) is
+    Default variant: the low-rank operands are bf16 -- t = bf16(bf16(x . v^T) * s) is
     the stored rank-r activation -- and both branches are ACCUMULATED IN FP32 and summed before
     the single rounding of the output to bf16.  With ``quantized_lowrank`` the rank-r branch
     consumes QDQ(x) and QDQ(v) in dtype D as the current reference file does
