@@ -322,6 +322,23 @@ __global__ __launch_bounds__(256) void rmsnorm_colsum_rows_kernel(const uint4* _
     for (uint32_t q = threadIdx.x; q < cpr * 2u; q += 256u) out[q] = sums[q >> 1][q & 1u];
 }
 
+// 1 / sqrt(ss / n + eps) as hi + lo: the remainders of the quotient, of the sum and of the root enter one Newton step.  With each
+// operation rounded, and a row's squares in one chain, bf16(x rstd) was the neighbouring value more often than in the formula that
+// autograd records, and the sums down the columns were off with it: 4096 x 3584, the binary32 gradient of gamma to double
+// precision 1.44e-5, the formula's 1.23e-5, now 0.91e-5.  The kernel takes no longer for it.  (Sums that are zero or infinite have
+// no remainders: the plain value.)
+struct Rstd { float hi, lo; };
+__device__ __forceinline__ Rstd rsqrt_mean(float ss, float n, float eps)
+{
+    const float q = ss / n, v = q + eps, b = v - q;
+    const float rest = ((q - (v - b)) + (eps - b)) + fmaf(-q, n, ss) / n;      // ss / n + eps = v + rest
+    const float y = 1.0f / sqrtf(v), h = v * y;
+    const float e = fmaf(-h, y, 1.0f) - (fmaf(v, y, -h) + rest * y) * y;       // 1 - (v + rest) y^2
+    const float step = 0.5f * y * e, hi = y + step;
+    if (!(fabsf(step) < y)) return {y, 0.0f};
+    return {hi, step - (hi - y)};
+}
+
 // ---------------------------------------------------------------------------------------------
 // Backward of the norm: one pass over x and the output gradient g instead of a chain of fifteen elementwise and reduction
 // kernels over binary32 copies.  In binary32, with xh = x * rstd:
@@ -368,14 +385,17 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_backward_rows_kernel(const uin
             const uint32_t xw[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w}, gw[4] = {gr[i].x, gr[i].y, gr[i].z, gr[i].w};
             const uint4 m = gm[i * 64 + lane];
             const uint32_t mw[4] = {m.x, m.y, m.z, m.w};
+            float ss8 = 0.0f, dot8 = 0.0f;                     // a chunk's own: the chunks' sums are added as they are
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float x0 = bf16_lo(xw[j]), x1 = bf16_hi(xw[j]);
-                ss = fmaf(x0, x0, ss);
-                ss = fmaf(x1, x1, ss);
-                dot = fmaf(bf16_lo(gw[j]) * bf16_lo(mw[j]), x0, dot);
-                dot = fmaf(bf16_hi(gw[j]) * bf16_hi(mw[j]), x1, dot);
+                ss8 = fmaf(x0, x0, ss8);
+                ss8 = fmaf(x1, x1, ss8);
+                dot8 = fmaf(bf16_lo(gw[j]) * bf16_lo(mw[j]), x0, dot8);
+                dot8 = fmaf(bf16_hi(gw[j]) * bf16_hi(mw[j]), x1, dot8);
             }
+            ss += ss8;
+            dot += dot8;
         }
         // the row stays packed: without this the compiler keeps every unpacked value alive to the second loop (256 registers, spills)
 #pragma unroll
@@ -383,7 +403,8 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_backward_rows_kernel(const uin
             asm volatile("" : "+v"(xr[i].x), "+v"(xr[i].y), "+v"(xr[i].z), "+v"(xr[i].w), "+v"(gr[i].x), "+v"(gr[i].y), "+v"(gr[i].z), "+v"(gr[i].w));
         ss = wave_sum_dpp(ss);
         dot = wave_sum_dpp(dot);
-        const float rstd = 1.0f / sqrtf(ss / fcols + eps);
+        const Rstd rs = rsqrt_mean(ss, fcols, eps);
+        const float rstd = rs.hi;
         const float mean = dot * rstd / fcols;                 // mean over the row of g gamma xh
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
@@ -395,7 +416,8 @@ __global__ __launch_bounds__(256, 2) void rmsnorm_backward_rows_kernel(const uin
             uint32_t w[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float h0 = bf16_lo(xw[j]) * rstd, h1 = bf16_hi(xw[j]) * rstd;
+                const float x0 = bf16_lo(xw[j]), x1 = bf16_hi(xw[j]);
+                const float h0 = fmaf(x0, rstd, x0 * rs.lo), h1 = fmaf(x1, rstd, x1 * rs.lo);
                 const float g0 = bf16_lo(gw[j]), g1 = bf16_hi(gw[j]);
                 if constexpr (SUMS) {
                     const uint32_t hb = rb_pair(h0, h1);

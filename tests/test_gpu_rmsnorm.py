@@ -115,3 +115,37 @@ def test_rmsnorm_backward(rows, cols):
     assert torch.equal(again[0], gx) and torch.equal(again[1], gg)
     only, none = ops.rmsnorm_backward(x, g, gamma, eps, want_gamma=False)
     assert none is None and torch.equal(only, gx)
+
+
+def test_rmsnorm_backward_gamma_precision():
+    """The binary32 gradient of gamma is no further from double precision than the formula that autograd records with create_graph.
+    Its terms hold bf16(x rstd), which is the neighbouring bf16 value where the error of rstd puts x rstd on the other side of a
+    midpoint: with rstd to twice binary32 from a sum of squares in binary32, in fewer elements than with rstd rounded."""
+    from metis_hip import ops
+    from metis_hip._lib import DTYPE_F32, load
+    rows, cols, eps = 4096, 3584, 1e-6
+    gamma = torch.ones(cols, dtype=torch.bfloat16, device="cuda")
+    gx = torch.empty(rows, cols, dtype=torch.bfloat16, device="cuda")
+    gg = torch.empty(cols, dtype=torch.float32, device="cuda")
+    L = load()
+    ws = torch.empty(L.metis_rmsnorm_backward_workspace_bytes(rows, cols), dtype=torch.uint8, device="cuda")
+    squares = formula = 0.0
+    for seed in range(8):
+        gen = torch.Generator("cuda").manual_seed(seed)
+        x = torch.randn(rows, cols, device="cuda", generator=gen).bfloat16()
+        g = (torch.randn(rows, cols, device="cuda", generator=gen) * 1e-3).bfloat16()
+        rc = L.metis_rmsnorm_backward(x.data_ptr(), g.data_ptr(), gamma.data_ptr(), eps, rows, cols, gx.data_ptr(), gg.data_ptr(), DTYPE_F32,
+                                      ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        xd = x.double()
+        xh = xd * (xd.pow(2).mean(-1, keepdim=True) + eps).rsqrt()
+        want = (g.double() * xh.to(torch.bfloat16).double()).sum(0)
+        squares += float((gg.double() - want).norm() / want.norm()) ** 2
+        xf = x.float()
+        recorded = (g.float() * (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + eps)).to(torch.bfloat16).float()).double().sum(0)
+        formula += float((recorded - want).norm() / want.norm()) ** 2
+    assert squares <= formula
+    # rows without remainders: zeros (rstd = eps^-1/2), and squares beyond binary32 (rstd = 0)
+    one = torch.ones(4, 16, dtype=torch.bfloat16, device="cuda")
+    for value, want in ((0.0, 1000.0), (1e30, 0.0)):
+        assert torch.equal(ops.rmsnorm_backward(one * value, one, one[0], eps)[0], one * want)
