@@ -82,11 +82,11 @@ __global__ __launch_bounds__(256) void scale_grad_kernel(const uint16_t* __restr
     __shared__ __attribute__((aligned(16))) float part[8][256 + 4];
     const int c0 = blockIdx.x * 8, tid = threadIdx.x;
     float acc[8] = {};
-    for (int l0 = tid; l0 < L; l0 += 256 * BATCH) {
+    for (int64_t l0 = tid; l0 < L; l0 += 256 * BATCH) {          // (64-bit: a step past the last row)
         uint4 a[BATCH], b[BATCH];
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) {
-            const int64_t l = (int64_t)l0 + 256 * i;
+            const int64_t l = l0 + 256 * i;
             a[i] = b[i] = make_uint4(0u, 0u, 0u, 0u);             // (rows past the end add zeros)
             if (l < L) {
                 a[i] = *reinterpret_cast<const uint4*>(g + l * R + c0);
