@@ -142,14 +142,16 @@ __device__ __forceinline__ void encode_rne_p32_tbl(const float (&v)[N], float am
 // significand bits, so a quotient whose low 20 bits are within 4 of 0 (mod 2^20) sends the block to the literal
 // sequence: about 1e-4 of blocks.  Quotients below 0.125 encode as 0 and quotients above 5.5 as 7 either way and
 // are never flagged (zeros are common, and every block's maximum has a quotient just below 6).  Checked on the host against the literal sequence on 9e8 cases around every threshold.
-__device__ __forceinline__ uint2 encode_rne_wide(const float (&v)[kBlock], float s)
+// N elements of a block with scalar s (8: half a block, one packed word)
+template <int N>
+__device__ __forceinline__ void encode_rne_wide_n(const float (&v)[N], float s, uint32_t (&w)[N / 8])
 {
     const float rs = __builtin_amdgcn_rcpf(s);                // 1 ulp
-    // the quotients are converted as they are formed (nothing but the two packed words stays live); the rare
+    // the quotients are converted as they are formed (nothing but the packed words stays live); the rare
     // flagged block is redone literally afterwards
     // all in vector integer ops (no compares): magnitudes outside [0.125, 5.5] are clamped to patterns that never flag,
     // bits 3..19 of (pattern + 4) are zero exactly for a flagged quotient, and the minimum over the block is kept
-    uint32_t lo = 0u, hi = 0u, least = 0xffffffffu;
+    uint32_t least = 0xffffffffu;
     auto quot = [&](int j) {
         const float q = div3(v[j], s, rs);
         uint32_t a = __float_as_uint(q) & 0x7fffffffu;
@@ -159,22 +161,22 @@ __device__ __forceinline__ uint2 encode_rne_wide(const float (&v)[kBlock], float
         least = m < least ? m : least;
         return q;
     };
-    lo = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(lo, quot(0), quot(1), 1.0f, 0);
-    lo = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(lo, quot(2), quot(3), 1.0f, 1);
-    lo = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(lo, quot(4), quot(5), 1.0f, 2);
-    lo = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(lo, quot(6), quot(7), 1.0f, 3);
-    hi = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(hi, quot(8), quot(9), 1.0f, 0);
-    hi = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(hi, quot(10), quot(11), 1.0f, 1);
-    hi = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(hi, quot(12), quot(13), 1.0f, 2);
-    hi = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(hi, quot(14), quot(15), 1.0f, 3);
+#pragma unroll
+    for (int k = 0; k < N / 8; ++k) {
+        uint32_t c = 0u;
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, quot(8 * k), quot(8 * k + 1), 1.0f, 0);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, quot(8 * k + 2), quot(8 * k + 3), 1.0f, 1);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, quot(8 * k + 4), quot(8 * k + 5), 1.0f, 2);
+        c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, quot(8 * k + 6), quot(8 * k + 7), 1.0f, 3);
+        w[k] = c;
+    }
     const bool flagged = least == 0u;
     if (__builtin_amdgcn_ballot_w64(flagged) != 0ull) {        // wave-uniform: a real branch around the long sequence
         // Element by element: the literal rule only for the positions at which some lane of the wave holds a flagged
         // quotient (tensors with short mantissas flag a few quotients in most waves: redoing whole blocks cost 40 %).
         const float h = rd<0>(s / 2.0f);
-        uint32_t w[2] = {lo, hi};
 #pragma unroll
-        for (int j = 0; j < kBlock; ++j) {
+        for (int j = 0; j < N; ++j) {
             const float q = div3(v[j], s, rs);
             uint32_t a = __float_as_uint(q) & 0x7fffffffu;
             a = a < 0x3e000010u ? 0x3e000010u : a;
@@ -188,10 +190,13 @@ __device__ __forceinline__ uint2 encode_rne_wide(const float (&v)[kBlock], float
                 if (fj) w[j >> 3] = (w[j >> 3] & ~(0xFu << sh)) | (code << sh);
             }
         }
-        lo = w[0];
-        hi = w[1];
     }
-    return make_uint2(lo, hi);
+}
+__device__ __forceinline__ uint2 encode_rne_wide(const float (&v)[kBlock], float s)
+{
+    uint32_t w[2];
+    encode_rne_wide_n<kBlock>(v, s, w);
+    return make_uint2(w[0], w[1]);
 }
 
 // Round-to-nearest, every op rounded to bf16.  With q = bf16(RN(|x| / h)) the reference's
@@ -446,6 +451,9 @@ __device__ __forceinline__ float fold_partial_maxima(const uint32_t* __restrict_
     __syncthreads();
     return fmaxf(fmaxf(fmax_s[0], fmax_s[1]), fmaxf(fmax_s[2], fmax_s[3]));
 }
+// (binary32 values that need not be bf16 values: IEEE divisions)
+__device__ __forceinline__ float block_scalar_ieee(float amax) { return amax / 6.0f + 1e-9f; }
+__device__ __forceinline__ float amax_unit_ieee(float amax) { return block_scalar_ieee(amax) / 448.0f; }
 template <int MODE>
 __device__ __forceinline__ float tensor_unit_of(float amax) { return rd<MODE>(block_scalar<MODE>(amax) / 448.0f); }
 template <int MODE>

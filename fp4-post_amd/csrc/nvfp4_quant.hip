@@ -33,8 +33,6 @@ namespace metis {
 // center (optional): one value per column, subtracted before anything else: x - center rounded to the
 // arithmetic's dtype, the centred residual of the reference's mean mode (src/Metis/Metis/bitlinear.py:
 // 330-333).  binary32 [cols] in binary32 arithmetic (always WIDE then), bf16 [cols] in bf16 arithmetic.
-__device__ __forceinline__ float block_scalar_ieee(float amax) { return amax / 6.0f + 1e-9f; }
-
 // Round-to-nearest rows of a contiguous bf16 tensor, the shape every activation and weight has: a kernel of its own
 // so that its loop carries no row/column arithmetic at all.  Software-pipelined: the next DEPTH blocks' bytes are in
 // flight while the current block is encoded.  Binary32 arithmetic takes the two-operation quotient for every block

@@ -141,17 +141,18 @@ class _NVFP4Base(BlockQuantFunc):
         return cls.pack(x, arith=arith, **more), cls.pack(x, col=True, arith=arith, **more)
 
     @classmethod
-    @torch.no_grad()
     def quantize_dequantize(cls, x: torch.Tensor):
         """Fused QDQ (quant.py:6-36 / 392-433): same shape and dtype as x."""
         cls._check(x)
-        if not cls.stochastic and x.is_cuda and x.dtype == torch.bfloat16 and x.numel():
-            # one call: the second launch forms scale bytes and dequantized values together
-            return ops.quantize_dequantize(x, _mode_of(x))[1].reshape(x.shape)
-        if not cls.stochastic and x.is_cuda and x.dtype == torch.float32 and x.numel() and x.data_ptr() % 16 == 0:
-            return ops.quantize_dequantize_f32(x)[1].reshape(x.shape)
-        p = cls.pack(x)
-        return ops.dequantize(p, x.dtype).reshape(x.shape)
+        if torch.is_grad_enabled():
+            x = x.detach()
+        if not cls.stochastic and x.is_cuda and x.numel():
+            if x.dtype == torch.bfloat16:
+                # values only, nothing packed on the way; large: one call whose second launch forms scale bytes and values together
+                return ops.roundtrip(x) if ops.roundtrip_pays(x) else ops.quantize_dequantize(x, _mode_of(x))[1].reshape(x.shape)
+            if x.dtype == torch.float32 and x.data_ptr() % 16 == 0:
+                return ops.roundtrip(x) if ops.roundtrip_pays(x) else ops.quantize_dequantize_f32(x)[1].reshape(x.shape)
+        return ops.dequantize(cls.pack(x), x.dtype).reshape(x.shape)
 
     @classmethod
     @torch.no_grad()

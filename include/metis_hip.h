@@ -100,6 +100,16 @@ int metis_nvfp4_quant_dequant_row_f32(const void *x, int64_t rows, int64_t cols,
                                       float *unit, void *out, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * The dequantized values of that round trip alone: no codes, scale bytes or unit are written.  x is read twice (once for
+ * the tensor maximum) instead of being packed and unpacked through memory; a small tensor is one launch and needs no
+ * workspace (metis_nvfp4_roundtrip_workspace_bytes is 0).
+ *   x, out    [rows, cols], contiguous: bf16 with METIS_MODE_PB16, float with METIS_MODE_P32_F32; 16-byte aligned
+ */
+size_t metis_nvfp4_roundtrip_workspace_bytes(int64_t rows, int64_t cols, int mode);
+int metis_nvfp4_roundtrip(const void *x, int64_t rows, int64_t cols, int mode, void *out, void *workspace,
+                          size_t workspace_bytes, void *stream);
+
+/*
  * metis_nvfp4_quant_row without a workspace argument and without any allocation: the scratch (per-workgroup
  * maxima and the parked block maxima) is a static device array inside the library.  No counterpart in the
  * reference; it exists for callers that cannot allocate device memory: code under HIP graph capture, tight

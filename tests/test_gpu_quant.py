@@ -739,6 +739,31 @@ def test_binary32_round_trip_from_one_call(ops, rows, cols):
     assert same_bits(q.quantize_dequantize(x).cpu(), out.cpu())
 
 
+# one launch / two launches (the line is 192 x 1024 elements in bf16, 128 x 1024 in binary32), odd tails, one block, leading dimensions
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 16), (3, 48), (5, 7, 80), (128, 1024), (129, 1024), (192, 1024), (193, 1024), (2049, 4080)])
+def test_round_trip_values_without_a_packed_tensor(ops, dtype, shape):
+    """ops.roundtrip: the values of quantize + dequantize bit for bit, with signed zeros, subnormal blocks, an infinity and a NaN."""
+    from metis_hip import quant_func
+    q = quant_func["nvfp4e2m1bnosr"]
+    mode = 1 if dtype == torch.bfloat16 else 0
+    bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
+    x = _f32_valued(shape[0] + shape[-1], 1, int(np.prod(shape))).reshape(shape).to(dtype).cuda()
+    flat = x.view(-1)
+    flat[::97] = -0.0
+    flat[:16] = 1e-39
+    for value in (None, float("inf"), float("nan")):
+        if value is not None:
+            flat[flat.numel() // 2] = value
+        want = ops.dequantize(ops.quantize(x, mode), dtype).reshape(shape)
+        for got in (ops.roundtrip(x), q.quantize_dequantize(x)):
+            assert got.shape == x.shape and got.dtype == dtype and not got.requires_grad
+            assert torch.equal(got.view(bits), want.view(bits)), (shape, value)
+    strided = x.movedim(0, -1)
+    if strided.shape[-1] % 16 == 0:
+        assert torch.equal(q.quantize_dequantize(strided).view(bits), q.quantize_dequantize(strided.contiguous()).view(bits))
+
+
 def test_both_packings_of_a_whole_row_count_are_tensors_of_their_own(ops):
     """Only a padded call hands out views (the row packing of the tensor's own rows)."""
     x = torch.randn(64, 128, device="cuda").bfloat16()
