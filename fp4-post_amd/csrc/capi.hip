@@ -85,6 +85,21 @@ int metis_rmsnorm_colmean(const void* x, const void* gamma, float eps, int64_t r
                            workspace_bytes, (hipStream_t)stream);
 }
 
+int metis_rmsnorm(const void* x, const void* gamma, float eps, int64_t rows, int64_t cols, void* normed, void* stream)
+{
+    return rmsnorm(x, gamma, eps, rows, cols, normed, (hipStream_t)stream);
+}
+
+int metis_token_mean_quant_applies(int64_t rows, int64_t cols, int after_norm) { return token_mean_quant_applies(rows, cols, after_norm); }
+
+int metis_token_mean_quant_deferred(const void* x, int64_t rows, int64_t cols, int after_norm, const void* cached, int64_t cached_count, void* mean,
+                                    float* mean32, void* codes, void* deferred, size_t deferred_bytes, const void* v, int64_t r, void* lr_workspace,
+                                    size_t lr_workspace_bytes, void* stream)
+{
+    return token_mean_quant(x, rows, cols, after_norm, cached, cached_count, mean, mean32, codes, deferred, deferred_bytes, v, r, lr_workspace,
+                            lr_workspace_bytes, (hipStream_t)stream);
+}
+
 size_t metis_rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols) { return rmsnorm_backward_workspace_bytes(rows, cols); }
 
 int metis_rmsnorm_backward(const void* x, const void* grad, const void* gamma, float eps, int64_t rows, int64_t cols, void* grad_x,

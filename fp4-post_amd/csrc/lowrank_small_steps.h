@@ -23,12 +23,13 @@ inline int lowrank_small_chunks(int64_t K, int* kc_out)
 }
 
 // One workgroup of the first step: K chunk `chunk` (kc elements), rows 64 mtile .. ; wave w owns columns 32 w .. of R
-// (waves past R / 32 have nothing to do), so the launch needs at least 2 R threads per workgroup.
+// (waves past R / 32 have nothing to do), so the launch needs at least 2 R threads per workgroup, or several workgroups for a chunk,
+// the first wave of each (wave0) further on in R.
 __device__ __forceinline__ void lowrank_small_partial_block(int chunk, int mtile, const uint16_t* __restrict__ x, int64_t ldx,
                                                             const uint16_t* __restrict__ v, int M, int R, int K, int kc,
-                                                            float* __restrict__ ws)
+                                                            float* __restrict__ ws, int wave0 = 0)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hi = lane >> 5;
+    const int lane = threadIdx.x & 63, wave = wave0 + (int)(threadIdx.x >> 6), hi = lane >> 5;
     if (wave * 32 >= R) return;
     const int m0 = mtile * 64;
     const int k0 = chunk * kc, k1 = min(k0 + kc, K);

@@ -1193,8 +1193,8 @@ int decode_prepare_deferred(const void* x, int64_t ldx, const void* v, int64_t R
     if (x) {
         if (const int rc = lowrank_small_partial(x, ldx, v, M, R, K, s, xv, t, workspace, workspace_bytes, st, &chunks)) return rc;
     } else {
-        // the partial sums are in the workspace already (quantize_row_deferred_partial on the same shapes)
-        if (R <= 0 || R % 32 || R > 128) return METIS_E_SHAPE;
+        // the partial sums are in the workspace already (quantize_row_deferred_partial or token_mean_quant on the same shapes)
+        if (R <= 0 || R % 32 || R > 256) return METIS_E_SHAPE;
         if (!xv || (t && !s) || ((uintptr_t)xv % 8) || ((uintptr_t)t % 8) || ((uintptr_t)s % 2)) return METIS_E_ARG;
         if (!workspace || ((uintptr_t)workspace % 16) || workspace_bytes < lowrank_small_workspace_bytes(M, R, K)) return METIS_E_WORKSPACE;
         int kc;

@@ -101,6 +101,12 @@ int rmsnorm_quantize(const void* x, const void* gamma, float eps, int64_t rows, 
 size_t rmsnorm_colmean_workspace_bytes(int64_t rows, int64_t cols);
 int rmsnorm_colmean(const void* x, const void* gamma, float eps, int64_t rows, int64_t cols, void* normed, void* mean, int mean_bf16,
                     const void* cached, int64_t cached_count, float* mean32, void* workspace, size_t workspace_bytes, hipStream_t st);
+int64_t rmsnorm_colmean_groups(int64_t rows);                 // partial rows of its sums
+int rmsnorm(const void* x, const void* gamma, float eps, int64_t rows, int64_t cols, void* normed, hipStream_t st);   // the normed tensor alone
+// column mean, centred packing (deferred scale bytes, bf16 arithmetic) and the projection's first step of few rows; token_mean_quant.hip
+int token_mean_quant_applies(int64_t rows, int64_t cols, int after_norm);
+int token_mean_quant(const void* x, int64_t rows, int64_t cols, int after_norm, const void* cached, int64_t cached_count, void* mean, float* mean32,
+                     void* codes, void* deferred, size_t bytes, const void* v, int64_t R, void* lr_workspace, size_t lr_workspace_bytes, hipStream_t st);
 // gradients of the norm (gx bf16, ggamma optional); rmsnorm_quant.hip
 size_t rmsnorm_backward_workspace_bytes(int64_t rows, int64_t cols);
 int rmsnorm_backward(const void* x, const void* g, const void* gamma, float eps, int64_t rows, int64_t cols, void* gx, void* ggamma,
@@ -169,6 +175,7 @@ int hadamard16(const void* x, int64_t rows, int64_t cols, int64_t ldx, int dtype
 
 // me[c] = mean over rows of x[:, c] (binary32 accumulation); nvfp4_gemv.hip
 size_t column_mean_workspace_bytes(int64_t cols);
+int64_t column_mean_slabs(int64_t rows, int64_t cols, int64_t* rows_per_slab);
 int column_mean(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_f32, void* out, int out_bf16, void* workspace,
                 size_t workspace_bytes, hipStream_t st, bool sum_only = false, const void* cached = nullptr,
                 int64_t cached_count = 0, float* out32 = nullptr);

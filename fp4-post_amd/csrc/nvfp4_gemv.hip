@@ -266,6 +266,18 @@ __global__ __launch_bounds__(64) void column_mean_finish_kernel(const float* __r
 
 size_t column_mean_workspace_bytes(int64_t cols) { return cols > 0 ? (size_t)kMeanMaxSlabs * (size_t)cols * sizeof(float) : 0; }
 
+// Slabs of the sum: enough workgroups to fill the device about eight times over, at least 16 rows each, at most kMeanMaxSlabs
+int64_t column_mean_slabs(int64_t rows, int64_t cols, int64_t* rows_per_slab)
+{
+    const int64_t strips = (cols + 255) / 256;
+    int64_t slabs = (8 * (int64_t)device_cus() + strips - 1) / strips;
+    if (slabs > (rows + 15) / 16) slabs = (rows + 15) / 16;
+    if (slabs > kMeanMaxSlabs) slabs = kMeanMaxSlabs;
+    if (slabs < 1) slabs = 1;
+    *rows_per_slab = (rows + slabs - 1) / slabs;
+    return (rows + *rows_per_slab - 1) / *rows_per_slab;
+}
+
 int column_mean(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_f32, void* out, int out_bf16, void* workspace,
                 size_t workspace_bytes, hipStream_t st, bool sum_only, const void* cached, int64_t cached_count, float* out32)
 {
@@ -278,13 +290,9 @@ int column_mean(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_f3
     if (((uintptr_t)x % (in_f32 ? 16 : 8)) || ((uintptr_t)out % 4)) return METIS_E_ARG;
     if (!workspace || ((uintptr_t)workspace % 16) || workspace_bytes < column_mean_workspace_bytes(cols)) return METIS_E_WORKSPACE;
     const uint32_t strips = (uint32_t)((cols + 255) / 256);
-    // enough workgroups to fill the device about eight times over, at least 16 rows each, at most kMeanMaxSlabs slabs
-    int64_t slabs = (8 * (int64_t)device_cus() + strips - 1) / strips;
-    if (slabs > (rows + 15) / 16) slabs = (rows + 15) / 16;
-    if (slabs > kMeanMaxSlabs) slabs = kMeanMaxSlabs;
-    if (slabs < 1) slabs = 1;
-    const uint32_t rows_per_slab = (uint32_t)((rows + slabs - 1) / slabs);
-    slabs = (rows + rows_per_slab - 1) / rows_per_slab;
+    int64_t per = 0;
+    const int64_t slabs = column_mean_slabs(rows, cols, &per);
+    const uint32_t rows_per_slab = (uint32_t)per;
     float* partial = static_cast<float*>(workspace);
     const dim3 grid(strips, (unsigned)slabs);
     if (in_f32)

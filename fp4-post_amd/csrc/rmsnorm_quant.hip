@@ -229,13 +229,14 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_rows_kernel(const uint4* __
 // a wave, then the four waves in order.  rmsnorm_colmean_finish_kernel adds the workgroups' partial rows in order and
 // applies the mean's division and rounding (and the running mean of decode calls) as column_mean_finish_kernel does.
 // ---------------------------------------------------------------------------------------------
-template <int NL>
+// SUMS = false: the normed tensor alone (a consumer that sees all rows of a column forms the sums itself, token_mean_quant.hip).
+template <int NL, bool SUMS = true>
 __global__ __launch_bounds__(256) void rmsnorm_colsum_rows_kernel(const uint4* __restrict__ x, const uint4* __restrict__ gamma, float eps,
                                                                   uint32_t rows, uint32_t cols, metis_u32x4_t* __restrict__ normed,
                                                                   float* __restrict__ partial)
 {
     __shared__ uint4 g_a[NL * 64], g_b[NL * 64];
-    __shared__ float4 sums[NL * 64][2];                        // column sums of the workgroup, chunk by chunk
+    __shared__ float4 sums[SUMS ? NL * 64 : 1][2];             // column sums of the workgroup, chunk by chunk
     const uint32_t cpr = cols / 8u;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const float fcols = (float)cols;
@@ -258,9 +259,9 @@ __global__ __launch_bounds__(256) void rmsnorm_colsum_rows_kernel(const uint4* _
         g_b[c] = make_uint4(g.z & 0xffffu, g.z & 0xffff0000u, g.w & 0xffffu, g.w & 0xffff0000u);
     }
     __syncthreads();
-    float acc[NL][8];
+    float acc[SUMS ? NL : 1][8];
 #pragma unroll
-    for (int i = 0; i < NL; ++i)
+    for (int i = 0; i < (SUMS ? NL : 1); ++i)
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[i][j] = 0.0f;
     for (; row < rows; row += wstep) {
@@ -290,13 +291,17 @@ __global__ __launch_bounds__(256) void rmsnorm_colsum_rows_kernel(const uint4* _
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t h = rb_pair(bf16_lo(in[j]) * rstd, bf16_hi(in[j]) * rstd);
                     w[j] = rb_pair(dot2_bf16(h, gl[j], 0.0f), dot2_bf16(h, gh[j], 0.0f));
-                    acc[i][2 * j] += bf16_lo(w[j]);
-                    acc[i][2 * j + 1] += bf16_hi(w[j]);
+                    if constexpr (SUMS) {
+                        acc[i][2 * j] += bf16_lo(w[j]);
+                        acc[i][2 * j + 1] += bf16_hi(w[j]);
+                    }
                 }
                 __builtin_nontemporal_store((metis_u32x4_t){w[0], w[1], w[2], w[3]}, normed + (size_t)row * cpr + c);
             }
         }
     }
+    if constexpr (!SUMS) return;
+    else {
     // the four waves' sums, added in wave order
 #pragma unroll 1
     for (uint32_t v = 0; v < 4u; ++v) {
@@ -320,6 +325,7 @@ __global__ __launch_bounds__(256) void rmsnorm_colsum_rows_kernel(const uint4* _
     }
     float4* out = reinterpret_cast<float4*>(partial + (size_t)blockIdx.x * cols);
     for (uint32_t q = threadIdx.x; q < cpr * 2u; q += 256u) out[q] = sums[q >> 1][q & 1u];
+    }
 }
 
 // 1 / sqrt(ss / n + eps) as hi + lo: the remainders of the quotient, of the sum and of the root enter one Newton step.  With each
@@ -530,6 +536,24 @@ static int colmean_grid(int64_t rows)
     const int64_t cap = (int64_t)device_cus() * 2;           // the column sums cost registers: two waves per SIMD
     if (g > cap) g = cap;
     return g < 1 ? 1 : (int)g;
+}
+
+int64_t rmsnorm_colmean_groups(int64_t rows) { return colmean_grid(rows); }
+
+int rmsnorm(const void* x, const void* gamma, float eps, int64_t rows, int64_t cols, void* normed, hipStream_t st)
+{
+    if (rows < 0 || cols < 0) return METIS_E_ARG;
+    if (cols % kBlock) return METIS_E_SHAPE;
+    if (cols > 4096) return METIS_E_ARG;                      // one wave per row
+    if (rows == 0 || cols == 0) return METIS_OK;
+    if (rows > INT32_MAX || !x || !gamma || !normed || ((uintptr_t)x % 16) || ((uintptr_t)gamma % 16) || ((uintptr_t)normed % 16)) return METIS_E_ARG;
+    const int64_t cap = (int64_t)device_cus() * 4, need = (rows + 3) / 4;
+    const int nl = (int)((cols / 8 + 63) / 64);
+#define METIS_RN(NL) hipLaunchKernelGGL((rmsnorm_colsum_rows_kernel<NL, false>), dim3((unsigned)(need < cap ? need : cap)), dim3(256), 0, st, (const uint4*)x, \
+        (const uint4*)gamma, eps, (uint32_t)rows, (uint32_t)cols, (metis_u32x4_t*)normed, (float*)nullptr)
+    if (nl <= 2) METIS_RN(2); else if (nl <= 4) METIS_RN(4); else METIS_RN(8);
+#undef METIS_RN
+    return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 
 size_t rmsnorm_colmean_workspace_bytes(int64_t rows, int64_t cols)

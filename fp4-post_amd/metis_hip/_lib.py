@@ -52,6 +52,9 @@ SIGNATURES = {
     "metis_nvfp4_decode_weight": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp]),
     "metis_rmsnorm_colmean_workspace_bytes": (_sz, [_i64, _i64]),
     "metis_rmsnorm_colmean": (_i32, [_vp, _vp, _f32, _i64, _i64, _vp, _vp, _i32, _vp, _i64, _vp, _vp, _sz, _vp]),
+    "metis_rmsnorm": (_i32, [_vp, _vp, _f32, _i64, _i64, _vp, _vp]),
+    "metis_token_mean_quant_applies": (_i32, [_i64, _i64, _i32]),
+    "metis_token_mean_quant_deferred": (_i32, [_vp, _i64, _i64, _i32, _vp, _i64, _vp, _vp, _vp, _vp, _sz, _vp, _i64, _vp, _sz, _vp]),
     "metis_rmsnorm_backward_workspace_bytes": (_sz, [_i64, _i64]),
     "metis_rmsnorm_backward": (_i32, [_vp, _vp, _vp, _f32, _i64, _i64, _vp, _vp, _i32, _vp, _sz, _vp]),
     "metis_linear_fwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _i32, _vp]),

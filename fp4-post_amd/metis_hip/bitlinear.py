@@ -337,6 +337,32 @@ class LinearLowbitFunction(torch.autograd.Function):
         return me.reshape(-1), None
 
     @staticmethod
+    def _mean_packed_at_once() -> bool:
+        """The mean mode in bf16 arithmetic with the reference's roundings and round to nearest: what ops.quantize does with a TokenMean centre."""
+        F = LinearLowbitFunction
+        return F.reference_rounding and F.compute_dtype == torch.bfloat16 and F.q_forward_input is Cast2NVFp4e2m1BlockNOSR
+
+    @staticmethod
+    def _token_mean_pack(input_: torch.Tensor, after_norm: bool, mean_cache=None, cache_key="default", projection=None):
+        """CenteredNVFP4 of an activation of few tokens from one launch (mean, running mean, centred packing as _token_mean2 and the
+        quantizer give them), or None where that launch does not apply.  projection (key, V): with the first step of x V^T."""
+        F = LinearLowbitFunction
+        x2 = _flat2d(input_)
+        if not ops.token_mean_applies(x2, after_norm):
+            return None
+        rows = x2.shape[0]
+        seq_len = input_.shape[1] if input_.dim() == 3 else input_.shape[0]
+        cached_mean, cached_count = mean_cache[cache_key] if (seq_len == 1 and mean_cache is not None and cache_key in mean_cache) else (None, 0)
+        if cached_count + rows > 2 ** 24:
+            return None
+        key, v = projection if projection is not None else (None, None)
+        tm = ops.TokenMean(after_norm, cached_mean, cached_count, v)
+        packed = F.q_forward_input.pack(x2, arith=F.compute_dtype, center=tm, deferred=True)
+        if mean_cache is not None:
+            mean_cache[cache_key] = (tm.mean.unsqueeze(0), cached_count + rows)
+        return CenteredNVFP4(packed, tm.mean, tm.mean32, None if tm.pending is None else (key, tm.pending))
+
+    @staticmethod
     def _mean_mode_packable() -> bool:
         F = LinearLowbitFunction
         return F.metis_mode == "mean" and not F.tp_simulate and not F.enable_nv_recipe
@@ -381,10 +407,11 @@ class LinearLowbitFunction(torch.autograd.Function):
 
     @staticmethod
     def _prepare_input(input_: torch.Tensor, mean_cache=None, cache_key="default", weights_cached: bool = True,
-                       keep_dense: bool | None = None):
+                       keep_dense: bool | None = None, projection=None):
         """Packed activation when a kernel path applies (direct: PackedNVFP4; mean mode: CenteredNVFP4; svd mode:
         LowRankNVFP4), else the dequantized tensor.  weights_cached: the layers that will read it keep their packed
-        weights across calls.  keep_dense (svd mode): a backward pass will follow; default: autograd is recording."""
+        weights across calls.  keep_dense (svd mode): a backward pass will follow; default: autograd is recording.
+        projection: see _token_mean_pack."""
         F = LinearLowbitFunction
         if (not F.enable_nv_recipe or F._nv_on_kernels()) and _packable(input_, F.q_forward_input):
             if not F.enable_activation_svd:
@@ -403,6 +430,10 @@ class LinearLowbitFunction(torch.autograd.Function):
             if F._mean_mode_packable():
                 # mean + QDQ(x - mean) (reference 311-336) without materialising either: the subtraction happens
                 # inside the quantizer and the mean's contribution to a matmul is a rank-one term
+                if F._mean_packed_at_once():
+                    at_once = F._token_mean_pack(input_.detach() if torch.is_grad_enabled() else input_, False, mean_cache, cache_key, projection)
+                    if at_once is not None:
+                        return at_once
                 me, me32 = F._token_mean2(input_, mean_cache=mean_cache, cache_key=cache_key)
                 more = {"deferred": True} if (F._bf16_rounding() and me.dtype == torch.bfloat16) else {}
                 return CenteredNVFP4(F.q_forward_input.pack(_flat2d(input_), arith=F.compute_dtype, center=me, **more), me, me32)
@@ -786,7 +817,8 @@ class _MetisFusedFunction(torch.autograd.Function):
                 xv, t, aop = ops.project_and_operand(_flat2d(x).to(cd), v.to(cd), s.to(cd), px,
                                                      ops.nv_operand_mode(px, [p_res], F.reference_rounding), pending=pending, rotate=p_res.rht)
             else:
-                xv, t, aop = ops.project_and_operand(_flat2d(x).to(cd), v.to(cd), s.to(cd), px, ops.MODE_PB16, None, pending=pending)
+                target, centre = (px.residual, px.mean) if isinstance(px, CenteredNVFP4) else (px, None)
+                xv, t, aop = ops.project_and_operand(_flat2d(x).to(cd), v.to(cd), s.to(cd), target, ops.MODE_PB16, centre, pending=pending)
         elif xv is None:
             # [L, r] rank-r projection and its product with s (bf16) on the library's kernels (split-K below 256 rows,
             # one pass over x from there on); the caller has it already when the quantizer's pass produced it
@@ -971,8 +1003,10 @@ class BitLinear(nn.Module):
         F = LinearLowbitFunction
         group = getattr(self, "activation_group", None)
         if group is None:
+            projection = self._own_projection(x)
+            more = {} if projection is None else {"projection": projection}
             return F._prepare_input(x, mean_cache=self.mean_cache, cache_key=f"{self.layer_name}.shared",
-                                    weights_cached=self._weights_cached())
+                                    weights_cached=self._weights_cached(), **more)
         input_ref = group.get("input_ref")
         if input_ref is not None and input_ref() is x and group.get("input_version") == _version_of(x):
             return group["quantized_input"]
@@ -1112,6 +1146,28 @@ class BitLinear(nn.Module):
                 return px, None, None, pending
         return None
 
+    def _own_projection(self, x: torch.Tensor):
+        """(None, V) for the launch that packs this layer's decode-sized activation under the mean mode, when no sibling shares it; None
+        otherwise.  (A prompt's mean and packing are one launch too; its projection is another kernel's.)"""
+        F = LinearLowbitFunction
+        rows = x.numel() // max(x.shape[-1], 1)
+        if not (F.enable_activation_svd and 0 < rows < 256 and F._mean_packed_at_once() and self._fusable()):
+            return None
+        v, s = _param(self._modules["vlinear"], "weight"), _param(self, "s")
+        if s.dtype != torch.bfloat16 or v.device != x.device or not ops.quantize_project_decode_applies(_flat2d(x), v, ops.MODE_PB16):
+            return None
+        return None, v.detach()
+
+    @staticmethod
+    def _group_projection(group, rows: int, cols: int, device):
+        """(key, stacked V) for the launch that packs a group's decode-sized activation: the factors of the group's last evaluation in one
+        call (the next one uses the sums if they are still the factors of now); None otherwise."""
+        cached = group.get("stacked_v")
+        if cached is None or not (0 < rows < 256 and cols % 256 == 0):
+            return None
+        v = cached[1]
+        return (cached[0], v) if (v.shape[1] == cols and v.shape[0] <= 256 and v.shape[0] % 32 == 0 and v.device == device) else None
+
     def _forward_group(self, x: torch.Tensor, shared_input):
         """All members of this layer's projection group on the shared activation in one call (no autograd):
         {id(member): output}, or None when the group does not qualify.  The siblings pick their result up when they
@@ -1150,7 +1206,9 @@ class BitLinear(nn.Module):
         elif (ops.grouped_operand_applies(px, packed, [m.args.forward_svd_rank for m in members], centre, F.reference_rounding)
                 and ops.project_and_operand_applies(x2, cached[1], cached[2], px)):
             # the projection's finishing step and the activation's GEMM operands in one launch
-            _, t_all, aop = ops.project_and_operand(x2, cached[1], cached[2], px, ops.MODE_PB16, centre)
+            pending = getattr(shared_input, "pending", None)       # its first step ran beside the quantizer, with these very factors
+            _, t_all, aop = ops.project_and_operand(x2, cached[1], cached[2], px, ops.MODE_PB16, centre,
+                                                    pending=pending[1] if pending is not None and pending[0] is cached[0] else None)
         else:
             _, t_all = ops.lowrank_project(x2, cached[1], cached[2])
         calls, c0 = [], 0
@@ -1336,6 +1394,9 @@ class BitLinear(nn.Module):
                 p_res = self._packed_residual()
                 if p_res is not None:
                     more = () if fused is None else fused[1:]
+                    if (group is None and getattr(shared_input, "pending", None) is not None and F._mean_in_operand(shared_input, p_res)
+                            and ops.grouped_operand_applies(shared_input.residual, [p_res], [r], shared_input.mean, F.reference_rounding)):
+                        more = (None, None, shared_input.pending[1])
                     wl = mods["warmup_linear"]
                     return _MetisFusedFunction.apply(x, _param(mods["vlinear"], "weight"), _param(self, "s"), _param(mods["ulinear"], "weight"),
                                                      _param(wl, "weight"), wl.bias, shared_input, p_res, *more)

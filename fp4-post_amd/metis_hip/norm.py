@@ -76,7 +76,7 @@ class FusedRMSNormQuant(nn.Module):
         h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + self.variance_epsilon)
         return self.weight * h.to(dtype)
 
-    def _mean_mode(self, x: torch.Tensor):
+    def _mean_mode(self, x: torch.Tensor, recording: bool):
         """The reference's default arguments (mean mode, src/grpo/grpo.py:66-69): the group's activation is
         mean + QDQ(normed - mean) with the column mean over tokens (src/Metis/Metis/bitlinear.py:311-336).  One pass
         over x writes the normed tensor and leaves its column sums; the centred quantizer then reads the normed tensor.
@@ -93,6 +93,13 @@ class FusedRMSNormQuant(nn.Module):
         cached_mean, cached_count = cache[key] if running else (None, 0)
         if cached_count + rows > 2 ** 24:
             return None
+        if F._mean_packed_at_once() and ops._token_mean_takes(rows, cols, 1, x.device.index or 0) and rows <= ops.TOKEN_MEAN_MAX_ROWS:
+            # few tokens: the launch that packs the normed tensor forms the mean itself
+            normed = ops.rmsnorm(x, self.weight, self.variance_epsilon)
+            projection = None if (recording or not BitLinear.grouped_inference) else BitLinear._group_projection(group, rows, cols, x.device)
+            packed = F._token_mean_pack(normed.reshape(x.shape), True, cache, key, projection)
+            if packed is not None:
+                return normed, packed
         normed, me, me32 = ops.rmsnorm_colmean(x, self.weight, self.variance_epsilon, cd, cached_mean, cached_count)
         cache[key] = (me.detach().unsqueeze(0), cached_count + rows)
         more = {"deferred": True} if (F._bf16_rounding() and me.dtype == torch.bfloat16) else {}
@@ -112,9 +119,10 @@ class FusedRMSNormQuant(nn.Module):
         if not fused:
             return self._plain(x)
         mode = MODE_P32 if F.compute_dtype == torch.float32 else MODE_PB16
+        recording = torch.is_grad_enabled()
         with torch.no_grad():
             if mean_mode:
-                got = self._mean_mode(x)
+                got = self._mean_mode(x, recording)
                 if got is None:
                     return self._plain(x)
                 normed, packed = got

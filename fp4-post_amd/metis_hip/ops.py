@@ -111,6 +111,7 @@ class CenteredNVFP4:
     residual: PackedNVFP4
     mean: torch.Tensor
     mean32: torch.Tensor | None = None       # the same values as float32 when the producer had them at hand
+    pending: tuple | None = None             # (what it was made with, partial sums of a rank-r projection) from the same launch
 
     @property
     def center32(self) -> torch.Tensor:
@@ -231,7 +232,7 @@ def _as_2d_for_quant(x: torch.Tensor, mode: int) -> tuple[torch.Tensor, int]:
 
 def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bool = False,
              noise: torch.Tensor | None = None, seed: int = 0, offset: int = 0,
-             center: torch.Tensor | None = None, resident: bool = False, spin_limit: int = 0,
+             center: torch.Tensor | TokenMean | None = None, resident: bool = False, spin_limit: int = 0,
              deferred: bool = False, pad_rows: int | None = None) -> PackedNVFP4:
     """NVFP4-quantize x (flattened to [R, C]).
 
@@ -240,7 +241,8 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
     sr=True  : stochastic rounding; `noise` (same shape as x, float32 for P32 / bf16 for PB16)
                overrides the internal Philox stream keyed by (seed, offset).
     center   : [C] vector subtracted from every row first (the reference's mean mode), in the arithmetic's
-               dtype: the packed tensor is that of x - center.
+               dtype: the packed tensor is that of x - center.  A TokenMean: the column mean of x itself, formed in the
+               same launch and left in it (deferred, bf16 arithmetic, see token_mean_applies).
     resident : round-to-nearest rows of a bf16 tensor as ONE launch (metis_nvfp4_quant_row_resident), same bytes: a
                workgroup that gives up waiting for the grid's maximum after `spin_limit` polls (0: library default)
                leaves its scale bytes to the last workgroup.
@@ -251,6 +253,10 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
                zero without one); no copy of x is made.  Only without caller noise.
     """
     x2, kmode = _as_2d_for_quant(x, mode)
+    if isinstance(center, TokenMean):
+        if not deferred or col or sr or kmode != MODE_PB16 or pad_rows is not None:
+            raise ValueError("a TokenMean centre: bf16 arithmetic, rows, round to nearest, scale bytes deferred")
+        return _quantize_token_mean(x2, center)
     rows, cols = x2.shape
     if pad_rows is not None and pad_rows != rows:
         return _quantize_col_padded(x2, kmode, mode, pad_rows, col, sr, noise, seed, offset, center)
@@ -595,6 +601,73 @@ def column_mean_running(x: torch.Tensor, cached: torch.Tensor | None, cached_cou
     return out, out32
 
 
+@functools.lru_cache(maxsize=4096)
+def _token_mean_takes(rows: int, cols: int, after_norm: int, device_index: int) -> bool:
+    return bool(load().metis_token_mean_quant_applies(rows, cols, after_norm))       # depends on the device's CU count only
+
+
+TOKEN_MEAN_MAX_ROWS = 768
+
+
+def token_mean_applies(x2: torch.Tensor, after_norm: bool) -> bool:
+    """quantize() with a TokenMean centre takes this tensor: few rows (a decode step, a short prompt), contiguous bf16.  Beyond 768 rows a
+    narrow tensor's strips are too few workgroups for the work (times beside the kernel, token_mean_quant.hip)."""
+    return (x2.is_cuda and x2.dtype == torch.bfloat16 and x2.dim() == 2 and 0 < x2.shape[0] <= TOKEN_MEAN_MAX_ROWS and x2.shape[1] % 32 == 0
+            and x2.is_contiguous() and x2.data_ptr() % 16 == 0
+            and _token_mean_takes(x2.shape[0], x2.shape[1], int(after_norm), x2.device.index or 0))
+
+
+@dataclass
+class TokenMean:
+    """A centre that quantize() forms itself in the launch that subtracts it: the column mean of the tensor over its rows, as
+    column_mean_running(x, cached, cached_count, bfloat16) gives it -- or, after_norm, as rmsnorm_colmean does of its normed tensor.
+    v (bf16 [r, cols], optional): the same launch leaves the partial sums of x . v^T for project_and_operand(..., pending=)."""
+    after_norm: bool = False
+    cached: torch.Tensor | None = None
+    cached_count: int = 0
+    v: torch.Tensor | None = None
+    # results
+    mean: torch.Tensor | None = None
+    mean32: torch.Tensor | None = None
+    pending: torch.Tensor | None = None
+
+
+def _quantize_token_mean(x2: torch.Tensor, tm: TokenMean) -> PackedNVFP4:
+    if not token_mean_applies(x2, tm.after_norm):
+        raise ValueError("a TokenMean centre: outside the call's domain (see token_mean_applies)")
+    after_norm, cached, cached_count, v = tm.after_norm, tm.cached, tm.cached_count, tm.v
+    rows, cols = x2.shape
+    dev = x2.device
+    cp = None
+    if cached is not None:
+        cached = cached.reshape(-1).to(device=dev, dtype=torch.bfloat16).contiguous()
+        if cached.numel() != cols:
+            raise ValueError(f"cached mean has {cached.numel()} values, the tensor {cols} columns")
+        cp = cached.data_ptr()
+    me = torch.empty(cols, dtype=torch.bfloat16, device=dev)
+    me32 = torch.empty(cols, dtype=torch.float32, device=dev)
+    codes = torch.empty(rows, cols // 2, dtype=torch.uint8, device=dev)
+    unit = torch.empty(1, dtype=torch.float32, device=dev)
+    size = _deferred_bytes(rows, cols)
+    parked = torch.empty(size, dtype=torch.uint8, device=dev)
+    pending, vp, R, need = None, None, 0, 0
+    if v is not None:
+        v = v.contiguous()
+        R = v.shape[0]
+        if v.dtype != torch.bfloat16 or v.shape[1] != cols or v.device != dev:
+            raise ValueError("TokenMean: v is bfloat16 [r, cols] on the tensor's device")
+        need = _lowrank_workspace_bytes(rows, R, cols)
+        pending = torch.empty(need, dtype=torch.uint8, device=dev)
+        vp = v.data_ptr()
+    rc = load().metis_token_mean_quant_deferred(x2.data_ptr(), rows, cols, int(after_norm), cp, int(cached_count), me.data_ptr(), me32.data_ptr(),
+                                                codes.data_ptr(), parked.data_ptr(), size, vp, R, None if pending is None else pending.data_ptr(),
+                                                need, _stream())
+    if rc:
+        check(rc, "metis_token_mean_quant_deferred", (rows, cols, R))
+    tm.mean, tm.mean32, tm.pending = me, me32, pending
+    return PackedNVFP4(codes, None, unit, rows, cols, MODE_PB16, deferred=parked)
+
+
 def matvec(p: PackedNVFP4, v: torch.Tensor | None = None, alpha: float = 1.0, *, out: torch.Tensor | None = None,
            split: torch.Tensor | None = None, split_col: int = 0, z: torch.Tensor | None = None,
            beta: float = 0.0) -> torch.Tensor | None:
@@ -848,8 +921,8 @@ def project_and_operand(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: P
     t = torch.empty_like(xv)
     out = torch.empty(_decode_operand_bytes(M, K), dtype=torch.uint8, device=dev)
     need = _lowrank_workspace_bytes(M, R, K)
-    if pending is not None and (pending.numel() < need or pending.device != dev or R > 128):
-        raise ValueError("project_and_operand: `pending` is not what quantize_project_decode returns for these shapes")
+    if pending is not None and (pending.numel() < need or pending.device != dev):
+        raise ValueError("project_and_operand: `pending` is not what quantize_project_decode or a TokenMean's call leaves for these shapes")
     ws = pending if pending is not None else torch.empty(need, dtype=torch.uint8, device=dev)
     d = p.__dict__
     rc = L.metis_decode_prepare_deferred(None if pending is not None else x2.data_ptr(), x2.stride(0), v.data_ptr(), R, s.data_ptr(),
@@ -1091,6 +1164,18 @@ def rmsnorm_quantize(x: torch.Tensor, gamma: torch.Tensor, eps: float, mode: int
     if normed is not None:
         normed = normed.reshape(x.shape)
     return normed, PackedNVFP4(codes, scales, unit, rows, cols, mode, decode_layout=dec)
+
+
+def rmsnorm(x: torch.Tensor, gamma: torch.Tensor, eps: float) -> torch.Tensor:
+    """The normed bf16 [R, C] of rmsnorm_colmean alone.  C <= 4096."""
+    x2 = _as_2d_bf16(x)
+    rows, cols = x2.shape
+    g = gamma.to(device=x2.device, dtype=torch.bfloat16).contiguous()
+    normed = torch.empty(rows, cols, dtype=torch.bfloat16, device=x2.device)
+    rc = load().metis_rmsnorm(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, normed.data_ptr(), _stream())
+    if rc:
+        check(rc, "metis_rmsnorm", x.shape)
+    return normed
 
 
 def rmsnorm_colmean(x: torch.Tensor, gamma: torch.Tensor, eps: float, mean_dtype: torch.dtype = torch.float32,

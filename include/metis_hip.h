@@ -280,6 +280,27 @@ int metis_rmsnorm_colmean(const void *x, const void *gamma, float eps, int64_t r
                           int64_t cached_count, float *mean32, void *workspace, size_t workspace_bytes,
                           void *stream);
 
+/* The normed tensor alone (x, gamma, normed as above). */
+int metis_rmsnorm(const void *x, const void *gamma, float eps, int64_t rows, int64_t cols, void *normed, void *stream);
+
+/*
+ * The mean mode's activation of few rows in one launch, bf16 arithmetic: the column mean over the rows (with the running mean of
+ * decode calls, as metis_column_mean_running), the packing of x - mean with its scale bytes deferred (as
+ * metis_nvfp4_quant_row_deferred with that centre) and, with v, the partial sums of the rank-r projection x . v^T that
+ * metis_decode_prepare_deferred(x = NULL) finishes.  The same bits as those calls.
+ *   x            bf16 [rows, cols], contiguous, 16-byte aligned, cols % 16 == 0
+ *   after_norm   1: the mean's sums in the order of metis_rmsnorm_colmean (x is a normed tensor), 0: of metis_column_mean
+ *   mean, mean32 bf16 and float [cols]
+ *   v            (optional) bf16 [r, cols], r % 32 == 0, r <= 256, cols % 64 == 0, rows < 256
+ *   lr_workspace metis_lowrank_project_workspace_bytes(rows, r, cols) bytes (with v)
+ * metis_token_mean_quant_applies: whether a shape is taken (METIS_E_TOO_LARGE otherwise): up to about a thousand rows.
+ */
+int metis_token_mean_quant_applies(int64_t rows, int64_t cols, int after_norm);
+int metis_token_mean_quant_deferred(const void *x, int64_t rows, int64_t cols, int after_norm, const void *cached,
+                                    int64_t cached_count, void *mean, float *mean32, void *codes, void *deferred,
+                                    size_t deferred_bytes, const void *v, int64_t r, void *lr_workspace,
+                                    size_t lr_workspace_bytes, void *stream);
+
 /*
  * Gradients of that RMSNorm (y = bf16(bf16(x rstd) gamma), src/Metis/models/llama.py:23-31) from one pass over x and the
  * gradient of y, in binary32 with xh = x * rstd:

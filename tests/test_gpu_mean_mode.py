@@ -682,3 +682,71 @@ def test_column_mean_of_the_normed_tensor_is_added_in_its_documented_order(rows,
         sums.append(s)
     total = (sums[0] + sums[1]) + (sums[2] + sums[3])
     assert torch.equal(me.cpu(), total / rows)
+
+
+# one row, one piece and a tail, a slab and one more, four slabs' edges, the decode limit, prompts up to the call's limit; a strip that
+# ends in half a block pair, widths around the XCD ranges of strips
+@pytest.mark.parametrize("rows", [1, 3, 16, 17, 63, 64, 65, 255, 256, 411, 768])
+@pytest.mark.parametrize("cols", [32, 96, 256, 1536, 8992])
+def test_mean_and_centred_packing_of_few_tokens_in_one_launch(rows, cols):
+    """ops.quantize with a TokenMean centre: mean, running mean, codes, scale bytes, unit and the projection's partial sums bit for bit as the
+    separate calls leave them, in both orders of the sums."""
+    from metis_hip import ops
+    x = _offset_activation(4000 + rows, rows, cols).cuda()
+    x.view(-1)[::53] = -0.0
+    gamma = (1 + 0.1 * torch.randn(cols, generator=torch.Generator().manual_seed(cols))).bfloat16().cuda()
+    kept = torch.randn(1, cols, generator=torch.Generator().manual_seed(7)).bfloat16().cuda()
+    for after_norm in (False, True):
+        if after_norm and cols > 4096:
+            continue
+        for cached, count in ((None, 0), (kept, 37)):
+            if after_norm:
+                src, me, me32 = ops.rmsnorm_colmean(x, gamma, 1e-6, torch.bfloat16, cached, count)
+                assert torch.equal(ops.rmsnorm(x, gamma, 1e-6), src)
+            else:
+                src = x
+                me, me32 = ops.column_mean_running(x, cached, count, torch.bfloat16)
+            want = ops.quantize(src, 1, center=me, deferred=True)
+            R = {32: 0, 96: 0, 256: 256, 1536: 64, 8992: 0}[cols]
+            v = torch.randn(R, cols, generator=torch.Generator().manual_seed(9)).bfloat16().cuda() if R and rows < 256 else None
+            assert ops.token_mean_applies(src, after_norm)
+
+            def at_once():
+                tm = ops.TokenMean(after_norm, cached, count, v)
+                return ops.quantize(src, 1, center=tm, deferred=True), tm.mean, tm.mean32, tm.pending
+            p, gme, gme32, pending = at_once()
+            torch.cuda.synchronize()
+            assert torch.equal(gme, me) and torch.equal(gme32, me32)
+            assert torch.equal(p.codes, want.codes) and torch.equal(p.scales, want.scales) and torch.equal(p.unit, want.unit)
+            assert (pending is None) == (v is None)
+            if v is not None:
+                s = torch.rand(R, generator=torch.Generator().manual_seed(11)).bfloat16().cuda()
+                q1, q2 = at_once(), at_once()
+                a = ops.project_and_operand(src, v, s, q1[0], ops.MODE_PB16, gme)
+                b = ops.project_and_operand(src, v, s, q2[0], ops.MODE_PB16, gme, pending=q2[3])
+                torch.cuda.synchronize()
+                assert all(torch.equal(l, r) for l, r in zip(a, b))
+
+
+def test_running_mean_of_decode_steps_through_the_one_launch_path():
+    """A BitLinear under the default arguments: prompt, then decode steps; the cache holds what the separate kernels would keep."""
+    from metis_hip import BitLinear, MetisArgs, ops
+    torch.manual_seed(3)
+    outs, means = [], []
+    for limit in (ops.TOKEN_MEAN_MAX_ROWS, 0):
+        torch.manual_seed(5)
+        layer = BitLinear(512, 256, args=MetisArgs(forward_svd_rank=32, cache_quantized_weight=True), dtype=torch.bfloat16).cuda()
+        layer.split()
+        keep, ops.TOKEN_MEAN_MAX_ROWS = ops.TOKEN_MEAN_MAX_ROWS, limit
+        try:
+            with torch.no_grad():
+                for step, shape in enumerate([(1, 300, 512), (4, 1, 512), (4, 1, 512)]):
+                    x = torch.randn(*shape, generator=torch.Generator().manual_seed(step)).bfloat16().cuda()
+                    outs.append(layer(x))
+        finally:
+            ops.TOKEN_MEAN_MAX_ROWS = keep
+        means.append({k: (m.clone(), n) for k, (m, n) in layer.mean_cache.items()})
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(outs[:3], outs[3:]))
+    assert means[0].keys() == means[1].keys()
+    assert all(torch.equal(means[0][k][0], means[1][k][0]) and means[0][k][1] == means[1][k][1] for k in means[0])
