@@ -560,6 +560,16 @@ int metis_lowrank_contract_tokens(const void* a, int64_t lda, const void* b, int
     return lowrank_tn(a, lda, b, L, C, R, out, out_dtype, transpose, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+size_t metis_lowrank_backward_workspace_bytes(int64_t L, int64_t N, int64_t K, int64_t R) { return lowrank_backward_workspace_bytes(L, N, K, R); }
+
+int metis_lowrank_backward(const void* dy, int64_t lddy, const void* t, int64_t N, const void* x, int64_t ldx, const void* gxv, int64_t K, int64_t L,
+                           int64_t R, void* gu, int gu_dtype, void* gv, int gv_dtype, const void* gt, const void* xv, void* gs, int gs_dtype,
+                           void* workspace, size_t workspace_bytes, void* stream)
+{
+    return lowrank_backward(dy, lddy, t, N, x, ldx, gxv, K, L, R, gu, gu_dtype, gv, gv_dtype, gt, xv, gs, gs_dtype, workspace, workspace_bytes,
+                            (hipStream_t)stream);
+}
+
 size_t metis_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) { return gemm_workspace_bytes(M, N, K); }
 
 int metis_linear_fwd_ws(const void* a_codes, const void* a_scales, const float* a_unit, const void* b_codes,

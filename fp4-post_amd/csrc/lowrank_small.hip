@@ -73,52 +73,14 @@ int lowrank_small(const void* x, int64_t ldx, const void* v, int64_t M, int64_t 
 // tensors, a few hundred KB: one workgroup per 8 columns walks all rows (a thread takes every 256th row, 16 bytes of
 // each tensor per row), and the 256 per-thread sums of a column are added in thread order -- a fixed order, one launch.
 // Bound by latency: eight rows of a thread are requested together (one at a time, each waited for, 6.7 us at 4096 x 32; this
-// 5.7), and the adder of a column reads half of its sums, four to a load, before it adds the first.
+// 5.7), and the adder of a column reads a quarter of its sums, four to a load, before it adds the first.  (A layer's backward pass runs it
+// beside its contractions over tokens, lowrank_backward.)
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void scale_grad_kernel(const uint16_t* __restrict__ g, const uint16_t* __restrict__ xv, int L, int R,
                                                          void* __restrict__ out, int out_f32)
 {
-    constexpr int BATCH = 8;
     __shared__ __attribute__((aligned(16))) float part[8][256 + 4];
-    const int c0 = blockIdx.x * 8, tid = threadIdx.x;
-    float acc[8] = {};
-    for (int64_t l0 = tid; l0 < L; l0 += 256 * BATCH) {          // (64-bit: a step past the last row)
-        uint4 a[BATCH], b[BATCH];
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-            const int64_t l = l0 + 256 * i;
-            a[i] = b[i] = make_uint4(0u, 0u, 0u, 0u);             // (rows past the end add zeros)
-            if (l < L) {
-                a[i] = *reinterpret_cast<const uint4*>(g + l * R + c0);
-                b[i] = *reinterpret_cast<const uint4*>(xv + l * R + c0);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-            const uint32_t aw[4] = {a[i].x, a[i].y, a[i].z, a[i].w}, bw[4] = {b[i].x, b[i].y, b[i].z, b[i].w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc[2 * j] += rb(bf16_lo(aw[j]) * bf16_lo(bw[j]));
-                acc[2 * j + 1] += rb(bf16_hi(aw[j]) * bf16_hi(bw[j]));
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) part[j][tid] = acc[j];
-    __syncthreads();
-    if (tid < 8) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            float4 v[32];
-#pragma unroll
-            for (int t = 0; t < 32; ++t) v[t] = *reinterpret_cast<const float4*>(&part[tid][128 * half + 4 * t]);
-#pragma unroll
-            for (int t = 0; t < 32; ++t) sum = (((sum + v[t].x) + v[t].y) + v[t].z) + v[t].w;
-        }
-        if (out_f32) static_cast<float*>(out)[c0 + tid] = sum;
-        else static_cast<uint16_t*>(out)[c0 + tid] = (uint16_t)bf16_bits(sum);
-    }
+    scale_grad_block((int)blockIdx.x, g, xv, L, R, out, out_f32, part);
 }
 
 int scale_grad(const void* g, const void* xv, int64_t L, int64_t R, void* out, int out_dtype, hipStream_t st)

@@ -109,4 +109,50 @@ __device__ __forceinline__ void lowrank_small_finish_block(int block, const floa
     }
 }
 
+// One workgroup (256 threads) of the gradient of the rank-r scale vector: columns 8 block .. + 7 (scale_grad_kernel, lowrank_small.hip).
+__device__ __forceinline__ void scale_grad_block(int block, const uint16_t* __restrict__ g, const uint16_t* __restrict__ xv, int L, int R,
+                                                 void* __restrict__ out, int out_f32, float (&part)[8][256 + 4])
+{
+    constexpr int BATCH = 8;
+    const int c0 = block * 8, tid = threadIdx.x;
+    float acc[8] = {};
+    for (int64_t l0 = tid; l0 < L; l0 += 256 * BATCH) {          // (64-bit: a step past the last row)
+        uint4 a[BATCH], b[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int64_t l = l0 + 256 * i;
+            a[i] = b[i] = make_uint4(0u, 0u, 0u, 0u);             // (rows past the end add zeros)
+            if (l < L) {
+                a[i] = *reinterpret_cast<const uint4*>(g + l * R + c0);
+                b[i] = *reinterpret_cast<const uint4*>(xv + l * R + c0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const uint32_t aw[4] = {a[i].x, a[i].y, a[i].z, a[i].w}, bw[4] = {b[i].x, b[i].y, b[i].z, b[i].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                acc[2 * j] += rb(bf16_lo(aw[j]) * bf16_lo(bw[j]));
+                acc[2 * j + 1] += rb(bf16_hi(aw[j]) * bf16_hi(bw[j]));
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) part[j][tid] = acc[j];
+    __syncthreads();
+    if (tid < 8) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float4 v[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) v[t] = *reinterpret_cast<const float4*>(&part[tid][64 * q + 4 * t]);
+#pragma unroll
+            for (int t = 0; t < 16; ++t) sum = (((sum + v[t].x) + v[t].y) + v[t].z) + v[t].w;
+        }
+        if (out_f32) static_cast<float*>(out)[c0 + tid] = sum;
+        else static_cast<uint16_t*>(out)[c0 + tid] = (uint16_t)bf16_bits(sum);
+    }
+}
+
 }  // namespace metis

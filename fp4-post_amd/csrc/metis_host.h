@@ -212,6 +212,12 @@ size_t lowrank_tn_workspace_bytes(int64_t L, int64_t C, int64_t R);
 int lowrank_tn(const void* a, int64_t lda, const void* b, int64_t L, int64_t C, int64_t R, void* out, int out_dtype, int transpose,
                void* workspace, size_t workspace_bytes, hipStream_t st);
 
+// both of a layer's contractions over tokens and scale_grad, side by side
+size_t lowrank_backward_workspace_bytes(int64_t L, int64_t N, int64_t K, int64_t R);
+int lowrank_backward(const void* dy, int64_t lddy, const void* t, int64_t N, const void* x, int64_t ldx, const void* gxv, int64_t K, int64_t L, int64_t R,
+                     void* gu, int gu_dtype, void* gv, int gv_dtype, const void* gt, const void* xv, void* gs, int gs_dtype, void* workspace,
+                     size_t workspace_bytes, hipStream_t st);
+
 int expand_f16(const void* codes, const void* scales, int64_t rows, int64_t cols, void* out, hipStream_t st);
 int gemm_expanded(const void* a_exp, const float* a_unit, const void* b_exp, const float* b_unit, int64_t M, int64_t N,
                   int64_t K, const void* t, const void* u, int64_t r, const void* bias, void* out, int out_dtype,

@@ -97,6 +97,8 @@ SIGNATURES = {
     "metis_lowrank_project_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "metis_lowrank_project": (_i32, [_vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),
     "metis_lowrank_project_rows": (_i32, [_vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
+    "metis_lowrank_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "metis_lowrank_backward": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _sz, _vp]),
     "metis_lowrank_scale_grad": (_i32, [_vp, _vp, _i64, _i64, _vp, _i32, _vp]),
     "metis_lowrank_project_rows_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "metis_lowrank_project_rows_ws": (_i32, [_vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _sz, _vp]),

@@ -892,10 +892,9 @@ class _MetisFusedFunction(torch.autograd.Function):
         # rank-r branch in bf16: one pass over dY for dY U, one for dY^T t, one over x for g_xv^T x
         # dY U [L, r] and its product with s (the gradient with respect to x V^T) from the same launch
         g_t, g_xv = ops.lowrank_project(dy2, _MetisFusedFunction._transposed_bf16(u), s.to(cd))
-        g_u = ops.lowrank_contract_tokens(dy2, t)                           # [N, r]
-        # sum of the bf16 products, as autograd forms it for torch.mul(s, y); rounded once to the parameter's dtype
-        g_s = ops.lowrank_scale_grad(g_t, xv, out_dtype=s.dtype if s.dtype in (torch.float32, torch.bfloat16) else torch.float32)
-        g_v = ops.lowrank_contract_tokens(x2, g_xv, transpose=True)         # [r, K]
+        # g_u [N, r], g_v [r, K]; g_s: sum of the bf16 products, as autograd forms it for torch.mul(s, y), rounded once to the
+        # parameter's dtype
+        g_u, g_v, g_s = ops.lowrank_backward(dy2, t, x2, g_xv, g_t, xv, s.dtype if s.dtype in (torch.float32, torch.bfloat16) else torch.float32)
         # residual branch on re-quantized operands
         qg = F.q_backward_outputgrad
         if F._packed_backward_applies(L, N, dy2) and ctx.p_res.rht is not None:

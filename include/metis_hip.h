@@ -643,6 +643,18 @@ int metis_lowrank_contract_tokens(const void *a, int64_t lda, const void *b, int
                                   size_t workspace_bytes, void *stream);
 
 /*
+ * A layer's two contractions and the gradient of its scale vector in two launches (contractions and scale gradient side by side,
+ * then both finishing steps) instead of five; the same bits as the three calls:
+ *     gu [N, R] = dy^T t        gv [R, K] = (x^T gxv)^T        gs [R] = sum_l bf16(gt[l] * xv[l])
+ *   dy [L, N], x [L, K] with row strides; t, gxv, gt, xv [L, R] contiguous; all bf16, 16-byte aligned; L > 0, R in {32, 64, 128}
+ *   workspace metis_lowrank_backward_workspace_bytes(L, N, K, R) bytes, 16-byte aligned, no initialisation
+ */
+size_t metis_lowrank_backward_workspace_bytes(int64_t L, int64_t N, int64_t K, int64_t R);
+int metis_lowrank_backward(const void *dy, int64_t lddy, const void *t, int64_t N, const void *x, int64_t ldx, const void *gxv,
+                           int64_t K, int64_t L, int64_t R, void *gu, int gu_dtype, void *gv, int gv_dtype, const void *gt,
+                           const void *xv, void *gs, int gs_dtype, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * One packed activation against several weight matrices in one call: the q/k/v (gate/up) projections of a
  * decoder layer, which the reference quantizes the activation once for (BitLinear._get_shared_quantized_input,
  * src/Metis/Metis/bitlinear.py:676-702) and then multiplies one by one.  Result i equals

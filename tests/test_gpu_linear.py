@@ -913,6 +913,26 @@ def test_gradient_of_the_rank_r_scale_vector(L, R):
     assert torch.equal(ops.lowrank_scale_grad(g, xv, out_dtype=torch.bfloat16), got.bfloat16())
 
 
+@pytest.mark.parametrize("L,N,K,R", [(1, 8, 72, 32), (63, 64, 64, 64), (65, 136, 24, 128), (700, 200, 1544, 32), (2103, 1536, 512, 64), (4096, 64, 2048, 128)])
+def test_gradients_of_the_rank_r_branch_side_by_side(L, N, K, R):
+    """ops.lowrank_backward: both contractions over tokens and the scale gradient with the bits of the three calls."""
+    from metis_hip import ops
+    g_ = torch.Generator().manual_seed(8200 + L)
+    make = lambda *shape: torch.randn(*shape, generator=g_).bfloat16().cuda()
+    dy, x = make(L, N + 8)[:, :N], make(L, K)
+    t, gxv, gt, xv = (make(L, R) for _ in range(4))
+    for dt in (torch.float32, torch.bfloat16):
+        gu, gv, gs = ops.lowrank_backward(dy, t, x, gxv, gt, xv, dt)
+        torch.cuda.synchronize()
+        assert torch.equal(gu, ops.lowrank_contract_tokens(dy, t)) and torch.equal(gv, ops.lowrank_contract_tokens(x, gxv, transpose=True))
+        assert torch.equal(gs, ops.lowrank_scale_grad(gt, xv, out_dtype=dt))
+    # one addend in 2^24 of the largest sum: binary32 accumulation of exact products, one rounding to bf16
+    want = dy.double().T @ t.double()
+    assert float((gu.double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5
+    strided = ops.lowrank_backward(dy, make(L, R + 1)[:, :R], x, gxv, gt, xv)       # not what the kernel reads: the separate calls
+    assert strided[0].shape == (N, R) and torch.equal(strided[1], gv)
+
+
 @pytest.mark.parametrize("L,R", [(1, 8), (255, 40), (257, 32), (2047, 32), (2049, 8), (4096, 32), (5000, 64)])
 def test_gradient_of_the_rank_r_scale_vector_is_added_in_its_documented_order(L, R):
     """256 sums of every 256th row, in row order, then these in order: binary32 on the CPU in that order gives the same bits."""
