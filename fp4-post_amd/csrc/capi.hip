@@ -306,6 +306,23 @@ int metis_nvfp4_quant_row_rht(const void* x, int64_t rows, int64_t cols, int64_t
                         (hipStream_t)stream);
 }
 
+int metis_nvfp4_quant_sr_both_copy(const void* x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld, uint64_t seed, uint64_t offset_row,
+                                   uint64_t offset_col, void* codes_row, void* scales_row, float* unit_row, void* codes_col, void* scales_col,
+                                   float* unit_col, void* copy, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (rows < 0 || rows > padded_rows || !copy) return METIS_E_ARG;
+    return quantize_both_sr(x, padded_rows, cols, ld, METIS_MODE_P32_F32, seed, offset_row, offset_col, codes_row, scales_row, unit_row, codes_col,
+                            scales_col, unit_col, workspace, workspace_bytes, (hipStream_t)stream, rows, copy);
+}
+
+int metis_nvfp4_quant_row_rht_copy(const void* x, int64_t rows, int64_t cols, int64_t ld, uint32_t sign_mask, int sr, uint64_t seed, uint64_t offset,
+                                   void* codes, void* scales, float* unit, void* copy, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (!copy) return METIS_E_ARG;
+    return quantize_rht(x, rows, cols, ld, METIS_MODE_P32_F32, sign_mask, sr != 0, seed, offset, codes, scales, unit, workspace, workspace_bytes,
+                        (hipStream_t)stream, copy);
+}
+
 int metis_hadamard16(const void* x, int64_t rows, int64_t cols, int64_t ldx, int dtype, int inverse, uint32_t sign_mask, void* out,
                      int64_t ldo, void* stream)
 {

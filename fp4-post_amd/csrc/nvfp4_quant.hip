@@ -176,12 +176,15 @@ __global__ __launch_bounds__(256) void quant_codes_contig_centered_kernel(const 
 // `_quantize_wgrad_operand` and `_get_quantized_weight` of src/Metis/Metis/bitlinear.py:395-405, 577-585.  In bf16
 // arithmetic the rotated values are rounded to bf16 (the reference's rotation returns the input dtype); in binary32
 // arithmetic they are binary32 values that need not be bf16 values, hence WIDE.
+// copy (HAD, binary32 input): the tensor itself rounded to bf16, [rows, cols] contiguous: the rank-r branch of the backward pass reads
+// a binary32 output gradient in bf16, and a conversion of its own would read all of it once more (45 us at 4096 x 8960; the step of
+// that projection, 1536 -> 8960, under the NV recipe: 597 us with it, 582 with the copy from here).
 template <int MODE, bool SR, bool WIDE = false, bool HAD = false>
 __global__ __launch_bounds__(256) void quant_codes_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, const void* __restrict__ noise,
     uint64_t seed, uint64_t offset, uint2* __restrict__ codes, void* __restrict__ ws_amax_v,
     uint32_t* __restrict__ ws_gmax, uint32_t nblocks, int in_f32, const void* __restrict__ center, uint32_t sign_mask,
-    uint32_t fill_to)
+    uint32_t fill_to, uint4* __restrict__ copy = nullptr)
 {
     static_assert(!WIDE || MODE == 0, "binary32 values imply binary32 arithmetic");
     static_assert(!HAD || WIDE || MODE == 1, "rotated binary32 values are not bf16 values");
@@ -198,6 +201,12 @@ __global__ __launch_bounds__(256) void quant_codes_kernel(
             for (int c = 0; c < 4; ++c) {
                 const float4 f = p[c];
                 v[4 * c] = f.x; v[4 * c + 1] = f.y; v[4 * c + 2] = f.z; v[4 * c + 3] = f.w;
+            }
+            if constexpr (HAD) {
+                if (copy) {
+                    copy[2 * (size_t)i] = make_uint4(rb_pair(v[0], v[1]), rb_pair(v[2], v[3]), rb_pair(v[4], v[5]), rb_pair(v[6], v[7]));
+                    copy[2 * (size_t)i + 1] = make_uint4(rb_pair(v[8], v[9]), rb_pair(v[10], v[11]), rb_pair(v[12], v[13]), rb_pair(v[14], v[15]));
+                }
             }
         } else {
             const uint4* p = reinterpret_cast<const uint4*>(x + (int64_t)row * ld + (int64_t)cb * kBlock);
@@ -481,13 +490,14 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
 // Same tile as the column kernel (256 rows x 64 columns per workgroup, wave g takes 16-row slabs 4g .. 4g+3): a lane
 // holds one column of a slab; the slab also goes through LDS (68-word rows) and comes back as row blocks, lane l
 // taking row l / 4, block l % 4.  Both packings share the tensor maximum, hence one partial maximum per workgroup.
+// copy (binary32 input): the tensor rounded to bf16 as well, as in quant_codes_kernel.
 // ---------------------------------------------------------------------------------------------
 constexpr uint32_t kBothRun = 16;
 template <int MODE, bool WIDE = false>
-__global__ __launch_bounds__(256) void quant_codes_both_kernel(
+__global__ __launch_bounds__(256, 5) void quant_codes_both_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, uint64_t seed, uint64_t offset_row, uint64_t offset_col,
     uint2* __restrict__ codes_row, void* __restrict__ amax_row_v, uint2* __restrict__ codes_col, void* __restrict__ amax_col_v,
-    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, uint32_t valid)
+    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, uint32_t valid, uint16_t* __restrict__ copy = nullptr)
 {
     static_assert(!WIDE || MODE == 0, "binary32 values imply binary32 arithmetic");
     using amax_t = typename std::conditional<WIDE, float, uint16_t>::type;
@@ -559,6 +569,16 @@ __global__ __launch_bounds__(256) void quant_codes_both_kernel(
                 for (int i = 0; i < NQ; ++i) *reinterpret_cast<uint4*>(&slab[g][i * RPI + lrow][lch * 4u]) = cur[i];
                 __builtin_amdgcn_wave_barrier();
                 if constexpr (WIDE) {
+                    const uint32_t col = tc * kColTileCols + lch * 4u;
+                    if (copy && col < cols) {                  // as loaded: 128 consecutive bytes of a row per 16 lanes
+#pragma unroll
+                        for (int i = 0; i < NQ; ++i) {
+                            const uint32_t row = b * kBlock + i * RPI + lrow;
+                            if (row < valid)
+                                *reinterpret_cast<uint2*>(copy + (size_t)row * cols + col) =
+                                    make_uint2(rb_pair(__uint_as_float(cur[i].x), __uint_as_float(cur[i].y)), rb_pair(__uint_as_float(cur[i].z), __uint_as_float(cur[i].w)));
+                        }
+                    }
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         const uint4 f = *reinterpret_cast<const uint4*>(&slab[g][rr][cb * kBlock + 4 * q]);
@@ -1184,7 +1204,8 @@ static void launch_contig(const void* x, void* codes, const Workspace& ws, uint3
 template <int MODE, bool SR, bool COL, bool WIDE = false, bool HAD = false>
 static int launch_quant(const void* x, int64_t rows, int64_t cols, int64_t ld, const void* noise, uint64_t seed,
                         uint64_t offset, void* codes, void* scales, float* unit, const Workspace& ws, hipStream_t st,
-                        int in_f32 = 0, const void* center = nullptr, uint32_t sign_mask = 0, void* decode = nullptr, int64_t valid = -1)
+                        int in_f32 = 0, const void* center = nullptr, uint32_t sign_mask = 0, void* decode = nullptr, int64_t valid = -1,
+                        void* copy = nullptr)
 {
     static_assert(!HAD || !COL, "the rotation runs along the last dimension, as the row blocks do");
     const uint32_t nblocks = (uint32_t)(rows * cols / kBlock);
@@ -1237,7 +1258,7 @@ static int launch_quant(const void* x, int64_t rows, int64_t cols, int64_t ld, c
         const int g1 = grid_for(nblocks);
         hipLaunchKernelGGL((quant_codes_kernel<MODE, SR, WIDE, HAD>), dim3(g1), dim3(256), 0, st, x, (uint32_t)rows,
                            (uint32_t)cols, ld, noise, seed, offset, (uint2*)codes, (void*)ws.amax, ws.gmax, nblocks, in_f32, center,
-                           sign_mask, 0u);
+                           sign_mask, 0u, (uint4*)copy);
         return launch_scales(WIDE ? METIS_MODE_P32_F32 : MODE, ws, (uint32_t)g1, scales, unit, nblocks, st);
     }
 }
@@ -1347,9 +1368,10 @@ static int both_capacity()
 // ---------------------------------------------------------------------------------------------
 int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, uint64_t seed, uint64_t offset_row,
                      uint64_t offset_col, void* codes_row, void* scales_row, float* unit_row, void* codes_col, void* scales_col,
-                     float* unit_col, void* workspace, size_t bytes, hipStream_t st, int64_t valid)
+                     float* unit_col, void* workspace, size_t bytes, hipStream_t st, int64_t valid, void* copy)
 {
     if (rows < 0 || cols < 0 || ld < cols || valid > rows) return METIS_E_ARG;
+    if (copy && (mode != METIS_MODE_P32_F32 || ((uintptr_t)copy % 16))) return METIS_E_ARG;
     if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16 && mode != METIS_MODE_P32_F32) return METIS_E_ARG;
     const bool f32in = mode == METIS_MODE_P32_F32;
     if (rows % kBlock || cols % kBlock) return METIS_E_SHAPE;
@@ -1374,7 +1396,7 @@ int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int 
     if (g > kMaxGroups) g = kMaxGroups;
 #define METIS_QB(M, W) hipLaunchKernelGGL((quant_codes_both_kernel<M, W>), dim3((unsigned)g), dim3(256), 0, st, x, (uint32_t)rows, \
                                           (uint32_t)cols, ld, seed, offset_row, offset_col, (uint2*)codes_row, (void*)wr.amax, (uint2*)codes_col, \
-                                          (void*)wc.amax, wr.gmax, tiles_c, (uint32_t)tiles, (uint32_t)(valid < 0 ? rows : valid))
+                                          (void*)wc.amax, wr.gmax, tiles_c, (uint32_t)tiles, (uint32_t)(valid < 0 ? rows : valid), (uint16_t*)copy)
     if (f32in) METIS_QB(0, true);
     else if (mode == 0) METIS_QB(0, false);
     else METIS_QB(1, false);
@@ -1719,9 +1741,10 @@ int quantize_lowrank_residual(const void* x, bool x_f32, const void* us, const v
 // in one pass over x.  Round to nearest, or stochastic rounding on the library's own stream.
 // ---------------------------------------------------------------------------------------------
 int quantize_rht(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, uint32_t sign_mask, bool sr, uint64_t seed,
-                 uint64_t offset, void* codes, void* scales, float* unit, void* workspace, size_t workspace_bytes, hipStream_t st)
+                 uint64_t offset, void* codes, void* scales, float* unit, void* workspace, size_t workspace_bytes, hipStream_t st, void* copy)
 {
     if (rows < 0 || cols < 0 || ld < cols || sign_mask > 0xffffu) return METIS_E_ARG;
+    if (copy && (mode != METIS_MODE_P32_F32 || ((uintptr_t)copy % 16))) return METIS_E_ARG;
     if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16 && mode != METIS_MODE_P32_F32) return METIS_E_ARG;
     const bool f32in = mode == METIS_MODE_P32_F32;
     if (cols % kBlock) return METIS_E_SHAPE;
@@ -1733,7 +1756,7 @@ int quantize_rht(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode
     Workspace ws;
     if (const int rc = carve_workspace(workspace, workspace_bytes, rows, cols, &ws)) return rc;
 #define METIS_QH(M, S, W) return launch_quant<M, S, false, W, true>(x, rows, cols, ld, nullptr, seed, offset, codes, scales, unit, ws, st, \
-                                                                    f32in, nullptr, sign_mask)
+                                                                    f32in, nullptr, sign_mask, nullptr, -1, copy)
     if (mode == METIS_MODE_PB16) { if (sr) METIS_QH(1, true, false); else METIS_QH(1, false, false); }
     if (sr) METIS_QH(0, true, true); else METIS_QH(0, false, true);
 #undef METIS_QH

@@ -440,7 +440,7 @@ class LinearLowbitFunction(torch.autograd.Function):
         return F.quantize_input(input_, mean_cache=mean_cache, cache_key=cache_key)
 
     @staticmethod
-    def _packed_grads(dy2, x2, pw_col, center_x, gx_dtype, gw_dtype, gx_lowrank=None, center_x32=None):
+    def _packed_grads(dy2, x2, pw_col, center_x, gx_dtype, gw_dtype, gx_lowrank=None, center_x32=None, packed_dy=None):
         """(grad_input [L, K], grad_weight [N, K]) on packed operands.  dgrad contracts over N, wgrad over tokens.
 
         Direct mode: dY^ = SR-Q(dY).  Mean mode (enable_backward_svd): dY^ = 1 me_dy^T + SR-Q(dY - me_dy)
@@ -451,7 +451,7 @@ class LinearLowbitFunction(torch.autograd.Function):
             gW = R_dy^T R_x + (sum_l R_dy) center_x^T + me_dy (sum_l R_x + L center_x)^T
         gx_lowrank = (t [L, r], u [K, r]) adds t u^T to grad_input inside the same launch (the rank-r branch's share).
         center_x32: center_x as float32 when the caller has it (the matrix-vector products read binary32: each use of the
-        bf16 one is a conversion launch).
+        bf16 one is a conversion launch).  packed_dy: both packings of dY when the caller has them (_pack_gradient).
         """
         F = LinearLowbitFunction
         cd = F.compute_dtype
@@ -471,7 +471,9 @@ class LinearLowbitFunction(torch.autograd.Function):
             more["pad_rows"] = L + (-L) % 32
             # the row quantizer's 16-byte loads: a gradient that starts elsewhere is copied
             dy2 = dy2 if dy2.data_ptr() % 16 == 0 else dy2.clone()
-        if me_dy is None and hasattr(qg, "pack_both"):
+        if packed_dy is not None:
+            p_dy, p_dyt = packed_dy
+        elif me_dy is None and hasattr(qg, "pack_both"):
             p_dy, p_dyt = qg.pack_both(dy2, arith=cd, **more)  # one pass over dY for both products
         else:
             p_dy, p_dyt = qg.pack(dy2, arith=cd, center=me_dy, **more), None
@@ -498,7 +500,28 @@ class LinearLowbitFunction(torch.autograd.Function):
         return gx, ops.linear_fwd(p_dyt, p_xt, t=t, u=u, out_dtype=gw_dtype)
 
     @staticmethod
-    def _packed_grads_nv(dy2, x2, pw, gx_dtype, gw_dtype, gx_lowrank=None):
+    def _pack_gradient(dy: torch.Tensor, rht):
+        """(packed dY, dY in bf16) from one pass over a binary32 output gradient in binary32 arithmetic -- what _packed_grads (both
+        packings, rht None) or _packed_grads_nv would pack, and the rounded tensor that the rank-r branch reads -- or None."""
+        F = LinearLowbitFunction
+        qg = F.q_backward_outputgrad
+        L, N = dy.shape
+        if (dy.dtype != torch.float32 or F.compute_dtype != torch.float32 or not dy.is_cuda or not dy.is_contiguous() or dy.data_ptr() % 16
+                or N % 32 or L == 0 or F.enable_backward_svd or not is_hip_nvfp4(qg)):
+            return None
+        pad = (-L) % 32
+        if rht is not None and pad:
+            return None                                        # filled up by a copy before it is packed
+        more = {"pad_rows": L + pad} if pad else {}
+        if rht is None and not qg.packs_both_at_once(dy, more.get("pad_rows")):
+            return None
+        rounded = torch.empty(L, N, dtype=torch.bfloat16, device=dy.device)
+        if rht is not None:
+            return qg.pack(dy, arith=torch.float32, rht=rht, bf16_copy=rounded), rounded
+        return qg.pack_both(dy, arith=torch.float32, bf16_copy=rounded, **more), rounded
+
+    @staticmethod
+    def _packed_grads_nv(dy2, x2, pw, gx_dtype, gw_dtype, gx_lowrank=None, packed_dy=None):
         """(grad_input, grad_weight) of the NV recipe (reference 443-513 with 395-405, 495-501) without leaving the
         packed kernels.  The reference rotates dY and the saved (already quantized) input tile by tile along their
         last dimension, quantizes, dequantizes and rotates back, and multiplies the results:
@@ -521,7 +544,7 @@ class LinearLowbitFunction(torch.autograd.Function):
             x2 = torch.cat((x2, x2.new_zeros(pad, K)), dim=0)
             if lt is not None:
                 lt = torch.cat((lt, lt.new_zeros(pad, lt.shape[1])), dim=0)
-        p_dy = F.q_backward_outputgrad.pack(dy2, arith=cd, rht=mask)
+        p_dy = packed_dy if packed_dy is not None else F.q_backward_outputgrad.pack(dy2, arith=cd, rht=mask)
         xq = F.q_forward_input.pack(x2, arith=cd).dequantize(torch.float32 if cd == torch.float32 else torch.bfloat16)
         p_x = F.q_backward_input.pack(xq, arith=cd, rht=mask)
         a_dy = ops.expand_tiled(p_dy, cache=False, mode=gmode)
@@ -886,7 +909,13 @@ class _MetisFusedFunction(torch.autograd.Function):
         F._check_backward_config()
         x, v, s, u, res, xv, t = ctx.saved_tensors
         cd = torch.bfloat16
-        dy2 = _flat2d(dy).to(cd)
+        packed_dy = None
+        if dy.dtype == torch.float32 and F._packed_backward_applies(*_flat2d(dy).shape, dy):
+            both = F._pack_gradient(_flat2d(dy), ctx.p_res.rht)          # the quantizer's pass leaves the bf16 tensor as well
+            if both is not None:
+                packed_dy, dy2 = both
+        if packed_dy is None:
+            dy2 = _flat2d(dy).to(cd)
         x2 = _flat2d(x).to(cd)
         L, N = dy2.shape
         # rank-r branch in bf16: one pass over dY for dY U, one for dY^T t, one over x for g_xv^T x
@@ -902,7 +931,7 @@ class _MetisFusedFunction(torch.autograd.Function):
             ar = F.compute_dtype
             dyq, xq_src = (_flat2d(dy), _flat2d(x)) if ar == torch.float32 else (dy2, x2)
             gx, g_res = F._packed_grads_nv(dyq, xq_src, ctx.p_res, cd, torch.bfloat16 if res.dtype == torch.bfloat16 else torch.float32,
-                                           gx_lowrank=(g_xv, _MetisFusedFunction._transposed_bf16(v)))
+                                           gx_lowrank=(g_xv, _MetisFusedFunction._transposed_bf16(v)), packed_dy=packed_dy)
         elif F._packed_backward_applies(L, N, dy2):
             ar = F.compute_dtype                               # arithmetic of the quantizers
             p_res_col = ctx.p_res.transposed                   # lives as long as the (cached) packed residual
@@ -913,7 +942,8 @@ class _MetisFusedFunction(torch.autograd.Function):
             # the rank-r branch's share of grad_input, g_xv V, rides in the dgrad launch as its low-rank extension
             gx, g_res = F._packed_grads(dyq, xq_src, p_res_col, ctx.center, cd,
                                         torch.bfloat16 if res.dtype == torch.bfloat16 else torch.float32,
-                                        gx_lowrank=(g_xv, _MetisFusedFunction._transposed_bf16(v)), center_x32=ctx.center32)
+                                        gx_lowrank=(g_xv, _MetisFusedFunction._transposed_bf16(v)), center_x32=ctx.center32,
+                                        packed_dy=packed_dy)
         else:
             gx = torch.matmul(g_xv, v.to(cd))                  # [L, K]
             cdt = F.compute_dtype

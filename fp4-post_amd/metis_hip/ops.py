@@ -458,13 +458,22 @@ def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tenso
     return PackedNVFP4(codes, scales, unit, rows, cols, mode), out
 
 
+def _check_bf16_copy(copy: torch.Tensor | None, x2: torch.Tensor, kmode: int) -> None:
+    if copy is not None and (kmode != _lib.MODE_P32_F32 or copy.dtype != torch.bfloat16 or copy.shape != x2.shape or not copy.is_contiguous()
+                             or copy.device != x2.device):
+        raise ValueError("bf16_copy: a contiguous bfloat16 tensor of the flattened shape, for a binary32 tensor in binary32 arithmetic")
+
+
 def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, offset_row: int = 0,
-                     offset_col: int = 0, pad_rows: int | None = None) -> tuple[PackedNVFP4, PackedNVFP4]:
+                     offset_col: int = 0, pad_rows: int | None = None,
+                     bf16_copy: torch.Tensor | None = None) -> tuple[PackedNVFP4, PackedNVFP4]:
     """(quantize(x, sr=True, offset=offset_row), quantize(x, col=True, sr=True, offset=offset_col)) from ONE pass over x:
     the two packings of an output gradient that the input-gradient and weight-gradient products contract.  Same
     bytes as the two calls.  Both dimensions of x flattened to [R, C] have to be multiples of 16; with pad_rows, that
-    and C: the column packing is that of x filled up with zero rows to pad_rows, the row packing that of x."""
+    and C: the column packing is that of x filled up with zero rows to pad_rows, the row packing that of x.
+    bf16_copy (a binary32 x in binary32 arithmetic): bf16 [R, C], contiguous: the same pass leaves x.to(bfloat16) in it."""
     x2, kmode = _as_2d_for_quant(x, mode)
+    _check_bf16_copy(bf16_copy, x2, kmode)
     have, cols = x2.shape
     rows = have if pad_rows is None else pad_rows
     if rows < have:
@@ -485,7 +494,13 @@ def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, of
         ws = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=dev).fill_(0)
         _workspaces[key] = ws
     (cr, sr_, ur), (cc, sc, uc) = packs
-    if rows * cols:
+    if bf16_copy is not None and rows * cols:
+        rc = L.metis_nvfp4_quant_sr_both_copy(x2.data_ptr(), have, rows, cols, x2.stride(0), seed & (2 ** 64 - 1), offset_row, offset_col,
+                                              cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(), uc.data_ptr(),
+                                              bf16_copy.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
+        if rc:
+            check(rc, "metis_nvfp4_quant_sr_both_copy", x.shape)
+    elif rows * cols:
         rc = L.metis_nvfp4_quant_sr_both_padded(x2.data_ptr(), have, rows, cols, x2.stride(0), kmode, seed & (2 ** 64 - 1), offset_row,
                                                 offset_col, cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(),
                                                 uc.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
@@ -527,10 +542,12 @@ def hadamard16(x: torch.Tensor, sign_mask: int, inverse: bool = False) -> torch.
     return out.reshape(x.shape)
 
 
-def quantize_rht(x: torch.Tensor, mode: int, sign_mask: int, *, sr: bool = False, seed: int = 0, offset: int = 0) -> PackedNVFP4:
+def quantize_rht(x: torch.Tensor, mode: int, sign_mask: int, *, sr: bool = False, seed: int = 0, offset: int = 0,
+                 bf16_copy: torch.Tensor | None = None) -> PackedNVFP4:
     """Row quantizer of the ROTATED tensor (NV recipe): rotation and quantization in one pass over x.  The result
-    carries `rht` = sign_mask; its dequantize() and tiled expansions rotate back."""
+    carries `rht` = sign_mask; its dequantize() and tiled expansions rotate back.  bf16_copy: as in quantize_both_sr."""
     x2, kmode = _as_2d_for_quant(x, mode)
+    _check_bf16_copy(bf16_copy, x2, kmode)
     rows, cols = x2.shape
     if cols % BLOCK:
         raise ValueError(f"last dimension {cols} is not a multiple of {BLOCK}")
@@ -539,6 +556,13 @@ def quantize_rht(x: torch.Tensor, mode: int, sign_mask: int, *, sr: bool = False
     scales = torch.empty(rows, cols // BLOCK, dtype=torch.uint8, device=dev)
     unit = torch.empty(1, dtype=torch.float32, device=dev)
     ws = _workspace(rows, cols, dev)
+    if bf16_copy is not None:
+        rc = load().metis_nvfp4_quant_row_rht_copy(x2.data_ptr(), rows, cols, x2.stride(0), int(sign_mask), int(sr), int(seed), int(offset),
+                                                   codes.data_ptr(), scales.data_ptr(), unit.data_ptr(), bf16_copy.data_ptr(), ws.data_ptr(),
+                                                   ws.numel(), _stream())
+        if rc:
+            check(rc, "metis_nvfp4_quant_row_rht_copy", (rows, cols))
+        return PackedNVFP4(codes, scales, unit, rows, cols, MODE_P32, rht=int(sign_mask))
     rc = load().metis_nvfp4_quant_row_rht(x2.data_ptr(), rows, cols, x2.stride(0), kmode, int(sign_mask), int(sr), int(seed), int(offset),
                                           codes.data_ptr(), scales.data_ptr(), unit.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
     if rc:

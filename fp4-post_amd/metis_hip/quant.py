@@ -88,21 +88,22 @@ class _NVFP4Base(BlockQuantFunc):
     @classmethod
     def pack(cls, x: torch.Tensor, col: bool = False, noise: torch.Tensor | None = None,
              arith: torch.dtype | None = None, center: torch.Tensor | None = None, rht: int | None = None,
-             deferred: bool = False, pad_rows: int | None = None) -> ops.PackedNVFP4:
+             deferred: bool = False, pad_rows: int | None = None, bf16_copy: torch.Tensor | None = None) -> ops.PackedNVFP4:
         """Packed NVFP4 (codes, E4M3 scale bytes, unit) of x in the arithmetic of x's dtype, or of `arith`
         when given: a bf16 tensor packed with arith=float32 gives what x.float() would, without the copy.
         center: per-column vector subtracted first (mean mode): the packed tensor is that of x - center.
         rht: sign mask of the NV recipe's rotation: the packed tensor is that of the rotated x (see ops.quantize_rht).
         deferred: round-to-nearest rows only: one launch now, the scale bytes when (and if) somebody reads them (ops.quantize).
         pad_rows: x stands for a tensor of pad_rows rows whose rows beyond x's own have a zero residual: col=True packs that
-        tensor, row blocks are those of x; either way the random stream advances as for the larger tensor."""
+        tensor, row blocks are those of x; either way the random stream advances as for the larger tensor.
+        bf16_copy (with rht): see ops.quantize_rht."""
         if torch.is_grad_enabled():
             with torch.no_grad():
-                return cls._pack(x, col, noise, arith, center, rht, deferred, pad_rows)
-        return cls._pack(x, col, noise, arith, center, rht, deferred, pad_rows)
+                return cls._pack(x, col, noise, arith, center, rht, deferred, pad_rows, bf16_copy)
+        return cls._pack(x, col, noise, arith, center, rht, deferred, pad_rows, bf16_copy)
 
     @classmethod
-    def _pack(cls, x, col, noise, arith, center, rht, deferred, pad_rows) -> ops.PackedNVFP4:
+    def _pack(cls, x, col, noise, arith, center, rht, deferred, pad_rows, bf16_copy=None) -> ops.PackedNVFP4:
         _need_gpu(x)
         drawn = x.numel() if pad_rows is None else pad_rows * x.shape[-1]
         more = {"pad_rows": pad_rows} if (col and pad_rows is not None) else {}
@@ -113,27 +114,40 @@ class _NVFP4Base(BlockQuantFunc):
             # NV recipe: the tensor is rotated tile by tile along its last dimension first (sign mask rht); row blocks only
             if col or noise is not None or center is not None:
                 raise ValueError("a rotated tensor is packed along its last dimension, without caller noise or centre")
+            copy = {} if bf16_copy is None else {"bf16_copy": bf16_copy}
             if cls.stochastic:
-                return ops.quantize_rht(x, mode, rht, sr=True, seed=_NVFP4Base.sr_seed, offset=cls._next_offset(x.numel()))
-            return ops.quantize_rht(x, mode, rht)
+                return ops.quantize_rht(x, mode, rht, sr=True, seed=_NVFP4Base.sr_seed, offset=cls._next_offset(x.numel()), **copy)
+            return ops.quantize_rht(x, mode, rht, **copy)
+        if bf16_copy is not None:
+            raise ValueError("bf16_copy: with the rotating quantizer, or in pack_both")
         if cls.stochastic:
             return ops.quantize(x, mode, col=col, sr=True, noise=noise, seed=_NVFP4Base.sr_seed,
                                 offset=cls._next_offset(drawn) if noise is None else 0, center=center, **more)
         return ops.quantize(x, mode, col=col, center=center, deferred=deferred, **more)
 
     @classmethod
+    def packs_both_at_once(cls, x: torch.Tensor, pad_rows: int | None = None) -> bool:
+        """pack_both(x) is one pass over x."""
+        rows = x.numel() // x.shape[-1] if x.numel() else 0
+        return cls.stochastic and rows > 0 and (pad_rows or rows) % 16 == 0 and x.dtype in (torch.bfloat16, torch.float32)
+
+    @classmethod
     @torch.no_grad()
     def pack_both(cls, x: torch.Tensor, arith: torch.dtype | None = None,
-                  pad_rows: int | None = None) -> tuple[ops.PackedNVFP4, ops.PackedNVFP4]:
+                  pad_rows: int | None = None, bf16_copy: torch.Tensor | None = None) -> tuple[ops.PackedNVFP4, ops.PackedNVFP4]:
         """(pack(x), pack(x, col=True)): the same two tensors, and under stochastic rounding the same draws in the same
         order, from one pass over x where the kernels have one (stochastic rounding, both dimensions multiples of 16).
-        pad_rows: as in pack."""
+        pad_rows: as in pack.  bf16_copy: see ops.quantize_both_sr; only where that one pass is taken (packs_both_at_once)."""
         _need_gpu(x)
         cls._check(x)
         rows = x.numel() // x.shape[-1] if x.numel() else 0
         more = {} if pad_rows is None else {"pad_rows": pad_rows}
         drawn = x.numel() if pad_rows is None else pad_rows * x.shape[-1]
-        if cls.stochastic and rows and (pad_rows or rows) % 16 == 0 and x.dtype in (torch.bfloat16, torch.float32):
+        if bf16_copy is not None:
+            if not cls.packs_both_at_once(x, pad_rows):
+                raise ValueError("bf16_copy: only where both packings come from one pass")
+            more["bf16_copy"] = bf16_copy
+        if cls.packs_both_at_once(x, pad_rows):
             mode = _mode_of(x) if arith is None else (MODE_P32 if arith == torch.float32 else MODE_PB16)
             first = cls._next_offset(drawn)
             second = cls._next_offset(drawn)

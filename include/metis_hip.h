@@ -421,6 +421,18 @@ int metis_nvfp4_quant_row_rht(const void *x, int64_t rows, int64_t cols, int64_t
                               uint32_t sign_mask, int sr, uint64_t seed, uint64_t offset, void *codes,
                               void *scales, float *unit, void *workspace, size_t workspace_bytes,
                               void *stream);
+/*
+ * metis_nvfp4_quant_sr_both_padded and metis_nvfp4_quant_row_rht of a binary32 tensor (METIS_MODE_P32_F32) that also leave the
+ * tensor rounded to bf16: copy bf16 [rows, cols], contiguous, 16-byte aligned.  The rank-r branch of a backward pass reads the
+ * output gradient in bf16 whatever the quantizers' arithmetic is.
+ */
+int metis_nvfp4_quant_sr_both_copy(const void *x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld, uint64_t seed,
+                                   uint64_t offset_row, uint64_t offset_col, void *codes_row, void *scales_row, float *unit_row,
+                                   void *codes_col, void *scales_col, float *unit_col, void *copy, void *workspace,
+                                   size_t workspace_bytes, void *stream);
+int metis_nvfp4_quant_row_rht_copy(const void *x, int64_t rows, int64_t cols, int64_t ld, uint32_t sign_mask, int sr,
+                                   uint64_t seed, uint64_t offset, void *codes, void *scales, float *unit, void *copy,
+                                   void *workspace, size_t workspace_bytes, void *stream);
 int metis_nvfp4_expand_tiled_rht(const void *codes, const void *scales, const float *unit, int64_t rows,
                                  int64_t cols, int mode, uint32_t sign_mask, int rotate_back,
                                  int transpose, void *out, void *stream);

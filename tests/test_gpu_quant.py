@@ -771,3 +771,32 @@ def test_both_packings_of_a_whole_row_count_are_tensors_of_their_own(ops):
     assert all(t_._base is None for t_ in (row.codes, row.scales, col.codes, col.scales))
     padded, _ = ops.quantize_both_sr(x[:50], 0, seed=1, pad_rows=64)
     assert (padded.rows, padded.codes.shape[0], padded.scales.shape[0]) == (50, 50, 50)
+
+
+# whole tiles of 256 x 64, remainders in rows and columns, a padded token count
+@pytest.mark.parametrize("rows,cols,pad", [(256, 64, None), (272, 96, None), (32, 2080, None), (411, 160, 416), (2048, 1536, None)])
+def test_quantizers_of_a_binary32_gradient_leave_its_bf16_rounding(ops, rows, cols, pad):
+    """bf16_copy of quantize_both_sr and quantize_rht: the packings of the plain calls, and x.to(bfloat16)."""
+    x = _f32_valued(rows * 3 + cols, rows, cols).cuda()
+    x.view(-1)[::89] = -0.0
+    x.view(-1)[5] = 1e-39
+    want = x.bfloat16()
+    more = {} if pad is None else {"pad_rows": pad}
+    copy = torch.full((rows, cols), 7.0, dtype=torch.bfloat16, device="cuda")
+    plain = ops.quantize_both_sr(x, 0, seed=3, offset_row=5, offset_col=1 << 30, **more)
+    got = ops.quantize_both_sr(x, 0, seed=3, offset_row=5, offset_col=1 << 30, bf16_copy=copy, **more)
+    torch.cuda.synchronize()
+    for a, b in zip(plain, got):
+        assert torch.equal(a.codes, b.codes) and torch.equal(a.scales, b.scales) and torch.equal(a.unit, b.unit)
+    assert same_bits(copy.cpu(), want.cpu())
+    copy.fill_(7.0)
+    for sr in (False, True):
+        a = ops.quantize_rht(x, 0, 0x5A3C, sr=sr, seed=3, offset=11)
+        b = ops.quantize_rht(x, 0, 0x5A3C, sr=sr, seed=3, offset=11, bf16_copy=copy)
+        torch.cuda.synchronize()
+        assert torch.equal(a.codes, b.codes) and torch.equal(a.scales, b.scales) and torch.equal(a.unit, b.unit)
+        assert same_bits(copy.cpu(), want.cpu())
+    with pytest.raises(ValueError):
+        ops.quantize_rht(x.bfloat16(), 0, 1, bf16_copy=copy)
+    with pytest.raises(ValueError):
+        ops.quantize_both_sr(x, 0, bf16_copy=copy.float(), **more)
