@@ -123,11 +123,10 @@ int metis_nvfp4_quant_dequant_row_f32(const void* x, int64_t rows, int64_t cols,
     return quantize_dequantize_row(x, rows, cols, METIS_MODE_P32_F32, codes, scales, unit, out, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
-size_t metis_nvfp4_roundtrip_workspace_bytes(int64_t rows, int64_t cols, int mode) { return roundtrip_workspace_bytes(rows, cols, mode); }
-
-int metis_nvfp4_roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, void* workspace, size_t workspace_bytes, void* stream)
+int metis_nvfp4_roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, void* workspace, size_t workspace_bytes, uint32_t spin_limit,
+                          void* stream)
 {
-    return roundtrip(x, rows, cols, mode, out, workspace, workspace_bytes, (hipStream_t)stream);
+    return roundtrip(x, rows, cols, mode, out, workspace, workspace_bytes, spin_limit, (hipStream_t)stream);
 }
 
 int metis_nvfp4_quant_row_static(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, void* codes, void* scales,

@@ -12,6 +12,7 @@
 #include "metis_device.h"
 #include "metis_host.h"
 #include "nvfp4_encode.h"
+#include "grid_max.h"
 #include "lowrank_small_steps.h"
 #include <atomic>
 #include <stdio.h>
@@ -761,92 +762,9 @@ __global__ __launch_bounds__(256) void quant_scales_f32_kernel(const float* __re
 // keeps the maxima of its (at most NB) blocks in registers across a grid-wide maximum, so in the ordinary case neither
 // the parked maxima nor a second launch are needed.
 //
-// The grid-wide maximum does not assume that all workgroups are resident together.  Workgroups arrive through a
-// two-level tree (64 groups of up to 64 workgroups) whose nodes are a maximum and an arrival counter, each updated by one
-// read-modify-write, so exactly one workgroup learns that it is the LAST to arrive and what the tensor maximum is.  It
-// exchanges {call tag, result, maximum} into 64 words (one per group, a line each), writes the tensor unit, and cleans
-// the tree for the next call.  Every other workgroup polls its group's word a bounded number of times.  One that gives
-// up -- because part of the grid is still waiting for a compute unit, held by another kernel or by these very pollers
-// -- parks its block maxima in the workspace, raises its flag, swaps {call tag, "somebody left"} into its group's word
-// and exits WITHOUT its scale bytes: the last workgroup finds that marker in what its exchange returns and writes
-// those bytes itself.  If the exchange came first, the leaver's swap fails, it reads the result and finishes its own
-// bytes after all.  That decision hangs on one word, so relaxed device-scope atomics suffice on the ordinary path (an
-// acquire or release at device scope writes back or invalidates a whole L2 on this part); only a workgroup that leaves
-// and the last workgroup that cleans up after one pay for fences.  Every wave exits after a bounded time whatever else
-// runs on the device, and the result is always complete and always the same bytes as the two-launch path.
-// The area starts zero-filled; a call leaves the tree clean and only tagged words behind.
+// The grid-wide maximum is the protocol of grid_max.h; a workgroup that leaves parks its block maxima in the workspace, and what it
+// leaves behind are its scale bytes.
 // ---------------------------------------------------------------------------------------------
-constexpr uint32_t kSpinLimit = 4096;            // polls (roughly a microsecond each) before a workgroup leaves its scale bytes behind
-constexpr uint32_t kGroups = 64;                 // groups, and the most members a group can have
-constexpr int kFusedMaxGrid = kGroups * kGroups;
-// locations inside the synchronisation area (uint32 units)
-__device__ __forceinline__ uint64_t* sync_generation(uint32_t* s) { return reinterpret_cast<uint64_t*>(s); }
-__device__ __forceinline__ uint32_t* sync_top(uint32_t* s) { return s + 4; }                           // {maximum, arrivals}
-__device__ __forceinline__ uint32_t* sync_group(uint32_t* s, uint32_t j) { return s + 64 + j * 32; }     // {maximum, arrivals}, a line each
-__device__ __forceinline__ uint64_t* sync_result(uint32_t* s, uint32_t j) { return reinterpret_cast<uint64_t*>(s + 2176 + j * 32); }
-__device__ __forceinline__ uint32_t* sync_left_flag(uint32_t* s, uint32_t b) { return s + 4224 + b; }
-static_assert((4224 + kFusedMaxGrid) * 4 <= kWsSyncBytes, "synchronisation area too small");
-
-#define METIS_AT_LOAD(p) __hip_atomic_load((p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-#define METIS_AT_STORE(p, v) __hip_atomic_store((p), (v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-#define METIS_AT_CAS(p, expected, desired) \
-    __hip_atomic_compare_exchange_strong((p), (expected), (desired), __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-#define METIS_AT_XCHG(p, v) __hip_atomic_exchange((p), (v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-
-// a group's result word: tag << 18 | kind << 16 | bf16 payload; kind 0: the tensor maximum, kind 1: a member has left
-__device__ __forceinline__ uint64_t result_word(uint64_t tag, uint32_t kind, uint32_t payload) { return (tag << 18) | ((uint64_t)kind << 16) | payload; }
-__device__ __forceinline__ bool is_result(uint64_t w, uint64_t tag) { return (w >> 16) == (tag << 2); }
-__device__ __forceinline__ bool is_left_marker(uint64_t w, uint64_t tag) { return (w >> 16) == ((tag << 2) | 1u); }
-
-struct GridMaxState {
-    float wave_part[4];
-    uint32_t last;               // this workgroup was the last to arrive
-    uint32_t known;              // result holds the tensor maximum
-    float result;
-    uint32_t nleft;
-    uint32_t left[256];          // workgroups of one slab of 256 flags that left their scale bytes behind
-};
-
-// Every thread, at kernel start (before its workgroup arrives, so before the counter can move): the tag of this call.
-__device__ __forceinline__ uint64_t grid_max_begin(uint32_t* sync)
-{
-    return METIS_AT_LOAD(sync_generation(sync)) + 1u;
-}
-
-// One more arrival with maximum `bits` at a tree node {maximum, arrivals}; true for the arrival that completes `expected`,
-// with the node's maximum.  Two relaxed read-modify-writes without retry: the counter's increment is made to depend on
-// the value the maximum's returns, so it is issued only after the maximum has been performed at the coherence point; the
-// arrival that sees the count complete therefore reads a maximum that every earlier arrival has folded in.
-__device__ __forceinline__ bool tree_arrive(uint32_t* node, uint32_t bits, uint32_t expected, uint32_t& folded)
-{
-    const uint32_t before = __hip_atomic_fetch_max(node, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t one = 1u + (before >> 31);                      // bit 31 of a non-negative float's pattern: always 0
-    if (__hip_atomic_fetch_add(node + 1, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != expected - 1u) return false;
-    folded = METIS_AT_LOAD(node);
-    METIS_AT_STORE(node, 0u);                                      // nobody else touches the node before the next call
-    METIS_AT_STORE(node + 1, 0u);
-    return true;
-}
-
-// Called by every thread of every workgroup, once: folds the workgroup maximum (a bf16 value) into the tree.
-__device__ __forceinline__ void grid_max_arrive(float thread_max, uint32_t* sync, GridMaxState& sh)
-{
-    const float m = wave_max(thread_max);
-    if ((threadIdx.x & 63) == 0) sh.wave_part[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t bits = __float_as_uint(fmaxf(fmaxf(sh.wave_part[0], sh.wave_part[1]), fmaxf(sh.wave_part[2], sh.wave_part[3])));
-        const uint32_t j = blockIdx.x % kGroups;
-        const uint32_t ngroups = gridDim.x < kGroups ? gridDim.x : kGroups;
-        const uint32_t members = (gridDim.x + kGroups - 1u - j) / kGroups;
-        uint32_t gm = 0u, fin = 0u;
-        const bool last = tree_arrive(sync_group(sync, j), bits, members, gm) && tree_arrive(sync_top(sync), gm, ngroups, fin);
-        sh.last = last ? 1u : 0u;
-        sh.known = sh.last;
-        sh.result = __uint_as_float(fin);
-    }
-}
-
 // One block in flight ahead of the one being encoded (as in phase 1 of the two-launch path), block maxima kept in
 // registers, and the arrival placed before the encoding of the thread's last block so that the tree's latency is covered.
 template <int MODE, int NB>

@@ -396,30 +396,29 @@ def quantize_dequantize_f32(x: torch.Tensor) -> tuple[PackedNVFP4, torch.Tensor]
     return PackedNVFP4(codes, scales, unit, rows, cols, MODE_P32), out
 
 
-@functools.lru_cache(maxsize=4096)
-def _roundtrip_workspace_bytes(rows: int, cols: int, mode: int) -> int:
-    return int(load().metis_nvfp4_roundtrip_workspace_bytes(rows, cols, mode))
-
-
-def roundtrip_pays(x: torch.Tensor) -> bool:
-    """Whether reading x twice beats packing it and unpacking the packed form: up to 40 MiB (the second read comes from the
-    memory-side cache, but it is all of x again; times beside the kernels, nvfp4_roundtrip.hip)."""
-    return x.numel() * x.element_size() <= 40 << 20
-
-
-def roundtrip(x: torch.Tensor) -> torch.Tensor:
-    """dequantize(quantize(x)) of a bf16 tensor in bf16 arithmetic or a binary32 tensor in binary32 arithmetic, round to
-    nearest, without the packed tensor in between: the same values in x's shape and type."""
+def roundtrip(x: torch.Tensor, spin_limit: int = 0) -> torch.Tensor | None:
+    """dequantize(quantize(x)) of a bf16 tensor in bf16 arithmetic or a binary32 tensor in binary32 arithmetic, round to nearest: the
+    same values in x's shape and type, from one launch that packs nothing.  None where the device's registers do not hold the
+    tensor's codes.  spin_limit: polls for the grid's maximum before a workgroup leaves its values to the last one (0: the
+    library's limit)."""
     x2 = x if (x.dim() == 2 and x.is_contiguous()) else x.reshape(-1, x.shape[-1]).contiguous()
     rows, cols = x2.shape
-    mode = MODE_PB16 if x.dtype == torch.bfloat16 else _lib.MODE_P32_F32
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    need = _roundtrip_workspace_bytes(rows, cols, mode)
-    ws = _workspace(1, BLOCK, x.device).data_ptr() if need else None
-    rc = load().metis_nvfp4_roundtrip(x2.data_ptr(), rows, cols, mode, out.data_ptr(), ws, need, _stream())
+    if rows * cols > _ROUNDTRIP_FOLDED and torch.cuda.is_current_stream_capturing():
+        # a graph has an area of its own for the grid's maximum: it may be replayed beside other work of the stream it was captured on
+        ws = torch.empty(_quant_workspace_bytes(1, BLOCK), dtype=torch.uint8, device=x.device).fill_(0)
+    else:
+        ws = _workspace(1, BLOCK, x.device)
+    rc = load().metis_nvfp4_roundtrip(x2.data_ptr(), rows, cols, MODE_PB16 if x.dtype == torch.bfloat16 else _lib.MODE_P32_F32, out.data_ptr(),
+                                      ws.data_ptr(), ws.numel(), int(spin_limit), _stream())
+    if rc == _lib.E_TOO_LARGE:
+        return None
     if rc:
         check(rc, "metis_nvfp4_roundtrip", x.shape)
     return out
+
+
+_ROUNDTRIP_FOLDED = 128 * 1024            # elements up to which no grid-wide maximum is taken in either type
 
 
 def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tensor, mode: int = MODE_P32,

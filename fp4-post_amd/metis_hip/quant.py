@@ -161,11 +161,13 @@ class _NVFP4Base(BlockQuantFunc):
         if torch.is_grad_enabled():
             x = x.detach()
         if not cls.stochastic and x.is_cuda and x.numel():
+            # values only, nothing packed on the way; too large: one call whose second launch forms scale bytes and values together
             if x.dtype == torch.bfloat16:
-                # values only, nothing packed on the way; large: one call whose second launch forms scale bytes and values together
-                return ops.roundtrip(x) if ops.roundtrip_pays(x) else ops.quantize_dequantize(x, _mode_of(x))[1].reshape(x.shape)
+                out = ops.roundtrip(x)
+                return out if out is not None else ops.quantize_dequantize(x, _mode_of(x))[1].reshape(x.shape)
             if x.dtype == torch.float32 and x.data_ptr() % 16 == 0:
-                return ops.roundtrip(x) if ops.roundtrip_pays(x) else ops.quantize_dequantize_f32(x)[1].reshape(x.shape)
+                out = ops.roundtrip(x)
+                return out if out is not None else ops.quantize_dequantize_f32(x)[1].reshape(x.shape)
         return ops.dequantize(cls.pack(x), x.dtype).reshape(x.shape)
 
     @classmethod

@@ -100,14 +100,16 @@ int metis_nvfp4_quant_dequant_row_f32(const void *x, int64_t rows, int64_t cols,
                                       float *unit, void *out, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
- * The dequantized values of that round trip alone: no codes, scale bytes or unit are written.  x is read twice (once for
- * the tensor maximum) instead of being packed and unpacked through memory; a small tensor is one launch and needs no
- * workspace (metis_nvfp4_roundtrip_workspace_bytes is 0).
- *   x, out    [rows, cols], contiguous: bf16 with METIS_MODE_PB16, float with METIS_MODE_P32_F32; 16-byte aligned
+ * The dequantized values of that round trip alone, in ONE launch that reads x once: no codes, scale bytes or unit are written, the
+ * codes stay in registers until the tensor maximum is known.  METIS_E_TOO_LARGE for a tensor whose codes the device's registers do
+ * not hold (beyond 8192 x 4096 in binary32, 16384 x 4096 in bf16 on a device of 256 compute units).  The grid-wide maximum works as in
+ * metis_nvfp4_quant_row_resident: bounded polls (spin_limit, 0 for the default), the result does not depend on them.
+ *   x, out     [rows, cols], contiguous: bf16 with METIS_MODE_PB16, float with METIS_MODE_P32_F32; 16-byte aligned
+ *   workspace  metis_nvfp4_workspace_bytes(1, 16) bytes, 256-byte aligned, zero when first used; calls that share it are ordered.
+ *              Not read for small tensors (up to 128 K elements)
  */
-size_t metis_nvfp4_roundtrip_workspace_bytes(int64_t rows, int64_t cols, int mode);
 int metis_nvfp4_roundtrip(const void *x, int64_t rows, int64_t cols, int mode, void *out, void *workspace,
-                          size_t workspace_bytes, void *stream);
+                          size_t workspace_bytes, uint32_t spin_limit, void *stream);
 
 /*
  * metis_nvfp4_quant_row without a workspace argument and without any allocation: the scratch (per-workgroup

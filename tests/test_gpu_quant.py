@@ -739,16 +739,17 @@ def test_binary32_round_trip_from_one_call(ops, rows, cols):
     assert same_bits(q.quantize_dequantize(x).cpu(), out.cpu())
 
 
-# one launch / two launches (the line is 192 x 1024 elements in bf16, 128 x 1024 in binary32), odd tails, one block, leading dimensions
+# one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (192 x 1024 elements in bf16, 128 x
+# 1024 in binary32), leading dimensions, four and eight half blocks per thread
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("shape", [(1, 16), (3, 48), (5, 7, 80), (128, 1024), (129, 1024), (192, 1024), (193, 1024), (2049, 4080)])
+@pytest.mark.parametrize("shape", [(1, 16), (3, 48), (5, 7, 80), (128, 1024), (129, 1024), (192, 1024), (193, 1024), (2049, 4080), (8191, 4096)])
 def test_round_trip_values_without_a_packed_tensor(ops, dtype, shape):
     """ops.roundtrip: the values of quantize + dequantize bit for bit, with signed zeros, subnormal blocks, an infinity and a NaN."""
     from metis_hip import quant_func
     q = quant_func["nvfp4e2m1bnosr"]
     mode = 1 if dtype == torch.bfloat16 else 0
     bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
-    x = _f32_valued(shape[0] + shape[-1], 1, int(np.prod(shape))).reshape(shape).to(dtype).cuda()
+    x = torch.randn(shape, generator=torch.Generator("cuda").manual_seed(shape[0] + shape[-1]), device="cuda").to(dtype)
     flat = x.view(-1)
     flat[::97] = -0.0
     flat[:16] = 1e-39
@@ -756,12 +757,38 @@ def test_round_trip_values_without_a_packed_tensor(ops, dtype, shape):
         if value is not None:
             flat[flat.numel() // 2] = value
         want = ops.dequantize(ops.quantize(x, mode), dtype).reshape(shape)
-        for got in (ops.roundtrip(x), q.quantize_dequantize(x)):
+        # (spin_limit=1: workgroups leave their values to the last one)
+        for got in (ops.roundtrip(x), ops.roundtrip(x, spin_limit=1), q.quantize_dequantize(x)):
             assert got.shape == x.shape and got.dtype == dtype and not got.requires_grad
             assert torch.equal(got.view(bits), want.view(bits)), (shape, value)
     strided = x.movedim(0, -1)
     if strided.shape[-1] % 16 == 0:
         assert torch.equal(q.quantize_dequantize(strided).view(bits), q.quantize_dequantize(strided.contiguous()).view(bits))
+
+
+def test_round_trip_beyond_the_registers_and_from_a_captured_graph(ops):
+    from metis_hip import quant_func
+    q = quant_func["nvfp4e2m1bnosr"]
+    big = torch.randn(12288, 4096, device="cuda")                # binary32: the codes do not fit
+    assert ops.roundtrip(big) is None
+    want = ops.dequantize(ops.quantize(big, 0), torch.float32)
+    assert torch.equal(q.quantize_dequantize(big).view(torch.int32), want.view(torch.int32))
+    del big, want
+    x = torch.randn(1024, 2048, device="cuda").bfloat16()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        q.quantize_dequantize(x)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = q.quantize_dequantize(x)
+    for k in range(4):
+        x.copy_(torch.randn(1024, 2048, device="cuda") * (1 + k))
+        eager = q.quantize_dequantize(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
 
 
 def test_both_packings_of_a_whole_row_count_are_tensors_of_their_own(ops):
