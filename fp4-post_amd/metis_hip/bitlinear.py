@@ -61,7 +61,12 @@ def _version_of(x: torch.Tensor):
 
 
 def _flat2d(x: torch.Tensor) -> torch.Tensor:
-    return x.reshape(-1, x.shape[-1])
+    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+
+
+def _as_lead(y: torch.Tensor, lead: torch.Size) -> torch.Tensor:
+    """y [rows, n] with x's leading dimensions again."""
+    return y if len(lead) == 1 else y.view(*lead, y.shape[-1])
 
 
 def _packable(x: torch.Tensor, q) -> bool:
@@ -357,7 +362,7 @@ class LinearLowbitFunction(torch.autograd.Function):
             return None
         key, v = projection if projection is not None else (None, None)
         tm = ops.TokenMean(after_norm, cached_mean, cached_count, v)
-        packed = F.q_forward_input.pack(x2, arith=F.compute_dtype, center=tm, deferred=True)
+        packed = ops.quantize(x2, ops.MODE_PB16, center=tm, deferred=True)
         if mean_cache is not None:
             mean_cache[cache_key] = (tm.mean.unsqueeze(0), cached_count + rows)
         return CenteredNVFP4(packed, tm.mean, tm.mean32, None if tm.pending is None else (key, tm.pending))
@@ -826,11 +831,34 @@ class LinearLowbit(nn.Module):
         return super()._apply(fn, recurse=recurse)
 
 
+def _autograd_may_see() -> bool:
+    """Whether something may want to record or transform what an autograd function computes: autograd itself, forward-mode
+    differentiation, torch.func's transforms, a tracer.  Without any of them the function's values are computed without the function
+    (a decode step pays 8 us for each apply)."""
+    return (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._functorch.maybe_current_level() is not None or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
 class _MetisFusedFunction(torch.autograd.Function):
     """y = ((x V^T) * s) U^T + deq(Q(x)) deq(Q(R))^T + b in one GEMM launch, with its gradients."""
 
     @staticmethod
+    def evaluate(x, v, s, u, res, bias, px, p_res, xv=None, t=None, pending=None):
+        """forward without a context to keep anything in."""
+        return _MetisFusedFunction._evaluate(x, v, s, u, bias, px, p_res, xv, t, pending)[0]
+
+    @staticmethod
     def forward(ctx, x, v, s, u, res, bias, px, p_res, xv=None, t=None, pending=None):
+        y, xv, t = _MetisFusedFunction._evaluate(x, v, s, u, bias, px, p_res, xv, t, pending)
+        ctx.center, ctx.center32 = (px.mean, px.center32) if isinstance(px, CenteredNVFP4) else (None, None)
+        ctx.save_for_backward(x, v, s, u, res, xv, t)               # t = bf16(xv * s): [L, r], kept for the gradient of U
+        ctx.p_res = p_res
+        ctx.has_bias = bias is not None
+        ctx.lead = x.shape[:-1]
+        return y
+
+    @staticmethod
+    def _evaluate(x, v, s, u, bias, px, p_res, xv, t, pending):
         F = LinearLowbitFunction
         cd = torch.bfloat16
         aop = None
@@ -841,7 +869,7 @@ class _MetisFusedFunction(torch.autograd.Function):
                                                      ops.nv_operand_mode(px, [p_res], F.reference_rounding), pending=pending, rotate=p_res.rht)
             else:
                 target, centre = (px.residual, px.mean) if isinstance(px, CenteredNVFP4) else (px, None)
-                xv, t, aop = ops.project_and_operand(_flat2d(x).to(cd), v.to(cd), s.to(cd), target, ops.MODE_PB16, centre, pending=pending)
+                xv, t, aop = ops.project_and_operand(_as_dtype(_flat2d(x), cd), _as_dtype(v, cd), _as_dtype(s, cd), target, ops.MODE_PB16, centre, pending=pending)
         elif xv is None:
             # [L, r] rank-r projection and its product with s (bf16) on the library's kernels (split-K below 256 rows,
             # one pass over x from there on); the caller has it already when the quantizer's pass produced it
@@ -861,33 +889,28 @@ class _MetisFusedFunction(torch.autograd.Function):
             else:
                 xv, t = ops.lowrank_project(x2, vb, sb)
         out_dtype = torch.float32 if F.compute_dtype == torch.float32 else torch.bfloat16
-        ctx.center = ctx.center32 = None
+        u = _as_dtype(u, cd)
         # binary32 arithmetic keeps a binary32 bias (as LinearLowbit and the centred path do); bf16 arithmetic adds it in bf16
         gemm_bias = None if bias is None else (bias.float() if F.compute_dtype == torch.float32 else bias.to(cd))
         if isinstance(px, CenteredNVFP4):
             # mean mode: the residual branch sees 1 me^T + R
-            ctx.center, ctx.center32 = px.mean, px.center32
             if F._mean_in_operand(px, p_res):
                 # bf16 arithmetic: the activation operand is the reference's bf16 tensor me + QDQ(x - me)
-                y = ops.linear_fwd_grouped(px.residual, [(p_res, t, u.to(cd), gemm_bias)], out_dtype=out_dtype, center=px.mean,
+                y = ops.linear_fwd_grouped(px.residual, [(p_res, t, u, gemm_bias)], out_dtype=out_dtype, center=px.mean,
                                            reference_rounding=True, a_operand=aop)[0]
             elif px.rows < 256:
                 # decode-sized: W^ me is accumulated inside the GEMM launch
-                y = ops.linear_fwd_grouped(px.residual, [(p_res, t, u.to(cd), None if bias is None else bias.float())],
+                y = ops.linear_fwd_grouped(px.residual, [(p_res, t, u, None if bias is None else bias.float())],
                                            out_dtype=out_dtype, center=px.center32)[0]
             else:
                 # the mean term rides in a binary32 bias
                 w_mean = ops.matvec(p_res, px.center32)
-                y = ops.linear_fwd(px.residual, p_res, t=t, u=u.to(cd), bias=w_mean if bias is None else w_mean + bias.float(),
+                y = ops.linear_fwd(px.residual, p_res, t=t, u=u, bias=w_mean if bias is None else w_mean + bias.float(),
                                    out_dtype=out_dtype)
         else:
-            y = ops.linear_fwd(px, p_res, t=t, u=u.to(cd), bias=gemm_bias, out_dtype=out_dtype,
+            y = ops.linear_fwd(px, p_res, t=t, u=u, bias=gemm_bias, out_dtype=out_dtype,
                                reference_rounding=F.reference_rounding, a_operand=aop)
-        ctx.save_for_backward(x, v, s, u, res, xv, t)               # t = bf16(xv * s): [L, r], kept for the gradient of U
-        ctx.p_res = p_res
-        ctx.has_bias = bias is not None
-        ctx.lead = x.shape[:-1]
-        return y.reshape(*ctx.lead, y.shape[-1]).to(F.compute_dtype)
+        return _as_dtype(_as_lead(y, x.shape[:-1]), F.compute_dtype), xv, t
 
     @staticmethod
     def _transposed_bf16(w: torch.Tensor) -> torch.Tensor:
@@ -1205,7 +1228,7 @@ class BitLinear(nn.Module):
         group = self.activation_group
         members = group["members"]
         rows = x.numel() // max(x.shape[-1], 1)
-        if not all(m._fusable() and m.compute_dtype == self.compute_dtype for m in members):
+        if not all([m is self or (m._fusable() and m.compute_dtype == self.compute_dtype) for m in members]):   # (the caller asked self)
             return None
         if rows >= 256 and not all([m._modules["warmup_linear"].cache_quantized_weight for m in members]):
             # weights packed for this one call: only if the group will use them (each member packs its own otherwise)
@@ -1219,7 +1242,7 @@ class BitLinear(nn.Module):
             return self._forward_group_tiled(x, shared_input, members, packed)
         rotated = any(p.rht is not None for p in packed)          # NV recipe: the activation's operand carries the rotation
         cd = torch.bfloat16
-        x2 = _flat2d(x).to(cd)
+        x2 = _as_dtype(_flat2d(x), cd)
         cached = self._stacked_factors(x2.device)
         centre = shared_input.center32 if isinstance(shared_input, CenteredNVFP4) else None
         px = shared_input.residual if centre is not None else shared_input
@@ -1236,7 +1259,7 @@ class BitLinear(nn.Module):
                 and ops.project_and_operand_applies(x2, cached[1], cached[2], px)):
             # the projection's finishing step and the activation's GEMM operands in one launch
             pending = getattr(shared_input, "pending", None)       # its first step ran beside the quantizer, with these very factors
-            _, t_all, aop = ops.project_and_operand(x2, cached[1], cached[2], px, ops.MODE_PB16, centre,
+            _, t_all, aop = ops.project_and_operand(x2, cached[1], cached[2], px, ops.MODE_PB16, centre, checked=True,
                                                     pending=pending[1] if pending is not None and pending[0] is cached[0] else None)
         else:
             _, t_all = ops.lowrank_project(x2, cached[1], cached[2])
@@ -1246,14 +1269,14 @@ class BitLinear(nn.Module):
             bias = m._modules["warmup_linear"].bias
             if bias is not None:
                 bias = m._bias_as(torch.float32 if (centre is not None and centre.dtype == torch.float32) else cd)
-            calls.append((p_res, t_all[:, c0:c0 + r], _param(m._modules["ulinear"], "weight").to(cd), bias))      # a column slice: no copy
+            calls.append((p_res, t_all[:, c0:c0 + r], _as_dtype(_param(m._modules["ulinear"], "weight"), cd), bias))      # a column slice: no copy
             c0 += r
         out_dtype = torch.float32 if F.compute_dtype == torch.float32 else torch.bfloat16
         # mean mode: every member also receives W^ me, inside the same launch (binary32)
         outs = ops.linear_fwd_grouped(px, calls, out_dtype=out_dtype, center=centre, reference_rounding=F.reference_rounding,
-                                      a_operand=aop)
+                                      a_operand=aop, checked=aop is not None and not rotated)
         lead = x.shape[:-1]
-        return {id(m): _as_dtype(y.reshape(*lead, y.shape[-1]), F.compute_dtype) for m, y in zip(members, outs)}
+        return {id(m): _as_dtype(_as_lead(y, lead), F.compute_dtype) for m, y in zip(members, outs)}
 
     def _output_key(self) -> tuple:
         """What this member's output depends on beside its input, as far as identities and version counters tell."""
@@ -1368,7 +1391,7 @@ class BitLinear(nn.Module):
             calls.append((p_res, t, _as_dtype(_param(m._modules["ulinear"], "weight"), cd), bias))
         outs = ops._linear_fwd_tiled_grouped(px, calls, torch.float32 if f32 else torch.bfloat16, shared_input.mean if in_operand else None, rounding)
         lead = x.shape[:-1]
-        return {id(m): _as_dtype(y.reshape(*lead, y.shape[-1]), F.compute_dtype) for m, y in zip(members, outs)}
+        return {id(m): _as_dtype(_as_lead(y, lead), F.compute_dtype) for m, y in zip(members, outs)}
 
     def _bias_as(self, dtype: torch.dtype) -> torch.Tensor:
         """The residual branch's bias in `dtype`, converted once per parameter version (decode calls are launch-bound)."""
@@ -1427,8 +1450,9 @@ class BitLinear(nn.Module):
                             and ops.grouped_operand_applies(shared_input.residual, [p_res], [r], shared_input.mean, F.reference_rounding)):
                         more = (None, None, shared_input.pending[1])
                     wl = mods["warmup_linear"]
-                    return _MetisFusedFunction.apply(x, _param(mods["vlinear"], "weight"), _param(self, "s"), _param(mods["ulinear"], "weight"),
-                                                     _param(wl, "weight"), wl.bias, shared_input, p_res, *more)
+                    call = _MetisFusedFunction.apply if _autograd_may_see() else _MetisFusedFunction.evaluate
+                    return call(x, _param(mods["vlinear"], "weight"), _param(self, "s"), _param(mods["ulinear"], "weight"),
+                                _param(wl, "weight"), wl.bias, shared_input, p_res, *more)
             if BitLinear.rollout_merge_active and not torch.is_grad_enabled():
                 return self._rollout_forward(shared_input, x.shape)
             y = self.vlinear(x, quantized_input=shared_input)

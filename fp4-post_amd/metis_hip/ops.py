@@ -214,8 +214,15 @@ def _as_2d_bf16(x: torch.Tensor) -> torch.Tensor:
         raise _lib.MetisHipError("metis_hip ops need a ROCm device tensor; there is no CPU path")
     if x.dtype != torch.bfloat16:
         x = x.to(torch.bfloat16)
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     return x2 if x2.is_contiguous() else x2.contiguous()
+
+
+def _bf16_row(c: torch.Tensor) -> torch.Tensor:
+    """A vector of one value per column as contiguous bf16 [cols] (what a mean of this library already is)."""
+    if c.dim() == 1 and c.dtype == torch.bfloat16 and c.is_contiguous():
+        return c
+    return c.reshape(-1).to(torch.bfloat16).contiguous()
 
 
 def _as_2d_for_quant(x: torch.Tensor, mode: int) -> tuple[torch.Tensor, int]:
@@ -663,7 +670,7 @@ def _quantize_token_mean(x2: torch.Tensor, tm: TokenMean) -> PackedNVFP4:
     dev = x2.device
     cp = None
     if cached is not None:
-        cached = cached.reshape(-1).to(device=dev, dtype=torch.bfloat16).contiguous()
+        cached = cached.to(device=dev, dtype=torch.bfloat16).contiguous()
         if cached.numel() != cols:
             raise ValueError(f"cached mean has {cached.numel()} values, the tensor {cols} columns")
         cp = cached.data_ptr()
@@ -782,7 +789,7 @@ def expand_tiled(p: PackedNVFP4, cache: bool = True, mode: int = MODE_P32, cente
     if center is not None:
         if mode != MODE_PB16 or p.rht is not None:
             raise ValueError("a centre goes into the bf16-arithmetic operand of an unrotated tensor")
-        center = center.reshape(-1).to(torch.bfloat16).contiguous()
+        center = _bf16_row(center)
         if center.numel() != p.cols:
             raise ValueError(f"center must have {p.cols} values, got {center.numel()}")
         key = (center.data_ptr(), center._version)
@@ -921,14 +928,16 @@ def project_and_operand_applies(x2: torch.Tensor, v: torch.Tensor, s: torch.Tens
 
 
 def project_and_operand(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: PackedNVFP4, mode: int = MODE_PB16,
-                        center: torch.Tensor | None = None, pending: torch.Tensor | None = None, rotate: int | None = None):
+                        center: torch.Tensor | None = None, pending: torch.Tensor | None = None, rotate: int | None = None,
+                        checked: bool = False):
     """(xv, t, operand) = lowrank_project(x2, v, s) and decode_operand(p, mode, center) of one decode-sized activation
     in two launches instead of three: the projection's finishing step rides in the operand launch.  Same bits.
     pending: the projection's partial sums as quantize_project_decode left them (the first of the two launches already
-    ran beside the quantizer): one launch.  rotate (sign mask): the operand of decode_operand(p, mode, rotate=...)."""
+    ran beside the quantizer): one launch.  rotate (sign mask): the operand of decode_operand(p, mode, rotate=...).
+    checked: the caller has just asked project_and_operand_applies."""
     if rotate is not None and center is not None:
         raise ValueError("a rotated operand takes no centre")
-    if not project_and_operand_applies(x2, v, s, p):
+    if not checked and not project_and_operand_applies(x2, v, s, p):
         raise ValueError("project_and_operand: outside the call's domain (see project_and_operand_applies)")
     M, K = x2.shape
     R = v.shape[0]
@@ -937,11 +946,11 @@ def project_and_operand(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: P
     v = v.contiguous()
     s = s.contiguous()
     if center is not None:
-        center = center.reshape(-1).to(torch.bfloat16).contiguous()
+        center = _bf16_row(center)
         if center.numel() != K:
             raise ValueError(f"center must have {K} values, got {center.numel()}")
     xv = torch.empty(M, R, dtype=torch.bfloat16, device=dev)
-    t = torch.empty_like(xv)
+    t = torch.empty(M, R, dtype=torch.bfloat16, device=dev)
     out = torch.empty(_decode_operand_bytes(M, K), dtype=torch.uint8, device=dev)
     need = _lowrank_workspace_bytes(M, R, K)
     if pending is not None and (pending.numel() < need or pending.device != dev):
@@ -1680,8 +1689,8 @@ def lowrank_backward(dy: torch.Tensor, t: torch.Tensor, x: torch.Tensor, gxv: to
 
 def linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.bfloat16,
                        center: torch.Tensor | None = None, split_k: bool = True,
-                       reference_rounding: bool = False, a_operand: torch.Tensor | None = None) -> list[torch.Tensor]:
-    return _linear_fwd_grouped(a, members, out_dtype, center, split_k, reference_rounding, a_operand)
+                       reference_rounding: bool = False, a_operand: torch.Tensor | None = None, checked: bool = False) -> list[torch.Tensor]:
+    return _linear_fwd_grouped(a, members, out_dtype, center, split_k, reference_rounding, a_operand, checked)
 
 
 def _grouped_members(members, M: int, K: int, out_dtype: torch.dtype, dev, decode_layout: bool):
@@ -1723,7 +1732,7 @@ def _grouped_members(members, M: int, K: int, out_dtype: torch.dtype, dev, decod
 
 def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.bfloat16,
                         center: torch.Tensor | None = None, split_k: bool = True,
-                        reference_rounding: bool = False, a_operand: torch.Tensor | None = None) -> list[torch.Tensor]:
+                        reference_rounding: bool = False, a_operand: torch.Tensor | None = None, checked: bool = False) -> list[torch.Tensor]:
     """[linear_fwd(a, b, t=t, u=u, bias=bias) for (b, t, u, bias) in members] in one call: a projection group
     (q/k/v, gate/up) that shares one packed activation.  Decode-sized batches run as a single launch.
 
@@ -1736,16 +1745,16 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
     inside the same launch where the shape allows, else through matvec and a binary32 bias.
 
     a_operand: decode_operand(a, MODE_PB16, center) when the caller has it already (project_and_operand); read only
-    where grouped_operand_applies says the call reads ready operands."""
+    where grouped_operand_applies says the call reads ready operands (checked: the caller has just asked it)."""
     M, K = a.rows, a.cols
     dev = a.codes.device
-    if a_operand is not None and split_k and grouped_operand_applies(a, [m[0] for m in members], [0 if m[1] is None else m[1].shape[1] for m in members],
-                                                                     center, reference_rounding):
+    if a_operand is not None and split_k and (checked or grouped_operand_applies(a, [m[0] for m in members], [0 if m[1] is None else m[1].shape[1] for m in members],
+                                                                     center, reference_rounding)):
         # the usual decode step: every question below has its answer
         arr, outs, keep = _grouped_members(members, M, K, out_dtype, dev, decode_layout_weights)
         need, _ = _grouped_plan(M, K, tuple([m[0].rows for m in members]), dev.index or 0)
         ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-        rc = load().metis_linear_fwd_grouped_operand(a_operand.data_ptr(), a.unit.data_ptr(), M, K, ctypes.addressof(arr), len(members),
+        rc = load().metis_linear_fwd_grouped_operand(a_operand.data_ptr(), a.__dict__["_unit"].data_ptr(), M, K, ctypes.addressof(arr), len(members),
                                                      DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, MODE_PB16,
                                                      None if ws is None else ws.data_ptr(), need, _stream())
         if rc:

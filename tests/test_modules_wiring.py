@@ -449,3 +449,26 @@ def test_scale_bytes_are_deferred_only_when_the_consumer_forms_them(monkeypatch)
     assert F._scales_formed_by_consumer(4096, False) and F._scales_formed_by_consumer(1, False)
     monkeypatch.setattr(F, "reference_rounding", False)
     assert not F._scales_formed_by_consumer(1, False)
+
+
+def test_values_without_the_autograd_function_only_where_nothing_may_record_or_transform_them():
+    """bitlinear._autograd_may_see: the fused function is passed by under no_grad alone, not inside forward-mode differentiation, a
+    torch.func transform or a tracer (which have to meet the function, or its refusal)."""
+    import torch.autograd.forward_ad as fwd
+    from metis_hip.bitlinear import _autograd_may_see
+    assert _autograd_may_see()
+    with torch.no_grad():
+        assert not _autograd_may_see()
+        with fwd.dual_level():
+            assert _autograd_may_see()
+        seen = []
+
+        def probe(x):
+            seen.append(_autograd_may_see())
+            return x * 2
+        torch.func.vmap(probe)(torch.ones(3, 2))
+        torch.func.jvp(probe, (torch.ones(2),), (torch.ones(2),))
+        torch.jit.trace(probe, torch.ones(2), check_trace=False)
+        assert seen and all(seen)
+    with torch.inference_mode():
+        assert not _autograd_may_see()
