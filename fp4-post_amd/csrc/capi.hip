@@ -314,6 +314,15 @@ int metis_nvfp4_quant_sr_both_copy(const void* x, int64_t rows, int64_t padded_r
                             scales_col, unit_col, workspace, workspace_bytes, (hipStream_t)stream, rows, copy);
 }
 
+int metis_nvfp4_quant_sr_both_centered(const void* x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld, int mode, const void* center,
+                                       uint64_t seed, uint64_t offset_row, uint64_t offset_col, void* codes_row, void* scales_row, float* unit_row,
+                                       void* codes_col, void* scales_col, float* unit_col, void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (rows < 0 || rows > padded_rows || !center) return METIS_E_ARG;
+    return quantize_both_sr(x, padded_rows, cols, ld, mode, seed, offset_row, offset_col, codes_row, scales_row, unit_row, codes_col, scales_col,
+                            unit_col, workspace, workspace_bytes, (hipStream_t)stream, rows, nullptr, center);
+}
+
 int metis_nvfp4_quant_row_rht_copy(const void* x, int64_t rows, int64_t cols, int64_t ld, uint32_t sign_mask, int sr, uint64_t seed, uint64_t offset,
                                    void* codes, void* scales, float* unit, void* copy, void* workspace, size_t workspace_bytes, void* stream)
 {

@@ -492,13 +492,17 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
 // holds one column of a slab; the slab also goes through LDS (68-word rows) and comes back as row blocks, lane l
 // taking row l / 4, block l % 4.  Both packings share the tensor maximum, hence one partial maximum per workgroup.
 // copy (binary32 input): the tensor rounded to bf16 as well, as in quant_codes_kernel.
+// CEN: one value per column is subtracted first (the mean mode's output gradient), bf16 in bf16 arithmetic, binary32 for a binary32
+// tensor; rows past `valid` have a zero residual.  The MLP step of 2103 tokens, 3584 -> 18944: 3824 us with two
+// passes over each dY, 3806 with one (the encoders bound it, not the second read).
 // ---------------------------------------------------------------------------------------------
 constexpr uint32_t kBothRun = 16;
-template <int MODE, bool WIDE = false>
-__global__ __launch_bounds__(256, 5) void quant_codes_both_kernel(
+template <int MODE, bool WIDE = false, bool CEN = false>
+__global__ __launch_bounds__(256, CEN ? 4 : 5) void quant_codes_both_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, uint64_t seed, uint64_t offset_row, uint64_t offset_col,
     uint2* __restrict__ codes_row, void* __restrict__ amax_row_v, uint2* __restrict__ codes_col, void* __restrict__ amax_col_v,
-    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, uint32_t valid, uint16_t* __restrict__ copy = nullptr)
+    uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, uint32_t valid, uint16_t* __restrict__ copy = nullptr,
+    const void* __restrict__ center = nullptr)
 {
     static_assert(!WIDE || MODE == 0, "binary32 values imply binary32 arithmetic");
     using amax_t = typename std::conditional<WIDE, float, uint16_t>::type;
@@ -555,6 +559,15 @@ __global__ __launch_bounds__(256, 5) void quant_codes_both_kernel(
         const uint32_t tr = tile / tiles_c, tc = tile - tr * tiles_c;
         const uint32_t c = tc * kColTileCols + lane;
         const uint32_t cbg = tc * 4u + cb;
+        // the centre of the lane's row block (as stored) and of its column
+        uint4 crow[CEN ? (WIDE ? 4 : 2) : 1];
+        float ccol = 0.0f;
+        if constexpr (CEN) {
+#pragma unroll
+            for (int q = 0; q < (WIDE ? 4 : 2); ++q)
+                crow[q] = live && cbg < nbpr ? reinterpret_cast<const uint4*>(center)[(size_t)cbg * (WIDE ? 4 : 2) + q] : make_uint4(0u, 0u, 0u, 0u);
+            if (live && c < cols) ccol = WIDE ? static_cast<const float*>(center)[c] : bf16_lo(static_cast<const uint16_t*>(center)[c]);
+        }
 #pragma unroll 1
         for (uint32_t k = 0; k < 4u; ++k) {
             if (k < 3u) fetch(wid, k + 1u, nxt);
@@ -595,6 +608,24 @@ __global__ __launch_bounds__(256, 5) void quant_codes_both_kernel(
                     for (int j = 0; j < kBlock; ++j) v[j] = __uint_as_float((slab[g][j][lane >> 1] << shift) & 0xffff0000u);
                 }
                 __builtin_amdgcn_wave_barrier();
+                if constexpr (CEN) {
+                    const bool row_in = b * kBlock + rr < valid;
+                    float cr[kBlock];
+                    if constexpr (WIDE) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            cr[4 * q] = __uint_as_float(crow[q].x); cr[4 * q + 1] = __uint_as_float(crow[q].y);
+                            cr[4 * q + 2] = __uint_as_float(crow[q].z); cr[4 * q + 3] = __uint_as_float(crow[q].w);
+                        }
+                    } else {
+                        unpack16(crow[0], crow[WIDE ? 0 : 1], cr);
+                    }
+#pragma unroll
+                    for (int j = 0; j < kBlock; ++j) {
+                        w[j] = row_in ? rd<MODE>(w[j] - cr[j]) : 0.0f;
+                        v[j] = b * kBlock + j < valid ? rd<MODE>(v[j] - ccol) : 0.0f;
+                    }
+                }
                 if (have_row) {
                     const float amr = block_amax(w);
                     gmax = fmaxf(gmax, amr);
@@ -1266,7 +1297,7 @@ int quantize_dequantize_row(const void* x, int64_t rows, int64_t cols, int mode,
 
 // Workgroups of quant_codes_both_kernel that the current device holds at once (its LDS slabs bound them): the grid is
 // no larger, so that every workgroup starts at once and walks the same number of tiles, give or take one.
-template <int MODE, bool WIDE>
+template <int MODE, bool WIDE, bool CEN>
 static int both_capacity()
 {
     static int cached[64] = {};
@@ -1274,7 +1305,7 @@ static int both_capacity()
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
     if (cached[dev] == 0) {
         int per_cu = 0;
-        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, quant_codes_both_kernel<MODE, WIDE>, 256, 0);
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, quant_codes_both_kernel<MODE, WIDE, CEN>, 256, 0);
         cached[dev] = (e != hipSuccess || per_cu <= 0) ? -1 : per_cu * device_cus();
     }
     return cached[dev] < 0 ? device_cus() * 4 : cached[dev];
@@ -1286,10 +1317,11 @@ static int both_capacity()
 // ---------------------------------------------------------------------------------------------
 int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode, uint64_t seed, uint64_t offset_row,
                      uint64_t offset_col, void* codes_row, void* scales_row, float* unit_row, void* codes_col, void* scales_col,
-                     float* unit_col, void* workspace, size_t bytes, hipStream_t st, int64_t valid, void* copy)
+                     float* unit_col, void* workspace, size_t bytes, hipStream_t st, int64_t valid, void* copy, const void* center)
 {
     if (rows < 0 || cols < 0 || ld < cols || valid > rows) return METIS_E_ARG;
     if (copy && (mode != METIS_MODE_P32_F32 || ((uintptr_t)copy % 16))) return METIS_E_ARG;
+    if (center && ((mode != METIS_MODE_P32_F32 && mode != METIS_MODE_PB16) || ((uintptr_t)center % 16))) return METIS_E_ARG;   // (a binary32 centre leaves binary32 residuals)
     if (mode != METIS_MODE_P32 && mode != METIS_MODE_PB16 && mode != METIS_MODE_P32_F32) return METIS_E_ARG;
     const bool f32in = mode == METIS_MODE_P32_F32;
     if (rows % kBlock || cols % kBlock) return METIS_E_SHAPE;
@@ -1309,15 +1341,17 @@ int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int 
     const uint32_t tiles_c = (uint32_t)((cols + kColTileCols - 1) / kColTileCols);
     const int64_t tiles = (int64_t)tiles_r * tiles_c;
     int64_t g = tiles;
-    const int64_t cap = f32in ? both_capacity<0, true>() : mode == 0 ? both_capacity<0, false>() : both_capacity<1, false>();
+    const int64_t cap = center ? (f32in ? both_capacity<0, true, true>() : both_capacity<1, false, true>())
+                               : f32in ? both_capacity<0, true, false>() : mode == 0 ? both_capacity<0, false, false>() : both_capacity<1, false, false>();
     if (g > cap) g = cap;
     if (g > kMaxGroups) g = kMaxGroups;
-#define METIS_QB(M, W) hipLaunchKernelGGL((quant_codes_both_kernel<M, W>), dim3((unsigned)g), dim3(256), 0, st, x, (uint32_t)rows, \
+#define METIS_QB(M, W, C) hipLaunchKernelGGL((quant_codes_both_kernel<M, W, C>), dim3((unsigned)g), dim3(256), 0, st, x, (uint32_t)rows, \
                                           (uint32_t)cols, ld, seed, offset_row, offset_col, (uint2*)codes_row, (void*)wr.amax, (uint2*)codes_col, \
-                                          (void*)wc.amax, wr.gmax, tiles_c, (uint32_t)tiles, (uint32_t)(valid < 0 ? rows : valid), (uint16_t*)copy)
-    if (f32in) METIS_QB(0, true);
-    else if (mode == 0) METIS_QB(0, false);
-    else METIS_QB(1, false);
+                                          (void*)wc.amax, wr.gmax, tiles_c, (uint32_t)tiles, (uint32_t)(valid < 0 ? rows : valid), (uint16_t*)copy, center)
+    if (center) { if (f32in) METIS_QB(0, true, true); else METIS_QB(1, false, true); }
+    else if (f32in) METIS_QB(0, true, false);
+    else if (mode == 0) METIS_QB(0, false, false);
+    else METIS_QB(1, false, false);
 #undef METIS_QB
     if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
     const int pm = f32in ? METIS_MODE_P32_F32 : mode;

@@ -72,6 +72,7 @@ SIGNATURES = {
                                   _vp, _vp, _sz, _vp]),
     "metis_nvfp4_quant_col_padded": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _i32, _u64, _u64, _vp, _vp, _vp, _vp, _sz, _vp]),
     "metis_nvfp4_quant_sr_both_padded": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _u64, _u64, _u64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "metis_nvfp4_quant_sr_both_centered": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _u64, _u64, _u64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "metis_nvfp4_quant_sr_both_copy": (_i32, [_vp, _i64, _i64, _i64, _i64, _u64, _u64, _u64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "metis_nvfp4_quant_row_rht_copy": (_i32, [_vp, _i64, _i64, _i64, ctypes.c_uint32, _i32, _u64, _u64, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "metis_nvfp4_deferred_bytes": (_sz, [_i64, _i64]),

@@ -478,8 +478,9 @@ class LinearLowbitFunction(torch.autograd.Function):
             dy2 = dy2 if dy2.data_ptr() % 16 == 0 else dy2.clone()
         if packed_dy is not None:
             p_dy, p_dyt = packed_dy
-        elif me_dy is None and hasattr(qg, "pack_both"):
-            p_dy, p_dyt = qg.pack_both(dy2, arith=cd, **more)  # one pass over dY for both products
+        elif hasattr(qg, "pack_both") and (me_dy is None or qg.packs_both_at_once(dy2, more.get("pad_rows"), True, cd)):
+            cen = {} if me_dy is None else {"center": me_dy}
+            p_dy, p_dyt = qg.pack_both(dy2, arith=cd, **cen, **more)  # one pass over dY for both products
         else:
             p_dy, p_dyt = qg.pack(dy2, arith=cd, center=me_dy, **more), None
         if me_dy is None and gx_lowrank is None:

@@ -472,13 +472,20 @@ def _check_bf16_copy(copy: torch.Tensor | None, x2: torch.Tensor, kmode: int) ->
 
 def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, offset_row: int = 0,
                      offset_col: int = 0, pad_rows: int | None = None,
-                     bf16_copy: torch.Tensor | None = None) -> tuple[PackedNVFP4, PackedNVFP4]:
+                     bf16_copy: torch.Tensor | None = None, center: torch.Tensor | None = None) -> tuple[PackedNVFP4, PackedNVFP4]:
     """(quantize(x, sr=True, offset=offset_row), quantize(x, col=True, sr=True, offset=offset_col)) from ONE pass over x:
     the two packings of an output gradient that the input-gradient and weight-gradient products contract.  Same
     bytes as the two calls.  Both dimensions of x flattened to [R, C] have to be multiples of 16; with pad_rows, that
     and C: the column packing is that of x filled up with zero rows to pad_rows, the row packing that of x.
-    bf16_copy (a binary32 x in binary32 arithmetic): bf16 [R, C], contiguous: the same pass leaves x.to(bfloat16) in it."""
+    bf16_copy (a binary32 x in binary32 arithmetic): bf16 [R, C], contiguous: the same pass leaves x.to(bfloat16) in it.
+    center: [C] subtracted from every row first, as in quantize; in bf16 arithmetic, or of a binary32 x in binary32 arithmetic."""
     x2, kmode = _as_2d_for_quant(x, mode)
+    if center is not None:
+        if bf16_copy is not None or kmode == MODE_P32:
+            raise ValueError("quantize_both_sr: a centre in bf16 arithmetic or for a binary32 tensor, and without bf16_copy")
+        center = center.reshape(-1).to(device=x2.device, dtype=torch.bfloat16 if kmode == MODE_PB16 else torch.float32).contiguous()
+        if center.numel() != x2.shape[1]:
+            raise ValueError(f"center must have one value per column ({x2.shape[1]}), got {center.numel()}")
     _check_bf16_copy(bf16_copy, x2, kmode)
     have, cols = x2.shape
     rows = have if pad_rows is None else pad_rows
@@ -500,7 +507,13 @@ def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, of
         ws = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=dev).fill_(0)
         _workspaces[key] = ws
     (cr, sr_, ur), (cc, sc, uc) = packs
-    if bf16_copy is not None and rows * cols:
+    if center is not None and rows * cols:
+        rc = L.metis_nvfp4_quant_sr_both_centered(x2.data_ptr(), have, rows, cols, x2.stride(0), kmode, center.data_ptr(), seed & (2 ** 64 - 1),
+                                                  offset_row, offset_col, cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(),
+                                                  uc.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
+        if rc:
+            check(rc, "metis_nvfp4_quant_sr_both_centered", x.shape)
+    elif bf16_copy is not None and rows * cols:
         rc = L.metis_nvfp4_quant_sr_both_copy(x2.data_ptr(), have, rows, cols, x2.stride(0), seed & (2 ** 64 - 1), offset_row, offset_col,
                                               cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(), uc.data_ptr(),
                                               bf16_copy.data_ptr(), ws.data_ptr(), ws.numel(), _stream())

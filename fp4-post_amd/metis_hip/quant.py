@@ -126,28 +126,32 @@ class _NVFP4Base(BlockQuantFunc):
         return ops.quantize(x, mode, col=col, center=center, deferred=deferred, **more)
 
     @classmethod
-    def packs_both_at_once(cls, x: torch.Tensor, pad_rows: int | None = None) -> bool:
+    def packs_both_at_once(cls, x: torch.Tensor, pad_rows: int | None = None, centered: bool = False, arith: torch.dtype | None = None) -> bool:
         """pack_both(x) is one pass over x."""
         rows = x.numel() // x.shape[-1] if x.numel() else 0
-        return cls.stochastic and rows > 0 and (pad_rows or rows) % 16 == 0 and x.dtype in (torch.bfloat16, torch.float32)
+        return (cls.stochastic and rows > 0 and (pad_rows or rows) % 16 == 0 and x.dtype in (torch.bfloat16, torch.float32)
+                and (not centered or arith is None or arith == x.dtype))
 
     @classmethod
     @torch.no_grad()
     def pack_both(cls, x: torch.Tensor, arith: torch.dtype | None = None,
-                  pad_rows: int | None = None, bf16_copy: torch.Tensor | None = None) -> tuple[ops.PackedNVFP4, ops.PackedNVFP4]:
+                  pad_rows: int | None = None, bf16_copy: torch.Tensor | None = None,
+                  center: torch.Tensor | None = None) -> tuple[ops.PackedNVFP4, ops.PackedNVFP4]:
         """(pack(x), pack(x, col=True)): the same two tensors, and under stochastic rounding the same draws in the same
         order, from one pass over x where the kernels have one (stochastic rounding, both dimensions multiples of 16).
-        pad_rows: as in pack.  bf16_copy: see ops.quantize_both_sr; only where that one pass is taken (packs_both_at_once)."""
+        pad_rows, center: as in pack.  bf16_copy: see ops.quantize_both_sr; only where that one pass is taken (packs_both_at_once)."""
         _need_gpu(x)
         cls._check(x)
         rows = x.numel() // x.shape[-1] if x.numel() else 0
         more = {} if pad_rows is None else {"pad_rows": pad_rows}
+        if center is not None:
+            more["center"] = center
         drawn = x.numel() if pad_rows is None else pad_rows * x.shape[-1]
         if bf16_copy is not None:
             if not cls.packs_both_at_once(x, pad_rows):
                 raise ValueError("bf16_copy: only where both packings come from one pass")
             more["bf16_copy"] = bf16_copy
-        if cls.packs_both_at_once(x, pad_rows):
+        if cls.packs_both_at_once(x, pad_rows, center is not None, arith):
             mode = _mode_of(x) if arith is None else (MODE_P32 if arith == torch.float32 else MODE_PB16)
             first = cls._next_offset(drawn)
             second = cls._next_offset(drawn)

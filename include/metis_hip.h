@@ -424,6 +424,16 @@ int metis_nvfp4_quant_row_rht(const void *x, int64_t rows, int64_t cols, int64_t
                               void *scales, float *unit, void *workspace, size_t workspace_bytes,
                               void *stream);
 /*
+ * metis_nvfp4_quant_sr_both_padded of x - center, one value per column (the output gradient of the mean mode): both packings that
+ * metis_nvfp4_quant_centered and metis_nvfp4_quant_col_padded give one after the other, rows past the tensor's own equal to the
+ * centre.  center bf16 [cols] with METIS_MODE_PB16, float [cols] with METIS_MODE_P32_F32 (a binary32 x); 16-byte aligned.
+ */
+int metis_nvfp4_quant_sr_both_centered(const void *x, int64_t rows, int64_t padded_rows, int64_t cols, int64_t ld, int mode,
+                                       const void *center, uint64_t seed, uint64_t offset_row, uint64_t offset_col,
+                                       void *codes_row, void *scales_row, float *unit_row, void *codes_col, void *scales_col,
+                                       float *unit_col, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * metis_nvfp4_quant_sr_both_padded and metis_nvfp4_quant_row_rht of a binary32 tensor (METIS_MODE_P32_F32) that also leave the
  * tensor rounded to bf16: copy bf16 [rows, cols], contiguous, 16-byte aligned.  The rank-r branch of a backward pass reads the
  * output gradient in bf16 whatever the quantizers' arithmetic is.

@@ -750,3 +750,23 @@ def test_running_mean_of_decode_steps_through_the_one_launch_path():
     assert all(torch.equal(a, b) for a, b in zip(outs[:3], outs[3:]))
     assert means[0].keys() == means[1].keys()
     assert all(torch.equal(means[0][k][0], means[1][k][0]) and means[0][k][1] == means[1][k][1] for k in means[0])
+
+
+@pytest.mark.parametrize("rows,cols,pad", [(256, 64, None), (32, 96, None), (272, 2080, None), (411, 160, 416), (2103, 512, 2112), (1, 32, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_both_packings_of_a_centred_gradient_from_one_pass(rows, cols, pad, dtype):
+    """ops.quantize_both_sr(center=): the bytes of the centred row and column quantizers called one after the other."""
+    from metis_hip import ops
+    mode = 1 if dtype == torch.bfloat16 else 0
+    x = _offset_activation(6000 + rows, rows, cols).to(dtype).cuda()
+    me = x.float().mean(dim=0).to(dtype)
+    more = {} if pad is None else {"pad_rows": pad}
+    row, col = ops.quantize_both_sr(x, mode, seed=9, offset_row=3, offset_col=1 << 33, center=me, **more)
+    want_row = ops.quantize(x, mode, sr=True, seed=9, offset=3, center=me)
+    want_col = ops.quantize(x, mode, col=True, sr=True, seed=9, offset=1 << 33, center=me, **more)
+    torch.cuda.synchronize()
+    for a, b in ((row, want_row), (col, want_col)):
+        assert torch.equal(a.codes, b.codes) and torch.equal(a.scales, b.scales) and torch.equal(a.unit, b.unit)
+    if dtype == torch.bfloat16:
+        with pytest.raises(ValueError):
+            ops.quantize_both_sr(x, 0, center=me, **more)          # a binary32 centre on bf16 values: the separate quantizers
