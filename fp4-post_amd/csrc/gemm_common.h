@@ -100,8 +100,10 @@ __device__ __forceinline__ bf16x8_t run_operand_bf16(const RunRegs<C>& r, int m,
     typedef float float2_t __attribute__((ext_vector_type(2)));
     const uint4 q = r.c[m >> 2];
     const uint32_t w = (m & 3) == 0 ? q.x : (m & 3) == 1 ? q.y : (m & 3) == 2 ? q.z : q.w;
-    const uint32_t byte = (r.sc[m >> 3] >> (8 * ((m >> 1) & 3))) & 0xffu;
-    const float dq = rb(e4m3_value(byte) * unit);
+    const uint32_t sc = r.sc[m >> 3];
+    const int sel = (m >> 1) & 3;                                  // (a constant once the caller's loop is unrolled)
+    const float sv = sel == 0 ? e4m3_value<0>(sc) : sel == 1 ? e4m3_value<1>(sc) : sel == 2 ? e4m3_value<2>(sc) : e4m3_value<3>(sc);
+    const float dq = rb(sv * unit);
     const float2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0);
     const float2_t p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
     const float2_t p2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2);

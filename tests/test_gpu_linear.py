@@ -1211,3 +1211,34 @@ def test_decode_quant_project_rejects_shapes_outside_its_domain():
     assert call(wsb=need - 1) != 0 and call(pb=16) != 0
     assert call(xp=None) != 0
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows", [1, 64, 256])
+def test_every_scale_byte_reaches_the_products(rows):
+    """Every E4M3 byte (both zeros, subnormal, largest; the two NaN bytes in the values alone) at every place of a scale word, through
+    dequantize and through the products that expand the weight themselves: one-hot rows pick single weight values, so sums are exact
+    and the reference's two roundings have to come out bit for bit."""
+    from metis_hip import ops
+    K, N = 512, 256
+    e2m1 = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6, -0.0, -0.5, -1, -1.5, -2, -3, -4, -6])
+    g = torch.Generator().manual_seed(17)
+    codes = torch.randint(0, 16, (N, K), generator=g)
+    sb = ((torch.arange(N)[:, None] + 37 * torch.arange(K // 16)[None, :]) % 256).to(torch.uint8)
+    unit = torch.tensor([0.0137])
+    pack = lambda c: (c[:, 0::2] | (c[:, 1::2] << 4)).to(torch.uint8)  # noqa: E731
+
+    def values(scales):
+        dq = (scales.view(torch.float8_e4m3fn).float() * unit).bfloat16().float().repeat_interleave(16, dim=1)
+        return (dq * e2m1[codes]).bfloat16()
+    w = ops.PackedNVFP4(pack(codes).cuda(), sb.cuda(), unit.cuda(), N, K, ops.MODE_PB16)
+    assert torch.equal(ops.dequantize(w, torch.bfloat16).cpu().nan_to_num(7.0), values(sb).nan_to_num(7.0))
+    sb[(sb & 127) == 127] = 0
+    w = ops.PackedNVFP4(pack(codes).cuda(), sb.cuda(), unit.cuda(), N, K, ops.MODE_PB16, persistent=True)
+    at = (torch.arange(rows) * 37 + 5) % K
+    one = torch.zeros(rows, K, dtype=torch.int64)
+    one[torch.arange(rows), at] = 2
+    a = ops.PackedNVFP4(pack(one).cuda(), torch.full((rows, K // 16), 0x38, dtype=torch.uint8, device="cuda"), torch.ones(1, device="cuda"),
+                        rows, K, ops.MODE_PB16)
+    op = ops.decode_operand(a, ops.MODE_PB16) if rows < 256 else None
+    got = ops.linear_fwd(a, w, reference_rounding=True, a_operand=op)
+    assert torch.equal(got.cpu(), values(sb)[:, at].T + 0.0)
