@@ -1457,151 +1457,157 @@ int deferred_scales(const void* deferred, int64_t rows, int64_t cols, int mode, 
 
 // ---------------------------------------------------------------------------------------------
 // "svd" mode of the activation / output-gradient decomposition (src/Metis/Metis/bitlinear.py:283-303): the tensor that is
-// quantized is x - ker with ker = (U diag(s)) V of rank r, and the caller goes on with ker + QDQ(x - ker).  ker is formed
-// in registers: a workgroup owns tiles of 64 rows x 256 columns, a thread one block of 16 columns in four rows, and the
-// factors pass through LDS sixteen ranks at a time.  Every element of ker is the chain
+// quantized is x - ker with ker = (U diag(s)) V of rank r, and the caller goes on with ker + QDQ(x - ker).  Every element of ker
+// is the chain
 //     acc = 0;  acc = fma(us[i][k], v[k][j], acc)  for k = 0 .. r-1 in that order, in binary32
 // (bf16 arithmetic: exact products of bf16 factors, the sum rounded to bf16 once, as a bf16 matrix product with
-// binary32 accumulation does) -- a fixed order, so that a CPU restatement reproduces the bits.  Then the residual
-// x - ker (rounded to the arithmetic's type) is encoded like any other block; the codes and the parked block maxima go
-// where the row quantizer puts them, and ker is written out only when the caller wants the dense result.
+// binary32 accumulation does) -- a fixed order, so that a CPU restatement reproduces the bits.  v_mfma_f32_32x32x2_f32 is that
+// chain for its two values of k (k = 0 from lanes 0..31, then k = 1 from lanes 32..63, each a fused multiply-add, subnormals
+// included; the tests hold it to the restatement bit for bit).
+//
+// A wave forms 32 rows x 64 columns and needs neither LDS nor a barrier: V's operand is a row of V as it lies (coalesced words), U's
+// are 16 bytes a lane along the rank, put in order by two half swaps, and 8 half swaps turn a lane's 16 sums into one block of 16
+// columns, ready for the encoder.  The four waves of a workgroup lie side by side: they read the same rows of U from L1 and write
+// whole lines of codes.  Then the residual x - ker (rounded to the arithmetic's type) is encoded like any other block; the codes and
+// the parked block maxima go where the row quantizer puts them, and ker is written out only when the caller wants the dense result.
+//
+// What bounds it: the SIMDs.  Binary32 MFMAs reach 137 TFLOP/s alone and vector FMAs 96, but the two do not run side by side (63 + 63
+// when mixed in one wave), so the products (14 us of the call at 4096 x 3584, r = 64) and the encoder's vector work add up.  Call
+// with its scales launch, in a graph, vector FMAs from LDS tiles before -> now: binary32 4096 x 3584 r = 64 39.5 -> 35.1 us, r = 32
+// 28.3 -> 26.7, 1000 x 2048 r = 64 19.1 -> 10.6, 128 x 1024 r = 32 13.4 -> 8.7; bf16 4096 x 3584 r = 64 39.3 -> 33.4, 2048 x 1536 r = 64
+// 19.7 -> 13.4.  64 rows a wave: 13.7 at 1000 x 2048 (half as many waves), 36.5 at the largest; x requested before the products: 38.1
+// (U's lines leave L1 meanwhile).
 // ---------------------------------------------------------------------------------------------
-constexpr int kLrRows = 64, kLrCols = 256, kLrRanks = 16;
+constexpr int kLrRows = 32, kLrCols = 256, kLrRanks = 16;
+typedef float lr_acc_t __attribute__((ext_vector_type(16)));
+
+// lanes 32..63 of a against lanes 0..31 of b
+__device__ __forceinline__ void swap_halves(float& a, float& b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
 
 template <int MODE, bool F32IN>
-__global__ __launch_bounds__(256) void quant_lowrank_residual_kernel(
+__global__ __launch_bounds__(256, 4) void quant_lowrank_residual_kernel(
     const void* __restrict__ xv, const void* __restrict__ usv, const void* __restrict__ vtv, uint32_t rows, uint32_t cols,
     uint32_t rank, uint2* __restrict__ codes, void* __restrict__ ws_amax_v, uint32_t* __restrict__ ws_gmax,
     void* __restrict__ ker_out, uint32_t tiles_c, uint32_t tiles)
 {
     static_assert(MODE == 0 || !F32IN, "bf16 arithmetic reads bf16 tensors");
-    // LDS layouts without bank conflicts: of V, quarter q of every thread's block of 16 lies side by side with the same
-    // quarter of the fifteen other blocks (a 16-byte read of sixteen lanes covers 256 contiguous bytes); the rows of
-    // U diag(s) are 80 bytes apart, so that the four row groups of a wave read from different banks.
-    __shared__ float4 s_v[kLrRanks][4][kLrCols / kBlock];
-    __shared__ __align__(16) float s_u[kLrRows][kLrRanks + 4];
-    const uint32_t t = threadIdx.x, cb = t & 15u, rg = t >> 4;
+    typedef typename std::conditional<MODE == 0, float, uint16_t>::type factor_t;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 31u, hi = lane >> 5;
     const uint32_t nbpr = cols / kBlock;
     float gmax = 0.0f;
     for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const uint32_t tr = tile / tiles_c, tc = tile - tr * tiles_c;
-        const uint32_t row0 = tr * kLrRows, col0 = tc * kLrCols;
-        float acc[4][kBlock];
+        const uint32_t row0 = tr * kLrRows, col0 = tc * kLrCols + wave * 64u;
+        if (col0 >= cols) continue;                             // (no barrier inside the loop)
+        // rows and columns beyond the tensor read its last ones: their products are not used
+        const factor_t* pv[2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (uint32_t b = 0; b < 2; ++b) pv[b] = static_cast<const factor_t*>(vtv) + (size_t)hi * cols + min(col0 + 32u * b + j, cols - 1u);
+        const factor_t* pu = static_cast<const factor_t*>(usv) + (size_t)min(row0 + j, rows - 1u) * rank + hi * 4u;
+        factor_t nv[2][4];                                      // V of ranks k0 + 2 s + hi
+        typedef typename std::conditional<MODE == 0, float4, uint2>::type four_t;
+        four_t nu;                                              // U diag(s) of ranks k0 + 4 hi ..
+        auto fetch = [&]() {
 #pragma unroll
-            for (int j = 0; j < kBlock; ++j) acc[i][j] = 0.0f;
-        // The factors of the next sixteen ranks are fetched into registers while the current ones are multiplied, and go to
-        // LDS between two barriers afterwards: their memory latency is off the critical path.
-        float pv[kBlock];
-        float4 pu;
-        auto fetch_chunk = [&](uint32_t k0) {
-            {   // V: rank k0 + t / 16, columns col0 + 16 (t % 16) ..; zeros beyond the tensor
-                const uint32_t k = k0 + rg, c = col0 + cb * kBlock;
+            for (int b = 0; b < 2; ++b) {
 #pragma unroll
-                for (int j = 0; j < kBlock; ++j) pv[j] = 0.0f;
-                if (c < cols) {
-                    if constexpr (MODE == 0) {
-                        const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(vtv) + (size_t)k * cols + c);
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) { const float4 f = p[q]; pv[4 * q] = f.x; pv[4 * q + 1] = f.y; pv[4 * q + 2] = f.z; pv[4 * q + 3] = f.w; }
-                    } else {
-                        const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(vtv) + (size_t)k * cols + c);
-                        unpack16(p[0], p[1], pv);
-                    }
-                }
+                for (int s = 0; s < 4; ++s) nv[b][s] = pv[b][(size_t)(2 * s) * cols];
+                pv[b] += (size_t)8 * cols;
             }
-            {   // U diag(s): row row0 + t / 4, ranks k0 + 4 (t % 4) ..
-                const uint32_t r = row0 + (t >> 2), k = k0 + (t & 3u) * 4u;
-                pu = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (r < rows) {
-                    if constexpr (MODE == 0) pu = *reinterpret_cast<const float4*>(static_cast<const float*>(usv) + (size_t)r * rank + k);
-                    else {
-                        const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(usv) + (size_t)r * rank + k);
-                        pu = make_float4(bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y));
-                    }
-                }
-            }
+            nu = *reinterpret_cast<const four_t*>(pu);
+            pu += 8;
         };
-        fetch_chunk(0);
-        for (uint32_t k0 = 0; k0 < rank; k0 += kLrRanks) {
-            __syncthreads();                                   // the previous chunk (or tile) has been read
-            {
+        lr_acc_t acc[2];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) s_v[rg][q][cb] = make_float4(pv[4 * q], pv[4 * q + 1], pv[4 * q + 2], pv[4 * q + 3]);
-                *reinterpret_cast<float4*>(&s_u[t >> 2][(t & 3u) * 4u]) = pu;
-            }
-            __syncthreads();
-            if (k0 + kLrRanks < rank) fetch_chunk(k0 + kLrRanks);
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int kq = 0; kq < kLrRanks / 4; ++kq) {
-                float4 u4[4];
+            for (int e = 0; e < 16; ++e) acc[b][e] = 0.0f;
+        fetch();
+        for (uint32_t k0 = 0; k0 < rank; k0 += 8) {
+            float fv[2][4];
+            float4 u;
+            if constexpr (MODE == 0) u = nu;
+            else u = make_float4(bf16_lo(nu.x), bf16_hi(nu.x), bf16_lo(nu.y), bf16_hi(nu.y));
 #pragma unroll
-                for (int i = 0; i < 4; ++i) u4[i] = *reinterpret_cast<const float4*>(&s_u[rg * 4 + i][kq * 4]);
+            for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    float vv[kBlock];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) { const float4 f = s_v[kq * 4 + kk][q][cb]; vv[4 * q] = f.x; vv[4 * q + 1] = f.y; vv[4 * q + 2] = f.z; vv[4 * q + 3] = f.w; }
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float uu = kk == 0 ? u4[i].x : kk == 1 ? u4[i].y : kk == 2 ? u4[i].z : u4[i].w;
-#pragma unroll
-                        for (int j = 0; j < kBlock; ++j) acc[i][j] = fmaf(uu, vv[j], acc[i][j]);
-                    }
+                for (int s = 0; s < 4; ++s) {
+                    if constexpr (MODE == 0) fv[b][s] = nv[b][s];
+                    else fv[b][s] = __uint_as_float((uint32_t)nv[b][s] << 16);
                 }
-            }
+            // (k0, k0 + 4), (k0 + 1, k0 + 5) -> (k0, k0 + 1), (k0 + 4, k0 + 5), and likewise the other pair
+            swap_halves(u.x, u.y);
+            swap_halves(u.z, u.w);
+            const float fu[4] = {u.x, u.z, u.y, u.w};
+            if (k0 + 8 < rank) fetch();
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fv[b][s], fu[s], acc[b], 0, 0, 0);
         }
-        const uint32_t cbg = tc * (kLrCols / kBlock) + cb;      // block column in the tensor
-        if (cbg < nbpr) {
+        const uint32_t row = row0 + j;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t row = row0 + rg * 4u + (uint32_t)i;
-                if (row >= rows) break;
-                const size_t e0 = (size_t)row * cols + (size_t)cbg * kBlock;
-                float v[kBlock];
-                if constexpr (F32IN) {
-                    const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(xv) + e0);
+        for (int b = 0; b < 2; ++b) {
+            // a lane holds columns 8 q + 4 hi + (0..3) of its row, q = 0..3: after the swaps the lower lanes have columns 0..15, the upper
+            // ones 16..31 of the 32
+            float ker[kBlock];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) { const float4 f = p[q]; v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w; }
-                } else {
-                    const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(xv) + e0);
-                    unpack16(p[0], p[1], v);
+            for (int e = 0; e < 8; ++e) {
+                float lo = acc[b][e], up = acc[b][e + 8];
+                swap_halves(lo, up);
+                ker[(e & 4) * 2 + (e & 3)] = lo;
+                ker[(e & 4) * 2 + (e & 3) + 4] = up;
+            }
+            const uint32_t cbg = col0 / kBlock + 2u * b + hi;
+            if (row >= rows || cbg >= nbpr) continue;
+            const size_t e0 = (size_t)row * cols + (size_t)cbg * kBlock;
+            float v[kBlock];
+            if constexpr (F32IN) {
+                const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(xv) + e0);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) { const float4 f = p[q]; v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w; }
+            } else {
+                const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(xv) + e0);
+                unpack16(p[0], p[1], v);
+            }
+            if constexpr (MODE == 0) {
+                if (ker_out) {
+                    float4* o = reinterpret_cast<float4*>(static_cast<float*>(ker_out) + e0);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) o[q] = make_float4(ker[4 * q], ker[4 * q + 1], ker[4 * q + 2], ker[4 * q + 3]);
                 }
-                if constexpr (MODE == 0) {
-                    if (ker_out) {
-                        float4* o = reinterpret_cast<float4*>(static_cast<float*>(ker_out) + e0);
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) o[q] = make_float4(acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]);
-                    }
+                for (int i = 0; i < kBlock; ++i) v[i] -= ker[i];
+            } else {
+                uint32_t kw[8];
 #pragma unroll
-                    for (int j = 0; j < kBlock; ++j) v[j] -= acc[i][j];
-                } else {
-                    uint32_t kw[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) kw[j] = bf16_bits(acc[i][2 * j]) | (bf16_bits(acc[i][2 * j + 1]) << 16);
-                    if (ker_out) {
-                        uint4* o = reinterpret_cast<uint4*>(static_cast<uint16_t*>(ker_out) + e0);
-                        o[0] = make_uint4(kw[0], kw[1], kw[2], kw[3]);
-                        o[1] = make_uint4(kw[4], kw[5], kw[6], kw[7]);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        v[2 * j] = rb(v[2 * j] - bf16_lo(kw[j]));
-                        v[2 * j + 1] = rb(v[2 * j + 1] - bf16_hi(kw[j]));
-                    }
+                for (int i = 0; i < 8; ++i) kw[i] = bf16_bits(ker[2 * i]) | (bf16_bits(ker[2 * i + 1]) << 16);
+                if (ker_out) {
+                    uint4* o = reinterpret_cast<uint4*>(static_cast<uint16_t*>(ker_out) + e0);
+                    o[0] = make_uint4(kw[0], kw[1], kw[2], kw[3]);
+                    o[1] = make_uint4(kw[4], kw[5], kw[6], kw[7]);
                 }
-                const float am = block_amax(v);
-                gmax = fmaxf(gmax, am);
-                const uint32_t blk = row * nbpr + cbg;
-                if constexpr (MODE == 0) {
-                    static_cast<float*>(ws_amax_v)[blk] = am;
-                    codes[blk] = encode_rne_wide(v, block_scalar_ieee(am));
-                } else {
-                    const float none[kBlock] = {};
-                    static_cast<uint16_t*>(ws_amax_v)[blk] = (uint16_t)(__float_as_uint(am) >> 16);
-                    codes[blk] = encode_block<1, false>(v, block_scalar<1>(am), none);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    v[2 * i] = rb(v[2 * i] - bf16_lo(kw[i]));
+                    v[2 * i + 1] = rb(v[2 * i + 1] - bf16_hi(kw[i]));
                 }
+            }
+            const float am = block_amax(v);
+            gmax = fmaxf(gmax, am);
+            const uint32_t blk = row * nbpr + cbg;
+            if constexpr (MODE == 0) {
+                static_cast<float*>(ws_amax_v)[blk] = am;
+                codes[blk] = encode_rne_wide(v, block_scalar_ieee(am));
+            } else {
+                const float none[kBlock] = {};
+                static_cast<uint16_t*>(ws_amax_v)[blk] = (uint16_t)(__float_as_uint(am) >> 16);
+                codes[blk] = encode_block<1, false>(v, block_scalar<1>(am), none);
             }
         }
     }
@@ -1662,7 +1668,6 @@ int quantize_lowrank_residual(const void* x, bool x_f32, const void* us, const v
     const uint32_t tiles_c = (uint32_t)((cols + kLrCols - 1) / kLrCols);
     const int64_t tiles = (int64_t)((rows + kLrRows - 1) / kLrRows) * tiles_c;
     int64_t g = tiles;
-    if (g > (int64_t)device_cus() * 3) g = (int64_t)device_cus() * 3;          // three workgroups per CU are resident (139 VGPRs)
     if (g > kMaxGroups) g = kMaxGroups;
     const uint32_t nblocks = (uint32_t)(rows * cols / kBlock);
 #define METIS_LR(M, F)                                                                                                          \

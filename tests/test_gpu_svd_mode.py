@@ -82,6 +82,24 @@ def test_against_the_oracle_on_ragged_shapes(rows, cols, r, dt):
     assert float(packed.unit.cpu()) == float(unit)
 
 
+@pytest.mark.parametrize("rows,cols,r", [(1, 48, 16), (31, 80, 16), (32, 64, 48), (33, 320, 64), (65, 272, 112)])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -68, 2.0 ** 60])
+def test_the_low_rank_product_is_the_ordered_chain(rows, cols, r, scale):
+    """ker is fma(us[i][k], v[k][j], acc), k upwards, in binary32: with x = that chain from the oracle the residual has to vanish, at the
+    edges of a wave's 32 rows and 64 columns, with products below and near the smallest normal number and near the largest one."""
+    from metis_hip import ops
+    from oracle import c_oracle
+    g = torch.Generator().manual_seed(rows + cols + r)
+    us, vt = (torch.randn(rows, r, generator=g) * scale), (torch.randn(r, cols, generator=g) * scale)
+    us[0, 1] = 0.0
+    ker = c_oracle.lowrank_product(us, vt)
+    if scale < 1:
+        assert ((ker.abs() < 2.0 ** -126) & (ker != 0)).any()
+    packed, dense = ops.quantize_lowrank_residual(ker.cuda(), us.cuda(), vt.cuda(), ops.MODE_P32, dense=True)
+    torch.cuda.synchronize()
+    assert not packed.codes.any() and torch.equal(dense.cpu(), ker)
+
+
 def test_shapes_the_kernel_does_not_take_are_refused():
     from metis_hip import ops
     x = torch.zeros(32, 64, dtype=torch.bfloat16, device="cuda")
