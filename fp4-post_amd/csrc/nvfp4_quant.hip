@@ -496,9 +496,10 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
 // tensor; rows past `valid` have a zero residual.  The MLP step of 2103 tokens, 3584 -> 18944: 3824 us with two
 // passes over each dY, 3806 with one (the encoders bound it, not the second read).
 // ---------------------------------------------------------------------------------------------
+// (Five waves per SIMD asked for where the compiler gives them anyway, bf16 without a centre, cost it two registers: 18944 x 3584 60.9 -> 63.2.)
 constexpr uint32_t kBothRun = 16;
 template <int MODE, bool WIDE = false, bool CEN = false>
-__global__ __launch_bounds__(256, CEN ? 4 : 5) void quant_codes_both_kernel(
+__global__ __launch_bounds__(256, CEN ? 4 : WIDE ? 5 : 1) void quant_codes_both_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, uint64_t seed, uint64_t offset_row, uint64_t offset_col,
     uint2* __restrict__ codes_row, void* __restrict__ amax_row_v, uint2* __restrict__ codes_col, void* __restrict__ amax_col_v,
     uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, uint32_t valid, uint16_t* __restrict__ copy = nullptr,
@@ -1340,7 +1341,12 @@ int quantize_both_sr(const void* x, int64_t rows, int64_t cols, int64_t ld, int 
     const uint32_t tiles_r = (uint32_t)((rows / kBlock + kColTileBlocks - 1) / kColTileBlocks);
     const uint32_t tiles_c = (uint32_t)((cols + kColTileCols - 1) / kColTileCols);
     const int64_t tiles = (int64_t)tiles_r * tiles_c;
-    int64_t g = tiles;
+    // One workgroup for every place of the last, partly filled, span of eight runs while they all fit the device: a grid of as many
+    // workgroups as tiles left the tiles behind the empty places to workgroups that had one already (two of 16 workgroups took all of
+    // 256 x 1024).  With the scale bytes, bf16 arithmetic, before -> now: 256 x 1024 42.3 -> 9.9 us, 512 x 1536 19.5 -> 10.0, 512 x 8960
+    // 16.3 -> 13.1, 1488 x 3648 16.9 -> 14.0, 2048 x 8960 26.2 -> 23.9; whole spans and tensors beyond the device's capacity as before.
+    const int64_t span = 8 * kBothRun;
+    int64_t g = (tiles + span - 1) / span * span;
     const int64_t cap = center ? (f32in ? both_capacity<0, true, true>() : both_capacity<1, false, true>())
                                : f32in ? both_capacity<0, true, false>() : mode == 0 ? both_capacity<0, false, false>() : both_capacity<1, false, false>();
     if (g > cap) g = cap;

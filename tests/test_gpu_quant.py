@@ -827,3 +827,15 @@ def test_quantizers_of_a_binary32_gradient_leave_its_bf16_rounding(ops, rows, co
         ops.quantize_rht(x.bfloat16(), 0, 1, bf16_copy=copy)
     with pytest.raises(ValueError):
         ops.quantize_both_sr(x, 0, bf16_copy=copy.float(), **more)
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 64), (256, 1024), (272, 1040), (512, 1536), (1488, 3648), (4112, 2064)])
+def test_both_packings_cover_a_partly_filled_span_of_tiles(rows, cols):
+    """Tiles that do not fill their last span of eight runs, fewer and more than the device holds at once: the bytes of the two calls."""
+    from metis_hip import ops
+    x = synthetic_activation(900 + rows, rows, cols).cuda()
+    for xin, mode, center in ((x, ops.MODE_PB16, None), (x.float() * 1.001, ops.MODE_P32, None), (x, ops.MODE_PB16, x.float().mean(0).bfloat16())):
+        got = ops.quantize_both_sr(xin, mode, seed=3, offset_row=5, offset_col=1 << 33, center=center)
+        want = [ops.quantize(xin, mode, col=c, sr=True, seed=3, offset=o, center=center) for c, o in ((False, 5), (True, 1 << 33))]
+        for p, q in zip(got, want):
+            assert torch.equal(p.codes, q.codes) and torch.equal(p.scales, q.scales) and torch.equal(p.unit, q.unit)
