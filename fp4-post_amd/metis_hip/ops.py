@@ -198,12 +198,19 @@ def _lowrank_rows_workspace_bytes(M: int, R: int, K: int, device_index: int) -> 
     return int(load().metis_lowrank_project_rows_workspace_bytes(M, R, K))       # depends on the device's CU count only
 
 
-def _workspace(rows: int, cols: int, device: torch.device) -> torch.Tensor:
-    need = _quant_workspace_bytes(rows, cols)
-    key = (device.index, _stream())
+def _workspace(rows: int, cols: int, device: torch.device, zeroed: bool = False, tensors: int = 1) -> torch.Tensor:
+    """Scratch of a quantizer's call (for `tensors` packings of [rows, cols]): kept per stream, grown as needed, zero when first used.
+    A captured call gets memory of its graph's pool that nobody else is handed, and takes no kept area: a fill recorded into a graph
+    has not run when the next eager call comes, a replay may run beside eager work of the stream it was captured on, and a kept
+    area is freed when it grows, whatever graph still writes to it.  zeroed: the call reads words that have to be zero (a maximum
+    taken over the grid); the others write every word that they read."""
+    need = tensors * _quant_workspace_bytes(rows, cols)
+    if torch.cuda.is_current_stream_capturing():
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        return ws.fill_(0) if zeroed else ws                       # (a fill kernel: no memset is recorded into a graph)
+    key = (device.index, _stream(), tensors)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < need:
-        # zero-filled once by a fill kernel (not a memset, which must not be recorded into a captured graph)
         ws = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=device).fill_(0)
         _workspaces[key] = ws
     return ws
@@ -289,7 +296,7 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
             check(rc, "metis_nvfp4_quant_row_deferred", x.shape)
         return PackedNVFP4(codes, None, unit, prow, pcol, mode, deferred=parked)
     scales = torch.empty(prow, pcol // BLOCK, dtype=torch.uint8, device=dev)
-    ws = _workspace(rows, cols, dev)
+    ws = _workspace(rows, cols, dev, zeroed=resident)
     if center is not None:
         cen = center.reshape(-1).to(device=dev, dtype=torch.bfloat16 if mode == MODE_PB16 else torch.float32).contiguous()
         if cen.numel() != cols:
@@ -411,11 +418,7 @@ def roundtrip(x: torch.Tensor, spin_limit: int = 0) -> torch.Tensor | None:
     x2 = x if (x.dim() == 2 and x.is_contiguous()) else x.reshape(-1, x.shape[-1]).contiguous()
     rows, cols = x2.shape
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    if rows * cols > _ROUNDTRIP_FOLDED and torch.cuda.is_current_stream_capturing():
-        # a graph has an area of its own for the grid's maximum: it may be replayed beside other work of the stream it was captured on
-        ws = torch.empty(_quant_workspace_bytes(1, BLOCK), dtype=torch.uint8, device=x.device).fill_(0)
-    else:
-        ws = _workspace(1, BLOCK, x.device)
+    ws = _workspace(1, BLOCK, x.device, zeroed=rows * cols > _ROUNDTRIP_FOLDED)
     rc = load().metis_nvfp4_roundtrip(x2.data_ptr(), rows, cols, MODE_PB16 if x.dtype == torch.bfloat16 else _lib.MODE_P32_F32, out.data_ptr(),
                                       ws.data_ptr(), ws.numel(), int(spin_limit), _stream())
     if rc == _lib.E_TOO_LARGE:
@@ -500,12 +503,7 @@ def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, of
         packs.append((torch.empty(prow, pcol // 2, dtype=torch.uint8, device=dev),
                       torch.empty(prow, pcol // BLOCK, dtype=torch.uint8, device=dev),
                       torch.empty(1, dtype=torch.float32, device=dev)))
-    need = 2 * L.metis_nvfp4_workspace_bytes(rows, cols)
-    key = (dev.index, _stream(), "both")
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=dev).fill_(0)
-        _workspaces[key] = ws
+    ws = _workspace(rows, cols, dev, tensors=2)
     (cr, sr_, ur), (cc, sc, uc) = packs
     if center is not None and rows * cols:
         rc = L.metis_nvfp4_quant_sr_both_centered(x2.data_ptr(), have, rows, cols, x2.stride(0), kmode, center.data_ptr(), seed & (2 ** 64 - 1),

@@ -791,6 +791,43 @@ def test_round_trip_beyond_the_registers_and_from_a_captured_graph(ops):
         assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
 
 
+def test_captured_quantizers_and_eager_calls_on_the_stream_of_the_capture(ops, monkeypatch):
+    """The first calls on a stream are captured ones, then an eager round trip comes on it before any replay, then replays beside larger
+    eager calls that make the kept scratch grow: every result has the bits of the calls on a stream of their own."""
+    from metis_hip import quant_func
+    q = quant_func["nvfp4e2m1bnosr"]
+    x = torch.randn(2048, 2048, device="cuda").bfloat16()
+
+    def calls():
+        row, col = ops.quantize_both_sr(x, 1, seed=3, offset_row=5, offset_col=1 << 30)
+        one = ops.quantize(x, 0, resident=True)
+        return (q.quantize_dequantize(x), row.codes, row.scales, col.codes, col.scales, one.codes, one.scales, ops.quantize(x, 1).scales,
+                q.quantize_dequantize(x[:64]))
+    calls()                                                        # code objects are loaded outside the capture
+    torch.cuda.synchronize()
+    monkeypatch.setattr(ops, "_workspaces", {})                    # as on a stream that nothing ran on yet
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        captured = calls()
+    assert not ops._workspaces
+    for k in range(4):
+        x.copy_(torch.randn(2048, 2048, device="cuda") * (1 + k))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            eager = q.quantize_dequantize(x)
+        torch.cuda.synchronize()
+        want = calls()
+        assert torch.equal(eager.view(torch.int16), want[0].view(torch.int16))
+        graph.replay()
+        with torch.cuda.stream(side):
+            ops.quantize(torch.randn(2048 + 512 * k, 4096, device="cuda").bfloat16(), 1)
+        torch.cuda.synchronize()
+        for a, b in zip(captured, want):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), k
+
+
 def test_both_packings_of_a_whole_row_count_are_tensors_of_their_own(ops):
     """Only a padded call hands out views (the row packing of the tensor's own rows)."""
     x = torch.randn(64, 128, device="cuda").bfloat16()

@@ -472,3 +472,36 @@ def test_values_without_the_autograd_function_only_where_nothing_may_record_or_t
         assert seen and all(seen)
     with torch.inference_mode():
         assert not _autograd_may_see()
+
+
+def test_scratch_made_under_capture_is_handed_to_nobody_else(monkeypatch):
+    """ops._workspace: a fill recorded into a graph has not run when the next eager call on that stream asks for words that are zero, and a
+    kept area is freed when it grows: captured calls neither leave areas behind nor take kept ones."""
+    from metis_hip import ops
+    monkeypatch.setattr(ops, "_workspaces", {})
+    monkeypatch.setattr(ops, "_stream", lambda: 77)
+    capturing = True
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    fill, recorded, run = torch.Tensor.fill_, [], []
+
+    def fill_(t, value):
+        (recorded if capturing else run).append(t.data_ptr())
+        return t if capturing else fill(t, value)
+    monkeypatch.setattr(torch.Tensor, "fill_", fill_)
+    cpu = torch.device("cpu")
+    first = ops._workspace(64, 64, cpu)
+    capturing = False
+    kept = ops._workspace(64, 64, cpu)
+    assert kept.data_ptr() != first.data_ptr() and run == [kept.data_ptr()] and not kept.any()
+    assert ops._workspace(1, 16, cpu) is kept                      # kept per stream, as before
+    capturing = True
+    captured = ops._workspace(64, 64, cpu)
+    assert captured.data_ptr() != kept.data_ptr() and captured.numel() >= ops._quant_workspace_bytes(64, 64)
+    assert not recorded                                            # (and a fill is recorded only for calls that read zero words)
+    zeroed = ops._workspace(1, 16, cpu, zeroed=True)
+    assert recorded == [zeroed.data_ptr()] and zeroed.data_ptr() != kept.data_ptr()
+    pair = ops._workspace(64, 64, cpu, tensors=2)
+    assert pair.numel() >= 2 * ops._quant_workspace_bytes(64, 64)
+    capturing = False
+    assert ops._workspace(64, 64, cpu) is kept
+    assert ops._workspace(64, 64, cpu, tensors=2).data_ptr() not in (kept.data_ptr(), pair.data_ptr())   # (two packings: an area of their own)
