@@ -85,8 +85,8 @@ int quantize_lowrank_residual(const void* x, bool x_f32, const void* us, const v
                               hipStream_t st);
 int quantize_dequantize_row(const void* x, int64_t rows, int64_t cols, int mode, void* codes, void* scales, float* unit, void* out,
                             void* workspace, size_t workspace_bytes, hipStream_t st);
-// the dequantized values alone, bf16 (METIS_MODE_PB16) or binary32 (METIS_MODE_P32_F32), in one launch; METIS_E_TOO_LARGE when the
-// device's registers do not hold the codes; nvfp4_roundtrip.hip
+// the dequantized values alone, bf16 (METIS_MODE_PB16) or binary32 (METIS_MODE_P32_F32), in one launch; METIS_E_TOO_LARGE when half
+// of the device's registers do not hold the codes; nvfp4_roundtrip.hip
 int roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, void* workspace, size_t workspace_bytes, uint32_t spin_limit,
               hipStream_t st);
 int dequantize(const void* codes, const void* scales, const float* unit, int64_t rows, int64_t cols, int mode, void* out,

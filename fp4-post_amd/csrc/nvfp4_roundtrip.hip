@@ -10,7 +10,7 @@ namespace metis {
 // ---------------------------------------------------------------------------------------------
 // A code depends on its block, the value it stands for also on the tensor maximum.  Between the two nothing has to leave the chip:
 //   small tensors: each workgroup folds the maximum of the whole tensor itself, from L2, then takes its own blocks;
-//   others, while the codes fit the registers: every workgroup reads and encodes its blocks, the maximum is taken over the grid,
+//   others, while the codes fit half of the registers: every workgroup reads and encodes its blocks, the maximum is taken over the grid,
 //   and the codes are decoded where they are.
 // One launch either way.  (Codes and parked maxima through memory, quantize_dequantize_row, move 5.3 B per bf16 element and 9.5 B per
 // binary32 element instead of 4 and 8, and take a second launch.)
@@ -134,12 +134,21 @@ __global__ __launch_bounds__(kRoundtripSmallThreads) void roundtrip_small_kernel
 }
 
 // ---------------------------------------------------------------------------------------------
-// A tensor whose codes fit the chip's registers: read once and encoded on the way (a half block leaves one word of codes and its
+// A tensor whose codes fit half of the chip's registers: read once and encoded on the way (a half block leaves one word of codes and its
 // block's maximum, a third of itself in bf16, a quarter in binary32), the maximum taken over the grid (grid_max.h), then decoded
 // and written: 4 or 8 B per element, nothing in between.  HBM-bound, with the wait for the grid's maximum (about 4 us) between the read
-// and the write.  Microseconds, packed form through memory in two launches | this: bf16 1024 x 4096 15.4 | 8.8 (eager), 4096 x 4096 21.7 |
-// 17.0, 8192 x 4096 36.0 | 30.4, 16384 x 4096 64.6 | 54.2; binary32 2048 x 4096 20.7 | 17.8, 8192 x 4096 57.4 | 45.5.  (x itself kept in
-// registers and encoded after the wait: 8192 x 4096 32.0.  x read a second time in a second launch: 35.2.)
+// and the write.  Microseconds between events, packed form through memory in two launches | this: bf16 2048 x 4096 24.1 | 13.6, 4096 x 4096
+// 25.0 | 20.5, 8192 x 4096 39.2 | 31.4; binary32 3072 x 4096 29.0 | 25.4, 4096 x 4096 34.7 | 30.2.  (x itself kept in registers and
+// encoded after the wait: 8192 x 4096 32.0.  x read a second time in a second launch: 35.2.)
+//
+// The grid is at most HALF of what the device holds (more half blocks to a thread instead).  Workgroups that wait keep their places, so
+// a grid that needs every place of the device makes no progress until whatever else runs has left all of it, and two of them in parts
+// on the device wait for each other until they give up; then one workgroup writes everything that was left, in milliseconds.  Per call
+// beside other work, packed form | half of the device | all of it: bf16 8192 x 4096 beside copies of 2 GiB 80 us | 56 | 881, three streams of
+// round trips 97 | 72 | 7165; binary32 4096 x 4096 beside exp of 512 Mi elements 65 | 50 | 4850, three streams 85 | 70 | 3314.  Between
+// a half and all of it (bf16 12288 x 4096, three quarters): three streams 140 | - | 956.  Alone, with all of the device | half:
+// bf16 4096 x 4096 17.5 | 18.4, 5120 x 4096 20.6 | 22.2, 8192 x 4096 31.0 | 30.6.  Tensors beyond take the packed form: bf16
+// 12288 x 4096 51.4 where all of the device gave 41.6, binary32 8192 x 4096 58.3 where it gave 45.9.
 // A workgroup that cannot wait any longer leaves its values to the last one, which reads x again.
 // ---------------------------------------------------------------------------------------------
 template <bool F32, int NH>
@@ -261,7 +270,7 @@ template <bool F32, int NH>
 static bool try_resident(const uint4* x, void* out, uint32_t nhalves, uint32_t* sync, uint32_t spin_limit, hipStream_t st)
 {
     const int64_t need = ((int64_t)nhalves + 256 * NH - 1) / (256 * NH);
-    if (need > resident_capacity<F32, NH>()) return false;
+    if (need > resident_capacity<F32, NH>() / 2) return false;     // (why half: beside the kernel)
     hipLaunchKernelGGL((roundtrip_resident_kernel<F32, NH>), dim3((unsigned)need), dim3(256), 0, st, x, out, nhalves, sync, spin_limit);
     return true;
 }

@@ -412,8 +412,8 @@ def quantize_dequantize_f32(x: torch.Tensor) -> tuple[PackedNVFP4, torch.Tensor]
 
 def roundtrip(x: torch.Tensor, spin_limit: int = 0) -> torch.Tensor | None:
     """dequantize(quantize(x)) of a bf16 tensor in bf16 arithmetic or a binary32 tensor in binary32 arithmetic, round to nearest: the
-    same values in x's shape and type, from one launch that packs nothing.  None where the device's registers do not hold the
-    tensor's codes.  spin_limit: polls for the grid's maximum before a workgroup leaves its values to the last one (0: the
+    same values in x's shape and type, from one launch that packs nothing.  None where half of the device's registers do not hold
+    the tensor's codes.  spin_limit: polls for the grid's maximum before a workgroup leaves its values to the last one (0: the
     library's limit)."""
     x2 = x if (x.dim() == 2 and x.is_contiguous()) else x.reshape(-1, x.shape[-1]).contiguous()
     rows, cols = x2.shape

@@ -101,9 +101,10 @@ int metis_nvfp4_quant_dequant_row_f32(const void *x, int64_t rows, int64_t cols,
 
 /*
  * The dequantized values of that round trip alone, in ONE launch that reads x once: no codes, scale bytes or unit are written, the
- * codes stay in registers until the tensor maximum is known.  METIS_E_TOO_LARGE for a tensor whose codes the device's registers do
- * not hold (beyond 8192 x 4096 in binary32, 16384 x 4096 in bf16 on a device of 256 compute units).  The grid-wide maximum works as in
- * metis_nvfp4_quant_row_resident: bounded polls (spin_limit, 0 for the default), the result does not depend on them.
+ * codes stay in registers until the tensor maximum is known.  METIS_E_TOO_LARGE for a tensor whose codes half of the device's
+ * registers do not hold (beyond 5120 x 4096 in binary32, 8192 x 4096 in bf16 on a device of 256 compute units: a grid that needs
+ * all of the device waits for every other kernel on it).  The grid-wide maximum works as in metis_nvfp4_quant_row_resident:
+ * bounded polls (spin_limit, 0 for the default), the result does not depend on them.
  *   x, out     [rows, cols], contiguous: bf16 with METIS_MODE_PB16, float with METIS_MODE_P32_F32; 16-byte aligned
  *   workspace  metis_nvfp4_workspace_bytes(1, 16) bytes, 256-byte aligned, zero when first used; calls that share it are ordered.
  *              Not read for small tensors (up to 128 K elements)

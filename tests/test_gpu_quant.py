@@ -740,9 +740,9 @@ def test_binary32_round_trip_from_one_call(ops, rows, cols):
 
 
 # one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (192 x 1024 elements in bf16, 128 x
-# 1024 in binary32), leading dimensions, four and eight half blocks per thread
+# 1024 in binary32), leading dimensions, four, eight and sixteen half blocks per thread, the last workgroup partly filled
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("shape", [(1, 16), (3, 48), (5, 7, 80), (128, 1024), (129, 1024), (192, 1024), (193, 1024), (2049, 4080), (8191, 4096)])
+@pytest.mark.parametrize("shape", [(1, 16), (3, 48), (5, 7, 80), (128, 1024), (129, 1024), (192, 1024), (193, 1024), (2049, 4080), (3001, 4080), (4099, 4096), (8191, 4096)])
 def test_round_trip_values_without_a_packed_tensor(ops, dtype, shape):
     """ops.roundtrip: the values of quantize + dequantize bit for bit, with signed zeros, subnormal blocks, an infinity and a NaN."""
     from metis_hip import quant_func
@@ -758,12 +758,50 @@ def test_round_trip_values_without_a_packed_tensor(ops, dtype, shape):
             flat[flat.numel() // 2] = value
         want = ops.dequantize(ops.quantize(x, mode), dtype).reshape(shape)
         # (spin_limit=1: workgroups leave their values to the last one)
-        for got in (ops.roundtrip(x), ops.roundtrip(x, spin_limit=1), q.quantize_dequantize(x)):
+        at_once = [ops.roundtrip(x), ops.roundtrip(x, spin_limit=1)]
+        if dtype == torch.float32 and x.numel() > 5120 * 4096:      # half of the device (256 CUs) does not hold the codes
+            assert at_once == [None, None]
+            at_once = []
+        for got in (*at_once, q.quantize_dequantize(x)):
             assert got.shape == x.shape and got.dtype == dtype and not got.requires_grad
             assert torch.equal(got.view(bits), want.view(bits)), (shape, value)
     strided = x.movedim(0, -1)
     if strided.shape[-1] % 16 == 0:
         assert torch.equal(q.quantize_dequantize(strided).view(bits), q.quantize_dequantize(strided.contiguous()).view(bits))
+
+
+def test_round_trips_on_several_streams_do_not_wait_for_each_other(ops, monkeypatch):
+    """A grid takes at most half of the device: three streams of the largest round trips side by side, no workgroup gives up waiting (its flag
+    in the area of the grid's maximum stays zero), and the bits are those of a call alone."""
+    from metis_hip import quant_func
+    q = quant_func["nvfp4e2m1bnosr"]
+    x = torch.randn(8192, 4096, device="cuda").bfloat16()
+    want = q.quantize_dequantize(x)
+    monkeypatch.setattr(ops, "_workspaces", {})
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    wide = torch.randn(8192, 8192, device="cuda").bfloat16()
+    outs = [None] * 3
+
+    def calls(n):
+        for _ in range(n):
+            for i, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    outs[i] = q.quantize_dequantize(x)
+    torch.cuda.synchronize()
+    calls(2)                                                       # the results' memory is there: no allocation waits for the device
+    torch.cuda.synchronize()
+    for _ in range(4):                                             # the calls are queued before the first one starts
+        wide @ wide
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    calls(12)
+    torch.cuda.synchronize()
+    for s in streams:
+        area = ops._workspaces[(x.device.index, s.cuda_stream, 1)]
+        assert int(area[16384:16384 + 8].view(torch.int64)) == 14   # the calls counted
+        assert not area[16384 + 4224 * 4:16384 + (4224 + 4096) * 4].any()
+    assert all(torch.equal(o.view(torch.int16), want.view(torch.int16)) for o in outs)
+    assert ops.roundtrip(torch.zeros(8208, 4096, dtype=torch.bfloat16, device="cuda")) is None
 
 
 def test_round_trip_beyond_the_registers_and_from_a_captured_graph(ops):
@@ -773,7 +811,11 @@ def test_round_trip_beyond_the_registers_and_from_a_captured_graph(ops):
     assert ops.roundtrip(big) is None
     want = ops.dequantize(ops.quantize(big, 0), torch.float32)
     assert torch.equal(q.quantize_dequantize(big).view(torch.int32), want.view(torch.int32))
-    del big, want
+    half = big.bfloat16()
+    assert ops.roundtrip(half) is None
+    want = ops.dequantize(ops.quantize(half, 1), torch.bfloat16)
+    assert torch.equal(q.quantize_dequantize(half).view(torch.int16), want.view(torch.int16))
+    del big, half, want
     x = torch.randn(1024, 2048, device="cuda").bfloat16()
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
