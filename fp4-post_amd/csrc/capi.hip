@@ -123,6 +123,11 @@ int metis_nvfp4_quant_dequant_row_f32(const void* x, int64_t rows, int64_t cols,
     return quantize_dequantize_row(x, rows, cols, METIS_MODE_P32_F32, codes, scales, unit, out, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+int metis_nvfp4_roundtrip_applies(int64_t rows, int64_t cols, int mode, size_t* workspace_bytes)
+{
+    return roundtrip_applies(rows, cols, mode, workspace_bytes);
+}
+
 int metis_nvfp4_roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, void* workspace, size_t workspace_bytes, uint32_t spin_limit,
                           void* stream)
 {

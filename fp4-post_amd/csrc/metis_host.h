@@ -89,6 +89,7 @@ int quantize_dequantize_row(const void* x, int64_t rows, int64_t cols, int mode,
 // of the device's registers do not hold the codes; nvfp4_roundtrip.hip
 int roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, void* workspace, size_t workspace_bytes, uint32_t spin_limit,
               hipStream_t st);
+int roundtrip_applies(int64_t rows, int64_t cols, int mode, size_t* bytes);   // its code for these sizes, and the bytes of scratch that it reads
 int dequantize(const void* codes, const void* scales, const float* unit, int64_t rows, int64_t cols, int mode, void* out,
                int out_dtype, hipStream_t st);
 int block_scalars(const void* x, int64_t rows, int64_t cols, int mode, void* s, hipStream_t st);

@@ -12,7 +12,7 @@ namespace metis {
 //   small tensors: each workgroup folds the maximum of the whole tensor itself, from L2, then takes its own blocks;
 //   others, while the codes fit half of the registers: every workgroup reads and encodes its blocks, the maximum is taken over the grid,
 //   and the codes are decoded where they are.
-// One launch either way.  (Codes and parked maxima through memory, quantize_dequantize_row, move 5.3 B per bf16 element and 9.5 B per
+// One launch either way (behind one that clears the area of the grid's maximum where the call is captured, ops.py).  (Codes and parked maxima through memory, quantize_dequantize_row, move 5.3 B per bf16 element and 9.5 B per
 // binary32 element instead of 4 and 8, and take a second launch.)
 // The values are those of quantize + dequantize bit for bit: the same maxima, the same encoders, the same products.
 // ---------------------------------------------------------------------------------------------
@@ -267,37 +267,64 @@ static int resident_capacity()
     return cached[dev] < 0 ? 0 : (cached[dev] > kFusedMaxGrid ? kFusedMaxGrid : cached[dev]);
 }
 template <bool F32, int NH>
-static bool try_resident(const uint4* x, void* out, uint32_t nhalves, uint32_t* sync, uint32_t spin_limit, hipStream_t st)
+static int64_t resident_grid(uint32_t nhalves) { return ((int64_t)nhalves + 256 * NH - 1) / (256 * NH); }
+template <bool F32, int NH>
+static bool resident_fits(uint32_t nhalves) { return resident_grid<F32, NH>(nhalves) <= resident_capacity<F32, NH>() / 2; }   // (why half: beside the kernel)
+
+// half blocks per thread of the widest grid that fits, 0: none does
+template <bool F32>
+static int resident_halves(uint32_t nhalves)
 {
-    const int64_t need = ((int64_t)nhalves + 256 * NH - 1) / (256 * NH);
-    if (need > resident_capacity<F32, NH>() / 2) return false;     // (why half: beside the kernel)
-    hipLaunchKernelGGL((roundtrip_resident_kernel<F32, NH>), dim3((unsigned)need), dim3(256), 0, st, x, out, nhalves, sync, spin_limit);
-    return true;
+    return resident_fits<F32, 4>(nhalves) ? 4 : resident_fits<F32, 8>(nhalves) ? 8 : resident_fits<F32, 16>(nhalves) ? 16 : 0;
 }
 
 template <bool F32>
-static bool launch_resident(const uint4* x, void* out, uint32_t nhalves, uint32_t* sync, uint32_t spin_limit, hipStream_t st)
+static void launch_resident(int nh, const uint4* x, void* out, uint32_t nhalves, uint32_t* sync, uint32_t spin_limit, hipStream_t st)
 {
-    return try_resident<F32, 4>(x, out, nhalves, sync, spin_limit, st) || try_resident<F32, 8>(x, out, nhalves, sync, spin_limit, st) ||
-           try_resident<F32, 16>(x, out, nhalves, sync, spin_limit, st);
+#define METIS_RT(NH) hipLaunchKernelGGL((roundtrip_resident_kernel<F32, NH>), dim3((unsigned)resident_grid<F32, NH>(nhalves)), dim3(256), 0, st, x, out, \
+                                        nhalves, sync, spin_limit)
+    if (nh == 4) METIS_RT(4); else if (nh == 8) METIS_RT(8); else METIS_RT(16);
+#undef METIS_RT
 }
 
 // The whole-tensor fold while it costs no more than taking the maximum over the grid.  Device time, fold | grid: bf16 128 x 1024 4.6 |
 // 6.8 us, 192 x 1024 5.6 | 6.9; binary32, twice the bytes to fold, 77 x 1536 6.0 | 6.9, 128 x 1024 6.2 | 6.9.
 static bool small_tensor(int64_t nhalves, bool f32) { return nhalves <= (f32 ? 16384 : 24576); }
 
-int roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, void* workspace, size_t bytes, uint32_t spin_limit, hipStream_t st)
+// What a call of these sizes takes: half blocks per thread of the resident kernel in *nh (0: the fold), or why it is refused.
+static int roundtrip_form(int64_t rows, int64_t cols, int mode, int* nh)
 {
+    *nh = 0;
     if (rows < 0 || cols < 0) return METIS_E_ARG;
     if (mode != METIS_MODE_PB16 && mode != METIS_MODE_P32_F32) return METIS_E_ARG;
     if (cols % kBlock) return METIS_E_SHAPE;
     if (rows == 0 || cols == 0) return METIS_OK;
-    if (!x || !out || ((uintptr_t)x % 16) || ((uintptr_t)out % 16)) return METIS_E_ARG;
     if (rows > ((int64_t)1 << 31) / cols) return METIS_E_TOO_LARGE;
     const uint32_t nhalves = (uint32_t)(rows * cols / 8);
     const bool f32 = mode == METIS_MODE_P32_F32;
+    if (small_tensor(nhalves, f32)) return METIS_OK;
+    *nh = f32 ? resident_halves<true>(nhalves) : resident_halves<false>(nhalves);
+    return *nh ? METIS_OK : METIS_E_TOO_LARGE;
+}
+
+int roundtrip_applies(int64_t rows, int64_t cols, int mode, size_t* bytes)
+{
+    int nh;
+    const int rc = roundtrip_form(rows, cols, mode, &nh);
+    if (bytes) *bytes = nh ? workspace_bytes(1, kBlock) : 0;
+    return rc;
+}
+
+int roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, void* workspace, size_t bytes, uint32_t spin_limit, hipStream_t st)
+{
+    int nh;
+    if (const int rc = roundtrip_form(rows, cols, mode, &nh)) return rc;
+    if (rows == 0 || cols == 0) return METIS_OK;
+    if (!x || !out || ((uintptr_t)x % 16) || ((uintptr_t)out % 16)) return METIS_E_ARG;
+    const uint32_t nhalves = (uint32_t)(rows * cols / 8);
+    const bool f32 = mode == METIS_MODE_P32_F32;
     const uint4* xv = static_cast<const uint4*>(x);
-    if (small_tensor(nhalves, f32)) {
+    if (nh == 0) {
         const unsigned g = (nhalves + kRoundtripSmallThreads - 1) / kRoundtripSmallThreads;
         if (f32) hipLaunchKernelGGL(roundtrip_small_kernel<true>, dim3(g), dim3(kRoundtripSmallThreads), 0, st, xv, out, nhalves);
         else hipLaunchKernelGGL(roundtrip_small_kernel<false>, dim3(g), dim3(kRoundtripSmallThreads), 0, st, xv, out, nhalves);
@@ -306,8 +333,8 @@ int roundtrip(const void* x, int64_t rows, int64_t cols, int mode, void* out, vo
     Workspace ws;
     if (const int rc = carve_workspace(workspace, bytes, 1, kBlock, &ws)) return rc;
     if (spin_limit == 0) spin_limit = kSpinLimit;
-    if (!(f32 ? launch_resident<true>(xv, out, nhalves, ws.sync, spin_limit, st) : launch_resident<false>(xv, out, nhalves, ws.sync, spin_limit, st)))
-        return METIS_E_TOO_LARGE;
+    if (f32) launch_resident<true>(nh, xv, out, nhalves, ws.sync, spin_limit, st);
+    else launch_resident<false>(nh, xv, out, nhalves, ws.sync, spin_limit, st);
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 

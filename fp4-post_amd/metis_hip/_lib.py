@@ -35,6 +35,7 @@ SIGNATURES = {
     "metis_nvfp4_quant_row": (_i32, [_vp, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "metis_nvfp4_quant_dequant_row": (_i32, [_vp, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "metis_nvfp4_quant_dequant_row_f32": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "metis_nvfp4_roundtrip_applies": (_i32, [_i64, _i64, _i32, _vp]),
     "metis_nvfp4_roundtrip": (_i32, [_vp, _i64, _i64, _i32, _vp, _vp, _sz, ctypes.c_uint32, _vp]),
     "metis_nvfp4_quant_row_static": (_i32, [_vp, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp]),
     "metis_nvfp4_quant_row_resident": (_i32, [_vp, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _sz, ctypes.c_uint32, _vp]),

@@ -206,8 +206,16 @@ def _workspace(rows: int, cols: int, device: torch.device, zeroed: bool = False,
     taken over the grid); the others write every word that they read."""
     need = tensors * _quant_workspace_bytes(rows, cols)
     if torch.cuda.is_current_stream_capturing():
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        return ws.fill_(0) if zeroed else ws                       # (a fill kernel: no memset is recorded into a graph)
+        return _captured_workspace(need, device, zeroed)
+    return _kept_workspace(need, device, tensors)
+
+
+def _captured_workspace(need: int, device: torch.device, zeroed: bool) -> torch.Tensor:
+    ws = torch.empty(need, dtype=torch.uint8, device=device)
+    return ws.fill_(0) if zeroed else ws                           # (a fill kernel: no memset is recorded into a graph)
+
+
+def _kept_workspace(need: int, device: torch.device, tensors: int = 1) -> torch.Tensor:
     key = (device.index, _stream(), tensors)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < need:
@@ -410,25 +418,47 @@ def quantize_dequantize_f32(x: torch.Tensor) -> tuple[PackedNVFP4, torch.Tensor]
     return PackedNVFP4(codes, scales, unit, rows, cols, MODE_P32), out
 
 
+@functools.lru_cache(maxsize=4096)
+def _roundtrip_scratch(rows: int, cols: int, kmode: int, device_index: int) -> int | None:
+    """Bytes of zeroed scratch that the round trip of this shape reads (0: a small tensor), None if it is too large; depends on the device's
+    capacity only."""
+    need = ctypes.c_size_t(0)
+    rc = load().metis_nvfp4_roundtrip_applies(rows, cols, kmode, ctypes.addressof(need))
+    if rc and rc != _lib.E_TOO_LARGE:
+        check(rc, "metis_nvfp4_roundtrip", (rows, cols))
+    return None if rc else need.value
+
+
+# Elements from which a captured round trip takes the grid-wide maximum.  In a graph its area is cleared in every replay, a launch of its
+# own (about 2 us): with it 768 x 4096 10.5 us in bf16 and 12.8 in binary32 where the two launches of the packed form take 9.8 and 11.7;
+# 1024 x 4096 10.6 and 14.2 against 11.1 and 14.4, 4096 x 4096 19.2 and 30.0 against 22.6 and 32.6.
+_ROUNDTRIP_CAPTURED = 1 << 22
+
+
 def roundtrip(x: torch.Tensor, spin_limit: int = 0) -> torch.Tensor | None:
     """dequantize(quantize(x)) of a bf16 tensor in bf16 arithmetic or a binary32 tensor in binary32 arithmetic, round to nearest: the
     same values in x's shape and type, from one launch that packs nothing.  None where half of the device's registers do not hold
-    the tensor's codes.  spin_limit: polls for the grid's maximum before a workgroup leaves its values to the last one (0: the
-    library's limit)."""
+    the tensor's codes, and in a capture where the packed form is faster.  spin_limit: polls for the grid's maximum before a
+    workgroup leaves its values to the last one (0: the library's limit)."""
     x2 = x if (x.dim() == 2 and x.is_contiguous()) else x.reshape(-1, x.shape[-1]).contiguous()
     rows, cols = x2.shape
-    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    ws = _workspace(1, BLOCK, x.device, zeroed=rows * cols > _ROUNDTRIP_FOLDED)
-    rc = load().metis_nvfp4_roundtrip(x2.data_ptr(), rows, cols, MODE_PB16 if x.dtype == torch.bfloat16 else _lib.MODE_P32_F32, out.data_ptr(),
-                                      ws.data_ptr(), ws.numel(), int(spin_limit), _stream())
-    if rc == _lib.E_TOO_LARGE:
+    kmode = MODE_PB16 if x.dtype == torch.bfloat16 else _lib.MODE_P32_F32
+    need = _roundtrip_scratch(rows, cols, kmode, x.device.index or 0)
+    if need is None:
         return None
+    ws = None
+    if need and torch.cuda.is_current_stream_capturing():
+        if rows * cols < _ROUNDTRIP_CAPTURED:
+            return None
+        ws = _captured_workspace(need, x.device, True)
+    elif need:
+        ws = _kept_workspace(need, x.device)
+    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    rc = load().metis_nvfp4_roundtrip(x2.data_ptr(), rows, cols, kmode, out.data_ptr(), None if ws is None else ws.data_ptr(), need, int(spin_limit),
+                                      _stream())
     if rc:
         check(rc, "metis_nvfp4_roundtrip", x.shape)
     return out
-
-
-_ROUNDTRIP_FOLDED = 128 * 1024            # elements up to which no grid-wide maximum is taken in either type
 
 
 def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tensor, mode: int = MODE_P32,

@@ -107,8 +107,11 @@ int metis_nvfp4_quant_dequant_row_f32(const void *x, int64_t rows, int64_t cols,
  * bounded polls (spin_limit, 0 for the default), the result does not depend on them.
  *   x, out     [rows, cols], contiguous: bf16 with METIS_MODE_PB16, float with METIS_MODE_P32_F32; 16-byte aligned
  *   workspace  metis_nvfp4_workspace_bytes(1, 16) bytes, 256-byte aligned, zero when first used; calls that share it are ordered.
- *              Not read for small tensors (up to 128 K elements)
+ *              Not read for small tensors, where it may be NULL
+ * metis_nvfp4_roundtrip_applies: the code that a call of these sizes returns on the current device (METIS_OK, METIS_E_TOO_LARGE, ...),
+ * and in *workspace_bytes how much scratch it reads: 0 for small tensors.
  */
+int metis_nvfp4_roundtrip_applies(int64_t rows, int64_t cols, int mode, size_t *workspace_bytes);
 int metis_nvfp4_roundtrip(const void *x, int64_t rows, int64_t cols, int mode, void *out, void *workspace,
                           size_t workspace_bytes, uint32_t spin_limit, void *stream);
 

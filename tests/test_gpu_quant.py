@@ -833,6 +833,41 @@ def test_round_trip_beyond_the_registers_and_from_a_captured_graph(ops):
         assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_what_a_captured_round_trip_records(ops, dtype, monkeypatch):
+    """A fill is recorded only in front of the kernel that reads the words, and that kernel only where the fill pays: below 4 Mi elements the
+    packed form is captured.  Eager calls of the same tensors take no other route than before; bits are equal after every replay."""
+    from metis_hip import quant_func
+    q = quant_func["nvfp4e2m1bnosr"]
+    fill, recorded = torch.Tensor.fill_, []
+
+    def fill_(t, value):
+        if torch.cuda.is_current_stream_capturing():
+            recorded.append(t)
+        return fill(t, value)
+    too_large = (8208, 4096) if dtype == torch.bfloat16 else (5152, 4096)
+    for shape, at_once, fills in (((128, 1024), True, 0), ((512, 1024), False, 0), ((1023, 4096), False, 0), ((1024, 4096), True, 1), (too_large, False, 0)):
+        x = torch.randn(shape, device="cuda").to(dtype)
+        assert (ops.roundtrip(x) is None) == (shape == too_large)
+        q.quantize_dequantize(x), ops.quantize_dequantize(x, 1), ops.quantize_dequantize_f32(x.float())
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        monkeypatch.setattr(torch.Tensor, "fill_", fill_)
+        with torch.cuda.graph(graph, stream=side):
+            values = ops.roundtrip(x)
+            assert len(recorded) == fills and (values is not None) == at_once, shape
+            out = q.quantize_dequantize(x)
+        monkeypatch.undo()
+        recorded.clear()
+        for k in range(3):
+            x.copy_(torch.randn(shape, device="cuda") * (1 + k))
+            want = q.quantize_dequantize(x)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out.view(torch.uint8), want.view(torch.uint8)) and (values is None or torch.equal(values, out)), (shape, k)
+
+
 def test_captured_quantizers_and_eager_calls_on_the_stream_of_the_capture(ops, monkeypatch):
     """The first calls on a stream are captured ones, then an eager round trip comes on it before any replay, then replays beside larger
     eager calls that make the kept scratch grow: every result has the bits of the calls on a stream of their own."""
