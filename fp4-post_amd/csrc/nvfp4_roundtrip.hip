@@ -287,9 +287,11 @@ static void launch_resident(int nh, const uint4* x, void* out, uint32_t nhalves,
 #undef METIS_RT
 }
 
-// The whole-tensor fold while it costs no more than taking the maximum over the grid.  Device time, fold | grid: bf16 128 x 1024 4.6 |
-// 6.8 us, 192 x 1024 5.6 | 6.9; binary32, twice the bytes to fold, 77 x 1536 6.0 | 6.9, 128 x 1024 6.2 | 6.9.
-static bool small_tensor(int64_t nhalves, bool f32) { return nhalves <= (f32 ? 16384 : 24576); }
+// The whole-tensor fold while it costs no more than taking the maximum over the grid: up to 256 Ki elements in bf16, 144 Ki in binary32,
+// twice the bytes to fold.  Device time, fold | grid: bf16 128 x 1024 4.6 | 6.6 us, 192 x 1024 5.6 | 6.6, 256 x 1024 6.55 | 6.65, 272 x 1024
+// 7.1 | 6.9, 320 x 1024 7.6 | 6.7; binary32 77 x 1536 5.8 | 6.6, 128 x 1024 6.2 | 6.7, 144 x 1024 6.6 | 6.9, 152 x 1024 7.0 | 6.8, 192 x 1024
+// 8.0 | 6.8.
+static bool small_tensor(int64_t nhalves, bool f32) { return nhalves <= (f32 ? 18432 : 32768); }
 
 // What a call of these sizes takes: half blocks per thread of the resident kernel in *nh (0: the fold), or why it is refused.
 static int roundtrip_form(int64_t rows, int64_t cols, int mode, int* nh)

@@ -739,10 +739,10 @@ def test_binary32_round_trip_from_one_call(ops, rows, cols):
     assert same_bits(q.quantize_dequantize(x).cpu(), out.cpu())
 
 
-# one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (192 x 1024 elements in bf16, 128 x
+# one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (256 x 1024 elements in bf16, 144 x
 # 1024 in binary32), leading dimensions, four, eight and sixteen half blocks per thread, the last workgroup partly filled
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("shape", [(1, 16), (3, 48), (5, 7, 80), (128, 1024), (129, 1024), (192, 1024), (193, 1024), (2049, 4080), (3001, 4080), (4099, 4096), (8191, 4096)])
+@pytest.mark.parametrize("shape", [(1, 16), (3, 48), (5, 7, 80), (128, 1024), (129, 1024), (144, 1024), (145, 1024), (192, 1024), (193, 1024), (256, 1024), (257, 1024), (2049, 4080), (3001, 4080), (4099, 4096), (8191, 4096)])
 def test_round_trip_values_without_a_packed_tensor(ops, dtype, shape):
     """ops.roundtrip: the values of quantize + dequantize bit for bit, with signed zeros, subnormal blocks, an infinity and a NaN."""
     from metis_hip import quant_func
