@@ -927,10 +927,14 @@ def test_gradients_of_the_rank_r_branch_side_by_side(L, N, K, R):
         assert torch.equal(gu, ops.lowrank_contract_tokens(dy, t)) and torch.equal(gv, ops.lowrank_contract_tokens(x, gxv, transpose=True))
         assert torch.equal(gs, ops.lowrank_scale_grad(gt, xv, out_dtype=dt))
     # one addend in 2^24 of the largest sum: binary32 accumulation of exact products, one rounding to bf16
+    def near(got, want):
+        return float((got.double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5
     want = dy.double().T @ t.double()
-    assert float((gu.double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5
-    strided = ops.lowrank_backward(dy, make(L, R + 1)[:, :R], x, gxv, gt, xv)       # not what the kernel reads: the separate calls
-    assert strided[0].shape == (N, R) and torch.equal(strided[1], gv)
+    assert near(gu, want) and near(gv, gxv.double().T @ x.double())
+    t2 = make(L, R + 1)[:, :R]                                     # not what the kernel reads: the separate calls
+    strided = ops.lowrank_backward(dy, t2, x, gxv, gt, xv)
+    assert strided[0].shape == (N, R) and near(strided[0], dy.double().T @ t2.double())
+    assert torch.equal(strided[1], gv) and torch.equal(strided[2], ops.lowrank_scale_grad(gt, xv))
 
 
 @pytest.mark.parametrize("L,R", [(1, 8), (255, 40), (257, 32), (2047, 32), (2049, 8), (4096, 32), (5000, 64)])

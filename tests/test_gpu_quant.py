@@ -943,13 +943,19 @@ def test_quantizers_of_a_binary32_gradient_leave_its_bf16_rounding(ops, rows, co
         ops.quantize_both_sr(x, 0, bf16_copy=copy.float(), **more)
 
 
-@pytest.mark.parametrize("rows,cols", [(16, 64), (256, 1024), (272, 1040), (512, 1536), (1488, 3648), (4112, 2064)])
-def test_both_packings_cover_a_partly_filled_span_of_tiles(rows, cols):
+# (the last two have more tiles of 256 x 64 than 256 compute units hold workgroups, 2664 and 2397 against at most 2048, so that a
+# workgroup goes on to a second tile with another column of centres: ragged rows with padding, and a last tile of 16 columns)
+@pytest.mark.parametrize("rows,cols,pad", [(16, 64, None), (256, 1024, None), (272, 1040, None), (512, 1536, None), (1488, 3648, None), (4112, 2064, None),
+                                           (2103, 18944, 2112), (4112, 8976, None)])
+def test_both_packings_cover_a_partly_filled_span_of_tiles(rows, cols, pad):
     """Tiles that do not fill their last span of eight runs, fewer and more than the device holds at once: the bytes of the two calls."""
     from metis_hip import ops
     x = synthetic_activation(900 + rows, rows, cols).cuda()
-    for xin, mode, center in ((x, ops.MODE_PB16, None), (x.float() * 1.001, ops.MODE_P32, None), (x, ops.MODE_PB16, x.float().mean(0).bfloat16())):
-        got = ops.quantize_both_sr(xin, mode, seed=3, offset_row=5, offset_col=1 << 33, center=center)
-        want = [ops.quantize(xin, mode, col=c, sr=True, seed=3, offset=o, center=center) for c, o in ((False, 5), (True, 1 << 33))]
+    more = {} if pad is None else {"pad_rows": pad}
+    wide = x.float() * 1.001
+    for xin, mode, center in ((x, ops.MODE_PB16, None), (wide, ops.MODE_P32, None), (x, ops.MODE_PB16, x.float().mean(0).bfloat16()),
+                              (wide, ops.MODE_P32, wide.mean(0))):
+        got = ops.quantize_both_sr(xin, mode, seed=3, offset_row=5, offset_col=1 << 33, center=center, **more)
+        want = [ops.quantize(xin, mode, col=c, sr=True, seed=3, offset=o, center=center, **(more if c else {})) for c, o in ((False, 5), (True, 1 << 33))]
         for p, q in zip(got, want):
             assert torch.equal(p.codes, q.codes) and torch.equal(p.scales, q.scales) and torch.equal(p.unit, q.unit)
