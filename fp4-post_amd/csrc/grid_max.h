@@ -18,8 +18,11 @@ namespace metis {
 // and the last workgroup that cleans up after one pay for fences.  Every wave exits after a bounded time whatever else
 // runs on the device, and the result is always complete and always the same bytes as the two-launch path.
 // The area starts zero-filled; a call leaves the tree clean and only tagged words behind.
+// What giving up costs: the polls (up to a few milliseconds), then one workgroup writes for all that left, at the speed of one.  The round
+// trip keeps its grid to half of the device, where this was not seen beside any other work; the single-launch quantizer is for callers
+// that have the device to themselves.
 // ---------------------------------------------------------------------------------------------
-constexpr uint32_t kSpinLimit = 4096;            // polls (roughly a microsecond each) before a workgroup leaves its scale bytes behind
+constexpr uint32_t kSpinLimit = 4096;            // polls (roughly a microsecond each) before a workgroup leaves its output behind
 constexpr uint32_t kGroups = 64;                 // groups, and the most members a group can have
 constexpr int kFusedMaxGrid = kGroups * kGroups;
 // locations inside the synchronisation area (uint32 units)
@@ -63,7 +66,7 @@ struct GridMaxState {
     uint32_t known;              // result holds the tensor maximum
     float result;
     uint32_t nleft;
-    uint32_t left[256];          // workgroups of one slab of 256 flags that left their scale bytes behind
+    uint32_t left[256];          // workgroups of one slab of 256 flags that left their output behind
 };
 
 // Every thread, at kernel start (before its workgroup arrives, so before the counter can move): the tag of this call.
@@ -87,7 +90,7 @@ __device__ __forceinline__ bool tree_arrive(uint32_t* node, uint32_t bits, uint3
     return true;
 }
 
-// Called by every thread of every workgroup, once: folds the workgroup maximum (a bf16 value) into the tree.
+// Called by every thread of every workgroup, once: folds the workgroup maximum (a bf16 or binary32 value, not negative) into the tree.
 __device__ __forceinline__ void grid_max_arrive(float thread_max, uint32_t* sync, GridMaxState& sh)
 {
     const float m = wave_max(thread_max);

@@ -1176,7 +1176,7 @@ int skinny_operand_rht(const void* codes, const void* scales, float* unit, const
 
 // lowrank_small + skinny_operand_deferred on the same activation (x [M, K] bf16 and its packed form) in two launches
 // instead of three: partial sums of the projection, then one launch that finishes it and builds the operands.
-// x = nullptr: the first of the two already ran beside the quantizer (quantize_row_deferred_partial): one launch.
+// x = nullptr: the first of the two already ran beside the quantizer (quantize_row_deferred_partial, token_mean_quant): one launch.
 int decode_prepare_deferred(const void* x, int64_t ldx, const void* v, int64_t R, const void* s, void* xv, void* t, void* workspace,
                             size_t workspace_bytes, const void* codes, const void* deferred, int64_t M, int64_t K, int qmode, int mode,
                             const void* center, float* unit_out, void* out, hipStream_t st, int rotate, uint32_t sign_mask)

@@ -11,7 +11,7 @@ namespace metis {
 
 // Caller-supplied scratch, carved as:
 //   [0, 16 KiB)        one partial maximum (uint32 bit pattern) per workgroup of phase 1
-//   [16 KiB, +65 KiB)  reduction area of the single-launch quantizer (zero when first used)
+//   [16 KiB, +65 KiB)  area of the grid-wide maximum, grid_max.h: single-launch quantizer, resident round trip (zero when first used)
 //   [81 KiB, ..)       one block maximum per block of 16: bf16 for bf16 input, binary32 for binary32 input
 struct Workspace {
     uint32_t* gmax;
@@ -19,7 +19,7 @@ struct Workspace {
     uint16_t* amax;
 };
 constexpr size_t kWsGmaxBytes = 4096 * 4;
-constexpr size_t kWsSyncBytes = 260 * 256;     // reduction area of the single-launch quantizer: header, 65 tree nodes and 64 result words on lines of their own, 4096 flags (33 KiB used)
+constexpr size_t kWsSyncBytes = 260 * 256;     // header, 65 tree nodes and 64 result words on lines of their own, 4096 flags, 64 more result words for binary32 maxima (41 472 bytes used)
 
 inline size_t workspace_bytes(int64_t rows, int64_t cols)
 {

@@ -1297,7 +1297,7 @@ int quantize_dequantize_row(const void* x, int64_t rows, int64_t cols, int mode,
 }
 
 // Workgroups of quant_codes_both_kernel that the current device holds at once (its LDS slabs bound them): the grid is
-// no larger, so that every workgroup starts at once and walks the same number of tiles, give or take one.
+// no larger, so that every workgroup starts at once.  How many tiles each then has is a matter of the spans (quantize_both_sr).
 template <int MODE, bool WIDE, bool CEN>
 static int both_capacity()
 {

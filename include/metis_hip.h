@@ -51,7 +51,7 @@ extern "C" {
 #define METIS_E_WORKSPACE (-3) /* workspace missing, misaligned or too small                   */
 #define METIS_E_LAUNCH (-4)    /* the HIP runtime rejected a launch                             */
 #define METIS_E_DEVICE (-5)    /* not a gfx950 device / required feature missing               */
-#define METIS_E_TOO_LARGE (-6) /* metis_nvfp4_quant_row_static: more elements than its scratch holds */
+#define METIS_E_TOO_LARGE (-6) /* more elements than the call takes (its scratch, the device's registers) */
 
 #define METIS_MODE_P32 0
 #define METIS_MODE_PB16 1
@@ -789,8 +789,9 @@ int metis_linear_fwd_grouped_bf16(const void *a_codes, const void *a_scales, con
  *                                step rides in the first blocks of the operand launch.  Same bits as the two calls
  *                                (`vlinear(x)`, `torch.mul(self.s, y)` and the quantized input of BitLinear.forward,
  *                                src/Metis/Metis/bitlinear.py:752-760).  x = NULL: the workspace already holds the
- *                                projection's partial sums, left there by metis_decode_quant_project_deferred on the
- *                                same rows, cols and R (R <= 128 then): one launch.  rotate != 0: the operand half is
+ *                                projection's partial sums, left there by metis_decode_quant_project_deferred (R <= 128) or
+ *                                metis_token_mean_quant_deferred (R <= 256) on the same rows, cols and R: one launch.
+ *                                rotate != 0: the operand half is
  *                                metis_nvfp4_decode_operand_rht with sign_mask (no centre then; codes 8-byte aligned)
  *   metis_nvfp4_decode_operand_rht  the operand for a call against a weight packed in the ROTATED domain (NV recipe:
  *                                metis_nvfp4_quant_row_rht with sign_mask; the forward multiplies with
