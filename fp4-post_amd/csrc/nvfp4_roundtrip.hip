@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kRoundtripSmallThreads) void roundtrip_small_kernel
 // on the device wait for each other until they give up; then one workgroup writes everything that was left, in milliseconds.  Per call
 // beside other work, packed form | half of the device | all of it: bf16 8192 x 4096 beside copies of 2 GiB 80 us | 56 | 881, binary32 4096 x
 // 4096 beside exp of 512 Mi elements 65 | 50 | 4850; one call on each of three streams, together 97 | 72 | 7165 and 85 | 70 | 3314.
-// Three quarters of the device (bf16 12288 x 4096): three streams 956, packed form 140.  Alone, with all of the device | half:
+// Three quarters of the device (bf16 12288 x 4096): three streams 956, packed form 140.  Alone, back to back, all of the device | half:
 // bf16 4096 x 4096 17.5 | 18.4, 5120 x 4096 20.6 | 22.2, 8192 x 4096 31.0 | 30.6.  Tensors beyond take the packed form: bf16
 // 12288 x 4096 51.4 where all of the device gave 41.6, binary32 8192 x 4096 58.3 where it gave 45.9.
 // A workgroup that cannot wait any longer leaves its values to the last one, which reads x again.
