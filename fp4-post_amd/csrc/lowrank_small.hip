@@ -35,18 +35,26 @@ size_t lowrank_small_workspace_bytes(int64_t M, int64_t R, int64_t K)
     return (size_t)lowrank_small_chunks(K, &kc) * (size_t)M * (size_t)R * sizeof(float);
 }
 
-// Argument checks and the first launch (partial sums per K chunk into the workspace); *chunks_out chunks wait for the
-// finishing step.  METIS_OK with *chunks_out == 0: nothing to do (M == 0).
-int lowrank_small_partial(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
-                          void* workspace, size_t workspace_bytes, hipStream_t st, int* chunks_out)
+int lowrank_small_check(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
+                        void* workspace, size_t workspace_bytes)
 {
-    *chunks_out = 0;
     if (M < 0 || R <= 0 || K <= 0 || ldx < K) return METIS_E_ARG;
     if (M >= 256 || R % 32 || R > 256 || K % 64 || ldx % 8) return METIS_E_SHAPE;
     if (M == 0) return METIS_OK;
     if (!x || !v || !xv || (t && !s)) return METIS_E_ARG;
     if (((uintptr_t)x % 16) || ((uintptr_t)v % 16) || ((uintptr_t)xv % 8) || ((uintptr_t)t % 8) || ((uintptr_t)s % 2)) return METIS_E_ARG;
     if (!workspace || ((uintptr_t)workspace % 16) || workspace_bytes < lowrank_small_workspace_bytes(M, R, K)) return METIS_E_WORKSPACE;
+    return METIS_OK;
+}
+
+// Argument checks and the first launch (partial sums per K chunk into the workspace); *chunks_out chunks wait for the
+// finishing step.  METIS_OK with *chunks_out == 0: nothing to do (M == 0).
+int lowrank_small_partial(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
+                          void* workspace, size_t workspace_bytes, hipStream_t st, int* chunks_out)
+{
+    *chunks_out = 0;
+    if (const int rc = lowrank_small_check(x, ldx, v, M, R, K, s, xv, t, workspace, workspace_bytes)) return rc;
+    if (M == 0) return METIS_OK;
     int kc;
     const int chunks = lowrank_small_chunks(K, &kc);
     hipLaunchKernelGGL(lowrank_small_partial_kernel, dim3((unsigned)chunks, (unsigned)((M + 63) / 64)), dim3((unsigned)(2 * R)), 0, st,

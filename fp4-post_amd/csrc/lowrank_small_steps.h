@@ -8,7 +8,11 @@
 namespace metis {
 
 typedef __bf16 lr_bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float lr_float16_t __attribute__((ext_vector_type(16)));
+typedef float lr_float4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ lr_float4_t lr_mfma(uint4 a, uint4 b, lr_float4_t c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lr_bf16x8_t, a), __builtin_bit_cast(lr_bf16x8_t, b), c, 0, 0, 0);
+}
 
 constexpr int kLrMaxChunks = 128;
 constexpr int kLrGroup = kLrMaxChunks / 4;     // chunks per thread of the finishing step
@@ -22,6 +26,9 @@ inline int lowrank_small_chunks(int64_t K, int* kc_out)
     return (int)((K + kc - 1) / kc);
 }
 
+// Both steps multiply on v_mfma_f32_16x16x32_bf16: lane l holds row l % 16 of either operand, elements 8 (l / 16) .. of 32; four sums of a lane are
+// consecutive columns r of one row of x.  A chunk's sum is one chain over its elements, 32 at a time, wherever it is formed.
+
 // One workgroup of the first step: K chunk `chunk` (kc elements), rows 64 mtile .. ; wave w owns columns 32 w .. of R
 // (waves past R / 32 have nothing to do), so the launch needs at least 2 R threads per workgroup, or several workgroups for a chunk,
 // the first wave of each (wave0) further on in R.
@@ -29,50 +36,117 @@ __device__ __forceinline__ void lowrank_small_partial_block(int chunk, int mtile
                                                             const uint16_t* __restrict__ v, int M, int R, int K, int kc,
                                                             float* __restrict__ ws, int wave0 = 0)
 {
-    const int lane = threadIdx.x & 63, wave = wave0 + (int)(threadIdx.x >> 6), hi = lane >> 5;
+    const int lane = threadIdx.x & 63, wave = wave0 + (int)(threadIdx.x >> 6), l16 = lane & 15, kg = lane >> 4;
     if (wave * 32 >= R) return;
     const int m0 = mtile * 64;
     const int k0 = chunk * kc, k1 = min(k0 + kc, K);
-    const uint16_t* vp = v + (int64_t)min(wave * 32 + (lane & 31), R - 1) * K + hi * 32;
-    const uint16_t* xp[2];
+    const uint16_t *vp[2], *xp[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) xp[i] = x + (int64_t)min(m0 + i * 32 + (lane & 31), M - 1) * ldx + hi * 32;
-    lr_float16_t acc[2];
+    for (int a = 0; a < 2; ++a) vp[a] = v + (int64_t)min(wave * 32 + a * 16 + l16, R - 1) * K + kg * 8;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int b = 0; b < 4; ++b) xp[b] = x + (int64_t)min(m0 + b * 16 + l16, M - 1) * ldx + kg * 8;
+    lr_float4_t acc[2][4];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = (lr_float4_t)(0.0f);
     for (int k = k0; k < k1; k += 64) {                        // kc % 64 == 0 and K % 64 == 0
-        uint4 rv[4], rx[2][4];
+        uint4 rv[2][2], rx[4][2];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) rv[q] = reinterpret_cast<const uint4*>(vp + k)[q];
+        for (int q = 0; q < 2; ++q) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int a = 0; a < 2; ++a) rv[a][q] = *reinterpret_cast<const uint4*>(vp[a] + k + 32 * q);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) rx[i][q] = reinterpret_cast<const uint4*>(xp[i] + k)[q];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const lr_bf16x8_t fv = __builtin_bit_cast(lr_bf16x8_t, rv[q]);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv, __builtin_bit_cast(lr_bf16x8_t, rx[i][q]), acc[i], 0, 0, 0);
+            for (int b = 0; b < 4; ++b) rx[b][q] = *reinterpret_cast<const uint4*>(xp[b] + k + 32 * q);
         }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) acc[a][b] = lr_mfma(rv[a][q], rx[b][q], acc[a][b]);
     }
-    // acc[i][e] of lane l: row m = m0 + 32 i + l % 32, column r = 32 wave + 8 (e / 4) + 4 (l / 32) + e % 4
     float* wp = ws + (size_t)chunk * M * R;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int m = m0 + i * 32 + (lane & 31);
+    for (int b = 0; b < 4; ++b) {
+        const int m = m0 + b * 16 + l16;
         if (m >= M) continue;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int r = wave * 32 + 8 * g + 4 * hi;
-            if (r < R)                                          // R % 4 == 0
-                *reinterpret_cast<float4*>(wp + (size_t)m * R + r) =
-                    make_float4(acc[i][4 * g], acc[i][4 * g + 1], acc[i][4 * g + 2], acc[i][4 * g + 3]);
+        for (int a = 0; a < 2; ++a) {
+            const int r = wave * 32 + a * 16 + 4 * kg;
+            if (r < R) *reinterpret_cast<lr_float4_t*>(wp + (size_t)m * R + r) = acc[a][b];     // R % 4 == 0
         }
     }
 }
+
+// rounds four consecutive sums of the projection (element id of [M, R]) and applies s
+__device__ __forceinline__ void lowrank_small_store(const float (&a)[4], int id, int r, const uint16_t* __restrict__ s, uint16_t* __restrict__ xv,
+                                                    uint16_t* __restrict__ t)
+{
+    uint32_t h[4], u[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = bf16_bits(a[e]);
+    *reinterpret_cast<uint2*>(xv + id) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    if (t) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(s[r + e]));
+        *reinterpret_cast<uint2*>(t + id) = make_uint2(u[0] | (u[1] << 16), u[2] | (u[3] << 16));
+    }
+}
+
+// Both steps of 16 rows x 16 columns in one block of 1024 threads, for a launch with other work that waits for nothing of the projection; K <= 4096.
+// Waves 4 g .. 4 g + 3 share the chunks of group g of the finishing step, a quarter each, requested together; the first of them adds the chunk sums of
+// all four in chunk order, so the bits are those of the two steps.  Every thread of the block has to call it (two barriers inside).
+// Blocks: lowrank_small_project_blocks(M, R).
+constexpr int kLrProjectThreads = 1024, kLrProjectK = 4096;
+__device__ __forceinline__ void lowrank_small_project_block(int block, const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v, int M,
+                                                            int R, int K, const uint16_t* __restrict__ s, uint16_t* __restrict__ xv,
+                                                            uint16_t* __restrict__ t)
+{
+    constexpr int MINE = kLrProjectK / 64 / 16;                // chunks of a wave
+    __shared__ lr_float4_t sums[4][3][MINE][64], group[3][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, kg = lane >> 4;
+    const int g = wave >> 2, w = wave & 3;
+    const int r0 = block % (R / 16) * 16, m = block / (R / 16) * 16 + l16;
+    const uint16_t* vp = v + (int64_t)(r0 + l16) * K + kg * 8;
+    const uint16_t* xp = x + (int64_t)min(m, M - 1) * ldx + kg * 8;
+    const int chunks = K / 64, per = (chunks + 3) / 4, own = (per + 3) / 4;
+    const int c0 = g * per + w * own, c1 = min(min(c0 + own, (g + 1) * per), chunks);
+    uint4 rv[MINE][2], rx[MINE][2];
+#pragma unroll
+    for (int i = 0; i < MINE; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const bool live = c0 + i < c1;
+            rv[i][q] = live ? *reinterpret_cast<const uint4*>(vp + (c0 + i) * 64 + 32 * q) : make_uint4(0u, 0u, 0u, 0u);
+            rx[i][q] = live ? *reinterpret_cast<const uint4*>(xp + (c0 + i) * 64 + 32 * q) : make_uint4(0u, 0u, 0u, 0u);
+        }
+    lr_float4_t total = (lr_float4_t)(0.0f);                   // (a chunk past the end adds zeros)
+#pragma unroll
+    for (int i = 0; i < MINE; ++i) {
+        lr_float4_t acc = (lr_float4_t)(0.0f);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc = lr_mfma(rv[i][q], rx[i][q], acc);
+        if (w > 0) sums[g][w - 1][i][lane] = acc;
+        else total += acc;
+    }
+    __syncthreads();
+    if (w == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int i = 0; i < MINE; ++i) total += sums[g][k][i][lane];
+        if (g > 0) group[g - 1][lane] = total;
+    }
+    __syncthreads();
+    if (wave > 0 || m >= M) return;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) total += group[i][lane];
+    const float a[4] = {total[0], total[1], total[2], total[3]};
+    const int r = r0 + 4 * kg;
+    lowrank_small_store(a, m * R + r, r, s, xv, t);
+}
+inline int lowrank_small_project_blocks(int64_t M, int64_t R) { return (int)((M + 15) / 16 * (R / 16)); }
 
 // One block of 256 threads: four threads per output quad (each a quarter of the chunks, folded in order), 64 quads.
 // Every thread of the block has to call it (one barrier inside).
@@ -98,15 +172,8 @@ __device__ __forceinline__ void lowrank_small_finish_block(int block, const floa
     if (g > 0 || !live) return;
 #pragma unroll
     for (int k = 0; k < 3; ++k) { const float4 b = fold[k][q]; a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
-    const uint32_t h[4] = {bf16_bits(a.x), bf16_bits(a.y), bf16_bits(a.z), bf16_bits(a.w)};
-    *reinterpret_cast<uint2*>(xv + id) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-    if (t) {
-        const int r = id % R;
-        uint32_t u[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) u[e] = bf16_bits(__uint_as_float(h[e] << 16) * bf16_lo(s[r + e]));
-        *reinterpret_cast<uint2*>(t + id) = make_uint2(u[0] | (u[1] << 16), u[2] | (u[3] << 16));
-    }
+    const float sums[4] = {a.x, a.y, a.z, a.w};
+    lowrank_small_store(sums, id, id % R, s, xv, t);
 }
 
 // One workgroup (256 threads) of the gradient of the rank-r scale vector: columns 8 block .. + 7 (scale_grad_kernel, lowrank_small.hip).

@@ -995,7 +995,7 @@ __device__ __forceinline__ uint4 rotated_operand_piece(const uint2 c, const uint
 }
 
 // RHT (sign_mask): the call multiplies with a weight packed in the rotated domain; see skinny_operand_rht_kernel.
-template <int PB16, int DEF, int QMODE, int RHT = 0>
+template <int PB16, int DEF, int QMODE, int RHT = 0, int THREADS = 256>
 __device__ __forceinline__ void skinny_operand_block(int block, int nblocks, const uint32_t* __restrict__ codes,
                                                      const uint8_t* __restrict__ scales, const float* __restrict__ unit_p,
                                                      const uint16_t* __restrict__ center, int M, int K, int tiles,
@@ -1007,13 +1007,13 @@ __device__ __forceinline__ void skinny_operand_block(int block, int nblocks, con
     const int64_t total = (int64_t)tiles * iters * 1024;
     float unit = 0.0f;
     if constexpr (DEF != 0) {
-        unit = tensor_unit_of<QMODE>(fold_partial_maxima(partials));
+        unit = tensor_unit_of<QMODE>(fold_partial_maxima<THREADS>(partials));
         if (block == 0 && threadIdx.x == 0) *unit_out = unit;
     } else if constexpr (PB16 != 0) {
         unit = *unit_p;
     }
     const uint16_t* __restrict__ maxima = reinterpret_cast<const uint16_t*>(scales);
-    for (int64_t idx = (int64_t)block * 256 + threadIdx.x; idx < total; idx += (int64_t)nblocks * 256) {
+    for (int64_t idx = (int64_t)block * THREADS + threadIdx.x; idx < total; idx += (int64_t)nblocks * THREADS) {
         const int lane = (int)(idx & 63), m = (int)((idx >> 6) & 15);
         const int64_t ti = idx >> 10;
         const int it = (int)(ti % iters), tile = (int)(ti / iters);
@@ -1101,6 +1101,24 @@ __global__ __launch_bounds__(256) void decode_prepare_kernel(int finish_blocks, 
                                               M, K, tiles, out, partials, unit_out, sign_mask);
 }
 
+// The same for an activation whose projection has not begun: the first blocks form it whole.
+template <int PB16, int QMODE, int RHT = 0>
+__global__ __launch_bounds__(kLrProjectThreads) void decode_project_kernel(int project_blocks, const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v,
+                                                             int R, const uint16_t* __restrict__ s, uint16_t* __restrict__ xv,
+                                                             uint16_t* __restrict__ t, const uint32_t* __restrict__ codes,
+                                                             const uint8_t* __restrict__ maxima, const uint16_t* __restrict__ center,
+                                                             int M, int K, int tiles, uint4* __restrict__ out,
+                                                             const uint32_t* __restrict__ partials, float* __restrict__ unit_out,
+                                                             uint32_t sign_mask)
+{
+    if ((int)blockIdx.x < project_blocks) {
+        lowrank_small_project_block((int)blockIdx.x, x, ldx, v, M, R, K, s, xv, t);
+        return;
+    }
+    skinny_operand_block<PB16, 1, QMODE, RHT, kLrProjectThreads>((int)blockIdx.x - project_blocks, (int)gridDim.x - project_blocks, codes, maxima,
+                                                                 nullptr, center, M, K, tiles, out, partials, unit_out, sign_mask);
+}
+
 size_t skinny_operand_bytes(int64_t M, int64_t K)
 {
     if (M <= 0 || K <= 0) return 0;
@@ -1185,8 +1203,13 @@ int skinny_operand_rht(const void* codes, const void* scales, float* unit, const
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 
-// lowrank_small + skinny_operand_deferred on the same activation (x [M, K] bf16 and its packed form) in two launches
-// instead of three: partial sums of the projection, then one launch that finishes it and builds the operands.
+// Whether the launch that builds the operands forms the whole projection: a block of 16 x 16 results reads 64 K bytes of x and V (1.7 us per 1024 of
+// K), while partial sums of K chunks cost a launch and M R binary32 values per chunk.  Microseconds, two launches | one: 64 x 1536, R = 192 8.6 | 5.5,
+// R = 64 6.6 | 5.4; 64 x 2560, R = 64 6.8 | 7.2, R = 128 7.9 | 7.1; 64 x 3584, R = 128 8.1 | 8.8, R = 192 9.5 | 8.9; 192 x 2048, R = 192 10.2 | 6.5.
+static bool project_whole(int64_t R, int64_t K) { return K <= kLrProjectK && K <= 1536 + 12 * R; }
+
+// lowrank_small + skinny_operand_deferred on the same activation (x [M, K] bf16 and its packed form) in one launch, or in two: partial
+// sums of the projection, then one launch that finishes it and builds the operands (project_whole).
 // x = nullptr: the first of the two already ran beside the quantizer (quantize_row_deferred_partial, token_mean_quant): one launch.
 int decode_prepare_deferred(const void* x, int64_t ldx, const void* v, int64_t R, const void* s, void* xv, void* t, void* workspace,
                             size_t workspace_bytes, const void* codes, const void* deferred, int64_t M, int64_t K, int qmode, int mode,
@@ -1201,6 +1224,21 @@ int decode_prepare_deferred(const void* x, int64_t ldx, const void* v, int64_t R
     Workspace ws;
     if (const int rc = carve_deferred(const_cast<void*>(deferred), deferred_bytes(M, K), M, K, &ws)) return rc;
     int chunks = 0;
+    if (x && project_whole(R, K)) {
+        if (const int rc = lowrank_small_check(x, ldx, v, M, R, K, s, xv, t, workspace, workspace_bytes)) return rc;
+        const int pb = lowrank_small_project_blocks(M, R), tiles = (int)((M + 63) / 64) * 2;
+        const int g = pb + tiles * (int)(K / 256);             // a thread per piece of the operands
+#define METIS_DJ(P, Q, H) hipLaunchKernelGGL((decode_project_kernel<P, Q, H>), dim3(g), dim3(kLrProjectThreads), 0, st, pb, (const uint16_t*)x, ldx, (const uint16_t*)v, \
+                                             (int)R, (const uint16_t*)s, (uint16_t*)xv, (uint16_t*)t, (const uint32_t*)codes, \
+                                             (const uint8_t*)ws.amax, (const uint16_t*)center, (int)M, (int)K, tiles, (uint4*)out, \
+                                             (const uint32_t*)ws.gmax, unit_out, sign_mask)
+#define METIS_DJH(P, Q) do { if (rotate) METIS_DJ(P, Q, 1); else METIS_DJ(P, Q, 0); } while (0)
+        if (mode == METIS_MODE_PB16) { if (qmode) METIS_DJH(1, 1); else METIS_DJH(1, 0); }
+        else { if (qmode) METIS_DJH(0, 1); else METIS_DJH(0, 0); }
+#undef METIS_DJH
+#undef METIS_DJ
+        return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
+    }
     if (x) {
         if (const int rc = lowrank_small_partial(x, ldx, v, M, R, K, s, xv, t, workspace, workspace_bytes, st, &chunks)) return rc;
     } else {

@@ -192,6 +192,8 @@ int lowrank_small(const void* x, int64_t ldx, const void* v, int64_t M, int64_t 
 // lowrank_small_finish_blocks(M, R) blocks (lowrank_small_steps.h)
 int lowrank_small_partial(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
                           void* workspace, size_t workspace_bytes, hipStream_t st, int* chunks_out);
+int lowrank_small_check(const void* x, int64_t ldx, const void* v, int64_t M, int64_t R, int64_t K, const void* s, void* xv, void* t,
+                        void* workspace, size_t workspace_bytes);       // its argument checks alone
 inline int lowrank_small_finish_blocks(int64_t M, int64_t R) { return (int)((M * R / 4 + 63) / 64); }
 
 // gradient of the rank-r scale vector: column sums of the bf16 products of two [L, R] tensors; lowrank_small.hip

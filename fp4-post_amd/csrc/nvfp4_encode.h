@@ -438,12 +438,14 @@ __device__ __forceinline__ void publish_group_max(float m, uint32_t* ws_gmax, ui
 // bytes itself (quant.py:21-23) -- the same expressions as quant_scales_kernel, so the same bits.
 constexpr uint32_t kDeferredPartials = 2048;
 // tensor maximum from the partial maxima: every thread of a 256-thread workgroup calls this
+template <int THREADS = 256>
 __device__ __forceinline__ float fold_partial_maxima(const uint32_t* __restrict__ partials)
 {
-    static_assert(kDeferredPartials == 256 * 8, "256 threads fold eight entries each");
-    __shared__ float fmax_s[4];
-    const uint4 a = reinterpret_cast<const uint4*>(partials)[threadIdx.x];
-    const uint4 b = reinterpret_cast<const uint4*>(partials)[threadIdx.x + 256];
+    static_assert(kDeferredPartials == 256 * 8 && THREADS >= 256, "256 threads fold eight entries each");
+    __shared__ float fmax_s[THREADS / 64];
+    const int i = THREADS == 256 ? (int)threadIdx.x : (int)threadIdx.x & 255;      // (more threads: every 256 of them fold all entries)
+    const uint4 a = reinterpret_cast<const uint4*>(partials)[i];
+    const uint4 b = reinterpret_cast<const uint4*>(partials)[i + 256];
     float m = fmaxf(fmaxf(fmaxf(__uint_as_float(a.x), __uint_as_float(a.y)), fmaxf(__uint_as_float(a.z), __uint_as_float(a.w))),
                     fmaxf(fmaxf(__uint_as_float(b.x), __uint_as_float(b.y)), fmaxf(__uint_as_float(b.z), __uint_as_float(b.w))));
     m = wave_max(m);

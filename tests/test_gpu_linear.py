@@ -1163,6 +1163,26 @@ def test_projection_finish_and_operand_build_in_one_launch(M, K, R, mode, centre
         ops.project_and_operand(x, v, s, p1, mode, centre)
 
 
+@pytest.mark.parametrize("M,K,R", [(1, 256, 32), (16, 768, 64), (17, 1792, 32), (65, 2304, 64), (255, 2048, 160), (31, 3840, 192), (64, 4096, 256), (48, 4096, 224)])
+def test_projection_formed_whole_beside_the_operand_build_has_the_bits_of_its_two_steps(M, K, R):
+    """Short contractions: one launch forms the projection and builds the operands.  Chunks that do not divide evenly among groups and waves, ragged
+    row tiles, either side of the line where the two steps take over; the projection is also one bf16 rounding of the double precision sum."""
+    from metis_hip import ops
+    g = torch.Generator().manual_seed(9 * M + K + R)
+    x = synthetic_activation(500 + M, M, K).cuda()
+    v = (torch.randn(R, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    s = torch.randn(R, generator=g).bfloat16().cuda()
+    xv0, t0 = ops.lowrank_project(x, v, s)
+    px = ops.quantize(x, 1, deferred=True)
+    xv, t, op = ops.project_and_operand(x, v, s, px)
+    assert torch.equal(xv, xv0) and torch.equal(t, t0)
+    assert torch.equal(op, ops.decode_operand(ops.quantize(x, 1), 1))
+    want = x.double() @ v.double().T
+    # a rounding to eight significant bits (half a unit in the last place: 2^-8 of the value at most), and binary32 sums of K products: (K / 16 + 16) 2^-24 of the sum of magnitudes at most
+    bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ v.double().abs().T) * (K / 16 + 16) * 2.0 ** -24
+    assert bool(((xv.double() - want).abs() <= bound).all())
+
+
 def test_decode_prepare_rejects_what_its_two_halves_reject():
     from metis_hip import _lib, ops
     L = _lib.load()
