@@ -155,6 +155,22 @@ def load():
     return _lib
 
 
+HOST_PATH = os.path.join(_HERE, "_metis_host.so")
+U8, B16, F32 = 0, 1, 2          # types of call()'s new tensors
+
+
+def call(name: str, device_index: int, specs: tuple, args: tuple):
+    """One entry point of the library with new tensors as outputs and scratch (csrc/host_calls.cpp): the tensors, or the return code if it
+    is not OK.  Replaced by the compiled function on first use; raises MetisHipError if it has not been built."""
+    global call
+    load()
+    if not os.path.exists(HOST_PATH):
+        raise MetisHipError(f"{HOST_PATH} not found: build it with `make -C fp4-post_amd/csrc` (or __graft_entry__.build()); there is no fallback path")
+    from . import _metis_host
+    call = _metis_host.call
+    return call(name, device_index, specs, args)
+
+
 def check(rc: int, what: str, shape=None):
     """Map a return code to the exception the reference raises for the same condition."""
     if rc == OK:

@@ -18,7 +18,7 @@ from torch import nn
 from . import ops
 from ._lib import MODE_P32, MODE_PB16
 from .ops import CenteredNVFP4
-from .bitlinear import BitLinear, LinearLowbitFunction, _version_of
+from .bitlinear import BitLinear, LinearLowbitFunction, _param, _version_of
 from .quant import is_hip_nvfp4
 
 
@@ -95,7 +95,7 @@ class FusedRMSNormQuant(nn.Module):
             return None
         if F._mean_packed_at_once() and ops._token_mean_takes(rows, cols, 1, x.device.index or 0) and rows <= ops.TOKEN_MEAN_MAX_ROWS:
             # few tokens: the launch that packs the normed tensor forms the mean itself
-            normed = ops.rmsnorm(x, self.weight, self.variance_epsilon)
+            normed = ops.rmsnorm(x, _param(self, "weight"), self.variance_epsilon)
             projection = None if (recording or not BitLinear.grouped_inference) else BitLinear._group_projection(group, rows, cols, x.device)
             packed = F._token_mean_pack(normed.reshape(x.shape), True, cache, key, projection)
             if packed is not None:
@@ -109,7 +109,8 @@ class FusedRMSNormQuant(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         F = LinearLowbitFunction
         cols = x.shape[-1]
-        fused = (x.is_cuda and x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16 and cols % 32 == 0
+        weight = _param(self, "weight")
+        fused = (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and cols % 32 == 0
                  and cols <= 16384 and is_hip_nvfp4(F.q_forward_input) and (not F.enable_nv_recipe or F._nv_on_kernels())
                  and x.numel() > 0)     # (NV recipe: the forward quantizes its activation unrotated, like any other)
         mean_mode = fused and F.enable_activation_svd
@@ -129,11 +130,11 @@ class FusedRMSNormQuant(nn.Module):
                 packed.residual.shared = True
             else:
                 cached = all(m._weights_cached() for m in self.group.get("members", ()))
-                normed, packed = ops.rmsnorm_quantize(x, self.weight, self.variance_epsilon, mode,
+                normed, packed = ops.rmsnorm_quantize(x, weight, self.variance_epsilon, mode,
                                                       deferred=F._scales_formed_by_consumer(x.numel() // cols, cached))
         normed = normed.reshape(x.shape)
-        out = _NormedWithGrad.apply(x, self.weight, normed, self.variance_epsilon) if torch.is_grad_enabled() and (
-            x.requires_grad or self.weight.requires_grad) else normed
+        out = _NormedWithGrad.apply(x, weight, normed, self.variance_epsilon) if torch.is_grad_enabled() and (
+            x.requires_grad or weight.requires_grad) else normed
         group = self.group
 
         def clear(ref):

@@ -12,7 +12,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from ._lib import DTYPE_BF16, DTYPE_F32, MODE_P32, MODE_PB16, check, load
+from ._lib import B16, DTYPE_BF16, DTYPE_F32, F32, MODE_P32, MODE_PB16, U8, check, load
 
 BLOCK = 16
 _workspaces: dict = {}
@@ -179,6 +179,11 @@ def _decode_operand_bytes(rows: int, cols: int) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
+def _decode_weight_bytes(rows: int, cols: int) -> int:
+    return int(load().metis_nvfp4_decode_weight_bytes(rows, cols))
+
+
+@functools.lru_cache(maxsize=4096)
 def _expand_tiled_bytes(rows: int, cols: int) -> int:
     return int(load().metis_nvfp4_expand_tiled_bytes(rows, cols))
 
@@ -186,6 +191,21 @@ def _expand_tiled_bytes(rows: int, cols: int) -> int:
 @functools.lru_cache(maxsize=4096)
 def _column_mean_bytes(cols: int) -> int:
     return int(load().metis_column_mean_workspace_bytes(cols))
+
+
+@functools.lru_cache(maxsize=4096)
+def _rmsnorm_colmean_bytes(rows: int, cols: int) -> int:
+    return max(int(load().metis_rmsnorm_colmean_workspace_bytes(rows, cols)), 16)
+
+
+@functools.lru_cache(maxsize=4096)
+def _rmsnorm_backward_bytes(rows: int, cols: int) -> int:
+    return int(load().metis_rmsnorm_backward_workspace_bytes(rows, cols))
+
+
+@functools.lru_cache(maxsize=4096)
+def _lowrank_backward_bytes(L_: int, N: int, K: int, R: int, device_index: int) -> int:
+    return int(load().metis_lowrank_backward_workspace_bytes(L_, N, K, R))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -287,9 +307,7 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
         raise ValueError(f"NVFP4 block shape (1, 16) does not divide tensor shape {tuple(x.shape)}")
     prow, pcol = (cols, rows) if col else (rows, cols)
     dev = x2.device
-    codes = torch.empty(prow, pcol // 2, dtype=torch.uint8, device=dev)
-    unit = torch.empty(1, dtype=torch.float32, device=dev)
-    L = load()
+    packed = ((U8, prow, pcol // 2), (U8, prow, pcol // BLOCK), (F32, 1))
     if (deferred and not col and not sr and (center is None or kmode == MODE_PB16) and kmode in (MODE_P32, MODE_PB16)
             and x2.stride(0) == cols and rows * cols > 0):
         cen = None
@@ -297,14 +315,14 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
             cen = center.reshape(-1).to(device=dev, dtype=torch.bfloat16).contiguous()
             if cen.numel() != cols:
                 raise ValueError(f"center must have one value per column ({cols}), got {cen.numel()}")
-        parked = torch.empty(_deferred_bytes(rows, cols), dtype=torch.uint8, device=dev)
-        rc = L.metis_nvfp4_quant_row_deferred(x2.data_ptr(), rows, cols, kmode, None if cen is None else cen.data_ptr(),
-                                              codes.data_ptr(), parked.data_ptr(), parked.numel(), _stream())
-        if rc:
-            check(rc, "metis_nvfp4_quant_row_deferred", x.shape)
-        return PackedNVFP4(codes, None, unit, prow, pcol, mode, deferred=parked)
-    scales = torch.empty(prow, pcol // BLOCK, dtype=torch.uint8, device=dev)
+        size = _deferred_bytes(rows, cols)
+        new = _lib.call("metis_nvfp4_quant_row_deferred", dev.index, (packed[0], packed[2], (U8, size)),
+                        (x2, rows, cols, kmode, cen, "0", "2", size, _stream()))
+        if new.__class__ is int:
+            check(new, "metis_nvfp4_quant_row_deferred", x.shape)
+        return PackedNVFP4(new[0], None, new[1], prow, pcol, mode, deferred=new[2])
     ws = _workspace(rows, cols, dev, zeroed=resident)
+    tail = ("0", "1", "2", ws, ws.numel(), _stream())
     if center is not None:
         cen = center.reshape(-1).to(device=dev, dtype=torch.bfloat16 if mode == MODE_PB16 else torch.float32).contiguous()
         if cen.numel() != cols:
@@ -312,40 +330,29 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
         nz = None
         if sr and noise is not None:
             nz = noise.reshape(rows, cols).to(torch.bfloat16 if mode == MODE_PB16 else torch.float32).contiguous()
-        rc = L.metis_nvfp4_quant_centered(x2.data_ptr(), rows, cols, x2.stride(0), kmode, cen.data_ptr(), int(sr), int(col),
-                                          None if nz is None else nz.data_ptr(), seed & (2 ** 64 - 1), offset,
-                                          codes.data_ptr(), scales.data_ptr(), unit.data_ptr(), ws.data_ptr(), ws.numel(),
-                                          _stream())
-        if rc:
-            check(rc, "metis_nvfp4_quant_centered", x.shape)
-        return PackedNVFP4(codes, scales, unit, prow, pcol, mode)
-    if sr:
+        name = "metis_nvfp4_quant_centered"
+        new = _lib.call(name, dev.index, packed, (x2, rows, cols, x2.stride(0), kmode, cen, int(sr), int(col), nz, seed & (2 ** 64 - 1), offset, *tail))
+    elif sr:
         nz = None
         if noise is not None:
             want = torch.bfloat16 if mode == MODE_PB16 else torch.float32
             nz = noise.reshape(rows, cols).to(want).contiguous()
-        fn = L.metis_nvfp4_quant_sr_col if col else L.metis_nvfp4_quant_sr_row
-        rc = fn(x2.data_ptr(), rows, cols, x2.stride(0), kmode, None if nz is None else nz.data_ptr(),
-                seed & (2 ** 64 - 1), offset, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(),
-                ws.data_ptr(), ws.numel(), _stream())
+        name = "metis_nvfp4_quant_sr_col" if col else "metis_nvfp4_quant_sr_row"
+        new = _lib.call(name, dev.index, packed, (x2, rows, cols, x2.stride(0), kmode, nz, seed & (2 ** 64 - 1), offset, *tail))
     elif resident and not col and kmode in (MODE_P32, MODE_PB16) and x2.stride(0) == cols:
-        rc = L.metis_nvfp4_quant_row_resident(x2.data_ptr(), rows, cols, kmode, codes.data_ptr(), scales.data_ptr(),
-                                              unit.data_ptr(), ws.data_ptr(), ws.numel(), int(spin_limit), _stream())
+        name = "metis_nvfp4_quant_row_resident"
+        new = _lib.call(name, dev.index, packed, (x2, rows, cols, kmode, "0", "1", "2", ws, ws.numel(), int(spin_limit), _stream()))
     elif (decode_layout_activations and not col and kmode in (MODE_P32, MODE_PB16) and 0 < rows < 256 and cols % 256 == 0
           and x2.stride(0) == cols):
-        dec = torch.empty(L.metis_nvfp4_decode_weight_bytes(rows, cols), dtype=torch.uint8, device=dev)
-        rc = L.metis_nvfp4_quant_row_decode(x2.data_ptr(), rows, cols, kmode, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(),
-                                            dec.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-        if rc:
-            check(rc, "metis_nvfp4_quant_row_decode", x.shape)
-        return PackedNVFP4(codes, scales, unit, prow, pcol, mode, decode_layout=dec)
+        name = "metis_nvfp4_quant_row_decode"
+        new = _lib.call(name, dev.index, packed + ((U8, _decode_weight_bytes(rows, cols)),),
+                        (x2, rows, cols, kmode, "0", "1", "2", "3", ws, ws.numel(), _stream()))
     else:
-        fn = L.metis_nvfp4_quant_col if col else L.metis_nvfp4_quant_row
-        rc = fn(x2.data_ptr(), rows, cols, x2.stride(0), kmode, codes.data_ptr(), scales.data_ptr(),
-                unit.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    if rc:
-        check(rc, "metis_nvfp4_quant", x.shape)
-    return PackedNVFP4(codes, scales, unit, prow, pcol, mode)
+        name = "metis_nvfp4_quant_col" if col else "metis_nvfp4_quant_row"
+        new = _lib.call(name, dev.index, packed, (x2, rows, cols, x2.stride(0), kmode, *tail))
+    if new.__class__ is int:
+        check(new, name, x.shape)
+    return PackedNVFP4(new[0], new[1], new[2], prow, pcol, mode, decode_layout=new[3] if len(new) > 3 else None)
 
 
 def _quantize_col_padded(x2, kmode, mode, pad_rows, col, sr, noise, seed, offset, center) -> PackedNVFP4:
@@ -360,16 +367,12 @@ def _quantize_col_padded(x2, kmode, mode, pad_rows, col, sr, noise, seed, offset
         cen = center.reshape(-1).to(device=dev, dtype=torch.bfloat16 if mode == MODE_PB16 else torch.float32).contiguous()
         if cen.numel() != cols:
             raise ValueError(f"center must have one value per column ({cols}), got {cen.numel()}")
-    codes = torch.empty(cols, pad_rows // 2, dtype=torch.uint8, device=dev)
-    scales = torch.empty(cols, pad_rows // BLOCK, dtype=torch.uint8, device=dev)
-    unit = torch.empty(1, dtype=torch.float32, device=dev)
     ws = _workspace(pad_rows, cols, dev)
-    rc = load().metis_nvfp4_quant_col_padded(x2.data_ptr(), rows, pad_rows, cols, x2.stride(0), kmode, None if cen is None else cen.data_ptr(),
-                                             int(sr), seed & (2 ** 64 - 1), offset, codes.data_ptr(), scales.data_ptr(), unit.data_ptr(),
-                                             ws.data_ptr(), ws.numel(), _stream())
-    if rc:
-        check(rc, "metis_nvfp4_quant_col_padded", (rows, cols))
-    return PackedNVFP4(codes, scales, unit, cols, pad_rows, mode)
+    new = _lib.call("metis_nvfp4_quant_col_padded", dev.index, ((U8, cols, pad_rows // 2), (U8, cols, pad_rows // BLOCK), (F32, 1)),
+                    (x2, rows, pad_rows, cols, x2.stride(0), kmode, cen, int(sr), seed & (2 ** 64 - 1), offset, "0", "1", "2", ws, ws.numel(), _stream()))
+    if new.__class__ is int:
+        check(new, "metis_nvfp4_quant_col_padded", (rows, cols))
+    return PackedNVFP4(*new, cols, pad_rows, mode)
 
 
 def quantize_dequantize(x: torch.Tensor, mode: int = MODE_P32) -> tuple[PackedNVFP4, torch.Tensor]:
@@ -453,12 +456,11 @@ def roundtrip(x: torch.Tensor, spin_limit: int = 0) -> torch.Tensor | None:
         ws = _captured_workspace(need, x.device, True)
     elif need:
         ws = _kept_workspace(need, x.device)
-    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    rc = load().metis_nvfp4_roundtrip(x2.data_ptr(), rows, cols, kmode, out.data_ptr(), None if ws is None else ws.data_ptr(), need, int(spin_limit),
-                                      _stream())
-    if rc:
-        check(rc, "metis_nvfp4_roundtrip", x.shape)
-    return out
+    new = _lib.call("metis_nvfp4_roundtrip", x.device.index, ((B16 if kmode == MODE_PB16 else F32, *x.shape),),
+                    (x2, rows, cols, kmode, "0", ws, need, int(spin_limit), _stream()))
+    if new.__class__ is int:
+        check(new, "metis_nvfp4_roundtrip", x.shape)
+    return new[0]
 
 
 def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tensor, mode: int = MODE_P32,
@@ -483,18 +485,16 @@ def quantize_lowrank_residual(x: torch.Tensor, us: torch.Tensor, vt: torch.Tenso
         raise ValueError(f"NVFP4 block shape (1, 16) does not divide {tuple(x.shape)} or the rank {r}")
     us, vt = us.contiguous(), vt.contiguous()
     dev = x2.device
-    codes = torch.empty(rows, cols // 2, dtype=torch.uint8, device=dev)
-    scales = torch.empty(rows, cols // BLOCK, dtype=torch.uint8, device=dev)
-    unit = torch.empty(1, dtype=torch.float32, device=dev)
-    out = torch.empty(rows, cols, dtype=want, device=dev) if dense else None
     ws = _workspace(rows, cols, dev)
-    rc = load().metis_nvfp4_quant_lowrank_residual(x2.data_ptr(), DTYPE_F32 if x2.dtype == torch.float32 else DTYPE_BF16, us.data_ptr(),
-                                                   vt.data_ptr(), rows, cols, r, mode, codes.data_ptr(), scales.data_ptr(),
-                                                   unit.data_ptr(), None if out is None else out.data_ptr(), ws.data_ptr(),
-                                                   ws.numel(), _stream())
-    if rc:
-        check(rc, "metis_nvfp4_quant_lowrank_residual", (rows, cols, r))
-    return PackedNVFP4(codes, scales, unit, rows, cols, mode), out
+    specs = ((U8, rows, cols // 2), (U8, rows, cols // BLOCK), (F32, 1))
+    if dense:
+        specs += ((F32 if want == torch.float32 else B16, rows, cols),)
+    new = _lib.call("metis_nvfp4_quant_lowrank_residual", dev.index, specs,
+                    (x2, DTYPE_F32 if x2.dtype == torch.float32 else DTYPE_BF16, us, vt, rows, cols, r, mode, "0", "1", "2", "3" if dense else None,
+                     ws, ws.numel(), _stream()))
+    if new.__class__ is int:
+        check(new, "metis_nvfp4_quant_lowrank_residual", (rows, cols, r))
+    return PackedNVFP4(new[0], new[1], new[2], rows, cols, mode), new[3] if dense else None
 
 
 def _check_bf16_copy(copy: torch.Tensor | None, x2: torch.Tensor, kmode: int) -> None:
@@ -527,32 +527,23 @@ def quantize_both_sr(x: torch.Tensor, mode: int = MODE_P32, *, seed: int = 0, of
     if rows % BLOCK or cols % BLOCK:
         raise ValueError(f"NVFP4 block shape (1, 16) does not divide tensor shape {tuple(x.shape)} both ways")
     dev = x2.device
-    L = load()
-    packs = []
-    for prow, pcol in ((rows, cols), (cols, rows)):
-        packs.append((torch.empty(prow, pcol // 2, dtype=torch.uint8, device=dev),
-                      torch.empty(prow, pcol // BLOCK, dtype=torch.uint8, device=dev),
-                      torch.empty(1, dtype=torch.float32, device=dev)))
+    specs = ((U8, rows, cols // 2), (U8, rows, cols // BLOCK), (F32, 1), (U8, cols, rows // 2), (U8, cols, rows // BLOCK), (F32, 1))
     ws = _workspace(rows, cols, dev, tensors=2)
-    (cr, sr_, ur), (cc, sc, uc) = packs
-    if center is not None and rows * cols:
-        rc = L.metis_nvfp4_quant_sr_both_centered(x2.data_ptr(), have, rows, cols, x2.stride(0), kmode, center.data_ptr(), seed & (2 ** 64 - 1),
-                                                  offset_row, offset_col, cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(),
-                                                  uc.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-        if rc:
-            check(rc, "metis_nvfp4_quant_sr_both_centered", x.shape)
-    elif bf16_copy is not None and rows * cols:
-        rc = L.metis_nvfp4_quant_sr_both_copy(x2.data_ptr(), have, rows, cols, x2.stride(0), seed & (2 ** 64 - 1), offset_row, offset_col,
-                                              cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(), uc.data_ptr(),
-                                              bf16_copy.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-        if rc:
-            check(rc, "metis_nvfp4_quant_sr_both_copy", x.shape)
-    elif rows * cols:
-        rc = L.metis_nvfp4_quant_sr_both_padded(x2.data_ptr(), have, rows, cols, x2.stride(0), kmode, seed & (2 ** 64 - 1), offset_row,
-                                                offset_col, cr.data_ptr(), sr_.data_ptr(), ur.data_ptr(), cc.data_ptr(), sc.data_ptr(),
-                                                uc.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-        if rc:
-            check(rc, "metis_nvfp4_quant_sr_both_padded", x.shape)
+    seeds, outs = (seed & (2 ** 64 - 1), offset_row, offset_col), ("0", "1", "2", "3", "4", "5")
+    if not rows * cols:
+        new = tuple([torch.empty(*size, dtype=torch.uint8 if kind == U8 else torch.float32, device=dev) for kind, *size in specs])
+    elif center is not None:
+        name = "metis_nvfp4_quant_sr_both_centered"
+        new = _lib.call(name, dev.index, specs, (x2, have, rows, cols, x2.stride(0), kmode, center, *seeds, *outs, ws, ws.numel(), _stream()))
+    elif bf16_copy is not None:
+        name = "metis_nvfp4_quant_sr_both_copy"
+        new = _lib.call(name, dev.index, specs, (x2, have, rows, cols, x2.stride(0), *seeds, *outs, bf16_copy, ws, ws.numel(), _stream()))
+    else:
+        name = "metis_nvfp4_quant_sr_both_padded"
+        new = _lib.call(name, dev.index, specs, (x2, have, rows, cols, x2.stride(0), kmode, *seeds, *outs, ws, ws.numel(), _stream()))
+    if new.__class__ is int:
+        check(new, name, x.shape)
+    cr, sr_, ur, cc, sc, uc = new
     if have != rows:
         cr, sr_ = cr[:have], sr_[:have]
     return PackedNVFP4(cr, sr_, ur, have, cols, mode), PackedNVFP4(cc, sc, uc, cols, rows, mode)
@@ -697,6 +688,7 @@ class TokenMean:
     cached: torch.Tensor | None = None
     cached_count: int = 0
     v: torch.Tensor | None = None
+    checked: bool = False                     # the caller has just asked token_mean_applies
     # results
     mean: torch.Tensor | None = None
     mean32: torch.Tensor | None = None
@@ -704,37 +696,33 @@ class TokenMean:
 
 
 def _quantize_token_mean(x2: torch.Tensor, tm: TokenMean) -> PackedNVFP4:
-    if not token_mean_applies(x2, tm.after_norm):
+    if not (tm.checked or token_mean_applies(x2, tm.after_norm)):
         raise ValueError("a TokenMean centre: outside the call's domain (see token_mean_applies)")
     after_norm, cached, cached_count, v = tm.after_norm, tm.cached, tm.cached_count, tm.v
     rows, cols = x2.shape
     dev = x2.device
-    cp = None
     if cached is not None:
         cached = cached.to(device=dev, dtype=torch.bfloat16).contiguous()
         if cached.numel() != cols:
             raise ValueError(f"cached mean has {cached.numel()} values, the tensor {cols} columns")
-        cp = cached.data_ptr()
-    me = torch.empty(cols, dtype=torch.bfloat16, device=dev)
-    me32 = torch.empty(cols, dtype=torch.float32, device=dev)
-    codes = torch.empty(rows, cols // 2, dtype=torch.uint8, device=dev)
-    unit = torch.empty(1, dtype=torch.float32, device=dev)
     size = _deferred_bytes(rows, cols)
-    parked = torch.empty(size, dtype=torch.uint8, device=dev)
-    pending, vp, R, need = None, None, 0, 0
+    specs = ((B16, cols), (F32, cols), (U8, rows, cols // 2), (F32, 1), (U8, size))
+    R = need = 0
+    pending = None
     if v is not None:
         v = v.contiguous()
         R = v.shape[0]
         if v.dtype != torch.bfloat16 or v.shape[1] != cols or v.device != dev:
             raise ValueError("TokenMean: v is bfloat16 [r, cols] on the tensor's device")
         need = _lowrank_workspace_bytes(rows, R, cols)
-        pending = torch.empty(need, dtype=torch.uint8, device=dev)
-        vp = v.data_ptr()
-    rc = load().metis_token_mean_quant_deferred(x2.data_ptr(), rows, cols, int(after_norm), cp, int(cached_count), me.data_ptr(), me32.data_ptr(),
-                                                codes.data_ptr(), parked.data_ptr(), size, vp, R, None if pending is None else pending.data_ptr(),
-                                                need, _stream())
-    if rc:
-        check(rc, "metis_token_mean_quant_deferred", (rows, cols, R))
+        specs += ((U8, need),)
+        pending = "5"
+    new = _lib.call("metis_token_mean_quant_deferred", dev.index, specs,
+                    (x2, rows, cols, after_norm, cached, int(cached_count), "0", "1", "2", "4", size, v, R, pending, need, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_token_mean_quant_deferred", (rows, cols, R))
+    me, me32, codes, unit, parked = new[:5]
+    pending = None if v is None else new[5]
     tm.mean, tm.mean32, tm.pending = me, me32, pending
     return PackedNVFP4(codes, None, unit, rows, cols, MODE_PB16, deferred=parked)
 
@@ -824,7 +812,7 @@ def expand_tiled(p: PackedNVFP4, cache: bool = True, mode: int = MODE_P32, cente
     cache=True keeps it on the packed tensor (weights); activations are expanded per call.
     center (bf16 [cols], mode PB16): p packs a centred residual; the operand is the mean mode's center + QDQ(x - center)
     rounded to bf16, the tensor the reference multiplies with in bf16 arithmetic."""
-    L = load()
+    dev, spec = p.codes.device.index, ((U8, _expand_tiled_bytes(p.rows, p.cols)),)
     d = p.__dict__
     lazy = d.get("deferred") is not None and d.get("_scales") is None and p.rht is None and p.cols % 32 == 0
     if center is not None:
@@ -837,38 +825,33 @@ def expand_tiled(p: PackedNVFP4, cache: bool = True, mode: int = MODE_P32, cente
         kept = d.get("_tiled_centered")
         if cache and kept is not None and kept[0] == key:
             return kept[1]
-        out = torch.empty(_expand_tiled_bytes(p.rows, p.cols), dtype=torch.uint8, device=p.codes.device)
-        if cache:
-            d["_tiled_centered"] = (key, out, center)                 # (the centre is kept alive with its address)
         if lazy:
-            rc = L.metis_nvfp4_expand_tiled_deferred(p.codes.data_ptr(), d["deferred"].data_ptr(), p.rows, p.cols, p.mode, mode,
-                                                     center.data_ptr(), d["_unit"].data_ptr(), out.data_ptr(), _stream())
+            new = _lib.call("metis_nvfp4_expand_tiled_deferred", dev, spec, (p.codes, d["deferred"], p.rows, p.cols, p.mode, mode, center, d["_unit"], "0", _stream()))
             d["_unit_ready"] = True
         else:
-            rc = L.metis_nvfp4_expand_tiled_centered(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols,
-                                                     center.data_ptr(), out.data_ptr(), _stream())
-        if rc:
-            check(rc, "metis_nvfp4_expand_tiled_centered", (p.rows, p.cols))
+            new = _lib.call("metis_nvfp4_expand_tiled_centered", dev, spec, (p.codes, p.scales, p.unit, p.rows, p.cols, center, "0", _stream()))
+        if new.__class__ is int:
+            check(new, "metis_nvfp4_expand_tiled_centered", (p.rows, p.cols))
+        out = new[0]
+        if cache:
+            d["_tiled_centered"] = (key, out, center)                 # (the centre is kept alive with its address)
         return out
     have = p.tiled_pb16 if mode == MODE_PB16 else p.tiled
     if have is not None:
         return have
-    out = torch.empty(_expand_tiled_bytes(p.rows, p.cols), dtype=torch.uint8, device=p.codes.device)
     if lazy:
         # the scale bytes were never written: this kernel forms them from the parked block maxima, and writes the unit
-        rc = L.metis_nvfp4_expand_tiled_deferred(p.codes.data_ptr(), d["deferred"].data_ptr(), p.rows, p.cols, p.mode, mode,
-                                                 None, d["_unit"].data_ptr(), out.data_ptr(), _stream())
-        if rc:
-            check(rc, "metis_nvfp4_expand_tiled_deferred", (p.rows, p.cols))
+        new = _lib.call("metis_nvfp4_expand_tiled_deferred", dev, spec, (p.codes, d["deferred"], p.rows, p.cols, p.mode, mode, None, d["_unit"], "0", _stream()))
+        if new.__class__ is int:
+            check(new, "metis_nvfp4_expand_tiled_deferred", (p.rows, p.cols))
         d["_unit_ready"] = True
     elif p.rht is not None:                   # NV recipe: the operand holds the values rotated back
-        rc = L.metis_nvfp4_expand_tiled_rht(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, mode,
-                                            p.rht, 1, 0, out.data_ptr(), _stream())
+        new = _lib.call("metis_nvfp4_expand_tiled_rht", dev, spec, (p.codes, p.scales, p.unit, p.rows, p.cols, mode, p.rht, 1, 0, "0", _stream()))
     else:
-        rc = L.metis_nvfp4_expand_tiled(p.codes.data_ptr(), p.scales.data_ptr(), p.unit.data_ptr(), p.rows, p.cols, mode,
-                                        out.data_ptr(), _stream())
-    if rc:
-        check(rc, "metis_nvfp4_expand_tiled", (p.rows, p.cols))
+        new = _lib.call("metis_nvfp4_expand_tiled", dev, spec, (p.codes, p.scales, p.unit, p.rows, p.cols, mode, "0", _stream()))
+    if new.__class__ is int:
+        check(new, "metis_nvfp4_expand_tiled", (p.rows, p.cols))
+    out = new[0]
     if cache and (tiled_weight_copies or not p.persistent):
         if mode == MODE_PB16:
             p.tiled_pb16 = out
@@ -982,7 +965,6 @@ def project_and_operand(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: P
         raise ValueError("project_and_operand: outside the call's domain (see project_and_operand_applies)")
     M, K = x2.shape
     R = v.shape[0]
-    L = load()
     dev = x2.device
     v = v.contiguous()
     s = s.contiguous()
@@ -990,21 +972,17 @@ def project_and_operand(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, p: P
         center = _bf16_row(center)
         if center.numel() != K:
             raise ValueError(f"center must have {K} values, got {center.numel()}")
-    xv = torch.empty(M, R, dtype=torch.bfloat16, device=dev)
-    t = torch.empty(M, R, dtype=torch.bfloat16, device=dev)
-    out = torch.empty(_decode_operand_bytes(M, K), dtype=torch.uint8, device=dev)
     need = _lowrank_workspace_bytes(M, R, K)
     if pending is not None and (pending.numel() < need or pending.device != dev):
         raise ValueError("project_and_operand: `pending` is not what quantize_project_decode or a TokenMean's call leaves for these shapes")
-    ws = pending if pending is not None else torch.empty(need, dtype=torch.uint8, device=dev)
+    specs = ((B16, M, R), (B16, M, R), (U8, _decode_operand_bytes(M, K)))
     d = p.__dict__
-    rc = L.metis_decode_prepare_deferred(None if pending is not None else x2.data_ptr(), x2.stride(0), v.data_ptr(), R, s.data_ptr(),
-                                         xv.data_ptr(), t.data_ptr(),
-                                         ws.data_ptr(), need, p.codes.data_ptr(), d["deferred"].data_ptr(), M, K, p.mode, mode,
-                                         None if center is None else center.data_ptr(), d["_unit"].data_ptr(), out.data_ptr(),
-                                         int(rotate is not None), int(rotate or 0), _stream())
-    if rc:
-        check(rc, "metis_decode_prepare_deferred", (M, K, R))
+    new = _lib.call("metis_decode_prepare_deferred", dev.index, specs if pending is not None else specs + ((U8, need),),
+                    (None if pending is not None else x2, x2.stride(0), v, R, s, "0", "1", "3" if pending is None else pending, need,
+                     p.codes, d["deferred"], M, K, p.mode, mode, center, d["_unit"], "2", rotate is not None, int(rotate or 0), _stream()))
+    if new.__class__ is int:
+        check(new, "metis_decode_prepare_deferred", (M, K, R))
+    xv, t, out = new[:3]
     d["_unit_ready"] = True
     return xv, t, out
 
@@ -1068,25 +1046,22 @@ def gemm_tiled(ax: torch.Tensor, a_unit: torch.Tensor, bx: torch.Tensor, b_unit:
     bias_f32 = bias is not None and bias.dtype == torch.float32
     if bias is not None:
         bias = bias.contiguous() if bias_f32 else bias.to(torch.bfloat16).contiguous()
-    out = torch.empty(M, N, dtype=out_dtype, device=dev)
     need = _tiled_workspace_bytes(M, N, K, mode, dev.index or 0) if split_k else 0
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-    rc = load().metis_linear_fwd_tiled(ax.data_ptr(), a_unit.data_ptr(), bx.data_ptr(), b_unit.data_ptr(), M, N, K,
-                                       None if t is None else t.data_ptr(), None if u is None else u.data_ptr(), r,
-                                       None if bias is None else bias.data_ptr(), int(bias_f32), out.data_ptr(),
-                                       DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, mode,
-                                       None if ws is None else ws.data_ptr(), need, _stream())
-    if rc:
-        check(rc, "metis_linear_fwd_tiled", (M, N, K))
-    return out
+    f32 = out_dtype == torch.float32
+    specs = ((F32 if f32 else B16, M, N), (U8, need)) if need else ((F32 if f32 else B16, M, N),)
+    new = _lib.call("metis_linear_fwd_tiled", dev.index, specs,
+                    (ax, a_unit, bx, b_unit, M, N, K, t, u, r, bias, bias_f32, "0", DTYPE_F32 if f32 else DTYPE_BF16, mode, "1" if need else None, need, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_linear_fwd_tiled", (M, N, K))
+    return new[0]
 
 
 def linear_fwd_tiled(a: PackedNVFP4, b: PackedNVFP4, *, t: torch.Tensor | None = None, u: torch.Tensor | None = None,
                      bias: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16,
                      a_tiled: torch.Tensor | None = None, reference_rounding: bool = False,
-                     split_k: bool = True, center: torch.Tensor | None = None, batch: "_TiledBatch | None" = None) -> torch.Tensor:
+                     split_k: bool = True, center: torch.Tensor | None = None, batch: "_TiledBatch | None" = None) -> torch.Tensor | None:
     """linear_fwd on tiled 16-bit expansions: b's is cached on b when b is persistent, a's is made here unless given.
-    batch: the product is queued there and its output, returned, is filled when the batch runs (linear_fwd_tiled_grouped).
+    batch: the product is queued there, for the launch that runs them all (linear_fwd_tiled_grouped); no output is returned.
 
     reference_rounding (both operands packed in bf16 arithmetic): operands are the reference's bf16 dequantized
     values and the epilogue rounds where the reference's all-bf16 forward rounds; otherwise exact products.
@@ -1134,23 +1109,21 @@ def _linear_fwd_tiled_grouped(a: PackedNVFP4, members, out_dtype, center, refere
     if center is not None and mode != MODE_PB16:
         raise ValueError("a centre inside the operand belongs to reference_rounding")
     ax = expand_tiled(a, cache=False, mode=mode, center=center)
-    batch = _TiledBatch(a, ax, len(members), out_dtype, mode)
-    outs = [linear_fwd_tiled(a, b, t=t, u=u, bias=bias, out_dtype=out_dtype, a_tiled=ax, reference_rounding=mode == MODE_PB16, center=center,
-                             batch=batch) for b, t, u, bias in members]
-    batch.run()
-    return outs
+    batch = _TiledBatch(a, ax, out_dtype, mode)
+    for b, t, u, bias in members:
+        linear_fwd_tiled(a, b, t=t, u=u, bias=bias, out_dtype=out_dtype, a_tiled=ax, reference_rounding=mode == MODE_PB16, center=center, batch=batch)
+    return batch.run()
 
 
 class _TiledBatch:
     """Products of one tiled activation that run as one launch."""
 
-    def __init__(self, a: PackedNVFP4, ax: torch.Tensor, count: int, out_dtype: torch.dtype, mode: int):
+    def __init__(self, a: PackedNVFP4, ax: torch.Tensor, out_dtype: torch.dtype, mode: int):
         self.a, self.ax, self.out_dtype, self.mode = a, ax, out_dtype, mode
-        self.members = (_lib.LinearMember * count)()
+        self.members: list = []                                    # as _lib.call takes them
         self.rows: list[int] = []
-        self.keep: list = []                                       # until the launch is enqueued
 
-    def add(self, bx, b, t, u, bias) -> torch.Tensor:
+    def add(self, bx, b, t, u, bias) -> None:
         M = self.a.rows
         r = ldt = 0
         if t is not None:
@@ -1167,23 +1140,22 @@ class _TiledBatch:
         bias_f32 = bias is not None and bias.dtype == torch.float32
         if bias is not None:
             bias = bias.contiguous() if bias_f32 else bias.to(torch.bfloat16).contiguous()
-        out = torch.empty(M, b.rows, dtype=self.out_dtype, device=self.ax.device)
-        self.members[len(self.rows)] = _lib.LinearMember(
-            bx.data_ptr(), None, b.unit.data_ptr(), None if t is None else t.data_ptr(), None if u is None else u.data_ptr(), r,
-            None if bias is None else bias.data_ptr(), out.data_ptr(), b.rows, int(bias_f32), ldt, None)
+        self.members.append((bx, None, b.unit, t, u, r, bias, _OUT[len(self.rows)], b.rows, bias_f32, ldt, None))
         self.rows.append(b.rows)
-        self.keep += [bx, t, u, bias]
-        return out
 
-    def run(self) -> None:
-        a, dev = self.a, self.ax.device
+    def run(self) -> list[torch.Tensor]:
+        a, dev, count = self.a, self.ax.device, len(self.rows)
         need = _tiled_group_workspace_bytes(a.rows, a.cols, tuple(self.rows), dev.index or 0)
-        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-        rc = load().metis_linear_fwd_tiled_grouped(self.ax.data_ptr(), a.unit.data_ptr(), a.rows, a.cols, ctypes.addressof(self.members),
-                                                   len(self.rows), DTYPE_F32 if self.out_dtype == torch.float32 else DTYPE_BF16, self.mode,
-                                                   None if ws is None else ws.data_ptr(), need, _stream())
-        if rc:
-            check(rc, "metis_linear_fwd_tiled_grouped", (a.rows, a.cols, self.rows))
+        f32 = self.out_dtype == torch.float32
+        specs = [(F32 if f32 else B16, a.rows, n) for n in self.rows]
+        if need:
+            specs.append((U8, need))
+        new = _lib.call("metis_linear_fwd_tiled_grouped", dev.index, tuple(specs),
+                        (self.ax, a.unit, a.rows, a.cols, self.members, count, DTYPE_F32 if f32 else DTYPE_BF16, self.mode, _OUT[count] if need else None, need,
+                         _stream()))
+        if new.__class__ is int:
+            check(new, "metis_linear_fwd_tiled_grouped", (a.rows, a.cols, self.rows))
+        return list(new[:count])
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1204,39 +1176,30 @@ def rmsnorm_quantize(x: torch.Tensor, gamma: torch.Tensor, eps: float, mode: int
         raise ValueError(f"NVFP4 block shape (1, 16) does not divide tensor shape {tuple(x.shape)}")
     g = gamma.to(device=x2.device, dtype=torch.bfloat16).contiguous()
     dev = x2.device
-    normed = torch.empty(rows, cols, dtype=torch.bfloat16, device=dev) if want_normed else None
-    codes = torch.empty(rows, cols // 2, dtype=torch.uint8, device=dev)
-    unit = torch.empty(1, dtype=torch.float32, device=dev)
+    # the packed tensor's parts, then the normed tensor if it is wanted
+    normed = "4" if want_normed else None
+    extra = ((B16, rows, cols),) if want_normed else ()
+    codes, unit = (U8, rows, cols // 2), (F32, 1)
     if deferred and rows * cols > 0:
-        L = load()
-        parked = torch.empty(_deferred_bytes(rows, cols), dtype=torch.uint8, device=dev)
-        rc = L.metis_rmsnorm_nvfp4_quant_deferred(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, mode,
-                                                  None if normed is None else normed.data_ptr(), codes.data_ptr(),
-                                                  parked.data_ptr(), parked.numel(), _stream())
-        if rc:
-            check(rc, "metis_rmsnorm_nvfp4_quant_deferred", x.shape)
-        if normed is not None:
-            normed = normed.reshape(x.shape)
-        return normed, PackedNVFP4(codes, None, unit, rows, cols, mode, deferred=parked)
-    scales = torch.empty(rows, cols // BLOCK, dtype=torch.uint8, device=dev)
+        size = _deferred_bytes(rows, cols)
+        name = "metis_rmsnorm_nvfp4_quant_deferred"
+        new = _lib.call(name, dev.index, (codes, unit, (U8, size), *extra), (x2, g, float(eps), rows, cols, mode, "3" if want_normed else None, "0", "2", size, _stream()))
+        if new.__class__ is int:
+            check(new, name, x.shape)
+        return new[3].reshape(x.shape) if want_normed else None, PackedNVFP4(new[0], None, new[1], rows, cols, mode, deferred=new[2])
     ws = _workspace(rows, cols, dev)
-    dec = None
-    if decode_layout_activations and 0 < rows < 256 and cols % 256 == 0:
-        L = load()
-        dec = torch.empty(L.metis_nvfp4_decode_weight_bytes(rows, cols), dtype=torch.uint8, device=dev)
-        rc = L.metis_rmsnorm_nvfp4_quant_decode(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, mode,
-                                                None if normed is None else normed.data_ptr(), codes.data_ptr(),
-                                                scales.data_ptr(), unit.data_ptr(), dec.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                _stream())
+    decode = decode_layout_activations and 0 < rows < 256 and cols % 256 == 0
+    specs = (codes, (U8, rows, cols // BLOCK), unit, (U8, _decode_weight_bytes(rows, cols) if decode else 0), *extra)
+    if decode:
+        name = "metis_rmsnorm_nvfp4_quant_decode"
+        new = _lib.call(name, dev.index, specs, (x2, g, float(eps), rows, cols, mode, normed, "0", "1", "2", "3", ws, ws.numel(), _stream()))
     else:
-        rc = load().metis_rmsnorm_nvfp4_quant(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, mode,
-                                              None if normed is None else normed.data_ptr(), codes.data_ptr(),
-                                              scales.data_ptr(), unit.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    if rc:
-        check(rc, "metis_rmsnorm_nvfp4_quant", x.shape)
-    if normed is not None:
-        normed = normed.reshape(x.shape)
-    return normed, PackedNVFP4(codes, scales, unit, rows, cols, mode, decode_layout=dec)
+        name = "metis_rmsnorm_nvfp4_quant"
+        new = _lib.call(name, dev.index, specs, (x2, g, float(eps), rows, cols, mode, normed, "0", "1", "2", ws, ws.numel(), _stream()))
+    if new.__class__ is int:
+        check(new, name, x.shape)
+    return (new[4].reshape(x.shape) if want_normed else None,
+            PackedNVFP4(new[0], new[1], new[2], rows, cols, mode, decode_layout=new[3] if decode else None))
 
 
 def rmsnorm(x: torch.Tensor, gamma: torch.Tensor, eps: float) -> torch.Tensor:
@@ -1244,11 +1207,10 @@ def rmsnorm(x: torch.Tensor, gamma: torch.Tensor, eps: float) -> torch.Tensor:
     x2 = _as_2d_bf16(x)
     rows, cols = x2.shape
     g = gamma.to(device=x2.device, dtype=torch.bfloat16).contiguous()
-    normed = torch.empty(rows, cols, dtype=torch.bfloat16, device=x2.device)
-    rc = load().metis_rmsnorm(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, normed.data_ptr(), _stream())
-    if rc:
-        check(rc, "metis_rmsnorm", x.shape)
-    return normed
+    new = _lib.call("metis_rmsnorm", x2.device.index, ((B16, rows, cols),), (x2, g, float(eps), rows, cols, "0", _stream()))
+    if new.__class__ is int:
+        check(new, "metis_rmsnorm", x.shape)
+    return new[0]
 
 
 def rmsnorm_colmean(x: torch.Tensor, gamma: torch.Tensor, eps: float, mean_dtype: torch.dtype = torch.float32,
@@ -1264,23 +1226,18 @@ def rmsnorm_colmean(x: torch.Tensor, gamma: torch.Tensor, eps: float, mean_dtype
         raise ValueError("rmsnorm_colmean: the mean is bfloat16 or float32")
     dev = x2.device
     g = gamma.to(device=dev, dtype=torch.bfloat16).contiguous()
-    normed = torch.empty(rows, cols, dtype=torch.bfloat16, device=dev)
-    me = torch.empty(cols, dtype=mean_dtype, device=dev)
-    me32 = me if mean_dtype == torch.float32 else torch.empty(cols, dtype=torch.float32, device=dev)
-    L = load()
-    ws = torch.empty(max(L.metis_rmsnorm_colmean_workspace_bytes(rows, cols), 16), dtype=torch.uint8, device=dev)
-    cp = None
+    f32 = mean_dtype == torch.float32
+    size = _rmsnorm_colmean_bytes(rows, cols)
     if cached is not None:
         cached = cached.reshape(-1).to(device=dev, dtype=mean_dtype).contiguous()
         if cached.numel() != cols:
             raise ValueError(f"cached mean must have one value per column ({cols}), got {cached.numel()}")
-        cp = cached.data_ptr()
-    rc = L.metis_rmsnorm_colmean(x2.data_ptr(), g.data_ptr(), float(eps), rows, cols, normed.data_ptr(), me.data_ptr(),
-                                 DTYPE_F32 if mean_dtype == torch.float32 else DTYPE_BF16, cp, int(cached_count),
-                                 None if me32 is me else me32.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    if rc:
-        check(rc, "metis_rmsnorm_colmean", x.shape)
-    return normed, me, me32
+    specs = ((B16, rows, cols), (U8, size), (F32 if f32 else B16, cols))
+    new = _lib.call("metis_rmsnorm_colmean", dev.index, specs if f32 else specs + ((F32, cols),),
+                    (x2, g, float(eps), rows, cols, "0", "2", DTYPE_F32 if f32 else DTYPE_BF16, cached, int(cached_count), None if f32 else "3", "1", size, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_rmsnorm_colmean", x.shape)
+    return new[0], new[2], new[2] if f32 else new[3]
 
 
 def rmsnorm_backward_applies(x: torch.Tensor, g: torch.Tensor, gamma: torch.Tensor) -> bool:
@@ -1302,19 +1259,13 @@ def rmsnorm_backward(x: torch.Tensor, g: torch.Tensor, gamma: torch.Tensor, eps:
     x2, g2 = dense(x, cols), dense(g, cols)
     gm = dense(gamma, cols)
     rows = x2.shape[0]
-    gx = torch.empty(rows, cols, dtype=torch.bfloat16, device=x.device)
-    L = load()
-    gg = ws = None
-    need = 0
-    if want_gamma:
-        gg = torch.empty(cols, dtype=torch.bfloat16, device=x.device)
-        need = L.metis_rmsnorm_backward_workspace_bytes(rows, cols)
-        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
-    rc = L.metis_rmsnorm_backward(x2.data_ptr(), g2.data_ptr(), gm.data_ptr(), float(eps), rows, cols, gx.data_ptr(),
-                                  None if gg is None else gg.data_ptr(), DTYPE_BF16, None if ws is None else ws.data_ptr(), need, _stream())
-    if rc:
-        check(rc, "metis_rmsnorm_backward", x.shape)
-    return gx.reshape(x.shape), gg
+    need = _rmsnorm_backward_bytes(rows, cols) if want_gamma else 0
+    specs = ((B16, rows, cols), (B16, cols), (U8, need)) if want_gamma else ((B16, rows, cols),)
+    new = _lib.call("metis_rmsnorm_backward", x.device.index, specs,
+                    (x2, g2, gm, float(eps), rows, cols, "0", "1" if want_gamma else None, DTYPE_BF16, "2" if want_gamma else None, need, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_rmsnorm_backward", x.shape)
+    return new[0].reshape(x.shape), new[1] if want_gamma else None
 
 
 @functools.lru_cache(maxsize=16)
@@ -1352,6 +1303,14 @@ def _grouped_plan(M: int, K: int, ns: tuple, device_index: int) -> tuple[int, bo
     L = load()
     need = int(L.metis_linear_grouped_workspace_bytes(M, K, ap, len(ns)))
     return need, bool(L.metis_linear_grouped_centered_supported(M, K, ap, len(ns), int(need > 0)))
+
+
+@functools.lru_cache(maxsize=4096)
+def _grouped_centre_fits_unsplit(M: int, K: int, ns: tuple) -> bool:
+    arr = (_lib.LinearMember * len(ns))()
+    for i, n in enumerate(ns):
+        arr[i].N = n
+    return bool(load().metis_linear_grouped_centered_supported(M, K, ctypes.cast(arr, ctypes.c_void_p), len(ns), 0))
 
 
 def _gemm_workspace(M: int, N: int, K: int, device: torch.device) -> torch.Tensor | None:
@@ -1529,29 +1488,16 @@ def lowrank_stack_applies(x2: torch.Tensor, factors) -> bool:
     return total in ONE_PASS_RANKS and _lowrank_operands(x2, *factors[0])
 
 
-_FactorArrays = [None] + [ctypes.c_int64 * (3 * n) for n in range(1, 5)]     # metis_lowrank_factor is three 64-bit words
-
-
 def _lowrank_project_stack(x2: torch.Tensor, v: FactorStack, s: FactorStack):
     (M, K), R = x2.shape, v.shape[0]
-    keep, words = [], []
-    for a, b in zip(v.parts, s.parts):
-        if not a.is_contiguous():
-            a = a.contiguous()
-        if not b.is_contiguous():
-            b = b.contiguous()
-        keep.append((a, b))
-        words += (a.data_ptr(), b.data_ptr(), a.shape[0])
-    arr = _FactorArrays[len(keep)](*words)
-    xv = torch.empty(M, R, dtype=torch.bfloat16, device=x2.device)
-    t = torch.empty_like(xv)
+    factors = [(a if a.is_contiguous() else a.contiguous(), b if b.is_contiguous() else b.contiguous(), a.shape[0]) for a, b in zip(v.parts, s.parts)]
     need = _lowrank_rows_workspace_bytes(M, R, K, x2.device.index or 0)
-    ws = torch.empty(need, dtype=torch.uint8, device=x2.device) if need else None
-    rc = load().metis_lowrank_project_rows_grouped(x2.data_ptr(), x2.stride(0), M, K, ctypes.addressof(arr), len(keep), xv.data_ptr(), t.data_ptr(),
-                                                   None if ws is None else ws.data_ptr(), need, _stream())
-    if rc:
-        check(rc, "metis_lowrank_project_rows_grouped", (M, [a.shape[0] for a, _ in keep], K))
-    return xv, t
+    specs = ((B16, M, R), (B16, M, R))
+    new = _lib.call("metis_lowrank_project_rows_grouped", x2.device.index, specs + ((U8, need),) if need else specs,
+                    (x2, x2.stride(0), M, K, factors, len(factors), "0", "1", "2" if need else None, need, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_lowrank_project_rows_grouped", (M, [f[2] for f in factors], K))
+    return new[0], new[1]
 
 
 def lowrank_project(x2: torch.Tensor, v: "torch.Tensor | FactorStack", s: "torch.Tensor | FactorStack | None" = None):
@@ -1569,24 +1515,20 @@ def lowrank_project(x2: torch.Tensor, v: "torch.Tensor | FactorStack", s: "torch
         xv = torch.matmul(x2, v.T)
         return xv if s is None else (xv, xv * s.to(xv.dtype))
     v = v.contiguous()
-    L = load()
-    xv = torch.empty(M, R, dtype=torch.bfloat16, device=x2.device)
-    t = None if s is None else torch.empty_like(xv)
-    sp = None if s is None else s.contiguous().data_ptr()
+    specs = ((B16, M, R),)
+    tp = None
+    if s is not None:
+        s, specs, tp = s.contiguous(), ((B16, M, R), (B16, M, R)), "1"
     if large:
-        need = _lowrank_rows_workspace_bytes(M, R, K, x2.device.index or 0)
-        ws = torch.empty(need, dtype=torch.uint8, device=x2.device) if need else None
-        rc = L.metis_lowrank_project_rows_ws(x2.data_ptr(), x2.stride(0), v.data_ptr(), M, R, K, sp, xv.data_ptr(),
-                                             None if t is None else t.data_ptr(), None if ws is None else ws.data_ptr(), need, _stream())
-        if rc:
-            check(rc, "metis_lowrank_project_rows_ws", (M, R, K))
-        return xv if s is None else (xv, t)
-    ws = torch.empty(_lowrank_workspace_bytes(M, R, K), dtype=torch.uint8, device=x2.device)
-    rc = L.metis_lowrank_project(x2.data_ptr(), x2.stride(0), v.data_ptr(), M, R, K, sp,
-                                 xv.data_ptr(), None if t is None else t.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
-    if rc:
-        check(rc, "metis_lowrank_project", (M, R, K))
-    return xv if s is None else (xv, t)
+        name, need = "metis_lowrank_project_rows_ws", _lowrank_rows_workspace_bytes(M, R, K, x2.device.index or 0)
+    else:
+        name, need = "metis_lowrank_project", _lowrank_workspace_bytes(M, R, K)
+    scratch = _OUT[len(specs)] if need else None
+    new = _lib.call(name, x2.device.index, specs + ((U8, need),) if need else specs,
+                    (x2, x2.stride(0), v, M, R, K, s, "0", tp, scratch, need, _stream()))
+    if new.__class__ is int:
+        check(new, name, (M, R, K))
+    return new[0] if s is None else (new[0], new[1])
 
 
 def quantize_project_applies(x2: torch.Tensor, v: torch.Tensor, mode: int) -> bool:
@@ -1610,19 +1552,13 @@ def quantize_project(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, mode: i
     L = load()
     v = v.contiguous()
     s = s.to(torch.bfloat16).contiguous()
-    xv = torch.empty(M, R, dtype=torch.bfloat16, device=dev)
-    t = torch.empty_like(xv)
-    codes = torch.empty(M, K // 2, dtype=torch.uint8, device=dev)
-    unit = torch.empty(1, dtype=torch.float32, device=dev)
-    parked = torch.empty(_deferred_bytes(M, K), dtype=torch.uint8, device=dev)
-    need = _lowrank_rows_workspace_bytes(M, R, K, dev.index or 0)
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-    rc = L.metis_nvfp4_quant_project_deferred(x2.data_ptr(), M, K, mode, v.data_ptr(), R, s.data_ptr(), xv.data_ptr(), t.data_ptr(),
-                                              codes.data_ptr(), parked.data_ptr(), parked.numel(),
-                                              None if ws is None else ws.data_ptr(), need, _stream())
-    if rc:
-        check(rc, "metis_nvfp4_quant_project_deferred", (M, K, R))
-    return PackedNVFP4(codes, None, unit, M, K, mode, deferred=parked), xv, t
+    size, need = _deferred_bytes(M, K), _lowrank_rows_workspace_bytes(M, R, K, dev.index or 0)
+    specs = ((B16, M, R), (B16, M, R), (U8, M, K // 2), (F32, 1), (U8, size))
+    new = _lib.call("metis_nvfp4_quant_project_deferred", dev.index, specs + ((U8, need),) if need else specs,
+                    (x2, M, K, mode, v, R, s, "0", "1", "2", "4", size, "5" if need else None, need, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_nvfp4_quant_project_deferred", (M, K, R))
+    return PackedNVFP4(new[2], None, new[3], M, K, mode, deferred=new[4]), new[0], new[1]
 
 
 def quantize_project_decode_applies(x2: torch.Tensor, v: torch.Tensor, mode: int) -> bool:
@@ -1645,16 +1581,12 @@ def quantize_project_decode(x2: torch.Tensor, v: torch.Tensor, mode: int = MODE_
     dev = x2.device
     L = load()
     v = v.contiguous()
-    codes = torch.empty(M, K // 2, dtype=torch.uint8, device=dev)
-    unit = torch.empty(1, dtype=torch.float32, device=dev)
-    parked = torch.empty(_deferred_bytes(M, K), dtype=torch.uint8, device=dev)
-    need = _lowrank_workspace_bytes(M, R, K)
-    pending = torch.empty(need, dtype=torch.uint8, device=dev)
-    rc = L.metis_decode_quant_project_deferred(x2.data_ptr(), M, K, mode, codes.data_ptr(), parked.data_ptr(), parked.numel(),
-                                               v.data_ptr(), R, pending.data_ptr(), need, _stream())
-    if rc:
-        check(rc, "metis_decode_quant_project_deferred", (M, K, R))
-    return PackedNVFP4(codes, None, unit, M, K, mode, deferred=parked), pending
+    size, need = _deferred_bytes(M, K), _lowrank_workspace_bytes(M, R, K)
+    new = _lib.call("metis_decode_quant_project_deferred", dev.index, ((U8, M, K // 2), (F32, 1), (U8, size), (U8, need)),
+                    (x2, M, K, mode, "0", "2", size, v, R, "3", need, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_decode_quant_project_deferred", (M, K, R))
+    return PackedNVFP4(new[0], None, new[1], M, K, mode, deferred=new[2]), new[3]
 
 
 def lowrank_contract_tokens(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,
@@ -1713,19 +1645,14 @@ def lowrank_backward(dy: torch.Tensor, t: torch.Tensor, x: torch.Tensor, gxv: to
           and scale_dtype in (torch.float32, torch.bfloat16))
     if not ok:
         return (lowrank_contract_tokens(dy, t), lowrank_contract_tokens(x, gxv, transpose=True), lowrank_scale_grad(gt, xv, out_dtype=scale_dtype))
-    dev = dy.device
-    L = load()
-    gu = torch.empty(N, R, dtype=torch.bfloat16, device=dev)
-    gv = torch.empty(R, K, dtype=torch.bfloat16, device=dev)
-    gs = torch.empty(R, dtype=scale_dtype, device=dev)
-    need = int(L.metis_lowrank_backward_workspace_bytes(L_, N, K, R))
-    ws = torch.empty(need, dtype=torch.uint8, device=dev)
-    rc = L.metis_lowrank_backward(dy.data_ptr(), dy.stride(0), t.data_ptr(), N, x.data_ptr(), x.stride(0), gxv.data_ptr(), K, L_, R,
-                                  gu.data_ptr(), DTYPE_BF16, gv.data_ptr(), DTYPE_BF16, gt.data_ptr(), xv.data_ptr(), gs.data_ptr(),
-                                  DTYPE_F32 if scale_dtype == torch.float32 else DTYPE_BF16, ws.data_ptr(), need, _stream())
-    if rc:
-        check(rc, "metis_lowrank_backward", (L_, N, K, R))
-    return gu, gv, gs
+    need = _lowrank_backward_bytes(L_, N, K, R, dy.device.index or 0)
+    f32 = scale_dtype == torch.float32
+    new = _lib.call("metis_lowrank_backward", dy.device.index, ((B16, N, R), (B16, R, K), (F32 if f32 else B16, R), (U8, need)),
+                    (dy, dy.stride(0), t, N, x, x.stride(0), gxv, K, L_, R, "0", DTYPE_BF16, "1", DTYPE_BF16, gt, xv, "2",
+                     DTYPE_F32 if f32 else DTYPE_BF16, "3", need, _stream()))
+    if new.__class__ is int:
+        check(new, "metis_lowrank_backward", (L_, N, K, R))
+    return new[0], new[1], new[2]
 
 
 def linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.bfloat16,
@@ -1734,11 +1661,11 @@ def linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.b
     return _linear_fwd_grouped(a, members, out_dtype, center, split_k, reference_rounding, a_operand, checked)
 
 
-def _grouped_members(members, M: int, K: int, out_dtype: torch.dtype, dev, decode_layout: bool):
-    """(member array, outputs, tensors to keep until the launch is enqueued) of a grouped call.  decode_layout: cached weights
-    are streamed in that layout (whole lines per load instruction) by the decode-sized kernel."""
-    arr = (_lib.LinearMember * len(members))()
-    outs, keep = [], []
+def _grouped_members(members, M: int, K: int, out_dtype: torch.dtype, decode_layout: bool):
+    """(members, specs of their outputs) of a grouped call as _lib.call takes them.  decode_layout: cached weights are streamed in that
+    layout (whole lines per load instruction) by the decode-sized kernel."""
+    words, specs = [], []
+    kind = F32 if out_dtype == torch.float32 else B16
     for i, (b, t, u, bias) in enumerate(members):
         if b.cols != K:
             raise ValueError(f"contraction mismatch: {K} vs {b.cols}")
@@ -1760,15 +1687,13 @@ def _grouped_members(members, M: int, K: int, out_dtype: torch.dtype, dev, decod
         bias_f32 = bias is not None and bias.dtype == torch.float32
         if bias is not None:
             bias = bias.contiguous() if bias_f32 else bias.to(torch.bfloat16).contiguous()
-        out = torch.empty(M, b.rows, dtype=out_dtype, device=dev)
-        keep += [t, u, bias]
-        outs.append(out)
-        dec = decode_weight(b) if (decode_layout and b.persistent) else None
-        arr[i] = _lib.LinearMember(b.codes.data_ptr(), b.scales.data_ptr(), b.unit.data_ptr(),
-                                   None if t is None else t.data_ptr(), None if u is None else u.data_ptr(), r,
-                                   None if bias is None else bias.data_ptr(), out.data_ptr(), b.rows, int(bias_f32), ldt,
-                                   None if dec is None else dec.data_ptr())
-    return arr, outs, keep
+        words.append((b.codes, b.scales, b.unit, t, u, r, bias, _OUT[i], b.rows, bias_f32, ldt,
+                      decode_weight(b) if (decode_layout and b.persistent) else None))
+        specs.append((kind, M, b.rows))
+    return words, specs
+
+
+_OUT = tuple([chr(ord("0") + i) for i in range(32)])              # the new tensors of a call, by position
 
 
 def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.bfloat16,
@@ -1789,18 +1714,16 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
     where grouped_operand_applies says the call reads ready operands (checked: the caller has just asked it)."""
     M, K = a.rows, a.cols
     dev = a.codes.device
+    if len(members) >= len(_OUT):                              # (beyond four members every one is a launch of its own)
+        rest = (out_dtype, center, split_k, reference_rounding, a_operand)
+        return _linear_fwd_grouped(a, members[:16], *rest) + _linear_fwd_grouped(a, members[16:], *rest)
     if a_operand is not None and split_k and (checked or grouped_operand_applies(a, [m[0] for m in members], [0 if m[1] is None else m[1].shape[1] for m in members],
                                                                      center, reference_rounding)):
         # the usual decode step: every question below has its answer
-        arr, outs, keep = _grouped_members(members, M, K, out_dtype, dev, decode_layout_weights)
+        words, specs = _grouped_members(members, M, K, out_dtype, decode_layout_weights)
         need, _ = _grouped_plan(M, K, tuple([m[0].rows for m in members]), dev.index or 0)
-        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-        rc = load().metis_linear_fwd_grouped_operand(a_operand.data_ptr(), a.__dict__["_unit"].data_ptr(), M, K, ctypes.addressof(arr), len(members),
-                                                     DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, MODE_PB16,
-                                                     None if ws is None else ws.data_ptr(), need, _stream())
-        if rc:
-            check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
-        return outs
+        return _grouped_call("metis_linear_fwd_grouped_operand", dev, words, specs, need,
+                             (a_operand, a.__dict__["_unit"], M, K, words, len(members), DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16, MODE_PB16))
     rounded = (reference_rounding and (center is None or center.dtype == torch.bfloat16) and a.mode == MODE_PB16
                and all(m[0].mode == MODE_PB16 for m in members))
     takes = len(members) <= 4 and all(_decode_kernel_takes(M, m[0].rows, K, 0 if m[1] is None else m[1].shape[1]) for m in members)
@@ -1826,59 +1749,49 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
     if rounded and not takes:
         return [linear_fwd(a, b, t=t, u=u, bias=bias, out_dtype=out_dtype, split_k=split_k, reference_rounding=True)
                 for b, t, u, bias in members]
-    arr, outs, keep = _grouped_members(members, M, K, out_dtype, dev, takes and M < 256 and decode_layout_weights)
-    L = load()
-    ap = ctypes.cast(arr, ctypes.c_void_p)
+    words, specs = _grouped_members(members, M, K, out_dtype, takes and M < 256 and decode_layout_weights)
     # split-K scratch (long K, few columns) and whether a centre fits the launch: functions of the shape alone
-    need, centre_ok = _grouped_plan(M, K, tuple(m[0].rows for m in members), dev.index or 0)
-    if not split_k:
-        need, centre_ok = 0, bool(load().metis_linear_grouped_centered_supported(
-            M, K, ctypes.cast(arr, ctypes.c_void_p), len(members), 0))
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    ns = tuple(m[0].rows for m in members)
+    need, centre_ok = _grouped_plan(M, K, ns, dev.index or 0) if split_k else (0, _grouped_centre_fits_unsplit(M, K, ns))
     dt = DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16
     if rotate is not None:
         op_mode = MODE_PB16 if rounded else MODE_P32          # (nv_operand_mode: what a caller that brings a_operand built it in)
         aop = a_operand if a_operand is not None else decode_operand(a, op_mode, None, rotate=rotate)
-        rc = L.metis_linear_fwd_grouped_operand(aop.data_ptr(), a.unit.data_ptr(), M, K, ap, len(members), dt, op_mode,
-                                                None if ws is None else ws.data_ptr(), need, _stream())
-        if rc:
-            check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
-        return outs
+        return _grouped_call("metis_linear_fwd_grouped_operand", dev, words, specs, need, (aop, a.unit, M, K, words, len(members), dt, op_mode))
     if operand:
         # (a quantizer call that deferred its scale bytes never gets them: the operand kernel forms them on the way)
         aop = a_operand if a_operand is not None else decode_operand(a, MODE_PB16, center)
-        rc = L.metis_linear_fwd_grouped_operand(aop.data_ptr(), a.unit.data_ptr(), M, K, ap, len(members), dt, MODE_PB16,
-                                                None if ws is None else ws.data_ptr(), need, _stream())
-        if rc:
-            check(rc, "metis_linear_fwd_grouped_operand", (M, K, [m[0].rows for m in members]))
-        return outs
+        return _grouped_call("metis_linear_fwd_grouped_operand", dev, words, specs, need, (aop, a.unit, M, K, words, len(members), dt, MODE_PB16))
     # the activation's decode layout (written by its quantizer) in place of the row-major packing: wide runs only
     a_dec = a.decode_layout if (takes and K % 256 == 0 and all(m[0].scales.data_ptr() % 8 == 0 for m in members)) else None
-    a_codes, a_scales = (a_dec.data_ptr(), None) if a_dec is not None else (a.codes.data_ptr(), a.scales.data_ptr())
+    a_codes, a_scales = (a_dec, None) if a_dec is not None else (a.codes, a.scales)
     if center is not None:
         center = center.reshape(-1).to(device=dev, dtype=torch.float32).contiguous()
         if center.numel() != K:
             raise ValueError(f"center must have {K} values, got {center.numel()}")
         aligned = center.data_ptr() % 16 == 0 and all(m[0].scales.data_ptr() % 8 == 0 for m in members) and a.scales.data_ptr() % 8 == 0
         if aligned and centre_ok:
-            rc = L.metis_linear_fwd_grouped_centered(a_codes, a_scales, a.unit.data_ptr(), M, K, ap,
-                                                     len(members), dt, center.data_ptr(),
-                                                     None if ws is None else ws.data_ptr(), need, _stream())
-            if rc:
-                check(rc, "metis_linear_fwd_grouped_centered", (M, K, [m[0].rows for m in members]))
-            return outs
+            return _grouped_call("metis_linear_fwd_grouped_centered", dev, words, specs, need,
+                                 (a_codes, a_scales, a.unit, M, K, words, len(members), dt, center))
         # two passes: W^ center as a binary32 bias per member
         shifted = []
         for b, t, u, bias in members:
             w_mean = matvec(b, center)
             shifted.append((b, t, u, w_mean if bias is None else w_mean + bias.float()))
         return _linear_fwd_grouped(a, shifted, out_dtype)
-    fn = L.metis_linear_fwd_grouped_bf16 if rounded else L.metis_linear_fwd_grouped
-    rc = fn(a_codes, a_scales, a.unit.data_ptr(), M, K, ap, len(members),
-            dt, None if ws is None else ws.data_ptr(), need, _stream())
-    if rc:
-        check(rc, "metis_linear_fwd_grouped_bf16" if rounded else "metis_linear_fwd_grouped", (M, K, [m[0].rows for m in members]))
-    return outs
+    return _grouped_call("metis_linear_fwd_grouped_bf16" if rounded else "metis_linear_fwd_grouped", dev, words, specs, need,
+                         (a_codes, a_scales, a.unit, M, K, words, len(members), dt))
+
+
+def _grouped_call(name: str, dev: torch.device, words: list, specs: list, need: int, args: tuple) -> list[torch.Tensor]:
+    """The launch of a grouped product with its split-K scratch; the members' outputs."""
+    count = len(specs)
+    if need:
+        specs.append((U8, need))
+    new = _lib.call(name, dev.index, tuple(specs), args + (_OUT[count] if need else None, need, _stream()))
+    if new.__class__ is int:
+        check(new, name, (args[2] if "operand" in name else args[3], [w[8] for w in words]))
+    return list(new[:count])
 
 
 def _tiled_backward_pays(M: int, N: int, K: int, device_index: int) -> bool:
@@ -1900,21 +1813,7 @@ def linear_dgrad(dy: PackedNVFP4, wt: PackedNVFP4, out_dtype: torch.dtype = torc
     L, N, K = dy.rows, dy.cols, wt.rows
     if dy.mode == wt.mode and _tiled_backward_pays(L, K, N, dy.codes.device.index or 0):
         return linear_fwd(dy, wt, out_dtype=out_dtype, tiled=True)          # out = deq(dy) . deq(wt)^T: the same product
-    out = torch.empty(L, K, dtype=out_dtype, device=dy.codes.device)
-    dt = DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16
-    ws = _gemm_workspace(L, K, N, out.device)
-    if ws is not None:
-        rc = load().metis_linear_dgrad_ws(dy.codes.data_ptr(), dy.scales.data_ptr(), dy.unit.data_ptr(), wt.codes.data_ptr(),
-                                          wt.scales.data_ptr(), wt.unit.data_ptr(), L, N, K, out.data_ptr(), dt,
-                                          ws.data_ptr(), ws.numel(), _stream())
-        if rc:
-            check(rc, "metis_linear_dgrad_ws", (L, N, K))
-        return out
-    rc = load().metis_linear_dgrad(dy.codes.data_ptr(), dy.scales.data_ptr(), dy.unit.data_ptr(), wt.codes.data_ptr(),
-                                   wt.scales.data_ptr(), wt.unit.data_ptr(), L, N, K, out.data_ptr(), dt, _stream())
-    if rc:
-        check(rc, "metis_linear_dgrad", (L, N, K))
-    return out
+    return _packed_product("dgrad", dy, wt, (L, K, N), (L, N, K), out_dtype)
 
 
 def linear_wgrad(dyt: PackedNVFP4, xt: PackedNVFP4, out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
@@ -1924,19 +1823,23 @@ def linear_wgrad(dyt: PackedNVFP4, xt: PackedNVFP4, out_dtype: torch.dtype = tor
     N, L, K = dyt.rows, dyt.cols, xt.rows
     if dyt.mode == xt.mode and _tiled_backward_pays(N, K, L, dyt.codes.device.index or 0):
         return linear_fwd(dyt, xt, out_dtype=out_dtype, tiled=True)
-    out = torch.empty(N, K, dtype=out_dtype, device=dyt.codes.device)
-    dt = DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16
-    ws = _gemm_workspace(N, K, L, out.device)
-    if ws is not None:
-        rc = load().metis_linear_wgrad_ws(dyt.codes.data_ptr(), dyt.scales.data_ptr(), dyt.unit.data_ptr(),
-                                          xt.codes.data_ptr(), xt.scales.data_ptr(), xt.unit.data_ptr(), L, N, K,
-                                          out.data_ptr(), dt, ws.data_ptr(), ws.numel(), _stream())
-        if rc:
-            check(rc, "metis_linear_wgrad_ws", (L, N, K))
-        return out
-    rc = load().metis_linear_wgrad(dyt.codes.data_ptr(), dyt.scales.data_ptr(), dyt.unit.data_ptr(),
-                                   xt.codes.data_ptr(), xt.scales.data_ptr(), xt.unit.data_ptr(), L, N, K,
-                                   out.data_ptr(), dt, _stream())
-    if rc:
-        check(rc, "metis_linear_wgrad", (L, N, K))
-    return out
+    return _packed_product("wgrad", dyt, xt, (N, K, L), (L, N, K), out_dtype)
+
+
+def _packed_product(which: str, a: PackedNVFP4, b: PackedNVFP4, product: tuple, shape: tuple, out_dtype: torch.dtype) -> torch.Tensor:
+    """metis_linear_dgrad / _wgrad with the split-K scratch of the product [M, N] over K; shape: the entry point's own three sizes."""
+    dev = a.codes.device
+    M, N, K = product
+    need = 0 if (M >= 256 and N < 256) else _linear_workspace_bytes(M, N, K, dev.index or 0)
+    f32 = out_dtype == torch.float32
+    specs = ((F32 if f32 else B16, M, N),)
+    args = (a.codes, a.scales, a.unit, b.codes, b.scales, b.unit, *shape, "0", DTYPE_F32 if f32 else DTYPE_BF16)
+    if need:
+        name = f"metis_linear_{which}_ws"
+        new = _lib.call(name, dev.index, specs + ((U8, need),), args + ("1", need, _stream()))
+    else:
+        name = f"metis_linear_{which}"
+        new = _lib.call(name, dev.index, specs, args + (_stream(),))
+    if new.__class__ is int:
+        check(new, name, shape)
+    return new[0]

@@ -2,6 +2,8 @@
 import os
 import re
 
+import pytest
+
 from metis_hip import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -48,3 +50,24 @@ def test_size_helpers_of_the_one_pass_entry_points_need_no_device():
         assert L.metis_nvfp4_deferred_bytes(rows, cols) == 2048 * 4 + (nb * 2 + 255) // 256 * 256
         assert L.metis_nvfp4_workspace_bytes(rows, cols) >= 16384 + nb * 4
     assert L.metis_nvfp4_deferred_bytes(0, 64) == 0
+
+
+def test_compiled_calls_take_the_arguments_that_the_abi_declares():
+    """_lib.call reaches its entry points through their declarations in metis_hip.h; what Python passes is counted and its kinds looked at before
+    anything is allocated on a device or launched.  (No call of this test gets that far.)"""
+    with pytest.raises(KeyError):
+        _lib.call("metis_no_such_entry", 0, (), ())
+    source = open(os.path.join(os.path.dirname(_lib.LIB_PATH), "..", "csrc", "host_calls.cpp")).read()
+    names = re.findall(r"METIS_ENTRY\((metis_\w+)\)", source)
+    assert len(names) > 30 and len(set(names)) == len(names)
+    for name in names:
+        args = _lib.SIGNATURES[name][1]
+        for n in (len(args) - 1, len(args) + 1):
+            with pytest.raises(TypeError, match=rf"{name} takes {len(args)} arguments"):
+                _lib.call(name, 0, (), (0,) * n)
+        with pytest.raises(TypeError):
+            _lib.call(name, 0, (), (0.5,) * len(args))              # a float for a pointer
+        with pytest.raises(TypeError):
+            _lib.call(name, 0, (), (0,) * (len(args) - 1) + ("0",))  # a new tensor that is not there
+    with pytest.raises(ValueError):
+        _lib.call("metis_rmsnorm", 0, ((7, 1),), (0,) * 7)
