@@ -138,10 +138,6 @@ struct SkinnyGroup {
     int a_decode;                // the activation comes in the decode layout too (a_codes points at it, a_scales unused)
 };
 
-// decode-sized calls of many column tiles on ready operands (metis_gemm_decode.hip)
-int decode_wide_tiles(int64_t M, int64_t tiles);
-int launch_decode_wide(const void* a_ops, int64_t M, int64_t K, const SkinnyGroup& grp, int tiles, int per_wg, int out_dtype, hipStream_t st);
-
 constexpr int L_BM = 256, L_BN = 256, L_STRIDE = BK + LDS_PAD;   // large-tile kernels: 256 x 256 per workgroup
 
 // MFMA : VALU : LDS interleave requested from the scheduler for one K=16 sub-step of N_MFMA MFMAs

@@ -797,21 +797,10 @@ __device__ __forceinline__ void skinny_tile(
         const int l = id & 63, g = (id >> 6) & 3, i = min(id >> 8, TM - 1);
         const int m = m0 + i * 32 + (l & 31), n = n0 + 8 * g + 4 * (l >> 5);
         float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        // (bf16 arithmetic: the two halves of K are summed apart, as gemm_decode_wide_kernel's two waves per tile have them)
-        constexpr int FIRST = PB16 != 0 && WAVES == 8 ? 4 : WAVES;
 #pragma unroll
-        for (int w = 0; w < FIRST; ++w)
+        for (int w = 0; w < WAVES; ++w)
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += red[w][i * 16 + 4 * g + e][l];
-        if constexpr (FIRST < WAVES) {
-            float v2[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int w = FIRST; w < WAVES; ++w)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v2[e] += red[w][i * 16 + 4 * g + e][l];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += v2[e];
-        }
         const bool live = id < TM * 256 && m < M && n < N;     // N % 4 == 0 is required
         if constexpr (PB16 != 0) {
             if (!part) {
@@ -1531,14 +1520,6 @@ int gemm_nvfp4_grouped(const void* a_codes, const void* a_scales, const float* a
                                 (const uint16_t*)g.u, (const uint16_t*)g.bias, g.out, nsplit > 1 ? part : nullptr, (int)g.N,
                                 (int)g.r, end, g.bias_is_f32 != 0, (int)(g.ldt ? g.ldt : g.r), dec ? 1 : 0};
         part += slots * (size_t)M * (size_t)g.N;
-    }
-    // bf16 arithmetic, many column tiles on ready operands, weights in the decode layout: a workgroup per compute unit (metis_gemm_decode.hip).
-    // (Low-rank terms of more than 256 columns are summed in another order here.)
-    if (a_dense && pb16 && nsplit == 1) {
-        bool wide = true;
-        for (int i = 0; i < count; ++i) wide = wide && grp.m[i].decode && grp.m[i].r <= 256;
-        const int per_wg = wide ? decode_wide_tiles(M, tiles) : 0;
-        if (per_wg > 0) return launch_decode_wide(a_codes, M, K, grp, (int)tiles, per_wg, out_dtype, st);
     }
 #define METIS_SKG(TM, C, W) return launch_skinny_grouped<TM, C, W>(a_codes, a_scales, a_unit, M, K, grp, (int)tiles, out_dtype, st, pb16, a_dense)
     if (tm == 1) {

@@ -470,35 +470,6 @@ def test_cached_weights_in_the_decode_layout_give_the_same_bits(M, K, Ns, r):
             assert int(got_c.sum()) == 0 and int(got_s.sum()) == 0
 
 
-@pytest.mark.parametrize("M,K,Ns,ranks", [(33, 256, (24580,), (32,)), (64, 512, (20004, 8196, 4), (64, 0, 32)), (65, 768, (16420, 16412), (96, 256)),
-                                          (255, 1792, (40960,), (0,)), (64, 3584, (18944, 18944), (64, 64)), (128, 2304, (26000, 4100), (32, 64))])
-def test_many_column_tiles_at_decode_size_have_the_bits_of_the_streaming_kernel(M, K, Ns, ranks):
-    """More than three and up to five column tiles per compute unit, more than 32 rows, bf16 arithmetic, weights in the decode layout: the activation
-    goes through LDS once per workgroup.  Sums are added in the order of the kernel that row-major weights take, so the bits are the
-    same: one to five tiles in the last workgroup, a workgroup with tiles of two and three matrices, ragged M and N, halves of K of different
-    length, low-rank terms absent, staged and beyond the staged columns, either output type."""
-    from metis_hip import ops
-    g = torch.Generator(device="cuda").manual_seed(M + K)
-    px = ops.quantize(synthetic_activation(460 + M, M, K).cuda(), 1)
-    plain, cached = [], []
-    for i, (N, r) in enumerate(zip(Ns, ranks)):
-        w = (torch.randn(N, K, generator=g, device="cuda") * 0.02).bfloat16()
-        pw, pc = ops.quantize(w, 1), ops.quantize(w, 1)
-        pw.decode_layout = pc.decode_layout = None
-        pc.persistent = True
-        t = torch.randn(M, r, generator=g, device="cuda").bfloat16() if r else None
-        u = (torch.randn(N, r, generator=g, device="cuda") * 0.1).bfloat16() if r else None
-        bias = (torch.randn(N, generator=g, device="cuda") * 0.1) if i != 1 else None
-        bias = bias.bfloat16() if bias is not None and i == 0 else bias
-        plain.append((pw, t, u, bias))
-        cached.append((pc, t, u, bias))
-    for dt in (torch.bfloat16, torch.float32):
-        want = ops.linear_fwd_grouped(px, plain, out_dtype=dt, reference_rounding=True)
-        got = ops.linear_fwd_grouped(px, cached, out_dtype=dt, reference_rounding=True)
-        for a, b in zip(got, want):
-            assert torch.equal(a, b)
-
-
 @pytest.mark.parametrize("M,K,Ns,r", [(64, 18944, (3584,), 64), (1, 8192, (256,), 0), (200, 16384, (132, 64), 32),
                                       (33, 8256, (96,), 32)])
 def test_decode_sized_products_with_a_long_contraction_split_k(M, K, Ns, r):
