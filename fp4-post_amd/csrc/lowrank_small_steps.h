@@ -9,10 +9,7 @@ namespace metis {
 
 typedef __bf16 lr_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float lr_float4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ lr_float4_t lr_mfma(uint4 a, uint4 b, lr_float4_t c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lr_bf16x8_t, a), __builtin_bit_cast(lr_bf16x8_t, b), c, 0, 0, 0);
-}
+typedef float lr_float16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kLrMaxChunks = 128;
 constexpr int kLrGroup = kLrMaxChunks / 4;     // chunks per thread of the finishing step
@@ -26,9 +23,6 @@ inline int lowrank_small_chunks(int64_t K, int* kc_out)
     return (int)((K + kc - 1) / kc);
 }
 
-// Both steps multiply on v_mfma_f32_16x16x32_bf16: lane l holds row l % 16 of either operand, elements 8 (l / 16) .. of 32; four sums of a lane are
-// consecutive columns r of one row of x.  A chunk's sum is one chain over its elements, 32 at a time, wherever it is formed.
-
 // One workgroup of the first step: K chunk `chunk` (kc elements), rows 64 mtile .. ; wave w owns columns 32 w .. of R
 // (waves past R / 32 have nothing to do), so the launch needs at least 2 R threads per workgroup, or several workgroups for a chunk,
 // the first wave of each (wave0) further on in R.
@@ -36,45 +30,47 @@ __device__ __forceinline__ void lowrank_small_partial_block(int chunk, int mtile
                                                             const uint16_t* __restrict__ v, int M, int R, int K, int kc,
                                                             float* __restrict__ ws, int wave0 = 0)
 {
-    const int lane = threadIdx.x & 63, wave = wave0 + (int)(threadIdx.x >> 6), l16 = lane & 15, kg = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = wave0 + (int)(threadIdx.x >> 6), hi = lane >> 5;
     if (wave * 32 >= R) return;
     const int m0 = mtile * 64;
     const int k0 = chunk * kc, k1 = min(k0 + kc, K);
-    const uint16_t *vp[2], *xp[4];
+    const uint16_t* vp = v + (int64_t)min(wave * 32 + (lane & 31), R - 1) * K + hi * 32;
+    const uint16_t* xp[2];
 #pragma unroll
-    for (int a = 0; a < 2; ++a) vp[a] = v + (int64_t)min(wave * 32 + a * 16 + l16, R - 1) * K + kg * 8;
+    for (int i = 0; i < 2; ++i) xp[i] = x + (int64_t)min(m0 + i * 32 + (lane & 31), M - 1) * ldx + hi * 32;
+    lr_float16_t acc[2];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) xp[b] = x + (int64_t)min(m0 + b * 16 + l16, M - 1) * ldx + kg * 8;
-    lr_float4_t acc[2][4];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = (lr_float4_t)(0.0f);
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
     for (int k = k0; k < k1; k += 64) {                        // kc % 64 == 0 and K % 64 == 0
-        uint4 rv[2][2], rx[4][2];
+        uint4 rv[4], rx[2][4];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
+        for (int q = 0; q < 4; ++q) rv[q] = reinterpret_cast<const uint4*>(vp + k)[q];
 #pragma unroll
-            for (int a = 0; a < 2; ++a) rv[a][q] = *reinterpret_cast<const uint4*>(vp[a] + k + 32 * q);
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int b = 0; b < 4; ++b) rx[b][q] = *reinterpret_cast<const uint4*>(xp[b] + k + 32 * q);
+            for (int q = 0; q < 4; ++q) rx[i][q] = reinterpret_cast<const uint4*>(xp[i] + k)[q];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const lr_bf16x8_t fv = __builtin_bit_cast(lr_bf16x8_t, rv[q]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv, __builtin_bit_cast(lr_bf16x8_t, rx[i][q]), acc[i], 0, 0, 0);
         }
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = lr_mfma(rv[a][q], rx[b][q], acc[a][b]);
     }
+    // acc[i][e] of lane l: row m = m0 + 32 i + l % 32, column r = 32 wave + 8 (e / 4) + 4 (l / 32) + e % 4
     float* wp = ws + (size_t)chunk * M * R;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const int m = m0 + b * 16 + l16;
+    for (int i = 0; i < 2; ++i) {
+        const int m = m0 + i * 32 + (lane & 31);
         if (m >= M) continue;
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int r = wave * 32 + a * 16 + 4 * kg;
-            if (r < R) *reinterpret_cast<lr_float4_t*>(wp + (size_t)m * R + r) = acc[a][b];     // R % 4 == 0
+        for (int g = 0; g < 4; ++g) {
+            const int r = wave * 32 + 8 * g + 4 * hi;
+            if (r < R)                                          // R % 4 == 0
+                *reinterpret_cast<float4*>(wp + (size_t)m * R + r) =
+                    make_float4(acc[i][4 * g], acc[i][4 * g + 1], acc[i][4 * g + 2], acc[i][4 * g + 3]);
         }
     }
 }
@@ -94,22 +90,31 @@ __device__ __forceinline__ void lowrank_small_store(const float (&a)[4], int id,
     }
 }
 
-// Both steps of 16 rows x 16 columns in one block of 1024 threads, for a launch with other work that waits for nothing of the projection; K <= 4096.
+// Both steps of 16 rows x 16 columns in one block of 1024 threads, for a launch with other work that waits for nothing of the projection; K <= 3072.
 // Waves 4 g .. 4 g + 3 share the chunks of group g of the finishing step, a quarter each, requested together; the first of them adds the chunk sums of
-// all four in chunk order, so the bits are those of the two steps.  Every thread of the block has to call it (two barriers inside).
-// Blocks: lowrank_small_project_blocks(M, R).
-constexpr int kLrProjectThreads = 1024, kLrProjectK = 4096;
+// all four in chunk order.  A chunk is the four products of the first step on 32 x 32 tiles with 16 rows of either operand in lanes 0 .. 15 and
+// 32 .. 47, so the bits are those of the two steps; the other lanes load half of those rows' elements and hand them over (v_permlane16_swap): their own
+// rows of the product are nobody's.  Every thread of the block has to call it (two barriers inside).  Blocks: lowrank_small_project_blocks(M, R).
+// what lanes 16 .. 31 and 48 .. 63 hold, in lanes 0 .. 15 and 32 .. 47
+__device__ __forceinline__ uint4 lr_from_odd_rows(uint4 a)
+{
+    return make_uint4(__builtin_amdgcn_permlane16_swap(a.x, a.x, false, false)[1], __builtin_amdgcn_permlane16_swap(a.y, a.y, false, false)[1],
+                      __builtin_amdgcn_permlane16_swap(a.z, a.z, false, false)[1], __builtin_amdgcn_permlane16_swap(a.w, a.w, false, false)[1]);
+}
+constexpr int kLrProjectThreads = 1024, kLrProjectK = 3072;
 __device__ __forceinline__ void lowrank_small_project_block(int block, const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v, int M,
                                                             int R, int K, const uint16_t* __restrict__ s, uint16_t* __restrict__ xv,
                                                             uint16_t* __restrict__ t)
 {
     constexpr int MINE = kLrProjectK / 64 / 16;                // chunks of a wave
-    __shared__ lr_float4_t sums[4][3][MINE][64], group[3][64];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, kg = lane >> 4;
+    __shared__ lr_float4_t sums[4][3][MINE][2][32], group[3][2][32];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l16 = lane & 15, hi = lane >> 5;
+    const bool keeps = (lane & 16) == 0;
+    const int slot = hi * 16 + l16;
     const int g = wave >> 2, w = wave & 3;
     const int r0 = block % (R / 16) * 16, m = block / (R / 16) * 16 + l16;
-    const uint16_t* vp = v + (int64_t)(r0 + l16) * K + kg * 8;
-    const uint16_t* xp = x + (int64_t)min(m, M - 1) * ldx + kg * 8;
+    const uint16_t* vp = v + (int64_t)(r0 + l16) * K + hi * 32 + (lane & 16);      // 32 bytes of a lane: pieces q = 0, 1 of the half chunk, or 2, 3
+    const uint16_t* xp = x + (int64_t)min(m, M - 1) * ldx + hi * 32 + (lane & 16);
     const int chunks = K / 64, per = (chunks + 3) / 4, own = (per + 3) / 4;
     const int c0 = g * per + w * own, c1 = min(min(c0 + own, (g + 1) * per), chunks);
     uint4 rv[MINE][2], rx[MINE][2];
@@ -118,33 +123,54 @@ __device__ __forceinline__ void lowrank_small_project_block(int block, const uin
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const bool live = c0 + i < c1;
-            rv[i][q] = live ? *reinterpret_cast<const uint4*>(vp + (c0 + i) * 64 + 32 * q) : make_uint4(0u, 0u, 0u, 0u);
-            rx[i][q] = live ? *reinterpret_cast<const uint4*>(xp + (c0 + i) * 64 + 32 * q) : make_uint4(0u, 0u, 0u, 0u);
+            rv[i][q] = live ? *reinterpret_cast<const uint4*>(vp + (c0 + i) * 64 + 8 * q) : make_uint4(0u, 0u, 0u, 0u);
+            rx[i][q] = live ? *reinterpret_cast<const uint4*>(xp + (c0 + i) * 64 + 8 * q) : make_uint4(0u, 0u, 0u, 0u);
         }
-    lr_float4_t total = (lr_float4_t)(0.0f);                   // (a chunk past the end adds zeros)
+    // sums e of a lane: row m, columns r0 + 8 (e / 4) + 4 hi + e % 4, e < 8
+    lr_float4_t total[2] = {(lr_float4_t)(0.0f), (lr_float4_t)(0.0f)};
+    lr_float16_t acc[MINE];
 #pragma unroll
-    for (int i = 0; i < MINE; ++i) {
-        lr_float4_t acc = (lr_float4_t)(0.0f);
+    for (int i = 0; i < MINE; ++i)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) acc = lr_mfma(rv[i][q], rx[i][q], acc);
-        if (w > 0) sums[g][w - 1][i][lane] = acc;
-        else total += acc;
-    }
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < MINE; ++i) {
+            const uint4 a = q < 2 ? rv[i][q] : lr_from_odd_rows(rv[i][q & 1]), b = q < 2 ? rx[i][q] : lr_from_odd_rows(rx[i][q & 1]);
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lr_bf16x8_t, a), __builtin_bit_cast(lr_bf16x8_t, b), acc[i], 0, 0, 0);
+        }
+#pragma unroll
+    for (int i = 0; i < MINE; ++i)                             // (a chunk past the end adds zeros)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const lr_float4_t a = {acc[i][4 * k], acc[i][4 * k + 1], acc[i][4 * k + 2], acc[i][4 * k + 3]};
+            if (w == 0) total[k] += a;
+            else if (keeps) sums[g][w - 1][i][k][slot] = a;
+        }
     __syncthreads();
     if (w == 0) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
+        for (int p = 0; p < 3; ++p)
 #pragma unroll
-            for (int i = 0; i < MINE; ++i) total += sums[g][k][i][lane];
-        if (g > 0) group[g - 1][lane] = total;
+            for (int i = 0; i < MINE; ++i)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) total[k] += sums[g][p][i][k][slot];
+        if (g > 0 && keeps) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) group[g - 1][k][slot] = total[k];
+        }
     }
     __syncthreads();
-    if (wave > 0 || m >= M) return;
+    if (wave > 0 || !keeps || m >= M) return;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) total += group[i][lane];
-    const float a[4] = {total[0], total[1], total[2], total[3]};
-    const int r = r0 + 4 * kg;
-    lowrank_small_store(a, m * R + r, r, s, xv, t);
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) total[k] += group[i][k][slot];
+        const float a[4] = {total[k][0], total[k][1], total[k][2], total[k][3]};
+        const int r = r0 + 8 * k + 4 * hi;
+        lowrank_small_store(a, m * R + r, r, s, xv, t);
+    }
 }
 inline int lowrank_small_project_blocks(int64_t M, int64_t R) { return (int)((M + 15) / 16 * (R / 16)); }
 

@@ -1192,10 +1192,10 @@ int skinny_operand_rht(const void* codes, const void* scales, float* unit, const
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 
-// Whether the launch that builds the operands forms the whole projection: a block of 16 x 16 results reads 64 K bytes of x and V (1.7 us per 1024 of
-// K), while partial sums of K chunks cost a launch and M R binary32 values per chunk.  Microseconds, two launches | one: 64 x 1536, R = 192 8.6 | 5.5,
-// R = 64 6.6 | 5.4; 64 x 2560, R = 64 6.8 | 7.2, R = 128 7.9 | 7.1; 64 x 3584, R = 128 8.1 | 8.8, R = 192 9.5 | 8.9; 192 x 2048, R = 192 10.2 | 6.5.
-static bool project_whole(int64_t R, int64_t K) { return K <= kLrProjectK && K <= 1536 + 12 * R; }
+// Whether the launch that builds the operands forms the whole projection: a block of 16 x 16 results reads 64 K bytes of x and V (1.6 us per 1024 of
+// K), while partial sums of K chunks cost a launch and M R binary32 values per chunk.  Microseconds, two launches | one: 64 x 1536, R = 192 8.6 | 6.3,
+// R = 64 6.6 | 6.3; 64 x 2048, R = 64 6.7 | 7.2, R = 128 7.7 | 7.2; 64 x 2560, R = 192 8.9 | 8.1; 4 x 3072, R = 192 6.8 | 7.4; 192 x 2048, R = 192 10.2 | 7.4.
+static bool project_whole(int64_t R, int64_t K) { return K <= kLrProjectK && K <= 896 + 10 * R; }
 
 // lowrank_small + skinny_operand_deferred on the same activation (x [M, K] bf16 and its packed form) in one launch, or in two: partial
 // sums of the projection, then one launch that finishes it and builds the operands (project_whole).

@@ -1134,7 +1134,7 @@ def test_projection_finish_and_operand_build_in_one_launch(M, K, R, mode, centre
         ops.project_and_operand(x, v, s, p1, mode, centre)
 
 
-@pytest.mark.parametrize("M,K,R", [(1, 256, 32), (16, 768, 64), (17, 1792, 32), (65, 2304, 64), (255, 2048, 160), (31, 3840, 192), (64, 4096, 256), (48, 4096, 224)])
+@pytest.mark.parametrize("M,K,R", [(1, 256, 32), (16, 768, 64), (17, 1792, 96), (65, 1536, 64), (255, 2048, 160), (31, 2816, 192), (64, 3072, 256), (48, 4096, 224)])
 def test_projection_formed_whole_beside_the_operand_build_has_the_bits_of_its_two_steps(M, K, R):
     """Short contractions: one launch forms the projection and builds the operands.  Chunks that do not divide evenly among groups and waves, ragged
     row tiles, either side of the line where the two steps take over; the projection is also one bf16 rounding of the double precision sum."""
