@@ -13,9 +13,10 @@
 // registers two steps ahead, with two barriers per step and the encoder between them, the loads in flight per compute unit were
 // what its registers held: 16384 x 3584, R = 64 25.7 -> 23.4 us, 8192 x 4096 22.2 -> 15.9; with the quantizer 40.9 -> 32.4 and
 // 27.9 -> 26.4, 4096 x 8960 31.2 -> 26.6.  The read of x alone at 5 TB/s: 23.5 and 13.4 from HBM; with codes and maxima written 30.8
-// and 17.6.  Bound by memory, with the quantizer by the encoder's vector work.  64 rows per workgroup read v half as often --
-// 16384 x 3584, R = 192 41 us in place of 48, the quantizing pass of 16384 x 18944 203 in place of 245 -- but their two row tiles
-// have to start at the same step of K: another order of the sums.)
+// and 17.6.)  Bound by memory; with a wide V by what a compute unit takes in, about 46 bytes a nanosecond, of which x is one part in
+// 1 + R / 32.  Where several workgroups would share a compute unit, one therefore owns two row tiles and fetches v once for both:
+// 16384 x 18944, R = 64, with the quantizer 248 -> 205 us, 16384 x 3584, R = 192 53 -> 48.5, from flushed caches 89 -> 74.  The order
+// of an element's sums depends on its row tile, so the two are chosen among those that start at the same step of K (nt_pair).
 //
 // lowrank_tn: the contraction runs down the rows of both operands, so each has to be turned: a workgroup owns 64
 // columns of a and one slice of the tokens; a step of 64 tokens is loaded row by row (coalesced) and staged in LDS as it
@@ -30,20 +31,20 @@
 
 namespace metis {
 
-constexpr int NT_ROWS = 32;                      // rows of x per workgroup
-// A form of the kernel: KS k per stage, NS stages in the ring; one thread per block of 16 of x.
-template <int RT, int KS, int NS> struct NtForm {
-    static constexpr int kThreads = NT_ROWS * KS / 16, kWaves = kThreads / 64;
+constexpr int NT_ROWS = 32;                      // rows of a row tile of x
+// A form of the kernel: TILES row tiles per workgroup, KS k per stage, NS stages in the ring; one thread per block of 16 of x.
+template <int TILES, int RT, int KS, int NS> struct NtForm {
+    static constexpr int kRows = TILES * NT_ROWS, kThreads = kRows * KS / 16, kWaves = kThreads / 64;
     static constexpr int kRowBytes = KS * 2, kRowsPerPiece = 1024 / kRowBytes, kChunks = kRowBytes / 16;
-    static constexpr int kStage = (NT_ROWS + RT * 32) * kRowBytes;            // bytes of a stage: x rows, then v rows
-    static constexpr int kLoads = kStage / 1024 / kWaves, kXLoads = NT_ROWS / kRowsPerPiece / kWaves;   // 1 KiB loads per wave and stage; those of x
+    static constexpr int kStage = (kRows + RT * 32) * kRowBytes;              // bytes of a stage: x rows, then v rows
+    static constexpr int kLoads = kStage / 1024 / kWaves, kXLoads = kRows / kRowsPerPiece / kWaves;   // 1 KiB loads per wave and stage; those of x
     // K is walked in steps of 256, whose quarters of 64 have sums of their own: the waves share the quarters of a stage and the
     // column tiles; a step is kStages stages, with a set of sums for each.
     static constexpr int kQuarters = KS / 64, kStages = 4 / kQuarters;
-    static constexpr int kColGroups = kWaves / kQuarters, kColTiles = (RT + kColGroups - 1) / kColGroups;
-    static constexpr int kRed = kStages * (kQuarters - 1) * RT * 4096 + 64;   // partial sums of the waves, then their maxima
+    static constexpr int kColGroups = kWaves / kQuarters / TILES, kColTiles = (RT + kColGroups - 1) / kColGroups;
+    static constexpr int kRed = kStages * (kQuarters - 1) * TILES * RT * 4096 + 64;   // partial sums of the waves, then their maxima
     static constexpr int kLds = NS * kStage > kRed ? NS * kStage : kRed;
-    static_assert((KS == 64 || KS == 128) && kColGroups * kQuarters == kWaves && kStage % (1024 * kWaves) == 0 && kXLoads >= 1,
+    static_assert((KS == 64 || KS == 128) && kColGroups * kQuarters * TILES == kWaves && kStage % (1024 * kWaves) == 0 && kXLoads >= 1,
                   "every wave loads whole pieces and multiplies a quarter");
 };
 // The factors of up to four projections of the same x, their columns side by side in xv and t: a group's members hand in
@@ -75,6 +76,40 @@ __device__ __forceinline__ const uint16_t* nt_v(const NtFactors& f, int col, int
     const int i = nt_member(f, col);
     return nt_pick(f.v, i) + (col - (i == 0 ? 0 : i == 1 ? f.end[0] : i == 2 ? f.end[1] : f.end[2])) * K;
 }
+// The step of its K range that row tile b starts at, of `steps`.
+constexpr int NT_ROTATE = 5;
+__device__ __forceinline__ int nt_first_step(int b, int steps) { return (int)((unsigned)b * NT_ROTATE % (unsigned)steps); }
+// The row tiles at the places `at` and `at + 1` of all `tiles`, ordered by the step that they start at; that step of the first, and
+// how many steps later the second starts.  An odd one out is returned twice.
+// Tiles b and b + p start alike, with p = steps or, if 5 divides it, steps / 5; tiles = a p + e: the p classes have a members, the
+// first e of them one more.  Class c = i / 5 (mod p; or i itself) is the i-th in the order; a lane looks at one class.
+__device__ __forceinline__ void nt_pair(int at, int tiles, int steps, int* tile0, int* tile1, int* rot, int* lag)
+{
+    *tile0 = *tile1 = at;
+    if (steps <= 0) { if (at + 1 < tiles) *tile1 = at + 1; return; }
+    const bool fives = steps % NT_ROTATE == 0;
+    const int p = fives ? steps / NT_ROTATE : steps, a = tiles / p, e = tiles % p, lane = threadIdx.x & 63;
+    const int inverse[NT_ROTATE] = {0, 4, 2, 3, 1};             // times p, plus 1: a multiple of 5
+    const unsigned fifth = fives ? 1u : (unsigned)(inverse[p % NT_ROTATE] * p + 1) / NT_ROTATE;
+    int larger = 0, found = 0;
+    for (int i0 = 0; i0 < p && found < 2; i0 += 64) {
+        const int i = i0 + lane, c = (int)((unsigned)i * fifth % (unsigned)p);
+        const unsigned long long more = __ballot(i < p && c < e);
+        const int begin = i * a + larger + __popcll(more & ((1ull << lane) - 1)), end = begin + a + (int)((more >> lane) & 1);
+        larger += __popcll(more);
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const unsigned long long hit = __ballot(i < p && at + w >= begin && at + w < end);
+            if (!hit) continue;
+            const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)hit) - 1);
+            const int t = __builtin_amdgcn_readlane(c, l) + p * (at + w - __builtin_amdgcn_readlane(begin, l));
+            const int r = fives ? (i0 + l) * NT_ROTATE : i0 + l;
+            if (w == 0) { *tile0 = *tile1 = t; *rot = r; }
+            else { *tile1 = t; *lag = r - *rot; }
+            ++found;
+        }
+    }
+}
 // Leaves at most VM of the wave's vector memory operations in flight.  Assembly with a memory clobber: no load or store of
 // the loop may move across it, the counts at its uses rely on that.
 template <int VM> __device__ __forceinline__ void nt_wait()
@@ -93,18 +128,17 @@ template <int VM> __device__ __forceinline__ void nt_wait()
 // steps from the row tile's own first one on, the quarters' sums at the end, in order -- so that a column of v gives the same
 // bits alone and beside any others, with and without the quantizer.
 // TAIL: K % 256 != 0.
-template <int RT, int QMODE, int KS, int NS, bool TAIL>
-__global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
+template <int TILES, int RT, int QMODE, int KS, int NS, bool TAIL>
+__global__ __launch_bounds__(TILES * NT_ROWS * KS / 16) void lowrank_nt_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const NtFactors fac, uint16_t* __restrict__ xv, uint16_t* __restrict__ t, int M, int K, float* __restrict__ part, uint2* __restrict__ codes,
-    uint16_t* __restrict__ q_amax, uint32_t* __restrict__ q_gmax, uint32_t fill_to, int rotate, int R)
+    uint16_t* __restrict__ q_amax, uint32_t* __restrict__ q_gmax, uint32_t fill_to, int R)
 {
-    using F = NtForm<RT, KS, NS>;
+    using F = NtForm<TILES, RT, KS, NS>;
     const int col0 = QMODE < 0 ? (int)blockIdx.z * RT * 32 : 0; // R: all columns; the workgroup's are RT * 32 of them from here on
     constexpr int STAGE = F::kStage, LPW = F::kLoads, XL = F::kXLoads, RPP = F::kRowsPerPiece, RB = F::kRowBytes;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];     // the ring, then the waves' partial sums
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int m0 = blockIdx.x * NT_ROWS;
     // TAIL (K % 64 == 0): the last step is cut.  A stage that begins past the end fetches the step's first again, the lanes of a
     // half that does its other half; the quarters past the end multiply zeros, and the threads of such blocks encode the ones that
     // were fetched once more (the same bytes).
@@ -113,14 +147,25 @@ __global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
     const int steps_all = (K + 255) / 256;
     const int per = (steps_all + (int)gridDim.y - 1) / (int)gridDim.y;
     const int first = (int)blockIdx.y * per, wide_steps = max(0, min(steps_all, first + per) - first);
-    const int steps = wide_steps * NH;                          // stages
     // Every row tile starts at a different step of its K range and wraps around: at any moment the workgroups then read
     // different column stripes of x instead of the same one.  With rows a multiple of 4 KiB long, pieces at the same offset
     // of every row can fall on the same few memory channels.  The binary32 sums of a tile are therefore added in an order
     // that depends on the tile, the same for every call.  (An offset of 5 steps per tile: 8192 x 4096 from flushed caches 31 us,
     // 39 without; other row lengths within 2 %.)
-    const int rot = (rotate && steps > 0) ? (int)((blockIdx.x * (unsigned)rotate) % (unsigned)wide_steps) : 0;
-    auto kof = [&](int st) { int q = st / NH + rot; if (q >= wide_steps) q -= wide_steps; return (first + q) * 256 + st % NH * KS; };
+    // Two row tiles: they share the walk and the pieces of v, and each keeps its own order.  nt_pair picks tiles that start at the
+    // same step or at neighbouring ones; the second then joins `lag` steps after the first and goes on as long after it.
+    int tile0 = (int)blockIdx.x, tile1 = (int)blockIdx.x, rot = 0, lag = 0;
+    if constexpr (TILES == 2) nt_pair(2 * (int)blockIdx.x, (M + NT_ROWS - 1) / NT_ROWS, wide_steps, &tile0, &tile1, &rot, &lag);
+    else rot = wide_steps > 0 ? nt_first_step(tile0, wide_steps) : 0;
+    const int steps = (wide_steps + lag) * NH;                  // stages
+    auto kof = [&](int st) {
+        int q = st / NH + rot;
+        if (q >= wide_steps) q -= wide_steps;
+        if (TILES == 2 && q >= wide_steps) q -= wide_steps;
+        return (first + q) * 256 + st % NH * KS;
+    };
+    // row r of the workgroup's
+    auto row_of = [&](int r) { return TILES == 2 ? (r < NT_ROWS ? tile0 * NT_ROWS : (tile1 - 1) * NT_ROWS) + r : tile0 * NT_ROWS + r; };
     auto fetched = [&](int k0) { return TAIL && k0 >= K ? k0 & ~255 : k0; };   // where the stage at k0 is fetched from
 
     // ---- loads go straight to LDS: piece p = j * waves + wave of a stage is 1 KiB, whole rows of x | v.  The 16-byte chunk c
@@ -134,7 +179,7 @@ __global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
     for (int j = 0; j < LPW; ++j) {
         const int row = ((j < XL ? j : j - XL) * F::kWaves + wave) * RPP + lane / F::kChunks;
         const int chunk = (lane % F::kChunks) ^ swz(row);
-        src[j] = (j < XL ? x + (int64_t)min(m0 + row, M - 1) * ldx : nt_v(fac, col0 + row, K)) + chunk * 8;
+        src[j] = (j < XL ? x + (int64_t)min(row_of(row), M - 1) * ldx : nt_v(fac, col0 + row, K)) + chunk * 8;
         upper |= (uint32_t)(chunk >> 3) << j;
     }
     auto issue = [&](int slot, int st) {
@@ -159,19 +204,22 @@ __global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
             for (int e = 0; e < 16; ++e) acc[h][j][e] = 0.0f;
     // wave: quarter of the stage, column group; lane l of an operand: row l % 32, chunk 2 ks + l / 32 of the quarter.
     // (An odd number of column tiles: the second group's last is its neighbour's again, and not written.)
-    const int qi = wave % F::kQuarters, cg = wave / F::kQuarters;
+    const int rt = TILES == 2 ? wave / (F::kWaves / 2) : 0;     // row tile
+    const int qi = wave % F::kQuarters, cg = wave / F::kQuarters % F::kColGroups;
     const int lr = lane & 31;
     int foff[4], coff[CT];
+    const int xoff = rt * NT_ROWS * RB;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) foff[ks] = lr * RB + (((qi * 8 + ks * 2 + (lane >> 5)) ^ swz(lr)) * 16);
 #pragma unroll
-    for (int j = 0; j < CT; ++j) coff[j] = (NT_ROWS + min(cg * CT + j, RT - 1) * 32) * RB;
-    auto multiply = [&](int slot, int k0, float16_t (&sums)[CT]) {
-        const bool out = TAIL && k0 + qi * 64 >= K;             // a select, not a branch: product and encoder stay interleaved
+    for (int j = 0; j < CT; ++j) coff[j] = (F::kRows + min(cg * CT + j, RT - 1) * 32) * RB;
+    auto multiply = [&](int slot, int step, int k0, float16_t (&sums)[CT]) {
+        // selects, not branches: product and encoder stay interleaved
+        const bool out = (TAIL && k0 + qi * 64 >= K) || (TILES == 2 && (rt ? step < lag : step >= wide_steps));
         const unsigned char* b = lds + slot * STAGE;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            bf16x8_t fa = *reinterpret_cast<const bf16x8_t*>(b + foff[ks]);
+            bf16x8_t fa = *reinterpret_cast<const bf16x8_t*>(b + xoff + foff[ks]);
             if (out) fa = bf16x8_t{};
 #pragma unroll
             for (int j = 0; j < CT; ++j) {
@@ -185,7 +233,7 @@ __global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
     // never skipped, which the counted waits rely on (the same bytes to the same place).
     float gmax = 0.0f;
     const int erow = tid / (KS / 16), eblk = tid % (KS / 16), eswz = swz(erow);
-    const int64_t eib = (int64_t)min(m0 + erow, M - 1) * (K / kBlock);
+    const int64_t eib = (int64_t)min(row_of(erow), M - 1) * (K / kBlock);
     auto encode = [&](int slot, int k0) {
         if constexpr (QMODE >= 0) {
             const unsigned char* b = lds + slot * STAGE + erow * RB;
@@ -221,7 +269,7 @@ __global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
             __syncthreads();
             if (st + NS - 1 < steps) issue(slot == 0 ? NS - 1 : slot - 1, st + NS - 1);
             const int k0 = kof(st);
-            multiply(slot, k0, acc[h]);
+            multiply(slot, step / NH, k0, acc[h]);
             encode(slot, fetched(k0));
             slot = slot + 1 == NS ? 0 : slot + 1;
         }
@@ -234,8 +282,8 @@ __global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
     }
     __syncthreads();                                            // the ring is free
     float* red = reinterpret_cast<float*>(lds);                 // [stage of the step][column tile][e][lane], then the waves' maxima
-    auto red_at = [&](int h, int jt, int e) -> float& { return red[((h * RT + jt) * 16 + e) * 64 + lane]; };
-    constexpr int MAXIMA = F::kStages * (F::kQuarters - 1) * RT * 1024;
+    auto red_at = [&](int h, int jt, int e) -> float& { return red[(((rt * NH + h) * RT + jt) * 16 + e) * 64 + lane]; };
+    constexpr int MAXIMA = F::kStages * (F::kQuarters - 1) * TILES * RT * 1024;
     if constexpr (QMODE >= 0) {
         float* smax = red + MAXIMA;
         const float wm = wave_max(gmax);
@@ -265,8 +313,8 @@ __global__ __launch_bounds__(NT_ROWS * KS / 16) void lowrank_nt_kernel(
         }
         for (uint32_t j = gsize + gid * F::kThreads + tid; j < fill_to; j += gsize * F::kThreads) q_gmax[j] = 0u;
     }
-    const int m = m0 + lr;
-    if (qi > 0 || m >= M) return;
+    const int m = row_of(rt * NT_ROWS + lr);
+    if (qi > 0 || m >= M || (TILES == 2 && rt && tile1 == tile0)) return;
 #pragma unroll
     for (int j = 0; j < CT; ++j) {
         const int jt = cg * CT + j;
@@ -362,15 +410,15 @@ static int nt_column_group(int64_t groups, int64_t R)
     return R % 64 == 0 && groups <= cus ? 64 : (int)R;
 }
 
-template <int RT, int QMODE, int KS, int NS, bool TAIL>
+template <int TILES, int RT, int QMODE, int KS, int NS, bool TAIL>
 static int launch_nt(int slices, hipStream_t st, const void* x, int64_t ldx, const NtFactors& fac, void* xv, void* t, int64_t M, int64_t R, int64_t K,
                      float* part, void* codes, uint16_t* amax, uint32_t* gmax)
 {
-    using F = NtForm<RT, KS, NS>;
+    using F = NtForm<TILES, RT, KS, NS>;
     static bool attr_set[64] = {};
-    if (const int rc = allow_dynamic_lds((const void*)lowrank_nt_kernel<RT, QMODE, KS, NS, TAIL>, F::kLds, attr_set)) return rc;
-    hipLaunchKernelGGL((lowrank_nt_kernel<RT, QMODE, KS, NS, TAIL>), dim3((unsigned)((M + NT_ROWS - 1) / NT_ROWS), (unsigned)slices, (unsigned)(R / (RT * 32))), dim3(F::kThreads), F::kLds, st,
-                       (const uint16_t*)x, ldx, fac, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part, (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, measure_int("METIS_NT_ROT", 5), (int)R);
+    if (const int rc = allow_dynamic_lds((const void*)lowrank_nt_kernel<TILES, RT, QMODE, KS, NS, TAIL>, F::kLds, attr_set)) return rc;
+    hipLaunchKernelGGL((lowrank_nt_kernel<TILES, RT, QMODE, KS, NS, TAIL>), dim3((unsigned)((M + F::kRows - 1) / F::kRows), (unsigned)slices, (unsigned)(R / (RT * 32))), dim3(F::kThreads), F::kLds, st,
+                       (const uint16_t*)x, ldx, fac, (uint16_t*)xv, (uint16_t*)t, (int)M, (int)K, part, (uint2*)codes, amax, gmax, (uint32_t)kDeferredPartials, (int)R);
     return METIS_OK;
 }
 
@@ -432,22 +480,33 @@ int lowrank_nt_grouped(const void* x, int64_t ldx, int64_t M, int64_t K, const L
     // 192 columns on V's share outweighs that (16384 x 18944 433 | 361).
     //   with the quantizer, R = 64, three | two stages of 128 k: 411 x 1536 12.8 | 11.7, 16384 x 3584 33.4 | 31.7; three where a compute
     //   unit has one workgroup and x comes from HBM: 8192 x 14336 91 | 105
-    const int64_t groups = ((M + NT_ROWS - 1) / NT_ROWS) * slices;
+    // Pairs of row tiles (stages of 128 k, three, from 192 columns on two) fetch v half as often.  They pay where single tiles would
+    // share compute units and V's pieces are most of what a unit takes in, or x comes from HBM.  Microseconds, single | pairs, with x in
+    // the memory-side cache and, after the dash, from HBM:
+    //   R = 192  16384 x 3584 52.9 | 48.5 - 88.8 | 74.2, 9000 x 4096 52 | 47 - 79 | 72, 16384 x 18944 - 380 | 327;  8192 x 4096 (256 tiles) 42 | 42
+    //   R = 256  16384 x 3584 65.5 | 58.5 - 106 | 82;   R = 128  16384 x 3584 37.6 | 36.9 - 66 | 59, 16384 x 8960 110 | 86 - 147 | 131
+    //   R = 96   16384 x 3584 35.4 | 37.3 - 61 | 57, 16384 x 8960 100 | 78 - 138 | 126
+    //   R = 64   16384 x 3584 25 | 25 - 53 | 52, 16384 x 6400 41 | 43 - 91 | 90, 12000 x 18944 140 | 114 - 184 | 159;  R = 32  16384 x 6400 35 | 40
+    //   with the quantizer, R = 64: 16384 x 3584 38 | 44 - 68 | 66, 9000 x 14336 145 | 123 - 175 | 150, 16384 x 18944 248 | 205 - 282 | 240
+    const int64_t tiles = (M + NT_ROWS - 1) / NT_ROWS, groups = tiles * slices;
     const bool tail = K % 256 != 0, shared = groups > device_cus() && (R > 128 || M * K <= (int64_t)1 << 27);
-#define METIS_NT(RT, Q, KS, NS) do { if (tail) rc = launch_nt<RT, Q, KS, NS, true>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); \
-                                     else rc = launch_nt<RT, Q, KS, NS, false>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); } while (0)
-#define METIS_NTS(RT, NS, NS64) do { if (shared) METIS_NT(RT, -1, 64, NS64); else METIS_NT(RT, -1, 128, NS); } while (0)
+    const bool pairs = slices == 1 && tiles > device_cus() && (R >= 128 || M * K > 120000000) && K <= 1 << 20;
+#define METIS_NT(T, RT, Q, KS, NS) do { if (tail) rc = launch_nt<T, RT, Q, KS, NS, true>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); \
+                                        else rc = launch_nt<T, RT, Q, KS, NS, false>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); } while (0)
+#define METIS_NTS(RT, NS, NS64) do { if (pairs) METIS_NT(2, RT, -1, 128, NS); else if (shared) METIS_NT(1, RT, -1, 64, NS64); else METIS_NT(1, RT, -1, 128, NS); } while (0)
     const int width = qmode < 0 ? nt_column_group(groups, R) : (int)R;
     const bool deep = groups <= device_cus() && M * K >= 100000000;
-#define METIS_NTQ(RT, Q) do { if (deep) METIS_NT(RT, Q, 128, 3); else METIS_NT(RT, Q, 128, 2); } while (0)
+#define METIS_NTQ(RT, Q) do { if (pairs) METIS_NT(2, RT, Q, 128, 3); else if (deep) METIS_NT(1, RT, Q, 128, 3); else METIS_NT(1, RT, Q, 128, 2); } while (0)
+#define METIS_NTC(RT) do { if (pairs) METIS_NT(2, RT, -1, 128, 3); else METIS_NT(1, RT, -1, 128, 3); } while (0)
     if (qmode == METIS_MODE_P32) { if (R == 32) METIS_NTQ(1, 0); else METIS_NTQ(2, 0); }
     else if (qmode >= 0) { if (R == 32) METIS_NTQ(1, 1); else METIS_NTQ(2, 1); }
-    else if (width == 32) METIS_NT(1, -1, 128, 3);
-    else if (width == 64) METIS_NT(2, -1, 128, 3);
+    else if (width == 32) METIS_NTC(1);
+    else if (width == 64) METIS_NTC(2);
     else if (width == 96) METIS_NTS(3, 3, 4);
     else if (width == 128) METIS_NTS(4, 3, 4);
     else if (width == 192) METIS_NTS(6, 2, 2);
     else METIS_NTS(8, 2, 2);
+#undef METIS_NTC
 #undef METIS_NTS
 #undef METIS_NTQ
 #undef METIS_NT

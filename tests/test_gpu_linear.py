@@ -792,6 +792,39 @@ def test_rank_r_projection_adds_in_its_documented_order(M, K):
             assert torch.equal(ops.quantize_project(xd, v, s, 0)[1], xv)
 
 
+@pytest.mark.parametrize("M,R,K", [(8200, 128, 64), (8200, 192, 320), (8225, 256, 1536), (16384, 128, 1280), (10000, 128, 3648), (8257, 64, 14656), (8224, 32, 14592)])
+def test_pairs_of_row_tiles_add_in_the_documented_order(M, R, K):
+    """Two row tiles per workgroup: more tiles than compute units, an odd number of them, one step, a few, a multiple of five, tiles
+    that start a step apart, K that ends in half a stage.  The products are 1, 2^24 and -2^24 as above, every row tile from its own
+    first step on; other members' columns and codes likewise."""
+    from metis_hip import ops
+    assert (M + 31) // 32 > torch.cuda.get_device_properties(0).multi_processor_count
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    steps = (K + 255) // 256
+    pick = torch.tensor([0.0, 1.0, 1.0, 2.0 ** 24, -2.0 ** 24], device="cuda")[torch.randint(5, (M, steps * 4), generator=g, device="cuda")]
+    pick[:, K // 64:] = 0.0
+    x = torch.zeros(M, K, device="cuda", dtype=torch.bfloat16)
+    at = torch.arange(K // 64, device="cuda") * 64 + torch.randint(64, (K // 64,), generator=g, device="cuda")
+    x[:, at] = pick[:, :K // 64].bfloat16()
+    q, rows, sums = pick.view(M, steps, 4), torch.arange(M, device="cuda"), torch.zeros(M, 4, device="cuda")
+    for i in range(steps):
+        sums = sums + q[rows, (rows // 32 * 5 + i) % steps]
+    want = (((sums[:, 0] + sums[:, 1]) + sums[:, 2]) + sums[:, 3]).bfloat16()[:, None]
+    v, s = torch.ones(R, K, device="cuda").bfloat16(), (torch.rand(R, generator=g, device="cuda") + 0.5).bfloat16()
+    vs, ss = v.split(R // 2 if R > 32 else R), s.split(R // 2 if R > 32 else R)
+    if R > 32 and ops.lowrank_stack_applies(x, list(zip(vs, ss))):
+        xv, t = ops.lowrank_project(x, ops.FactorStack(vs), ops.FactorStack(ss))
+    else:
+        xv, t = ops.lowrank_project(x, v, s)
+    assert torch.equal(xv, want.expand(M, R)) and torch.equal(t, xv * s)
+    if R <= 64:
+        for mode in (0, 1):
+            p, qxv, qt = ops.quantize_project(x, v, s, mode)
+            ref = ops.quantize(x, mode)
+            assert torch.equal(p.codes, ref.codes) and torch.equal(p.scales, ref.scales) and torch.equal(p.unit, ref.unit)
+            assert torch.equal(qxv, xv) and torch.equal(qt, t)
+
+
 @pytest.mark.parametrize("R", [96, 192, 256])
 def test_wide_ranks_take_what_the_library_product_took(R):
     """Ranks 96, 192 and 256 from 256 rows on: an unaligned V, rows that overlap, operands that autograd records and large products
