@@ -51,6 +51,35 @@ __host__ __device__ __forceinline__ int xt_swz(int q) { return ((q >> 2) & 1) | 
 //        block maximum per block instead of E4M3 bytes, `partials` the partial tensor maxima.  The kernel forms the
 //        tensor unit (written to unit_out by the first workgroup) and every scale byte itself, in the arithmetic the
 //        tensor was quantized in (QMODE) -- the expressions of quant_scales_kernel, so the bytes it would have written.
+// Rotating back on the matrix cores: out[c] = sign_c / 16 * sum_k H[c][k] x[k], one 16 x 16 product for many blocks.  The values of
+// a block are small multiples of one number (12 units per scale in exact binary16 codes times E4M3; bf16 values of one scale span less than
+// 17 bits), so their binary32 sums are exact in any order: the bits of sixteen ordered additions.  binary16 operands go in without their
+// 2^-8, which would be subnormal, and take it and the sixteenth from the matrix; bf16 sums are scaled afterwards, so that they overflow where they did.
+typedef float xt_float4_t __attribute__((ext_vector_type(4)));
+template <int PB16> __device__ __forceinline__ uint16_t rotation_entry(int c, int k, uint32_t sign_mask)
+{
+    return (uint16_t)((PB16 ? 0x3f80u : 0x0c00u) | (((uint32_t)__popc(c & k) ^ (sign_mask >> c)) & 1u) << 15);   // 1 in bf16, 2^-12 in binary16
+}
+// Eight codes times their block's scale as operands of that product.
+template <int PB16> __device__ __forceinline__ uint4 rotation_operand(uint32_t c, uint32_t scale_byte, float unit)
+{
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    if constexpr (PB16 != 0) {
+        const float dq = rb(e4m3_value(scale_byte) * unit);
+        const float2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 0), p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 1);
+        const float2_t p2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 2), p3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 3);
+        return make_uint4(rb_pair(p0[0] * dq, p0[1] * dq), rb_pair(p1[0] * dq, p1[1] * dq), rb_pair(p2[0] * dq, p2[1] * dq), rb_pair(p3[0] * dq, p3[1] * dq));
+    } else {
+        const _Float16 h = (_Float16)e4m3_value(scale_byte);
+        return expand8(c, half2_t{h, h});
+    }
+}
+template <int PB16> __device__ __forceinline__ uint32_t rotated_pair(float a, float b)
+{
+    if constexpr (PB16 != 0) return rb_pair(a * 0.0625f, b * 0.0625f);
+    const half2_t h = {(_Float16)a, (_Float16)b};
+    return __builtin_bit_cast(uint32_t, h);
+}
 template <int PB16, int RHT = 0, int DEF = 0, int QMODE = 0, int AHEAD = 8>
 __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restrict__ codes, const uint8_t* __restrict__ scales,
                                                         const float* __restrict__ unit_p, uint4* __restrict__ out, int rows,
@@ -63,7 +92,18 @@ __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restri
     static_assert(DEF == 0 || RHT == 0, "deferred scale bytes: unrotated tensors");
     const int lane = threadIdx.x & 63;
     const int kt = K / 32, kgroups = (kt + 7) / 8;
-    const int q = lane >> 2, chunk = (lane & 3) ^ xt_swz(q);
+    // RHT: lane l of the 32 x 32 x 16 product holds half l / 32 of block l % 32 of the tile, going in and coming out: its rows 0-3 and
+    // 8-11 are the columns of the first half, 4-7 and 12-15 of the second, 16-31 are zero.
+    const int q = RHT ? (lane & 31) >> 1 : lane >> 2, chunk = RHT ? 2 * (lane & 1) + (lane >> 5) : (lane & 3) ^ xt_swz(q);
+    const int place = RHT ? q * 4 + (chunk ^ xt_swz(q)) : lane;
+    uint32_t rotation[4] = {0u, 0u, 0u, 0u};
+    if constexpr (RHT != 0) {
+        const int m = lane & 31, c = (m & 3) | ((m & 8) >> 1) | ((m & 4) << 1);
+        if (m < kBlock) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) rotation[j >> 1] |= (uint32_t)rotation_entry<PB16>(c, 8 * (lane >> 5) + j, sign_mask) << (16 * (j & 1));
+        }
+    }
     const int64_t nunits = (int64_t)row_tiles * kgroups;
     float unit = 0.0f;
     if constexpr (DEF != 0) {
@@ -96,50 +136,21 @@ __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restri
                 }
             }
             uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (live) {                                          // lane pairs (l, l ^ 1) share their row: both live or neither
+            if constexpr (RHT != 0) {
+                const uint4 o = rotation_operand<PB16>(cw[i % AHEAD], sw[i % AHEAD], unit);
+                const uint4 h = make_uint4(rotation[0], rotation[1], rotation[2], rotation[3]);
+                float16_t acc;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+                if constexpr (PB16 != 0) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, h), __builtin_bit_cast(bf16x8_t, o), acc, 0, 0, 0);
+                else acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, h), __builtin_bit_cast(half8_t, o), acc, 0, 0, 0);
+                if (live) v = make_uint4(rotated_pair<PB16>(acc[0], acc[1]), rotated_pair<PB16>(acc[2], acc[3]), rotated_pair<PB16>(acc[4], acc[5]), rotated_pair<PB16>(acc[6], acc[7]));
+            } else if (live) {
                 const uint32_t c = cw[i % AHEAD];
                 uint32_t sb;
                 if constexpr (DEF != 0) sb = scale_byte_of<QMODE>((uint16_t)sw[i % AHEAD], unit);
                 else sb = sw[i % AHEAD];
-                if constexpr (RHT != 0) {
-                    const float dq = PB16 ? rb(e4m3_value(sb) * unit) : e4m3_value(sb) * 0.00390625f;
-                    const float2_t p[4] = {__builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 1),
-                                           __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 2), __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 3)};
-                    float mine[8], blk[kBlock];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) mine[j] = PB16 ? rb(p[j >> 1][j & 1] * dq) : p[j >> 1][j & 1] * dq;
-                    const int half = chunk & 1;                  // which half of the block this lane holds
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        // the neighbouring lane's value through DPP (quad_perm 1,0,3,2): no trip through the LDS crossbar
-                        const float other = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mine[j]), 0xB1, 0xf, 0xf, false));
-                        blk[j] = half ? other : mine[j];
-                        blk[8 + j] = half ? mine[j] : other;
-                    }
-                    // This lane's half of the rotated block alone, n = 8 half + j: H[k][n] = H[k][j] for k < 8 and
-                    // H[k][j] (-1)^half for k >= 8, so the second half of the inputs changes sign with `half` and the sums run
-                    // in the order of hadamard16_inverse (a - b and a + (-b) are the same operation).  No array is indexed
-                    // by a run-time value: such an array would be moved to LDS.
-                    const uint32_t flip = (uint32_t)half << 31;
-#pragma unroll
-                    for (int k = 8; k < kBlock; ++k) blk[k] = __uint_as_float(__float_as_uint(blk[k]) ^ flip);
-                    float o[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        float acc = blk[0];
-#pragma unroll
-                        for (int k = 1; k < kBlock; ++k) acc = (__builtin_popcount(k & j) & 1) ? acc - blk[k] : acc + blk[k];
-                        o[j] = __uint_as_float(__float_as_uint(acc * 0.0625f) ^ (((sign_mask >> (8 * half + j)) & 1u) << 31));
-                    }
-                    if constexpr (PB16 != 0) {
-                        v.x = rb_pair(o[0], o[1]); v.y = rb_pair(o[2], o[3]); v.z = rb_pair(o[4], o[5]); v.w = rb_pair(o[6], o[7]);
-                    } else {
-                        const half2_t h0 = {(_Float16)o[0], (_Float16)o[1]}, h1 = {(_Float16)o[2], (_Float16)o[3]};
-                        const half2_t h2 = {(_Float16)o[4], (_Float16)o[5]}, h3 = {(_Float16)o[6], (_Float16)o[7]};
-                        v.x = __builtin_bit_cast(uint32_t, h0); v.y = __builtin_bit_cast(uint32_t, h1);
-                        v.z = __builtin_bit_cast(uint32_t, h2); v.w = __builtin_bit_cast(uint32_t, h3);
-                    }
-                } else if constexpr (PB16 != 0) {
+                if constexpr (PB16 != 0) {
                     const float dq = rb(e4m3_value(sb) * unit);
                     const float2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 0);
                     const float2_t p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 1);
@@ -160,7 +171,7 @@ __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restri
                     v = expand8(c, scale_pair(sb));
                 }
             }
-            out[((int64_t)rb_ * kt + kb) * 64 + lane] = v;
+            out[((int64_t)rb_ * kt + kb) * 64 + place] = v;
         }
     }
 }
@@ -178,12 +189,11 @@ static bool expand_two_ahead(int64_t units)
 // Transposing variant: the packed [R, C] tensor (blocks along C) becomes the tiled operand [C, R], the layout a GEMM
 // that contracts over R (tokens) reads -- the wgrad operands dY^T and X^T and the dgrad operand W^T of
 // src/Metis/Metis/bitlinear.py:502-510.  An output tile (16 operand rows x 32 k) is one block of 16 from each of 32
-// source rows: lane l % 32 dequantizes (and, RHT, rotates back) one whole block in registers, the wave turns two
+// source rows: lane l % 32 dequantizes one whole block in registers, the wave turns two
 // tiles through LDS and writes them as 2 x 1 KiB of consecutive bytes.  R % 32 == 0.
-template <int PB16, int RHT>
+template <int PB16>
 __global__ __launch_bounds__(256) void expand_xt_t_kernel(const uint2* __restrict__ codes, const uint8_t* __restrict__ scales,
-                                                          const float* __restrict__ unit_p, uint4* __restrict__ out, int R, int C,
-                                                          uint32_t sign_mask)
+                                                          const float* __restrict__ unit_p, uint4* __restrict__ out, int R, int C)
 {
     typedef float float2_t __attribute__((ext_vector_type(2)));
     __shared__ __attribute__((aligned(16))) uint16_t turn[4][2][16][40];       // [wave][tile][operand row][k], 80-byte rows
@@ -210,7 +220,6 @@ __global__ __launch_bounds__(256) void expand_xt_t_kernel(const uint2* __restric
 #pragma unroll
                 for (int j = 0; j < kBlock; ++j) blk[j] = rb(blk[j]);
             }
-            if constexpr (RHT != 0) hadamard16_inverse(blk, sign_mask);
 #pragma unroll
             for (int j = 0; j < kBlock; ++j)
                 turn[wave][half][j][sl] = PB16 ? (uint16_t)bf16_bits(blk[j]) : __builtin_bit_cast(uint16_t, (_Float16)blk[j]);
@@ -227,6 +236,77 @@ __global__ __launch_bounds__(256) void expand_xt_t_kernel(const uint2* __restric
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);
         __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// The same for a rotated tensor (NV recipe).  A 16 x 16 x 16 product rotates 16 blocks, one from each of 16 source rows, and turns
+// them: with the blocks as its rows lane l receives column l % 16 of four of them.  Two products, of the source rows 8 i + (0..3) and
+// 8 i + (4..7), therefore leave a lane eight consecutive k of one operand row, a whole slot of the tile: no trip through LDS.
+// A wave owns 32 source rows and eight blocks of each: lane l loads block l / 16 (and 4 + l / 16) of rows 8 (l / 4 % 4) + l % 4 (+ 4),
+// and the four lanes of a row exchange quarters, so that each holds its quarter of all four blocks.
+// HBM-bound (0.5625 B read, 2 B written per element).  The sixteen-term sums on the vector units had taken 4096 x 8960 34.4 us here and
+// 32.0 in the plain expansion.
+template <int PB16>
+__global__ __launch_bounds__(256) void expand_xt_t_rht_kernel(const uint2* __restrict__ codes, const uint8_t* __restrict__ scales,
+                                                              const float* __restrict__ unit_p, uint4* __restrict__ out, int R, int C, uint32_t sign_mask)
+{
+    typedef short short4_t __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int cb_n = C / 16, kt = R / 32, groups = (cb_n + 7) / 8;
+    const int64_t nunits = (int64_t)groups * kt;
+    const float unit = PB16 ? *unit_p : 0.0f;
+    uint32_t rotation[2] = {0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) rotation[j >> 1] |= (uint32_t)rotation_entry<PB16>(n, 4 * g + j, sign_mask) << (16 * (j & 1));
+    const uint2 h = make_uint2(rotation[0], rotation[1]);
+    const int place = n * 4 + (g ^ xt_swz(n));
+    for (int64_t un = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); un < nunits; un += (int64_t)gridDim.x * 4) {
+        const int kb = (int)(un / groups), cb0 = (int)(un - (int64_t)kb * groups) * 8;   // consecutive waves: consecutive blocks of a row
+        uint2 c[2][2];
+        uint32_t sb[2][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                const int cb = cb0 + 4 * w + g;
+                const int64_t ib = (int64_t)(kb * 32 + 8 * (n >> 2) + 4 * s + (n & 3)) * cb_n + cb;
+                c[s][w] = make_uint2(0u, 0u);
+                sb[s][w] = 0u;
+                if (cb < cb_n) { c[s][w] = codes[ib]; sb[s][w] = scales[ib]; }
+            }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            uint32_t quarter[2][2], byte[2][2];                  // [s][block & 1]: two blocks, b and b + 2
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                // lanes of groups 0, 1 now hold quarters 0, 1 of the blocks g and g + 2, those of 2, 3 quarters 2, 3 of g - 2 and g
+                const auto x = __builtin_amdgcn_permlane32_swap(c[s][w].x, c[s][w].y, false, false);
+                const uint32_t even = __builtin_amdgcn_perm(x[1], x[0], 0x05040100u), odd = __builtin_amdgcn_perm(x[1], x[0], 0x07060302u);
+                const auto y = __builtin_amdgcn_permlane16_swap(even, odd, false, false);
+                quarter[s][0] = y[0];
+                quarter[s][1] = y[1];
+                const auto z = __builtin_amdgcn_permlane32_swap(sb[s][w], sb[s][w], false, false);
+                const auto t = __builtin_amdgcn_permlane16_swap(z[0] | z[1] << 16, z[0] | z[1] << 16, false, false);
+                byte[s][0] = t[0];
+                byte[s][1] = t[1];
+            }
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int cb = cb0 + 4 * w + b;
+                xt_float4_t acc[2];
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const uint4 o = rotation_operand<PB16>(quarter[s][b & 1] >> (16 * (b >> 1)), byte[s][b & 1] >> (16 * (b >> 1)) & 0xffu, unit);
+                    const uint2 a = make_uint2(o.x, o.y);
+                    acc[s] = xt_float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (PB16 != 0) acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4_t, a), __builtin_bit_cast(short4_t, h), acc[s], 0, 0, 0);
+                    else acc[s] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(half4_t, a), __builtin_bit_cast(half4_t, h), acc[s], 0, 0, 0);
+                }
+                if (cb < cb_n)
+                    out[((int64_t)cb * kt + kb) * 64 + place] = make_uint4(rotated_pair<PB16>(acc[0][0], acc[0][1]), rotated_pair<PB16>(acc[0][2], acc[0][3]),
+                                                                           rotated_pair<PB16>(acc[1][0], acc[1][1]), rotated_pair<PB16>(acc[1][2], acc[1][3]));
+            }
+        }
     }
 }
 
@@ -374,14 +454,15 @@ int expand_xt_transposed(const void* codes, const void* scales, const float* uni
     if (rows == 0 || cols == 0) return METIS_OK;
     if (!codes || !scales || !out || ((uintptr_t)codes % 8) || ((uintptr_t)out % 16)) return METIS_E_ARG;
     if (mode == METIS_MODE_PB16 && !unit) return METIS_E_ARG;
-    const int64_t units = (cols / 16) * ((rows / 32 + 1) / 2);
+    const int64_t units = rht ? (cols / 16 + 7) / 8 * (rows / 32) : (cols / 16) * ((rows / 32 + 1) / 2);
     int64_t g = (units + 3) / 4;
     const int64_t cap = (int64_t)device_cus() * 16;
     if (g > cap) g = cap;
-#define METIS_EXT(P, R) hipLaunchKernelGGL((expand_xt_t_kernel<P, R>), dim3((unsigned)g), dim3(256), 0, st, (const uint2*)codes, \
-                                           (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols, sign_mask)
-    if (mode == METIS_MODE_PB16) { if (rht) METIS_EXT(1, 1); else METIS_EXT(1, 0); }
-    else { if (rht) METIS_EXT(0, 1); else METIS_EXT(0, 0); }
+#define METIS_EXT(P) do { if (rht) hipLaunchKernelGGL((expand_xt_t_rht_kernel<P>), dim3((unsigned)g), dim3(256), 0, st, (const uint2*)codes, \
+                                                      (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols, sign_mask); \
+                          else hipLaunchKernelGGL((expand_xt_t_kernel<P>), dim3((unsigned)g), dim3(256), 0, st, (const uint2*)codes, \
+                                                  (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols); } while (0)
+    if (mode == METIS_MODE_PB16) METIS_EXT(1); else METIS_EXT(0);
 #undef METIS_EXT
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import rel_fro, same_bits, synthetic_activation, t
+from helpers import rel_fro, same_bits, synthetic_activation, t, untile
 
 pytestmark = pytest.mark.gpu
 
@@ -155,6 +155,34 @@ def test_tiled_operands_rotate_a_packed_block_back(mode):
     gw2 = ops.gemm_tiled(ops.expand_tiled_transposed(pa, mode=mode), pa.unit, ops.expand_tiled_transposed(pa, mode=mode), pa.unit,
                          K, K, L, mode=mode, out_dtype=torch.float32)
     assert rel_fro(gw2.double().cpu(), (da.T @ da).cpu()) <= tol
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("R,C", [(33, 32), (17, 544), (100, 96), (32, 16), (64, 48), (96, 144), (160, 2064), (416, 1152)])
+def test_operands_of_a_rotated_tensor_bit_for_bit(R, C, mode):
+    """Plain (C % 32 == 0) and transposed (R % 32 == 0) operands of arbitrary codes and scale bytes, with rows and blocks left over in
+    their last tiles: the sums of a block are exact, so every element is the rotated-back value rounded once."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(R * 10000 + C)
+    codes = torch.randint(256, (R, C // 2), generator=g, device="cuda").to(torch.uint8)
+    scales = torch.randint(0x7f, (R, C // 16), generator=g, device="cuda").to(torch.uint8)
+    unit = torch.tensor([0.37], device="cuda")
+    p = ops.PackedNVFP4(codes, scales, unit, R, C, mode)
+    p.rht = _mask()
+    mag = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6], dtype=torch.float64, device="cuda")
+    nib = torch.stack((codes & 15, codes >> 4), -1).reshape(R, C).long()
+    val = mag[nib & 7] * (1 - 2 * (nib >> 3))
+    sc = scales.view(torch.float8_e4m3fn).float().repeat_interleave(16, 1)
+    if mode:
+        x = (val * (sc * unit).bfloat16().double()).bfloat16().double()
+    else:
+        x = val * sc.double() / 256
+    dt = torch.bfloat16 if mode else torch.float16
+    want = _rot(x.cpu(), inverse=True).float().to(dt).cuda()
+    if C % 32 == 0:
+        assert torch.equal(untile(ops.expand_tiled(p, cache=False, mode=mode), R, C, dt), want)
+    if R % 32 == 0:
+        assert torch.equal(untile(ops.expand_tiled_transposed(p, mode=mode), C, R, dt), want.T)
 
 
 @pytest.mark.parametrize("tag", ["p32", "pb16"])
