@@ -273,12 +273,33 @@ __global__ __launch_bounds__(256) void quant_codes_kernel(
 // ---------------------------------------------------------------------------------------------
 constexpr int kColTileBlocks = 16, kColTileCols = 64;
 // a finished tile leaves LDS: thread t takes column t / 4, blocks 4 (t % 4) .. +3: 32 contiguous bytes of codes, 8 of maxima
-template <typename amax_t>
+template <bool QUADS = true, typename amax_t>
 __device__ __forceinline__ void store_col_tile(const uint2 (&s_codes)[kColTileCols][kColTileBlocks + 1], const amax_t (&s_amax)[kColTileCols][kColTileBlocks + 2],
                                                uint2* __restrict__ codes, amax_t* __restrict__ amax, uint32_t tc, uint32_t tr, uint32_t cols, uint32_t nbc)
 {
+    // A full tile of a packing with whole quads of blocks per column: a column's sixteen blocks are 128 consecutive bytes of codes, two per
+    // lane, and their maxima go four to a lane.  Block by block (eight stores of 8 and 2 bytes a thread, each touching a quarter of its
+    // lines) every column kernel waited for its stores.  Both launches, bf16 arithmetic: 18944 x 3584 58.1 -> 51.8 us, 4096 x 14336
+    // 50.3 -> 43.6; stochastic 4096 x 8960 34.6 -> 30.6; both packings of 4096 x 8960 45.2 -> 40.5, of 2112 x 18944 59.6 -> 51.2.
+    // (QUADS: without it both packings of a binary32 tensor, which have no register left for it.)
+    typedef uint32_t quad_t __attribute__((ext_vector_type(4), aligned(8)));
     const uint32_t oc = threadIdx.x >> 2, part = threadIdx.x & 3u;
     const uint32_t c2 = tc * kColTileCols + oc, b0 = tr * kColTileBlocks + part * 4u;
+    if (QUADS && nbc % 4u == 0u && (tr + 1u) * kColTileBlocks <= nbc) {             // (the same for the workgroup)
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i) {
+            const uint32_t cl = i * 32u + (threadIdx.x >> 3), pair = (threadIdx.x & 7u) * 2u, c3 = tc * kColTileCols + cl;
+            const uint2 lo = s_codes[cl][pair], hi = s_codes[cl][pair + 1u];
+            if (c3 < cols) *reinterpret_cast<quad_t*>(codes + (int64_t)c3 * nbc + tr * kColTileBlocks + pair) = (quad_t){lo.x, lo.y, hi.x, hi.y};
+        }
+        if (c2 < cols) {
+            struct __attribute__((aligned(4 * sizeof(amax_t)))) four_t { amax_t a[4]; } f;
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i) f.a[i] = s_amax[oc][part * 4u + i];
+            *reinterpret_cast<four_t*>(amax + (int64_t)c2 * nbc + b0) = f;
+        }
+        return;
+    }
     if (c2 >= cols) return;
 #pragma unroll
     for (uint32_t i = 0; i < 4u; ++i) {
@@ -379,11 +400,36 @@ __global__ __launch_bounds__(256) void quant_codes_col_kernel(
     publish_group_max(gmax, ws_gmax);
 }
 
+// Column `lane` of a 16 x 64 slab of bf16 values in LDS (rows of `words` words), as binary32 values: four transposing reads, in each of
+// which a group of sixteen lanes hands in 4 rows x 16 columns in pieces of four and takes out four rows of a column each.  (Sixteen reads of
+// a word that two lanes share, shifted and masked, are twice the vector instructions: both packings of 8192 x 4096 with a centre
+// 47.8 -> 44.0 us; the column kernel gains with fewer workgroups, see kColPerCu.)
+__device__ __forceinline__ void column_of_slab(const uint32_t* slab, int words, uint32_t lane, float (&v)[kBlock])
+{
+    typedef short short4_t __attribute__((ext_vector_type(4)));
+    typedef short4_t __attribute__((address_space(3))) * lds_ptr_t;
+    const uint32_t* p = slab + ((lane >> 2) & 3u) * words + (lane >> 4) * 8u + (lane & 3u) * 2u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint2 d = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr_t)(p + 4 * q * words)));
+        v[4 * q] = __uint_as_float(d.x << 16);
+        v[4 * q + 1] = __uint_as_float(d.x & 0xffff0000u);
+        v[4 * q + 2] = __uint_as_float(d.y << 16);
+        v[4 * q + 3] = __uint_as_float(d.y & 0xffff0000u);
+    }
+}
+
 // The same with whole 16-byte loads: a wave requests its next 16-row slab of the tile (consecutive lanes consecutive 16-byte
 // chunks) while it encodes the current one, and turns it in LDS -- written as loaded, read back as columns, as
 // quant_codes_both_kernel does.  A lane's sixteen 2-byte loads per block, each waited for in place, left the kernel above at
 // 3 TB/s; now the vector units (Philox, or the encoder and the turning) and HBM bound it together.  Needs 16-byte-aligned rows (ld and cols multiples of 16 bytes) and
-// takes no caller noise; same bytes.
+// takes no caller noise; same bytes.  Binary32 arithmetic on bf16 values takes its quotients in two operations under the table of block
+// maxima, as the row kernel does (18944 x 3584 with scale bytes 82 -> 64 us).
+// Five workgroups per compute unit: enough loads in flight, and fewer partial lines open at once in each die's L2 than with eight.
+// With scale bytes, eight | six | five | four: 18944 x 3584 51.5 | 50.0 | 48.3 | 48.2 us, 4096 x 14336 44.2 | 43.2 | 41.5 | 40.0,
+// stochastic 2112 x 18944 36.6 | 35.6 | 34.1 | 34.2; binary32 arithmetic, bound by its encoder, 4096 x 14336 52.9 | 56.2 | 54.5 | 57.2,
+// 18944 x 3584 64.5 | 61.2 | 64.4 | 67.7.
+constexpr int kColPerCu = 5;
 template <int MODE, bool SR, bool WIDE = false, bool F32IN = false>
 __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, uint64_t seed, uint64_t offset, uint2* __restrict__ codes,
@@ -397,7 +443,7 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
     amax_t* __restrict__ ws_amax = static_cast<amax_t*>(ws_amax_v);
     __shared__ uint2 s_codes[kColTileCols][kColTileBlocks + 1];
     __shared__ amax_t s_amax[kColTileCols][kColTileBlocks + 2];
-    constexpr int kSlabWords = F32IN ? kColTileCols + 4 : kColTileCols / 2 + 4;
+    constexpr int kSlabWords = F32IN ? kColTileCols + 4 : kColTileCols / 2;
     __shared__ __attribute__((aligned(16))) uint32_t slab[4][kBlock][kSlabWords];
     constexpr int NQ = F32IN ? 4 : 2, CPR = F32IN ? 16 : 8, RPI = 64 / CPR, EPC = F32IN ? 4 : 8;   // loads per lane, chunks per slab row, rows per load, elements per chunk
     const uint32_t nbc = rows / kBlock;
@@ -419,9 +465,12 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
                 q[i] = in && row0 + i * RPI + lrow < valid ? *reinterpret_cast<const uint4*>(p + (int64_t)(i * RPI) * ld) : make_uint4(0u, 0u, 0u, 0u);
         }
     };
+    constexpr bool kTable = MODE == 0 && !SR && !WIDE;
+    __shared__ uint32_t table[kTable ? kQuotientTableWords : 1];
     float gmax = 0.0f;
     uint4 cur[NQ], nxt[NQ];
     fetch(blockIdx.x, 0u, cur);
+    if constexpr (kTable) stage_quotient_table(table);
     for (uint32_t tile = blockIdx.x; tile < tiles_total; tile += gridDim.x) {
         const uint32_t tr = tile / tiles_c, tc = tile - tr * tiles_c;
         const uint32_t c = tc * kColTileCols + lane;
@@ -440,9 +489,7 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
 #pragma unroll
                 for (int j = 0; j < kBlock; ++j) v[j] = __uint_as_float(slab[g][j][lane]);
             } else {
-                const uint32_t shift = (lane & 1u) ? 0u : 16u;  // a bf16 is the upper half of its binary32 value
-#pragma unroll
-                for (int j = 0; j < kBlock; ++j) v[j] = __uint_as_float((slab[g][j][lane >> 1] << shift) & 0xffff0000u);
+                column_of_slab(&slab[g][0][0], kSlabWords, lane, v);
             }
             __builtin_amdgcn_wave_barrier();
             uint2 packed = make_uint2(0u, 0u);
@@ -466,7 +513,11 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
                     else packed = encode_rne_wide(v, sc);
                 } else {
                     if constexpr (SR) packed = encode_sr_hardware<MODE>(v, block_scalar<MODE>(am), seed, offset, (int64_t)c * nbc + b);
-                    else packed = encode_block<MODE, false>(v, block_scalar<MODE>(am), none);
+                    else if constexpr (kTable) {
+                        uint32_t w[2];
+                        encode_rne_p32_tbl<kBlock>(v, am, block_scalar<MODE>(am), table, w);
+                        packed = make_uint2(w[0], w[1]);
+                    } else packed = encode_block<MODE, false>(v, block_scalar<MODE>(am), none);
                 }
             }
             s_codes[lane][bl] = packed;
@@ -604,9 +655,7 @@ __global__ __launch_bounds__(256, CEN ? 4 : WIDE ? 5 : 1) void quant_codes_both_
                     for (int j = 0; j < kBlock; ++j) v[j] = __uint_as_float(slab[g][j][lane]);
                 } else {
                     unpack16(*reinterpret_cast<const uint4*>(&slab[g][rr][cb * 8u]), *reinterpret_cast<const uint4*>(&slab[g][rr][cb * 8u + 4u]), w);
-                    const uint32_t shift = (lane & 1u) ? 0u : 16u;  // a bf16 is the upper half of its binary32 value
-#pragma unroll
-                    for (int j = 0; j < kBlock; ++j) v[j] = __uint_as_float((slab[g][j][lane >> 1] << shift) & 0xffff0000u);
+                    column_of_slab(&slab[g][0][0], kSlabWords, lane, v);
                 }
                 __builtin_amdgcn_wave_barrier();
                 if constexpr (CEN) {
@@ -652,7 +701,7 @@ __global__ __launch_bounds__(256, CEN ? 4 : WIDE ? 5 : 1) void quant_codes_both_
         }
         if (!live) continue;
         __syncthreads();
-        store_col_tile(s_codes, s_amax, codes_col, amax_col, tc, tr, cols, nbc);
+        store_col_tile<!WIDE || CEN>(s_codes, s_amax, codes_col, amax_col, tc, tr, cols, nbc);
         __syncthreads();
     }
     publish_group_max(gmax, ws_gmax);
@@ -1164,13 +1213,13 @@ static int launch_quant(const void* x, int64_t rows, int64_t cols, int64_t ld, c
         const uint32_t tiles_c = (uint32_t)((cols + kColTileCols - 1) / kColTileCols);
         const int64_t tiles = (int64_t)tiles_r * tiles_c;
         int64_t g = tiles;
-        const int64_t cap = (int64_t)device_cus() * 8;
+        const int64_t cap = (int64_t)device_cus() * kColPerCu;
         if (g > cap) g = cap;
         if (g > kMaxGroups) g = kMaxGroups;
         const int per16 = (WIDE && in_f32) ? 4 : 8;              // elements of 16 bytes
         if (!noise && cols % per16 == 0 && ld % per16 == 0 && (uintptr_t)x % 16 == 0) {
-            // with scale bytes, one element | 16 bytes per load: 18944 x 3584 round to nearest 62.0 | 58.3 us, 4096 x 8960 stochastic
-            // 35.7 | 30.4, 2112 x 18944 stochastic with a centre 45.6 | 36.7
+            // with scale bytes, one element | 16 bytes per load (both with narrow stores): 18944 x 3584 round to nearest 62.0 | 58.3 us,
+            // 4096 x 8960 stochastic 35.7 | 30.4, 2112 x 18944 stochastic with a centre 45.6 | 36.7
 #define METIS_QCS(F) hipLaunchKernelGGL((quant_codes_col_slab_kernel<MODE, SR, WIDE, F>), dim3((unsigned)g), dim3(256), 0, st, x, (uint32_t)rows, \
                                         (uint32_t)cols, ld, seed, offset, (uint2*)codes, (void*)ws.amax, ws.gmax, tiles_c, (uint32_t)tiles, center, \
                                         (uint32_t)(valid < 0 ? rows : valid))

@@ -122,6 +122,26 @@ def test_rne_col(ops, shape, tag, mode):
 
 
 @pytest.mark.parametrize("tag,mode", MODES)
+@pytest.mark.parametrize("rows,cols", [(16, 8), (64, 64), (240, 72), (256, 64), (320, 136), (528, 192), (1024, 1032), (272, 63)])
+def test_col_quant_whole_and_partial_tiles(ops, tag, mode, rows, cols):
+    """Tiles that are stored in quads of blocks (256 rows, a multiple of 64 rows in all) beside those that are not, tiles that end within
+    their 64 columns, one column too few for whole loads; block maxima of many binades, so that the quotient table's exceptions are met.
+    Exact: bytes against the oracle's.  (Scalars from 5.2e-7 on: 1e-9 is then below half a bf16 ulp and cannot move a bf16 scalar.  Below,
+    the oracle's CPU addition takes 1e-9 as a bf16 number, the library and the oracle in C as a binary32 one.)"""
+    from oracle import metis_oracle as O
+    g = torch.Generator().manual_seed(rows * 7 + cols)
+    x = (torch.randn(rows, cols, generator=g) * torch.exp2(torch.randint(-12, 30, (rows // 16, cols), generator=g).float()).repeat_interleave(16, 0)).bfloat16()
+    x[::5, ::3] = 0
+    p = ops.quantize(x.cuda(), mode, col=True)
+    codes, scales, unit, _ = O.nvfp4_pack_col(_oracle_in(x, mode))
+    _check_packed(p, codes, scales, unit, f"{rows} x {cols}")
+    if cols % 16 == 0:
+        a, b = ops.quantize_both_sr(x.cuda(), mode, seed=3, offset_row=5, offset_col=77)
+        want = ops.quantize(x.t().contiguous().cuda(), mode, sr=True, seed=3, offset=77)      # (its stream goes by output block)
+        assert torch.equal(b.codes, want.codes) and torch.equal(b.scales, want.scales) and torch.equal(b.unit, a.unit)
+
+
+@pytest.mark.parametrize("tag,mode", MODES)
 @pytest.mark.parametrize("col", [False, True])
 def test_sr_explicit_noise(ops, golden, tag, mode, col):
     from oracle import metis_oracle as O
