@@ -720,39 +720,26 @@ __global__ __launch_bounds__(256) void quant_scales_kernel(const uint16_t* __res
 {
     // grid row 1 (if launched): a second packing of the same tensor (same partial maxima, its own parked block maxima)
     if (blockIdx.y) { ws_amax = ws_amax2; scales = scales2; unit_out = unit_out2; }
-    __shared__ float smax[4];
     const uint32_t nocts = nblocks / 8u;
     const uint32_t step = gridDim.x * 256u;
     uint32_t q = blockIdx.x * 256u + threadIdx.x;
     // first eight parked maxima are requested before the reduction so that both round trips overlap
     uint4 a = make_uint4(0u, 0u, 0u, 0u);
     if (q < nocts) a = reinterpret_cast<const uint4*>(ws_amax)[q];
-    float m = 0.0f;
-    for (uint32_t g = threadIdx.x; g < ngroups; g += 256u) m = fmaxf(m, __uint_as_float(ws_gmax[g]));
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    const float amax = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
+    const float amax = fold_group_maxima(ws_gmax, ngroups);
     // max over blocks of scalar(amax_block) = scalar(max amax_block): the scalar map is monotone
     const float unit = tensor_unit_of<MODE>(amax);
     if (blockIdx.x == 0 && threadIdx.x == 0) *unit_out = unit;
 
-    auto four_bytes = [&](uint32_t w0, uint32_t w1) {
-        const float t0 = rd<MODE>(block_scalar<MODE>(bf16_lo(w0)) / unit);
-        const float t1 = rd<MODE>(block_scalar<MODE>(bf16_hi(w0)) / unit);
-        const float t2 = rd<MODE>(block_scalar<MODE>(bf16_lo(w1)) / unit);
-        const float t3 = rd<MODE>(block_scalar<MODE>(bf16_hi(w1)) / unit);
-        const int w = __builtin_amdgcn_cvt_pk_fp8_f32(t0, t1, 0, false);
-        return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(t2, t3, w, true);
-    };
+    const ScaleBytes<MODE, false> bytes(unit);
     while (q < nocts) {
         const uint32_t nxt = q + step;
         uint4 n = a;
         if (nxt < nocts) n = reinterpret_cast<const uint4*>(ws_amax)[nxt];
-        uint2 o;
-        o.x = four_bytes(a.x, a.y);
-        o.y = four_bytes(a.z, a.w);
-        reinterpret_cast<uint2*>(scales)[q] = o;
+        const float am[8] = {bf16_lo(a.x), bf16_hi(a.x), bf16_lo(a.y), bf16_hi(a.y), bf16_lo(a.z), bf16_hi(a.z), bf16_lo(a.w), bf16_hi(a.w)};
+        uint32_t o[2];
+        bytes(am, o);
+        reinterpret_cast<uint2*>(scales)[q] = make_uint2(o[0], o[1]);
         a = n; q = nxt;
     }
     // ragged tail (block count not a multiple of eight)
@@ -773,13 +760,7 @@ __global__ __launch_bounds__(256) void quant_scales_decode_kernel(const uint16_t
                                                                   uint8_t* __restrict__ scales, float* __restrict__ unit_out,
                                                                   uint8_t* __restrict__ decode, int rows, int cols, int blocks)
 {
-    __shared__ float smax[4];
-    float m = 0.0f;
-    for (uint32_t g = threadIdx.x; g < ngroups; g += 256u) m = fmaxf(m, __uint_as_float(ws_gmax[g]));
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    const float unit = tensor_unit_of<MODE>(fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])));
+    const float unit = tensor_unit_of<MODE>(fold_group_maxima(ws_gmax, ngroups));
     if (blockIdx.x == 0 && threadIdx.x == 0) *unit_out = unit;
     const int iters = cols / 256, l = threadIdx.x & 63, j = threadIdx.x >> 6, h = l >> 5;
     for (int b = blockIdx.x; b < blocks; b += gridDim.x) {
@@ -818,21 +799,24 @@ __global__ __launch_bounds__(256) void quant_scales_f32_kernel(const float* __re
                                                                uint8_t* __restrict__ scales2 = nullptr, float* __restrict__ unit_out2 = nullptr)
 {
     if (blockIdx.y) { ws_amax = ws_amax2; scales = scales2; unit_out = unit_out2; }
-    __shared__ float smax[4];
-    float m = 0.0f;
-    for (uint32_t g = threadIdx.x; g < ngroups; g += 256u) m = fmaxf(m, __uint_as_float(ws_gmax[g]));
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    const float amax = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
+    const uint32_t nquads = nblocks / 4u, step = gridDim.x * 256u;
+    uint32_t q = blockIdx.x * 256u + threadIdx.x;
+    // the next quad is always requested ahead, the first one before the reduction
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (q < nquads) a = reinterpret_cast<const float4*>(ws_amax)[q];
+    const float amax = fold_group_maxima(ws_gmax, ngroups);
     const float unit = block_scalar_ieee(amax) / 448.0f;      // the scalar map is monotone: max of scalars = scalar of max
     if (blockIdx.x == 0 && threadIdx.x == 0) *unit_out = unit;
-    const uint32_t nquads = nblocks / 4u, step = gridDim.x * 256u;
-    for (uint32_t q = blockIdx.x * 256u + threadIdx.x; q < nquads; q += step) {
-        const float4 a = reinterpret_cast<const float4*>(ws_amax)[q];
-        const int w = __builtin_amdgcn_cvt_pk_fp8_f32(block_scalar_ieee(a.x) / unit, block_scalar_ieee(a.y) / unit, 0, false);
-        reinterpret_cast<uint32_t*>(scales)[q] =
-            (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(block_scalar_ieee(a.z) / unit, block_scalar_ieee(a.w) / unit, w, true);
+    const ScaleBytes<0, true> bytes(unit);
+    while (q < nquads) {
+        const uint32_t nxt = q + step;
+        float4 n = a;
+        if (nxt < nquads) n = reinterpret_cast<const float4*>(ws_amax)[nxt];
+        const float am[4] = {a.x, a.y, a.z, a.w};
+        uint32_t o[1];
+        bytes(am, o);
+        reinterpret_cast<uint32_t*>(scales)[q] = o[0];
+        a = n; q = nxt;
     }
     for (uint32_t k = nquads * 4u + blockIdx.x * 256u + threadIdx.x; k < nblocks; k += step)
         scales[k] = (uint8_t)e4m3_byte(block_scalar_ieee(ws_amax[k]) / unit);
@@ -1042,18 +1026,12 @@ __global__ __launch_bounds__(256) void quant_scales_dequant_kernel(const uint32_
 {
     static_assert(!WIDE || MODE == 0, "binary32 values imply binary32 arithmetic");
     using amax_t = typename std::conditional<WIDE, float, uint32_t>::type;
-    __shared__ float smax[4];
     const uint32_t step = gridDim.x * 256u;
     uint32_t i = blockIdx.x * 256u + threadIdx.x;               // half-block index
     uint32_t cw = 0u;
     amax_t aw = 0;
     if (i < nhalves) { cw = codes[i]; aw = ws_amax[i >> 1]; }
-    float m = 0.0f;
-    for (uint32_t g = threadIdx.x; g < ngroups; g += 256u) m = fmaxf(m, __uint_as_float(ws_gmax[g]));
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    const float amax = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
+    const float amax = fold_group_maxima(ws_gmax, ngroups);
     float unit;
     if constexpr (WIDE) unit = block_scalar_ieee(amax) / 448.0f;
     else unit = tensor_unit_of<MODE>(amax);

@@ -122,6 +122,36 @@ def test_rne_col(ops, shape, tag, mode):
 
 
 @pytest.mark.parametrize("tag,mode", MODES)
+@pytest.mark.parametrize("top", [1e-9, 1e-7, 3.0e-5, 0.75, 6.0, 448.0, 1.5e17, 1.5e30, 3.3e38])
+def test_scale_bytes_of_every_bf16_maximum(ops, tag, mode, top):
+    """A block for every finite bf16 maximum up to `top`, the tensor's: units from the smallest there is to beyond 2^60, where bf16
+    arithmetic divides.  Exact: bytes and unit of the oracle in C."""
+    from oracle import c_oracle as C
+    pat = torch.arange(0, 0x7F80, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    am = pat[pat.float() <= torch.tensor(top).bfloat16().float()]
+    x = torch.zeros(am.numel(), 16, dtype=torch.bfloat16)
+    x[:, 3] = -am
+    cc, cs, cu, _ = C.nvfp4_pack(x, mode)
+    _check_packed(ops.quantize(x.cuda(), mode), cc, cs, cu, f"top={top}")
+
+
+@pytest.mark.parametrize("top", [2.5e-8, 1.0, 3.7e5])
+def test_scale_bytes_next_to_the_converter_thresholds(ops, top):
+    """Binary32 maxima whose quotient by the unit lies 0 .. 12 ulps from a threshold of the E4M3 conversion (midpoints of neighbouring
+    values, subnormal ones too).  Exact: the oracle's bytes, from IEEE divisions."""
+    from oracle import metis_oracle as O
+    unit = (torch.tensor(top) / 6 + 1e-9) / 448
+    values = torch.arange(0, 0x7F, dtype=torch.uint8).view(torch.float8_e4m3fn).float()
+    mid = (values[1:] + values[:-1]) / 2
+    am = ((mid[mid < 448] * unit - 1e-9) * 6).clamp_min(0)
+    am = torch.cat([(am.view(torch.int32) + d).clamp_min(0).view(torch.float32) for d in range(-12, 13)] + [torch.tensor([top])])
+    x = torch.zeros(am.numel(), 16)
+    x[:, 7] = am
+    codes, scales, u, _ = O.nvfp4_pack(x)
+    _check_packed(ops.quantize(x.cuda(), 0), codes, scales, u, f"top={top}")
+
+
+@pytest.mark.parametrize("tag,mode", MODES)
 @pytest.mark.parametrize("rows,cols", [(16, 8), (64, 64), (240, 72), (256, 64), (320, 136), (528, 192), (1024, 1032), (272, 63)])
 def test_col_quant_whole_and_partial_tiles(ops, tag, mode, rows, cols):
     """Tiles that are stored in quads of blocks (256 rows, a multiple of 64 rows in all) beside those that are not, tiles that end within
