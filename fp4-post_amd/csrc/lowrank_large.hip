@@ -674,44 +674,88 @@ __global__ __launch_bounds__(256) void lowrank_tn_kernel(const TnProblem p0, con
     lowrank_tn_block<RT>(b < first ? p0 : p1, b < first ? b : b - first, L);
 }
 
-// Adds the token slices in order; out [C, R] or, transposed, [R, C]; bf16 or binary32.  A thread has four consecutive r of a
-// column; the lanes of a wave follow the output: consecutive quads of a row, or consecutive columns.
-__global__ __launch_bounds__(256) void lowrank_tn_finish_kernel(const TnProblem p0, const TnProblem p1, int R, int first)
+// Adds the token slices in order; out [C, R] or, transposed, [R, C]; bf16 or binary32.  A thread has four consecutive r of a column, so
+// that a wave reads whole lines of the partial sums; transposed, a workgroup turns its columns through LDS and writes 32 or 64 bytes (bf16)
+// of a row at a time.  (The lanes over the output's columns fetched 16 bytes of every line, and each line once per quad of r.)  What bounds
+// it is what a compute unit takes in and one round trip to the memory behind the slices' L2s: eight slices are requested together.
+// With the launch before it, both contractions of a layer, tokens x N, K, R, before | now: 4096 x 1536, 8960, 32 32.4 | 25.0 us, 4096 x 8960,
+// 1536, 32 27.3 | 25.6, 2103 x 3584, 18944, 64 44.6 | 31.1, 2103 x 18944, 3584, 64 35.0 | 32.0, 8192 x 4096, 4096, 64 47.9 | 45.7, 1000 x 2048,
+// 2568, 128 20.7 | 17.0.  From a rank of 64 on 32 columns to a workgroup leave compute units idle: 31.1, 34.3, 49.5, 18.7.
+template <int N, int BATCH>
+__device__ __forceinline__ void tn_sum_slices(const TnProblem& p, const float* const (&src)[N], const bool (&live)[N], int64_t CR, float4 (&sum)[N])
+{
+#pragma unroll
+    for (int u = 0; u < N; ++u) sum[u] = live[u] ? *reinterpret_cast<const float4*>(src[u]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int z0 = 1; z0 < p.slices; z0 += BATCH) {
+        float4 v[BATCH][N];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+            if (z0 + i < p.slices) {
+#pragma unroll
+                for (int u = 0; u < N; ++u)
+                    if (live[u]) v[i][u] = *reinterpret_cast<const float4*>(src[u] + (int64_t)(z0 + i) * CR);
+            }
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+            if (z0 + i < p.slices) {
+#pragma unroll
+                for (int u = 0; u < N; ++u)
+                    if (live[u]) { sum[u].x += v[i][u].x; sum[u].y += v[i][u].y; sum[u].z += v[i][u].z; sum[u].w += v[i][u].w; }
+            }
+    }
+}
+__device__ __forceinline__ void tn_store_quad(const TnProblem& p, int64_t o, const float4 f)    // four consecutive elements of the output
 {
     typedef uint32_t pair_t __attribute__((ext_vector_type(2), aligned(4)));
     typedef uint32_t quad_t __attribute__((ext_vector_type(4), aligned(4)));
+    if (p.out_f32)
+        *reinterpret_cast<quad_t*>(static_cast<float*>(p.out) + o) =
+            (quad_t){__float_as_uint(f.x), __float_as_uint(f.y), __float_as_uint(f.z), __float_as_uint(f.w)};
+    else
+        *reinterpret_cast<pair_t*>(static_cast<uint16_t*>(p.out) + o) =
+            (pair_t){bf16_bits(f.x) | (bf16_bits(f.y) << 16), bf16_bits(f.z) | (bf16_bits(f.w) << 16)};
+}
+constexpr int tn_turn(int rt) { return rt == 1 ? 32 : 16; }     // columns that a workgroup turns, 256 quads and more
+template <int RT>
+__global__ __launch_bounds__(256) void lowrank_tn_finish_kernel(const TnProblem p0, const TnProblem p1, int first)
+{
+    constexpr int R = RT * 32, TN_TURN = tn_turn(RT), Q = RT * TN_TURN / 32;
+    __shared__ float turn[R][TN_TURN + 1];
     const bool second = (int)blockIdx.x >= first;
     const TnProblem& p = second ? p1 : p0;
-    const int64_t q = (int64_t)((int)blockIdx.x - (second ? first : 0)) * 256 + threadIdx.x;
+    const int block = (int)blockIdx.x - (second ? first : 0), tid = (int)threadIdx.x;
     const int64_t CR = (int64_t)p.C * R;
-    if (q * 4 >= CR) return;
-    const int64_t c = p.transpose ? q % p.C : q / (R / 4), r = (p.transpose ? q / p.C : q % (R / 4)) * 4;
-    const float* src = p.part + c * R + r;
-    constexpr int BATCH = 8;                                    // slices requested together
-    float4 sum = *reinterpret_cast<const float4*>(src);
-    for (int z0 = 1; z0 < p.slices; z0 += BATCH) {
-        float4 v[BATCH];
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i)
-            if (z0 + i < p.slices) v[i] = *reinterpret_cast<const float4*>(src + (int64_t)(z0 + i) * CR);
-#pragma unroll
-        for (int i = 0; i < BATCH; ++i)
-            if (z0 + i < p.slices) { sum.x += v[i].x; sum.y += v[i].y; sum.z += v[i].z; sum.w += v[i].w; }
+    if (!p.transpose) {
+        const int64_t o = ((int64_t)block * 256 + tid) * 4;
+        const float* const src[1] = {p.part + o};
+        const bool live[1] = {o < CR};
+        float4 sum[1];
+        tn_sum_slices<1, 8>(p, src, live, CR, sum);
+        if (live[0]) tn_store_quad(p, o, sum[0]);
+        return;
     }
-    const float f[4] = {sum.x, sum.y, sum.z, sum.w};
-    if (p.transpose) {
+    const int64_t c0 = (int64_t)block * TN_TURN;
+    const float* src[Q];
+    bool live[Q];
+    float4 sum[Q];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int64_t o = (r + e) * p.C + c;
-            if (p.out_f32) static_cast<float*>(p.out)[o] = f[e];
-            else static_cast<uint16_t*>(p.out)[o] = (uint16_t)bf16_bits(f[e]);
-        }
-    } else if (p.out_f32) {
-        *reinterpret_cast<quad_t*>(static_cast<float*>(p.out) + c * R + r) =
-            (quad_t){__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
-    } else {
-        *reinterpret_cast<pair_t*>(static_cast<uint16_t*>(p.out) + c * R + r) =
-            (pair_t){bf16_bits(f[0]) | (bf16_bits(f[1]) << 16), bf16_bits(f[2]) | (bf16_bits(f[3]) << 16)};
+    for (int u = 0; u < Q; ++u) {
+        const int64_t o = c0 * R + (int64_t)(u * 256 + tid) * 4;     // (the columns of a workgroup are one piece of each slice)
+        src[u] = p.part + o;
+        live[u] = o < CR;
+    }
+    tn_sum_slices<Q, 8 / Q>(p, src, live, CR, sum);
+#pragma unroll
+    for (int u = 0; u < Q; ++u) {
+        const int c = (u * 256 + tid) / (R / 4), r = (u * 256 + tid) % (R / 4) * 4;
+        turn[r][c] = sum[u].x; turn[r + 1][c] = sum[u].y; turn[r + 2][c] = sum[u].z; turn[r + 3][c] = sum[u].w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < Q; ++u) {
+        const int r = (u * 256 + tid) / (TN_TURN / 4), c = (u * 256 + tid) % (TN_TURN / 4) * 4;
+        if (c0 + c < p.C)                                            // (C is a multiple of 8)
+            tn_store_quad(p, (int64_t)r * p.C + c0 + c, make_float4(turn[r][c], turn[r][c + 1], turn[r][c + 2], turn[r][c + 3]));
     }
 }
 
@@ -754,15 +798,19 @@ static int launch_tn(const TnProblem& p0, const TnProblem& p1, int L, int R, int
 {
     const int64_t blocks = scale_blocks + (int64_t)p0.groups * p0.slices + (int64_t)p1.groups * p1.slices;
     if (blocks > INT32_MAX) return METIS_E_ARG;
-#define METIS_TN(RT) hipLaunchKernelGGL((lowrank_tn_kernel<RT>), dim3((unsigned)blocks), dim3(256), 0, st, p0, p1, L, scale_blocks, (const uint16_t*)g, \
-                                        (const uint16_t*)xv, scale_out, scale_f32)
+    auto finishing = [&](const TnProblem& p) {
+        const int64_t per = p.transpose ? tn_turn(R / 32) : 256 * 4 / R;          // columns to a workgroup; R divides 1024
+        return p.C ? ((int64_t)p.C + per - 1) / per : 0;
+    };
+    const int64_t f0 = finishing(p0), f1 = finishing(p1);
+#define METIS_TN(RT) do { hipLaunchKernelGGL((lowrank_tn_kernel<RT>), dim3((unsigned)blocks), dim3(256), 0, st, p0, p1, L, scale_blocks, (const uint16_t*)g, \
+                                             (const uint16_t*)xv, scale_out, scale_f32); \
+                          if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH; \
+                          hipLaunchKernelGGL((lowrank_tn_finish_kernel<RT>), dim3((unsigned)(f0 + f1)), dim3(256), 0, st, p0, p1, (int)f0); } while (0)
     if (R == 32) METIS_TN(1);
     else if (R == 64) METIS_TN(2);
     else METIS_TN(4);
 #undef METIS_TN
-    if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;
-    const int64_t f0 = ((int64_t)p0.C * R / 4 + 255) / 256, f1 = ((int64_t)p1.C * R / 4 + 255) / 256;
-    hipLaunchKernelGGL(lowrank_tn_finish_kernel, dim3((unsigned)(f0 + f1)), dim3(256), 0, st, p0, p1, R, (int)f0);
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 

@@ -970,6 +970,21 @@ def test_gradients_of_the_rank_r_branch_side_by_side(L, N, K, R):
     assert torch.equal(strided[1], gv) and torch.equal(strided[2], ops.lowrank_scale_grad(gt, xv))
 
 
+@pytest.mark.parametrize("R", [32, 64, 128])
+@pytest.mark.parametrize("L,C", [(1, 8), (300, 16), (515, 24), (700, 40), (4608, 8), (2311, 1000)])
+def test_token_contractions_in_both_layouts_at_the_edges_of_a_turned_piece(L, C, R):
+    """[C, R] and [R, C] in bf16 and binary32, from one slice of the tokens to eighteen and from less than the columns that a workgroup
+    turns to many pieces: small whole numbers, every sum of which binary32 holds, so the outputs are exact."""
+    from metis_hip import ops
+    g_ = torch.Generator().manual_seed(8300 + L + R)
+    a, b = (torch.randint(-8, 9, (L, n), generator=g_).bfloat16() for n in (C, R))
+    want = a.double().T @ b.double()
+    for dt in (torch.bfloat16, torch.float32):
+        for transpose in (False, True):
+            got = ops.lowrank_contract_tokens(a.cuda(), b.cuda(), dt, transpose).cpu()
+            assert torch.equal(got, (want.T if transpose else want).to(dt)), (dt, transpose)
+
+
 @pytest.mark.parametrize("L,R", [(1, 8), (255, 40), (257, 32), (2047, 32), (2049, 8), (4096, 32), (5000, 64)])
 def test_gradient_of_the_rank_r_scale_vector_is_added_in_its_documented_order(L, R):
     """256 sums of every 256th row, in row order, then these in order: binary32 on the CPU in that order gives the same bits."""
