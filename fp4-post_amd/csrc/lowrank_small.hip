@@ -4,8 +4,10 @@
 //
 // The output is tiny (M x R) and the contraction long (K up to 18944): the vendor library runs such a product as one
 // or a few workgroups walking all of K (35 us at 64 x 64 x 18944).  Here K is cut into up to 128 chunks of one to three
-// 64-element steps (the product is latency-bound: a step is one round trip to memory), one workgroup per chunk and
-// 64 rows; wave w owns 32 columns of R (R / 32 waves, at most 8); a lane streams 64 contiguous bytes of its row per
+// 64-element steps (the product is latency-bound: a step is one round trip to memory), one wave, a workgroup of its own, per chunk, 32
+// rows and 32 columns of R (a workgroup per chunk and 64 rows left three of four compute units idle while it looked up its lines: with the
+// finishing launch, 64 x 3584, R = 192 9.2 -> 7.0 us, 64 x 18944, R = 64 8.8 -> 7.4, 5 x 1536, R = 192 6.1 -> 5.1, 255 x 3584, R = 192 15.2 ->
+// 14.7; the captured decode step of 64 sequences, hidden 3584, 162.5 -> 156.0); a lane streams 64 contiguous bytes of its row per
 // step straight into MFMA operands (both operands with the same mapping, so K may be visited in that permuted order).
 // Partial sums go to a caller-supplied workspace [chunks][M][R] and a second small kernel adds them in chunk order
 // (four threads per output quad, each a quarter of the chunks, folded in order), rounds to bf16 and applies s.
@@ -14,11 +16,11 @@
 
 namespace metis {
 
-__global__ __launch_bounds__(512) void lowrank_small_partial_kernel(const uint16_t* __restrict__ x, int64_t ldx,
-                                                                    const uint16_t* __restrict__ v, int M, int R, int K, int kc,
-                                                                    float* __restrict__ ws)
+__global__ __launch_bounds__(64) void lowrank_small_partial_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                                   const uint16_t* __restrict__ v, int M, int R, int K, int kc,
+                                                                   float* __restrict__ ws)
 {
-    lowrank_small_partial_block((int)blockIdx.x, (int)blockIdx.y, x, ldx, v, M, R, K, kc, ws);
+    lowrank_small_partial_wave<1, true>((int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, x, ldx, v, M, R, K, kc, ws);
 }
 
 __global__ __launch_bounds__(256) void lowrank_small_finish_kernel(const float* __restrict__ ws, int chunks, int MR, int R,
@@ -57,7 +59,7 @@ int lowrank_small_partial(const void* x, int64_t ldx, const void* v, int64_t M, 
     if (M == 0) return METIS_OK;
     int kc;
     const int chunks = lowrank_small_chunks(K, &kc);
-    hipLaunchKernelGGL(lowrank_small_partial_kernel, dim3((unsigned)chunks, (unsigned)((M + 63) / 64)), dim3((unsigned)(2 * R)), 0, st,
+    hipLaunchKernelGGL(lowrank_small_partial_kernel, dim3((unsigned)chunks, (unsigned)((M + 31) / 32), (unsigned)(R / 32)), dim3(64), 0, st,
                        (const uint16_t*)x, ldx, (const uint16_t*)v, (int)M, (int)R, (int)K, kc, (float*)workspace);
     *chunks_out = chunks;
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;

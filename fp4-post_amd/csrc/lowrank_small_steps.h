@@ -23,55 +23,95 @@ inline int lowrank_small_chunks(int64_t K, int* kc_out)
     return (int)((K + kc - 1) / kc);
 }
 
-// One workgroup of the first step: K chunk `chunk` (kc elements), rows 64 mtile .. ; wave w owns columns 32 w .. of R
-// (waves past R / 32 have nothing to do), so the launch needs at least 2 R threads per workgroup, or several workgroups for a chunk,
-// the first wave of each (wave0) further on in R.
-__device__ __forceinline__ void lowrank_small_partial_block(int chunk, int mtile, const uint16_t* __restrict__ x, int64_t ldx,
-                                                            const uint16_t* __restrict__ v, int M, int R, int K, int kc,
-                                                            float* __restrict__ ws, int wave0 = 0)
+// One wave of the first step: K chunk `chunk` (kc elements), RT tiles of 32 rows from 32 RT mtile on, columns 32 ct .. of R.  Every load
+// touches 64 lines, which a compute unit's L1 looks up one a cycle: a step (4 + 4 RT loads) is bound by that and by one round trip to
+// memory.  AHEAD: the next step is requested before this one is multiplied (32 more registers, which cost a launch with other work more
+// than they give).
+template <int RT, bool AHEAD>
+__device__ __forceinline__ void lowrank_small_partial_wave(int chunk, int mtile, int ct, const uint16_t* __restrict__ x, int64_t ldx,
+                                                           const uint16_t* __restrict__ v, int M, int R, int K, int kc, float* __restrict__ ws)
 {
-    const int lane = threadIdx.x & 63, wave = wave0 + (int)(threadIdx.x >> 6), hi = lane >> 5;
-    if (wave * 32 >= R) return;
-    const int m0 = mtile * 64;
+    const int lane = threadIdx.x & 63, hi = lane >> 5;
+    const int m0 = mtile * (32 * RT);
     const int k0 = chunk * kc, k1 = min(k0 + kc, K);
-    const uint16_t* vp = v + (int64_t)min(wave * 32 + (lane & 31), R - 1) * K + hi * 32;
-    const uint16_t* xp[2];
+    const uint16_t* vp = v + (int64_t)min(ct * 32 + (lane & 31), R - 1) * K + hi * 32;
+    const uint16_t* xp[RT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) xp[i] = x + (int64_t)min(m0 + i * 32 + (lane & 31), M - 1) * ldx + hi * 32;
-    lr_float16_t acc[2];
+    for (int i = 0; i < RT; ++i) xp[i] = x + (int64_t)min(m0 + i * 32 + (lane & 31), M - 1) * ldx + hi * 32;
+    lr_float16_t acc[RT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
-    for (int k = k0; k < k1; k += 64) {                        // kc % 64 == 0 and K % 64 == 0
-        uint4 rv[4], rx[2][4];
+    auto fetch = [&](uint4 (&rv)[4], uint4 (&rx)[RT][4], int k) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) rv[q] = reinterpret_cast<const uint4*>(vp + k)[q];
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < RT; ++i)
 #pragma unroll
             for (int q = 0; q < 4; ++q) rx[i][q] = reinterpret_cast<const uint4*>(xp[i] + k)[q];
+    };
+    uint4 nv[4], nx[RT][4];
+    if constexpr (AHEAD) fetch(nv, nx, k0);
+    for (int k = k0; k < k1; k += 64) {                        // kc % 64 == 0 and K % 64 == 0
+        uint4 rv[4], rx[RT][4];
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                rv[q] = nv[q];
+#pragma unroll
+                for (int i = 0; i < RT; ++i) rx[i][q] = nx[i][q];
+            }
+            if (k + 64 < k1) fetch(nv, nx, k + 64);
+        } else {
+            fetch(rv, rx, k);
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const lr_bf16x8_t fv = __builtin_bit_cast(lr_bf16x8_t, rv[q]);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < RT; ++i)
                 acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv, __builtin_bit_cast(lr_bf16x8_t, rx[i][q]), acc[i], 0, 0, 0);
         }
     }
-    // acc[i][e] of lane l: row m = m0 + 32 i + l % 32, column r = 32 wave + 8 (e / 4) + 4 (l / 32) + e % 4
+    // acc[i][e] of lane l: row m = m0 + 32 i + l % 32, column r = 32 ct + 8 (e / 4) + 4 (l / 32) + e % 4
     float* wp = ws + (size_t)chunk * M * R;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < RT; ++i) {
         const int m = m0 + i * 32 + (lane & 31);
         if (m >= M) continue;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int r = wave * 32 + 8 * g + 4 * hi;
+            const int r = ct * 32 + 8 * g + 4 * hi;
             if (r < R)                                          // R % 4 == 0
                 *reinterpret_cast<float4*>(wp + (size_t)m * R + r) =
                     make_float4(acc[i][4 * g], acc[i][4 * g + 1], acc[i][4 * g + 2], acc[i][4 * g + 3]);
         }
+    }
+}
+
+// The first step in a launch of 256-thread workgroups with other work: single tiles of 32 x 32, a workgroup with one wave for each, or
+// (wide) four waves of 64 rows x 32 columns that share the rows' lines.  Microseconds with the quantizer, wide | single: 64 x 3584, R = 64
+// 3.3 | 2.8, R = 128 4.3 | 3.0, 64 x 18944, R = 64 4.9 | 4.0, 5 x 18944, R = 128 4.5 | 3.2, 128 x 3584, R = 128 4.6 | 3.7, 128 x 8960, R = 128 6.1 | 5.2,
+// 255 x 8960, R = 64 6.2 | 5.7, 192 x 18944, R = 32 5.7 | 5.6; where the compute units have more than ten steps of tiles each, re-reading V costs
+// more: 192 x 8960, R = 128 6.6 | 8.3, 255 x 18944, R = 64 9.0 | 11.9.  (64 rows and fewer: 64 x 18944, R = 128 7.2 | 5.6.)
+inline bool lowrank_small_wide(int64_t M, int64_t R, int64_t K, int cus)
+{
+    return M > 64 && (M + 31) / 32 * (R / 32) * (K / 64) > 10 * (int64_t)cus;
+}
+inline int lowrank_small_partial_blocks(int64_t M, int64_t R, int chunks, bool wide)
+{
+    return chunks * (int)(wide ? (M + 63) / 64 * ((R + 127) / 128) : (M + 31) / 32 * (R / 32));
+}
+__device__ __forceinline__ void lowrank_small_partial_block(int block, int chunks, bool wide, const uint16_t* __restrict__ x, int64_t ldx,
+                                                            const uint16_t* __restrict__ v, int M, int R, int K, int kc, float* __restrict__ ws)
+{
+    const int chunk = block % chunks, rest = block / chunks, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (wide) {
+        const int mtiles = (M + 63) / 64, ct = rest / mtiles * 4 + wave;
+        if (ct * 32 < R) lowrank_small_partial_wave<2, false>(chunk, rest % mtiles, ct, x, ldx, v, M, R, K, kc, ws);
+    } else if (wave == 0) {
+        lowrank_small_partial_wave<1, false>(chunk, rest / (R / 32), rest % (R / 32), x, ldx, v, M, R, K, kc, ws);
     }
 }
 

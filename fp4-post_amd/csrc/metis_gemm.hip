@@ -1211,10 +1211,15 @@ int skinny_operand_rht(const void* codes, const void* scales, float* unit, const
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 
-// Whether the launch that builds the operands forms the whole projection: a block of 16 x 16 results reads 64 K bytes of x and V (1.6 us per 1024 of
-// K), while partial sums of K chunks cost a launch and M R binary32 values per chunk.  Microseconds, two launches | one: 64 x 1536, R = 192 8.6 | 6.3,
-// R = 64 6.6 | 6.3; 64 x 2048, R = 64 6.7 | 7.2, R = 128 7.7 | 7.2; 64 x 2560, R = 192 8.9 | 8.1; 4 x 3072, R = 192 6.8 | 7.4; 192 x 2048, R = 192 10.2 | 7.4.
-static bool project_whole(int64_t R, int64_t K) { return K <= kLrProjectK && K <= 896 + 10 * R; }
+// Whether the launch that builds the operands forms the whole projection: a block of 16 x 16 results reads 64 K bytes of x and V (1.7 us per 1024 of
+// K, less with few rows), while partial sums of K chunks cost a launch and grow with the number of 32 x 32 x 64 steps (2.7 us per 1000).  Microseconds,
+// two launches | one: 64 x 1536, R = 192 5.9 | 6.2, 64 x 1024, R = 192 5.5 | 5.5, R = 64 5.2 | 5.4; 1 x 1024 5.0 | 4.8, 1 x 1536, R = 64 5.06 | 5.15;
+// 128 x 1024, R = 128 5.6 | 5.5; 128 x 1536, R = 192 6.6 | 6.2, R = 128 6.1 | 6.1; 192 x 1536, R = 64 6.0 | 6.2, R = 128 6.7 | 6.2; 192 x 2048, R = 128
+// 7.2 | 7.1, R = 192 8.2 | 7.2; 128 x 2560, R = 192 7.6 | 8.0; 192 x 3072, R = 192 10.1 | 8.9, R = 128 8.3 | 8.8.
+static bool project_whole(int64_t M, int64_t R, int64_t K)
+{
+    return K <= kLrProjectK && (M + 31) / 32 * (R / 32) * (K / 64) > (K - 1024) * 5 / 8 + (M < 16 ? 9 * M : 148);
+}
 
 // lowrank_small + skinny_operand_deferred on the same activation (x [M, K] bf16 and its packed form) in one launch, or in two: partial
 // sums of the projection, then one launch that finishes it and builds the operands (project_whole).
@@ -1232,7 +1237,7 @@ int decode_prepare_deferred(const void* x, int64_t ldx, const void* v, int64_t R
     Workspace ws;
     if (const int rc = carve_deferred(const_cast<void*>(deferred), deferred_bytes(M, K), M, K, &ws)) return rc;
     int chunks = 0;
-    if (x && project_whole(R, K)) {
+    if (x && project_whole(M, R, K)) {
         if (const int rc = lowrank_small_check(x, ldx, v, M, R, K, s, xv, t, workspace, workspace_bytes)) return rc;
         const int pb = lowrank_small_project_blocks(M, R), tiles = (int)((M + 63) / 64) * 2;
         const int g = pb + tiles * (int)(K / 256);             // a thread per piece of the operands

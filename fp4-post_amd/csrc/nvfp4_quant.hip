@@ -96,21 +96,19 @@ __global__ __launch_bounds__(256) void quant_codes_contig_kernel(const uint4* __
 }
 
 // A decode-sized activation's quantizer (scale bytes deferred) and the first step of its rank-r projection
-// (lowrank_small_steps.h) in one launch: both only read x.  Blocks 0 .. qgrid-1 quantize, the others take one K chunk of
-// 64 rows each (R <= 128: four waves cover the columns).
+// (lowrank_small_steps.h) in one launch: both only read x.  Blocks 0 .. qgrid-1 quantize, the others form the partial sums.
 template <int MODE>
 __global__ __launch_bounds__(256) void decode_quant_partial_kernel(uint32_t qgrid, const uint4* __restrict__ x, uint2* __restrict__ codes,
                                                                    uint16_t* __restrict__ ws_amax, uint32_t* __restrict__ ws_gmax,
                                                                    uint32_t nblocks, uint32_t fill_to, int64_t ldx,
                                                                    const uint16_t* __restrict__ v, int M, int R, int K, int kc, int chunks,
-                                                                   float* __restrict__ lr_ws)
+                                                                   int wide, float* __restrict__ lr_ws)
 {
     if (blockIdx.x < qgrid) {
         quant_codes_contig_block<MODE, 1>(blockIdx.x, qgrid, x, codes, ws_amax, ws_gmax, nblocks, fill_to);
         return;
     }
-    const int b = (int)(blockIdx.x - qgrid);
-    lowrank_small_partial_block(b % chunks, b / chunks, reinterpret_cast<const uint16_t*>(x), ldx, v, M, R, K, kc, lr_ws);
+    lowrank_small_partial_block((int)(blockIdx.x - qgrid), chunks, wide != 0, reinterpret_cast<const uint16_t*>(x), ldx, v, M, R, K, kc, lr_ws);
 }
 
 // The same loop with a centre subtracted first (mean mode, src/Metis/Metis/bitlinear.py:311-336: the tensor that is
@@ -1467,10 +1465,11 @@ int quantize_row_deferred_partial(const void* x, int64_t rows, int64_t cols, int
     const int g1 = deferred_grid(nblocks, kContigPerCu);
     int kc;
     const int chunks = lowrank_small_chunks(cols, &kc);
-    const int g = g1 + chunks * (int)((rows + 63) / 64);
+    const bool wide = lowrank_small_wide(rows, R, cols, device_cus());
+    const int g = g1 + lowrank_small_partial_blocks(rows, R, chunks, wide);
 #define METIS_QP(MODE) hipLaunchKernelGGL((decode_quant_partial_kernel<MODE>), dim3(g), dim3(256), 0, st, (uint32_t)g1, (const uint4*)x, \
                                           (uint2*)codes, ws.amax, ws.gmax, nblocks, kDeferredPartials, cols, (const uint16_t*)v, \
-                                          (int)rows, (int)R, (int)cols, kc, chunks, (float*)lr_workspace)
+                                          (int)rows, (int)R, (int)cols, kc, chunks, (int)wide, (float*)lr_workspace)
     if (mode == 0) METIS_QP(0); else METIS_QP(1);
 #undef METIS_QP
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;

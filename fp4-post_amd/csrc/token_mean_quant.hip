@@ -29,7 +29,7 @@ constexpr uint32_t kStrip = 32, kMaxPieces = 256;
 struct TokenMeanProjection {             // the first step of x . v^T rides in the workgroups behind the strips (R = 0: none)
     const uint16_t* v;
     float* ws;
-    int R, kc, chunks, mtiles;
+    int R, kc, chunks, wide;
 };
 
 template <int NORM>
@@ -40,8 +40,7 @@ __global__ __launch_bounds__(256) void token_mean_quant_kernel(uint32_t strip_bl
                                                                uint32_t* __restrict__ ws_gmax, const TokenMeanProjection pr)
 {
     if (blockIdx.x >= strip_blocks) {
-        const int b = (int)(blockIdx.x - strip_blocks), rest = b / pr.chunks;
-        lowrank_small_partial_block(b % pr.chunks, rest % pr.mtiles, x, cols, pr.v, (int)rows, pr.R, (int)cols, pr.kc, pr.ws, rest / pr.mtiles * 4);
+        lowrank_small_partial_block((int)(blockIdx.x - strip_blocks), pr.chunks, pr.wide != 0, x, cols, pr.v, (int)rows, pr.R, (int)cols, pr.kc, pr.ws);
         return;
     }
     __shared__ __attribute__((aligned(16))) float sums[kMaxPieces][kStrip];
@@ -186,8 +185,8 @@ int token_mean_quant(const void* x, int64_t rows, int64_t cols, int after_norm, 
         pr.ws = (float*)lr_workspace;
         pr.R = (int)R;
         pr.chunks = lowrank_small_chunks(cols, &pr.kc);
-        pr.mtiles = (int)((rows + 63) / 64);
-        more = pr.chunks * pr.mtiles * (int)((R + 127) / 128);    // four waves of 32 columns of R each
+        pr.wide = lowrank_small_wide(rows, R, cols, device_cus());
+        more = lowrank_small_partial_blocks(rows, R, pr.chunks, pr.wide != 0);
     }
     Workspace ws;
     if (const int rc = carve_deferred(deferred, bytes, rows, cols, &ws)) return rc;

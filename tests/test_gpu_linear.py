@@ -1202,6 +1202,29 @@ def test_projection_formed_whole_beside_the_operand_build_has_the_bits_of_its_tw
     assert bool(((xv.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,K,R", [(1, 1024, 64), (16, 1024, 64), (64, 1024, 192), (65, 1536, 192), (128, 1536, 192), (33, 3584, 96), (255, 3072, 256),
+                                   (65, 8960, 128), (192, 8960, 128), (255, 18944, 32), (160, 18944, 64)])
+def test_decode_sized_projection_has_the_same_bits_whichever_launch_forms_it(M, K, R):
+    """Partial sums by single tiles in a launch of their own, by single tiles or by four waves of 64 rows beside the quantizer, and the whole projection
+    beside the operand build: sizes on either side of each line, ragged row tiles, chunks of one to three steps, the last one shorter."""
+    from metis_hip import ops
+    g = torch.Generator().manual_seed(7 * M + K + R)
+    x = synthetic_activation(900 + M, M, K).cuda()
+    v = (torch.randn(R, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    s = torch.randn(R, generator=g).bfloat16().cuda()
+    xv, t = ops.lowrank_project(x, v, s)
+    again = [ops.project_and_operand(x, v, s, ops.quantize(x, 1, deferred=True))[:2]]
+    if R <= 128:
+        p, pending = ops.quantize_project_decode(x, v, 1)
+        again.append(ops.project_and_operand(x, v, s, p, 1, None, pending=pending)[:2])
+    for xv1, t1 in again:
+        assert torch.equal(xv1, xv) and torch.equal(t1, t)
+    # one rounding to eight significant bits, and binary32 sums of K exact products in whatever order: (K / 16 + 16) 2^-24 of the sum of magnitudes at most
+    want = x.double() @ v.double().T
+    bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ v.double().abs().T) * (K / 16 + 16) * 2.0 ** -24
+    assert bool(((xv.double() - want).abs() <= bound).all())
+
+
 def test_decode_prepare_rejects_what_its_two_halves_reject():
     from metis_hip import _lib, ops
     L = _lib.load()
