@@ -1225,6 +1225,22 @@ def test_decode_sized_projection_has_the_same_bits_whichever_launch_forms_it(M, 
     assert bool(((xv.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,K,R", [(256, 18944, 64), (259, 9216, 32), (300, 10240, 96), (777, 2048, 64)])
+def test_projection_of_a_short_prompt_adds_any_number_of_slices(M, K, R):
+    """Two to sixteen slices of K: more and fewer than are requested together, a last workgroup of the finishing launch that is not full."""
+    from metis_hip import ops
+    g = torch.Generator().manual_seed(5 * M + K + R)
+    x = synthetic_activation(700 + M, M, K).cuda()
+    v = (torch.randn(R, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    s = torch.randn(R, generator=g).bfloat16().cuda()
+    xv, t = ops.lowrank_project(x, v, s)
+    assert torch.equal(t, xv * s) and torch.equal(ops.lowrank_project(x, v), xv)
+    # one rounding to eight significant bits, and binary32 sums of K exact products in whatever order: (K / 16 + 16) 2^-24 of the sum of magnitudes at most
+    want = x.double() @ v.double().T
+    bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ v.double().abs().T) * (K / 16 + 16) * 2.0 ** -24
+    assert bool(((xv.double() - want).abs() <= bound).all())
+
+
 def test_decode_prepare_rejects_what_its_two_halves_reject():
     from metis_hip import _lib, ops
     L = _lib.load()
