@@ -3,15 +3,17 @@
 //
 //   call(name, device_index, specs, args) -> tuple of tensors, or the entry point's return code if it is not METIS_OK
 //
-// specs: one (type, size, ...) per tensor to allocate on the device, type 0 uint8, 1 bfloat16, 2 float32.  args: the entry point's arguments in order;
-// an int or a float is passed as it is, None is a null pointer, a tensor is its address, a text of one character the address of the new tensor at its distance from "0", a list of
-// tuples an array of structures of 64-bit words (metis_linear_member, metis_lowrank_factor) given by its words.  Number and kinds of the arguments are
-// checked against the declaration in metis_hip.h.  The interpreter's lock is released during the call, as ctypes releases it.
+// specs: one (type, size, ...) per tensor to allocate on the device, type 0 uint8, 1 bfloat16, 2 float32.  args: the entry point's arguments in order,
+// each taken as the declaration in metis_hip.h says: for an integer whatever Python takes for an index (its low bits, as ctypes passes it), for a float
+// whatever has a float value, for an address None, a tensor, an integer or the new tensor at a text of one character's distance from "0", for an array of
+// structures (metis_linear_member, metis_lowrank_factor) a list of tuples of their 64-bit words, as many as the argument behind it says.  Anything else
+// is a TypeError or a ValueError.  The interpreter's lock is released during the call, as ctypes releases it.
 //
 // Per call and new tensor the same through ctypes and torch.empty cost 5.1 and 1.7 us, here 3.9 and 1.0 (launch included): an eager decode step
 // of five sequences (hidden 1536, 19 launches, 46 new tensors) 415 -> 367 us, a prompt of 411 tokens 462 -> 410, a small round trip 8.2 -> 6.8.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <cstddef>
 #include <ATen/ops/empty.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -24,17 +26,43 @@
 
 namespace {
 
-struct Value {
+enum Kind : uint8_t { kInteger, kReal, kAddress, kMembers, kFactors };
+template <class T>
+constexpr Kind kind_of()
+{
+    using P = std::remove_cv_t<std::remove_pointer_t<T>>;
+    if (std::is_floating_point<T>::value) return kReal;
+    if (!std::is_pointer<T>::value) return kInteger;
+    if (std::is_same<P, metis_linear_member>::value) return kMembers;
+    return std::is_same<P, metis_lowrank_factor>::value ? kFactors : kAddress;
+}
+template <class... A> struct Kinds { static constexpr Kind of[] = {kind_of<A>()...}; };
+template <class... A> constexpr const Kind* kinds(int (*)(A...)) { return Kinds<A...>::of; }
+// an array of structures is followed by their number
+constexpr bool counted(const Kind* k, size_t n)
+{
+    for (size_t i = 0; i < n; ++i)
+        if ((k[i] == kMembers || k[i] == kFactors) && (i + 1 == n || k[i + 1] != kInteger)) return false;
+    return true;
+}
+
+// the words of the structures
+constexpr Kind kMember[] = {kAddress, kAddress, kAddress, kAddress, kAddress, kInteger, kAddress, kAddress, kInteger, kInteger, kInteger, kAddress};
+constexpr Kind kFactor[] = {kAddress, kAddress, kInteger};
+static_assert(sizeof(metis_linear_member) == sizeof(kMember) * 8 && offsetof(metis_linear_member, r) == 5 * 8 && offsetof(metis_linear_member, N) == 8 * 8 &&
+              offsetof(metis_linear_member, bias_is_f32) == 9 * 8 && offsetof(metis_linear_member, ldt) == 10 * 8, "kMember follows the declaration");
+static_assert(sizeof(metis_lowrank_factor) == sizeof(kFactor) * 8 && offsetof(metis_lowrank_factor, r) == 2 * 8, "kFactor follows the declaration");
+
+union Value {
     int64_t i;
     double f;
-    bool is_float;
 };
 
 template <class T>
 T as(const Value& v)
 {
     if constexpr (std::is_pointer<T>::value) return reinterpret_cast<T>(static_cast<uintptr_t>(v.i));
-    else if constexpr (std::is_floating_point<T>::value) return static_cast<T>(v.is_float ? v.f : static_cast<double>(v.i));
+    else if constexpr (std::is_floating_point<T>::value) return static_cast<T>(v.f);
     else return static_cast<T>(v.i);
 }
 
@@ -46,24 +74,16 @@ int spread(int (*fn)(A...), const Value* v, std::index_sequence<I...>)
 template <class... A>
 constexpr size_t arity(int (*)(A...)) { return sizeof...(A); }
 template <class... A>
-bool kinds_fit(int (*)(A...), const Value* v)                  // a float only where the entry point takes one
-{
-    constexpr bool takes[] = {std::is_floating_point<A>::value...};
-    for (size_t i = 0; i < sizeof...(A); ++i)
-        if (v[i].is_float && !takes[i]) return false;
-    return true;
-}
-template <class... A>
 int spread_all(int (*fn)(A...), const Value* v) { return spread(fn, v, std::index_sequence_for<A...>()); }
 
 struct Entry {
     const char* name;
     size_t args;
-    bool (*fits)(const Value*);
+    const Kind* kinds;
     int (*run)(const Value*);
 };
-#define METIS_ENTRY(fn) {#fn, arity(fn), [](const Value* v) { return kinds_fit(fn, v); }, [](const Value* v) { return spread_all(fn, v); }}
-const Entry kEntries[] = {
+#define METIS_ENTRY(fn) {#fn, arity(fn), kinds(fn), [](const Value* v) { return spread_all(fn, v); }}
+constexpr Entry kEntries[] = {
     METIS_ENTRY(metis_nvfp4_quant_row),
     METIS_ENTRY(metis_nvfp4_quant_col),
     METIS_ENTRY(metis_nvfp4_quant_col_padded),
@@ -108,6 +128,13 @@ const Entry kEntries[] = {
     METIS_ENTRY(metis_lowrank_backward),
 };
 constexpr size_t kMaxArgs = 32, kMaxOuts = 32;
+constexpr bool all_counted()
+{
+    for (const Entry& e : kEntries)
+        if (e.args > kMaxArgs || !counted(e.kinds, e.args)) return false;
+    return true;
+}
+static_assert(all_counted(), "at most kMaxArgs arguments, and a number behind every array of structures");
 PyObject* g_index = nullptr;                                   // name -> position in kEntries
 
 struct Outputs {
@@ -117,26 +144,36 @@ struct Outputs {
     ~Outputs() { for (size_t i = 0; i < count; ++i) Py_XDECREF(obj[i]); }
 };
 
-// one argument; false with a Python error set
-bool value_of(PyObject* o, const Outputs& outs, Value* v)
+// one argument or word of the given kind; false with a Python error set
+bool value_of(PyObject* o, Kind kind, const Outputs& outs, Value* v)
 {
-    v->is_float = false;
-    v->f = 0.0;
-    if (o == Py_None) { v->i = 0; return true; }
-    if (PyLong_Check(o)) {                                     // (also bool; 64-bit seeds may use the sign bit)
+    if (kind == kReal) {
+        v->f = PyFloat_AsDouble(o);
+        return !(v->f == -1.0 && PyErr_Occurred());
+    }
+    if ((kind == kInteger || kind == kAddress) && PyLong_Check(o)) {   // (also bool; 64-bit seeds may use the sign bit)
         v->i = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(o));
         return !(v->i == -1 && PyErr_Occurred());
     }
-    if (THPVariable_Check(o)) {
-        v->i = static_cast<int64_t>(reinterpret_cast<uintptr_t>(THPVariable_Unpack(o).data_ptr()));
-        return true;
+    if (kind == kInteger) {
+        PyObject* n = PyNumber_Index(o);
+        if (!n) return false;
+        v->i = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(n));
+        Py_DECREF(n);
+        return !(v->i == -1 && PyErr_Occurred());
     }
-    if (PyFloat_Check(o)) { v->f = PyFloat_AS_DOUBLE(o); v->is_float = true; v->i = 0; return true; }
-    if (PyUnicode_Check(o) && PyUnicode_GET_LENGTH(o) == 1) {
-        const int k = static_cast<int>(PyUnicode_READ_CHAR(o, 0)) - '0';
-        if (k >= 0 && static_cast<size_t>(k) < outs.count) { v->i = outs.at[k]; return true; }
+    if (kind == kAddress) {
+        if (o == Py_None) { v->i = 0; return true; }
+        if (THPVariable_Check(o)) {
+            v->i = static_cast<int64_t>(reinterpret_cast<uintptr_t>(THPVariable_Unpack(o).data_ptr()));
+            return true;
+        }
+        if (PyUnicode_Check(o) && PyUnicode_GET_LENGTH(o) == 1) {
+            const int k = static_cast<int>(PyUnicode_READ_CHAR(o, 0)) - '0';
+            if (k >= 0 && static_cast<size_t>(k) < outs.count) { v->i = outs.at[k]; return true; }
+        }
     }
-    PyErr_Format(PyExc_TypeError, "call: an argument of type %s", Py_TYPE(o)->tp_name);
+    PyErr_Format(PyExc_TypeError, kind == kAddress ? "call: %s for an address" : "call: %s for a list of structures", Py_TYPE(o)->tp_name);
     return false;
 }
 
@@ -184,6 +221,7 @@ PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n)
     Value v[kMaxArgs];
     std::vector<int64_t> words[2];                             // arrays of structures; filled whole before their address is taken
     size_t arrays = 0;
+    Py_ssize_t listed = 0;                                     // structures of the last array
     const size_t given = static_cast<size_t>(PyTuple_GET_SIZE(a[3]));
     if (given != e.args || given > kMaxArgs) {
         PyErr_Format(PyExc_TypeError, "%s takes %zu arguments (%zu given)", e.name, e.args, given);
@@ -191,25 +229,35 @@ PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n)
     }
     for (size_t i = 0; i < given; ++i) {
         PyObject* o = PyTuple_GET_ITEM(a[3], static_cast<Py_ssize_t>(i));
-        if (!PyList_Check(o)) {
-            if (!value_of(o, outs, &v[i])) return nullptr;
+        const bool members = e.kinds[i] == kMembers;
+        if (!PyList_Check(o) || (!members && e.kinds[i] != kFactors)) {
+            if (!value_of(o, e.kinds[i], outs, &v[i])) return nullptr;
+            if (i > 0 && (e.kinds[i - 1] == kMembers || e.kinds[i - 1] == kFactors) && v[i].i != listed) {
+                PyErr_Format(PyExc_ValueError, "%s: %zd structures for %lld", e.name, listed, static_cast<long long>(v[i].i));
+                return nullptr;
+            }
             continue;
         }
         if (arrays == 2) { PyErr_SetString(PyExc_ValueError, "call: too many arrays"); return nullptr; }
         std::vector<int64_t>& w = words[arrays++];
+        const Kind* layout = members ? kMember : kFactor;
+        const Py_ssize_t size = members ? sizeof(kMember) : sizeof(kFactor);
+        listed = PyList_GET_SIZE(o);
+        w.reserve(static_cast<size_t>(listed * size));
         for (Py_ssize_t k = 0; k < PyList_GET_SIZE(o); ++k) {
             PyObject* m = PyList_GET_ITEM(o, k);
-            if (!PyTuple_Check(m)) { PyErr_SetString(PyExc_TypeError, "call: a structure is a tuple of its words"); return nullptr; }
-            for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(m); ++j) {
+            if (!PyTuple_Check(m) || PyTuple_GET_SIZE(m) != size) {
+                PyErr_Format(PyExc_TypeError, "%s: a structure is a tuple of its %zd words", e.name, size);
+                return nullptr;
+            }
+            for (Py_ssize_t j = 0; j < size; ++j) {
                 Value x;
-                if (!value_of(PyTuple_GET_ITEM(m, j), outs, &x)) return nullptr;
-                if (x.is_float) { PyErr_SetString(PyExc_TypeError, "call: a structure's words are integers and addresses"); return nullptr; }
+                if (!value_of(PyTuple_GET_ITEM(m, j), layout[j], outs, &x)) return nullptr;
                 w.push_back(x.i);
             }
         }
-        v[i] = Value{static_cast<int64_t>(reinterpret_cast<uintptr_t>(w.data())), 0.0, false};
+        v[i].i = static_cast<int64_t>(reinterpret_cast<uintptr_t>(w.data()));
     }
-    if (!e.fits(v)) { PyErr_Format(PyExc_TypeError, "%s: a float for an integer or an address", e.name); return nullptr; }
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = e.run(v);
@@ -234,7 +282,6 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_metis_host", nullptr, -1, met
 
 PyMODINIT_FUNC PyInit__metis_host()
 {
-    static_assert(sizeof(metis_linear_member) == 12 * 8 && sizeof(metis_lowrank_factor) == 3 * 8, "structures of 64-bit words");
     PyObject* m = PyModule_Create(&module_def);
     g_index = PyDict_New();
     if (!m || !g_index) return nullptr;

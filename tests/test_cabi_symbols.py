@@ -1,18 +1,24 @@
 """The shared library loads without a GPU and exports every symbol include/metis_hip.h declares."""
+import ctypes
 import os
 import re
 
+import numpy as np
 import pytest
+import torch
 
 from metis_hip import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def _declared():
+def _header():
     text = open(os.path.join(ROOT, "include", "metis_hip.h")).read()
-    text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
-    return sorted(set(re.findall(r"\b(metis_[a-z0-9_]+)\s*\(", text)))
+    return re.sub(r"/\*.*?\*/", "", text, flags=re.S)
+
+
+def _declared():
+    return sorted(set(re.findall(r"\b(metis_[a-z0-9_]+)\s*\(", _header())))
 
 
 def test_every_declared_symbol_is_exported_and_bound():
@@ -71,3 +77,44 @@ def test_compiled_calls_take_the_arguments_that_the_abi_declares():
             _lib.call(name, 0, (), (0,) * (len(args) - 1) + ("0",))  # a new tensor that is not there
     with pytest.raises(ValueError):
         _lib.call("metis_rmsnorm", 0, ((7, 1),), (0,) * 7)
+
+
+def test_compiled_calls_take_every_argument_by_its_declared_kind():
+    """What ctypes refused for an integer, a float or an address is refused here too, what it took for one has the same value, and an array of
+    structures is as long as its number says.  (No call gets beyond the entry points' own argument checks.)"""
+    source = open(os.path.join(os.path.dirname(_lib.LIB_PATH), "..", "csrc", "host_calls.cpp")).read()
+    structures = {"metis_linear_member": 12, "metis_lowrank_factor": 3}
+    words = {kind: (None,) * 5 + (0, None, None, 0, 0, 0, None) if n == 12 else (None, None, 0) for kind, n in structures.items()}
+    header = _header()
+    for name in re.findall(r"METIS_ENTRY\((metis_\w+)\)", source):
+        declared = [" ".join(a.split()) for a in re.search(rf"\b{name}\(([^)]*)\)", header).group(1).split(",")]
+        types = _lib.SIGNATURES[name][1]
+        assert len(declared) == len(types)
+        arrays = {i: kind for i, a in enumerate(declared) for kind in structures if kind in a}
+        good = []
+        for i, t in enumerate(types):
+            good.append([words[arrays[i]]] if i in arrays else 1 if i - 1 in arrays else None if t is ctypes.c_void_p else 0.0 if t is ctypes.c_float else 0)
+
+        def call(i, value):
+            return _lib.call(name, 0, (), tuple(good[:i] + [value] + good[i + 1:]))
+
+        for i, t in enumerate(types):
+            if i in arrays:
+                bad = [None, 0, torch.zeros(4), (), "0", [()], [words[arrays[i]][1:]], [words[arrays[i]] + (0,)], [list(words[arrays[i]])]]
+                bad += [[words[arrays[i]][:k] + (0.5,) + words[arrays[i]][k + 1:]] for k in range(len(words[arrays[i]]))]
+                with pytest.raises(ValueError, match=f"{name}: 2 structures for 1"):
+                    call(i, [words[arrays[i]]] * 2)
+            elif t is ctypes.c_void_p:
+                bad = [0.5, np.int64(16), "00", "0", (), [words["metis_lowrank_factor"]]]
+            elif t is ctypes.c_float:
+                bad = [None, "1", torch.zeros(2), ()]
+            else:
+                bad = [None, 0.5, "1", torch.zeros(2, dtype=torch.int64), torch.tensor(0.5), (), [words["metis_lowrank_factor"]]]
+            for value in bad:
+                with pytest.raises((TypeError, ValueError, RuntimeError)):
+                    call(i, value)
+    # numbers of other libraries, and tensors that hold one: 33 columns are no whole blocks, 32 without a tensor are an argument error
+    row = "metis_nvfp4_quant_row"
+    for columns in (33, np.int64(33), np.uint8(33), torch.tensor(33), torch.tensor([33])):
+        assert _lib.call(row, 0, (), (None, 16, columns, 64, 0, None, None, None, None, 0, None)) == _lib.E_SHAPE
+    assert _lib.call(row, 0, (), (None, 16, 32, 64, 0, None, None, None, None, 0, None)) == _lib.E_ARG
