@@ -15,6 +15,7 @@
 #include <Python.h>
 #include <cstddef>
 #include <ATen/ops/empty.h>
+#include <c10/util/SmallVector.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <tuple>
@@ -199,18 +200,18 @@ PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n)
     if (count > static_cast<Py_ssize_t>(kMaxOuts)) { PyErr_SetString(PyExc_ValueError, "call: too many tensors"); return nullptr; }
     for (Py_ssize_t i = 0; i < count; ++i) {
         PyObject* s = PyTuple_GET_ITEM(a[2], i);
-        int64_t sizes[8];
+        c10::SmallVector<int64_t, 8> sizes;
         const Py_ssize_t dims = PyTuple_Check(s) ? PyTuple_GET_SIZE(s) - 1 : -1;
         const long type = dims >= 0 ? PyLong_AsLong(PyTuple_GET_ITEM(s, 0)) : -1;
-        if (dims < 0 || dims > 8 || type < 0 || type > 2) {
+        if (dims < 0 || type < 0 || type > 2) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "call: a spec is (0 | 1 | 2, size, ...)");
             return nullptr;
         }
         for (Py_ssize_t d = 0; d < dims; ++d) {
-            sizes[d] = PyLong_AsLongLong(PyTuple_GET_ITEM(s, d + 1));
-            if (sizes[d] == -1 && PyErr_Occurred()) return nullptr;
+            sizes.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(s, d + 1)));
+            if (sizes.back() == -1 && PyErr_Occurred()) return nullptr;
         }
-        at::Tensor t = at::empty(at::IntArrayRef(sizes, static_cast<size_t>(dims)),
+        at::Tensor t = at::empty(sizes,
                                  at::TensorOptions().dtype(types[type]).device(at::Device(at::kCUDA, static_cast<at::DeviceIndex>(device))));
         outs.at[outs.count] = static_cast<int64_t>(reinterpret_cast<uintptr_t>(t.data_ptr()));
         outs.obj[outs.count] = THPVariable_Wrap(std::move(t));

@@ -118,3 +118,9 @@ def test_compiled_calls_take_every_argument_by_its_declared_kind():
     for columns in (33, np.int64(33), np.uint8(33), torch.tensor(33), torch.tensor([33])):
         assert _lib.call(row, 0, (), (None, 16, columns, 64, 0, None, None, None, None, 0, None)) == _lib.E_SHAPE
     assert _lib.call(row, 0, (), (None, 16, 32, 64, 0, None, None, None, None, 0, None)) == _lib.E_ARG
+
+
+def test_compiled_calls_allocate_tensors_of_any_number_of_dimensions():
+    """(The device does not exist: the allocation itself fails, not what is asked of it.)"""
+    with pytest.raises(RuntimeError):
+        _lib.call("metis_nvfp4_roundtrip", 99, ((_lib.F32, *(1,) * 11, 16),), (None, 1, 16, 0, "0", None, 0, 0, None))

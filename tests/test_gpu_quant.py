@@ -789,6 +789,14 @@ def test_binary32_round_trip_from_one_call(ops, rows, cols):
     assert same_bits(q.quantize_dequantize(x).cpu(), out.cpu())
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_round_trip_of_a_tensor_of_many_dimensions(dt):
+    from metis_hip import quant_func
+    x = torch.randn(2, 3, *(1,) * 8, 32, generator=torch.Generator().manual_seed(3)).to(dt).cuda()
+    got = quant_func["nvfp4e2m1bnosr"].quantize_dequantize(x)
+    assert got.shape == x.shape and torch.equal(got.reshape(6, 32), quant_func["nvfp4e2m1bnosr"].quantize_dequantize(x.reshape(6, 32)))
+
+
 # one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (256 x 1024 elements in bf16, 144 x
 # 1024 in binary32), leading dimensions, four, eight and sixteen half blocks per thread, the last workgroup partly filled
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
