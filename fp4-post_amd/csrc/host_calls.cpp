@@ -7,13 +7,15 @@
 // each taken as the declaration in metis_hip.h says: for an integer whatever Python takes for an index (its low bits, as ctypes passes it), for a float
 // whatever has a float value, for an address None, a tensor, an integer or the new tensor at a text of one character's distance from "0", for an array of
 // structures (metis_linear_member, metis_lowrank_factor) a list of tuples of their 64-bit words, as many as the argument behind it says.  Anything else
-// is a TypeError or a ValueError.  The interpreter's lock is released during the call, as ctypes releases it.
+// is a TypeError or a ValueError, before anything is allocated.  The interpreter's lock is released for the allocations and the call, as torch.empty and
+// ctypes release it.
 //
 // Per call and new tensor the same through ctypes and torch.empty cost 5.1 and 1.7 us, here 3.9 and 1.0 (launch included): an eager decode step
 // of five sequences (hidden 1536, 19 launches, 46 new tensors) 415 -> 367 us, a prompt of 411 tokens 462 -> 410, a small round trip 8.2 -> 6.8.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <cstddef>
+#include <cstring>
 #include <ATen/ops/empty.h>
 #include <c10/util/SmallVector.h>
 #include <torch/csrc/Exceptions.h>
@@ -54,7 +56,7 @@ static_assert(sizeof(metis_linear_member) == sizeof(kMember) * 8 && offsetof(met
               offsetof(metis_linear_member, bias_is_f32) == 9 * 8 && offsetof(metis_linear_member, ldt) == 10 * 8, "kMember follows the declaration");
 static_assert(sizeof(metis_lowrank_factor) == sizeof(kFactor) * 8 && offsetof(metis_lowrank_factor, r) == 2 * 8, "kFactor follows the declaration");
 
-union Value {
+union Value {                                                  // (a float's bits lie in the word)
     int64_t i;
     double f;
 };
@@ -138,40 +140,45 @@ constexpr bool all_counted()
 static_assert(all_counted(), "at most kMaxArgs arguments, and a number behind every array of structures");
 PyObject* g_index = nullptr;                                   // name -> position in kEntries
 
+// the new tensors, and where their addresses go once they exist
 struct Outputs {
-    PyObject* obj[kMaxOuts];
-    int64_t at[kMaxOuts];
     size_t count = 0;
-    ~Outputs() { for (size_t i = 0; i < count; ++i) Py_XDECREF(obj[i]); }
+    c10::SmallVector<std::pair<int64_t*, size_t>, 16> at;
+};
+// The interpreter's lock given up: an allocation may wait for the device, or for memory that it has to get back first.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
 };
 
 // one argument or word of the given kind; false with a Python error set
-bool value_of(PyObject* o, Kind kind, const Outputs& outs, Value* v)
+bool value_of(PyObject* o, Kind kind, Outputs& outs, int64_t* v)
 {
     if (kind == kReal) {
-        v->f = PyFloat_AsDouble(o);
-        return !(v->f == -1.0 && PyErr_Occurred());
+        const double f = PyFloat_AsDouble(o);
+        memcpy(v, &f, sizeof f);
+        return !(f == -1.0 && PyErr_Occurred());
     }
     if ((kind == kInteger || kind == kAddress) && PyLong_Check(o)) {   // (also bool; 64-bit seeds may use the sign bit)
-        v->i = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(o));
-        return !(v->i == -1 && PyErr_Occurred());
+        *v = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(o));
+        return !(*v == -1 && PyErr_Occurred());
     }
     if (kind == kInteger) {
         PyObject* n = PyNumber_Index(o);
         if (!n) return false;
-        v->i = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(n));
+        *v = static_cast<int64_t>(PyLong_AsUnsignedLongLongMask(n));
         Py_DECREF(n);
-        return !(v->i == -1 && PyErr_Occurred());
+        return !(*v == -1 && PyErr_Occurred());
     }
     if (kind == kAddress) {
-        if (o == Py_None) { v->i = 0; return true; }
+        if (o == Py_None) { *v = 0; return true; }
         if (THPVariable_Check(o)) {
-            v->i = static_cast<int64_t>(reinterpret_cast<uintptr_t>(THPVariable_Unpack(o).data_ptr()));
+            *v = static_cast<int64_t>(reinterpret_cast<uintptr_t>(THPVariable_Unpack(o).data_ptr()));
             return true;
         }
         if (PyUnicode_Check(o) && PyUnicode_GET_LENGTH(o) == 1) {
             const int k = static_cast<int>(PyUnicode_READ_CHAR(o, 0)) - '0';
-            if (k >= 0 && static_cast<size_t>(k) < outs.count) { v->i = outs.at[k]; return true; }
+            if (k >= 0 && static_cast<size_t>(k) < outs.count) { outs.at.push_back({v, static_cast<size_t>(k)}); return true; }
         }
     }
     PyErr_Format(PyExc_TypeError, kind == kAddress ? "call: %s for an address" : "call: %s for a list of structures", Py_TYPE(o)->tp_name);
@@ -195,36 +202,33 @@ PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n)
     if (device == -1 && PyErr_Occurred()) return nullptr;
 
     static const at::ScalarType types[] = {at::kByte, at::kBFloat16, at::kFloat};
+    struct { at::ScalarType type; size_t begin, dims; } spec[kMaxOuts];
+    c10::SmallVector<int64_t, 64> sizes;
     Outputs outs;
     const Py_ssize_t count = PyTuple_GET_SIZE(a[2]);
     if (count > static_cast<Py_ssize_t>(kMaxOuts)) { PyErr_SetString(PyExc_ValueError, "call: too many tensors"); return nullptr; }
     for (Py_ssize_t i = 0; i < count; ++i) {
         PyObject* s = PyTuple_GET_ITEM(a[2], i);
-        c10::SmallVector<int64_t, 8> sizes;
         const Py_ssize_t dims = PyTuple_Check(s) ? PyTuple_GET_SIZE(s) - 1 : -1;
         const long type = dims >= 0 ? PyLong_AsLong(PyTuple_GET_ITEM(s, 0)) : -1;
         if (dims < 0 || type < 0 || type > 2) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "call: a spec is (0 | 1 | 2, size, ...)");
             return nullptr;
         }
+        spec[i] = {types[type], sizes.size(), static_cast<size_t>(dims)};
         for (Py_ssize_t d = 0; d < dims; ++d) {
             sizes.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(s, d + 1)));
             if (sizes.back() == -1 && PyErr_Occurred()) return nullptr;
         }
-        at::Tensor t = at::empty(sizes,
-                                 at::TensorOptions().dtype(types[type]).device(at::Device(at::kCUDA, static_cast<at::DeviceIndex>(device))));
-        outs.at[outs.count] = static_cast<int64_t>(reinterpret_cast<uintptr_t>(t.data_ptr()));
-        outs.obj[outs.count] = THPVariable_Wrap(std::move(t));
-        if (!outs.obj[outs.count]) return nullptr;
         ++outs.count;
     }
 
     Value v[kMaxArgs];
-    std::vector<int64_t> words[2];                             // arrays of structures; filled whole before their address is taken
+    std::vector<int64_t> words[2];                             // arrays of structures; never moved once their words are asked for
     size_t arrays = 0;
     Py_ssize_t listed = 0;                                     // structures of the last array
     const size_t given = static_cast<size_t>(PyTuple_GET_SIZE(a[3]));
-    if (given != e.args || given > kMaxArgs) {
+    if (given != e.args) {
         PyErr_Format(PyExc_TypeError, "%s takes %zu arguments (%zu given)", e.name, e.args, given);
         return nullptr;
     }
@@ -232,7 +236,7 @@ PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n)
         PyObject* o = PyTuple_GET_ITEM(a[3], static_cast<Py_ssize_t>(i));
         const bool members = e.kinds[i] == kMembers;
         if (!PyList_Check(o) || (!members && e.kinds[i] != kFactors)) {
-            if (!value_of(o, e.kinds[i], outs, &v[i])) return nullptr;
+            if (!value_of(o, e.kinds[i], outs, &v[i].i)) return nullptr;
             if (i > 0 && (e.kinds[i - 1] == kMembers || e.kinds[i - 1] == kFactors) && v[i].i != listed) {
                 PyErr_Format(PyExc_ValueError, "%s: %zd structures for %lld", e.name, listed, static_cast<long long>(v[i].i));
                 return nullptr;
@@ -244,31 +248,35 @@ PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n)
         const Kind* layout = members ? kMember : kFactor;
         const Py_ssize_t size = members ? sizeof(kMember) : sizeof(kFactor);
         listed = PyList_GET_SIZE(o);
-        w.reserve(static_cast<size_t>(listed * size));
-        for (Py_ssize_t k = 0; k < PyList_GET_SIZE(o); ++k) {
-            PyObject* m = PyList_GET_ITEM(o, k);
-            if (!PyTuple_Check(m) || PyTuple_GET_SIZE(m) != size) {
+        w.resize(static_cast<size_t>(listed * size));
+        for (Py_ssize_t k = 0; k < listed; ++k) {
+            PyObject* m = k < PyList_GET_SIZE(o) ? PyList_GET_ITEM(o, k) : nullptr;
+            if (!m || !PyTuple_Check(m) || PyTuple_GET_SIZE(m) != size) {
                 PyErr_Format(PyExc_TypeError, "%s: a structure is a tuple of its %zd words", e.name, size);
                 return nullptr;
             }
-            for (Py_ssize_t j = 0; j < size; ++j) {
-                Value x;
-                if (!value_of(PyTuple_GET_ITEM(m, j), layout[j], outs, &x)) return nullptr;
-                w.push_back(x.i);
-            }
+            for (Py_ssize_t j = 0; j < size; ++j)
+                if (!value_of(PyTuple_GET_ITEM(m, j), layout[j], outs, &w[static_cast<size_t>(k * size + j)])) return nullptr;
         }
         v[i].i = static_cast<int64_t>(reinterpret_cast<uintptr_t>(w.data()));
     }
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = e.run(v);
-    Py_END_ALLOW_THREADS
+    c10::SmallVector<at::Tensor, 8> fresh;
+    {
+        Unlocked unlocked;
+        const at::Device on(at::kCUDA, static_cast<at::DeviceIndex>(device));
+        for (Py_ssize_t i = 0; i < count; ++i)
+            fresh.push_back(at::empty(at::IntArrayRef(sizes.data() + spec[i].begin, spec[i].dims), at::TensorOptions().dtype(spec[i].type).device(on)));
+        for (const auto& at : outs.at) *at.first = static_cast<int64_t>(reinterpret_cast<uintptr_t>(fresh[at.second].data_ptr()));
+        rc = e.run(v);
+    }
     if (rc != METIS_OK) return PyLong_FromLong(rc);
     PyObject* result = PyTuple_New(count);
     if (!result) return nullptr;
     for (Py_ssize_t i = 0; i < count; ++i) {
-        PyTuple_SET_ITEM(result, i, outs.obj[i]);              // the reference moves into the tuple
-        outs.obj[i] = nullptr;
+        PyObject* t = THPVariable_Wrap(std::move(fresh[static_cast<size_t>(i)]));
+        if (!t) { Py_DECREF(result); return nullptr; }
+        PyTuple_SET_ITEM(result, i, t);                        // the reference moves into the tuple
     }
     return result;
     END_HANDLE_TH_ERRORS

@@ -2,6 +2,9 @@
 import ctypes
 import os
 import re
+import sys
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -124,3 +127,39 @@ def test_compiled_calls_allocate_tensors_of_any_number_of_dimensions():
     """(The device does not exist: the allocation itself fails, not what is asked of it.)"""
     with pytest.raises(RuntimeError):
         _lib.call("metis_nvfp4_roundtrip", 99, ((_lib.F32, *(1,) * 11, 16),), (None, 1, 16, 0, "0", None, 0, 0, None))
+
+
+def test_compiled_calls_give_up_the_interpreter_while_they_allocate():
+    """No thread is made to hand over the interpreter here, so another one runs only where the calls let it.  (The device does not exist: every
+    call ends in its allocation.)"""
+    args = ("metis_nvfp4_roundtrip", 99, ((_lib.F32, 1, 16),), (None, 1, 16, 0, "0", None, 0, 0, None))
+    turns, stop = [0], False
+
+    def other():
+        while not stop:
+            turns[0] += 1
+            time.sleep(0)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    with pytest.raises(RuntimeError):
+        _lib.call(*args)
+    sys.setswitchinterval(1000.0)
+    try:
+        thread.start()
+        while not turns[0]:
+            time.sleep(0.001)
+        before = turns[0]
+        for _ in range(20000):
+            try:
+                _lib.call(*args)
+            except RuntimeError:
+                pass
+            if turns[0] > before + 10:
+                break
+        ran = turns[0] - before
+    finally:
+        sys.setswitchinterval(interval)
+        stop = True
+        thread.join()
+    assert ran > 10
