@@ -361,8 +361,8 @@ class LinearLowbitFunction(torch.autograd.Function):
         if cached_count + rows > 2 ** 24:
             return None
         key, v = projection if projection is not None else (None, None)
-        tm = ops.TokenMean(after_norm, cached_mean, cached_count, v, True)
-        packed = ops.quantize(x2, ops.MODE_PB16, center=tm, deferred=True)
+        tm = ops.TokenMean(after_norm, cached_mean, cached_count, v)
+        packed = ops.quantize(x2, ops.MODE_PB16, center=tm, deferred=True, checked=True)
         if mean_cache is not None:
             mean_cache[cache_key] = (tm.mean.unsqueeze(0), cached_count + rows)
         return CenteredNVFP4(packed, tm.mean, tm.mean32, None if tm.pending is None else (key, tm.pending))

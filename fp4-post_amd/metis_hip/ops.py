@@ -275,7 +275,7 @@ def _as_2d_for_quant(x: torch.Tensor, mode: int) -> tuple[torch.Tensor, int]:
 def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bool = False,
              noise: torch.Tensor | None = None, seed: int = 0, offset: int = 0,
              center: torch.Tensor | TokenMean | None = None, resident: bool = False, spin_limit: int = 0,
-             deferred: bool = False, pad_rows: int | None = None) -> PackedNVFP4:
+             deferred: bool = False, pad_rows: int | None = None, checked: bool = False) -> PackedNVFP4:
     """NVFP4-quantize x (flattened to [R, C]).
 
     col=False: blocks of 16 along C -> PackedNVFP4 of shape (R, C).
@@ -284,7 +284,7 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
                overrides the internal Philox stream keyed by (seed, offset).
     center   : [C] vector subtracted from every row first (the reference's mean mode), in the arithmetic's
                dtype: the packed tensor is that of x - center.  A TokenMean: the column mean of x itself, formed in the
-               same launch and left in it (deferred, bf16 arithmetic, see token_mean_applies).
+               same launch and left in it (deferred, bf16 arithmetic, see token_mean_applies; checked: the caller has just asked it of x).
     resident : round-to-nearest rows of a bf16 tensor as ONE launch (metis_nvfp4_quant_row_resident), same bytes: a
                workgroup that gives up waiting for the grid's maximum after `spin_limit` polls (0: library default)
                leaves its scale bytes to the last workgroup.
@@ -298,7 +298,7 @@ def quantize(x: torch.Tensor, mode: int = MODE_P32, *, col: bool = False, sr: bo
     if isinstance(center, TokenMean):
         if not deferred or col or sr or kmode != MODE_PB16 or pad_rows is not None:
             raise ValueError("a TokenMean centre: bf16 arithmetic, rows, round to nearest, scale bytes deferred")
-        return _quantize_token_mean(x2, center)
+        return _quantize_token_mean(x2, center, checked and x2 is x)
     rows, cols = x2.shape
     if pad_rows is not None and pad_rows != rows:
         return _quantize_col_padded(x2, kmode, mode, pad_rows, col, sr, noise, seed, offset, center)
@@ -688,15 +688,14 @@ class TokenMean:
     cached: torch.Tensor | None = None
     cached_count: int = 0
     v: torch.Tensor | None = None
-    checked: bool = False                     # the caller has just asked token_mean_applies
     # results
     mean: torch.Tensor | None = None
     mean32: torch.Tensor | None = None
     pending: torch.Tensor | None = None
 
 
-def _quantize_token_mean(x2: torch.Tensor, tm: TokenMean) -> PackedNVFP4:
-    if not (tm.checked or token_mean_applies(x2, tm.after_norm)):
+def _quantize_token_mean(x2: torch.Tensor, tm: TokenMean, checked: bool) -> PackedNVFP4:
+    if not (checked or token_mean_applies(x2, tm.after_norm)):
         raise ValueError("a TokenMean centre: outside the call's domain (see token_mean_applies)")
     after_norm, cached, cached_count, v = tm.after_norm, tm.cached, tm.cached_count, tm.v
     rows, cols = x2.shape

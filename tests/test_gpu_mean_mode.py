@@ -728,6 +728,19 @@ def test_mean_and_centred_packing_of_few_tokens_in_one_launch(rows, cols):
                 assert all(torch.equal(l, r) for l, r in zip(a, b))
 
 
+def test_a_token_mean_asks_of_every_tensor_whether_its_launch_takes_it():
+    """The answer belongs to a call: the same TokenMean with a tensor of too many rows, or of another alignment, is refused."""
+    from metis_hip import ops
+    x = torch.randn(64, 256, generator=torch.Generator().manual_seed(2)).bfloat16().cuda()
+    tm = ops.TokenMean()
+    assert ops.token_mean_applies(x, False)
+    p = ops.quantize(x, ops.MODE_PB16, center=tm, deferred=True, checked=True)
+    assert torch.equal(p.codes, ops.quantize(x, ops.MODE_PB16, center=tm.mean).codes)
+    for bad in (torch.zeros(ops.TOKEN_MEAN_MAX_ROWS + 1, 256, dtype=torch.bfloat16, device="cuda"), torch.zeros(64 * 256 + 8, dtype=torch.bfloat16, device="cuda")[4:-4].view(64, 256)):
+        with pytest.raises(ValueError, match="outside the call's domain"):
+            ops.quantize(bad, ops.MODE_PB16, center=tm, deferred=True)
+
+
 def test_running_mean_of_decode_steps_through_the_one_launch_path():
     """A BitLinear under the default arguments: prompt, then decode steps; the cache holds what the separate kernels would keep."""
     from metis_hip import BitLinear, MetisArgs, ops
