@@ -194,13 +194,13 @@ def _column_mean_bytes(cols: int) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
-def _rmsnorm_colmean_bytes(rows: int, cols: int) -> int:
-    return max(int(load().metis_rmsnorm_colmean_workspace_bytes(rows, cols)), 16)
+def _rmsnorm_colmean_bytes(rows: int, cols: int, device_index: int) -> int:
+    return max(int(load().metis_rmsnorm_colmean_workspace_bytes(rows, cols)), 16)        # depends on the device's CU count only
 
 
 @functools.lru_cache(maxsize=4096)
-def _rmsnorm_backward_bytes(rows: int, cols: int) -> int:
-    return int(load().metis_rmsnorm_backward_workspace_bytes(rows, cols))
+def _rmsnorm_backward_bytes(rows: int, cols: int, device_index: int) -> int:
+    return int(load().metis_rmsnorm_backward_workspace_bytes(rows, cols))                # likewise
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1226,7 +1226,7 @@ def rmsnorm_colmean(x: torch.Tensor, gamma: torch.Tensor, eps: float, mean_dtype
     dev = x2.device
     g = gamma.to(device=dev, dtype=torch.bfloat16).contiguous()
     f32 = mean_dtype == torch.float32
-    size = _rmsnorm_colmean_bytes(rows, cols)
+    size = _rmsnorm_colmean_bytes(rows, cols, dev.index or 0)
     if cached is not None:
         cached = cached.reshape(-1).to(device=dev, dtype=mean_dtype).contiguous()
         if cached.numel() != cols:
@@ -1258,7 +1258,7 @@ def rmsnorm_backward(x: torch.Tensor, g: torch.Tensor, gamma: torch.Tensor, eps:
     x2, g2 = dense(x, cols), dense(g, cols)
     gm = dense(gamma, cols)
     rows = x2.shape[0]
-    need = _rmsnorm_backward_bytes(rows, cols) if want_gamma else 0
+    need = _rmsnorm_backward_bytes(rows, cols, x.device.index or 0) if want_gamma else 0
     specs = ((B16, rows, cols), (B16, cols), (U8, need)) if want_gamma else ((B16, rows, cols),)
     new = _lib.call("metis_rmsnorm_backward", x.device.index, specs,
                     (x2, g2, gm, float(eps), rows, cols, "0", "1" if want_gamma else None, DTYPE_BF16, "2" if want_gamma else None, need, _stream()))
@@ -1305,7 +1305,7 @@ def _grouped_plan(M: int, K: int, ns: tuple, device_index: int) -> tuple[int, bo
 
 
 @functools.lru_cache(maxsize=4096)
-def _grouped_centre_fits_unsplit(M: int, K: int, ns: tuple) -> bool:
+def _grouped_centre_fits_unsplit(M: int, K: int, ns: tuple, device_index: int) -> bool:
     arr = (_lib.LinearMember * len(ns))()
     for i, n in enumerate(ns):
         arr[i].N = n
@@ -1751,7 +1751,7 @@ def _linear_fwd_grouped(a: PackedNVFP4, members, out_dtype: torch.dtype = torch.
     words, specs = _grouped_members(members, M, K, out_dtype, takes and M < 256 and decode_layout_weights)
     # split-K scratch (long K, few columns) and whether a centre fits the launch: functions of the shape alone
     ns = tuple(m[0].rows for m in members)
-    need, centre_ok = _grouped_plan(M, K, ns, dev.index or 0) if split_k else (0, _grouped_centre_fits_unsplit(M, K, ns))
+    need, centre_ok = _grouped_plan(M, K, ns, dev.index or 0) if split_k else (0, _grouped_centre_fits_unsplit(M, K, ns, dev.index or 0))
     dt = DTYPE_F32 if out_dtype == torch.float32 else DTYPE_BF16
     if rotate is not None:
         op_mode = MODE_PB16 if rounded else MODE_P32          # (nv_operand_mode: what a caller that brings a_operand built it in)

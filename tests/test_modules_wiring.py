@@ -505,3 +505,22 @@ def test_scratch_made_under_capture_is_handed_to_nobody_else(monkeypatch):
     capturing = False
     assert ops._workspace(64, 64, cpu) is kept
     assert ops._workspace(64, 64, cpu, tensors=2).data_ptr() not in (kept.data_ptr(), pair.data_ptr())   # (two packings: an area of their own)
+
+
+@pytest.mark.parametrize("size,shape,entry", [("_rmsnorm_colmean_bytes", (64, 512), "metis_rmsnorm_colmean_workspace_bytes"),
+                                              ("_rmsnorm_backward_bytes", (64, 512), "metis_rmsnorm_backward_workspace_bytes"),
+                                              ("_lowrank_backward_bytes", (64, 512, 512, 32), "metis_lowrank_backward_workspace_bytes"),
+                                              ("_grouped_centre_fits_unsplit", (64, 512, (96, 32)), "metis_linear_grouped_centered_supported")])
+def test_sizes_that_follow_a_device_are_kept_for_each_device(monkeypatch, size, shape, entry):
+    """A device with more compute units asks for more scratch (and splits other shapes): what one was told is not another's answer."""
+    from metis_hip import ops
+    units = 1
+    monkeypatch.setattr(ops, "load", lambda: SimpleNamespace(**{entry: lambda *a: 1024 * units if entry.endswith("_bytes") else units - 1}))
+    ask = getattr(ops, size)
+    ask.cache_clear()
+    try:
+        first = ask(*shape, 0)
+        units = 2
+        assert ask(*shape, 0) == first and ask(*shape, 1) != first
+    finally:
+        ask.cache_clear()
