@@ -2,6 +2,7 @@
 import ctypes
 import os
 import re
+import subprocess
 import sys
 import threading
 import time
@@ -163,3 +164,13 @@ def test_compiled_calls_give_up_the_interpreter_while_they_allocate():
         stop = True
         thread.join()
     assert ran > 10
+
+
+def test_the_library_builds_without_torch():
+    """What `make` would run: the library and the probes for any interpreter, Python's way into the library for the one that has torch."""
+    csrc = os.path.join(os.path.dirname(_lib.LIB_PATH), "..", "csrc")
+    for python, has_torch in ((sys.executable, True), (f"{sys.executable} -S -I", False), ("no-such-interpreter", False)):
+        run = subprocess.run(["make", "-B", "-n", "-C", csrc, f"PYTHON={python}"], capture_output=True, text=True)
+        assert run.returncode == 0, run.stderr
+        assert "libmetis_hip.so" in run.stdout and "libmetis_ceilings.so" in run.stdout
+        assert ("host_calls.cpp" in run.stdout) == has_torch
