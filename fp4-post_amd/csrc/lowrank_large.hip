@@ -692,31 +692,36 @@ __global__ __launch_bounds__(256) void lowrank_tn_kernel(const TnProblem p0, con
 // that a wave reads whole lines of the partial sums; transposed, a workgroup turns its columns through LDS and writes 32 or 64 bytes (bf16)
 // of a row at a time.  (The lanes over the output's columns fetched 16 bytes of every line, and each line once per quad of r.)  What bounds
 // it is what a compute unit takes in and one round trip to the memory behind the slices' L2s: eight slices are requested together.
-// With the launch before it, both contractions of a layer, tokens x N, K, R, before | now: 4096 x 1536, 8960, 32 32.4 | 25.0 us, 4096 x 8960,
-// 1536, 32 27.3 | 25.6, 2103 x 3584, 18944, 64 44.6 | 31.1, 2103 x 18944, 3584, 64 35.0 | 32.0, 8192 x 4096, 4096, 64 47.9 | 45.7, 1000 x 2048,
-// 2568, 128 20.7 | 17.0.  From a rank of 64 on 32 columns to a workgroup leave compute units idle: 31.1, 34.3, 49.5, 18.7.
+// With the launch before it, both contractions of a layer, tokens x N, K, R, lanes over the output's columns | now: 4096 x 1536, 8960, 32 33.2 | 23.1 us,
+// 4096 x 8960, 1536, 32 28.0 | 23.5, 2103 x 3584, 18944, 64 46.3 | 32.7, 2103 x 18944, 3584, 64 36.5 | 33.0, 8192 x 4096, 4096, 64 49.3 | 45.3,
+// 1000 x 2048, 2568, 128 21.6 | 17.1, 411 x 1536, 8960, 64 14.7 | 11.0.  From a rank of 64 on 32 columns to a workgroup leave compute units idle.
+// No load stands under a condition of its lane's (a lane past the end reads the last quad), and none of a whole batch under any: the eight would wait
+// for each other.  One contraction, the loads of live lanes under their condition | now: 4608 x 1536, R = 32 (18 slices) 13.0 | 9.4 us, 20000 x 64,
+// R = 64 (63) 26.7 | 11.9, 20000 x 256, R = 128 transposed (63) 45.7 | 23.3; 2103 x 3584, R = 64 (7) 13.6 | 12.8.
 template <int N, int BATCH>
-__device__ __forceinline__ void tn_sum_slices(const TnProblem& p, const float* const (&src)[N], const bool (&live)[N], int64_t CR, float4 (&sum)[N])
+__device__ __forceinline__ void tn_sum_slices(const TnProblem& p, const float* const (&src)[N], int64_t CR, float4 (&sum)[N])
 {
+    const int slices = p.slices;
 #pragma unroll
-    for (int u = 0; u < N; ++u) sum[u] = live[u] ? *reinterpret_cast<const float4*>(src[u]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int z0 = 1; z0 < p.slices; z0 += BATCH) {
+    for (int u = 0; u < N; ++u) sum[u] = *reinterpret_cast<const float4*>(src[u]);
+    auto add = [&](int z0, auto in) {                            // in(i): there is a slice z0 + i
         float4 v[BATCH][N];
 #pragma unroll
         for (int i = 0; i < BATCH; ++i)
-            if (z0 + i < p.slices) {
+            if (in(i)) {
 #pragma unroll
-                for (int u = 0; u < N; ++u)
-                    if (live[u]) v[i][u] = *reinterpret_cast<const float4*>(src[u] + (int64_t)(z0 + i) * CR);
+                for (int u = 0; u < N; ++u) v[i][u] = *reinterpret_cast<const float4*>(src[u] + (int64_t)(z0 + i) * CR);
             }
 #pragma unroll
         for (int i = 0; i < BATCH; ++i)
-            if (z0 + i < p.slices) {
+            if (in(i)) {
 #pragma unroll
-                for (int u = 0; u < N; ++u)
-                    if (live[u]) { sum[u].x += v[i][u].x; sum[u].y += v[i][u].y; sum[u].z += v[i][u].z; sum[u].w += v[i][u].w; }
+                for (int u = 0; u < N; ++u) { sum[u].x += v[i][u].x; sum[u].y += v[i][u].y; sum[u].z += v[i][u].z; sum[u].w += v[i][u].w; }
             }
-    }
+    };
+    int z0 = 1;
+    for (; z0 + BATCH <= slices; z0 += BATCH) add(z0, [](int) { return true; });
+    if (z0 < slices) add(z0, [&](int i) { return z0 + i < slices; });
 }
 __device__ __forceinline__ void tn_store_quad(const TnProblem& p, int64_t o, const float4 f)    // four consecutive elements of the output
 {
@@ -741,24 +746,21 @@ __global__ __launch_bounds__(256) void lowrank_tn_finish_kernel(const TnProblem 
     const int64_t CR = (int64_t)p.C * R;
     if (!p.transpose) {
         const int64_t o = ((int64_t)block * 256 + tid) * 4;
-        const float* const src[1] = {p.part + o};
-        const bool live[1] = {o < CR};
+        const float* const src[1] = {p.part + (o < CR ? o : CR - 4)};
         float4 sum[1];
-        tn_sum_slices<1, 8>(p, src, live, CR, sum);
-        if (live[0]) tn_store_quad(p, o, sum[0]);
+        tn_sum_slices<1, 8>(p, src, CR, sum);
+        if (o < CR) tn_store_quad(p, o, sum[0]);
         return;
     }
     const int64_t c0 = (int64_t)block * TN_TURN;
     const float* src[Q];
-    bool live[Q];
     float4 sum[Q];
 #pragma unroll
     for (int u = 0; u < Q; ++u) {
         const int64_t o = c0 * R + (int64_t)(u * 256 + tid) * 4;     // (the columns of a workgroup are one piece of each slice)
-        src[u] = p.part + o;
-        live[u] = o < CR;
+        src[u] = p.part + (o < CR ? o : CR - 4);
     }
-    tn_sum_slices<Q, 8 / Q>(p, src, live, CR, sum);
+    tn_sum_slices<Q, 8>(p, src, CR, sum);
 #pragma unroll
     for (int u = 0; u < Q; ++u) {
         const int c = (u * 256 + tid) / (R / 4), r = (u * 256 + tid) % (R / 4) * 4;

@@ -985,6 +985,19 @@ def test_token_contractions_in_both_layouts_at_the_edges_of_a_turned_piece(L, C,
             assert torch.equal(got, (want.T if transpose else want).to(dt)), (dt, transpose)
 
 
+@pytest.mark.parametrize("R", [32, 64, 128])
+@pytest.mark.parametrize("L,C", [(2048, 8), (2304, 72), (2560, 40), (4352, 24), (20000, 64)])
+def test_token_contractions_of_whole_and_partial_batches_of_slices(L, C, R):
+    """8, 9, 10, 17 and 63 slices of the tokens, eight of which are requested together, and lanes past the last quad: small whole numbers again."""
+    from metis_hip import ops
+    g = torch.Generator().manual_seed(R + L)
+    a, b = (torch.randint(-8, 9, (L, n), generator=g).bfloat16() for n in (C, R))
+    want = a.double().T @ b.double()
+    for transpose in (False, True):
+        got = ops.lowrank_contract_tokens(a.cuda(), b.cuda(), torch.float32, transpose).cpu()
+        assert torch.equal(got, (want.T if transpose else want).float())
+
+
 @pytest.mark.parametrize("L,R", [(1, 8), (255, 40), (257, 32), (2047, 32), (2049, 8), (4096, 32), (5000, 64)])
 def test_gradient_of_the_rank_r_scale_vector_is_added_in_its_documented_order(L, R):
     """256 sums of every 256th row, in row order, then these in order: binary32 on the CPU in that order gives the same bits."""
