@@ -80,7 +80,8 @@ __device__ __forceinline__ const uint16_t* nt_v(const NtFactors& f, int col, int
 constexpr int NT_ROTATE = 5;
 __device__ __forceinline__ int nt_first_step(int b, int steps) { return (int)((unsigned)b * NT_ROTATE % (unsigned)steps); }
 // The row tiles at the places `at` and `at + 1` of all `tiles`, ordered by the step that they start at; that step of the first, and
-// how many steps later the second starts.  An odd one out is returned twice.
+// how many steps later the second starts: none within a class, between neighbouring classes one, or five where 5 divides `steps` (up to five where
+// some classes are empty).  An odd one out is returned twice.
 // Tiles b and b + p start alike, with p = steps or, if 5 divides it, steps / 5; tiles = a p + e: the p classes have a members, the
 // first e of them one more.  Class c = i / 5 (mod p; or i itself) is the i-th in the order; a lane looks at one class.
 __device__ __forceinline__ void nt_pair(int at, int tiles, int steps, int* tile0, int* tile1, int* rot, int* lag)
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(TILES * NT_ROWS * KS / 16) void lowrank_nt_kernel(
     // that depends on the tile, the same for every call.  (An offset of 5 steps per tile: 8192 x 4096 from flushed caches 31 us,
     // 39 without; other row lengths within 2 %.)
     // Two row tiles: they share the walk and the pieces of v, and each keeps its own order.  nt_pair picks tiles that start at the
-    // same step or at neighbouring ones; the second then joins `lag` steps after the first and goes on as long after it.
+    // same step or `lag` (at most five) steps apart; the second then joins that much after the first and goes on as long after it.
     int tile0 = (int)blockIdx.x, tile1 = (int)blockIdx.x, rot = 0, lag = 0;
     if constexpr (TILES == 2) nt_pair(2 * (int)blockIdx.x, (M + NT_ROWS - 1) / NT_ROWS, wide_steps, &tile0, &tile1, &rot, &lag);
     else rot = wide_steps > 0 ? nt_first_step(tile0, wide_steps) : 0;
@@ -406,6 +407,34 @@ size_t lowrank_nt_workspace_bytes(int64_t M, int64_t R, int64_t K)
     return sl > 1 ? (size_t)sl * M * R * 4 : 0;
 }
 
+// Whether the row tiles go in pairs (stages of 128 k, three, from 192 columns on two), which fetch v half as often.  Only where single tiles would
+// share compute units, and where a pair's walk is not much longer than a tile's: the workgroup whose two tiles start `lag` steps apart ends the
+// launch.  They pay where x no longer fits the memory-side cache, or V's pieces are most of what a unit takes in.  Microseconds, single | pairs, on
+// an x just read and, after the dash, on one from HBM; lags in brackets where there is one:
+//   R = 192  16384 x 3584 50 | 44 - 94 | 80, 8704 x 2048 (1 of 8) 35 | 30 - 54 | 50, 8225 x 3840 51 | 44 - 96 | 77, 8225 x 5120 (5 of 20) 62 | 61 - 116 | 101;
+//            8225 x 2560 (5 of 10) 38 | 41 - 70 | 66, 8225 x 320 (1 of 2) 18.0 | 18.6, 8225 x 128 14.4 | 15.3
+//   R = 256  16384 x 3584 61 | 54 - 112 | 87, 8704 x 1536 (1 of 6) 34 | 32 - 57 | 49;  16384 x 1024 31 | 33, 16384 x 320 25 | 28, 12345 x 2560 (5 of 10) 50 | 55
+//   R = 128  16384 x 3584 35.3 | 34.5 - 72 | 65, 8225 x 3072 (1 of 12) 29.5 | 28.8 - 56 | 49, 8225 x 7680 (5 of 30) 63 | 60 - 117 | 98, 16384 x 5120 47 | 44 - 98 | 88;
+//            rows of whole 4 KiB 8225 x 4096 33.2 | 34.9, 16384 x 2048 24.1 | 24.8, 8225 x 8192 56 | 58; short ones 8704 x 1536 (1 of 6) 19.3 | 19.9,
+//            16384 x 1024 17.6 | 18.3; lags 10240 x 3840 (5 of 15) 37 | 39, 12345 x 5120 (5 of 20) 46.6 | 47.8
+//   beyond 120 M elements  R = 128 16384 x 8960 106 | 87 - 152 | 140, R = 96 8225 x 14592 126 | 91 - 186 | 144, R = 64 12000 x 18944 143 | 121 - 191 | 169;
+//            16384 x 7680 (5 of 30) R = 96 59.6 | 63.3, R = 64 46.6 | 47.0; below 120 M, R = 64 16384 x 6400 41 | 43
+//   R = 32   10240 x 14336 73 | 66 - 138 | 124, 16384 x 8960 59 | 55;  8225 x 14592 49 | 57, 9000 x 14336 52 | 54, 16384 x 6400 35 | 40
+//   with the quantizer, R = 64: 8225 x 14592 150 | 127 - 190 | 162, 16384 x 18944 247 | 213 - 288 | 247;  R = 32 8225 x 18944 142 | 156 - 186 | 180,
+//            16384 x 8960 94 | 102 - 139 | 143, 12000 x 18944 165 | 169 - 210 | 201
+static bool nt_pairs(int64_t tiles, int64_t M, int64_t R, int64_t K, bool quantizes)
+{
+    if (tiles <= device_cus() || K > 1 << 20) return false;
+    const int64_t steps = (K + 255) / 256;
+    const bool fives = steps % NT_ROTATE == 0;
+    const int64_t p = fives ? steps / NT_ROTATE : steps;         // classes of tiles that start alike (nt_pair)
+    const int64_t lag = p == 1 || tiles % (2 * p) == 0 ? 0 : fives || tiles < p ? NT_ROTATE : 1;
+    if (R == 32 && quantizes) return false;
+    if (M * K > (R == 32 ? 140000000 : 120000000) && 7 * lag <= steps) return true;
+    if (R >= 192) return K > 1024 && 3 * lag <= steps;
+    return R == 128 && K > 2560 && K % 2048 != 0 && 6 * lag <= steps;
+}
+
 // Columns per workgroup without the quantizer, for `groups` workgroups per column range.  Where these leave compute units
 // idle, the time is that of one workgroup's stages, and a stage of R columns takes the longer the more of v it fetches and
 // multiplies (and the wide forms' rings hold only two of them): workgroups of 32 or 64 columns side by side (gridDim.z) read x
@@ -494,26 +523,19 @@ int lowrank_nt_grouped(const void* x, int64_t ldx, int64_t M, int64_t K, const L
     // 192 columns on V's share outweighs that (16384 x 18944 433 | 361).
     //   with the quantizer, R = 64, three | two stages of 128 k: 411 x 1536 12.8 | 11.7, 16384 x 3584 33.4 | 31.7; three where a compute
     //   unit has one workgroup and x comes from HBM: 8192 x 14336 91 | 105
-    // Pairs of row tiles (stages of 128 k, three, from 192 columns on two) fetch v half as often.  They pay where single tiles would
-    // share compute units and V's pieces are most of what a unit takes in, or x comes from HBM.  Microseconds, single | pairs, with x in
-    // the memory-side cache and, after the dash, from HBM:
-    //   R = 192  16384 x 3584 52.9 | 48.5 - 88.8 | 74.2, 9000 x 4096 52 | 47 - 79 | 72, 16384 x 18944 - 380 | 327;  8192 x 4096 (256 tiles) 42 | 42
-    //   R = 256  16384 x 3584 65.5 | 58.5 - 106 | 82;   R = 128  16384 x 3584 37.6 | 36.9 - 66 | 59, 16384 x 8960 110 | 86 - 147 | 131
-    //   R = 96   16384 x 3584 35.4 | 37.3 - 61 | 57, 16384 x 8960 100 | 78 - 138 | 126
-    //   R = 64   16384 x 3584 25 | 25 - 53 | 52, 16384 x 6400 41 | 43 - 91 | 90, 12000 x 18944 140 | 114 - 184 | 159;  R = 32  16384 x 6400 35 | 40
-    //   with the quantizer, R = 64: 16384 x 3584 38 | 44 - 68 | 66, 9000 x 14336 145 | 123 - 175 | 150, 16384 x 18944 248 | 205 - 282 | 240
     const int64_t tiles = (M + NT_ROWS - 1) / NT_ROWS, groups = tiles * slices;
     const bool tail = K % 256 != 0, shared = groups > device_cus() && (R > 128 || M * K <= (int64_t)1 << 27);
-    const bool pairs = slices == 1 && tiles > device_cus() && (R >= 128 || M * K > 120000000) && K <= 1 << 20;
+    const bool pairs = slices == 1 && nt_pairs(tiles, M, R, K, qmode >= 0);
 #define METIS_NT(T, RT, Q, KS, NS) do { if (tail) rc = launch_nt<T, RT, Q, KS, NS, true>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); \
                                         else rc = launch_nt<T, RT, Q, KS, NS, false>(slices, st, x, ldx, fac, xv, t, M, R, K, part, codes, q.amax, q.gmax); } while (0)
 #define METIS_NTS(RT, NS, NS64) do { if (pairs) METIS_NT(2, RT, -1, 128, NS); else if (shared) METIS_NT(1, RT, -1, 64, NS64); else METIS_NT(1, RT, -1, 128, NS); } while (0)
     const int width = qmode < 0 ? nt_column_group(groups, R) : (int)R;
     const bool deep = groups <= device_cus() && M * K >= 100000000;
-#define METIS_NTQ(RT, Q) do { if (pairs) METIS_NT(2, RT, Q, 128, 3); else if (deep) METIS_NT(1, RT, Q, 128, 3); else METIS_NT(1, RT, Q, 128, 2); } while (0)
+#define METIS_NTQ1(RT, Q) do { if (deep) METIS_NT(1, RT, Q, 128, 3); else METIS_NT(1, RT, Q, 128, 2); } while (0)
+#define METIS_NTQ(RT, Q) do { if (pairs) METIS_NT(2, RT, Q, 128, 3); else METIS_NTQ1(RT, Q); } while (0)
 #define METIS_NTC(RT) do { if (pairs) METIS_NT(2, RT, -1, 128, 3); else METIS_NT(1, RT, -1, 128, 3); } while (0)
-    if (qmode == METIS_MODE_P32) { if (R == 32) METIS_NTQ(1, 0); else METIS_NTQ(2, 0); }
-    else if (qmode >= 0) { if (R == 32) METIS_NTQ(1, 1); else METIS_NTQ(2, 1); }
+    if (qmode == METIS_MODE_P32) { if (R == 32) METIS_NTQ1(1, 0); else METIS_NTQ(2, 0); }
+    else if (qmode >= 0) { if (R == 32) METIS_NTQ1(1, 1); else METIS_NTQ(2, 1); }
     else if (width == 32) METIS_NTC(1);
     else if (width == 64) METIS_NTC(2);
     else if (width == 96) METIS_NTS(3, 3, 4);
@@ -523,6 +545,7 @@ int lowrank_nt_grouped(const void* x, int64_t ldx, int64_t M, int64_t K, const L
 #undef METIS_NTC
 #undef METIS_NTS
 #undef METIS_NTQ
+#undef METIS_NTQ1
 #undef METIS_NT
     if (rc) return rc;
     if (hipGetLastError() != hipSuccess) return METIS_E_LAUNCH;

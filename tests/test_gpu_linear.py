@@ -825,6 +825,33 @@ def test_pairs_of_row_tiles_add_in_the_documented_order(M, R, K):
             assert torch.equal(qxv, xv) and torch.equal(qt, t)
 
 
+@pytest.mark.parametrize("M,R,K", [(8225, 192, 1088), (8225, 256, 1536), (8230, 192, 3840), (8300, 192, 3840), (8225, 128, 3136), (8225, 128, 7680), (8193, 192, 3584), (10240, 32, 14336), (8225, 64, 14592)])
+def test_pairs_of_row_tiles_that_start_any_number_of_steps_apart(M, R, K):
+    """Sizes whose tiles do go in pairs: all of a pair's start together, or some a step or five steps apart; one tile left over, K that ends in half a
+    step."""
+    test_pairs_of_row_tiles_add_in_the_documented_order(M, R, K)
+
+
+@pytest.mark.parametrize("M,R,K", [(8225, 192, 3584), (8300, 192, 3840), (8225, 192, 1088), (16384, 192, 3584), (8225, 128, 7680), (8225, 128, 1536), (8225, 64, 320), (300, 96, 320)])
+def test_one_infinity_in_v_stays_in_its_column(M, R, K):
+    """Pairs of row tiles that do and do not start together, single ones, a cut last step: what a tile's walk steps over is no part of its sums, so the
+    column is the infinity's sign times x's there, NaN where x is 0, and the others are what they are without it."""
+    from metis_hip import ops
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    v, s = torch.randn(R, K, generator=g, device="cuda").bfloat16(), (torch.rand(R, generator=g, device="cuda") + 0.5).bfloat16()
+    x[::7, K - 40] = 0
+    vs, ss = v.split(R // 2 if R % 64 == 0 else R), s.split(R // 2 if R % 64 == 0 else R)
+    project = lambda: ops.lowrank_project(x, ops.FactorStack(vs), ops.FactorStack(ss)) if ops.lowrank_stack_applies(x, list(zip(vs, ss))) else ops.lowrank_project(x, v, s)
+    without, _ = project()
+    v[R - 3, K - 40] = float("inf")
+    xv, t = project()
+    want = without.clone()
+    want[:, R - 3] = x[:, K - 40] * float("inf")
+    assert torch.equal(torch.nan_to_num(xv, 7.0), torch.nan_to_num(want, 7.0)) and torch.equal(xv.isnan(), want.isnan())
+    assert torch.equal(torch.nan_to_num(t, 7.0), torch.nan_to_num(want * s, 7.0))
+
+
 @pytest.mark.parametrize("R", [96, 192, 256])
 def test_wide_ranks_take_what_the_library_product_took(R):
     """Ranks 96, 192 and 256 from 256 rows on: an unaligned V, rows that overlap, operands that autograd records and large products
