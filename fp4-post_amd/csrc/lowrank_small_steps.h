@@ -94,14 +94,20 @@ __device__ __forceinline__ void lowrank_small_partial_wave(int chunk, int mtile,
 // (wide) four waves of 64 rows x 32 columns that share the rows' lines.  Microseconds with the quantizer, wide | single: 64 x 3584, R = 64
 // 3.3 | 2.8, R = 128 4.3 | 3.0, 64 x 18944, R = 64 4.9 | 4.0, 5 x 18944, R = 128 4.5 | 3.2, 128 x 3584, R = 128 4.6 | 3.7, 128 x 8960, R = 128 6.1 | 5.2,
 // 255 x 8960, R = 64 6.2 | 5.7, 192 x 18944, R = 32 5.7 | 5.6; where the compute units have more than ten steps of tiles each, re-reading V costs
-// more: 192 x 8960, R = 128 6.6 | 8.3, 255 x 18944, R = 64 9.0 | 11.9.  (64 rows and fewer: 64 x 18944, R = 128 7.2 | 5.6.)
-inline bool lowrank_small_wide(int64_t M, int64_t R, int64_t K, int cus)
-{
-    return M > 64 && (M + 31) / 32 * (R / 32) * (K / 64) > 10 * (int64_t)cus;
-}
+// more: 192 x 8960, R = 128 6.6 | 8.3, 255 x 18944, R = 64 9.0 | 11.9.  (64 rows and fewer: 64 x 18944, R = 128 7.2 | 5.6.)  From five steps on it
+// does so too where the wide workgroups fill one round of the compute units: 192 x 5120, R = 128 (240 of 256) 6.1 | 6.6, R = 96 5.3 | 5.4, 128 x 14336,
+// R = 64 (224) 5.4 | 5.7, 255 x 3584, R = 96 (224) 5.1 | 5.4; but 192 x 3584, R = 128 (168) 5.5 | 5.2, 224 x 5120, R = 128 (320) 7.5 | 7.1, R = 32
+// (one wave in four) 128 x 18944 (198) 5.4 | 5.1, 96 x 14336, R = 96 (224, half of their second rows empty) 6.0 | 5.7.
 inline int lowrank_small_partial_blocks(int64_t M, int64_t R, int chunks, bool wide)
 {
     return chunks * (int)(wide ? (M + 63) / 64 * ((R + 127) / 128) : (M + 31) / 32 * (R / 32));
+}
+inline bool lowrank_small_wide(int64_t M, int64_t R, int64_t K, int cus)
+{
+    const int64_t steps = (M + 31) / 32 * (R / 32) * (K / 64);
+    int kc;
+    const int blocks = lowrank_small_partial_blocks(M, R, lowrank_small_chunks(K, &kc), true);
+    return M > 64 && (steps > 10 * (int64_t)cus || (M > 96 && R > 32 && steps >= 5 * (int64_t)cus && blocks > cus * 3 / 4 && blocks <= cus));
 }
 __device__ __forceinline__ void lowrank_small_partial_block(int block, int chunks, bool wide, const uint16_t* __restrict__ x, int64_t ldx,
                                                             const uint16_t* __restrict__ v, int M, int R, int K, int kc, float* __restrict__ ws)

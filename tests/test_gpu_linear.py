@@ -1265,6 +1265,12 @@ def test_decode_sized_projection_has_the_same_bits_whichever_launch_forms_it(M, 
     assert bool(((xv.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,K,R", [(192, 5120, 128), (161, 5120, 96), (128, 14336, 64), (255, 3584, 128), (97, 14336, 64)])
+def test_decode_sized_projection_by_workgroups_that_fill_one_round(M, K, R):
+    """Four waves of 64 rows beside the quantizer at sizes where their workgroups fill the compute units once: the same bits again."""
+    test_decode_sized_projection_has_the_same_bits_whichever_launch_forms_it(M, K, R)
+
+
 @pytest.mark.parametrize("M,K,R", [(256, 18944, 64), (259, 9216, 32), (300, 10240, 96), (777, 2048, 64)])
 def test_projection_of_a_short_prompt_adds_any_number_of_slices(M, K, R):
     """Two to sixteen slices of K: more and fewer than are requested together, a last workgroup of the finishing launch that is not full."""
