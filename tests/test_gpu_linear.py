@@ -1242,6 +1242,28 @@ def test_projection_formed_whole_beside_the_operand_build_has_the_bits_of_its_tw
     assert bool(((xv.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M,K,R,whole", [(1, 256, 32, True), (128, 1280, 128, True), (192, 1792, 128, True), (160, 2304, 192, True), (255, 2560, 256, True),
+                                         (255, 2816, 192, True), (255, 3072, 256, True), (17, 1792, 96, False), (64, 3072, 256, False), (48, 4096, 224, False)])
+def test_which_launch_forms_the_projection_beside_the_operand_build(M, K, R, whole):
+    """Chunks that four groups of four waves share unevenly (2, 2, 2, 1 of 1792, 3, 3, 3, 2 of 2816) in the one launch, and sizes beyond its line.  Only the
+    two steps write to the workspace; the bits are those of the projection by itself either way."""
+    from metis_hip import _lib, ops
+    L = _lib.load()
+    g = torch.Generator().manual_seed(3 * M + K + R)
+    x = synthetic_activation(40 + M, M, K).cuda()
+    v = (torch.randn(R, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    s = torch.randn(R, generator=g).bfloat16().cuda()
+    p = ops.quantize(x, 1, deferred=True)
+    ws = torch.full((L.metis_lowrank_project_workspace_bytes(M, R, K),), 0xA5, dtype=torch.uint8, device="cuda")
+    xv, t = torch.empty(M, R, dtype=torch.bfloat16, device="cuda"), torch.empty(M, R, dtype=torch.bfloat16, device="cuda")
+    out, unit = torch.empty(L.metis_nvfp4_decode_operand_bytes(M, K), dtype=torch.uint8, device="cuda"), torch.empty(1, device="cuda")
+    assert L.metis_decode_prepare_deferred(x.data_ptr(), K, v.data_ptr(), R, s.data_ptr(), xv.data_ptr(), t.data_ptr(), ws.data_ptr(), ws.numel(), p.codes.data_ptr(),
+                                           p.deferred.data_ptr(), M, K, 1, 1, None, unit.data_ptr(), out.data_ptr(), 0, 0, torch.cuda.current_stream().cuda_stream) == 0
+    xv0, t0 = ops.lowrank_project(x, v, s)
+    assert torch.equal(xv, xv0) and torch.equal(t, t0) and torch.equal(out, ops.decode_operand(ops.quantize(x, 1), 1))
+    assert bool((ws == 0xA5).all()) == whole
+
+
 @pytest.mark.parametrize("M,K,R", [(1, 1024, 64), (16, 1024, 64), (64, 1024, 192), (65, 1536, 192), (128, 1536, 192), (33, 3584, 96), (255, 3072, 256),
                                    (65, 8960, 128), (192, 8960, 128), (255, 18944, 32), (160, 18944, 64)])
 def test_decode_sized_projection_has_the_same_bits_whichever_launch_forms_it(M, K, R):
