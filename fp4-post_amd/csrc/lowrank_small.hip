@@ -7,7 +7,8 @@
 // 64-element steps (the product is latency-bound: a step is one round trip to memory), one wave, a workgroup of its own, per chunk, 32
 // rows and 32 columns of R (a workgroup per chunk and 64 rows left three of four compute units idle while it looked up its lines: with the
 // finishing launch, 64 x 3584, R = 192 9.2 -> 7.0 us, 64 x 18944, R = 64 8.8 -> 7.4, 5 x 1536, R = 192 6.1 -> 5.1, 255 x 3584, R = 192 15.2 ->
-// 14.7; the captured decode step of 64 sequences, hidden 3584, 162.5 -> 156.0); a lane streams 64 contiguous bytes of its row per
+// 14.7, 255 x 18944, R = 64 15.6 -> 13.4, R = 256 33.8 -> 33.5, 192 x 8960, R = 128 11.9 -> 11.9, 128 x 14336, R = 96 11.1 -> 11.3; the captured decode
+// step of 64 sequences, hidden 3584, 162.5 -> 156.0); a lane streams 64 contiguous bytes of its row per
 // step straight into MFMA operands (both operands with the same mapping, so K may be visited in that permuted order).
 // Partial sums go to a caller-supplied workspace [chunks][M][R] and a second small kernel adds them in chunk order
 // (four threads per output quad, each a quarter of the chunks, folded in order), rounds to bf16 and applies s.

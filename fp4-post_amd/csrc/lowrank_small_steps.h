@@ -136,17 +136,18 @@ __device__ __forceinline__ void lowrank_small_store(const float (&a)[4], int id,
     }
 }
 
-// Both steps of 16 rows x 16 columns in one block of 1024 threads, for a launch with other work that waits for nothing of the projection; K <= 3072.
-// Waves 4 g .. 4 g + 3 share the chunks of group g of the finishing step, a quarter each, requested together; the first of them adds the chunk sums of
-// all four in chunk order.  A chunk is the four products of the first step on 32 x 32 tiles with 16 rows of either operand in lanes 0 .. 15 and
-// 32 .. 47, so the bits are those of the two steps; the other lanes load half of those rows' elements and hand them over (v_permlane16_swap): their own
-// rows of the product are nobody's.  Every thread of the block has to call it (two barriers inside).  Blocks: lowrank_small_project_blocks(M, R).
 // what lanes 16 .. 31 and 48 .. 63 hold, in lanes 0 .. 15 and 32 .. 47
 __device__ __forceinline__ uint4 lr_from_odd_rows(uint4 a)
 {
     return make_uint4(__builtin_amdgcn_permlane16_swap(a.x, a.x, false, false)[1], __builtin_amdgcn_permlane16_swap(a.y, a.y, false, false)[1],
                       __builtin_amdgcn_permlane16_swap(a.z, a.z, false, false)[1], __builtin_amdgcn_permlane16_swap(a.w, a.w, false, false)[1]);
 }
+
+// Both steps of 16 rows x 16 columns in one block of 1024 threads, for a launch with other work that waits for nothing of the projection; K <= 3072.
+// Waves 4 g .. 4 g + 3 share the chunks of group g of the finishing step, a quarter each, requested together; the first of them adds the chunk sums of
+// all four in chunk order.  A chunk is the four products of the first step on 32 x 32 tiles with 16 rows of either operand in lanes 0 .. 15 and
+// 32 .. 47, so the bits are those of the two steps; the other lanes load half of those rows' elements and hand them over (v_permlane16_swap): their own
+// rows of the product are nobody's.  Every thread of the block has to call it (two barriers inside).  Blocks: lowrank_small_project_blocks(M, R).
 constexpr int kLrProjectThreads = 1024, kLrProjectK = 3072;
 __device__ __forceinline__ void lowrank_small_project_block(int block, const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ v, int M,
                                                             int R, int K, const uint16_t* __restrict__ s, uint16_t* __restrict__ xv,

@@ -1215,7 +1215,9 @@ int skinny_operand_rht(const void* codes, const void* scales, float* unit, const
 // K, less with few rows), while partial sums of K chunks cost a launch and grow with the number of 32 x 32 x 64 steps (2.7 us per 1000).  Microseconds,
 // two launches | one: 64 x 1536, R = 192 5.9 | 6.2, 64 x 1024, R = 192 5.5 | 5.5, R = 64 5.2 | 5.4; 1 x 1024 5.0 | 4.8, 1 x 1536, R = 64 5.06 | 5.15;
 // 128 x 1024, R = 128 5.6 | 5.5; 128 x 1536, R = 192 6.6 | 6.2, R = 128 6.1 | 6.1; 192 x 1536, R = 64 6.0 | 6.2, R = 128 6.7 | 6.2; 192 x 2048, R = 128
-// 7.2 | 7.1, R = 192 8.2 | 7.2; 128 x 2560, R = 192 7.6 | 8.0; 192 x 3072, R = 192 10.1 | 8.9, R = 128 8.3 | 8.8.
+// 7.2 | 7.1, R = 192 8.2 | 7.2; 128 x 2560, R = 192 7.6 | 8.0; 192 x 3072, R = 192 10.1 | 8.9, R = 128 8.3 | 8.8.  Below 1024 the one launch always:
+// 1 x 256, R = 32 5.6 | 5.3, 5 x 512, R = 192 5.8 | 5.4, 64 x 768, R = 64 5.9 | 5.6, 255 x 512, R = 128 6.3 | 5.7, 255 x 768, R = 256 8.4 | 7.6; the exceptions
+// are 255 x 256 and 255 x 512 at R = 256 (more blocks than compute units) 6.4 | 7.5 and 7.4 | 7.5.
 static bool project_whole(int64_t M, int64_t R, int64_t K)
 {
     return K <= kLrProjectK && (M + 31) / 32 * (R / 32) * (K / 64) > (K - 1024) * 5 / 8 + (M < 16 ? 9 * M : 148);

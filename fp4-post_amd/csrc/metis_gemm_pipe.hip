@@ -27,30 +27,6 @@ namespace metis {
 // consecutive rows 16 different units of a 256-byte period.
 __host__ __device__ __forceinline__ int xt_swz(int q) { return ((q >> 2) & 1) | ((((q >> 1) ^ (q >> 3)) & 1) << 1); }
 
-// ---------------------------------------------------------------------------------------------
-// packed NVFP4 -> tiled 16-bit operands.  One wave per tile: lane l writes slot l (row l / 4).  A wave walks
-// eight consecutive k tiles of one tile row, so the 128-byte lines of codes it touches are used whole.
-// HBM-bound: 0.5625 B read, 2 B written per element.  The unit's eight words of codes and eight scales (AHEAD) are requested
-// together: one at a time, between the stores, the lines of codes (16 bytes of each of 16 rows per load) were pushed out of L2
-// by the output before the next visit.  16384 x 18944 from a deferred activation 249 -> 209 us, 16384 x 3584 36.9 -> 32.6,
-// the 18944 x 3584 weight 48.0 -> 41.3, 8192 x 4096 17.0 -> 16.3.  Streaming stores on top change nothing (214, 31.7).
-//   PB16 = 0: binary16, e2m1(code) * e4m3(scale) * 2^-8, exact (the tensor unit is applied by the GEMM)
-//   PB16 = 1: bf16, the reference's dequantized value with every op rounded to bf16
-//             (src/Metis/Metis/quant.py:23-24, 32-35: bf16(bf16(e4m3 * unit) * v / 2)), unit included
-// ---------------------------------------------------------------------------------------------
-//   RHT: the packed tensor is a rotated one (NV recipe); every block of 16 is rotated back after dequantization,
-//        (q H) / 16 * sign, as `_apply_hadamard_blocks(..., inverse=True)` does after the QDQ
-//        (src/Metis/Metis/bitlinear.py:395-405, 577-585).  The two lanes that hold the halves of a block exchange
-//        them and both run the 16-point butterflies.  PB16 = 0: the result is rounded to binary16 once (the sum of a
-//        block needs at most 12 significant bits); PB16 = 1: dequantized values and result rounded to bf16 as the
-//        reference's bf16 tensors are.
-//   center (PB16 without RHT): the packed tensor is the centred residual of the mean mode; the operand is the
-//        reference's me + QDQ(x - me) with the sum rounded to bf16 (src/Metis/Metis/bitlinear.py:330-333 in bf16
-//        arithmetic): one bf16 value per column.
-//   DEF: the quantizer stopped after its first phase (deferred scale bytes, nvfp4_quant.hip): `scales` holds one bf16
-//        block maximum per block instead of E4M3 bytes, `partials` the partial tensor maxima.  The kernel forms the
-//        tensor unit (written to unit_out by the first workgroup) and every scale byte itself, in the arithmetic the
-//        tensor was quantized in (QMODE) -- the expressions of quant_scales_kernel, so the bytes it would have written.
 // Rotating back on the matrix cores: out[c] = sign_c / 16 * sum_k H[c][k] x[k], one 16 x 16 product for many blocks.  The values of
 // a block are small multiples of one number (12 units per scale in exact binary16 codes times E4M3; bf16 values of one scale span less than
 // 17 bits), so their binary32 sums are exact in any order: the bits of sixteen ordered additions.  binary16 operands go in without their
@@ -80,6 +56,30 @@ template <int PB16> __device__ __forceinline__ uint32_t rotated_pair(float a, fl
     const half2_t h = {(_Float16)a, (_Float16)b};
     return __builtin_bit_cast(uint32_t, h);
 }
+
+// ---------------------------------------------------------------------------------------------
+// packed NVFP4 -> tiled 16-bit operands.  One wave per tile: lane l writes slot l (row l / 4).  A wave walks
+// eight consecutive k tiles of one tile row, so the 128-byte lines of codes it touches are used whole.
+// HBM-bound: 0.5625 B read, 2 B written per element.  The unit's eight words of codes and eight scales (AHEAD) are requested
+// together: one at a time, between the stores, the lines of codes (16 bytes of each of 16 rows per load) were pushed out of L2
+// by the output before the next visit.  16384 x 18944 from a deferred activation 249 -> 209 us, 16384 x 3584 36.9 -> 32.6,
+// the 18944 x 3584 weight 48.0 -> 41.3, 8192 x 4096 17.0 -> 16.3.  Streaming stores on top change nothing (214, 31.7).
+//   PB16 = 0: binary16, e2m1(code) * e4m3(scale) * 2^-8, exact (the tensor unit is applied by the GEMM)
+//   PB16 = 1: bf16, the reference's dequantized value with every op rounded to bf16
+//             (src/Metis/Metis/quant.py:23-24, 32-35: bf16(bf16(e4m3 * unit) * v / 2)), unit included
+// ---------------------------------------------------------------------------------------------
+//   RHT: the packed tensor is a rotated one (NV recipe); every block of 16 is rotated back after dequantization,
+//        (q H) / 16 * sign, as `_apply_hadamard_blocks(..., inverse=True)` does after the QDQ
+//        (src/Metis/Metis/bitlinear.py:395-405, 577-585).  One 32 x 32 x 16 product rotates the 32 blocks of a
+//        tile.  PB16 = 0: the result is rounded to binary16 once (the sum of a block needs at most 12 significant bits);
+//        PB16 = 1: dequantized values and result rounded to bf16 as the reference's bf16 tensors are.
+//   center (PB16 without RHT): the packed tensor is the centred residual of the mean mode; the operand is the
+//        reference's me + QDQ(x - me) with the sum rounded to bf16 (src/Metis/Metis/bitlinear.py:330-333 in bf16
+//        arithmetic): one bf16 value per column.
+//   DEF: the quantizer stopped after its first phase (deferred scale bytes, nvfp4_quant.hip): `scales` holds one bf16
+//        block maximum per block instead of E4M3 bytes, `partials` the partial tensor maxima.  The kernel forms the
+//        tensor unit (written to unit_out by the first workgroup) and every scale byte itself, in the arithmetic the
+//        tensor was quantized in (QMODE) -- the expressions of quant_scales_kernel, so the bytes it would have written.
 template <int PB16, int RHT = 0, int DEF = 0, int QMODE = 0, int AHEAD = 8>
 __global__ __launch_bounds__(256) void expand_xt_kernel(const uint32_t* __restrict__ codes, const uint8_t* __restrict__ scales,
                                                         const float* __restrict__ unit_p, uint4* __restrict__ out, int rows,

@@ -1548,7 +1548,6 @@ def quantize_project(x2: torch.Tensor, v: torch.Tensor, s: torch.Tensor, mode: i
     M, K = x2.shape
     R = v.shape[0]
     dev = x2.device
-    L = load()
     v = v.contiguous()
     s = s.to(torch.bfloat16).contiguous()
     size, need = _deferred_bytes(M, K), _lowrank_rows_workspace_bytes(M, R, K, dev.index or 0)
@@ -1578,7 +1577,6 @@ def quantize_project_decode(x2: torch.Tensor, v: torch.Tensor, mode: int = MODE_
     M, K = x2.shape
     R = v.shape[0]
     dev = x2.device
-    L = load()
     v = v.contiguous()
     size, need = _deferred_bytes(M, K), _lowrank_workspace_bytes(M, R, K)
     new = _lib.call("metis_decode_quant_project_deferred", dev.index, ((U8, M, K // 2), (F32, 1), (U8, size), (U8, need)),
