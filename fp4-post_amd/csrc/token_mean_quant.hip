@@ -175,6 +175,7 @@ int token_mean_quant(const void* x, int64_t rows, int64_t cols, int after_norm, 
     if (!token_mean_pieces(rows, cols, after_norm, &pieces, &per)) return METIS_E_TOO_LARGE;
     if (!x || !mean || !mean32 || !codes || ((uintptr_t)x % 16) || ((uintptr_t)mean % 4) || ((uintptr_t)mean32 % 4) || ((uintptr_t)codes % 8)) return METIS_E_ARG;
     if (cached && (cached_count < 0 || cached_count > (1 << 24) || ((uintptr_t)cached % 2))) return METIS_E_ARG;
+    const uint32_t strip_blocks = (uint32_t)(((cols + kStrip - 1) / kStrip + 7) / 8 * 8);
     TokenMeanProjection pr = {};
     int more = 0;
     if (v) {
@@ -185,12 +186,16 @@ int token_mean_quant(const void* x, int64_t rows, int64_t cols, int after_norm, 
         pr.ws = (float*)lr_workspace;
         pr.R = (int)R;
         pr.chunks = lowrank_small_chunks(cols, &pr.kc);
-        pr.wide = lowrank_small_wide(rows, R, cols, device_cus());
-        more = lowrank_small_partial_blocks(rows, R, pr.chunks, pr.wide != 0);
+        // A workgroup of this launch holds the strips' LDS, whatever it does: four to a compute unit.  Single tiles, one wave in four, as long as they and
+        // the strips are on the device together; beyond, four waves of 64 rows.  Microseconds, four waves | single: 64 x 8960, R = 160 (704 of them, and
+        // 280 strips) 6.5 | 5.0, 48 x 8960, R = 128 6.0 | 4.9, 96 x 8960, R = 96 (910) 5.8 | 5.2, 128 x 1536, R = 256 5.1 | 4.8, 192 x 1536, R = 128 (624)
+        // 5.2 | 5.4; 160 x 8960, R = 64 (980) 5.8 | 6.1, 160 x 18944, R = 32 (1087) 6.6 | 7.5, 1 x 14336, R = 256 (1344) 4.5 | 5.0, 64 x 18944, R = 256 8.8 | 11.7.
+        const int single = lowrank_small_partial_blocks(rows, R, pr.chunks, false);
+        pr.wide = 4 * ((int64_t)strip_blocks + single) > 15 * (int64_t)device_cus();
+        more = pr.wide ? lowrank_small_partial_blocks(rows, R, pr.chunks, true) : single;
     }
     Workspace ws;
     if (const int rc = carve_deferred(deferred, bytes, rows, cols, &ws)) return rc;
-    const uint32_t strip_blocks = (uint32_t)(((cols + kStrip - 1) / kStrip + 7) / 8 * 8);
 #define METIS_TM(N) hipLaunchKernelGGL((token_mean_quant_kernel<N>), dim3(strip_blocks + (unsigned)more), dim3(256), 0, st, strip_blocks, \
         (const uint16_t*)x, (uint32_t)rows, (uint32_t)cols, pieces, per, (const uint16_t*)cached, (float)cached_count, (uint16_t*)mean, mean32, \
         (uint2*)codes, ws.amax, ws.gmax, pr)

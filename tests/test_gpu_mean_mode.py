@@ -741,6 +741,20 @@ def test_a_token_mean_asks_of_every_tensor_whether_its_launch_takes_it():
             ops.quantize(bad, ops.MODE_PB16, center=tm, deferred=True)
 
 
+@pytest.mark.parametrize("rows,cols,R", [(1, 14336, 256), (64, 8960, 160), (160, 8960, 64), (33, 18944, 64), (255, 1536, 192), (255, 18944, 32)])
+def test_projection_beside_the_mean_has_the_bits_of_its_own_launch(rows, cols, R):
+    """Its partial sums by single tiles and by four waves of 64 rows, on either side of what is on the device together with the strips."""
+    from metis_hip import ops
+    g = torch.Generator().manual_seed(rows + cols + R)
+    x = torch.randn(rows, cols, generator=g).bfloat16().cuda()
+    v, s = (torch.randn(R, cols, generator=g) * cols ** -0.5).bfloat16().cuda(), torch.randn(R, generator=g).bfloat16().cuda()
+    tm = ops.TokenMean(v=v)
+    p = ops.quantize(x, ops.MODE_PB16, center=tm, deferred=True)
+    xv, t, _ = ops.project_and_operand(x, v, s, p, ops.MODE_PB16, tm.mean, pending=tm.pending)
+    want = ops.lowrank_project(x, v, s)
+    assert torch.equal(xv, want[0]) and torch.equal(t, want[1])
+
+
 def test_running_mean_of_decode_steps_through_the_one_launch_path():
     """A BitLinear under the default arguments: prompt, then decode steps; the cache holds what the separate kernels would keep."""
     from metis_hip import BitLinear, MetisArgs, ops
