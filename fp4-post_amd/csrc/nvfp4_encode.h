@@ -434,7 +434,7 @@ __device__ __forceinline__ void publish_group_max(float m, uint32_t* ws_gmax, ui
 }
 
 // The tensor maximum from ngroups published partial maxima, in a workgroup of 256 threads.  Eight entries are requested together: taken one
-// after the other, each waited for in L2, they were half of what phase 2 took.
+// after the other, each waited for in L2, they were half of what phase 2 took (4096 x 3584 11.0 -> 10.1 us, stochastic 14.3 -> 12.1, binary32 23.4 -> 21.1).
 __device__ __forceinline__ float fold_group_maxima(const uint32_t* __restrict__ ws_gmax, uint32_t ngroups)
 {
     __shared__ float smax[4];
@@ -483,14 +483,16 @@ __device__ __forceinline__ uint32_t scale_byte_of(uint32_t amax_bf16, float unit
     return e4m3_byte(rd<MODE>(block_scalar<MODE>(__uint_as_float(amax_bf16 << 16)) / unit));
 }
 
-// The scale bytes of four or eight block maxima against one unit, without an IEEE division for each.
+// The scale bytes of four or eight block maxima against one unit, without an IEEE division for each where that pays.
 // bf16 arithmetic: the quotient is rounded to bf16, for which quot2 will do while the unit's reciprocal and its remainder are normal
-// numbers (see encode_rne_pb16_n).  Binary32 arithmetic: div3, and for binary32 maxima div6 under it, are within 6 binary32 ulps of the
-// quotient that the IEEE sequence rounds to; the byte can differ only if one of the converter's thresholds lies between, and these (odd
-// multiples of half an E4M3 ulp, the subnormals' too, and 464) have zero low 19 significand bits.  Quotients within 8 of such a number,
-// zero, infinite ones and NaN send their wave to the divisions: about one wave of 64 x 8 in seventy.
-// With fold_group_maxima: the residual quantizer of 4096 x 3584, r = 64 with its bytes 32.9 -> 30.9 us; training steps 1657 -> 1652 (4096
-// tokens, 1536 -> 8960) and 3797 -> 3785 us (2103 tokens, 3584 -> 18944); a projection under the NV recipe 566 -> 562.
+// numbers (see encode_rne_pb16_n).  Binary32 maxima: div3 and div6 under it are within 6 binary32 ulps of the quotient that the IEEE
+// sequence rounds to; the byte can differ only if one of the converter's thresholds lies between, and these (odd multiples of half an
+// E4M3 ulp, the subnormals' too, and 464) have zero low 19 significand bits.  Quotients within 8 of such a number, zero, infinite ones and
+// NaN send their wave to the divisions: about one wave of 64 x 4 in 140.
+// Microseconds of a call, divisions | these: bf16 arithmetic 16 x 64 stochastic 5.13 | 5.04, 4096 x 3584 11.96 | 11.71, both packings 20.87 | 20.17; binary32
+// maxima 4096 x 14336 51.8 | 50.3, stochastic 49.7 | 48.5, the residual quantizer of 4096 x 3584, r = 64 31.0 | 30.9, to 2048 x 2048 alike.  bf16 maxima in
+// binary32 arithmetic, whose scalars need no divisions of their own, divide: 4096 x 3584 10.05 (divisions) | 10.20, 16 x 64 4.94 | 5.06, the norm's 16384 x 4096
+// 65.6 | 66.2.
 template <int MODE, bool WIDE> struct ScaleBytes {
     float unit, reciprocal;
     SplitReciprocal split;
@@ -503,11 +505,11 @@ template <int MODE, bool WIDE> struct ScaleBytes {
     template <int N> __device__ __forceinline__ void operator()(const float (&amax)[N], uint32_t (&out)[N / 4]) const
     {
         float t[N];
-        bool literal = MODE != 0 && !quick;
+        bool literal = MODE == 0 || !quick;
         if constexpr (MODE != 0) {
 #pragma unroll
             for (int i = 0; i < N; ++i) t[i] = rb(quot2(block_scalar<MODE>(amax[i]), split));
-        } else {
+        } else if constexpr (WIDE) {
             uint32_t least = 0xffffffffu;
 #pragma unroll
             for (int i = 0; i < N; ++i) {
