@@ -242,17 +242,17 @@ __global__ __launch_bounds__(256) void expand_xt_t_kernel(const uint2* __restric
 // The same for a rotated tensor (NV recipe).  A 16 x 16 x 16 product rotates 16 blocks, one from each of 16 source rows, and turns
 // them: with the blocks as its rows lane l receives column l % 16 of four of them.  Two products, of the source rows 8 i + (0..3) and
 // 8 i + (4..7), therefore leave a lane eight consecutive k of one operand row, a whole slot of the tile: no trip through LDS.
-// A wave owns 32 source rows and eight blocks of each: lane l loads block l / 16 (and 4 + l / 16) of rows 8 (l / 4 % 4) + l % 4 (+ 4),
-// and the four lanes of a row exchange quarters, so that each holds its quarter of all four blocks.
+// A wave owns 32 source rows and four blocks of each (QUADS = 2: eight): lane l loads block l / 16 (and 4 + l / 16) of rows 8 (l / 4 % 4) + l % 4
+// (+ 4), and the four lanes of a row exchange quarters, so that each holds its quarter of all four blocks.
 // HBM-bound (0.5625 B read, 2 B written per element).  The sixteen-term sums on the vector units had taken 4096 x 8960 34.4 us here and
 // 32.0 in the plain expansion.
-template <int PB16>
-__global__ __launch_bounds__(256) void expand_xt_t_rht_kernel(const uint2* __restrict__ codes, const uint8_t* __restrict__ scales,
+template <int PB16, int QUADS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void expand_xt_t_rht_kernel(const uint2* __restrict__ codes, const uint8_t* __restrict__ scales,
                                                               const float* __restrict__ unit_p, uint4* __restrict__ out, int R, int C, uint32_t sign_mask)
 {
     typedef short short4_t __attribute__((ext_vector_type(4)));
     const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-    const int cb_n = C / 16, kt = R / 32, groups = (cb_n + 7) / 8;
+    const int cb_n = C / 16, kt = R / 32, groups = (cb_n + 4 * QUADS - 1) / (4 * QUADS);
     const int64_t nunits = (int64_t)groups * kt;
     const float unit = PB16 ? *unit_p : 0.0f;
     uint32_t rotation[2] = {0u, 0u};
@@ -260,14 +260,14 @@ __global__ __launch_bounds__(256) void expand_xt_t_rht_kernel(const uint2* __res
     for (int j = 0; j < 4; ++j) rotation[j >> 1] |= (uint32_t)rotation_entry<PB16>(n, 4 * g + j, sign_mask) << (16 * (j & 1));
     const uint2 h = make_uint2(rotation[0], rotation[1]);
     const int place = n * 4 + (g ^ xt_swz(n));
-    for (int64_t un = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); un < nunits; un += (int64_t)gridDim.x * 4) {
-        const int kb = (int)(un / groups), cb0 = (int)(un - (int64_t)kb * groups) * 8;   // consecutive waves: consecutive blocks of a row
-        uint2 c[2][2];
-        uint32_t sb[2][2];
+    for (int64_t un = (int64_t)blockIdx.x * WAVES + (threadIdx.x >> 6); un < nunits; un += (int64_t)gridDim.x * WAVES) {
+        const int kb = (int)(un / groups), cb0 = (int)(un - (int64_t)kb * groups) * (4 * QUADS);   // consecutive waves: consecutive blocks of a row
+        uint2 c[2][QUADS];
+        uint32_t sb[2][QUADS];
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int w = 0; w < 2; ++w) {
+            for (int w = 0; w < QUADS; ++w) {
                 const int cb = cb0 + 4 * w + g;
                 const int64_t ib = (int64_t)(kb * 32 + 8 * (n >> 2) + 4 * s + (n & 3)) * cb_n + cb;
                 c[s][w] = make_uint2(0u, 0u);
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void expand_xt_t_rht_kernel(const uint2* __res
                 if (cb < cb_n) { c[s][w] = codes[ib]; sb[s][w] = scales[ib]; }
             }
 #pragma unroll
-        for (int w = 0; w < 2; ++w) {
+        for (int w = 0; w < QUADS; ++w) {
             uint32_t quarter[2][2], byte[2][2];                  // [s][block & 1]: two blocks, b and b + 2
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
@@ -454,16 +454,22 @@ int expand_xt_transposed(const void* codes, const void* scales, const float* uni
     if (rows == 0 || cols == 0) return METIS_OK;
     if (!codes || !scales || !out || ((uintptr_t)codes % 8) || ((uintptr_t)out % 16)) return METIS_E_ARG;
     if (mode == METIS_MODE_PB16 && !unit) return METIS_E_ARG;
+    // A rotated tensor: four blocks a wave, a workgroup of its own each, while that is at most sixteen a compute unit; beyond, eight blocks and four waves.
+    // Before the matrix cores it was a block a lane.  Microseconds of the kernel (binary16 operands), a block a lane | eight blocks | four: 64 x 3584 3.28 |
+    // 4.04 | 2.80, 256 x 3584 3.52 | 4.20 | 3.10, 512 x 4096 4.28 | 4.48 | 3.72, 2048 x 4096 (sixteen) 8.72 | 7.20 | 6.96, 4096 x 3584 (28) 14.4 | 10.2 | 11.4.
+    const int64_t cus = device_cus(), narrow = (cols / 16 + 3) / 4 * (rows / 32);
+    const bool spread = rht && narrow <= 16 * cus;
     const int64_t units = rht ? (cols / 16 + 7) / 8 * (rows / 32) : (cols / 16) * ((rows / 32 + 1) / 2);
-    int64_t g = (units + 3) / 4;
-    const int64_t cap = (int64_t)device_cus() * 16;
-    if (g > cap) g = cap;
-#define METIS_EXT(P) do { if (rht) hipLaunchKernelGGL((expand_xt_t_rht_kernel<P>), dim3((unsigned)g), dim3(256), 0, st, (const uint2*)codes, \
-                                                      (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols, sign_mask); \
+    int64_t g = spread ? narrow : (units + 3) / 4;
+    if (g > 16 * cus) g = 16 * cus;
+#define METIS_EXR(P, Q, W) hipLaunchKernelGGL((expand_xt_t_rht_kernel<P, Q, W>), dim3((unsigned)g), dim3(64 * W), 0, st, (const uint2*)codes, \
+                                              (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols, sign_mask)
+#define METIS_EXT(P) do { if (spread) METIS_EXR(P, 1, 1); else if (rht) METIS_EXR(P, 2, 4); \
                           else hipLaunchKernelGGL((expand_xt_t_kernel<P>), dim3((unsigned)g), dim3(256), 0, st, (const uint2*)codes, \
                                                   (const uint8_t*)scales, unit, (uint4*)out, (int)rows, (int)cols); } while (0)
     if (mode == METIS_MODE_PB16) METIS_EXT(1); else METIS_EXT(0);
 #undef METIS_EXT
+#undef METIS_EXR
     return hipGetLastError() == hipSuccess ? METIS_OK : METIS_E_LAUNCH;
 }
 

@@ -185,6 +185,14 @@ def test_operands_of_a_rotated_tensor_bit_for_bit(R, C, mode):
         assert torch.equal(untile(ops.expand_tiled_transposed(p, mode=mode), C, R, dt), want.T)
 
 
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("R,C", [(2048, 4096), (2080, 4048), (2112, 4112)])
+def test_operands_of_a_rotated_tensor_on_either_side_of_sixteen_waves_a_compute_unit(R, C, mode):
+    """The transposed operand by waves of four blocks and 32 rows (as many as that line allows), and by waves of eight blocks, the last ones with five
+    and with one of them."""
+    test_operands_of_a_rotated_tensor_bit_for_bit(R, C, mode)
+
+
 @pytest.mark.parametrize("tag", ["p32", "pb16"])
 def test_linear_lowbit_nv_recipe_on_the_packed_kernels_against_reference_vectors(tag):
     """LinearLowbit with enable_nv_recipe, 64 tokens, 96 -> 64 features: forward, grad_input and grad_weight against
