@@ -433,19 +433,23 @@ __device__ __forceinline__ void publish_group_max(float m, uint32_t* ws_gmax, ui
     publish_group_max(m, ws_gmax, fill_to, blockIdx.x, gridDim.x);
 }
 
-// The tensor maximum from ngroups published partial maxima, in a workgroup of 256 threads.  Eight entries are requested together: taken one
-// after the other, each waited for in L2, they were half of what phase 2 took (4096 x 3584 11.0 -> 10.1 us, stochastic 14.3 -> 12.1, binary32 23.4 -> 21.1).
+// The tensor maximum from ngroups (at least one) published partial maxima, in a workgroup of 256 threads.  Eight entries are requested together: taken
+// one after the other, each waited for in L2, they were half of what phase 2 took (4096 x 3584 11.0 -> 10.1 us, stochastic 14.3 -> 12.1, binary32 23.4 ->
+// 21.1).  The first is requested by itself and is the only one of a tensor of up to 256 workgroups, where eight of the same cost more than one:
+// the scale bytes' launch of 16 x 64 takes 2.01 us in place of 2.32 (one entry after the other 2.24), of 256 x 3584 2.97 in place of 3.12 (2.95).
 __device__ __forceinline__ float fold_group_maxima(const uint32_t* __restrict__ ws_gmax, uint32_t ngroups)
 {
     __shared__ float smax[4];
+    const uint32_t first = ws_gmax[min((uint32_t)threadIdx.x, ngroups - 1u)];                    // (an entry twice does no harm)
     float m = 0.0f;
-    for (uint32_t g0 = threadIdx.x; g0 < ngroups; g0 += 8u * 256u) {
+    for (uint32_t g0 = 256u + threadIdx.x; g0 < ngroups; g0 += 8u * 256u) {
         uint32_t v[8];
 #pragma unroll
-        for (uint32_t i = 0; i < 8u; ++i) v[i] = ws_gmax[min(g0 + i * 256u, ngroups - 1u)];     // (an entry twice does no harm)
+        for (uint32_t i = 0; i < 8u; ++i) v[i] = ws_gmax[min(g0 + i * 256u, ngroups - 1u)];
 #pragma unroll
         for (uint32_t i = 0; i < 8u; ++i) m = fmaxf(m, __uint_as_float(v[i]));
     }
+    m = fmaxf(m, __uint_as_float(first));
     m = wave_max(m);
     if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = m;
     __syncthreads();

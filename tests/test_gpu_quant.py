@@ -797,6 +797,20 @@ def test_round_trip_of_a_tensor_of_many_dimensions(dt):
     assert got.shape == x.shape and torch.equal(got.reshape(6, 32), quant_func["nvfp4e2m1bnosr"].quantize_dequantize(x.reshape(6, 32)))
 
 
+@pytest.mark.parametrize("dt,mode", [(torch.bfloat16, 0), (torch.bfloat16, 1), (torch.float32, 0)])
+@pytest.mark.parametrize("rows", [1, 255, 256, 257, 513, 1025])
+def test_the_tensor_maximum_is_found_in_whichever_workgroup_it_lies(ops, rows, dt, mode):
+    """Up to 256 partial maxima, one to a thread, and more of them, eight requested together: the largest value in the first, a middle and the last block
+    gives the tensor's unit."""
+    x = (torch.rand(rows, 4096, generator=torch.Generator().manual_seed(rows)) - 0.5).to(dt).cuda()
+    for at in (0, rows * 2048 + 5, rows * 4096 - 1):
+        y = x.clone()
+        y.view(-1)[at] = -417.0
+        row = at // 4096
+        for sr in (False, True):
+            assert torch.equal(ops.quantize(y, mode, sr=sr).unit, ops.quantize(y[row:row + 1], mode).unit)
+
+
 # one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (256 x 1024 elements in bf16, 144 x
 # 1024 in binary32), leading dimensions, four, eight and sixteen half blocks per thread, the last workgroup partly filled
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
