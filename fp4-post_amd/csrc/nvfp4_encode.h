@@ -492,7 +492,8 @@ __device__ __forceinline__ uint32_t scale_byte_of(uint32_t amax_bf16, float unit
 // numbers (see encode_rne_pb16_n).  Binary32 maxima: div3 and div6 under it are within 6 binary32 ulps of the quotient that the IEEE
 // sequence rounds to; the byte can differ only if one of the converter's thresholds lies between, and these (odd multiples of half an
 // E4M3 ulp, the subnormals' too, and 464) have zero low 19 significand bits.  Quotients within 8 of such a number, zero, infinite ones and
-// NaN send their wave to the divisions: about one wave of 64 x 4 in 140.
+// NaN send their wave to the divisions: about one wave of 64 x 4 in 140, and always the one of the largest block, whose quotient is 448: a tensor of
+// few waves divides from the start (divide).
 // Microseconds of a call, divisions | these: bf16 arithmetic 16 x 64 stochastic 5.13 | 5.04, 4096 x 3584 11.96 | 11.71, both packings 20.87 | 20.17; binary32
 // maxima 4096 x 14336 51.8 | 50.3, stochastic 49.7 | 48.5, the residual quantizer of 4096 x 3584, r = 64 31.0 | 30.9, to 2048 x 2048 alike.  bf16 maxima in
 // binary32 arithmetic, whose scalars need no divisions of their own, divide: 4096 x 3584 10.05 (divisions) | 10.20, 16 x 64 4.94 | 5.06, the norm's 16384 x 4096
@@ -506,14 +507,14 @@ template <int MODE, bool WIDE> struct ScaleBytes {
     {
         return rd<MODE>((WIDE ? block_scalar_ieee(amax) : block_scalar<MODE>(amax)) / unit);
     }
-    template <int N> __device__ __forceinline__ void operator()(const float (&amax)[N], uint32_t (&out)[N / 4]) const
+    template <int N> __device__ __forceinline__ void operator()(const float (&amax)[N], uint32_t (&out)[N / 4], bool divide = false) const
     {
         float t[N];
         bool literal = MODE == 0 || !quick;
         if constexpr (MODE != 0) {
 #pragma unroll
             for (int i = 0; i < N; ++i) t[i] = rb(quot2(block_scalar<MODE>(amax[i]), split));
-        } else if constexpr (WIDE) {
+        } else if (WIDE && !divide) {
             uint32_t least = 0xffffffffu;
 #pragma unroll
             for (int i = 0; i < N; ++i) {

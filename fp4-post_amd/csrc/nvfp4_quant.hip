@@ -789,11 +789,11 @@ __global__ __launch_bounds__(256) void quant_scales_decode_kernel(const uint16_t
     }
 }
 
-// Phase 2 for parked binary32 maxima (binary32 input): IEEE divisions, four blocks per thread.
+// Phase 2 for parked binary32 maxima (binary32 input), four blocks per thread.
 __global__ __launch_bounds__(256) void quant_scales_f32_kernel(const float* __restrict__ ws_amax,
                                                                const uint32_t* __restrict__ ws_gmax, uint32_t ngroups,
                                                                uint8_t* __restrict__ scales, float* __restrict__ unit_out,
-                                                               uint32_t nblocks, const float* __restrict__ ws_amax2 = nullptr,
+                                                               uint32_t nblocks, bool divide, const float* __restrict__ ws_amax2 = nullptr,
                                                                uint8_t* __restrict__ scales2 = nullptr, float* __restrict__ unit_out2 = nullptr)
 {
     if (blockIdx.y) { ws_amax = ws_amax2; scales = scales2; unit_out = unit_out2; }
@@ -812,7 +812,7 @@ __global__ __launch_bounds__(256) void quant_scales_f32_kernel(const float* __re
         if (nxt < nquads) n = reinterpret_cast<const float4*>(ws_amax)[nxt];
         const float am[4] = {a.x, a.y, a.z, a.w};
         uint32_t o[1];
-        bytes(am, o);
+        bytes(am, o, divide);
         reinterpret_cast<uint32_t*>(scales)[q] = o[0];
         a = n; q = nxt;
     }
@@ -1109,9 +1109,11 @@ int launch_scales(int mode, const Workspace& ws, uint32_t ngroups, void* scales,
 {
     const int g2 = grid_for((nblocks + 7) / 8);
     const dim3 grid((unsigned)g2, amax2 ? 2u : 1u);            // a second packing of the same tensor rides in grid row 1
+    // Binary32 maxima: divisions below 2048 blocks, where one workgroup of few waves does it all (ScaleBytes).  Microseconds of the launch, divisions |
+    // quotients by three operations first: 16 x 64 2.05 | 2.16, 5 x 1536 2.23 | 2.34; 32 x 1024 2.46 | 2.41, 512 x 4096 3.51 | 3.40.
     if (mode == METIS_MODE_P32_F32)
         hipLaunchKernelGGL(quant_scales_f32_kernel, grid, dim3(256), 0, st, (const float*)ws.amax, ws.gmax, ngroups,
-                           (uint8_t*)scales, unit, nblocks, (const float*)amax2, (uint8_t*)scales2, unit2);
+                           (uint8_t*)scales, unit, nblocks, nblocks < 2048u, (const float*)amax2, (uint8_t*)scales2, unit2);
     else if (mode == 0)
         hipLaunchKernelGGL((quant_scales_kernel<0>), grid, dim3(256), 0, st, ws.amax, ws.gmax, ngroups,
                            (uint8_t*)scales, unit, nblocks, (const uint16_t*)amax2, (uint8_t*)scales2, unit2);

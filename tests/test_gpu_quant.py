@@ -811,6 +811,22 @@ def test_the_tensor_maximum_is_found_in_whichever_workgroup_it_lies(ops, rows, d
             assert torch.equal(ops.quantize(y, mode, sr=sr).unit, ops.quantize(y[row:row + 1], mode).unit)
 
 
+@pytest.mark.parametrize("blocks", [1, 4, 63, 2047, 2048, 2051])
+def test_scale_bytes_of_binary32_maxima_by_divisions_and_by_three_operations(ops, blocks):
+    """Either side of 2048 blocks, and one tensor inside another that takes the other way: maxima whose quotients are the converter's thresholds and their
+    neighbours among them."""
+    from oracle import metis_oracle as O
+    g = torch.Generator().manual_seed(blocks)
+    x = torch.randn(blocks, 16, generator=g) * torch.exp2(torch.randint(-14, 1, (blocks, 1), generator=g).float())
+    x[:, 0] = torch.nextafter(torch.randint(1, 449, (blocks,), generator=g).float() + 0.5 * torch.randint(0, 2, (blocks,), generator=g), torch.tensor(float("inf"))) / 64
+    x[0, 0] = 448.0 / 64 * 6
+    codes, scales, unit, _ = O.nvfp4_pack(x)
+    p = ops.quantize(x.cuda(), 0)
+    _check_packed(p, codes, scales, unit, f"{blocks} blocks")
+    more = ops.quantize(torch.cat([x, torch.zeros(4096, 16)]).cuda(), 0)
+    assert torch.equal(more.scales[:blocks], p.scales) and torch.equal(more.unit, p.unit)
+
+
 # one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (256 x 1024 elements in bf16, 144 x
 # 1024 in binary32), leading dimensions, four, eight and sixteen half blocks per thread, the last workgroup partly filled
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
