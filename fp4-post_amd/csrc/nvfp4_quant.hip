@@ -422,13 +422,15 @@ __device__ __forceinline__ void column_of_slab(const uint32_t* slab, int words, 
 // quant_codes_both_kernel does.  A lane's sixteen 2-byte loads per block, each waited for in place, left the kernel above at
 // 3 TB/s; now the vector units (Philox, or the encoder and the turning) and HBM bound it together.  Needs 16-byte-aligned rows (ld and cols multiples of 16 bytes) and
 // takes no caller noise; same bytes.  Binary32 arithmetic on bf16 values takes its quotients in two operations under the table of block
-// maxima, as the row kernel does (18944 x 3584 with scale bytes 82 -> 64 us).
+// maxima, as the row kernel does (18944 x 3584 with scale bytes 82 -> 64 us).  TABLE = false: without it, for tensors of up to 48 rows, of whose tiles one
+// wave in four has blocks: the table takes it longer to read than to do without (16 x 64 3.70 | 3.42 us, 32 x 1024 4.92 | 4.71; 64 x 3584 5.50 | 5.48, 256 x 1536
+// 5.28 | 5.44).
 // Five workgroups per compute unit: enough loads in flight, and fewer partial lines open at once in each die's L2 than with eight.
 // With scale bytes, eight | six | five | four: 18944 x 3584 51.5 | 50.0 | 48.3 | 48.2 us, 4096 x 14336 44.2 | 43.2 | 41.5 | 40.0,
 // stochastic 2112 x 18944 36.6 | 35.6 | 34.1 | 34.2; binary32 arithmetic, bound by its encoder, 4096 x 14336 52.9 | 56.2 | 54.5 | 57.2,
 // 18944 x 3584 64.5 | 61.2 | 64.4 | 67.7.
 constexpr int kColPerCu = 5;
-template <int MODE, bool SR, bool WIDE = false, bool F32IN = false>
+template <int MODE, bool SR, bool WIDE = false, bool F32IN = false, bool TABLE = true>
 __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
     const void* __restrict__ xv, uint32_t rows, uint32_t cols, int64_t ld, uint64_t seed, uint64_t offset, uint2* __restrict__ codes,
     void* __restrict__ ws_amax_v, uint32_t* __restrict__ ws_gmax, uint32_t tiles_c, uint32_t tiles_total, const void* __restrict__ center, uint32_t valid)
@@ -463,7 +465,7 @@ __global__ __launch_bounds__(256) void quant_codes_col_slab_kernel(
                 q[i] = in && row0 + i * RPI + lrow < valid ? *reinterpret_cast<const uint4*>(p + (int64_t)(i * RPI) * ld) : make_uint4(0u, 0u, 0u, 0u);
         }
     };
-    constexpr bool kTable = MODE == 0 && !SR && !WIDE;
+    constexpr bool kTable = TABLE && MODE == 0 && !SR && !WIDE;
     __shared__ uint32_t table[kTable ? kQuotientTableWords : 1];
     float gmax = 0.0f;
     uint4 cur[NQ], nxt[NQ];
@@ -1198,11 +1200,13 @@ static int launch_quant(const void* x, int64_t rows, int64_t cols, int64_t ld, c
         if (!noise && cols % per16 == 0 && ld % per16 == 0 && (uintptr_t)x % 16 == 0) {
             // with scale bytes, one element | 16 bytes per load (both with narrow stores): 18944 x 3584 round to nearest 62.0 | 58.3 us,
             // 4096 x 8960 stochastic 35.7 | 30.4, 2112 x 18944 stochastic with a centre 45.6 | 36.7
-#define METIS_QCS(F) hipLaunchKernelGGL((quant_codes_col_slab_kernel<MODE, SR, WIDE, F>), dim3((unsigned)g), dim3(256), 0, st, x, (uint32_t)rows, \
+#define METIS_QCS(F, T) hipLaunchKernelGGL((quant_codes_col_slab_kernel<MODE, SR, WIDE, F, T>), dim3((unsigned)g), dim3(256), 0, st, x, (uint32_t)rows, \
                                         (uint32_t)cols, ld, seed, offset, (uint2*)codes, (void*)ws.amax, ws.gmax, tiles_c, (uint32_t)tiles, center, \
                                         (uint32_t)(valid < 0 ? rows : valid))
-            if (WIDE && in_f32) METIS_QCS(WIDE);
-            else METIS_QCS(false);
+            constexpr bool table = MODE == 0 && !SR && !WIDE;
+            if (WIDE && in_f32) METIS_QCS(WIDE, false);
+            else if (rows < 64) METIS_QCS(false, false);
+            else METIS_QCS(false, table);
 #undef METIS_QCS
         } else if (WIDE && in_f32)
             hipLaunchKernelGGL((quant_codes_col_kernel<MODE, SR, WIDE, WIDE>), dim3((unsigned)g), dim3(256), 0, st, x,

@@ -827,6 +827,17 @@ def test_scale_bytes_of_binary32_maxima_by_divisions_and_by_three_operations(ops
     assert torch.equal(more.scales[:blocks], p.scales) and torch.equal(more.unit, p.unit)
 
 
+@pytest.mark.parametrize("rows", [16, 48, 64, 80])
+@pytest.mark.parametrize("cols", [8, 64, 1032])
+def test_column_packing_of_few_rows_without_the_table_of_block_maxima(ops, rows, cols):
+    """Binary32 arithmetic on bf16 values, either side of 64 rows: the packing is the row packing of the transpose."""
+    x = synthetic_activation(rows + cols, rows, cols).cuda()
+    x.view(-1)[::61] = 0
+    p, want = ops.quantize(x, 0, col=True), ops.quantize(x.T.contiguous(), 0)
+    _check_packed(p, want.codes.cpu(), want.scales.cpu(), want.unit.cpu())
+    assert torch.equal(ops.quantize(x.float(), 0, col=True).codes, want.codes)
+
+
 # one block, odd tails, either side of the line between the whole-tensor fold and the grid's maximum (256 x 1024 elements in bf16, 144 x
 # 1024 in binary32), leading dimensions, four, eight and sixteen half blocks per thread, the last workgroup partly filled
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
