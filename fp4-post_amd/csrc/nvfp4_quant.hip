@@ -1510,7 +1510,8 @@ int deferred_scales(const void* deferred, int64_t rows, int64_t cols, int mode, 
 // the parked block maxima go where the row quantizer puts them, and ker is written out only when the caller wants the dense result.
 //
 // What bounds it: the SIMDs.  Binary32 MFMAs reach 137 TFLOP/s alone and vector FMAs 96, but the two do not run side by side (63 + 63
-// when mixed in one wave), so the products (14 us of the call at 4096 x 3584, r = 64) and the encoder's vector work add up.  Call
+// when mixed in one wave).  At 4096 x 3584, r = 64 the matrix units are busy 12 and the vector units 9 of the kernel's 27 us; 1.75 of two rounds of
+// workgroups are filled.  Call
 // with its scales launch, in a graph, vector FMAs from LDS tiles before -> now: binary32 4096 x 3584 r = 64 39.5 -> 35.1 us (30.9 with the scale bytes as they are formed now), r = 32
 // 28.3 -> 26.7, 1000 x 2048 r = 64 19.1 -> 10.6, 128 x 1024 r = 32 13.4 -> 8.7; bf16 4096 x 3584 r = 64 39.3 -> 33.4, 2048 x 1536 r = 64
 // 19.7 -> 13.4.  64 rows a wave: 13.7 at 1000 x 2048 (half as many waves), 36.5 at the largest; x requested before the products: 38.1
